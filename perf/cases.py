@@ -150,9 +150,9 @@ def _uniform(seed, tag, shape, lo, hi):
 # Sublayers add to a stream that is larger than what one of them adds (their
 # last matrix is drawn smaller by the root of the number of sublayers), and
 # head norms sharpen attention to a handful of keys, as in trained models.
-EMBED_STD = 0.5
+EMBED_STD = 1.5
 OUT_STD = 0.02 / math.sqrt(72.0)
-HEAD_NORM = 1.5
+HEAD_NORM = 1.25
 
 
 def _projection(case, seed, name, shape, std=0.02):
@@ -230,8 +230,8 @@ def _model(case):
         return mc
     mc = get_model_config(case["model"])
     # e4m3 rounding decides otherwise after any other bf16 rounding, layer
-    # by layer; four layers keep outputs comparable
-    mc.num_layers = min(LAYERS[case["model"]], 4 if case["fp8"] else 99)
+    # by layer; two layers keep outputs comparable
+    mc.num_layers = min(LAYERS[case["model"]], 2 if case["fp8"] else 99)
     mc.quantization = "fp8" if case["fp8"] else None
     return mc
 
@@ -365,13 +365,11 @@ def work(case):
 
 
 def tolerance(case):
-    # measured against exact(); about four times the distance between two
-    # bf16 implementations that round in other places
-    if case["model"] == "Vatunex":
-        return {"rel": 3e-2}
-    if case["model"] == "Qwen3-30B-A3B":
-        return {"rel": 5e-2}     # near-ties of the router fall either way
-    return {"rel": 2e-1 if case["fp8"] else 4e-2}
+    # about four times what exact() is away: 0.0075 (bf16), 0.009 (fp8,
+    # also the distance of two implementations that round in other places),
+    # 0.007 (Vatunex), 0.005 (experts; near-ties of the router fall either
+    # way)
+    return {"rel": 2e-2 if case["model"] == "Qwen3-30B-A3B" else 3e-2}
 
 
 # ------------------------------------------------------------------ exact
