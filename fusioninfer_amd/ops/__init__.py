@@ -236,9 +236,8 @@ def paged_attention_decode(
     return ref.paged_attention_decode(q, k_cache, v_cache, block_tables, seq_lens, scale)
 
 
-# q rows per prefill workgroup (NW waves x 32) — kernel contract; the
-# FI_PF_NW env selects the 4-wave variant on both sides (see
-# prefill_attention.hip launcher)
+# rows per entry of the prefill tile table (128 or 256); the kernel cuts
+# entries into the row blocks of its workgroups itself
 import os as _os
 
 PREFILL_TILE_ROWS = (4 if _os.environ.get("FI_PF_NW", "8").startswith("4")
@@ -246,19 +245,17 @@ PREFILL_TILE_ROWS = (4 if _os.environ.get("FI_PF_NW", "8").startswith("4")
 
 
 def prefill_tile_rows(seq_lens) -> int:
-    """Per-batch workgroup width: 128-row (4-wave) workgroups once any
-    sequence is >=4096 new tokens — the narrower shape halves the
-    causal-raggedness idle and measured +10% at 1x8192 (it loses ~5% at
-    many short sequences, so the default stays 256)."""
+    """Rows per tile-table entry of a batch: 128 once any sequence has 4096
+    new tokens, so that a ragged end leaves fewer empty row blocks."""
     if seq_lens and max(seq_lens) >= 4096:
         return 128
     return PREFILL_TILE_ROWS
 
 
 def build_prefill_tiles(seq_lens, device=None, rows=None):
-    """Host-side tile table for the prefill kernel: one workgroup per
-    `rows` q-rows of each sequence (rows must be 128 or 256 and MATCH
-    the tile_rows passed to the kernel).
+    """Host-side tile table for the prefill kernel: one entry per `rows`
+    q-rows of each sequence (rows must be 128 or 256 and MATCH the
+    tile_rows passed to the kernel).
 
     seq_lens: list[int]. Returns (tile_seq, tile_row0) int32 tensors.
     """

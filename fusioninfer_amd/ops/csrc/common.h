@@ -79,6 +79,14 @@ __host__ __device__ __forceinline__ constexpr int ceil_div(int a, int b) {
   return (a + b - 1) / b;
 }
 
+// How a launch of the prefill attention kernel is laid out: query heads and
+// rows of a workgroup, workgroup row blocks per tile-table entry and in all,
+// and whether K/V ranges are cut into equal parts.
+struct PrefillPlan {
+  int waves, hpb, rows, sub, nq, slots;
+  bool split;
+};
+
 // pack 8 f32 into 8 OCP-e4m3 bytes (two u32 words) via v_cvt_pk_fp8_f32
 FI_DEV void pack_fp8x8(const float* v, unsigned int out[2]) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -106,6 +114,45 @@ FI_DEV void unpack_fp8x4(u32 w, float out[4]) {
   out[3] = hi[1];
 #else
   out[0] = out[1] = out[2] = out[3] = 0.f;
+#endif
+}
+
+// 16 bytes per lane from global memory straight to LDS: lane l's land at
+// lds + 16 l. Base and LDS address are wave-uniform, the byte offset is per
+// lane. In asm because the compiler makes every LDS read wait for all DMAs
+// it knows of; whoever reads the data waits with s_waitcnt vmcnt (DMAs of a
+// wave complete in order) and, for other waves' data, a barrier.
+FI_DEV void dma_to_lds16(u32 lds, const void* base, u32 offset) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %2"
+      :
+      : "s"(lds), "v"(offset), "s"(base)
+      : "memory");  // m0: reserved, set in front of every use
+#endif
+}
+
+// Integers that no kernel of the launch writes, read through the scalar
+// cache (at a wave-uniform index they return on lgkmcnt, not behind the
+// DMAs).
+typedef const __attribute__((address_space(4))) int* ConstInts;
+FI_DEV ConstInts const_ints(const int* p) {
+  return (ConstInts)(reinterpret_cast<uintptr_t>(p));
+}
+
+// Transposing LDS read of 16-bit values: within 16 lanes, lane 4i+j points
+// at entries 4j..4j+3 of row i of a 4 x 16 block and receives the four rows'
+// entries of column (lane & 15).
+FI_DEV __attribute__((ext_vector_type(4))) short lds_read_tr4(
+    const unsigned char* p) {
+  typedef __attribute__((ext_vector_type(4))) short v4;
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) v4*)(p));
+#else
+  return v4{0, 0, 0, 0};
 #endif
 }
 

@@ -29,10 +29,13 @@ void launch_paged_attn_decode(u16*, float*, float*, const u16*, const void*,
                               const void*, const int*, const int*, int,
                               int64_t, int, int, int, int, int, float, bool,
                               hipStream_t);
+PrefillPlan plan_prefill_attn(int, int, int, int, int, int);
+int64_t prefill_piece_floats(const PrefillPlan&, int);
 void launch_prefill_attn(u16*, const u16*, const void*, const void*,
                          const int*, const int*, const int*, const int*,
-                         const int*, int, int, int64_t, int64_t, int64_t, int,
-                         int, int, float, bool, int, hipStream_t);
+                         const int*, int, int64_t, int64_t, int64_t, int, int,
+                         int, float, bool, const PrefillPlan&, float*,
+                         hipStream_t);
 
 }  // namespace fi
 
@@ -265,6 +268,13 @@ void paged_attention_decode(at::Tensor out, at::Tensor q, at::Tensor k_cache,
       current_stream());
 }
 
+// room for the pieces of cut query tiles
+at::Tensor prefill_pieces(const fi::PrefillPlan& pl, const at::Tensor& q) {
+  if (!pl.split) return at::Tensor();
+  return at::empty({fi::prefill_piece_floats(pl, q.size(2))},
+                   q.options().dtype(at::kFloat));
+}
+
 void prefill_attention(at::Tensor out, at::Tensor q, at::Tensor k,
                        at::Tensor v, at::Tensor tile_seq, at::Tensor tile_row0,
                        at::Tensor cu_seqlens, double scale,
@@ -283,13 +293,17 @@ void prefill_attention(at::Tensor out, at::Tensor q, at::Tensor k,
   TORCH_CHECK(q.stride(2) == 1 && q.stride(1) == head_dim);
   TORCH_CHECK(k.stride(2) == 1 && k.stride(1) == head_dim);
   TORCH_CHECK(v.stride(2) == 1 && v.stride(1) == head_dim);
+  const fi::PrefillPlan pl = fi::plan_prefill_attn(
+      tile_seq.size(0), tile_rows, num_q_heads, num_kv_heads, q.size(0),
+      k.size(0));
+  at::Tensor pieces = prefill_pieces(pl, q);
   fi::launch_prefill_attn(
       bf16_ptr(out), bf16_cptr(q), bf16_cptr(k), bf16_cptr(v),
       tile_seq.data_ptr<int>(), tile_row0.data_ptr<int>(),
-      cu_seqlens.data_ptr<int>(), nullptr, nullptr, 0, tile_seq.size(0),
+      cu_seqlens.data_ptr<int>(), nullptr, nullptr, 0,
       q.stride(0), k.stride(0), v.stride(0), num_q_heads, num_kv_heads,
-      head_dim, static_cast<float>(scale), false,
-      static_cast<int>(tile_rows / 32), current_stream());
+      head_dim, static_cast<float>(scale), false, pl,
+      pl.split ? pieces.data_ptr<float>() : nullptr, current_stream());
 }
 
 void prefill_attention_paged(at::Tensor out, at::Tensor q, at::Tensor k_cache,
@@ -314,14 +328,18 @@ void prefill_attention_paged(at::Tensor out, at::Tensor q, at::Tensor k_cache,
   const int num_kv_heads = k_cache.size(1);
   TORCH_CHECK(k_cache.size(2) == 16, "cache block_size must be 16");
   TORCH_CHECK(q.stride(2) == 1 && q.stride(1) == head_dim);
+  const fi::PrefillPlan pl = fi::plan_prefill_attn(
+      tile_seq.size(0), tile_rows, num_q_heads, num_kv_heads, q.size(0),
+      block_tables.size(1) * 16);
+  at::Tensor pieces = prefill_pieces(pl, q);
   fi::launch_prefill_attn(
       bf16_ptr(out), bf16_cptr(q), k_cache.data_ptr(), v_cache.data_ptr(),
       tile_seq.data_ptr<int>(), tile_row0.data_ptr<int>(),
       cu_seqlens.data_ptr<int>(), block_tables.data_ptr<int>(),
-      seq_lens_k.data_ptr<int>(), block_tables.size(1), tile_seq.size(0),
+      seq_lens_k.data_ptr<int>(), block_tables.size(1),
       q.stride(0), 0, 0, num_q_heads, num_kv_heads, head_dim,
-      static_cast<float>(scale), fp8,
-      static_cast<int>(tile_rows / 32), current_stream());
+      static_cast<float>(scale), fp8, pl,
+      pl.split ? pieces.data_ptr<float>() : nullptr, current_stream());
 }
 
 }  // namespace

@@ -1,541 +1,766 @@
-// Varlen causal prefill / context attention (flash-style, MFMA) — v3.
+// Varlen causal prefill / context attention (flash-style, MFMA).
 //
 // out[t, h, :] = softmax(Q K^T * scale, causal) V, GQA, bf16 in / fp32
 // accumulate. PAGED variant reads K/V from the paged cache via block tables
 // (q rows are only each sequence's NEW tokens — prefix-cache hits and
 // chunked prefill skip cached tokens).
 //
-// v3 structure (the 8-wave 32x32 swapped-operand ladder of
-// cdna_hip_programming.md §B):
-//  * workgroup = 8 waves; wave w owns q rows [row0 + 32w, +32); 256 q rows
-//    per workgroup; KV tiles of 64 staged once per workgroup.
-//  * K by global_load_lds (double-buffered, T2 swizzle on the SOURCE
-//    address); V register-staged early (T14) and written TRANSPOSED
-//    (V^T, swizzled rows) so the PV B-fragment is a clean ds_read_b128.
-//  * SWAPPED QK^T: S^T = mfma_f32_32x32x16_bf16(A=K, B=Q) puts each q
-//    row's scores lane-local (C col = lane&31 = q row) — the online
-//    softmax is pure in-register VALU + ONE shfl_xor(32) per reduction
-//    (v2's cross-lane softmax + P-LDS round trip measured 14 VALU insts
-//    per MFMA; this removes both).
-//  * P -> PV A-fragments in-register: pack bf16 pairs + permlane32_swap
-//    half-exchange (guide T12); PV = mfma_32x32x16(A=P, B=V^T read).
-//  * C-fragment row map (32x32): row = (r&3) + 8*(r>>2) + 4*(lane>>5),
-//    col = lane&31.
+// A workgroup holds 32 query vectors per wave of one K/V head: R rows times
+// HPB query heads that share it (HPB = the largest of 4, 2, 1 that divides
+// the group). Rows of one workgroup lie close together, so causal raggedness
+// costs at most one K/V tile per wave.
+//
+// Per K/V tile of 64 tokens:
+//  * K and V rows go from global memory to LDS by DMA, one or two tiles
+//    ahead, ONE barrier per tile. The DMA is written in asm: the compiler
+//    orders every LDS read after every DMA builtin it can see (it emitted
+//    vmcnt(0) in front of each tile's reads, which waited for the tile just
+//    requested); the waits here are the real ones.
+//  * S^T = K Q^T (mfma_32x32x16, A = K): a query's scores sit in one lane
+//    (and its half-wave partner), the softmax is in-register.
+//  * O^T += V^T P^T (A = V^T read from the row-major tile with the LDS
+//    transpose read, B = P^T): the order of the keys within a 16-deep step
+//    is the one in which the score registers already hold them, so P needs
+//    a pack and no lane exchange, and the running maximum, the sum and the
+//    final division stay lane-local too. V staged through registers and
+//    written transposed in 2-byte pieces was the largest part of the tile
+//    before.
+//  * Rows are stored swizzled in 16-byte chunks so that both read patterns
+//    touch every bank evenly.
+// Bound by the vector ALU beside the matrix cores: a tile costs a wave 1024
+// cycles of MFMA and about as many of exponentials, maxima and packs, which
+// two waves per SIMD overlap in part. LDS reads (each wave reads the whole
+// tile) are at two thirds of their rate then.
+//
+// Measured (32 query heads, 8 K/V heads, D 128; before -> now): 8 x 1024
+// tokens 225 -> 101 us (680 TFLOP/s); 1 x 8192 1405 -> 546 us (1008); 4099
+// tokens behind 16384 cached 2867 -> 1250 us (990, split); 43 behind 16384
+// 792 -> 85 us (split).
+//
+// SPLIT: when whole query tiles would leave the chip idle, the K/V tiles of
+// all query tiles form one line that up to 256 workgroups cut into equal
+// parts; a query tile that is cut leaves unnormalised fp32 pieces behind and
+// a second kernel adds them up.
+//
+// C-fragment row map (32x32): row = (r&3) + 8*(r>>2) + 4*(lane>>5),
+// col = lane&31.
 //
 // Capability parity: the paged-attention prefill the reference delegates
 // to vLLM.
 
 #include "common.h"
 
-#include <type_traits>
+#include <cmath>
 
 namespace fi {
 
+typedef __attribute__((ext_vector_type(4))) short short4v;
 typedef __attribute__((ext_vector_type(8))) short short8;
 typedef __attribute__((ext_vector_type(16))) float floatx16;
 
-constexpr int kWaves = 8;
-constexpr int kQPerWave = 32;                 // q rows per wave (1 MFMA block)
-constexpr int kQBlock = kWaves * kQPerWave;   // 256 q rows per workgroup
 constexpr int kKVTile = 64;                   // kv tokens per LDS tile
 constexpr float kPNegInf = -1e30f;
-// defer-max threshold (guide T13): skip the O/l rescale while the tile max
-// grows by <= this much — P is then bounded by e^8, which f32 accumulation
-// absorbs (max-abs error ~3x vs THR=0 per the guide's measurement; the
-// spiked-scores test forces the rescale branch). Scores are in BASE-2
-// units (q pre-scaled by log2e), so the e^8 bound is 8*log2e here.
+// keep the running maximum while a tile's exceeds it by no more than this
+// (base-2 units, e^8): P is then bounded by e^8, which f32 accumulation
+// absorbs, and the accumulators are rescaled only where it matters
 constexpr float kDeferThr = 11.5416f;
 
-// byte-address XOR swizzles, bijective within a ROWB-byte row (guide T2/G4)
-template <int ROWB>
-FI_DEV int swz(int row, int byte_in_row) {
-  constexpr int kMask = (ROWB / 16 > 16 ? 16 : ROWB / 16) - 1;
-  return row * ROWB + (byte_in_row ^ ((row & kMask) << 4));
-}
-
-// C-fragment row for reg r in a 32x32 MFMA (hi1 = lane>>5)
 FI_DEV constexpr int crow(int r, int hi1) {
   return (r & 3) + 8 * (r >> 2) + 4 * hi1;
 }
 
-FI_DEV u32 pack_bf16x2(float lo, float hi) {
-  return static_cast<u32>(f32_to_bf16(lo)) |
-         (static_cast<u32>(f32_to_bf16(hi)) << 16);
+// the other half-wave's value of the same lane & 31
+FI_DEV float half_swap(float v) {
+  const auto s = __builtin_amdgcn_permlane32_swap(
+      __float_as_int(v), __float_as_int(v), false, false);
+  return __int_as_float((threadIdx.x & 32) ? s[0] : s[1]);
 }
 
-// FP8 (PAGED only): the cache holds OCP e4m3 at scale 1.0. K cannot use
-// global_load_lds (the LDS tile must stay bf16 for the MFMA fragments), so
-// both K and V go through the V-style register-stage pipeline with a
-// v_cvt_pk_f32_fp8 dequant between load and ds_write — half the HBM bytes
-// per tile for ~8 extra VALU ops per 16 elements.
-// WPS = target waves per SIMD (__launch_bounds__ 2nd arg, guide §1).
-// Measured: WPS=3 spills ~55 slots and LOSES 40% — the kernel is
-// register-bound at 2 waves/SIMD; keep 2.
-// NW = waves per workgroup (q rows = NW*32). 8 = round-1 shape; 4 halves
-// the causal-raggedness idle (a wave's tiles stop at its own diagonal
-// but it still barriers with later waves) at the cost of re-reading K/V
-// tiles from L2 by 2x more workgroups — A/B'd on hardware (FI_PF_NW).
-template <int D, bool PAGED, bool FP8, int WPS = 2, int NW = kWaves>
-__global__ __launch_bounds__(NW * kWaveSize, WPS) void prefill_attn_kernel(
-    u16* __restrict__ out,        // [T, Hq, D]
-    const u16* __restrict__ q,    // [T] rows, stride q_stride
-    const void* __restrict__ k_p, // dense rows OR k_cache when PAGED
-    const void* __restrict__ v_p, // dense rows OR v_cache when PAGED
-    const int* __restrict__ tile_seq,    // [ntiles] sequence index
-    const int* __restrict__ tile_row0,   // [ntiles] first NEW q row
-    const int* __restrict__ cu_seqlens,  // [nseqs+1] over NEW tokens
-    const int* __restrict__ block_tables,  // [S, max_blocks] (PAGED)
-    const int* __restrict__ seq_lens_k,    // [S] total ctx len (PAGED)
-    const int max_blocks,
-    const int64_t q_stride, const int64_t k_stride, const int64_t v_stride,
-    const int num_q_heads, const int num_kv_heads, const float scale) {
-  using CT = typename std::conditional<FP8, unsigned char, u16>::type;
-  const CT* k = static_cast<const CT*>(k_p);
-  const CT* v = static_cast<const CT*>(v_p);
-  constexpr int KF = D / 16;           // QK^T 16-deep k-chunks over head dim
-  constexpr int CB = D / 32;           // PV output 32-col blocks
-  constexpr int kKRowB = D * 2;        // K row bytes (D=128 -> 256)
-  // V^T rows at their natural 128 B with the (row&7)<<4 in-row swizzle.
-  // Round 1 padded them to 256 B for the conflict-free (row&15)<<4
-  // swizzle — but that put the workgroup at 98 KB LDS = ONE block/CU
-  // (2 waves/SIMD), and PMC showed the kernel latency-bound there
-  // (MfmaUtil 11%, SQ_WAIT dominant). 64 KB -> 2 blocks/CU buys 2x the
-  // latency hiding for a measured 2.6% bank-conflict cost on the PV
-  // reads.
-  constexpr int kVTRowB = 128;
+struct PrefillArgs {
+  u16* out;               // [T, Hq, D]
+  const u16* q;           // [T] rows, stride q_stride
+  const void* k;          // dense rows OR k_cache when PAGED
+  const void* v;
+  const int* tile_seq;    // [ntiles] sequence index
+  const int* tile_row0;   // [ntiles] first NEW q row
+  const int* cu_seqlens;  // [nseqs+1] over NEW tokens
+  const int* block_tables;  // [S, max_blocks] (PAGED)
+  const int* seq_lens_k;    // [S] total ctx len (PAGED)
+  float* piece_o;           // [slots][2][256 * D]  (SPLIT)
+  float* piece_ml;          // [slots][2][waves][64][2] (SPLIT)
+  int4* cut;                // [slots] what a part's end cuts (SPLIT)
+  int64_t q_stride, k_stride, v_stride;
+  int max_blocks, num_q_heads, num_kv_heads;
+  int hpb;                  // query heads per workgroup
+  int rows;                 // rows per workgroup
+  int slots;                // workgroups of the SPLIT form
+  int sub;                  // query tiles per entry of the tile table
+  int nq;                   // query tiles in all
+  float scale;
+};
 
-  const int head = blockIdx.y;
-  const int kv_head = head / (num_q_heads / num_kv_heads);
+// one query tile: rows [row0, ..) of a sequence and its K/V tiles
+struct QTile {
+  int seq, row0, seq_start, seq_len, k_len, work;
+};
+
+template <bool PAGED>
+FI_DEV QTile q_tile(const PrefillArgs& p, int qt) {
+  QTile t;
+  const int rows = p.rows;
+  const int tile = qt / p.sub;
+  t.seq = p.tile_seq[tile];
+  t.row0 = p.tile_row0[tile] + (qt - tile * p.sub) * rows;
+  t.seq_start = p.cu_seqlens[t.seq];
+  t.seq_len = p.cu_seqlens[t.seq + 1] - t.seq_start;
+  t.k_len = PAGED ? p.seq_lens_k[t.seq] : t.seq_len;
+  t.work = 0;
+  if (t.row0 < t.seq_len)
+    t.work = (t.k_len - t.seq_len + min(t.row0 + rows, t.seq_len) - 1) /
+                 kKVTile + 1;
+  return t;
+}
+
+FI_DEV QTile uniform_tile(QTile t) {
+  t.seq = __builtin_amdgcn_readfirstlane(t.seq);
+  t.row0 = __builtin_amdgcn_readfirstlane(t.row0);
+  t.seq_start = __builtin_amdgcn_readfirstlane(t.seq_start);
+  t.seq_len = __builtin_amdgcn_readfirstlane(t.seq_len);
+  t.k_len = __builtin_amdgcn_readfirstlane(t.k_len);
+  t.work = __builtin_amdgcn_readfirstlane(t.work);
+  return t;
+}
+
+// the K/V tiles of all query tiles of one head group, by one wave
+template <bool PAGED>
+FI_DEV int total_work(const PrefillArgs& p, int lane) {
+  int sum = 0;
+  for (int i = lane; i < p.nq; i += kWaveSize) sum += q_tile<PAGED>(p, i).work;
+#pragma unroll
+  for (int off = 32; off; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  return __builtin_amdgcn_readfirstlane(sum);
+}
+
+// query tile that holds place `at` of a head group's line, and the place
+// within it; every wave of the launch computes the same
+template <bool PAGED>
+FI_DEV int find_tile(const PrefillArgs& p, int lane, int at, int* within) {
+  int before = 0;
+  for (int i0 = 0; i0 < p.nq; i0 += kWaveSize) {
+    const int i = i0 + lane;
+    const int w = i < p.nq ? q_tile<PAGED>(p, i).work : 0;
+    int incl = w;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int o = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += o;
+    }
+    const unsigned long long hit = __ballot(before + incl > at);
+    if (hit) {
+      const int l = __builtin_ctzll(hit);
+      *within = __builtin_amdgcn_readfirstlane(
+          at - before - (__shfl(incl, l, 64) - __shfl(w, l, 64)));
+      return i0 + l;
+    }
+    before += __builtin_amdgcn_readfirstlane(__shfl(incl, 63, 64));
+  }
+  *within = 0;
+  return p.nq;
+}
+
+// place of a workgroup's part in the whole line: neighbours on one XCD
+// (every eighth workgroup) take neighbouring parts and share K/V in its L2
+FI_DEV int split_slot(int b, int slots) {
+  return (b & 7) * (slots / 8) + (b >> 3);
+}
+struct Parts {
+  int64_t each;  // tiles of a part; the first `more` parts have one more
+  int more;
+  FI_DEV Parts(int64_t total, int slots)
+      : each(total / slots), more(static_cast<int>(total % slots)) {}
+  FI_DEV int64_t begin(int slot) const {
+    return slot * each + min(slot, more);
+  }
+};
+
+// FP8 (PAGED only): the cache holds OCP e4m3. LDS tiles stay bf16, so K and
+// V pass through registers with an exact conversion (half the bytes from
+// memory), one tile ahead.
+//
+// SPLIT runs one workgroup of 8 waves per CU, which reads K/V half as often,
+// with three buffers; the other form two workgroups of 4 waves with two, so
+// that one computes while the other fills its first tile (8 x 1024 tokens:
+// 101 us against 116 us with 8 waves; equal from 4096 rows on).
+constexpr int attn_waves(bool split) { return split ? 8 : 4; }
+
+template <int D, bool PAGED, bool FP8, bool SPLIT>
+__global__ __launch_bounds__(attn_waves(SPLIT) * kWaveSize, 2)
+void prefill_attn_kernel(const PrefillArgs p) {
+  constexpr int kWaves = attn_waves(SPLIT), kBufs = SPLIT ? 3 : 2;
+  constexpr int KF = D / 16;           // QK^T 16-deep steps over head dim
+  constexpr int CB = D / 32;           // 32-dim blocks of the output
+  constexpr int kRowB = D * 2;         // bytes of a K or V row
+  constexpr int kChunk = D / 8;        // 16-byte chunks of a row
+  constexpr int kTileB = kKVTile * kRowB;
+  constexpr int kRowsPerDma = 1024 / kRowB;
+  constexpr int kWRows = kKVTile / kWaves;   // rows a wave copies
+  constexpr int kDma = kWRows / kRowsPerDma;  // DMAs per wave and matrix
+  static_assert(D == 128 || D == 64, "swizzles are for these row sizes");
+
+  __shared__ __attribute__((aligned(1024)))
+  unsigned char smem[2 * kBufs * kTileB];
+  const u32 lds0 = static_cast<u32>(reinterpret_cast<uintptr_t>(
+      (__attribute__((address_space(3))) unsigned char*)smem));
+
   const int tid = threadIdx.x;
-  const int wave = tid / kWaveSize;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWaveSize);
   const int lane = tid % kWaveSize;
-  const int col = lane & 31;           // this lane's q row (within the wave)
+  const int col = lane & 31;           // this lane's query vector
   const int hi1 = lane >> 5;
+  const int wph = kWaves / p.hpb;      // waves per query head
 
-  const int seq = tile_seq[blockIdx.x];
-  const int seq_start = cu_seqlens[seq];
-  const int seq_len = cu_seqlens[seq + 1] - seq_start;  // NEW q rows
-  const int k_len = PAGED ? seq_lens_k[seq] : seq_len;  // total kv rows
-  const int ctx_start = k_len - seq_len;
-  const int wg_row0 = tile_row0[blockIdx.x];
-  const int row0 = wg_row0 + wave * kQPerWave;
-  const bool active = row0 < seq_len;
-  const int* bt_row = PAGED
-      ? block_tables + static_cast<int64_t>(seq) * max_blocks : nullptr;
-  auto kv_off = [&](int r, int64_t dense_stride) -> int64_t {
-    if (PAGED) {
-      const int blk = bt_row[r >> 4];
-      return ((static_cast<int64_t>(blk) * num_kv_heads + kv_head) * 16 +
-              (r & 15)) * D;
-    }
-    return (seq_start + r) * dense_stride + static_cast<int64_t>(kv_head) * D;
+  // swizzled chunk of a row: K rows are read one chunk per lane over 32
+  // rows, V rows four lanes to 32 bytes over 8 rows
+  auto k_swz = [](int row) { return D == 128 ? row & 15 : (row >> 1) & 7; };
+  auto v_swz = [](int row) {
+    return D == 128 ? (row & 3) << 2 : ((row >> 1) & 1) << 2;
   };
-
-  // LDS: TRIPLE-buffered K (glds target, prefetch depth 2 so a K tile
-  // stays in flight ACROSS the tile barrier — round-2: with 2 buffers
-  // every barrier drained the glds queue, the guide's ~20% structural
-  // stall) + double-buffered V^T; ONE barrier per tile, raw s_barrier +
-  // counted vmcnt for bf16 (guide §5 "pipelining across barriers").
-  // ONE __shared__ object (guide §5 ".s-level traps" (a)).
-  __shared__ u16 smem[3 * kKVTile * D + 2 * D * (kVTRowB / 2)];
-  auto k_lds = [&](int i) -> u16* { return smem + i * (kKVTile * D); };
-  u16* vt_lds0 = smem + 3 * kKVTile * D;
-  u16* vt_lds1 = vt_lds0 + D * (kVTRowB / 2);
-
-  // ---- Q fragments (the QK^T B operand): lane holds
-  // Q[row0+col][f*16 + hi1*8 .. +8] for each 16-deep k-chunk f
-  // Q pre-scaled by scale*log2e ONCE: the softmax then runs in base-2
-  // (exp2 of the raw MFMA scores) with no per-tile scale multiply and no
-  // exp argument multiply — ~64 fewer VALU ops per lane per tile.
-  // exp2(s*scale*log2e) == exp(s*scale) exactly as a function; the bf16
-  // re-round of q*scale adds ~2^-9 relative score noise (within the
-  // kernel's fp32-reference tolerance).
-  short8 b_q[KF];
-  if (active) {
-    const int qr = min(row0 + col, seq_len - 1);
-    const u16* qrow = q + (seq_start + qr) * q_stride +
-                      static_cast<int64_t>(head) * D;
-    const float qs = scale * 1.4426950408889634f;  // log2(e)
+  int k_off[KF], v_off[CB];
 #pragma unroll
-    for (int f = 0; f < KF; ++f) {
-      short8 raw = *reinterpret_cast<const short8*>(qrow + f * 16 + hi1 * 8);
-      bf16x8 h = __builtin_bit_cast(bf16x8, raw);
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        h.h[j] = f32_to_bf16(bf16_to_f32(h.h[j]) * qs);
-      b_q[f] = __builtin_bit_cast(short8, h);
-    }
-  }
-
-  // online-softmax state: ONE q row per lane (lanes j and j+32 share row j)
-  float m_row = kPNegInf, l_row = 0.f;
-  floatx16 o_acc[CB];
-#pragma unroll
-  for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) o_acc[cb][r] = 0.f;
-
-  const int wg_q_max = ctx_start + min(wg_row0 + NW * kQPerWave, seq_len) - 1;
-  const int num_kv_tiles = wg_q_max / kKVTile + 1;
-  const int my_q_max = ctx_start + min(row0 + kQPerWave, seq_len) - 1;
-
-  // ---- staging (same pipeline as v2.1) --------------------------------
-  constexpr int kKTileBytes = kKVTile * kKRowB;
-  constexpr int kGldsPerWave = kKTileBytes / (NW * kWaveSize * 16);
-  auto stage_k_glds = [&](int t, u16* kbuf) {
-    const int kv0 = t * kKVTile;
-#pragma unroll
-    for (int i = 0; i < kGldsPerWave; ++i) {
-      const int base_off = wave * (kKTileBytes / NW) + i * (kWaveSize * 16);
-      const int X = base_off + lane * 16;
-      const int row = X / kKRowB;
-      const int sbyte = X % kKRowB;
-      constexpr int kMask = (kKRowB / 16 > 16 ? 16 : kKRowB / 16) - 1;
-      const int byte = sbyte ^ ((row & kMask) << 4);
-      const int src_row = min(kv0 + row, k_len - 1);
-      const CT* gsrc = k + kv_off(src_row, k_stride) + byte / sizeof(u16);
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void*)gsrc,
-          (__attribute__((address_space(3))) void*)(
-              reinterpret_cast<char*>(kbuf) + base_off),
-          16, 0, 0);
-    }
-  };
-  constexpr int kChunks = D / 16;
-  // each thread owns VITER (c16, token) staging positions so every NW
-  // covers the full 64 x D tile (NW=8/D=128: 1; NW=4/D=128: 2)
-  constexpr int VITER = ceil_div(kChunks, NW);
-  const int v_kv = tid % kKVTile;
-  const int v_c0 = tid / kKVTile;  // first 16-dim chunk; step NW per iter
-  // 16 fp8 bytes (one uint4) -> two bf16x8
-  auto cvt_fp8x16 = [](uint4 raw, bf16x8& lo, bf16x8& hi) {
-    const u32 w[4] = {raw.x, raw.y, raw.z, raw.w};
-    float f[16];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) unpack_fp8x4(w[i], &f[i * 4]);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      lo.h[j] = f32_to_bf16(f[j]);
-      hi.h[j] = f32_to_bf16(f[8 + j]);
-    }
-  };
-  bf16x8 vreg0[VITER], vreg1[VITER];
-  auto vload = [&](int t) {
-    const int src = min(t * kKVTile + v_kv, k_len - 1);
-    const CT* vrow = v + kv_off(src, v_stride);
-#pragma unroll
-    for (int it = 0; it < VITER; ++it) {
-      const int c16 = v_c0 + it * NW;
-      if (c16 >= kChunks) break;
-      if (FP8) {
-        cvt_fp8x16(*reinterpret_cast<const uint4*>(vrow + c16 * 16),
-                   vreg0[it], vreg1[it]);
-      } else {
-        vreg0[it] = *reinterpret_cast<const bf16x8*>(vrow + c16 * 16);
-        vreg1[it] = *reinterpret_cast<const bf16x8*>(
-            reinterpret_cast<const u16*>(vrow + c16 * 16) + 8);
-      }
-    }
-  };
-  // FP8 K staging: same (row, 16-col chunk) ownership as V, but written
-  // UNtransposed into the K tile layout ([64 rows][D] bf16, row swizzle);
-  // each converted 16-elem group is one 16-B-aligned ds_write_b128 pair
-  bf16x8 kreg0[VITER], kreg1[VITER];
-  auto kload_fp8 = [&](int t) {
-    const int src = min(t * kKVTile + v_kv, k_len - 1);
-    const CT* krow = k + kv_off(src, k_stride);
-#pragma unroll
-    for (int it = 0; it < VITER; ++it) {
-      const int c16 = v_c0 + it * NW;
-      if (c16 >= kChunks) break;
-      cvt_fp8x16(*reinterpret_cast<const uint4*>(krow + c16 * 16),
-                 kreg0[it], kreg1[it]);
-    }
-  };
-  auto kwrite_fp8 = [&](u16* kbuf) {
-    char* kbase = reinterpret_cast<char*>(kbuf);
-#pragma unroll
-    for (int it = 0; it < VITER; ++it) {
-      const int c16 = v_c0 + it * NW;
-      if (c16 >= kChunks) break;
-      *reinterpret_cast<bf16x8*>(
-          kbase + swz<kKRowB>(v_kv, (c16 * 16) * 2)) = kreg0[it];
-      *reinterpret_cast<bf16x8*>(
-          kbase + swz<kKRowB>(v_kv, (c16 * 16 + 8) * 2)) = kreg1[it];
-    }
-  };
-  auto vwrite = [&](u16* vt_buf) {
-    char* vbase = reinterpret_cast<char*>(vt_buf);
-#pragma unroll
-    for (int it = 0; it < VITER; ++it) {
-      const int c16 = v_c0 + it * NW;
-      if (c16 >= kChunks) break;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        *reinterpret_cast<u16*>(
-            vbase + swz<kVTRowB>(c16 * 16 + j, v_kv * 2)) = vreg0[it].h[j];
-        *reinterpret_cast<u16*>(
-            vbase + swz<kVTRowB>(c16 * 16 + j + 8, v_kv * 2)) = vreg1[it].h[j];
-      }
-    }
-  };
-
-  // hoist the swizzled LDS read offsets (constant per lane) out of the
-  // tile loop — the swz() address math was otherwise recomputed per tile
-  int k_off[2][KF];
-  int v_off[4][CB];
-#pragma unroll
-  for (int f = 0; f < KF; ++f) {
-    k_off[0][f] = swz<kKRowB>(col, f * 32 + hi1 * 16);
-    k_off[1][f] = swz<kKRowB>(32 + col, f * 32 + hi1 * 16);
-  }
-#pragma unroll
-  for (int kc = 0; kc < 4; ++kc)
+  for (int f = 0; f < KF; ++f)
+    k_off[f] = col * kRowB + (((2 * f + hi1) ^ k_swz(col)) * 16);
+  {
+    const int row = 4 * hi1 + ((lane & 15) >> 2);
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb)
-      v_off[kc][cb] = swz<kVTRowB>(cb * 32 + col, kc * 32 + hi1 * 16);
-
-  // outstanding-vmem count a tile barrier leaves in flight: the NEWEST
-  // K-tile glds (kGldsPerWave wave ops) + the newest V loads (2 per
-  // VITER) — everything older (incl. the K tile consumed next) drains.
-  // Staging is UNCONDITIONAL with clamped source rows, so the count is
-  // a compile-time constant on every iteration (no ragged tail).
-  constexpr int kAhead = kGldsPerWave + 2 * VITER;
-  auto tile_barrier = [&] {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAhead) : "memory");
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-  };
-
-  // prologue: K(0)+K(1) and V(0)+V(1) in flight, vt[0] published
-  if (FP8) {
-    kload_fp8(0);
-    vload(0);
-    kwrite_fp8(k_lds(0));
-    vwrite(vt_lds0);
-    if (num_kv_tiles > 1) {
-      kload_fp8(1);
-      vload(1);
-    }
-    __syncthreads();        // publishes K(0) + vt[0]
-  } else {
-    stage_k_glds(0, k_lds(0));
-    vload(0);
-    stage_k_glds(1, k_lds(1));
-    // drain K(0) (own portion; the barrier below publishes cross-wave)
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAhead) : "memory");
-    vwrite(vt_lds0);
-    vload(1);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();   // publishes K(0) + vt[0]
+      v_off[cb] = row * kRowB +
+                  (((cb * 4 + ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1)) ^
+                    v_swz(row)) * 16) + (lane & 1) * 8;
   }
 
-  for (int t = 0; t < num_kv_tiles; ++t) {
-    const int kv0 = t * kKVTile;
-    u16* kbuf = FP8 ? k_lds(t & 1) : k_lds(t % 3);
-    u16* kbuf_next = k_lds((t + 1) & 1);  // fp8 staging target
-    const u16* vt_cur = (t & 1) ? vt_lds1 : vt_lds0;
-    u16* vt_next = (t & 1) ? vt_lds0 : vt_lds1;
+  // a negative scale turns the queries round, a zero one clears them, so
+  // that the maximum can be taken over unscaled scores
+  const float sgn = p.scale > 0.f ? 1.f : (p.scale < 0.f ? -1.f : 0.f);
+  const float c = p.scale == 0.f
+      ? 1.f : fabsf(p.scale) * 1.4426950408889634f;  // log2(e)
 
-    // depth-2 K prefetch (clamped rows: past-the-end tiles re-read the
-    // last row — a few hundred wasted bytes beat a ragged vmcnt count)
-    if (!FP8) stage_k_glds(t + 2, k_lds((t + 2) % 3));
+  int64_t pos = 0, pos_end = 1;
+  int slot = 0, hg = 0, qt, from = 0;
+  // SPLIT: (head group, query tile, slot behind the last piece's, 0) of the
+  // tile that begins in this part and is cut by its end; -1: none
+  int4 cut = make_int4(0, -1, 0, 0);
+  if (SPLIT) {
+    const int u = total_work<PAGED>(p, lane);
+    const int64_t total = static_cast<int64_t>(u) * (p.num_q_heads / p.hpb);
+    slot = split_slot(blockIdx.x, p.slots);
+    const Parts parts(total, p.slots);
+    pos = parts.begin(slot);
+    pos_end = parts.begin(slot + 1);
+    if (pos < pos_end) {
+      hg = static_cast<int>(pos / u);
+      qt = find_tile<PAGED>(p, lane, static_cast<int>(pos - int64_t(hg) * u),
+                            &from);
+    }
+    // the tile at the end: the part itself or a later one finishes it
+    if (pos < pos_end && pos_end < total) {
+      const int h = static_cast<int>(pos_end / u);
+      int within;
+      const int i = find_tile<PAGED>(
+          p, lane, static_cast<int>(pos_end - int64_t(h) * u), &within);
+      if (within > 0 && pos_end - within >= pos) {
+        const int64_t end = pos_end - within + q_tile<PAGED>(p, i).work;
+        cut = make_int4(h, i, slot + 1, 0);
+        while (cut.z < p.slots && parts.begin(cut.z) < end) ++cut.z;
+      }
+    }
+    if (tid == 0) p.cut[slot] = cut;
+  } else {
+    // head groups side by side (neighbouring workgroups go to different
+    // XCDs), the longest query tiles first
+    const int groups = p.num_q_heads / p.hpb;
+    hg = blockIdx.x % groups;
+    qt = p.nq - 1 - blockIdx.x / groups;
+  }
 
-    const bool compute = active && kv0 <= my_q_max;
-    floatx16 s_acc[2];  // S^T for kv blocks [kv0, +32) and [kv0+32, +64)
-    if (compute) {
-      const char* kbase = reinterpret_cast<const char*>(kbuf);
+  while (pos < pos_end) {
+    const QTile t = uniform_tile(q_tile<PAGED>(p, qt));
+    if (t.work == 0) {                 // rows past the sequence's end
+      if (!SPLIT) return;
+      if (++qt == p.nq) { qt = 0; ++hg; }
+      continue;
+    }
+    const int ta = from;
+    const int tb = SPLIT
+        ? static_cast<int>(min(static_cast<int64_t>(t.work),
+                               from + (pos_end - pos)))
+        : t.work;
+    const int head = hg * p.hpb + wave / wph;
+    const int kv_head = hg * p.hpb / (p.num_q_heads / p.num_kv_heads);
+    const int ctx_start = t.k_len - t.seq_len;
+    const int row0 = t.row0 + (wave % wph) * 32;
+    const bool active = row0 < t.seq_len;
+    const int last_blk = (t.k_len - 1) >> 4;
+    const ConstInts bt_row = const_ints(
+        PAGED ? p.block_tables + static_cast<int64_t>(t.seq) * p.max_blocks
+              : nullptr);
+
+    // ---- staging ---------------------------------------------------------
+    // wave w copies rows 8w..8w+7 of a tile: half a cache block. Rows past
+    // the end repeat the last one (finite values; their scores are masked).
+    auto block_of = [&](int tile) {
+      return bt_row[min(tile * 4 + wave * kWRows / 16, last_blk)];
+    };
+    auto stage_dma = [&](int tile, int blk, int buf) {
+      const u32 kdst = lds0 + buf * kTileB + wave * kWRows * kRowB;
+      const u32 vdst = kdst + kBufs * kTileB;
+      const u16* kb;
+      const u16* vb;
+      int first, limit;                // row of the wave, last valid row
+      int64_t ks, vs;
+      if (PAGED) {
+        const int64_t base =
+            (static_cast<int64_t>(blk) * p.num_kv_heads + kv_head) * 16 * D;
+        kb = static_cast<const u16*>(p.k) + base;
+        vb = static_cast<const u16*>(p.v) + base;
+        const int b = min(tile * 4 + wave * kWRows / 16, last_blk);
+        first = wave * kWRows & 15;
+        limit = t.k_len - 1 - b * 16;
+        ks = vs = D;
+      } else {
+        const int r0 = min(tile * kKVTile, t.k_len - 1);
+        kb = static_cast<const u16*>(p.k) +
+             (t.seq_start + r0) * p.k_stride + int64_t(kv_head) * D;
+        vb = static_cast<const u16*>(p.v) +
+             (t.seq_start + r0) * p.v_stride + int64_t(kv_head) * D;
+        first = wave * kWRows;
+        limit = t.k_len - 1 - r0;
+        ks = p.k_stride;
+        vs = p.v_stride;
+      }
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
+      for (int i = 0; i < kDma; ++i) {
+        const int r = i * kRowsPerDma + lane / kChunk;  // row of the wave
+        const int tr = wave * kWRows + r;                    // row of the tile
+        const int src = min(first + r, limit);
+        const u32 ko = static_cast<u32>(
+            src * static_cast<int>(ks) * 2 +
+            (((lane % kChunk) ^ k_swz(tr)) * 16));
+        const u32 vo = static_cast<u32>(
+            src * static_cast<int>(vs) * 2 +
+            (((lane % kChunk) ^ v_swz(tr)) * 16));
+        dma_to_lds16(kdst + i * 1024, kb, ko);
+        dma_to_lds16(vdst + i * 1024, vb, vo);
+      }
+    };
+    // fp8: a thread owns 16 dims of one row of K and of V
+    constexpr int kParts = D / 16;
+    constexpr int kStep = kWaves * kWaveSize / kParts;  // rows per step
+    constexpr int kSteps = ceil_div(kKVTile, kStep);
+    const int f_row0 = tid / kParts, f_part = tid % kParts;
+    const bool f_own = kStep <= kKVTile || f_row0 < kKVTile;
+    uint4 k_raw[kSteps], v_raw[kSteps];
+    auto load_fp8 = [&](int tile) {
+      if (!f_own) return;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s_acc[b][r] = 0.f;
-      // ---- swapped QK^T: S^T[kv 64 x q 32] ----
-      __builtin_amdgcn_s_setprio(1);
+      for (int i = 0; i < kSteps; ++i) {
+        const int src = min(tile * kKVTile + f_row0 + i * kStep, t.k_len - 1);
+        const int64_t off =
+            ((static_cast<int64_t>(bt_row[src >> 4]) * p.num_kv_heads +
+              kv_head) * 16 + (src & 15)) * D + f_part * 16;
+        k_raw[i] = *reinterpret_cast<const uint4*>(
+            static_cast<const unsigned char*>(p.k) + off);
+        v_raw[i] = *reinterpret_cast<const uint4*>(
+            static_cast<const unsigned char*>(p.v) + off);
+      }
+    };
+    auto write_fp8 = [&](int buf) {
+      if (!f_own) return;
+      auto put = [&](unsigned char* dst, const uint4& raw, int f_row,
+                     int swz) {
+        const u32 w[4] = {raw.x, raw.y, raw.z, raw.w};
+        float f[16];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) unpack_fp8x4(w[i], &f[i * 4]);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          bf16x8 o;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) o.h[j] = f32_to_bf16(f[h * 8 + j]);
+          *reinterpret_cast<bf16x8*>(
+              dst + f_row * kRowB + (((f_part * 2 + h) ^ swz) * 16)) = o;
+        }
+      };
+#pragma unroll
+      for (int i = 0; i < kSteps; ++i) {
+        const int r = f_row0 + i * kStep;
+        put(smem + buf * kTileB, k_raw[i], r, k_swz(r));
+        put(smem + (kBufs + buf) * kTileB, v_raw[i], r, v_swz(r));
+      }
+    };
+
+    // the previous query tile's LDS reads are over in every wave
+    if (SPLIT) __builtin_amdgcn_s_barrier();
+    int blk = 0;
+    if (FP8) {
+      load_fp8(ta);
+      write_fp8(0);
+      if (ta + 1 < tb) load_fp8(ta + 1);
+    } else {
+      stage_dma(ta, PAGED ? block_of(ta) : 0, 0);
+      if (kBufs == 3 && ta + 1 < tb)
+        stage_dma(ta + 1, PAGED ? block_of(ta + 1) : 0, 1);
+      if (PAGED) blk = block_of(ta + kBufs - 1);
+    }
+
+    // ---- query fragments (B operand of S^T): lane holds
+    // Q[row0+col][f*16 + hi1*8 .. +8]
+    short8 b_q[KF];
+    if (active) {
+      const int qr = min(row0 + col, t.seq_len - 1);
+      const u16* qrow = p.q + (t.seq_start + qr) * p.q_stride +
+                        static_cast<int64_t>(head) * D;
 #pragma unroll
       for (int f = 0; f < KF; ++f) {
-        const short8 a_k0 =
-            *reinterpret_cast<const short8*>(kbase + k_off[0][f]);
-        const short8 a_k1 =
-            *reinterpret_cast<const short8*>(kbase + k_off[1][f]);
-        s_acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            a_k0, b_q[f], s_acc[0], 0, 0, 0);
-        s_acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            a_k1, b_q[f], s_acc[1], 0, 0, 0);
+        b_q[f] = *reinterpret_cast<const short8*>(qrow + f * 16 + hi1 * 8);
+        if (sgn != 1.f) {
+          bf16x8 h = __builtin_bit_cast(bf16x8, b_q[f]);
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            h.h[j] = f32_to_bf16(bf16_to_f32(h.h[j]) * sgn);
+          b_q[f] = __builtin_bit_cast(short8, h);
+        }
       }
-      __builtin_amdgcn_s_setprio(0);
+      // arrived here, not at their first use: that is inside the loop,
+      // where the wait would take in the DMAs of every tile
+#pragma unroll
+      for (int f = 0; f < KF; ++f) asm volatile("" : "+v"(b_q[f]));
+    }
 
-      // ---- in-register online softmax (row = col, lane-local) ----
-      const int q_pos = ctx_start + row0 + col;     // this lane's q row
-      const bool row_valid = row0 + col < seq_len;
-      // interior tiles (all kv strictly before every valid q row, no
-      // ragged tail, no invalid rows) skip the per-element masking
-      const bool need_mask =
-          (kv0 + kKVTile - 1 > ctx_start + row0)
-          || (kv0 + kKVTile > k_len)
-          || (row0 + kQPerWave > seq_len);
-      if (need_mask) {
+    float m_row = kPNegInf, l_row = 0.f;   // l of this half-wave's keys
+    floatx16 o_acc[CB];
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o_acc[cb][r] = 0.f;
+
+    const int my_q_max = ctx_start + min(row0 + 32, t.seq_len) - 1;
+    const int q_pos = ctx_start + row0 + col;
+    int buf = 0;
+    for (int tile = ta; tile < tb; ++tile) {
+      const int kv0 = tile * kKVTile;
+      // this tile has landed (this wave's part; the barrier covers the
+      // others'), and nobody reads the buffer that is filled next
+      if (!FP8) {
+        if (kBufs == 3 && tile + 1 < tb)
+          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kDma) : "memory");
+        else
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      const int buf1 = buf == kBufs - 1 ? 0 : buf + 1;
+      if (FP8) {
+        if (tile + 1 < tb) write_fp8(buf1);
+        if (tile + 2 < tb) load_fp8(tile + 2);
+      } else if (tile + kBufs - 1 < tb) {
+        stage_dma(tile + kBufs - 1, blk,
+                  kBufs == 2 ? buf1 : (buf1 == kBufs - 1 ? 0 : buf1 + 1));
+        if (PAGED) blk = block_of(tile + kBufs);
+      }
+
+      if (active && kv0 <= my_q_max) {
+        const unsigned char* kbase = smem + buf * kTileB;
+        const unsigned char* vbase = smem + (kBufs + buf) * kTileB;
+        // ---- S^T[kv 64 x q 32] ----
+        floatx16 s_acc[2];
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int f = 0; f < KF; ++f)
+#pragma unroll
+          for (int b = 0; b < 2; ++b) {
+            const short8 a_k = *reinterpret_cast<const short8*>(
+                kbase + k_off[f] + b * 32 * kRowB);
+            if (f == 0) {
+              const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f,
+                                     0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+              s_acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                  a_k, b_q[f], zero, 0, 0, 0);
+            } else {
+              s_acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                  a_k, b_q[f], s_acc[b], 0, 0, 0);
+            }
+          }
+        __builtin_amdgcn_s_setprio(0);
+
+        // ---- online softmax; only tiles at the diagonal or the end mask
+        if (kv0 + kKVTile - 1 > ctx_start + row0) {
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+              if (kv0 + 32 * b + crow(r, hi1) > q_pos)
+                s_acc[b][r] = -INFINITY;
+        }
+        float rm = fmaxf(s_acc[0][0], s_acc[1][0]);
+#pragma unroll
+        for (int r = 1; r < 16; ++r)
+          rm = fmaxf(rm, fmaxf(s_acc[0][r], s_acc[1][r]));
+        rm = fmaxf(rm, half_swap(rm));
+        if (!__all((rm - m_row) * c <= kDeferThr)) {
+          const float m_new = fmaxf(m_row, rm);
+          const float alpha = __builtin_amdgcn_exp2f((m_row - m_new) * c);
+          m_row = m_new;
+          l_row *= alpha;
+#pragma unroll
+          for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o_acc[cb][r] *= alpha;
+        }
+        const float mc = m_row * c;
+        float rs[4] = {0.f, 0.f, 0.f, 0.f};
+        short8 b_p[4];
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int kv_pos = kv0 + 32 * b + crow(r, hi1);
-            if (!row_valid || kv_pos > q_pos || kv_pos >= k_len)
-              s_acc[b][r] = kPNegInf;
+          for (int h = 0; h < 2; ++h) {
+            bf16x8 w;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              const float pv = __builtin_amdgcn_exp2f(
+                  fmaf(s_acc[b][8 * h + j], c, -mc));
+              rs[j & 3] += pv;
+              w.h[j] = f32_to_bf16(pv);
+            }
+            b_p[2 * b + h] = __builtin_bit_cast(short8, w);
           }
-      }  // interior tiles: scores already scaled (q pre-scale) — no pass
-      float rm = kPNegInf;
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) rm = fmaxf(rm, s_acc[b][r]);
-      rm = fmaxf(rm, __shfl_xor(rm, 32, 64));
-      float alpha;
-      if (m_row > kPNegInf && __all(rm - m_row <= kDeferThr)) {
-        alpha = 1.f;  // defer-max: keep the old running max, skip rescale
-      } else {
-        const float m_new = fmaxf(m_row, rm);
-        if (m_new <= kPNegInf) {
-          alpha = 0.f;  // row has seen no unmasked score yet (o is 0)
-        } else {
-          alpha = (m_row <= kPNegInf) ? 0.f : __builtin_amdgcn_exp2f(m_row - m_new);
-          m_row = m_new;
-        }
-      }
-      float rs = 0.f;
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float pv = (m_row <= kPNegInf || s_acc[b][r] <= kPNegInf)
-                               ? 0.f
-                               : __builtin_amdgcn_exp2f(s_acc[b][r] - m_row);
-          s_acc[b][r] = pv;  // reuse as P (bounded by e^kDeferThr)
-          rs += pv;
-        }
-      rs += __shfl_xor(rs, 32, 64);
-      l_row = l_row * alpha + rs;
+        l_row += (rs[0] + rs[1]) + (rs[2] + rs[3]);
 
-      // rescale o: alpha is per-ROW (lane-local); o_acc rows follow the
-      // crow map, so gather the right alpha per reg via shfl
-      if (__any(alpha != 1.f)) {
+        // ---- O^T[D x q 32] += V^T[D x 64] P^T[64 x 32] ----
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float a_r = __shfl(alpha, crow(r, hi1), 64);
+        for (int kc = 0; kc < 4; ++kc)
 #pragma unroll
-          for (int cb = 0; cb < CB; ++cb) o_acc[cb][r] *= a_r;
-        }
+          for (int cb = 0; cb < CB; ++cb) {
+            const unsigned char* a = vbase + v_off[cb] + kc * 16 * kRowB;
+            const short4v lo = lds_read_tr4(a);
+            const short4v hi = lds_read_tr4(a + 8 * kRowB);
+            const short8 a_v = {lo[0], lo[1], lo[2], lo[3],
+                                hi[0], hi[1], hi[2], hi[3]};
+            o_acc[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                a_v, b_p[kc], o_acc[cb], 0, 0, 0);
+          }
+        __builtin_amdgcn_s_setprio(0);
       }
+      buf = buf1;
     }
 
-    if (compute) {
-      const char* vbase = reinterpret_cast<const char*>(vt_cur);
-      // ---- P -> A-fragments in-register (pack pairs + half swap) ----
-      // A-frag for kv chunk [32b + 16c, +16): lane needs kv {hi1*8..+8} of
-      // that range; own regs hold kv {..}+4*hi1 interleaved, the partner
-      // half-wave holds the other 4-run — one permlane32_swap per pair
-      // merges them (guide T12).
-      short8 a_p[4];
+    // ---- epilogue ----
+    l_row += half_swap(l_row);
+    const bool whole = !SPLIT || (ta == 0 && tb == t.work);
+    if (whole) {
+      if (active && row0 + col < t.seq_len) {
+        const float inv = l_row > 0.f ? 1.f / l_row : 0.f;
+        u16* orow = p.out + (static_cast<int64_t>(t.seq_start + row0 + col) *
+                                 p.num_q_heads + head) * D;
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
+        for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          const int base = 8 * c;
-          const u32 u1 = pack_bf16x2(s_acc[b][base + 0], s_acc[b][base + 1]);
-          const u32 u2 = pack_bf16x2(s_acc[b][base + 2], s_acc[b][base + 3]);
-          const u32 v1 = pack_bf16x2(s_acc[b][base + 4], s_acc[b][base + 5]);
-          const u32 v2 = pack_bf16x2(s_acc[b][base + 6], s_acc[b][base + 7]);
-          const auto s1 = __builtin_amdgcn_permlane32_swap(
-              static_cast<int>(u1), static_cast<int>(v1), false, false);
-          const auto s2 = __builtin_amdgcn_permlane32_swap(
-              static_cast<int>(u2), static_cast<int>(v2), false, false);
-          typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
-          u32x4 w;
-          w.x = static_cast<u32>(s1[0]);
-          w.y = static_cast<u32>(s2[0]);
-          w.z = static_cast<u32>(s1[1]);
-          w.w = static_cast<u32>(s2[1]);
-          a_p[2 * b + c] = __builtin_bit_cast(short8, w);
-        }
-
-      // ---- PV: O[32 q x D] += P[32 x 64] V[64 x D] ----
-      __builtin_amdgcn_s_setprio(1);
+          for (int r = 0; r < 16; r += 4) {
+            bf16x4 w;
 #pragma unroll
-      for (int kc = 0; kc < 4; ++kc) {   // 4 x 16-deep kv chunks
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb) {
-          const short8 b_v =
-              *reinterpret_cast<const short8*>(vbase + v_off[kc][cb]);
-          o_acc[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              a_p[kc], b_v, o_acc[cb], 0, 0, 0);
-        }
+            for (int j = 0; j < 4; ++j)
+              w.h[j] = f32_to_bf16(o_acc[cb][r + j] * inv);
+            *reinterpret_cast<bf16x4*>(orow + cb * 32 + crow(r, hi1)) = w;
+          }
       }
-      __builtin_amdgcn_s_setprio(0);
-    }
-    // stage K/V(t+1) (regs already resident) and prefetch (t+2)
-    if (FP8) {
-      if (t + 1 < num_kv_tiles) {
-        kwrite_fp8(kbuf_next);
-        vwrite(vt_next);
-        if (t + 2 < num_kv_tiles) {
-          kload_fp8(t + 2);
-          vload(t + 2);
-        }
-      }
-      // fp8: register-staged K, no glds in flight — plain barrier
-      __syncthreads();
     } else {
-      vwrite(vt_next);   // unconditional: garbage past the end, never read
-      vload(t + 2);      // clamped rows
-      // ONE raw barrier: publishes vt[(t+1)&1] (lgkmcnt) and drains
-      // K(t+1) (counted vmcnt) while K(t+2)+V(t+2) STAY IN FLIGHT
-      // across it — the whole point of the 3rd K buffer
-      tile_barrier();
-    }
-  }
-
-  // ---- epilogue: normalize (l gathered per crow row) and store ----
-  if (active) {
-    const float inv_own = (l_row > 0.f) ? 1.f / l_row : 0.f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int qr = row0 + crow(r, hi1);
-      if (qr >= seq_len) continue;
-      const float inv = __shfl(inv_own, crow(r, hi1), 64);
-      u16* orow = out + (static_cast<int64_t>(seq_start + qr) * num_q_heads +
-                         head) * D;
+      const int piece = slot * 2 + (ta > 0 ? 0 : 1);
+      float* o = p.piece_o + (static_cast<int64_t>(piece) * kWaves + wave) *
+                                 32 * D + lane;
 #pragma unroll
       for (int cb = 0; cb < CB; ++cb)
-        orow[cb * 32 + col] = f32_to_bf16(o_acc[cb][r] * inv);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[(cb * 16 + r) * 64] = o_acc[cb][r];
+      float2* ml = reinterpret_cast<float2*>(p.piece_ml) +
+                   (static_cast<int64_t>(piece) * kWaves + wave) * 64 + lane;
+      *ml = make_float2(m_row, l_row);
+    }
+    if (!SPLIT) return;
+    pos += tb - ta;
+    from = 0;
+    if (++qt == p.nq) { qt = 0; ++hg; }
+  }
+}
+
+// Adds up the pieces of the query tile that a part's end cuts, in the block
+// of the part in which the tile begins. blockIdx.y: 32 query vectors (a wave
+// of the attention kernel); a wave here takes eight accumulator registers of
+// every lane, of up to eight pieces at once so that their loads overlap.
+template <int D, bool PAGED>
+__global__ __launch_bounds__(D / 16 * kWaveSize)
+void prefill_attn_join_kernel(const PrefillArgs p) {
+  constexpr int kRegs = 8, kGroup = 8;
+  const int slot = blockIdx.x, qwave = blockIdx.y, kWaves = gridDim.y;
+  const int part = threadIdx.x / kWaveSize, lane = threadIdx.x % kWaveSize;
+  const int4 cut = p.cut[slot];
+  if (cut.y < 0) return;
+  const int hg = cut.x;
+  const QTile t = q_tile<PAGED>(p, cut.y);
+  const int wph = kWaves / p.hpb;
+  const int row0 = t.row0 + (qwave % wph) * 32;
+  if (row0 >= t.seq_len) return;
+  const float c = p.scale == 0.f
+      ? 1.f : fabsf(p.scale) * 1.4426950408889634f;
+
+  float m = kPNegInf, l = 0.f, o[kRegs];
+#pragma unroll
+  for (int r = 0; r < kRegs; ++r) o[r] = 0.f;
+  for (int s0 = slot; s0 < cut.z; s0 += kGroup) {
+    float2 ml[kGroup];
+    float x[kGroup][kRegs];
+#pragma unroll
+    for (int g = 0; g < kGroup; ++g) {
+      const int s = s0 + g;
+      const bool there = s < cut.z;  // otherwise the first again, weight 0
+      const int64_t piece =
+          static_cast<int64_t>(there ? s * 2 + (s == slot ? 1 : 0)
+                                     : slot * 2 + 1) * kWaves + qwave;
+      ml[g] = reinterpret_cast<const float2*>(p.piece_ml)[piece * 64 + lane];
+      if (!there) ml[g] = make_float2(kPNegInf, 0.f);
+      const float* src = p.piece_o + piece * 32 * D + part * kRegs * 64 + lane;
+#pragma unroll
+      for (int r = 0; r < kRegs; ++r) x[g][r] = src[r * 64];
+    }
+    float mx = m;
+#pragma unroll
+    for (int g = 0; g < kGroup; ++g) mx = fmaxf(mx, ml[g].x);
+    const float a = __builtin_amdgcn_exp2f((m - mx) * c);
+    m = mx;
+    l *= a;
+#pragma unroll
+    for (int r = 0; r < kRegs; ++r) o[r] *= a;
+#pragma unroll
+    for (int g = 0; g < kGroup; ++g) {
+      const float b = __builtin_amdgcn_exp2f((ml[g].x - mx) * c);
+      l += ml[g].y * b;
+#pragma unroll
+      for (int r = 0; r < kRegs; ++r) o[r] = fmaf(x[g][r], b, o[r]);
     }
   }
+  const int col = lane & 31, hi1 = lane >> 5;
+  if (row0 + col >= t.seq_len) return;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  u16* orow = p.out + (static_cast<int64_t>(t.seq_start + row0 + col) *
+                           p.num_q_heads + hg * p.hpb + qwave / wph) * D;
+#pragma unroll
+  for (int r = 0; r < kRegs; r += 4) {
+    bf16x4 w;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w.h[j] = f32_to_bf16(o[r + j] * inv);
+    const int reg = part * kRegs + r;  // of the tile kernel's accumulators
+    *reinterpret_cast<bf16x4*>(orow + reg / 16 * 32 + crow(reg % 16, hi1)) = w;
+  }
+}
+
+// Heads of a workgroup and query tiles of a launch, and whether to split.
+//
+// The host knows bounds: query tiles (nq), the longest K/V range and the
+// number of new rows. Whole query tiles take ceil(fill) rounds of the chip,
+// fill = workgroups / 256 (below one round a lone workgroup runs about 1.4
+// times as fast); the split form takes `fill` of them and about 35 us more
+// for its schedule, the pieces and the second launch, which is what 26 tiles
+// take. Where the new rows are most of the context, tiles differ in length
+// and longest-first already evens them out. Measured, whole / split in us:
+// 16 rows behind 2000: 47 / 33; 1024 behind 1024: 53 / 61; 1024 behind 8192:
+// 217 / 178; 4099 behind 16384: 1448 / 1250; 4096 behind 16384 (exactly two
+// rounds): 1190 / 1224; 2048 from the start: 57 / 100.
+PrefillPlan plan_prefill_attn(int ntiles, int tile_rows, int num_q_heads,
+                              int num_kv_heads, int new_rows, int max_k_len) {
+  const int group = num_q_heads / num_kv_heads;
+  auto layout = [&](bool split) {
+    PrefillPlan pl;
+    pl.split = split;
+    pl.waves = attn_waves(split);
+    pl.hpb = group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1);
+    pl.rows = pl.waves * 32 / pl.hpb;
+    pl.sub = ceil_div(tile_rows, pl.rows);
+    pl.nq = ntiles * pl.sub;
+    pl.slots = 0;
+    return pl;
+  };
+  PrefillPlan pl = layout(true);
+  const int64_t blocks = static_cast<int64_t>(pl.nq) *
+                         (num_q_heads / pl.hpb);
+  const int64_t tiles = ceil_div(max_k_len, kKVTile);
+  const double fill = blocks / 256.0;
+  const double idle = fill < 1.0 ? 1.0 - std::min(1.0, 1.4 * fill)
+                                 : std::ceil(fill) - 1.04 * fill;
+  if (2 * static_cast<int64_t>(new_rows) > max_k_len || idle * tiles <= 26)
+    return layout(false);
+  // parts of at least eight tiles, in whole rounds over the XCDs
+  pl.slots = static_cast<int>(std::min<int64_t>(
+      256, std::max<int64_t>(8, blocks * tiles / 8 / 8 * 8)));
+  return pl;
+}
+
+int64_t prefill_piece_floats(const PrefillPlan& pl, int head_dim) {
+  return static_cast<int64_t>(pl.slots) *
+         (2 * pl.waves * (32 * head_dim + kWaveSize * 2) + 4);
 }
 
 void launch_prefill_attn(u16* out, const u16* q, const void* k, const void* v,
                          const int* tile_seq, const int* tile_row0,
                          const int* cu_seqlens, const int* block_tables,
-                         const int* seq_lens_k, int max_blocks, int ntiles,
+                         const int* seq_lens_k, int max_blocks,
                          int64_t q_stride, int64_t k_stride, int64_t v_stride,
                          int num_q_heads, int num_kv_heads, int head_dim,
-                         float scale, bool fp8, int nw, hipStream_t stream) {
+                         float scale, bool fp8, const PrefillPlan& pl,
+                         float* pieces, hipStream_t stream) {
   const bool paged = block_tables != nullptr;
-  // nw = waves per workgroup (4 or 8), chosen per batch by the host
-  // (ops.prefill_tile_rows: 128-row tiles for long sequences); the tile
-  // table must have been built with rows == nw*32
-  dim3 grid(ntiles, num_q_heads), block(nw * kWaveSize);
+  PrefillArgs a;
+  a.out = out;
+  a.q = q;
+  a.k = k;
+  a.v = v;
+  a.tile_seq = tile_seq;
+  a.tile_row0 = tile_row0;
+  a.cu_seqlens = cu_seqlens;
+  a.block_tables = block_tables;
+  a.seq_lens_k = seq_lens_k;
+  a.piece_o = pieces;
+  a.piece_ml = pieces ? pieces + static_cast<int64_t>(pl.slots) * 2 *
+                                     pl.waves * 32 * head_dim
+                      : nullptr;
+  a.cut = reinterpret_cast<int4*>(
+      pieces ? a.piece_ml + static_cast<int64_t>(pl.slots) * 2 * pl.waves *
+                                kWaveSize * 2
+             : nullptr);
+  a.q_stride = q_stride;
+  a.k_stride = k_stride;
+  a.v_stride = v_stride;
+  a.max_blocks = max_blocks;
+  a.num_q_heads = num_q_heads;
+  a.num_kv_heads = num_kv_heads;
+  a.hpb = pl.hpb;
+  a.rows = pl.rows;
+  a.slots = pl.slots;
+  a.sub = pl.sub;
+  a.nq = pl.nq;
+  a.scale = scale;
+  const dim3 block(pl.waves * kWaveSize);
+  const dim3 grid(num_q_heads / pl.hpb * pl.nq);
 #define FI_PF_LAUNCH(DD, PP, F8)                                              \
   do {                                                                        \
-    if (nw == 4)                                                              \
-      hipLaunchKernelGGL((prefill_attn_kernel<DD, PP, F8, 2, 4>), grid,       \
-                         block, 0, stream, out, q, k, v, tile_seq,            \
-                         tile_row0, cu_seqlens, block_tables, seq_lens_k,     \
-                         max_blocks, q_stride, k_stride, v_stride,            \
-                         num_q_heads, num_kv_heads, scale);                   \
-    else                                                                      \
-      hipLaunchKernelGGL((prefill_attn_kernel<DD, PP, F8, 2, 8>), grid,       \
-                         block, 0, stream, out, q, k, v, tile_seq,            \
-                         tile_row0, cu_seqlens, block_tables, seq_lens_k,     \
-                         max_blocks, q_stride, k_stride, v_stride,            \
-                         num_q_heads, num_kv_heads, scale);                   \
+    if (pl.split) {                                                           \
+      hipLaunchKernelGGL((prefill_attn_kernel<DD, PP, F8, true>),             \
+                         dim3(pl.slots), block, 0, stream, a);                \
+      hipLaunchKernelGGL((prefill_attn_join_kernel<DD, PP>),                  \
+                         dim3(pl.slots, pl.waves),                            \
+                         dim3(DD / 16 * kWaveSize), 0, stream, a);            \
+    } else {                                                                  \
+      hipLaunchKernelGGL((prefill_attn_kernel<DD, PP, F8, false>), grid,      \
+                         block, 0, stream, a);                                \
+    }                                                                         \
   } while (0)
   if (fp8 && !paged) abort();  // fp8 KV is a cache format; dense is bf16
   if (head_dim == 128) {

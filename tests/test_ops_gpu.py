@@ -276,6 +276,63 @@ def test_prefill_attention_paged(ctx_lens, new_lens):
     assert_close_bf16(out.cpu(), expected, atol=3e-2, rtol=3e-2)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize(
+    "hq,hk,ctx_lens,new_lens,scale_by",
+    [
+        # whole row blocks: ends on, before and behind K/V tiles (64) and
+        # row blocks (128 / heads per workgroup), groups of 1, 2, 3, 8
+        (4, 4, [129, 64, 1], [129, 1, 1], 1.0),
+        (4, 2, [65, 200], [65, 63], -1.0),
+        (6, 2, [300], [257], 0.0),
+        (16, 2, [97, 31], [33, 31], 1.0),
+        # cut K/V ranges: one row, a row block and one row, several requests
+        # whose row blocks share parts, parts that end on a row block
+        (8, 2, [2100], [1], 1.0),
+        (8, 2, [4400, 2049], [65, 3], 1.0),
+        (3, 3, [3000, 40, 2500], [130, 40, 2], -1.0),
+        (16, 2, [2560, 2560], [64, 64], 1.0),
+    ],
+)
+def test_prefill_attention_row_blocks_and_parts(hq, hk, ctx_lens, new_lens,
+                                                scale_by, head_dim, fp8):
+    """Edges of row blocks, K/V tiles and equal parts against the fp32
+    reference. Bound: P and the output are rounded to bf16 (2^-9 each) and
+    |v| stays below 5, hence 2e-2."""
+    g = torch.Generator().manual_seed(11)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g).to(torch.bfloat16).to(DEV)
+
+    bs = 16
+    need = [(c + bs - 1) // bs for c in ctx_lens]
+    perm = (torch.randperm(sum(need), generator=g) + 1).int()
+    bt = torch.zeros(len(need), max(need), dtype=torch.int32)
+    for s, row in enumerate(perm.split(need)):
+        bt[s, :need[s]] = row
+    q = rnd(sum(new_lens), hq, head_dim)
+    k_cache = rnd(sum(need) + 1, hk, bs, head_dim)
+    v_cache = rnd(sum(need) + 1, hk, bs, head_dim)
+    if fp8:
+        k_cache, v_cache = _fp8_cache(k_cache), _fp8_cache(v_cache)
+    else:
+        # rows behind a context's end are never read
+        for s, c in enumerate(ctx_lens):
+            if c % bs:
+                v_cache[int(bt[s, need[s] - 1]), :, c % bs:] = float("nan")
+                k_cache[int(bt[s, need[s] - 1]), :, c % bs:] = float("nan")
+    cu = torch.tensor([0] + list(torch.tensor(new_lens).cumsum(0)),
+                      dtype=torch.int32)
+    lens = torch.tensor(ctx_lens, dtype=torch.int32)
+    scale = scale_by / math.sqrt(head_dim)
+    out = ops.prefill_attention_paged(q, k_cache, v_cache, bt.to(DEV),
+                                      cu.to(DEV), lens.to(DEV), scale)
+    want = ref.prefill_attention_paged(q.cpu(), k_cache.cpu(), v_cache.cpu(),
+                                       bt, cu, lens, scale)
+    assert_close_bf16(out.cpu(), want, atol=2e-2, rtol=2e-2)
+
+
 # ------------------------------------------------------------ fp8 KV cache
 
 def _fp8_cache(t):
