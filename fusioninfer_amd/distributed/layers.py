@@ -2,16 +2,17 @@
 
 Column-parallel shards the output dim (no comm on forward); row-parallel
 shards the input dim and all-reduces the partial outputs over RCCL/xGMI.
-GEMMs go through torch.nn.functional.linear (hipBLASLt) — plain library
-GEMMs; the fused hot ops are hand-written HIP (fusioninfer_amd/ops).
+GEMMs go through ops.linear: a streaming kernel for the few rows of a
+decode step, the library (hipBLASLt) for more; the fused hot ops are
+hand-written HIP (fusioninfer_amd/ops).
 """
 
 from __future__ import annotations
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
+import fusioninfer_amd.ops as ops
 from fusioninfer_amd.distributed import parallel_state as ps
 
 
@@ -39,7 +40,7 @@ class ColumnParallelLinear(nn.Module):
         self.weight = nn.Parameter(shard.contiguous(), requires_grad=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return F.linear(x, self.weight)
+        return ops.linear(x, self.weight)
 
 
 class MergedColumnParallelLinear(nn.Module):
@@ -76,7 +77,7 @@ class MergedColumnParallelLinear(nn.Module):
         )
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return F.linear(x, self.weight, self.bias)
+        return ops.linear(x, self.weight, self.bias)
 
 
 class RowParallelLinear(nn.Module):
@@ -93,13 +94,13 @@ class RowParallelLinear(nn.Module):
         self.weight = nn.Parameter(shard.contiguous(), requires_grad=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        out = F.linear(x, self.weight)
+        out = ops.linear(x, self.weight)
         return ps.tp_all_reduce(out)
 
     def forward_with_lora(self, x, lora, layer_idx, target):
         """LoRA delta added BEFORE the TP all-reduce (A is input-sharded,
         so per-rank deltas are partial sums)."""
-        out = F.linear(x, self.weight)
+        out = ops.linear(x, self.weight)
         if lora is not None:
             lora.apply(layer_idx, target, x, out)
         return ps.tp_all_reduce(out)
@@ -113,4 +114,4 @@ class ReplicatedLinear(nn.Module):
         )
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return F.linear(x, self.weight)
+        return ops.linear(x, self.weight)

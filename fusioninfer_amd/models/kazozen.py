@@ -27,7 +27,6 @@ from typing import Dict, Iterable, List, Optional, Tuple
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from fusioninfer_amd.config import ModelConfig
 from fusioninfer_amd.distributed import parallel_state as ps
@@ -38,7 +37,7 @@ from fusioninfer_amd.models.mixers import (
     WindowedSinkAttention,
     WindowedSinkAttentionConfig,
 )
-from fusioninfer_amd.ops import seqmix
+from fusioninfer_amd.ops import linear, seqmix
 
 ARCHITECTURE = "Kazozen"
 
@@ -277,7 +276,7 @@ class KazozenLM(nn.Module):
                                         self.final_norm_b, a.eps, self.dtype)
 
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
-        logits = F.linear(hidden, self.embed_tokens).float()
+        logits = linear(hidden, self.embed_tokens).float()
         if self.arch.logit_cap > 0:
             seqmix.tanh_cap_(logits, self.arch.logit_cap)
         return logits

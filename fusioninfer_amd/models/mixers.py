@@ -104,7 +104,7 @@ from fusioninfer_amd.distributed.layers import (
     ReplicatedLinear,
     RowParallelLinear,
 )
-from fusioninfer_amd.ops import seqmix
+from fusioninfer_amd.ops import linear, seqmix
 
 
 @dataclasses.dataclass
@@ -448,8 +448,8 @@ class TalkingWindowAttention(nn.Module):
             q, cache["k"], cache["v"], meta.seq_bt, meta.row_seq,
             meta.positions, c.scale, c.window, self.r1, self.r2, self.talk,
             c.heads, seq_cu=meta.seq_cu, tiles=meta.seq_tiles)
-        return F.linear(o.view(o.shape[0], c.heads * c.vdim),
-                        self.o_proj.weight, self.o_bias)
+        return linear(o.view(o.shape[0], c.heads * c.vdim),
+                      self.o_proj.weight, self.o_bias)
 
 
 class GatedDeltaMixer(nn.Module):
@@ -1637,8 +1637,8 @@ class NormedHeadAttention(nn.Module):
             qn, cache["k"], cache["v"], meta.seq_bt, meta.row_seq,
             meta.positions, c.scale, sink=self.sink, seq_cu=meta.seq_cu,
             tiles=meta.seq_tiles, window=c.window)
-        return F.linear(o.view(o.shape[0], c.heads * c.vdim),
-                        self.o_proj.weight, self.o_bias)
+        return linear(o.view(o.shape[0], c.heads * c.vdim),
+                      self.o_proj.weight, self.o_bias)
 
 
 class SelectiveScanMixer(nn.Module):

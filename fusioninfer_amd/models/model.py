@@ -1,7 +1,7 @@
 """Decoder-only transformer (Llama/Qwen3 family) on the FusionInfer-AMD ops.
 
 Every hot op is a hand-written CDNA4 HIP kernel (fusioninfer_amd/ops);
-GEMMs are hipBLASLt via F.linear. TP sharding is Megatron-style: heads
+GEMMs go through ops.linear. TP sharding is Megatron-style: heads
 sharded for attention, intermediate sharded for the MLP, one RCCL
 all-reduce after o_proj and one after down_proj per layer.
 
@@ -148,18 +148,17 @@ class MLP(nn.Module):
         self.inter_per_rank = cfg.intermediate_size // ps.tp_world_size()
 
     def forward(self, x, lora=None) -> torch.Tensor:
-        gu = self.gate_up_proj(x)
         if self.fp8:
             # fused SwiGLU + fp8 row quant straight into the fp8 down_proj
-            return self.down_proj(ops.silu_and_mul_fp8(gu))
+            return self.down_proj(ops.silu_and_mul_fp8(self.gate_up_proj(x)))
         if lora is not None:
+            gu = self.gate_up_proj(x)
             lora.apply(self.layer_idx, "gate_up", x, gu)
-        act = ops.silu_and_mul(gu)
-        if lora is not None:
             return self.down_proj.forward_with_lora(
-                act, lora, self.layer_idx, "down"
+                ops.silu_and_mul(gu), lora, self.layer_idx, "down"
             )
-        return self.down_proj(act)
+        return self.down_proj(
+            ops.linear_silu_mul(x, self.gate_up_proj.weight))
 
 
 class MoEMLP(nn.Module):

@@ -70,6 +70,58 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
     return ref.silu_and_mul(x)
 
 
+# ---------------------------------------------------------------- linear
+
+SKINNY_ROWS = 16  # rows of x up to which the streaming kernel serves a GEMM
+
+
+def _skinny_ok(x, w, unit: int) -> bool:
+    """Whether x W^T can run on the streaming kernel: few bf16 rows, whole
+    128-value stages of K, whole tiles of N, 16-byte aligned rows, nothing
+    to differentiate. A family that builds only its own extension keeps the
+    library's GEMM."""
+    return (
+        _C is not None and x.is_cuda and w.is_cuda and x.dim() == 2 and w.dim() == 2
+        and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+        and 1 <= x.shape[0] <= SKINNY_ROWS
+        and x.shape[1] == w.shape[1] and 0 < x.shape[1] <= 1 << 24
+        and x.shape[1] % 128 == 0
+        and 0 < w.shape[0] <= 1 << 24 and w.shape[0] % unit == 0
+        and x.stride(1) == 1 and x.stride(0) % 8 == 0
+        and x.stride(0) <= 1 << 24
+        and w.is_contiguous()
+        and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+        and not (torch.is_grad_enabled()
+                 and (x.requires_grad or w.requires_grad))
+    )
+
+
+def linear(x: torch.Tensor, w: torch.Tensor,
+           bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x W^T (+ bias): up to SKINNY_ROWS bf16 rows stream W once through the
+    skinny kernel (1.1 to 2 times the library's speed there, see its notes),
+    anything else is the library's GEMM."""
+    if _skinny_ok(x, w, 16) and (bias is None or (
+            bias.dtype == torch.bfloat16 and bias.is_contiguous()
+            and not (torch.is_grad_enabled() and bias.requires_grad))):
+        out = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype,
+                          device=x.device)
+        _C.skinny_gemm(out, x, w, bias, False)
+        return out
+    return torch.nn.functional.linear(x, w, bias)
+
+
+def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(x G^T) * (x U^T) with w = [G; U]; few rows in one kernel, whose
+    gate and up values are not rounded in between."""
+    if _skinny_ok(x, w, 32):
+        out = torch.empty((x.shape[0], w.shape[0] // 2), dtype=x.dtype,
+                          device=x.device)
+        _C.skinny_gemm(out, x, w, None, True)
+        return out
+    return silu_and_mul(linear(x, w))
+
+
 # ------------------------------------------------------- fp8 fused epilogues
 #
 # The fp8 serving mode quantizes activations per-token for torch._scaled_mm;

@@ -121,16 +121,30 @@ FI_DEV void unpack_fp8x4(u32 w, float out[4]) {
 // lds + 16 l. Base and LDS address are wave-uniform, the byte offset is per
 // lane. In asm because the compiler makes every LDS read wait for all DMAs
 // it knows of; whoever reads the data waits with s_waitcnt vmcnt (DMAs of a
-// wave complete in order) and, for other waves' data, a barrier.
+// wave complete in order) and, for other waves' data, a barrier. The wait
+// states are those of an m0 write and of a base that the vector unit wrote.
 FI_DEV void dma_to_lds16(u32 lds, const void* base, u32 offset) {
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile(
       "s_mov_b32 m0, %0\n\t"
-      "s_nop 0\n\t"
+      "s_nop 4\n\t"
       "global_load_lds_dwordx4 %1, %2"
       :
       : "s"(lds), "v"(offset), "s"(base)
       : "memory");  // m0: reserved, set in front of every use
+#endif
+}
+
+// the same for data that is read once: it leaves the caches first
+FI_DEV void dma_to_lds16_nt(u32 lds, const void* base, u32 offset) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 4\n\t"
+      "global_load_lds_dwordx4 %1, %2 nt"
+      :
+      : "s"(lds), "v"(offset), "s"(base)
+      : "memory");
 #endif
 }
 

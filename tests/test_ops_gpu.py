@@ -682,3 +682,60 @@ def test_moe_router_topk_matches_torch():
             etv = etv / etv.sum(-1, keepdim=True)
         assert torch.equal(ti.long(), eti), (T, E, k)
         torch.testing.assert_close(tv, etv, atol=2e-6, rtol=2e-6)
+
+
+# ------------------------------------------------------------ skinny GEMM
+
+
+@pytest.mark.parametrize("rows", [1, 3, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("n,k,bias", [
+    (16, 128, False),      # one tile, one stage: most waves hold nothing
+    (48, 384, True),       # fewer stages than waves
+    (4112, 1024, True),    # more tiles than workgroups, 16 rows each
+    (6144, 640, False),    # 32-row tiles, uneven split of K
+    (16448, 2048, True),   # 32-row tiles in several rounds
+])
+def test_skinny_linear(rows, n, k, bias):
+    """Few rows against a float64 product; one bf16 rounding of the result
+    (2^-9 relative) and fp32 sums of k products."""
+    g = torch.Generator().manual_seed(n + k + rows)
+    w = torch.randn(n, k, generator=g).to(torch.bfloat16).to(DEV)
+    b = torch.randn(n, generator=g).to(torch.bfloat16).to(DEV) if bias \
+        else None
+    # rows of a wider tensor, as a split projection hands out
+    x = torch.randn(rows, 2 * k, generator=g).to(torch.bfloat16).to(DEV)[:, k:]
+    assert ops._skinny_ok(x, w, 16)
+    out = ops.linear(x, w, b)
+    want = x.double() @ w.double().T + (0.0 if b is None else b.double())
+    err = (out.double() - want).abs()
+    assert (err <= want.abs() * 2 ** -8 + 1e-4 * k ** 0.5).all()
+    if n % 32 == 0 and not bias:
+        out = ops.linear_silu_mul(x, w)
+        prod = x.double() @ w.double().T
+        want = torch.nn.functional.silu(prod[:, : n // 2]) * prod[:, n // 2:]
+        err = (out.double() - want).abs()
+        assert (err <= want.abs() * 2 ** -8 + 1e-3 * k ** 0.5).all()
+
+
+def test_skinny_linear_leaves_other_calls_to_the_library():
+    """Row counts, types, strides and sizes that the kernel does not take
+    give what torch gives; gradients still flow."""
+    F = torch.nn.functional
+
+    def rnd(*shape, dtype=torch.bfloat16):
+        return torch.randn(*shape, device=DEV).to(dtype)
+
+    w = rnd(64, 256)
+    cases = [
+        (rnd(17, 256), w), (rnd(0, 256), w), (rnd(2, 3, 256), w),
+        (rnd(4, 256, dtype=torch.float32), w.float()),
+        (rnd(256, 4).T, w), (rnd(4, 264)[:, 4:260], w),
+        (rnd(4, 192), rnd(64, 192)), (rnd(4, 256), rnd(40, 256)),
+        (rnd(4, 256), rnd(256, 64).T),
+    ]
+    for x, m in cases:
+        assert not ops._skinny_ok(x, m, 16)
+        torch.testing.assert_close(ops.linear(x, m), F.linear(x, m))
+    x = rnd(4, 256).requires_grad_()
+    ops.linear(x, w).sum().backward()
+    assert x.grad is not None
