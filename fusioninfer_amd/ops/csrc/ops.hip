@@ -25,10 +25,11 @@ void launch_reshape_and_cache(const u16*, const u16*, void*, void*,
 template <bool GATHER>
 void launch_kv_block_copy(u16*, u16*, u16*, const int*, int, int64_t,
                           hipStream_t);
-void launch_paged_attn_decode(u16*, float*, float*, const u16*, const void*,
-                              const void*, const int*, const int*, int,
-                              int64_t, int, int, int, int, int, float, bool,
-                              hipStream_t);
+bool decode_attn_supported(int, int);
+int64_t decode_piece_floats(int, int, int, int);
+void launch_paged_attn_decode(u16*, const u16*, const void*, const void*,
+                              const int*, const int*, int, int64_t, int, int,
+                              int, int, float, bool, float*, hipStream_t);
 PrefillPlan plan_prefill_attn(int, int, int, int, int, int);
 int64_t prefill_piece_floats(const PrefillPlan&, int);
 void launch_prefill_attn(u16*, const u16*, const void*, const void*,
@@ -237,16 +238,14 @@ void scatter_kv_blocks(at::Tensor staging, at::Tensor k_cache,
 
 void paged_attention_decode(at::Tensor out, at::Tensor q, at::Tensor k_cache,
                             at::Tensor v_cache, at::Tensor block_tables,
-                            at::Tensor seq_lens,
-                            c10::optional<at::Tensor> ml_ws,
-                            c10::optional<at::Tensor> acc_ws,
-                            int64_t num_parts, double scale) {
+                            at::Tensor seq_lens, double scale) {
   CHECK_BF16_CUDA(out);
   CHECK_BF16_CUDA(q);
   const bool fp8 = cache_is_fp8(k_cache);
   TORCH_CHECK(block_tables.scalar_type() == at::kInt &&
               block_tables.is_contiguous());
   TORCH_CHECK(seq_lens.scalar_type() == at::kInt);
+  seq_lens = seq_lens.contiguous();
   TORCH_CHECK(q.dim() == 3);  // [S, Hq, D], rows may be strided
   const int num_seqs = q.size(0);
   const int num_heads = q.size(1);
@@ -254,20 +253,25 @@ void paged_attention_decode(at::Tensor out, at::Tensor q, at::Tensor k_cache,
   const int num_kv_heads = k_cache.size(1);
   TORCH_CHECK(k_cache.size(2) == 16, "cache block_size must be 16");
   TORCH_CHECK(q.stride(2) == 1 && q.stride(1) == head_dim);
-  float* ml = nullptr;
-  float* acc = nullptr;
-  if (num_parts > 1) {
-    TORCH_CHECK(ml_ws && acc_ws, "workspace required when num_parts > 1");
-    ml = ml_ws->data_ptr<float>();
-    acc = acc_ws->data_ptr<float>();
-  }
+  TORCH_CHECK(fi::decode_attn_supported(head_dim, num_heads / num_kv_heads) &&
+                  num_heads % num_kv_heads == 0,
+              "decode attention takes head sizes 64 and 128 and 1, 2, 4 or 8 "
+              "query heads per K/V head");
+  if (num_seqs == 0) return;
+  // query rows are copied in 16-byte pieces
+  if (q.stride(0) % 8 != 0 ||
+      reinterpret_cast<uintptr_t>(q.data_ptr()) % 16 != 0)
+    q = q.clone(at::MemoryFormat::Contiguous);
+  at::Tensor pieces = at::empty(
+      {fi::decode_piece_floats(num_seqs, num_kv_heads, head_dim,
+                               num_heads / num_kv_heads)},
+      q.options().dtype(at::kFloat));
   fi::launch_paged_attn_decode(
-      bf16_ptr(out), ml, acc, bf16_cptr(q), k_cache.data_ptr(),
-      v_cache.data_ptr(), block_tables.data_ptr<int>(),
-      seq_lens.data_ptr<int>(), num_seqs, q.stride(0), block_tables.size(1),
-      num_kv_heads, head_dim, num_heads / num_kv_heads,
-      static_cast<int>(num_parts), static_cast<float>(scale), fp8,
-      current_stream());
+      bf16_ptr(out), bf16_cptr(q), k_cache.data_ptr(), v_cache.data_ptr(),
+      block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(), num_seqs,
+      q.stride(0), block_tables.size(1), num_kv_heads, head_dim,
+      num_heads / num_kv_heads, static_cast<float>(scale), fp8,
+      pieces.data_ptr<float>(), current_stream());
 }
 
 // room for the pieces of cut query tiles

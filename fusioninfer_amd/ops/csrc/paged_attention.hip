@@ -1,24 +1,33 @@
-// Paged-attention DECODE kernels for CDNA4 (gfx950) — v2 (flash-decoding).
+// Paged-attention DECODE for CDNA4 (gfx950): one query row per sequence
+// against the paged KV cache ([num_blocks, Hk, 16, D], bf16 or e4m3).
+// Memory-bound: every sequence's K and V are read once, each read serves the
+// G query heads of a K/V head.
 //
-// One-token attention per sequence against the paged KV cache
-// ([num_blocks, Hk, 16, D] bf16). Memory-bound: stream each sequence's K/V
-// once at near-HBM rate, reusing every K/V read across the GQA group
-// (G q-heads per kv-head).
+// All (sequence, K/V head) contexts form one line of steps (16 * PP tokens);
+// up to 1024 waves, four per CU, take equal parts of it, so ragged and few
+// long contexts load the chip as evenly as many equal ones, and the launch
+// shape does not depend on the lengths (hipGraph replay). A wave streams its
+// part through a private ring in LDS by DMA, three steps ahead: 96 KB in
+// flight per CU, no barrier anywhere. The next context's queries arrive
+// through the same queue, so the ring runs on over the borders of contexts.
+// A context that is cut leaves unnormalised fp32 pieces; a second kernel
+// adds them up.
 //
-// Grid: (num_seqs, num_kv_heads, num_partitions) — the context is split
-// into 512-token partitions (flash-decoding) so small decode batches still
-// fill 256 CUs; partial (m, l, acc) go to an fp32 workspace and a second
-// kernel merges partitions. num_partitions == 1 writes output directly.
+// Per step, with heads as MFMA columns (16, of which G count):
+//   S[token, head] = K Q^T            mfma 16x16x32, A = K rows from LDS
+//   O^T[dim, head] += V^T P^T         A = V through the transposing LDS
+//                                     read, B = P as the scores' registers
+//                                     already hold it (the order of the
+//                                     tokens within a step is theirs)
+// A lane keeps one head's statistics; e4m3 rows are converted exactly after
+// the LDS read. 96 KB in flight and a few hundred cycles of work per 8 KB
+// step leave memory as the only bound.
 //
-// Within a workgroup: 4 waves process interleaved 16-token chunks (1 chunk
-// == 1 cache block, so a chunk's K/V are contiguous). Per chunk:
-//   phase A (scores): lane = token*4 + i, lane reads K[token][i*32 .. +32]
-//     as 4x bf16x8 (64 B); dot with q (fp32 in LDS, read as float4 =
-//     ds_read_b128); 2-level shfl_xor reduce; online-softmax state (m, l
-//     per G) wave-uniform in registers; probs parked in per-wave LDS.
-//   phase B (PV): lane = dim pair, per-token V rows read 256 B coalesced;
-//     fp32 accumulator acc[G][2] per lane.
-// Cross-wave flash-merge through LDS ends the workgroup.
+// Measured at 32 query heads, D 128, both kernels, us (TB/s of K/V), before
+// -> now: 256 contexts of 1024-1279 tokens, 8 K/V heads 278 (4.3) -> 207
+// (5.8); 6 of 20-32 thousand 168 (3.9) -> 109 (6.0); 13 of 70-4100 42 -> 25;
+// 64 of 512-2048 e4m3 101 (1.6) -> 34 (4.7), with 4 K/V heads bf16 58 (2.7)
+// -> 35 (4.6); one of 301 12.0 -> 10.1, one of 8000 19.5 -> 15.0.
 //
 // Capability parity: the paged-attention decode the reference delegates to
 // its vLLM containers (SURVEY.md §2.3 "Paged-attention decode kernel").
@@ -29,545 +38,627 @@
 
 namespace fi {
 
-constexpr int kBlockSz = 16;     // cache block size (tokens)
-constexpr int kPartChunks = 32;  // 512 tokens per partition
-constexpr float kNegInf = -1e30f;
+namespace {
 
-// kNWaves is a launch-time choice: 8 waves when the grid underfills the
-// chip (small decode batches: measured +46% at batch<=8), 4 when it is
-// full (4-wave measured ~5% faster there).
-// FP8: the cache holds OCP e4m3 at scale 1.0 — half the KV bytes of bf16
-// (this kernel is KV-bandwidth-bound); v_cvt_pk_f32_fp8 dequant on load.
-// HS (head split): waves are partitioned into HS head-groups of G/HS
-// heads each; a wave streams chunks at stride kNWaves/HS for ITS head
-// slice only. G=8 runs HS=2 so the per-wave state is the G=4 footprint —
-// the monolithic G=8 variant spilled ~500 B/lane (W=8) or sat at
-// occupancy 1 (W=4).
+typedef __attribute__((ext_vector_type(4))) short short4v;
 typedef __attribute__((ext_vector_type(8))) short short8;
 typedef __attribute__((ext_vector_type(4))) float floatx4;
 
-// MFA (bf16 only): phase A runs QK^T on the MATRIX CORES instead of
-// per-lane FMAs + 6-7-deep shfl_xor reduction chains (PMC showed the
-// old phase A WAIT-dominant on those serial permlanes). One
-// mfma_f32_16x16x32_bf16 per 32-dim slice: A = Q fragment with the G2
-// head rows REPLICATED over all 16 rows (so every 16-lane col group
-// holds a full copy of the scores and the softmax reductions are
-// 4-deep within a group, wave-uniform by construction — alpha needs no
-// broadcast), B = K fragment (lane reads K[tok=l&15][(l>>4)*8..+8]:
-// same bytes as the scalar path, different pattern, block stays
-// L2-resident). The K-dim reduction happens INSIDE the MFMA.
-template <int D, int G, int kNWaves, bool FP8, int HS = 1,
-          bool MFA = false>
-__global__ __launch_bounds__(kNWaves * kWaveSize) void paged_attn_decode_kernel(
-    u16* __restrict__ out,            // [S, Hq, D] (written when 1 partition)
-    float* __restrict__ ml_ws,        // [S, Hq, P, 2] (multi-partition)
-    float* __restrict__ acc_ws,       // [S, Hq, P, D]
-    const u16* __restrict__ q,        // [S] rows, stride q_stride, Hq*D elems
-    const void* __restrict__ k_cache_p,  // [B, Hk, 16, D] bf16 (FP8: e4m3)
-    const void* __restrict__ v_cache_p,
-    const int* __restrict__ block_tables,  // [S, max_blocks]
-    const int* __restrict__ seq_lens,      // [S]
-    const int64_t q_stride, const int max_blocks, const int num_kv_heads,
-    const float scale) {
-  using CT = typename std::conditional<FP8, unsigned char, u16>::type;
-  const CT* k_cache = static_cast<const CT*>(k_cache_p);
-  const CT* v_cache = static_cast<const CT*>(v_cache_p);
-  const int seq = blockIdx.x;
-  const int kv_head = blockIdx.y;
-  const int part = blockIdx.z;
-  const int num_parts = gridDim.z;
-  const int tid = threadIdx.x;
-  const int wave = tid / kWaveSize;
-  const int lane = tid % kWaveSize;
-  // head-split decomposition: wave = cwave * HSE + hsplit
-  // (HSE clamps HS to G so dead template branches in the launcher's
-  // runtime dispatch still compile — e.g. G=1 never runs with HS=2)
-  constexpr int HSE = (HS > G) ? 1 : HS;
-  constexpr int G2 = G / HSE;         // heads this wave carries
-  constexpr int kCWaves = kNWaves / HSE;  // waves streaming chunks together
-  const int hsplit = wave % HSE;
-  const int cwave = wave / HSE;
+constexpr int kPage = 16;        // tokens of a cache block
+constexpr int kDecWaves = 4;     // waves of a workgroup
+constexpr int kDecSlots = 1024;  // parts of the line
+constexpr int kRing = 4;         // steps of a wave's ring
+constexpr int kMaxGroup = 8;
+constexpr int kMinPages = 4;     // a part is no shorter than this
+constexpr float kNegInf = -1e30f;
+// see the prefill kernel: rescale only when the maximum grows by more than
+// this (base-2 units)
+constexpr float kDeferThr = 11.5416f;
 
-  const int ctx = seq_lens[seq];
-  const int num_chunks = (ctx + kBlockSz - 1) / kBlockSz;
-  const int chunk_lo = part * kPartChunks;
-  const int chunk_hi = min(num_chunks, chunk_lo + kPartChunks);
-  const int num_heads = num_kv_heads * G;
+struct DecodeArgs {
+  u16* out;                 // [S, Hq, D]
+  const u16* q;             // [S] rows, stride q_stride, Hq * D values
+  const unsigned char* k;   // cache bytes
+  const unsigned char* v;
+  const int* block_tables;  // [S, max_blocks]
+  const int* seq_lens;      // [S]
+  float* piece_o;           // [slots][2][G][D]
+  float* piece_ml;          // [slots][2][G][2]
+  int2* cut;                // [S][Hk] parts [first, behind) of a cut
+                            // context; first -1: it was not cut
+  int64_t q_stride;
+  int num_seqs, max_blocks, num_kv_heads, group;
+  float scale;
+};
 
-  // empty partition: publish "nothing" and leave
-  if (chunk_lo >= num_chunks) {
-    if (tid < G) {
-      const int h = kv_head * G + tid;
-      float* ml = ml_ws + ((static_cast<int64_t>(seq) * num_heads + h) *
-                               num_parts + part) * 2;
-      ml[0] = kNegInf;
-      ml[1] = 0.f;
+template <int PP>
+FI_DEV int steps_of(int ctx) {
+  return (max(ctx, 1) + kPage * PP - 1) / (kPage * PP);
+}
+
+struct Place {
+  int seq, head, step;
+};
+
+// The line: sequences in order, of each its K/V heads, of each its steps.
+// The first 64 sequences' steps and their running sum stay in the lanes.
+template <int PP>
+struct Line {
+  int n, incl, lane;
+  int64_t total;  // steps of all
+
+  FI_DEV void chunk(const DecodeArgs& p, int i0, int* n_, int* incl_) const {
+    const int i = i0 + lane;
+    int x = i < p.num_seqs ? steps_of<PP>(p.seq_lens[i]) : 0;
+    *n_ = x;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int o = __shfl_up(x, off, 64);
+      if (lane >= off) x += o;
     }
-    return;
+    *incl_ = x;
   }
 
-  __shared__ float q_lds[MFA ? 1 : G][MFA ? 1 : D];
-  __shared__ float p_lds[kNWaves][kBlockSz][G2];
-  __shared__ float merge_m[kNWaves][G2];
-  __shared__ float merge_l[kNWaves][G2];
-  __shared__ float merge_acc[kNWaves][G2][D];
-
-  // MFA: per-wave replicated-row Q fragments, built once (Q is fixed
-  // for the whole kernel). Row i of A carries head i % G2, pre-scaled
-  // by scale*log2e and re-rounded to bf16 (same trick as the prefill
-  // kernel's pre-scaled Q).
-  short8 av_q[(MFA && !FP8) ? D / 32 : 1];
-  long long av8_q[(MFA && FP8) ? D / 32 : 1];
-  __shared__ float qsc_lds[(MFA && FP8) ? G : 1];
-  float qsc_r[G2];  // fp8 MFA: per-head dequant*softmax scalar
-  if constexpr (MFA && !FP8) {
-    const u16* q_row = q + seq * q_stride +
-                       static_cast<int64_t>(kv_head) * G * D;
-    const int head = hsplit * G2 + ((lane & 15) % G2);
+  FI_DEV Line(const DecodeArgs& p, int lane_) : lane(lane_) {
+    chunk(p, 0, &n, &incl);
+    int sum = 0;
+#pragma unroll 4
+    for (int i = kWaveSize + lane; i < p.num_seqs; i += kWaveSize)
+      sum += steps_of<PP>(p.seq_lens[i]);
+    if (p.num_seqs > kWaveSize) {
 #pragma unroll
-    for (int kk = 0; kk < D / 32; ++kk) {
-      const int d0 = kk * 32 + (lane >> 4) * 8;
-      u16 tmp[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        tmp[e] = f32_to_bf16(bf16_to_f32(q_row[head * D + d0 + e]) *
-                             scale * 1.4426950408889634f);
-      av_q[kk] = *reinterpret_cast<short8*>(tmp);
+      for (int off = 32; off; off >>= 1) sum += __shfl_xor(sum, off, 64);
     }
-  } else if constexpr (MFA && FP8) {
-    // Q quantized to e4m3 per HEAD; the dequant scale folds into the
-    // post-MFMA per-head scalar together with scale*log2e (the model
-    // already folded the cache's k_scale into `scale`)
-    const u16* q_row = q + seq * q_stride +
-                       static_cast<int64_t>(kv_head) * G * D;
-    if (tid < G) {
-      float mx = 1e-8f;
-      for (int d = 0; d < D; ++d)
-        mx = fmaxf(mx, fabsf(bf16_to_f32(q_row[tid * D + d])));
-      qsc_lds[tid] = mx / 448.f;
-    }
-    __syncthreads();
-    const int head = hsplit * G2 + ((lane & 15) % G2);
-    const float inv_qs = 1.f / qsc_lds[head];
-#pragma unroll
-    for (int kk = 0; kk < D / 32; ++kk) {
-      const int d0 = kk * 32 + (lane >> 4) * 8;
-      float f[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        f[e] = bf16_to_f32(q_row[head * D + d0 + e]) * inv_qs;
-      u32 w[2];
-      pack_fp8x8(f, w);
-      av8_q[kk] = static_cast<long long>(
-          (static_cast<unsigned long long>(w[1]) << 32) | w[0]);
-    }
-#pragma unroll
-    for (int g = 0; g < G2; ++g)
-      qsc_r[g] = qsc_lds[hsplit * G2 + g] * scale * 1.4426950408889634f;
-  } else {
-    // stage q (G heads) into LDS as fp32 (pre-scaled)
-    const u16* q_row = q + seq * q_stride +
-                       static_cast<int64_t>(kv_head) * G * D;
-    for (int e = tid; e < G * D; e += kNWaves * kWaveSize)
-      // scale*log2e: scores land in base-2 units so the softmax
-      // uses bare v_exp_f32 (exp2) with no argument multiply
-      q_lds[e / D][e % D] =
-          bf16_to_f32(q_row[e]) * scale * 1.4426950408889634f;
-    __syncthreads();
+    total = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(
+                sum + __shfl(incl, 63, 64))) * p.num_kv_heads;
   }
 
-  // online-softmax state, wave-uniform (every lane holds the same copy)
-  float m[G2], l[G2], acc[G2][2];
-#pragma unroll
-  for (int g = 0; g < G2; ++g) {
-    m[g] = kNegInf;
-    l[g] = 0.f;
-    acc[g][0] = acc[g][1] = 0.f;
-  }
-
-  const int tok = lane / 4;          // phase-A token within chunk
-  const int quad = lane % 4;         // phase-A dim quarter
-  constexpr int DPQ = D / 4;         // dims per phase-A lane
-  constexpr int KQ4 = DPQ * sizeof(CT) / 16;  // 16-B K loads per lane per chunk
-
-  // software-prefetch: this wave's NEXT chunk's K flies while the current
-  // chunk's softmax + PV run (the phases were serialized on K latency)
-  auto kv_base_of = [&](int chunk) -> int64_t {
-    const int block_id = block_tables[seq * max_blocks + chunk];
-    return ((static_cast<int64_t>(block_id) * num_kv_heads + kv_head) *
-            kBlockSz) * D;
-  };
-  uint4 kraw[KQ4];
-  auto load_k = [&](int64_t kv_base, uint4* dst) {
-    if constexpr (MFA && FP8) {
-      // fp8 B-fragment: 8 e4m3 bytes per lane per 32-dim slice
-      const CT* k_row = k_cache + kv_base + (lane & 15) * D;
-#pragma unroll
-      for (int kk = 0; kk < D / 32; ++kk)
-        reinterpret_cast<unsigned long long*>(dst)[kk] =
-            *reinterpret_cast<const unsigned long long*>(
-                k_row + kk * 32 + (lane >> 4) * 8);
-    } else if constexpr (MFA) {
-      // B-fragment pattern: lane supplies K[tok = l&15][(l>>4)*8 + e]
-      const CT* k_row = k_cache + kv_base + (lane & 15) * D;
-#pragma unroll
-      for (int kk = 0; kk < KQ4; ++kk)
-        dst[kk] = *reinterpret_cast<const uint4*>(
-            k_row + kk * 32 + (lane >> 4) * 8);
-    } else {
-      const CT* k_row = k_cache + kv_base + tok * D + quad * DPQ;
-#pragma unroll
-      for (int j8 = 0; j8 < KQ4; ++j8)
-        dst[j8] = reinterpret_cast<const uint4*>(k_row)[j8];
-    }
-  };
-  int64_t kv_base = 0;
-  if (chunk_lo + cwave < chunk_hi) {
-    kv_base = kv_base_of(chunk_lo + cwave);
-    load_k(kv_base, kraw);
-  }
-
-  for (int chunk = chunk_lo + cwave; chunk < chunk_hi; chunk += kCWaves) {
-    const int token_pos = chunk * kBlockSz + tok;
-    const int64_t kv_base_cur = kv_base;
-
-    // ---- phase A: scores for 16 tokens x G2 heads ----
-    // streaming convert+FMA: per 16-B K group, convert 8 elements and
-    // fold them into all G2 head accumulators immediately — kf[8] live
-    // instead of kf[32] (round-2 register diet: the G=4/D=128 variant
-    // was 218 VGPR -> 2 waves/SIMD; PMC showed WAIT-dominant)
-    float s[G2];
-#pragma unroll
-    for (int g = 0; g < G2; ++g) s[g] = 0.f;
-    if constexpr (MFA) {
-      // QK^T on the matrix cores: K-dim reduction inside the MFMA, no
-      // cross-lane score reduction needed. c[row=g][col=lane&15].
-      floatx4 c = {0.f, 0.f, 0.f, 0.f};
-      if constexpr (FP8) {
-#pragma unroll
-        for (int kk = 0; kk < D / 32; ++kk)
-          c = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
-              av8_q[kk],
-              static_cast<long long>(
-                  reinterpret_cast<const unsigned long long*>(kraw)[kk]),
-              c, 0, 0, 0);
-#pragma unroll
-        for (int g = 0; g < G2; ++g) s[g] = c[g] * qsc_r[g];
-      } else {
-#pragma unroll
-        for (int kk = 0; kk < KQ4; ++kk)
-          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              av_q[kk], __builtin_bit_cast(short8, kraw[kk]), c, 0, 0, 0);
-#pragma unroll
-        for (int g = 0; g < G2; ++g) s[g] = c[g];
+  FI_DEV Place find(const DecodeArgs& p, int64_t at) const {
+    const int hk = p.num_kv_heads;
+    int64_t before = 0;
+    int cn = n, ci = incl;
+    for (int i0 = 0;;) {
+      const unsigned long long hit =
+          __ballot(before + static_cast<int64_t>(ci) * hk > at);
+      if (hit) {
+        const int l = __builtin_ctzll(hit);
+        const int nl = __builtin_amdgcn_readfirstlane(__shfl(cn, l, 64));
+        const int in =
+            static_cast<int>(at - before) -
+            (__builtin_amdgcn_readfirstlane(__shfl(ci, l, 64)) - nl) * hk;
+        return {i0 + l, in / nl, in % nl};
       }
+      before += static_cast<int64_t>(
+          __builtin_amdgcn_readfirstlane(__shfl(ci, 63, 64))) * hk;
+      i0 += kWaveSize;
+      if (i0 >= p.num_seqs) return {p.num_seqs - 1, hk - 1, 0};  // not reached
+      chunk(p, i0, &cn, &ci);
+    }
+  }
+};
+
+// part s of the line is [begin(s), begin(s + 1))
+struct Parts {
+  int64_t each, total;
+  FI_DEV Parts(int64_t t, int min_each)
+      : each(max((t + kDecSlots - 1) / kDecSlots,
+                 static_cast<int64_t>(min_each))),
+        total(t) {}
+  FI_DEV int64_t begin(int s) const { return min(s * each, total); }
+};
+
+// value of the lane with the other 16 (32) bit
+FI_DEV float swap16(float x) {
+  const auto s = __builtin_amdgcn_permlane16_swap(
+      __float_as_int(x), __float_as_int(x), false, false);
+  return __int_as_float((threadIdx.x & 16) ? s[0] : s[1]);
+}
+FI_DEV float swap32(float x) {
+  const auto s = __builtin_amdgcn_permlane32_swap(
+      __float_as_int(x), __float_as_int(x), false, false);
+  return __int_as_float((threadIdx.x & 32) ? s[0] : s[1]);
+}
+
+// eight e4m3 bytes to bf16, exact
+FI_DEV short8 fp8_to_bf16(uint2 w) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf2;
+  typedef __attribute__((ext_vector_type(4))) u32 u4;
+  u4 o;
+  o.x = __builtin_bit_cast(
+      u32, bf2(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w.x, 1.f, false)));
+  o.y = __builtin_bit_cast(
+      u32, bf2(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w.x, 1.f, true)));
+  o.z = __builtin_bit_cast(
+      u32, bf2(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w.y, 1.f, false)));
+  o.w = __builtin_bit_cast(
+      u32, bf2(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w.y, 1.f, true)));
+  return __builtin_bit_cast(short8, o);
+#else
+  return short8{};
+#endif
+}
+
+// Transposing LDS read of bytes: within 16 lanes, lane 2i+j points at
+// entries 8j..8j+7 of row i of an 8 x 16 block and receives the eight rows'
+// entries of column (lane & 15).
+FI_DEV uint2 lds_read_tr8(const unsigned char* p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef __attribute__((ext_vector_type(2))) int i2;
+  const i2 r = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+      (__attribute__((address_space(3))) i2*)(p));
+  return make_uint2(r.x, r.y);
+#else
+  return make_uint2(0, 0);
+#endif
+}
+
+template <int D, bool FP8>
+struct DecShape {
+  static constexpr int kRowB = D * (FP8 ? 1 : 2);
+  // pages of a step: 8 KB of K and V together (4 KB for the smallest rows)
+  static constexpr int PP = kRowB == 256 ? 1 : 2;
+};
+
+template <int D, bool FP8>
+__global__ __launch_bounds__(kDecWaves * kWaveSize)
+void paged_attn_decode_kernel(const DecodeArgs p) {
+  constexpr int kRowB = DecShape<D, FP8>::kRowB, PP = DecShape<D, FP8>::PP;
+  constexpr int KK = D / 32, DT = D / 16;
+  constexpr int kChunk = kRowB / 16;           // 16-byte chunks of a row
+  constexpr int kRowsDma = 1024 / kRowB;       // rows of a DMA
+  constexpr int kPageDma = kPage / kRowsDma;   // DMAs of a page
+  constexpr int kMatB = PP * kPage * kRowB;    // K (or V) bytes of a step
+  constexpr int kLoads = 2 * PP * kPageDma;    // DMAs of a step
+  constexpr int kQB = kMaxGroup * D * 2;       // a context's queries
+  constexpr int kWaveB = kRing * (2 * kMatB + kQB);
+  static_assert(kDecWaves * kWaveB <= 160 * 1024, "LDS");
+  __shared__ __attribute__((aligned(1024)))
+  unsigned char smem[kDecWaves * kWaveB];
+
+  const int lane = threadIdx.x % kWaveSize;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+  const int slot = blockIdx.x * kDecWaves + wave;
+  unsigned char* ring = smem + wave * kWaveB;
+  unsigned char* qring = ring + kRing * 2 * kMatB;
+  const u32 ring_lds = static_cast<u32>(reinterpret_cast<uintptr_t>(
+      (__attribute__((address_space(3))) unsigned char*)ring));
+  const u32 q_lds = ring_lds + kRing * 2 * kMatB;
+  const int G = p.group, hk = p.num_kv_heads;
+
+  const Line<PP> line(p, lane);
+  const Parts parts(line.total, kMinPages / PP);
+  const int64_t lo = parts.begin(slot), hi = parts.begin(slot + 1);
+  if (lo >= hi) return;
+
+  // ---- producer ----
+  auto k_swz = [](int row) {
+    return kRowB == 256 ? row & 15
+                        : (kRowB == 128 ? (row >> 1) & 7 : (row >> 2) & 3);
+  };
+  auto v_swz = [](int row) {
+    return FP8 ? (kRowB == 128 ? (row >> 1) & 7 : (row >> 2) & 3)
+               : (kRowB == 256 ? (row & 7) << 1 : ((row >> 1) & 3) << 1);
+  };
+  const ConstInts lens = const_ints(p.seq_lens);
+  const ConstInts tables = const_ints(p.block_tables);
+  const Place first = line.find(p, lo);
+  const int total = static_cast<int>(hi - lo);
+  struct Cursor {
+    int seq, head, step, ctx, steps;
+  };
+  auto at_seq = [&](int seq, int head, int step) {
+    Cursor c;
+    c.seq = __builtin_amdgcn_readfirstlane(seq);
+    c.head = __builtin_amdgcn_readfirstlane(head);
+    c.step = __builtin_amdgcn_readfirstlane(step);
+    c.ctx = max(lens[c.seq], 1);
+    c.steps = steps_of<PP>(c.ctx);
+    return c;
+  };
+  auto next_context = [&](const Cursor& c) {
+    if (c.head + 1 < hk) {
+      Cursor n = c;
+      n.head = c.head + 1;
+      n.step = 0;
+      return n;
+    }
+    return at_seq(c.seq + 1, 0, 0);
+  };
+  Cursor in = at_seq(first.seq, first.head, first.step);
+  int page[PP], in_slot = 0, in_q = 0, issued = 0;
+  auto load_pages = [&] {
+#pragma unroll
+    for (int i = 0; i < PP; ++i)
+      page[i] = tables[static_cast<int64_t>(in.seq) * p.max_blocks +
+                       min(in.step * PP + i, (in.ctx - 1) / kPage)];
+  };
+  auto request_q = [&] {
+    const u16* src = p.q + in.seq * p.q_stride +
+                     static_cast<int64_t>(in.head) * G * D;
+    for (int b = 0; b < G * D * 2; b += 1024)
+      dma_to_lds16(q_lds + in_q * kQB + b, src,
+                   min(b + lane * 16, G * D * 2 - 16));
+  };
+  auto request = [&] {
+    const u32 dst = ring_lds + in_slot * 2 * kMatB;
+#pragma unroll
+    for (int i = 0; i < PP; ++i) {
+      const int64_t base =
+          (static_cast<int64_t>(page[i]) * hk + in.head) * (kPage * kRowB);
+      // rows behind the context's end repeat its last one (finite values,
+      // masked scores)
+      const int limit =
+          in.ctx - 1 - min(in.step * PP + i, (in.ctx - 1) / kPage) * kPage;
+#pragma unroll
+      for (int j = 0; j < kPageDma; ++j) {
+        const int r = j * kRowsDma + lane / kChunk;  // of the page
+        const int sr = i * kPage + r;                // of the step
+        const u32 row = min(r, limit) * kRowB;
+        const u32 at = (i * kPage + j * kRowsDma) * kRowB;
+        dma_to_lds16_nt(dst + at, p.k + base,
+                        row + ((lane % kChunk) ^ k_swz(sr)) * 16);
+        dma_to_lds16_nt(dst + kMatB + at, p.v + base,
+                        row + ((lane % kChunk) ^ v_swz(sr)) * 16);
+      }
+    }
+    ++issued;
+    if (++in_slot == kRing) in_slot = 0;
+    if (issued == total) return;
+    if (++in.step == in.steps) {
+      in = next_context(in);
+      if (++in_q == kRing) in_q = 0;
+      load_pages();
+      request_q();
     } else {
+      load_pages();
+    }
+  };
+  load_pages();
+  request_q();
+  for (int i = 0; i < kRing - 1; ++i)
+    if (issued < total) request();
+
+  // ---- consumer ----
+  const int tok = lane & 15, g = lane >> 4;  // also: head column, quarter
+  int k_off[KK], v_off[DT];
 #pragma unroll
-      for (int j8 = 0; j8 < KQ4; ++j8) {
-        float kf8[16 / sizeof(CT)];
-        if (FP8) {
-          const u32 w[4] = {kraw[j8].x, kraw[j8].y, kraw[j8].z, kraw[j8].w};
+  for (int kk = 0; kk < KK; ++kk)
+    k_off[kk] = FP8
+        ? tok * kRowB + (((kk * 2 + (g >> 1)) ^ k_swz(tok)) * 16) +
+              (g & 1) * 8
+        : tok * kRowB + (((kk * 4 + g) ^ k_swz(tok)) * 16);
+  {
+    // row this lane points at: tokens 4g.. of a page; bytes: of both pages
+    const int r = FP8 ? (tok >> 1) : (tok >> 2);
+    const int row = FP8 ? (r >> 2) * kPage + 4 * g + (r & 3) : 4 * g + r;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) unpack_fp8x4(w[i], &kf8[i * 4]);
-        } else {
-          const bf16x8 kv8 = __builtin_bit_cast(bf16x8, kraw[j8]);
+    for (int dt = 0; dt < DT; ++dt)
+      v_off[dt] = FP8
+          ? row * kRowB + ((dt ^ v_swz(row)) * 16) + (tok & 1) * 8
+          : row * kRowB + (((dt * 2 + ((tok & 3) >> 1)) ^ v_swz(row)) * 16) +
+                (tok & 1) * 8;
+  }
+  const float sgn = p.scale > 0.f ? 1.f : (p.scale < 0.f ? -1.f : 0.f);
+  const float c = p.scale == 0.f
+      ? 1.f : fabsf(p.scale) * 1.4426950408889634f;  // log2(e)
+
+  Cursor at = at_seq(first.seq, first.head, first.step);
+  int ring_slot = 0, q_slot = 0, done = 0;
+  while (done < total) {
+    const int n = min(at.steps - at.step, total - done);
+    const bool begins = at.step == 0, ends = at.step + n == at.steps;
+    short8 b_q[KK];
+    float m_row = kNegInf, l_row = 0.f;
+    floatx4 o_acc[DT];
 #pragma unroll
-          for (int j = 0; j < 8; ++j) kf8[j] = bf16_to_f32(kv8.h[j]);
-        }
-        constexpr int EPG = 16 / sizeof(CT);  // elems per 16-B group
+    for (int dt = 0; dt < DT; ++dt) o_acc[dt] = {0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < n; ++i, ++done) {
+      // everything up to this step has landed, queries included: newer
+      // requests are at most those of the steps behind it
+      if (issued - done >= kRing - 1)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kRing - 2) * kLoads)
+                     : "memory");
+      else if (issued - done == 2)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (i == 0) {
 #pragma unroll
-        for (int g = 0; g < G2; ++g) {
+        for (int kk = 0; kk < KK; ++kk) {
+          b_q[kk] = *reinterpret_cast<const short8*>(
+              qring + q_slot * kQB + min(tok, G - 1) * (D * 2) +
+              (kk * 4 + g) * 16);
+          if (sgn != 1.f) {
+            bf16x8 h = __builtin_bit_cast(bf16x8, b_q[kk]);
 #pragma unroll
-          for (int j4 = 0; j4 < EPG / 4; ++j4) {
-            // float4 -> ds_read_b128 (4x fewer LDS cycles than scalar)
-            const float4 qv = *reinterpret_cast<const float4*>(
-                &q_lds[hsplit * G2 + g][quad * DPQ + j8 * EPG + j4 * 4]);
-            s[g] = fmaf(kf8[j4 * 4 + 0], qv.x, s[g]);
-            s[g] = fmaf(kf8[j4 * 4 + 1], qv.y, s[g]);
-            s[g] = fmaf(kf8[j4 * 4 + 2], qv.z, s[g]);
-            s[g] = fmaf(kf8[j4 * 4 + 3], qv.w, s[g]);
+            for (int j = 0; j < 8; ++j)
+              h.h[j] = f32_to_bf16(bf16_to_f32(h.h[j]) * sgn);
+            b_q[kk] = __builtin_bit_cast(short8, h);
           }
         }
+        // read before the slot is requested again
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       }
-    }
-    // preload THIS chunk's V before the softmax so its latency hides
-    // under the reductions (it was serialized behind phase A before)
-    u32 vball[kBlockSz];
-    const CT* v_rows = v_cache + kv_base_cur;
-    if (lane < D / 2) {
-#pragma unroll
-      for (int t = 0; t < kBlockSz; ++t)
-        vball[t] = FP8
-            ? static_cast<u32>(*reinterpret_cast<const u16*>(
-                  v_rows + t * D + 2 * lane))
-            : *reinterpret_cast<const u32*>(v_rows + t * D + 2 * lane);
-    }
-    // issue next chunk's K now; it lands under softmax + PV
-    if (chunk + kCWaves < chunk_hi) {
-      kv_base = kv_base_of(chunk + kCWaves);
-      load_k(kv_base, kraw);
-    }
-    // fence: stop the scheduler from hoisting phase-B work (and its live
-    // ranges) above the softmax — cross-phase overlap doubled VGPRs
-    // (G2 is always <= 4: G=8 is head-split)
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (MFA) {
-      // this lane's score column is token l&15 (replicated per group)
-      const int col_pos = chunk * kBlockSz + (lane & 15);
-#pragma unroll
-      for (int g = 0; g < G2; ++g)
-        if (col_pos >= ctx) s[g] = kNegInf;
-    } else {
-      // reduce over the 4 dim-quarters (lanes 4t..4t+3)
-#pragma unroll
-      for (int g = 0; g < G2; ++g) {
-        s[g] += __shfl_xor(s[g], 1, 64);
-        s[g] += __shfl_xor(s[g], 2, 64);
-        if (token_pos >= ctx) s[g] = kNegInf;
-      }
-    }
+      if (issued < total) request();
 
-    // chunk max over tokens (MFA: 4-deep within the replicated 16-lane
-    // col group; scalar path: xor 4..32 spans the 16 token groups)
-    float alpha[G2];
+      const unsigned char* kb = ring + ring_slot * 2 * kMatB;
+      const unsigned char* vb = kb + kMatB;
+      floatx4 s[PP];
 #pragma unroll
-    for (int g = 0; g < G2; ++g) {
-      float cm = s[g];
-      if constexpr (MFA) {
+      for (int pg = 0; pg < PP; ++pg) {
+        s[pg] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int off = 1; off < 16; off <<= 1)
-          cm = fmaxf(cm, __shfl_xor(cm, off, 64));
-      } else {
-#pragma unroll
-        for (int off = 4; off < 64; off <<= 1)
-          cm = fmaxf(cm, __shfl_xor(cm, off, 64));
+        for (int kk = 0; kk < KK; ++kk) {
+          const unsigned char* a = kb + pg * kPage * kRowB + k_off[kk];
+          const short8 a_k = FP8
+              ? fp8_to_bf16(*reinterpret_cast<const uint2*>(a))
+              : *reinterpret_cast<const short8*>(a);
+          s[pg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_k, b_q[kk],
+                                                          s[pg], 0, 0, 0);
+        }
       }
-      const float m_new = fmaxf(m[g], cm);
-      alpha[g] = __builtin_amdgcn_exp2f(m[g] - m_new);
-      if (m[g] <= kNegInf && m_new <= kNegInf) alpha[g] = 0.f;
-      m[g] = m_new;
-    }
-
-    // probs + row-sum
+      if (at.step == at.steps - 1) {
+        const int t0 = at.step * PP * kPage + 4 * g;
 #pragma unroll
-    for (int g = 0; g < G2; ++g) {
-      float p = (s[g] <= kNegInf) ? 0.f
-                : __builtin_amdgcn_exp2f(s[g] - m[g]);
-      if constexpr (MFA) {
-        if (lane < 16) p_lds[wave][lane][g] = p;
-        float psum = p;
+        for (int pg = 0; pg < PP; ++pg)
 #pragma unroll
-        for (int off = 1; off < 16; off <<= 1)
-          psum += __shfl_xor(psum, off, 64);
-        l[g] = l[g] * alpha[g] + psum;  // each token counted once
-      } else {
-        // every token is replicated on 4 lanes -> scale by 1/4
-        if (quad == 0) p_lds[wave][tok][g] = p;
-        float psum = p;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1)
-          psum += __shfl_xor(psum, off, 64);
-        l[g] = l[g] * alpha[g] + psum * 0.25f;
+          for (int r = 0; r < 4; ++r)
+            if (t0 + pg * kPage + r >= at.ctx) s[pg][r] = -INFINITY;
       }
-    }
-
-    __builtin_amdgcn_sched_barrier(0);
-    // ---- phase B: PV accumulate; lane covers dims {2l, 2l+1} ----
-    // (vball preloaded before the softmax; p is 0 for padding tokens —
-    // phase A masks every invalid position — so the full block is safe)
+      float rm = s[0][0];
 #pragma unroll
-    for (int g = 0; g < G2; ++g) {
-      acc[g][0] *= alpha[g];
-      acc[g][1] *= alpha[g];
-    }
-    if (lane < D / 2) {
-      for (int t = 0; t < kBlockSz; ++t) {
-        float v0, v1;
-        if (FP8) {
-          float vf[4];
-          unpack_fp8x4(vball[t], vf);
-          v0 = vf[0];
-          v1 = vf[1];
+      for (int pg = 0; pg < PP; ++pg)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) rm = fmaxf(rm, s[pg][r]);
+      rm = fmaxf(rm, swap16(rm));
+      rm = fmaxf(rm, swap32(rm));
+      if (!__all((rm - m_row) * c <= kDeferThr)) {
+        const float m_new = fmaxf(m_row, rm);
+        const float alpha = __builtin_amdgcn_exp2f((m_row - m_new) * c);
+        m_row = m_new;
+        l_row *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o_acc[dt][r] *= alpha;
+      }
+      const float mc = m_row * c;
+      u16 pb[PP * 4];
+#pragma unroll
+      for (int pg = 0; pg < PP; ++pg)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float e =
+              __builtin_amdgcn_exp2f(fmaf(s[pg][r], c, -mc));
+          l_row += e;
+          pb[pg * 4 + r] = f32_to_bf16(e);
+        }
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        if constexpr (PP == 1) {
+          const short4v b = {static_cast<short>(pb[0]),
+                             static_cast<short>(pb[1]),
+                             static_cast<short>(pb[2]),
+                             static_cast<short>(pb[3])};
+          o_acc[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+              lds_read_tr4(vb + v_off[dt]), b, o_acc[dt], 0, 0, 0);
         } else {
-          v0 = bf16_to_f32(static_cast<u16>(vball[t] & 0xffff));
-          v1 = bf16_to_f32(static_cast<u16>(vball[t] >> 16));
+          const short8 b = {
+              static_cast<short>(pb[0]), static_cast<short>(pb[1]),
+              static_cast<short>(pb[2]), static_cast<short>(pb[3]),
+              static_cast<short>(pb[4]), static_cast<short>(pb[5]),
+              static_cast<short>(pb[6]), static_cast<short>(pb[7])};
+          short8 a;
+          if constexpr (FP8) {
+            a = fp8_to_bf16(lds_read_tr8(vb + v_off[dt]));
+          } else {
+            const short4v x = lds_read_tr4(vb + v_off[dt]);
+            const short4v y = lds_read_tr4(vb + v_off[dt] + kPage * kRowB);
+            a = short8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+          }
+          o_acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              a, b, o_acc[dt], 0, 0, 0);
         }
+      }
+      if (++ring_slot == kRing) ring_slot = 0;
+      ++at.step;
+    }
+
+    // ---- this context (or this part of it) is done; column = head,
+    // register r of tile dt = dim 16 dt + 4 g + r
+    l_row += swap16(l_row);
+    l_row += swap32(l_row);
+    if (begins && lane == 0) {
+      const int64_t end = lo + done - n + at.steps;
+      p.cut[at.seq * hk + at.head] = ends
+          ? make_int2(-1, 0)
+          : make_int2(slot, static_cast<int>((end + parts.each - 1) /
+                                             parts.each));
+    }
+    if (tok < G) {
+      if (begins && ends) {
+        const float inv = 1.f / l_row;
+        u16* o = p.out +
+                 (static_cast<int64_t>(at.seq) * hk * G + at.head * G + tok) *
+                     D + 4 * g;
 #pragma unroll
-        for (int g = 0; g < G2; ++g) {
-          const float p = p_lds[wave][t][g];
-          acc[g][0] = fmaf(p, v0, acc[g][0]);
-          acc[g][1] = fmaf(p, v1, acc[g][1]);
+        for (int dt = 0; dt < DT; ++dt) {
+          bf16x4 w;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) w.h[r] = f32_to_bf16(o_acc[dt][r] * inv);
+          *reinterpret_cast<bf16x4*>(o + dt * 16) = w;
+        }
+      } else {
+        const int64_t piece =
+            static_cast<int64_t>(slot * 2 + (begins ? 1 : 0)) * G + tok;
+        float* o = p.piece_o + piece * D + 4 * g;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+          *reinterpret_cast<floatx4*>(o + dt * 16) = o_acc[dt];
+        if (g == 0) {
+          p.piece_ml[piece * 2] = m_row;
+          p.piece_ml[piece * 2 + 1] = l_row;
         }
       }
     }
-  }
-
-  // ---- cross-wave flash merge (within each head-group) ----
-  if (lane < G2) {
-    merge_m[wave][lane] = m[lane];
-    merge_l[wave][lane] = l[lane];
-  }
-  if (lane < D / 2) {
-#pragma unroll
-    for (int g = 0; g < G2; ++g) {
-      merge_acc[wave][g][2 * lane] = acc[g][0];
-      merge_acc[wave][g][2 * lane + 1] = acc[g][1];
-    }
-  }
-  __syncthreads();
-
-  // head-group hsplit's G2 heads are distributed over its kCWaves waves
-#pragma unroll
-  for (int g = 0; g < G2; ++g) {
-    if ((g % kCWaves) != cwave || lane >= D / 2) continue;
-    float gm = kNegInf;
-#pragma unroll
-    for (int c = 0; c < kCWaves; ++c)
-      gm = fmaxf(gm, merge_m[c * HSE + hsplit][g]);
-    float L = 0.f, o0 = 0.f, o1 = 0.f;
-#pragma unroll
-    for (int c = 0; c < kCWaves; ++c) {
-      const int w = c * HSE + hsplit;
-      const float mw = merge_m[w][g];
-      const float f = (mw <= kNegInf) ? 0.f
-                      : __builtin_amdgcn_exp2f(mw - gm);
-      L += merge_l[w][g] * f;
-      o0 = fmaf(merge_acc[w][g][2 * lane], f, o0);
-      o1 = fmaf(merge_acc[w][g][2 * lane + 1], f, o1);
-    }
-    const int h = kv_head * G + hsplit * G2 + g;
-    if (num_parts == 1) {
-      const float inv = 1.f / L;
-      u16* o_row = out + (static_cast<int64_t>(seq) * num_heads + h) * D;
-      const u32 obits = static_cast<u32>(f32_to_bf16(o0 * inv)) |
-                        (static_cast<u32>(f32_to_bf16(o1 * inv)) << 16);
-      *reinterpret_cast<u32*>(o_row + 2 * lane) = obits;
-    } else {
-      const int64_t slot = (static_cast<int64_t>(seq) * num_heads + h) *
-                               gridDim.z + part;
-      if (lane == 0) {
-        ml_ws[slot * 2] = gm;
-        ml_ws[slot * 2 + 1] = L;
-      }
-      float2* arow = reinterpret_cast<float2*>(acc_ws + slot * D);
-      arow[lane] = make_float2(o0, o1);
+    if (done < total) {
+      at = next_context(at);
+      if (++q_slot == kRing) q_slot = 0;
     }
   }
 }
 
-// merge partials: grid (S, Hq), one wave; lane covers dims {2l, 2l+1}
+// Adds up a cut context's pieces. A block takes a context, or, where there
+// are few, one query head of it; its waves share the pieces, a long
+// context's are loaded sixteen at a time.
+constexpr int kJoinWaves = 8;
+
 template <int D>
-__global__ __launch_bounds__(kWaveSize) void paged_attn_reduce_kernel(
-    u16* __restrict__ out,            // [S, Hq, D]
-    const float* __restrict__ ml_ws,  // [S, Hq, P, 2]
-    const float* __restrict__ acc_ws, // [S, Hq, P, D]
-    const int num_parts) {
-  const int seq = blockIdx.x;
-  const int h = blockIdx.y;
-  const int num_heads = gridDim.y;
-  const int lane = threadIdx.x;
-  if (lane >= D / 2) return;
-  const int64_t base = (static_cast<int64_t>(seq) * num_heads + h) * num_parts;
-
-  float gm = kNegInf;
-  for (int p = 0; p < num_parts; ++p)
-    gm = fmaxf(gm, ml_ws[(base + p) * 2]);
-  float L = 0.f, o0 = 0.f, o1 = 0.f;
-  for (int p = 0; p < num_parts; ++p) {
-    const float mp = ml_ws[(base + p) * 2];
-    if (mp <= kNegInf) continue;
-    const float f = __builtin_amdgcn_exp2f(mp - gm);
-    L += ml_ws[(base + p) * 2 + 1] * f;
-    const float2 a =
-        reinterpret_cast<const float2*>(acc_ws + (base + p) * D)[lane];
-    o0 = fmaf(a.x, f, o0);
-    o1 = fmaf(a.y, f, o1);
+__global__ __launch_bounds__(kJoinWaves * kWaveSize)
+void paged_attn_join_kernel(const DecodeArgs p, const int heads) {
+  constexpr int V = D / 64;
+  __shared__ float part[kJoinWaves][D + 2];
+  const int blocks = p.group / heads;   // of a context
+  const int context = blockIdx.x / blocks;
+  const int2 cut = p.cut[context];
+  if (cut.x < 0) return;
+  const int lane = threadIdx.x % kWaveSize, G = p.group;
+  const int wave = threadIdx.x / kWaveSize;
+  const int sub = wave / heads, subs = kJoinWaves / heads;
+  const int h = (blockIdx.x % blocks) * heads + wave % heads;
+  const int first = cut.x;
+  const float c = p.scale == 0.f
+      ? 1.f : fabsf(p.scale) * 1.4426950408889634f;
+  float m = kNegInf, l = 0.f, o[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) o[j] = 0.f;
+  // `count` pieces from s0 on, loads first; fewer there: the first again,
+  // with weight 0
+  auto add = [&](int s0, auto count) {
+    constexpr int N = decltype(count)::value;
+    float pm[N], pl[N], x[N][V];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int s = s0 + i * subs;
+      const bool there = s < cut.y;
+      const int64_t piece = static_cast<int64_t>(
+          s == first || !there ? first * 2 + 1 : s * 2) * G + h;
+      pm[i] = p.piece_ml[piece * 2];
+      pl[i] = p.piece_ml[piece * 2 + 1];
+      if (!there) {
+        pm[i] = kNegInf;
+        pl[i] = 0.f;
+      }
+#pragma unroll
+      for (int j = 0; j < V; ++j)
+        x[i][j] = p.piece_o[piece * D + lane * V + j];
+    }
+    float mx = m;
+#pragma unroll
+    for (int i = 0; i < N; ++i) mx = fmaxf(mx, pm[i]);
+    const float a = __builtin_amdgcn_exp2f((m - mx) * c);
+    m = mx;
+    l *= a;
+#pragma unroll
+    for (int j = 0; j < V; ++j) o[j] *= a;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const float b = __builtin_amdgcn_exp2f((pm[i] - mx) * c);
+      l = fmaf(pl[i], b, l);
+#pragma unroll
+      for (int j = 0; j < V; ++j) o[j] = fmaf(x[i][j], b, o[j]);
+    }
+  };
+  int s0 = first + sub;
+  for (; s0 + 3 * subs < cut.y; s0 += 16 * subs)
+    add(s0, std::integral_constant<int, 16>());
+  for (; s0 < cut.y; s0 += 2 * subs)
+    add(s0, std::integral_constant<int, 2>());
+  if (lane == 0) {
+    part[wave][D] = m;
+    part[wave][D + 1] = l;
   }
-  const float inv = 1.f / L;
-  u16* o_row = out + (static_cast<int64_t>(seq) * num_heads + h) * D;
-  const u32 obits = static_cast<u32>(f32_to_bf16(o0 * inv)) |
-                    (static_cast<u32>(f32_to_bf16(o1 * inv)) << 16);
-  *reinterpret_cast<u32*>(o_row + 2 * lane) = obits;
+#pragma unroll
+  for (int j = 0; j < V; ++j) part[wave][lane * V + j] = o[j];
+  __syncthreads();
+  if (sub) return;
+  float mx = kNegInf;
+  for (int i = 0; i < subs; ++i) mx = fmaxf(mx, part[i * heads + wave % heads][D]);
+  l = 0.f;
+#pragma unroll
+  for (int j = 0; j < V; ++j) o[j] = 0.f;
+  for (int i = 0; i < subs; ++i) {
+    const float b = __builtin_amdgcn_exp2f((part[i * heads + wave % heads][D] - mx) * c);
+    l = fmaf(part[i * heads + wave % heads][D + 1], b, l);
+#pragma unroll
+    for (int j = 0; j < V; ++j)
+      o[j] = fmaf(part[i * heads + wave % heads][lane * V + j], b, o[j]);
+  }
+  const float inv = 1.f / l;
+  u16* row = p.out + (static_cast<int64_t>(context) * G + h) * D + lane * V;
+#pragma unroll
+  for (int j = 0; j < V; ++j) row[j] = f32_to_bf16(o[j] * inv);
 }
 
-void launch_paged_attn_decode(u16* out, float* ml_ws, float* acc_ws,
-                              const u16* q, const void* k_cache,
+}  // namespace
+
+bool decode_attn_supported(int head_dim, int group) {
+  return (head_dim == 128 || head_dim == 64) &&
+         (group == 1 || group == 2 || group == 4 || group == 8);
+}
+
+int64_t decode_piece_floats(int num_seqs, int num_kv_heads, int head_dim,
+                            int group) {
+  return static_cast<int64_t>(kDecSlots) * 2 * group * (head_dim + 2) +
+         2 * static_cast<int64_t>(num_seqs) * num_kv_heads;
+}
+
+void launch_paged_attn_decode(u16* out, const u16* q, const void* k_cache,
                               const void* v_cache, const int* block_tables,
                               const int* seq_lens, int num_seqs,
                               int64_t q_stride, int max_blocks,
                               int num_kv_heads, int head_dim, int group,
-                              int num_parts, float scale, bool fp8,
+                              float scale, bool fp8, float* pieces,
                               hipStream_t stream) {
-  const bool wide = num_seqs * num_kv_heads * num_parts < 256;
-  const int nwaves = wide ? 8 : 4;
-  dim3 grid(num_seqs, num_kv_heads, num_parts), block(nwaves * kWaveSize);
-  // FI_DECODE_MFMA=0 falls back to the scalar-FMA phase A (both dtypes;
-  // the fp8 MFA variant quantizes Q to e4m3 per head)
-  static const bool mfa = [] {
-    const char* e = getenv("FI_DECODE_MFMA");
-    return !(e && e[0] == '0');
-  }();
-// fp8 MFA dispatch is G=8-only: kbench showed +41-43% there (G2=4
-// after head-split) but -21% at G=4 fp8, where the scalar HS=2 path
-// with halved KV bytes was already latency-optimal.
-#define FI_LAUNCH_1(DD, GG, NW, F8, HSP)                                      \
-  if (mfa && (!F8 || GG == 8)) {                                              \
-    hipLaunchKernelGGL(                                                       \
-        (paged_attn_decode_kernel<DD, GG, NW, F8, HSP, true>), grid,          \
-        block, 0, stream, out, ml_ws, acc_ws, q, k_cache, v_cache,            \
-        block_tables, seq_lens, q_stride, max_blocks, num_kv_heads, scale);   \
-  } else {                                                                    \
-    hipLaunchKernelGGL((paged_attn_decode_kernel<DD, GG, NW, F8, HSP>), grid, \
-                       block, 0, stream, out, ml_ws, acc_ws, q, k_cache,      \
-                       v_cache, block_tables, seq_lens, q_stride, max_blocks, \
-                       num_kv_heads, scale);                                  \
-  }
-// Head-split policy, A/B'd on hardware (2026-09-14 kbench):
-// - G=8 always runs HS=2 (monolithic spilled; HS=4 measured a wash at
-//   full grids and -12% wide).
-// - G=4 runs HS=2 only at FULL grids (4-wave blocks): the G2=2 state
-//   compiles to 149 VGPR = 3 waves/SIMD, measured +2.5% bf16 / +8% fp8
-//   at b256; at WIDE grids (8-wave, small batches) the halved chunk
-//   parallelism lost 12-19%, so wide keeps the monolithic G=4 shape.
-// (The streaming-convert phase A + early V preload apply everywhere.)
-#define FI_LAUNCH_HS(DD, GG, HSW, HSN)                                        \
-  if (fp8) {                                                                  \
-    if (wide) { FI_LAUNCH_1(DD, GG, 8, true, HSW); }                          \
-    else      { FI_LAUNCH_1(DD, GG, 4, true, HSN); }                          \
-  } else {                                                                    \
-    if (wide) { FI_LAUNCH_1(DD, GG, 8, false, HSW); }                         \
-    else      { FI_LAUNCH_1(DD, GG, 4, false, HSN); }                         \
-  }                                                                           \
-  if (num_parts > 1) {                                                        \
-    dim3 rgrid(num_seqs, num_kv_heads * GG), rblock(kWaveSize);               \
-    hipLaunchKernelGGL((paged_attn_reduce_kernel<DD>), rgrid, rblock, 0,      \
-                       stream, out, ml_ws, acc_ws, num_parts);                \
-  }
-#define FI_LAUNCH(DD, GG)                                                     \
-  if (GG == 8)      { FI_LAUNCH_HS(DD, GG, 2, 2) }                            \
-  else if (GG == 4) { FI_LAUNCH_HS(DD, GG, 1, 2) }                            \
-  else              { FI_LAUNCH_HS(DD, GG, 1, 1) }
+  DecodeArgs a;
+  a.out = out;
+  a.q = q;
+  a.k = static_cast<const unsigned char*>(k_cache);
+  a.v = static_cast<const unsigned char*>(v_cache);
+  a.block_tables = block_tables;
+  a.seq_lens = seq_lens;
+  a.piece_o = pieces;
+  a.piece_ml = pieces + static_cast<int64_t>(kDecSlots) * 2 * group * head_dim;
+  a.cut = reinterpret_cast<int2*>(
+      a.piece_ml + static_cast<int64_t>(kDecSlots) * 2 * group * 2);
+  a.q_stride = q_stride;
+  a.num_seqs = num_seqs;
+  a.max_blocks = max_blocks;
+  a.num_kv_heads = num_kv_heads;
+  a.group = group;
+  a.scale = scale;
+  const dim3 block(kDecWaves * kWaveSize);
+  // one context of 8000 tokens leaves 125 pieces: a block per query head
+  // takes 5 us where a block per context takes 11
+  const int contexts = num_seqs * num_kv_heads;
+  const int heads = contexts < 256 ? 1 : group;
+#define FI_DEC(DD, F8)                                                        \
+  do {                                                                        \
+    hipLaunchKernelGGL((paged_attn_decode_kernel<DD, F8>),                    \
+                       dim3(kDecSlots / kDecWaves), block, 0, stream, a);     \
+    hipLaunchKernelGGL((paged_attn_join_kernel<DD>),                          \
+                       dim3(contexts * (group / heads)),                      \
+                       dim3(kJoinWaves * kWaveSize), 0, stream, a, heads);    \
+  } while (0)
   if (head_dim == 128) {
-    switch (group) {
-      case 1: FI_LAUNCH(128, 1); break;
-      case 2: FI_LAUNCH(128, 2); break;
-      case 4: FI_LAUNCH(128, 4); break;
-      case 8: FI_LAUNCH(128, 8); break;
-      default: abort();
-    }
-  } else if (head_dim == 64) {
-    switch (group) {
-      case 1: FI_LAUNCH(64, 1); break;
-      case 2: FI_LAUNCH(64, 2); break;
-      case 4: FI_LAUNCH(64, 4); break;
-      case 8: FI_LAUNCH(64, 8); break;
-      default: abort();
-    }
+    if (fp8) FI_DEC(128, true);
+    else FI_DEC(128, false);
   } else {
-    abort();
+    if (fp8) FI_DEC(64, true);
+    else FI_DEC(64, false);
   }
-#undef FI_LAUNCH
-#undef FI_LAUNCH_1
+#undef FI_DEC
 }
 
 }  // namespace fi

@@ -333,6 +333,64 @@ def test_prefill_attention_row_blocks_and_parts(hq, hk, ctx_lens, new_lens,
     assert_close_bf16(out.cpu(), want, atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize(
+    "group,hk,lens,scale_by",
+    [
+        # ends around pages (16) and two-page steps
+        (4, 2, [1, 15, 16, 17, 31, 32, 33], 1.0),
+        # contexts shorter than a part, more of them than lanes, several
+        # borders inside one part
+        (2, 3, [1 + (7 * i) % 50 for i in range(150)], -1.0),
+        # one context over many parts; parts that cut it unevenly
+        (8, 1, [5000], 1.0),
+        (1, 4, [3, 2500, 16, 900], 1.0),
+        # long and short in turn: whole contexts between cut ones
+        (4, 8, [1200, 5, 1201, 64, 3000, 1] * 6, 0.0),
+    ],
+)
+def test_paged_attention_decode_parts(group, hk, lens, scale_by, head_dim,
+                                      fp8):
+    """Borders of pages, contexts and parts against the fp32 reference (same
+    bound as above); what lies behind a context's end is never read."""
+    g = torch.Generator().manual_seed(13)
+    bs, S = 16, len(lens)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g).to(torch.bfloat16).to(DEV)
+
+    need = [(c + bs - 1) // bs for c in lens]
+    perm = (torch.randperm(sum(need), generator=g) + 1).int()
+    bt = torch.zeros(S, max(need) + 3, dtype=torch.int32)
+    for s, row in enumerate(perm.split(need)):
+        bt[s, :need[s]] = row
+    # the query part of a merged projection
+    q = rnd(S, 2 * group * hk * head_dim)[:, : group * hk * head_dim]
+    q = q.view(S, group * hk, head_dim)
+    k_cache = rnd(sum(need) + 1, hk, bs, head_dim)
+    v_cache = rnd(sum(need) + 1, hk, bs, head_dim)
+    if fp8:
+        k_cache, v_cache = _fp8_cache(k_cache), _fp8_cache(v_cache)
+    else:
+        for s, c in enumerate(lens):
+            if c % bs:
+                v_cache[int(bt[s, need[s] - 1]), :, c % bs:] = float("nan")
+                k_cache[int(bt[s, need[s] - 1]), :, c % bs:] = float("nan")
+    scale = scale_by / math.sqrt(head_dim)
+    sl = torch.tensor(lens, dtype=torch.int32)
+    out = ops.paged_attention_decode(q, k_cache, v_cache, bt.to(DEV),
+                                     sl.to(DEV), scale)
+    want = ref.paged_attention_decode(q.cpu(), k_cache.cpu(), v_cache.cpu(),
+                                      bt, sl, scale)
+    assert_close_bf16(out.cpu(), want, atol=2e-2, rtol=2e-2)
+    # rows off the 16-byte grid give the same
+    off = torch.empty(S, q[0].numel() + 1, dtype=q.dtype, device=DEV)[:, 1:]
+    off = off.view(S, group * hk, head_dim).copy_(q)
+    assert torch.equal(out, ops.paged_attention_decode(
+        off, k_cache, v_cache, bt.to(DEV), sl.to(DEV), scale))
+
+
 # ------------------------------------------------------------ fp8 KV cache
 
 def _fp8_cache(t):
