@@ -39,6 +39,7 @@ SOURCES = [
 MOE_SOURCES = [
     "moe_bindings.hip",
     "moe_gemm.hip",
+    "moe_tile.hip",
     "moe_plain.hip",
 ]
 

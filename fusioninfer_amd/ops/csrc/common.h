@@ -148,6 +148,42 @@ FI_DEV void dma_to_lds16_nt(u32 lds, const void* base, u32 offset) {
 #endif
 }
 
+// the same through a buffer descriptor (base, 0, bytes, format): scalar
+// base + vector offset + scalar offset; what lies behind the end reads as 0
+typedef __attribute__((ext_vector_type(4))) u32 u32x4;
+FI_DEV u32x4 descriptor_of(const void* p, u32 bytes) {
+  const uint64_t a = reinterpret_cast<uint64_t>(p);
+  return u32x4{static_cast<u32>(a), static_cast<u32>(a >> 32), bytes,
+               0x00020000u};
+}
+FI_DEV void buffer_to_lds16(u32 lds, u32x4 desc, u32 voff, u32 soff) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 4\n\t"
+      "buffer_load_dwordx4 %1, %2, %3 offen lds"
+      :
+      : "s"(lds), "v"(voff), "s"(desc), "s"(soff)
+      : "memory");
+#endif
+}
+
+// 16-byte loads at scalar base + vector offset + scalar offset (bytes)
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __amdgpu_buffer_rsrc_t BufferRsrc;
+FI_DEV BufferRsrc buffer_of(const void* p, u32 bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes,
+                                           0x00020000);
+}
+FI_DEV u32x4 buffer_load16(BufferRsrc r, u32 voff, u32 soff) {
+  return __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+}
+#else
+struct BufferRsrc {};
+FI_DEV BufferRsrc buffer_of(const void*, u32) { return {}; }
+FI_DEV u32x4 buffer_load16(BufferRsrc, u32, u32) { return {}; }
+#endif
+
 // Integers that no kernel of the launch writes, read through the scalar
 // cache (at a wave-uniform index they return on lgkmcnt, not behind the
 // DMAs).

@@ -35,6 +35,9 @@
 
 namespace fi {
 
+void launch_moe_tile(u16*, const u16*, const u16*, const int*, const int*,
+                     const int*, int, int, int, int, int, float, hipStream_t);
+
 namespace {
 
 typedef __attribute__((ext_vector_type(8))) short short8;
@@ -492,8 +495,8 @@ __global__ __launch_bounds__(256) void moe_gemm_fp8_kernel(
 // 4x the output columns of v1.
 void launch_moe_gemm(u16* out, const u16* a, const u16* b,
                      const int* sorted_ids, const int* expert_ids,
-                     const int* n_valid, int max_mtiles, int K, int N,
-                     int block_m, int mode, float limit,
+                     const int* n_valid, int max_mtiles, int rows, int K,
+                     int N, int block_m, int mode, float limit,
                      hipStream_t stream) {
   if (block_m == 16) {
     const dim3 grid(max_mtiles, N / 64);
@@ -514,52 +517,8 @@ void launch_moe_gemm(u16* out, const u16* a, const u16* b,
                          dim3(256), 0, stream, out, a, b, sorted_ids,
                          expert_ids, n_valid, K, N, limit);
   } else {  // block_m == 128
-    // FI_MOE_STAGE_A=0 falls back to the register-gather form (A/B knob)
-    static const bool stage_a = [] {
-      const char* e = getenv("FI_MOE_STAGE_A");
-      return !(e && e[0] == '0');
-    }();
-    if (mode == 1) {
-      const dim3 grid(max_mtiles, N / 64);
-      if (stage_a)
-        hipLaunchKernelGGL((moe_gemm_kernel<2, 2, 4, 2, 1, true>), grid,
-                           dim3(256), 0, stream, out, a, b, sorted_ids,
-                           expert_ids, n_valid, K, N, limit);
-      else
-        hipLaunchKernelGGL((moe_gemm_kernel<2, 2, 4, 2, 1, false>), grid,
-                           dim3(256), 0, stream, out, a, b, sorted_ids,
-                           expert_ids, n_valid, K, N, limit);
-    } else if (mode == 3) {
-      const dim3 grid(max_mtiles, N / 64);
-      if (stage_a)
-        hipLaunchKernelGGL((moe_gemm_kernel<2, 2, 4, 2, 3, true>), grid,
-                           dim3(256), 0, stream, out, a, b, sorted_ids,
-                           expert_ids, n_valid, K, N, limit);
-      else
-        hipLaunchKernelGGL((moe_gemm_kernel<2, 2, 4, 2, 3, false>), grid,
-                           dim3(256), 0, stream, out, a, b, sorted_ids,
-                           expert_ids, n_valid, K, N, limit);
-    } else if (mode == 2) {
-      const dim3 grid(max_mtiles, N / 64);
-      if (stage_a)
-        hipLaunchKernelGGL((moe_gemm_kernel<2, 2, 4, 2, 2, true>), grid,
-                           dim3(256), 0, stream, out, a, b, sorted_ids,
-                           expert_ids, n_valid, K, N, limit);
-      else
-        hipLaunchKernelGGL((moe_gemm_kernel<2, 2, 4, 2, 2, false>), grid,
-                           dim3(256), 0, stream, out, a, b, sorted_ids,
-                           expert_ids, n_valid, K, N, limit);
-    } else {
-      const dim3 grid(max_mtiles, N / 128);
-      if (stage_a)
-        hipLaunchKernelGGL((moe_gemm_kernel<2, 2, 4, 4, 0, true>), grid,
-                           dim3(256), 0, stream, out, a, b, sorted_ids,
-                           expert_ids, n_valid, K, N, limit);
-      else
-        hipLaunchKernelGGL((moe_gemm_kernel<2, 2, 4, 4, 0, false>), grid,
-                           dim3(256), 0, stream, out, a, b, sorted_ids,
-                           expert_ids, n_valid, K, N, limit);
-    }
+    launch_moe_tile(out, a, b, sorted_ids, expert_ids, n_valid, max_mtiles,
+                    rows, K, N, mode, limit, stream);
   }
 }
 

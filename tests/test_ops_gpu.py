@@ -797,3 +797,54 @@ def test_skinny_linear_leaves_other_calls_to_the_library():
     x = rnd(4, 256).requires_grad_()
     ops.linear(x, w).sum().backward()
     assert x.grad is not None
+
+
+# ------------------------------------------------- grouped GEMM, 128 rows
+
+
+@pytest.mark.parametrize("k", [32, 96, 128, 224, 768])
+@pytest.mark.parametrize("n,gate_up,act", [
+    (64, True, None),          # less than one column tile
+    (320, True, None),         # ragged last tile, ragged wave
+    (192, True, "clamped_glu"),
+    (64, False, "relu_sq"),
+    (128, False, None),
+    (640, False, None),        # two and a half column tiles
+])
+def test_moe_gemm_row_blocks_of_128(k, n, gate_up, act):
+    """Experts with no row, one row, a whole block, a block and one row and
+    many, against float64 products; one bf16 rounding of the result (2^-9)
+    and fp32 sums of k products of unit variance."""
+    g = torch.Generator().manual_seed(k + n)
+    T, top, bm = 700, 2, 128
+    sizes = [0, 1, 128, 129, 300, 0, 842]   # assignments, 2 T in all
+    experts = torch.cat([torch.full((c,), e) for e, c in enumerate(sizes)])
+    topi = experts[torch.randperm(T * top, generator=g)].view(T, top)
+    topi = topi.int().to(DEV)
+    gather = gate_up or act is not None
+    nb = 2 * n if gate_up else n
+    w = torch.randn(len(sizes), k, nb, generator=g).to(torch.bfloat16).to(DEV)
+    sid, eid, nv, pos, PM = ops.moe_align(topi, 0, len(sizes), bm)
+    rows = torch.randn(T if gather else PM, k, generator=g)
+    rows = rows.to(torch.bfloat16).to(DEV)
+    out = torch.empty(PM, n, dtype=torch.bfloat16, device=DEV)
+    ops.moe_gemm(out, rows, ops.pack_moe_weights(w), sid, eid, nv, bm,
+                 gate_up, act, 3.0)
+    assert int(nv) == sum(-(-c // bm) for c in sizes)
+    for m in range(int(nv)):
+        at = slice(m * bm, (m + 1) * bm)
+        a = rows[sid[at].long()] if gather else rows[at]
+        y = a.double() @ w[int(eid[m])].double()
+        slack = 1e-5 * k ** 0.5
+        if act == "clamped_glu":
+            gt, up = y[:, :n].clamp(max=3.0), y[:, n:].clamp(-3.0, 3.0)
+            y = gt * torch.sigmoid(1.702 * gt) * (up + 1.0)
+            slack *= 20
+        elif gate_up:
+            y = torch.nn.functional.silu(y[:, :n]) * y[:, n:]
+            slack *= 20 * k ** 0.5
+        elif act == "relu_sq":
+            y = y.clamp(min=0).square()
+            slack *= 20 * k ** 0.5
+        err = (out[at].double() - y).abs()
+        assert (err <= y.abs() * 2 ** -8 + slack).all(), m
