@@ -543,8 +543,12 @@ class MoEMLP(nn.Module):
         combine. No host syncs — MoE decode is hipGraph-capturable."""
         T, H = x.shape
         E_local = self.e_end - self.e_start
-        logits = x.float() @ self.router_weight.float().T
-        topv, topi = self._router_topk(logits)
+        if x.is_cuda:
+            topv, topi = ops.moe_router(x, self.router_weight, self.top_k,
+                                        self.norm_topk)
+        else:
+            topv, topi = self._router_topk(
+                x.float() @ self.router_weight.float().T)
         # block_m: 16 in the few-rows-per-expert (decode) regime, 128 when
         # segments are long enough for the 4x in-register B-reuse variant
         block_m = 128 if T * self.top_k >= 64 * E_local else 16

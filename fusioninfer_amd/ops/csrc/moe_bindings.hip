@@ -24,8 +24,11 @@ void launch_moe_gemm_fp8(u16*, const unsigned char*, const float*,
                          const unsigned char*, const float*, const int*,
                          const int*, const int*, int, int, int, int, bool,
                          hipStream_t);
-void launch_moe_align(const int*, int*, int*, int*, int*, int, int, int,
+int64_t moe_align_scratch(int, int);
+void launch_moe_align(const int*, int*, int*, int*, int*, int*, int, int, int,
                       int, int, int, hipStream_t);
+void launch_moe_router_logits(const u16*, const u16*, float*, int, int, int,
+                              hipStream_t);
 void launch_moe_router_topk(const float*, float*, int*, int, int, int,
                             bool, hipStream_t);
 void launch_moe_route(const float*, float*, int*, int, int, int, bool, bool,
@@ -283,10 +286,31 @@ void moe_align(at::Tensor topi, at::Tensor sorted_ids, at::Tensor expert_ids,
   TORCH_CHECK(e_end - e_start <= 1024, "moe_align: E_local > 1024");
   TORCH_CHECK(PM % block_m == 0 && expert_ids.numel() == PM / block_m);
   TORCH_CHECK(pos.numel() == n);
+  at::Tensor scratch = at::empty(
+      {fi::moe_align_scratch(n, e_end - e_start)}, topi.options());
   fi::launch_moe_align(topi.data_ptr<int>(), sorted_ids.data_ptr<int>(),
                        expert_ids.data_ptr<int>(), n_valid.data_ptr<int>(),
-                       pos.data_ptr<int>(), n, (int)topk, (int)e_start,
+                       pos.data_ptr<int>(), scratch.data_ptr<int>(), n,
+                       (int)topk, (int)e_start,
                        (int)e_end, (int)block_m, PM, current_stream());
+}
+
+void moe_router_logits(at::Tensor x, at::Tensor w, at::Tensor logits) {
+  CHECK_BF16_CUDA(x);
+  CHECK_BF16_CUDA(w);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.is_contiguous() &&
+              w.is_contiguous());
+  const int T = x.size(0), K = x.size(1), E = w.size(0);
+  TORCH_CHECK(w.size(1) == K && K % 32 == 0 && K > 0 && E % 16 == 0 && E > 0,
+              "moe_router_logits: experts in sixteens, width in 32s");
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0);
+  TORCH_CHECK(logits.scalar_type() == at::kFloat && logits.is_contiguous() &&
+              logits.numel() == static_cast<int64_t>(T) * E);
+  if (T == 0) return;
+  fi::launch_moe_router_logits(bf16_cptr(x), bf16_cptr(w),
+                               logits.data_ptr<float>(), T, E, K,
+                               current_stream());
 }
 
 void moe_router_topk(at::Tensor logits, at::Tensor topv, at::Tensor topi,
@@ -320,6 +344,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_align", &moe_align,
         "single-kernel block alignment of expert assignments "
         "(vLLM moe_align_block_size analog)");
+  m.def("moe_router_logits", &moe_router_logits,
+        "fp32 router logits of a few bf16 rows");
   m.def("moe_router_topk", &moe_router_topk,
         "fused router tail: softmax + top-k + optional renormalize");
   m.def("moe_route_grouped", &moe_route_grouped,

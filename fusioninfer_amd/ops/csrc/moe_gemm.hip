@@ -567,140 +567,4 @@ void launch_moe_gemm_fp8(u16* out, const unsigned char* a,
   }
 }
 
-// Device-side MoE block alignment in ONE kernel (replaces the ~12-op
-// torch composition in MoEMLP._moe_align: scatter_add histogram,
-// argsort, cumsums, searchsorted, scatters — measured ~6% of 30B MoE
-// GPU time plus a dozen eager launches per layer during prefill).
-// Single workgroup: ≤16K assignments and ≤1024 local experts make LDS
-// histograms + __syncthreads phases trivial. Within-expert slot order
-// is atomicAdd arrival order (NOT the stable argsort order) — the
-// grouped GEMM computes each row's K-loop identically wherever it sits
-// in the expert's segment and the combine gathers by pos, so outputs
-// are bit-identical regardless of slot permutation. vLLM parity:
-// moe_align_block_size (csrc/moe/moe_align_sum_kernels.cu).
-namespace {
-__global__ void moe_align_kernel(
-    const int* __restrict__ topi,  // [n] = T*topk flattened GLOBAL ids
-    int* __restrict__ sorted_ids,  // [PM]   (zeroed here; pad rows -> 0)
-    int* __restrict__ expert_ids,  // [PM / block_m]
-    int* __restrict__ n_valid,     // [1] real m-tile count
-    int* __restrict__ pos,         // [n]  padded slot (-1 = non-local)
-    const int n, const int topk, const int e_start, const int e_end,
-    const int block_m, const int PM) {
-  const int E = e_end - e_start;  // <= 1024 by LDS sizing below
-  __shared__ int cnt[1025], pad0[1025], tcum[1025], off[1025];
-  const int tid = threadIdx.x, nt = blockDim.x;
-  for (int i = tid; i <= E; i += nt) cnt[i] = 0;
-  for (int i = tid; i < PM; i += nt) sorted_ids[i] = 0;
-  __syncthreads();
-  for (int i = tid; i < n; i += nt) {
-    const int e = topi[i];
-    const int key = (e >= e_start && e < e_end) ? e - e_start : E;
-    atomicAdd(&cnt[key], 1);
-  }
-  __syncthreads();
-  if (tid == 0) {
-    int tiles = 0;
-    for (int e = 0; e < E; ++e) {
-      pad0[e] = tiles * block_m;
-      tiles += (cnt[e] + block_m - 1) / block_m;
-      tcum[e] = tiles;
-    }
-    n_valid[0] = tiles;
-  }
-  __syncthreads();
-  // expert of m-tile t = first e with tcum[e] > t (searchsorted
-  // right=True), clamped to E-1 for the padded tail
-  for (int t = tid; t < PM / block_m; t += nt) {
-    int lo = 0, hi = E - 1, ans = E - 1;
-    while (lo <= hi) {
-      const int mid = (lo + hi) >> 1;
-      if (tcum[mid] > t) { ans = mid; hi = mid - 1; }
-      else lo = mid + 1;
-    }
-    expert_ids[t] = ans;
-  }
-  for (int i = tid; i <= E; i += nt) off[i] = 0;
-  __syncthreads();
-  for (int i = tid; i < n; i += nt) {
-    const int e = topi[i];
-    const int key = (e >= e_start && e < e_end) ? e - e_start : E;
-    if (key == E) { pos[i] = -1; continue; }
-    const int p = pad0[key] + atomicAdd(&off[key], 1);
-    pos[i] = p;
-    sorted_ids[p] = i / topk;
-  }
-}
-}  // namespace
-
-void launch_moe_align(const int* topi, int* sorted_ids, int* expert_ids,
-                      int* n_valid, int* pos, int n, int topk, int e_start,
-                      int e_end, int block_m, int PM, hipStream_t stream) {
-  hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(1024), 0, stream, topi,
-                     sorted_ids, expert_ids, n_valid, pos, n, topk, e_start,
-                     e_end, block_m, PM);
-}
-
-// Fused router tail: softmax + top-k + (optional) renormalize in ONE
-// wave-per-token kernel (replaces torch softmax/gatherTopK/bitonic-
-// sort/div — ~3.5% of 30B MoE GPU time and 6 launches per layer).
-// With renorm (norm_topk_prob), weights = softmax over the top-k
-// LOGITS (the global partition cancels); without it, global softmax
-// probabilities. Ties pick the smaller expert index.
-namespace {
-__global__ void moe_router_topk_kernel(
-    const float* __restrict__ logits,  // [T, E] fp32
-    float* __restrict__ topv,          // [T, k]
-    int* __restrict__ topi,            // [T, k]
-    const int T, const int E, const int k, const bool renorm) {
-  const int t = blockIdx.x * (blockDim.x / kWaveSize)
-      + threadIdx.x / kWaveSize;
-  if (t >= T) return;
-  const int lane = threadIdx.x % kWaveSize;
-  const float* row = logits + static_cast<int64_t>(t) * E;
-  // two logit slots per lane (E <= 128)
-  float l0 = lane < E ? row[lane] : -INFINITY;
-  float l1 = lane + 64 < E ? row[lane + 64] : -INFINITY;
-  float m = fmaxf(l0, l1);
-#pragma unroll
-  for (int off = 32; off; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-  float s = (lane < E ? __expf(l0 - m) : 0.f) +
-            (lane + 64 < E ? __expf(l1 - m) : 0.f);
-#pragma unroll
-  for (int off = 32; off; off >>= 1) s += __shfl_xor(s, off);
-  float a0 = l0, a1 = l1;  // remaining candidates
-  float ksum = 0.f;
-  for (int it = 0; it < k; ++it) {
-    float v = a0 >= a1 ? a0 : a1;
-    int idx = a0 >= a1 ? lane : lane + 64;
-#pragma unroll
-    for (int off = 32; off; off >>= 1) {
-      const float ov = __shfl_xor(v, off);
-      const int oi = __shfl_xor(idx, off);
-      if (ov > v || (ov == v && oi < idx)) { v = ov; idx = oi; }
-    }
-    const float e = __expf(v - m);
-    ksum += e;
-    if (lane == 0) {
-      topi[t * k + it] = idx;
-      topv[t * k + it] = renorm ? e : e / s;
-    }
-    if (idx == lane) a0 = -INFINITY;
-    if (idx == lane + 64) a1 = -INFINITY;
-  }
-  if (renorm && lane == 0) {
-    for (int it = 0; it < k; ++it) topv[t * k + it] /= ksum;
-  }
-}
-}  // namespace
-
-void launch_moe_router_topk(const float* logits, float* topv, int* topi,
-                            int T, int E, int k, bool renorm,
-                            hipStream_t stream) {
-  const int waves = 4;  // 4 tokens per 256-thread block
-  hipLaunchKernelGGL(moe_router_topk_kernel,
-                     dim3(ceil_div(T, waves)), dim3(waves * kWaveSize), 0,
-                     stream, logits, topv, topi, T, E, k, renorm);
-}
-
 }  // namespace fi

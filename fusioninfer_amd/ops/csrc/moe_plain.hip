@@ -372,6 +372,50 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(
   Act<A>::st(out + static_cast<int64_t>(t) * H + c, acc);
 }
 
+// Rows of whole 16-byte vectors: a thread takes one vector of a token, all
+// of its experts' rows are requested before the first is used. Bound by
+// reading the rows (8765 tokens, top 8, width 2048: 287 MB and 36 MB out,
+// 172 us with one value per thread, 61 now).
+template <typename A>
+__global__ __launch_bounds__(256) void moe_combine_vec_kernel(
+    A* __restrict__ out, const A* __restrict__ y, const int* __restrict__ pos,
+    const float* __restrict__ w, const int topk, const int H) {
+  constexpr int V = 16 / sizeof(A), kAhead = 8;
+  struct alignas(16) Vec {
+    A v[V];
+  };
+  const int t = blockIdx.x;
+  const int c = (blockIdx.y * 256 + threadIdx.x) * V;
+  if (c >= H) return;
+  float acc[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) acc[j] = 0.f;
+  for (int k0 = 0; k0 < topk; k0 += kAhead) {
+    Vec r[kAhead];
+    float wk[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const int k = k0 + i;
+      const int p = k < topk ? pos[t * topk + k] : -1;
+      wk[i] = 0.f;
+      r[i] = Vec{};
+      if (p >= 0) {
+        wk[i] = w[t * topk + k];
+        r[i] = *reinterpret_cast<const Vec*>(
+            y + static_cast<int64_t>(p) * H + c);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i)
+#pragma unroll
+      for (int j = 0; j < V; ++j) acc[j] += wk[i] * Act<A>::ld(&r[i].v[j]);
+  }
+  Vec o;
+#pragma unroll
+  for (int j = 0; j < V; ++j) Act<A>::st(&o.v[j], acc[j]);
+  *reinterpret_cast<Vec*>(out + static_cast<int64_t>(t) * H + c) = o;
+}
+
 }  // namespace
 
 void launch_moe_route(const float* logits, float* topv, int* topi, int T,
@@ -427,6 +471,16 @@ void launch_moe_gemm_plain(A* out, const A* a, const A* w,
 template <typename A>
 void launch_moe_combine(A* out, const A* y, const int* pos, const float* w,
                         int tokens, int topk, int H, hipStream_t stream) {
+  constexpr int V = 16 / sizeof(A);
+  const bool vec = H % V == 0 &&
+      (reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(y)) %
+          16 == 0;
+  if (vec) {
+    hipLaunchKernelGGL(moe_combine_vec_kernel<A>,
+                       dim3(tokens, ceil_div(H / V, 256)), dim3(256), 0,
+                       stream, out, y, pos, w, topk, H);
+    return;
+  }
   const dim3 grid(ceil_div(H, 256), tokens);
   hipLaunchKernelGGL(moe_combine_kernel<A>, grid, dim3(256), 0, stream, out,
                      y, pos, w, topk, H);

@@ -698,6 +698,10 @@ def test_moe_align_kernel_matches_python():
         (300, 8, 16, 4, 12, 16),  # EP slice: half the experts non-local
         (256, 8, 8, 0, 8, 128),   # prefill block_m
         (1, 8, 128, 0, 128, 16),  # decode single token, many experts
+        (512, 8, 128, 0, 128, 16),   # the most of the one-workgroup form
+        (4097, 1, 3, 0, 3, 128),     # one more: two launches, odd shares
+        (3000, 8, 128, 32, 96, 128),
+        (1100, 4, 1000, 0, 1000, 16),
     ]
     for T, k, E, e0, e1, bm in cases:
         topi = torch.randint(0, E, (T, k), device=DEV)
@@ -740,6 +744,71 @@ def test_moe_router_topk_matches_torch():
             etv = etv / etv.sum(-1, keepdim=True)
         assert torch.equal(ti.long(), eti), (T, E, k)
         torch.testing.assert_close(tv, etv, atol=2e-6, rtol=2e-6)
+
+
+@pytest.mark.parametrize("T,E,K,k,renorm", [
+    (1, 128, 2048, 8, True),
+    (17, 16, 32, 16, False),    # one step: three waves hold nothing
+    (64, 48, 288, 3, True),     # odd share of K, part of a batch of loads
+    (512, 128, 2048, 128, True),  # every expert chosen
+    (513, 112, 1024, 8, False),   # the library's product
+    (5, 40, 256, 2, True),
+])
+def test_moe_router(T, E, K, k, renorm):
+    """Router against a float64 product: the same experts
+    where their gap exceeds what fp32 sums of K products can move, weights
+    to that accuracy."""
+    g = torch.Generator().manual_seed(T + E)
+    x = torch.randn(T, K, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(E, K, generator=g) * 0.05).to(torch.bfloat16).to(DEV)
+    tv, ti = ops.moe_router(x, w, k, renorm)
+    logits = x.double() @ w.double().T
+    probs = torch.softmax(logits, -1)
+    ev, ei = probs.topk(k, -1)
+    gap = -torch.diff(logits.sort(-1, descending=True).values[:, :k + 1])
+    sure = (gap > 1e-4).all(-1) if gap.numel() else torch.ones(T, dtype=bool)
+    assert torch.equal(ti.long()[sure], ei[sure])
+    if renorm:
+        ev = ev / ev.sum(-1, keepdim=True)
+    torch.testing.assert_close(tv.double(), ev, atol=1e-5, rtol=1e-4)
+
+
+def test_moe_router_topk_ties():
+    """Equal logits: the smaller index first; every expert once."""
+    for E, k in [(128, 8), (128, 128), (70, 70), (5, 5)]:
+        logits = torch.zeros(3, E, device=DEV)
+        logits[1, E // 2:] = 1.0
+        logits[2, ::2] = -float("inf")
+        tv, ti = ops.moe_router_topk(logits, k, False)
+        half = [*range(E // 2, E), *range(E // 2)]
+        odd = [*range(1, E, 2), *range(0, E, 2)]
+        assert ti[0].tolist() == list(range(k))
+        assert ti[1].tolist() == half[:k]
+        assert ti[2].tolist() == odd[:k]
+        torch.testing.assert_close(tv[0], torch.full_like(tv[0], 1 / E))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,top,H", [(3, 1, 8), (7, 9, 2056), (5, 8, 4096),
+                                     (4, 2, 30)])
+def test_moe_combine_widths(T, top, H, dtype):
+    """Whole vectors and ragged widths, more experts than one batch of
+    loads, absent rows (whose memory may hold anything)."""
+    g = torch.Generator().manual_seed(H)
+    y = torch.randn(T * top + 1, H, generator=g).to(dtype).to(DEV)
+    y[T * top] = float("nan")
+    pos = torch.randperm(T * top, generator=g).int()
+    pos[1::3] = -1
+    w = torch.rand(T * top, generator=g)
+    out = torch.empty(T, H, dtype=dtype, device=DEV)
+    ops.moe_combine(out, y, pos.to(DEV), w.to(DEV))
+    rows = y.double()[pos.clamp(min=0).long().to(DEV)]
+    rows[(pos < 0).to(DEV)] = 0.0
+    want = (rows * w.double().to(DEV)[:, None]).view(T, top, H).sum(1)
+    # half a unit of the result's type, and fp32 sums
+    half = 2 ** -8 if dtype == torch.bfloat16 else 0.0
+    err = (out.double() - want).abs()
+    assert (err <= want.abs() * half + 1e-5).all()
 
 
 # ------------------------------------------------------------ skinny GEMM
