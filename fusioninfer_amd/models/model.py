@@ -83,17 +83,15 @@ class Attention(nn.Module):
         q = qkv[:, : self.q_size]
         k = qkv[:, self.q_size : self.q_size + self.kv_size]
         v = qkv[:, self.q_size + self.kv_size :]
-        ops.rope_qk_norm_(
-            q, k, meta.positions, cos_sin,
-            self.num_heads, self.num_kv_heads, self.head_dim,
-            self.q_norm_weight, self.k_norm_weight, self.eps,
-        )
         k_cache, v_cache = kv_cache
         fp8_kv = k_cache.dtype == torch.float8_e4m3fn
         ks = self.k_scale if fp8_kv else 1.0
         vs = self.v_scale if fp8_kv else 1.0
-        ops.reshape_and_cache(k, v, k_cache, v_cache, meta.slot_mapping,
-                              1.0 / ks, 1.0 / vs)
+        ops.rope_qk_norm_cache_(
+            q, k, v, meta.positions, cos_sin, k_cache, v_cache,
+            meta.slot_mapping, self.num_heads, self.q_norm_weight,
+            self.k_norm_weight, self.eps, 1.0 / ks, 1.0 / vs,
+        )
         # K's dequant scale folds EXACTLY into the softmax scalar:
         # scale*(Q . ks*K8) == (scale*ks)*(Q . K8); V's is a linear
         # post-multiply on the attention output (applied below).
@@ -105,7 +103,7 @@ class Attention(nn.Module):
         if np_ > 0:
             # context attention over the paged cache (the new tokens' K/V
             # were just written above); cached prefixes are never recomputed
-            o = ops.prefill_attention_paged(
+            ops.prefill_attention_paged(
                 q[:np_].view(np_, self.num_heads, self.head_dim),
                 k_cache,
                 v_cache,
@@ -116,18 +114,18 @@ class Attention(nn.Module):
                 tile_seq=meta.tile_seq,
                 tile_row0=meta.tile_row0,
                 tile_rows=meta.tile_rows or None,
+                out=out[:np_].view(np_, self.num_heads, self.head_dim),
             )
-            out[:np_] = o.view(np_, self.q_size)
         if nd > 0:
-            o = ops.paged_attention_decode(
+            ops.paged_attention_decode(
                 q[np_:].view(nd, self.num_heads, self.head_dim),
                 k_cache,
                 v_cache,
                 meta.block_tables,
                 meta.seq_lens,
                 scale,
+                out=out[np_:].view(nd, self.num_heads, self.head_dim),
             )
-            out[np_:] = o.view(nd, self.q_size)
         if vs != 1.0:
             out *= vs
         if meta.lora is not None:

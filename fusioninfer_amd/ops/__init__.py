@@ -206,6 +206,28 @@ def rope_qk_norm_(
     return q, k
 
 
+def rope_qk_norm_cache_(q, k, v, positions, cos_sin, k_cache, v_cache,
+                        slot_mapping, num_q_heads: int,
+                        q_weight: Optional[torch.Tensor] = None,
+                        k_weight: Optional[torch.Tensor] = None,
+                        eps: float = 1e-6, k_inv_scale: float = 1.0,
+                        v_inv_scale: float = 1.0):
+    """rope_qk_norm_ followed by reshape_and_cache, in one kernel on the
+    GPU, where K's result is then in the cache alone (k is left as it is).
+    Returns q."""
+    if q.is_cuda:
+        _require_native()
+        _C.rope_qk_norm_cache(q, k, v, q_weight, k_weight, cos_sin, positions,
+                              k_cache, v_cache, slot_mapping, num_q_heads,
+                              eps, k_inv_scale, v_inv_scale)
+        return q
+    rope_qk_norm_(q, k, positions, cos_sin, num_q_heads, k_cache.shape[1],
+                  k_cache.shape[3], q_weight, k_weight, eps)
+    reshape_and_cache(k, v, k_cache, v_cache, slot_mapping, k_inv_scale,
+                      v_inv_scale)
+    return q
+
+
 # ---------------------------------------------------------------- kv cache
 
 def reshape_and_cache(k, v, k_cache, v_cache, slot_mapping,
@@ -255,16 +277,19 @@ def paged_attention_decode(
     block_tables: torch.Tensor,  # [S, max_blocks] int32
     seq_lens: torch.Tensor,      # [S] int32
     scale: Optional[float] = None,
+    out: Optional[torch.Tensor] = None,  # [S, Hq, D] contiguous
 ) -> torch.Tensor:
     if scale is None:
         scale = 1.0 / math.sqrt(q.shape[-1])
     if q.is_cuda:
         _require_native()
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+        if out is None:
+            out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
         _C.paged_attention_decode(out, q, k_cache, v_cache, block_tables,
                                   seq_lens, scale)
         return out
-    return ref.paged_attention_decode(q, k_cache, v_cache, block_tables, seq_lens, scale)
+    o = ref.paged_attention_decode(q, k_cache, v_cache, block_tables, seq_lens, scale)
+    return o if out is None else out.copy_(o)
 
 
 # rows per entry of the prefill tile table (128 or 256); the kernel cuts
@@ -340,6 +365,7 @@ def prefill_attention_paged(
     tile_seq: Optional[torch.Tensor] = None,
     tile_row0: Optional[torch.Tensor] = None,
     tile_rows: Optional[int] = None,
+    out: Optional[torch.Tensor] = None,  # [Tnew, Hq, D] contiguous
 ) -> torch.Tensor:
     """Context attention: new tokens attend over the paged cache (their own
     K/V must already be written via reshape_and_cache)."""
@@ -353,16 +379,18 @@ def prefill_attention_paged(
             tile_seq, tile_row0 = build_prefill_tiles(
                 lens, device=q.device, rows=tile_rows
             )
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+        if out is None:
+            out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
         _C.prefill_attention_paged(
             out, q, k_cache, v_cache, tile_seq, tile_row0, cu_seqlens_q,
             block_tables, seq_lens_k, scale,
             tile_rows or PREFILL_TILE_ROWS,
         )
         return out
-    return ref.prefill_attention_paged(
+    o = ref.prefill_attention_paged(
         q, k_cache, v_cache, block_tables, cu_seqlens_q, seq_lens_k, scale
     )
+    return o if out is None else out.copy_(o)
 
 
 # ---------------------------------------------------------------- MoE

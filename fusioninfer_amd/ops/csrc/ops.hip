@@ -16,9 +16,10 @@ void launch_silu_and_mul(u16*, const u16*, int64_t, int, hipStream_t);
 template <bool SILU_MUL>
 void launch_row_quant_fp8(unsigned char*, float*, const u16*, int, int,
                           hipStream_t);
-void launch_rope_qk_norm(u16*, u16*, int64_t, int64_t, const u16*, const u16*,
-                         const float*, const int*, int, int, int, int, float,
-                         hipStream_t);
+void launch_rope_qk_norm(u16*, u16*, const u16*, int64_t, int64_t, int64_t,
+                         const u16*, const u16*, const float*, const int*, int,
+                         int, int, int, float, void*, void*, const int*, int,
+                         bool, float, float, hipStream_t);
 void launch_reshape_and_cache(const u16*, const u16*, void*, void*,
                               const int*, int64_t, int64_t, int, int, int,
                               int, bool, float, float, hipStream_t);
@@ -176,13 +177,57 @@ void rope_qk_norm(at::Tensor q, at::Tensor k,
   // q/k may be row-strided slices of the fused qkv projection output
   TORCH_CHECK(q.dim() == 2 && k.dim() == 2);
   TORCH_CHECK(q.stride(1) == 1 && k.stride(1) == 1);
+  TORCH_CHECK(head_dim == 64 || head_dim == 128,
+              "rope: heads of 64 or 128 values");
   const int tokens = q.size(0);
   fi::launch_rope_qk_norm(
-      bf16_ptr(q), bf16_ptr(k), q.stride(0), k.stride(0),
+      bf16_ptr(q), bf16_ptr(k), nullptr, q.stride(0), k.stride(0), 0,
       q_weight ? bf16_cptr(*q_weight) : nullptr,
       k_weight ? bf16_cptr(*k_weight) : nullptr, cos_sin.data_ptr<float>(),
       positions.data_ptr<int>(), tokens, num_q_heads, num_kv_heads, head_dim,
-      static_cast<float>(eps), current_stream());
+      static_cast<float>(eps), nullptr, nullptr, nullptr, 1, false, 1.f, 1.f,
+      current_stream());
+}
+
+// rope_qk_norm of q in place; k's result and v go to the paged cache alone
+void rope_qk_norm_cache(at::Tensor q, at::Tensor k, at::Tensor v,
+                        c10::optional<at::Tensor> q_weight,
+                        c10::optional<at::Tensor> k_weight,
+                        at::Tensor cos_sin, at::Tensor positions,
+                        at::Tensor k_cache, at::Tensor v_cache,
+                        at::Tensor slot_mapping, int64_t num_q_heads,
+                        double eps, double k_inv_scale, double v_inv_scale) {
+  CHECK_BF16_CUDA(q);
+  CHECK_BF16_CUDA(k);
+  CHECK_BF16_CUDA(v);
+  const bool fp8 = cache_is_fp8(k_cache);
+  TORCH_CHECK(cos_sin.scalar_type() == at::kFloat && cos_sin.is_cuda());
+  TORCH_CHECK(positions.scalar_type() == at::kInt && positions.is_cuda());
+  TORCH_CHECK(slot_mapping.scalar_type() == at::kInt &&
+              slot_mapping.is_cuda());
+  TORCH_CHECK(q.dim() == 2 && k.dim() == 2 && v.dim() == 2);
+  TORCH_CHECK(q.stride(1) == 1 && k.stride(1) == 1 && v.stride(1) == 1);
+  const int tokens = q.size(0);
+  const int kv_heads = k_cache.size(1), head_dim = k_cache.size(3);
+  TORCH_CHECK(head_dim == 64 || head_dim == 128,
+              "rope: heads of 64 or 128 values");
+  TORCH_CHECK(q.size(1) == num_q_heads * head_dim &&
+              k.size(1) == kv_heads * head_dim && v.size(1) == k.size(1) &&
+              k.size(0) == tokens && v.size(0) == tokens &&
+              positions.numel() >= tokens && slot_mapping.numel() >= tokens &&
+              cos_sin.size(-1) == head_dim);
+  TORCH_CHECK(k_cache.is_contiguous() && v_cache.is_contiguous() &&
+              v_cache.sizes() == k_cache.sizes() &&
+              v_cache.scalar_type() == k_cache.scalar_type());
+  fi::launch_rope_qk_norm(
+      bf16_ptr(q), bf16_ptr(k), bf16_cptr(v), q.stride(0), k.stride(0),
+      v.stride(0), q_weight ? bf16_cptr(*q_weight) : nullptr,
+      k_weight ? bf16_cptr(*k_weight) : nullptr, cos_sin.data_ptr<float>(),
+      positions.data_ptr<int>(), tokens, num_q_heads, kv_heads, head_dim,
+      static_cast<float>(eps), k_cache.data_ptr(), v_cache.data_ptr(),
+      slot_mapping.data_ptr<int>(), k_cache.size(2), fp8,
+      static_cast<float>(k_inv_scale), static_cast<float>(v_inv_scale),
+      current_stream());
 }
 
 void reshape_and_cache(at::Tensor k, at::Tensor v, at::Tensor k_cache,
@@ -247,6 +292,7 @@ void paged_attention_decode(at::Tensor out, at::Tensor q, at::Tensor k_cache,
   TORCH_CHECK(seq_lens.scalar_type() == at::kInt);
   seq_lens = seq_lens.contiguous();
   TORCH_CHECK(q.dim() == 3);  // [S, Hq, D], rows may be strided
+  TORCH_CHECK(out.is_contiguous() && out.sizes() == q.sizes());
   const int num_seqs = q.size(0);
   const int num_heads = q.size(1);
   const int head_dim = q.size(2);
@@ -329,6 +375,7 @@ void prefill_attention_paged(at::Tensor out, at::Tensor q, at::Tensor k_cache,
               seq_lens_k.scalar_type() == at::kInt);
   TORCH_CHECK(block_tables.is_contiguous());
   TORCH_CHECK(q.dim() == 3);
+  TORCH_CHECK(out.is_contiguous() && out.sizes() == q.sizes());
   const int num_q_heads = q.size(1);
   const int head_dim = q.size(2);
   const int num_kv_heads = k_cache.size(1);
@@ -394,6 +441,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("quant_fp8_rows", &quant_fp8_rows, "per-row dynamic fp8 quant");
   m.def("rope_qk_norm", &rope_qk_norm,
         "fused per-head qk RMSNorm + NeoX RoPE (in-place)");
+  m.def("rope_qk_norm_cache", &rope_qk_norm_cache,
+        "rope_qk_norm with K and V scattered into the paged cache");
   m.def("reshape_and_cache", &reshape_and_cache, "scatter K/V into paged cache");
   m.def("gather_kv_blocks", &gather_kv_blocks, "pack KV blocks for PD send");
   m.def("scatter_kv_blocks", &scatter_kv_blocks, "unpack KV blocks from PD recv");

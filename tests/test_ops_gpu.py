@@ -157,6 +157,44 @@ def test_reshape_and_cache():
     torch.testing.assert_close(v_cache.cpu(), v_ref)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("T,Hq,Hk,D,pad", [
+    (1, 16, 8, 128, 0),
+    (33, 8, 2, 64, 8),    # a wave's last heads are missing
+    (130, 5, 1, 128, 1),  # odd heads; rows at any address
+    (7, 1, 1, 64, 3),
+])
+def test_rope_qk_norm_cache(T, Hq, Hk, D, pad, fp8):
+    """One kernel against the two it stands for: q, both caches, bit for bit
+    what rope_qk_norm_ and reshape_and_cache leave, rows of negative slots
+    left out."""
+    torch.manual_seed(2)
+    qkv = torch.randn(T, (Hq + 2 * Hk) * D + pad, device=DEV,
+                      dtype=torch.bfloat16)[:, pad:]
+    cos_sin = ops.compute_cos_sin_cache(D, 512, 10000.0).to(DEV)
+    positions = torch.randint(0, 512, (T,), dtype=torch.int32, device=DEV)
+    qw = torch.randn(D, dtype=torch.bfloat16, device=DEV)
+    slots = torch.randperm(160, device=DEV)[:T].to(torch.int32)
+    if T > 2:
+        slots[1] = -1
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    caches = [torch.zeros(10, Hk, 16, D, device=DEV).to(dt)
+              for _ in range(4)]
+    cut = lambda t: (t[:, :Hq * D], t[:, Hq * D:(Hq + Hk) * D],
+                     t[:, (Hq + Hk) * D:])
+    q, k, v = cut(qkv.clone())
+    ops.rope_qk_norm_(q, k, positions, cos_sin, Hq, Hk, D, qw, None)
+    ops.reshape_and_cache(k.contiguous(), v.contiguous(), *caches[:2], slots,
+                          1 / 3., 1 / 4.)
+    got, k0, v0 = cut(qkv)
+    ops.rope_qk_norm_cache_(got, k0, v0, positions, cos_sin, *caches[2:],
+                            slots, Hq, qw, None, 1e-6, 1 / 3., 1 / 4.)
+    assert torch.equal(got, q)
+    for a, b in zip(caches[:2], caches[2:]):
+        assert a.float().abs().sum() > 0
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
 def test_kv_block_gather_scatter_roundtrip():
     Hk, D, bs, nblocks = 2, 128, 16, 20
     k_cache = torch.randn(nblocks, Hk, bs, D, dtype=torch.bfloat16, device=DEV)
