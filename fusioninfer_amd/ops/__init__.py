@@ -72,23 +72,53 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
 
 # ---------------------------------------------------------------- linear
 
-SKINNY_ROWS = 16  # rows of x up to which the streaming kernel serves a GEMM
+SKINNY_ROWS = 16  # rows of x up to which a GEMM always streams W
+PART_ROWS = 256   # and up to which it does for the sizes below
 
 
-def _skinny_ok(x, w, unit: int) -> bool:
-    """Whether x W^T can run on the streaming kernel: few bf16 rows, whole
+def _streams(M: int, N: int, K: int, silu_mul: bool = False) -> bool:
+    """Whether the streaming kernels beat the library's GEMM for x [M, K],
+    W [N, K]. Up to 16 rows they always do. Above, the library is as good or
+    better where its tiles fill the chip by themselves, and loses where N is
+    too small for that or W too large to be read at 4.3 TB/s. Library / here
+    in us: 6144 x 4096 at 17, 64, 128, 256 rows 14.6 / 13.7, 17.8 / 17.6,
+    25.3 / 22.9, 39.7 / 28.8; 4096 x 4096 12.8 / 11.0, 14.7 / 13.8, 23.7 /
+    18.3, 22.0 / 22.8; 4096 x 12288 23.6 / 20.8, 36.7 / 26.1, 66 / 33, 53 /
+    45; 5120 x 2048 12.5 / 9.7, 12.9 / 12.4, 15.2 / 16.2; 8192 x 4096 15.7 /
+    19.1, 18.6 / 22.0, 26.3 / 27.6; 28672 x 4096 54 / 41, 51 / 40, 54 / 65;
+    51200 x 5120 94 / 87, 99 / 115, 110 / 134; 151936 x 4096 255 / 201, 262 /
+    238, 279 / 266, 350 / 391; 2048 x 2048 8.2 / 8.4, 8.9 / 11.8. With
+    silu_mul the pass over the product goes (5 us of 24576 x 4096: 50 / 36,
+    51 / 39, 55 / 45, 67 / 63): taken where tiles of 96 rows fill the chip
+    once."""
+    if M <= SKINNY_ROWS:
+        return True
+    if M > PART_ROWS or N * K < 1 << 23:
+        return False
+    if M <= 64:
+        return not (6144 < N < 9216
+                    or M > 32 and 32768 < N < 1 << 17)
+    if N >= 1 << 17:
+        return M <= 128
+    return K >= 4096 and (3072 <= N <= 6144
+                          or silu_mul and 224 < -(-N // 96) <= 256)
+
+
+def _skinny_ok(x, w, unit: int, silu_mul: bool = False) -> bool:
+    """Whether x W^T can run on the streaming kernels: few bf16 rows, whole
     128-value stages of K, whole tiles of N, 16-byte aligned rows, nothing
     to differentiate. A family that builds only its own extension keeps the
     library's GEMM."""
     return (
         _C is not None and x.is_cuda and w.is_cuda and x.dim() == 2 and w.dim() == 2
         and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
-        and 1 <= x.shape[0] <= SKINNY_ROWS
+        and 1 <= x.shape[0] <= PART_ROWS
         and x.shape[1] == w.shape[1] and 0 < x.shape[1] <= 1 << 24
         and x.shape[1] % 128 == 0
         and 0 < w.shape[0] <= 1 << 24 and w.shape[0] % unit == 0
         and x.stride(1) == 1 and x.stride(0) % 8 == 0
-        and x.stride(0) <= 1 << 24
+        and x.stride(0) <= 1 << (24 if x.shape[0] <= SKINNY_ROWS else 22)
+        and _streams(x.shape[0], w.shape[0], x.shape[1], silu_mul)
         and w.is_contiguous()
         and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
         and not (torch.is_grad_enabled()
@@ -98,15 +128,14 @@ def _skinny_ok(x, w, unit: int) -> bool:
 
 def linear(x: torch.Tensor, w: torch.Tensor,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """x W^T (+ bias): up to SKINNY_ROWS bf16 rows stream W once through the
-    skinny kernel (1.1 to 2 times the library's speed there, see its notes),
-    anything else is the library's GEMM."""
+    """x W^T (+ bias): a few bf16 rows stream W once through the kernels for
+    that, anything else is the library's GEMM."""
     if _skinny_ok(x, w, 16) and (bias is None or (
             bias.dtype == torch.bfloat16 and bias.is_contiguous()
             and not (torch.is_grad_enabled() and bias.requires_grad))):
         out = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype,
                           device=x.device)
-        _C.skinny_gemm(out, x, w, bias, False)
+        _C.few_rows_gemm(out, x, w, bias, False)
         return out
     return torch.nn.functional.linear(x, w, bias)
 
@@ -114,10 +143,10 @@ def linear(x: torch.Tensor, w: torch.Tensor,
 def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x G^T) * (x U^T) with w = [G; U]; few rows in one kernel, whose
     gate and up values are not rounded in between."""
-    if _skinny_ok(x, w, 32):
+    if _skinny_ok(x, w, 32, True):
         out = torch.empty((x.shape[0], w.shape[0] // 2), dtype=x.dtype,
                           device=x.device)
-        _C.skinny_gemm(out, x, w, None, True)
+        _C.few_rows_gemm(out, x, w, None, True)
         return out
     return silu_and_mul(linear(x, w))
 

@@ -33,7 +33,7 @@ SOURCES = [
     "cache.hip",
     "paged_attention.hip",
     "prefill_attention.hip",
-    "skinny_gemm.hip",
+    "skinny_gemm.hip", "part_gemm.hip",
 ]
 
 MOE_SOURCES = [

@@ -40,6 +40,9 @@ void launch_prefill_attn(u16*, const u16*, const void*, const void*,
                          hipStream_t);
 void launch_skinny_gemm(u16*, const u16*, const u16*, const u16*, int, int,
                         int, int64_t, int64_t, bool, hipStream_t);
+int64_t part_gemm_floats(int, int, int);
+void launch_part_gemm(u16*, float*, const u16*, const u16*, const u16*, int,
+                      int, int, int64_t, int64_t, bool, hipStream_t);
 
 }  // namespace fi
 
@@ -396,20 +399,20 @@ void prefill_attention_paged(at::Tensor out, at::Tensor q, at::Tensor k_cache,
 }
 
 // out [M, N] (silu_mul: [M, N / 2]) = x [M, K] @ w [N, K]^T (+ bias)
-void skinny_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
+void few_rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
                  c10::optional<at::Tensor> bias, bool silu_mul) {
   CHECK_BF16_CUDA(out);
   CHECK_BF16_CUDA(x);
   CHECK_BF16_CUDA(w);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2);
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
-  TORCH_CHECK(M >= 1 && M <= 16 && w.size(1) == K && K % 128 == 0 &&
+  TORCH_CHECK(M >= 1 && M <= 256 && w.size(1) == K && K % 128 == 0 &&
                   K > 0 && N > 0 && N % (silu_mul ? 32 : 16) == 0 &&
                   K <= (1 << 24) && N <= (1 << 24),
-              "skinny_gemm: unsupported sizes");
+              "few_rows_gemm: unsupported sizes");
   TORCH_CHECK(out.size(0) == M && out.size(1) == (silu_mul ? N / 2 : N));
   TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % 8 == 0 &&
-              x.stride(0) <= (1 << 24) && w.is_contiguous() &&
+              x.stride(0) <= (1 << (M <= 16 ? 24 : 22)) && w.is_contiguous() &&
               out.stride(1) == 1 && out.stride(0) % 4 == 0);
   TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
               reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 &&
@@ -421,9 +424,17 @@ void skinny_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
                 bias->is_contiguous() && bias->numel() == N);
     b = bf16_cptr(*bias);
   }
-  fi::launch_skinny_gemm(bf16_ptr(out), bf16_cptr(x), bf16_cptr(w), b, M, N,
-                         K, x.stride(0), out.stride(0), silu_mul,
-                         current_stream());
+  if (M <= 16) {
+    fi::launch_skinny_gemm(bf16_ptr(out), bf16_cptr(x), bf16_cptr(w), b, M, N,
+                           K, x.stride(0), out.stride(0), silu_mul,
+                           current_stream());
+    return;
+  }
+  at::Tensor pieces = at::empty({fi::part_gemm_floats(M, N, K)},
+                                x.options().dtype(at::kFloat));
+  fi::launch_part_gemm(bf16_ptr(out), pieces.data_ptr<float>(), bf16_cptr(x),
+                       bf16_cptr(w), b, M, N, K, x.stride(0), out.stride(0),
+                       silu_mul, current_stream());
 }
 
 }  // namespace
@@ -446,7 +457,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("reshape_and_cache", &reshape_and_cache, "scatter K/V into paged cache");
   m.def("gather_kv_blocks", &gather_kv_blocks, "pack KV blocks for PD send");
   m.def("scatter_kv_blocks", &scatter_kv_blocks, "unpack KV blocks from PD recv");
-  m.def("skinny_gemm", &skinny_gemm, "x W^T for up to 16 rows of x");
+  m.def("few_rows_gemm", &few_rows_gemm, "x W^T for up to 256 rows of x");
   m.def("paged_attention_decode", &paged_attention_decode,
         "paged decode attention");
   m.def("prefill_attention", &prefill_attention, "varlen causal MFMA prefill");

@@ -882,6 +882,51 @@ def test_skinny_linear(rows, n, k, bias):
         assert (err <= want.abs() * 2 ** -8 + 1e-3 * k ** 0.5).all()
 
 
+@pytest.mark.parametrize("rows", [17, 32, 33, 64, 65, 128, 129, 256])
+@pytest.mark.parametrize("n,k,bias", [
+    (16, 128, True),        # one ragged tile, one or two stages
+    (224, 384, False),      # fewer stages than workgroups; odd tiles
+    (4128, 2560, True),     # cut tiles, a ragged last one, several pieces
+    (288, 16384, False),    # a tile in many pieces
+    (24608, 256, False),    # whole tiles and one more
+])
+def test_linear_in_parts(rows, n, k, bias):
+    """17 to 256 rows against a float64 product; one bf16 rounding of the
+    result (2^-9 relative) and fp32 sums of k products."""
+    g = torch.Generator().manual_seed(n + k + rows)
+    w = torch.randn(n, k, generator=g).to(torch.bfloat16).to(DEV)
+    b = torch.randn(n, generator=g).to(torch.bfloat16).to(DEV) if bias \
+        else None
+    x = torch.randn(rows, 2 * k, generator=g).to(torch.bfloat16).to(DEV)[:, k:]
+    out = torch.empty(rows, n, dtype=torch.bfloat16, device=DEV)
+    ops._C.few_rows_gemm(out, x, w, b, False)
+    prod = x.double() @ w.double().T
+    want = prod + (0.0 if b is None else b.double())
+    assert ((out.double() - want).abs()
+            <= want.abs() * 2 ** -8 + 1e-4 * k ** 0.5).all()
+    if n % 32 == 0 and not bias:
+        out = torch.empty(rows, n // 2, dtype=torch.bfloat16, device=DEV)
+        ops._C.few_rows_gemm(out, x, w, None, True)
+        want = torch.nn.functional.silu(prod[:, : n // 2]) * prod[:, n // 2:]
+        assert ((out.double() - want).abs()
+                <= want.abs() * 2 ** -8 + 1e-3 * k ** 0.5).all()
+
+
+def test_linear_takes_parts_by_size():
+    """The sizes that stream and those that stay with the library give the
+    same product."""
+    for rows, n, k, streams in [(48, 4096, 4096, True), (48, 64, 256, False),
+                                (48, 8192, 1024, False),
+                                (200, 5120, 4096, True),
+                                (200, 2048, 4096, False)]:
+        x = torch.randn(rows, k, device=DEV).to(torch.bfloat16)
+        w = torch.randn(n, k, device=DEV).to(torch.bfloat16)
+        assert ops._skinny_ok(x, w, 16) == streams
+        want = x.double() @ w.double().T
+        assert ((ops.linear(x, w).double() - want).abs()
+                <= want.abs() * 2 ** -8 + 1e-4 * k ** 0.5).all()
+
+
 def test_skinny_linear_leaves_other_calls_to_the_library():
     """Row counts, types, strides and sizes that the kernel does not take
     give what torch gives; gradients still flow."""
