@@ -668,9 +668,8 @@ class RoutedExperts(nn.Module):
             return out.to(x.dtype)
         E = self.experts
         fast = self._mfma_fits()
-        block_m = 16
-        if fast and T * self.top >= 64 * E:
-            block_m = 128
+        block_m = ops.moe_block_rows(T * self.top, E, self.ff,
+                                     self.width) if fast else 16
         sorted_ids, expert_ids, n_valid, pos, PM = ops.moe_align(
             topi, 0, E, block_m)
         act = torch.empty(PM, self.ff, dtype=x.dtype, device=x.device)

@@ -547,14 +547,14 @@ class MoEMLP(nn.Module):
         else:
             topv, topi = self._router_topk(
                 x.float() @ self.router_weight.float().T)
-        # block_m: 16 in the few-rows-per-expert (decode) regime, 128 when
-        # segments are long enough for the 4x in-register B-reuse variant
-        block_m = 128 if T * self.top_k >= 64 * E_local else 16
+        inter = self.gate_up_t.shape[2] // 2
+        # of the assignments, those that land on this rank's experts
+        block_m = ops.moe_block_rows(
+            T * self.top_k * E_local // self.num_experts, E_local, inter, H)
         sorted_ids, expert_ids, n_valid, pos, PM = self._moe_align(
             topi, block_m
         )
         gu_packed, dn_packed = self._packed_weights()
-        inter = self.gate_up_t.shape[2] // 2
         act = torch.empty(PM, inter, dtype=x.dtype, device=x.device)
         ops.moe_gemm(act, x, gu_packed, sorted_ids, expert_ids, n_valid,
                      block_m, gate_up=True)

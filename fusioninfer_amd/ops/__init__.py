@@ -537,6 +537,25 @@ def moe_gemm_fp8(out, a, a_scales, b_packed, b_scales, sorted_ids,
                             gate_up)
 
 
+def moe_block_rows(assignments: int, experts: int, ff: int,
+                   width: int) -> int:
+    """Rows per block of the grouped bf16 GEMMs. Blocks of 16 stream the
+    weights once per block, blocks of 128 are bound by the matrix cores at
+    several times the work: they win as soon as experts take up two small
+    blocks, if there are column tiles of 128 enough for every CU. gate_up +
+    down with 16 / 128 rows, us: 128 experts of 2048 x 768, 8, 16, 24, 62
+    rows each on average 200 / 268, 281 / 266, 405 / 266, 870 / 267; 8
+    experts of 2048 x 3072, 16 and 32 rows 77 / 91, 120 / 92; 16 of 1536 x
+    512, 16 and 32 rows 26 / 41, 40 / 41."""
+    if assignments >= 64 * experts:
+        return 128
+    if width % 128 or ff % 64:
+        return 16
+    if experts * -(-ff // 128) >= 256:
+        return 128 if assignments > 16 * experts else 16
+    return 128 if assignments >= 32 * experts else 16
+
+
 def moe_align(topi: torch.Tensor, e_start: int, e_end: int, block_m: int):
     """Single-kernel device-side block alignment of expert assignments
     (GPU only; MoEMLP._moe_align's torch composition is the CPU

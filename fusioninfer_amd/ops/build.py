@@ -41,7 +41,7 @@ MOE_SOURCES = [
     "moe_gemm.hip",
     "moe_tile.hip",
     "moe_plain.hip",
-    "moe_router.hip",
+    "moe_router.hip", "moe_stream.hip",
 ]
 
 

@@ -964,11 +964,36 @@ def test_skinny_linear_leaves_other_calls_to_the_library():
     (640, False, None),        # two and a half column tiles
 ])
 def test_moe_gemm_row_blocks_of_128(k, n, gate_up, act):
+    check_moe_gemm(k, n, gate_up, act, 128)
+
+
+@pytest.mark.parametrize("k", [32, 224, 512, 768, 1024, 2080, 2624])
+@pytest.mark.parametrize("n,gate_up,act", [
+    (64, True, None), (320, True, "clamped_glu"), (192, False, "relu_sq"),
+    (128, False, None),
+])
+def test_moe_gemm_row_blocks_of_16(k, n, gate_up, act):
+    """Waves with no step, two, three, four and eight steps of K, more than
+    one stretch with a remainder."""
+    check_moe_gemm(k, n, gate_up, act, 16)
+
+
+def test_moe_block_rows():
+    """Small blocks where 128 rows have no kernel; as before from 64 rows
+    per expert on."""
+    assert ops.moe_block_rows(63 * 8, 8, 96, 2048) == 16
+    assert ops.moe_block_rows(63 * 8, 8, 128, 64) == 16
+    assert ops.moe_block_rows(64 * 8, 8, 96, 64) == 128
+    assert ops.moe_block_rows(512, 128, 768, 2048) == 16
+    assert ops.moe_block_rows(4096, 128, 768, 2048) == 128
+
+
+def check_moe_gemm(k, n, gate_up, act, bm):
     """Experts with no row, one row, a whole block, a block and one row and
     many, against float64 products; one bf16 rounding of the result (2^-9)
     and fp32 sums of k products of unit variance."""
     g = torch.Generator().manual_seed(k + n)
-    T, top, bm = 700, 2, 128
+    T, top = 700, 2
     sizes = [0, 1, 128, 129, 300, 0, 842]   # assignments, 2 T in all
     experts = torch.cat([torch.full((c,), e) for e, c in enumerate(sizes)])
     topi = experts[torch.randperm(T * top, generator=g)].view(T, top)
