@@ -65,9 +65,9 @@ SEQMIX_SOURCES = [
 ]
 
 EXTENSIONS = {
-    "core": ("_C", SOURCES, ["common.h"]),
+    "core": ("_C", SOURCES, ["common.h", "prefill_kernel.h"]),
     "seqmix": ("_C_seqmix", SEQMIX_SOURCES, ["common.h", "seqmix.h", "seqmix_bind.h",
-                "seqmix_hyper.h", "seqmix_scan.h"]),
+                "seqmix_hyper.h", "seqmix_scan.h", "prefill_kernel.h"]),
     "moe": ("_C_moe", MOE_SOURCES, ["common.h", "seqmix.h"]),
 }
 

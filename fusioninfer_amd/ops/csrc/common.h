@@ -135,6 +135,19 @@ FI_DEV void dma_to_lds16(u32 lds, const void* base, u32 offset) {
 #endif
 }
 
+// the same with an address of its own per lane
+FI_DEV void dma_to_lds16_at(u32 lds, const void* from) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 4\n\t"
+      "global_load_lds_dwordx4 %1, off"
+      :
+      : "s"(lds), "v"(from)
+      : "memory");
+#endif
+}
+
 // the same for data that is read once: it leaves the caches first
 FI_DEV void dma_to_lds16_nt(u32 lds, const void* base, u32 offset) {
 #if defined(__HIP_DEVICE_COMPILE__)

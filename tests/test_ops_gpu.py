@@ -1025,3 +1025,54 @@ def check_moe_gemm(k, n, gate_up, act, bm):
             slack *= 20 * k ** 0.5
         err = (out[at].double() - y).abs()
         assert (err <= y.abs() * 2 ** -8 + slack).all(), m
+
+
+# --------------------------- attention with sink, gate and window, bf16 rows
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("heads,groups,block,window,keep,gate", [
+    (4, 1, 16, 0, 0, None),
+    (8, 1, 1, 0, 0, "head"),       # rows of their own blocks
+    (6, 3, 16, 64, 0, "entry"),    # window of a tile: nothing kept
+    (3, 3, 8, 100, 70, "head"),    # kept keys beyond the first tile
+    (2, 2, 1, 33, 5, "entry"),
+    (5, 1, 16, 300, 1, None),      # window wider than some contexts
+])
+def test_sink_attention_row_tiles(D, heads, groups, block, window, keep,
+                                  gate):
+    """Portions of 1, 32, 129 and 300 rows, some behind cached keys, against
+    the fp32 reference on the same bf16 values. Weights and results are
+    rounded once to bf16 each: at most 2^-8 of the largest value."""
+    from fusioninfer_amd.ops import seqmix
+
+    g = torch.Generator().manual_seed(D + heads + window)
+    new, past = [1, 32, 129, 300], [40, 0, 277, 64]
+    ctx = [a + b for a, b in zip(new, past)]
+    need = [-(-c // block) for c in ctx]
+    order = torch.randperm(sum(need) + 2, generator=g)
+    table = torch.zeros(len(new), max(need), dtype=torch.int32)
+    for i, n in enumerate(need):
+        table[i, :n] = order[sum(need[:i]):sum(need[:i + 1])]
+    T = sum(new)
+    q = torch.randn(T, heads, D, generator=g).bfloat16()
+    k = torch.randn(len(order), groups, block, D, generator=g).bfloat16()
+    v = torch.randn(len(order), groups, block, D, generator=g).bfloat16()
+    sink = torch.randn(heads, generator=g) * 3
+    og = {"head": torch.randn(T, heads, generator=g).bfloat16(),
+          "entry": torch.randn(T, heads * D, generator=g).bfloat16()}.get(gate)
+    cu = torch.tensor([0, *torch.tensor(new).cumsum(0)], dtype=torch.int32)
+    rows = torch.cat([torch.full((n,), i) for i, n in enumerate(new)]).int()
+    pos = torch.cat([torch.arange(p, p + n) for n, p in zip(new, past)]).int()
+    want = seqmix.sink_paged_attention(
+        q.float(), k.float(), v.float(), table, rows, pos, D ** -0.5,
+        sink=sink, out_gate=None if og is None else og.float(), seq_cu=cu,
+        window=window, keep_first=keep)
+    dev = lambda t: None if t is None else t.to(DEV)
+    got = seqmix.sink_paged_attention(
+        dev(q), dev(k), dev(v), dev(table), dev(rows), dev(pos), D ** -0.5,
+        sink=dev(sink), out_gate=dev(og), seq_cu=dev(cu),
+        tiles=seqmix.build_attention_tiles(new, device=DEV), window=window,
+        keep_first=keep)
+    err = (got.cpu().float() - want.view(got.shape)).abs().max()
+    assert err <= 2 ** -8 * v.float().abs().max()
