@@ -134,8 +134,8 @@ template <typename A>
 void launch_sink_attention_rows(A*, float*, float*, const A*, const A*,
                                 const A*, int, const int*, int, const int*,
                                 const int*, const float*, const A*, int64_t,
-                                int, int, int, int, int, int, int, int, float,
-                                int, int, int, hipStream_t);
+                                int, int, int, int, int, int, int, int,
+                                int64_t, float, int, int, int, hipStream_t);
 template <typename A>
 void launch_pair_embed(float*, A*, const int64_t*, const A*, float, const A*,
                        int64_t, int64_t, int64_t, int*, const int*,
@@ -973,7 +973,7 @@ void sink_paged_attention(at::Tensor out, at::Tensor q, at::Tensor k_cache,
                         row_seq.data_ptr<int>(), positions.data_ptr<int>(),
                         sp, reinterpret_cast<const A*>(gp), g_stride,
                         gate_elem, row0, rows, H, G, DK, (int)DV, bs,
-                        (float)scale, ns, (int)window, (int)keep_first,
+                        k_cache.numel() / DK, (float)scale, ns, (int)window, (int)keep_first,
                         stream()));
   }
 }

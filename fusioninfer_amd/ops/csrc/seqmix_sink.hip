@@ -15,6 +15,9 @@
 //    kernel, which also adds the sink to the denominator, applies the
 //    gate and rounds. Decoded rows use it, and prompt rows whose sizes
 //    the tiled form does not cover.
+//  * split form on the matrix cores (bf16, the sizes of FI_SPAN): up to 16
+//    heads, the span's keys straight into fragments and its values into LDS
+//    at once, so that a span costs one trip to memory.
 //  * tiled MFMA form: a 4-wave workgroup takes 64*QS consecutive rows of
 //    one (sequence, head) and walks the keys 0..last row's position in
 //    LDS-staged tiles; S^T = K Q^T and O^T = V^T P^T run on the matrix
@@ -229,6 +232,190 @@ __global__ __launch_bounds__(256) void sink_attention_split_kernel(
   }
 }
 
+typedef __attribute__((ext_vector_type(4))) float floatx4;
+typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
+
+// The same span by four waves of 64 keys each. Bound by latency: a decode
+// step has a few hundred spans of 64 KB. 4 rows of 1.8 thousand keys: 28 us
+// by the form above with its chain of dependent loads, 9 here.
+//  * S^T = K Q^T, A = K read in fragment order from the cache, B = Q: a lane
+//    ends with four keys of one head, again and again 16 keys on.
+//  * O^T = V^T P^T, A = V^T by the transposing LDS read. The keys of a
+//    32-deep step are taken in the order in which the lanes hold them. The
+//    weights stay what fp32 holds: three bf16 terms each, exact products,
+//    fp32 sums.
+template <int DK, int DV>
+__global__ __launch_bounds__(256) void sink_attention_span_kernel(
+    float* __restrict__ part_ml,      // [rows, H, ns, 2]
+    float* __restrict__ part_o,       // [rows, H, ns, DV]
+    const u16* __restrict__ q,        // [T, H, DK]
+    const u16* __restrict__ k_cache, const u16* __restrict__ v_cache,
+    int v_row, const int* __restrict__ seq_bt, int bt_stride,
+    const int* __restrict__ row_seq, const int* __restrict__ positions,
+    int row0, int H, int G, int bs, float scale, int ns, int window,
+    int keep_first) {
+  constexpr int KS = DK / 32, VB = DV / 16;
+  constexpr int kRowB = DV * 2, kChunks = DV / 8, kRows = 64 / kChunks;
+  constexpr int kHeads = 16, kPad = DV + 4;
+  static_assert(DK % 32 == 0 && (DV == 64 || DV == 128 || DV == 256));
+  constexpr int kValB = kSpanKeys * kRowB, kSumB = 4 * kHeads * kPad * 4;
+  __shared__ __attribute__((aligned(1024)))
+  unsigned char smem[kValB > kSumB ? kValB : kSumB];
+  __shared__ float red[2][4][kHeads];
+
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int r = blockIdx.x, t = row0 + r;
+  const int rep = H / G;
+  const int nbg = (rep + kHeads - 1) / kHeads;
+  const int g = blockIdx.y / nbg;
+  const int h0 = g * rep + (blockIdx.y % nbg) * kHeads;
+  const int nh = min(kHeads, (g + 1) * rep - h0);
+  const int span = blockIdx.z;
+  const int p = positions[t];
+  const int j0 = span * kSpanKeys;
+  // the combine step never reads a span that is not live
+  if (!span_live(p, j0, window, keep_first)) return;
+  const int* bt = seq_bt + static_cast<int64_t>(row_seq[t]) * bt_stride;
+
+  // lane l: cache row of this wave's key l; past the end the last one again
+  const int key = min(j0 + wave * 64 + lane, p);
+  const int at = (bt[key / bs] * G + g) * bs + key % bs;
+
+  unsigned char* vals = smem + wave * 64 * kRowB;
+  const u32 vals_lds = static_cast<u32>(reinterpret_cast<uintptr_t>(
+      (__attribute__((address_space(3))) unsigned char*)vals));
+  auto swz = [](int row) {
+    return DV == 64 ? ((row >> 1) & 1) << 2 : (row & 3) << 2;
+  };
+#pragma unroll
+  for (int i = 0; i < 64 / kRows; ++i) {
+    const int row = i * kRows + lane / kChunks;
+    dma_to_lds16_at(vals_lds + i * 1024,
+                    v_cache + static_cast<int64_t>(__shfl(at, row)) * v_row +
+                        ((lane % kChunks) ^ swz(row)) * 8);
+  }
+  typedef __attribute__((ext_vector_type(8))) short short8;
+  const int c16 = lane & 15, g4 = lane >> 4;
+  short8 qf[KS], kf[4][KS];
+#pragma unroll
+  for (int kk = 0; kk < KS; ++kk)
+    qf[kk] = c16 < nh
+        ? *reinterpret_cast<const short8*>(
+              q + (static_cast<int64_t>(t) * H + h0 + c16) * DK + kk * 32 +
+              g4 * 8)
+        : short8{0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+  for (int n = 0; n < 4; ++n) {
+    const u16* kp = k_cache + static_cast<int64_t>(__shfl(at, n * 16 + c16)) *
+                                  DK + g4 * 8;
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk)
+      kf[n][kk] = *reinterpret_cast<const short8*>(kp + kk * 32);
+  }
+  floatx4 sc[4];
+#pragma unroll
+  for (int n = 0; n < 4; ++n) {
+    sc[n] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk)
+      sc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[n][kk], qf[kk],
+                                                      sc[n], 0, 0, 0);
+  }
+
+  // statistics of the span, per head (lane & 15)
+  float m = -INFINITY;
+  bool see[4][4];
+#pragma unroll
+  for (int n = 0; n < 4; ++n)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      see[n][i] = key_visible(p, j0 + wave * 64 + n * 16 + g4 * 4 + i, window,
+                              keep_first);
+      sc[n][i] *= scale;
+      if (see[n][i]) m = fmaxf(m, sc[n][i]);
+    }
+  m = fmaxf(m, __shfl_xor(m, 16));
+  m = fmaxf(m, __shfl_xor(m, 32));
+  if (g4 == 0) red[0][wave][c16] = m;
+  __syncthreads();
+  m = fmaxf(fmaxf(red[0][0][c16], red[0][1][c16]),
+            fmaxf(red[0][2][c16], red[0][3][c16]));
+  float l = 0.f;
+#pragma unroll
+  for (int n = 0; n < 4; ++n)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      sc[n][i] = see[n][i] ? expf(sc[n][i] - m) : 0.f;
+      l += sc[n][i];
+    }
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+  if (g4 == 0) red[1][wave][c16] = l;
+
+  // this wave's values have landed
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  floatx4 o[VB];
+#pragma unroll
+  for (int db = 0; db < VB; ++db) o[db] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int st = 0; st < 2; ++st) {
+    short8 w[3];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float rest = sc[2 * st + i / 4][i % 4];
+#pragma unroll
+      for (int x = 0; x < 3; ++x) {
+        const u16 b = f32_to_bf16(rest);
+        w[x][i] = static_cast<short>(b);
+        rest -= bf16_to_f32(b);
+      }
+    }
+    const int row = st * 32 + g4 * 4 + (c16 >> 2);
+    const unsigned char* vr = vals + row * kRowB + (lane & 1) * 8;
+#pragma unroll
+    for (int db = 0; db < VB; ++db) {
+      const int ch = db * 2 + ((lane & 3) >> 1);
+      const short4v lo = lds_read_tr4(vr + (ch ^ swz(row)) * 16);
+      const short4v hi =
+          lds_read_tr4(vr + 16 * kRowB + (ch ^ swz(row + 16)) * 16);
+      const short8 v = {lo[0], lo[1], lo[2], lo[3],
+                        hi[0], hi[1], hi[2], hi[3]};
+#pragma unroll
+      for (int x = 0; x < 3; ++x)
+        o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, w[x], o[db], 0, 0,
+                                                        0);
+    }
+  }
+  __syncthreads();                     // the values are no longer needed
+  float* sums = reinterpret_cast<float*>(smem);
+#pragma unroll
+  for (int db = 0; db < VB; ++db)
+    *reinterpret_cast<floatx4*>(sums + (wave * kHeads + c16) * kPad + db * 16 +
+                                g4 * 4) = o[db];
+  __syncthreads();
+  for (int i = tid; i < nh * (DV / 4); i += 256) {
+    const int h = i / (DV / 4), d = i % (DV / 4) * 4;
+    floatx4 v = *reinterpret_cast<const floatx4*>(sums + h * kPad + d);
+#pragma unroll
+    for (int x = 1; x < 4; ++x)
+      v += *reinterpret_cast<const floatx4*>(sums + (x * kHeads + h) * kPad +
+                                             d);
+    *reinterpret_cast<floatx4*>(
+        part_o + ((static_cast<int64_t>(r) * H + h0 + h) * ns + span) * DV +
+        d) = v;
+  }
+  if (tid < nh) {
+    float* ml =
+        part_ml + ((static_cast<int64_t>(r) * H + h0 + tid) * ns + span) * 2;
+    ml[0] = m;                         // of head tid, as lane & 15 is
+    ml[1] = red[1][0][tid] + red[1][1][tid] + red[1][2][tid] +
+            red[1][3][tid];
+  }
+}
+
+// One wave per (row, head). A span's weight is worked out by one lane each,
+// and four spans' values are requested together.
 template <typename A>
 __global__ __launch_bounds__(64) void sink_attention_combine_kernel(
     A* __restrict__ out,              // [T, H, DV]
@@ -236,6 +423,7 @@ __global__ __launch_bounds__(64) void sink_attention_combine_kernel(
     const int* __restrict__ positions, const float* __restrict__ sink,
     const A* __restrict__ gate, int64_t g_stride, int gate_elem, int row0,
     int H, int DV, int ns, int window, int keep_first) {
+  __shared__ float weight[64];
   const int r = blockIdx.x, h = blockIdx.y;
   const int t = row0 + r;
   const int lane = threadIdx.x;
@@ -250,13 +438,19 @@ __global__ __launch_bounds__(64) void sink_attention_combine_kernel(
   }
   const float* ml = part_ml + (static_cast<int64_t>(r) * H + h) * ns * 2;
   const float* po = part_o + (static_cast<int64_t>(r) * H + h) * ns * DV;
-  auto live = [&](int s) { return s < s_keep || s >= s_win; };
+  // the i-th live span
+  const int live = s_keep >= nsp ? nsp : s_keep + nsp - s_win;
+  auto span_of = [&](int i) { return i < s_keep ? i : s_win + i - s_keep; };
   float m = sink != nullptr ? sink[h] : -INFINITY;
-  for (int s = 0; s < nsp; ++s)
-    if (live(s)) m = fmaxf(m, ml[2 * s]);
-  float l = sink != nullptr ? expf(sink[h] - m) : 0.f;
-  for (int s = 0; s < nsp; ++s)
-    if (live(s)) l += ml[2 * s + 1] * expf(ml[2 * s] - m);
+  for (int i = lane; i < live; i += 64) m = fmaxf(m, ml[2 * span_of(i)]);
+  m = wave_reduce_max(m);
+  float l = 0.f;
+  for (int i = lane; i < live; i += 64) {
+    const int s = span_of(i);
+    l += ml[2 * s + 1] * expf(ml[2 * s] - m);
+  }
+  l = wave_reduce_sum(l);
+  if (sink != nullptr) l += expf(sink[h] - m);
   float f = 1.0f / l;
   const A* gp = nullptr;
   if (gate != nullptr) {
@@ -266,19 +460,42 @@ __global__ __launch_bounds__(64) void sink_attention_combine_kernel(
       f *= sigmoidf_acc(Act<A>::ld(gate + t * g_stride + h));
   }
   A* op = out + (static_cast<int64_t>(t) * H + h) * DV;
-  for (int d = lane; d < DV; d += 64) {
-    float acc = 0.f;
-    for (int s = 0; s < nsp; ++s)
-      if (live(s))
-        acc += po[static_cast<int64_t>(s) * DV + d] * expf(ml[2 * s] - m);
-    acc *= f;
-    if (gp != nullptr) acc *= sigmoidf_acc(Act<A>::ld(gp + d));
-    Act<A>::st(op + d, acc);
+  for (int d0 = 0; d0 < DV; d0 += 256) {
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};   // columns d0 + 64 c + lane
+    for (int i0 = 0; i0 < live; i0 += 64) {
+      __syncthreads();
+      const int mine = i0 + lane;
+      weight[lane] =
+          mine < live ? expf(ml[2 * span_of(mine)] - m) : 0.f;
+      __syncthreads();
+      const int n = min(64, live - i0);
+      for (int i = 0; i < n; i += 4) {
+        float v[4][4];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const float* src = po + static_cast<int64_t>(span_of(
+                                      i0 + min(i + x, n - 1))) * DV + d0;
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            v[x][c] = d0 + 64 * c + lane < DV ? src[64 * c + lane] : 0.f;
+        }
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+          if (i + x < n)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) acc[c] += v[x][c] * weight[i + x];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int d = d0 + 64 * c + lane;
+      if (d >= DV) break;
+      float v = acc[c] * f;
+      if (gp != nullptr) v *= sigmoidf_acc(Act<A>::ld(gp + d));
+      Act<A>::st(op + d, v);
+    }
   }
 }
-
-typedef __attribute__((ext_vector_type(4))) float floatx4;
-typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 
 template <typename A, int DK, int DV, int BN, int QS, int HP>
 __global__ __launch_bounds__(256) void sink_attention_tile_kernel(
@@ -754,10 +971,40 @@ void launch_sink_attention_rows(A* out, float* part_ml, float* part_o,
                                 const float* sink, const A* gate,
                                 int64_t g_stride, int gate_elem, int row0,
                                 int rows, int H, int G, int DK, int DV,
-                                int block_size, float scale, int ns,
-                                int window, int keep_first, hipStream_t s) {
+                                int block_size, int64_t cache_rows,
+                                float scale, int ns, int window,
+                                int keep_first, hipStream_t s) {
   if (rows == 0) return;
+  auto combine = [&] {
+    hipLaunchKernelGGL(sink_attention_combine_kernel<A>, dim3(rows, H),
+                       dim3(64), 0, s, out, part_ml, part_o, positions, sink,
+                       gate, g_stride, gate_elem, row0, H, DV, ns, window,
+                       keep_first);
+  };
   const int rep = H / G;
+  if constexpr (std::is_same<A, u16>::value) {
+    // 16-byte pieces of rows; cache rows counted in 32 bits
+    auto aligned = [](const void* p) {
+      return reinterpret_cast<uintptr_t>(p) % 16 == 0;
+    };
+    if (aligned(q) && aligned(k_cache) && aligned(v_cache) &&
+        aligned(part_o) && v_row % 8 == 0 && cache_rows < (int64_t(1) << 31)) {
+      const dim3 grid(rows, G * ((rep + 15) / 16), ns);
+#define FI_SPAN(K_, V_)                                                        \
+  if (DK == K_ && DV == V_) {                                                  \
+    hipLaunchKernelGGL((sink_attention_span_kernel<K_, V_>), grid, dim3(256),  \
+                       0, s, part_ml, part_o, q, k_cache, v_cache, v_row,      \
+                       seq_bt, bt_stride, row_seq, positions, row0, H, G,      \
+                       block_size, scale, ns, window, keep_first);             \
+    return combine();                                                          \
+  }
+      FI_SPAN(64, 64)
+      FI_SPAN(128, 128)
+      FI_SPAN(192, 128)
+      FI_SPAN(288, 256)
+#undef FI_SPAN
+    }
+  }
   const int hb = min(kHeadBatch, rep);
   const int nbg = (rep + hb - 1) / hb;
   int dv_round = 1;
@@ -800,9 +1047,7 @@ void launch_sink_attention_rows(A* out, float* part_ml, float* part_o,
     else FI_SPLIT(1);
   }
 #undef FI_SPLIT
-  hipLaunchKernelGGL(sink_attention_combine_kernel<A>, dim3(rows, H), dim3(64),
-                     0, s, out, part_ml, part_o, positions, sink, gate,
-                     g_stride, gate_elem, row0, H, DV, ns, window, keep_first);
+  combine();
 }
 
 #define FI_INST(A)                                                             \
@@ -813,7 +1058,7 @@ void launch_sink_attention_rows(A* out, float* part_ml, float* part_o,
   template void launch_sink_attention_rows<A>(                                 \
       A*, float*, float*, const A*, const A*, const A*, int, const int*, int,  \
       const int*, const int*, const float*, const A*, int64_t, int, int, int,  \
-      int, int, int, int, int, float, int, int, int, hipStream_t);
+      int, int, int, int, int, int64_t, float, int, int, int, hipStream_t);
 FI_INST(float)
 FI_INST(u16)
 #undef FI_INST

@@ -1076,3 +1076,62 @@ def test_sink_attention_row_tiles(D, heads, groups, block, window, keep,
         keep_first=keep)
     err = (got.cpu().float() - want.view(got.shape)).abs().max()
     assert err <= 2 ** -8 * v.float().abs().max()
+
+
+@pytest.mark.parametrize("DK,DV", [(64, 64), (128, 128), (192, 128),
+                                   (288, 256)])
+@pytest.mark.parametrize("heads,groups,block,window,keep,gate", [
+    (1, 1, 16, 0, 0, None),
+    (16, 1, 16, 0, 0, "head"),
+    (20, 1, 1, 300, 260, "entry"),   # two batches of heads; kept span
+    (12, 3, 8, 40, 0, "head"),
+])
+def test_sink_attention_spans(DK, DV, heads, groups, block, window, keep,
+                              gate):
+    """Single rows at the edges of waves and spans of keys, values a slice of
+    the key rows where they are smaller, against float64. The weights are not
+    rounded: one bf16 rounding of the result, 2^-8 of it, and fp32 sums."""
+    from fusioninfer_amd.ops import seqmix
+
+    g = torch.Generator().manual_seed(DK + heads + window)
+    ctx = [1, 16, 64, 65, 256, 257, 1000, 64 * 256 + 3]
+    need = [-(-c // block) for c in ctx]
+    order = torch.randperm(sum(need) + 2, generator=g)
+    table = torch.zeros(len(ctx), max(need), dtype=torch.int32)
+    for i, n in enumerate(need):
+        table[i, :n] = order[sum(need[:i]):sum(need[:i + 1])]
+    T, own = len(ctx), DK == DV
+    q = torch.randn(T, heads, DK, generator=g).bfloat16()
+    k = torch.randn(len(order), groups, block, DK, generator=g).bfloat16()
+    v = torch.randn(len(order), groups, block, DV, generator=g).bfloat16() \
+        if own else k[..., :DV]
+    sink = torch.randn(heads, generator=g) * 3
+    og = {"head": torch.randn(T, heads, generator=g).bfloat16(),
+          "entry": torch.randn(T, heads * DV, generator=g).bfloat16()
+          }.get(gate)
+    rows = torch.arange(T).int()
+    pos = torch.tensor(ctx).int() - 1
+    dev = lambda t: None if t is None else t.to(DEV)
+    got = seqmix.sink_paged_attention(
+        dev(q), dev(k), dev(v) if own else None, dev(table), dev(rows),
+        dev(pos), DK ** -0.5, sink=dev(sink), value_dims=DV,
+        out_gate=dev(og), window=window, keep_first=keep)
+    rep = heads // groups
+    for i, c in enumerate(ctx):
+        j = torch.arange(c)
+        at = (table[i, j // block].long(), j % block)
+        see = j >= c - window if window else j >= 0
+        see |= j < keep
+        for h in range(heads):
+            kk = k[at[0], h // rep, at[1]].double()
+            s = kk @ q[i, h].double() * DK ** -0.5
+            s[~see] = -float("inf")
+            w = torch.softmax(torch.cat([s, sink[h:h + 1].double()]), 0)[:-1]
+            want = w @ v[at[0], h // rep, at[1]].double()
+            if gate == "head":
+                want = want * torch.sigmoid(og[i, h].double())
+            elif gate == "entry":
+                want = want * torch.sigmoid(
+                    og[i, h * DV:(h + 1) * DV].double())
+            err = (got[i, h].cpu().double() - want).abs()
+            assert (err <= want.abs() * 2 ** -8 + 2e-5).all(), (i, h)
