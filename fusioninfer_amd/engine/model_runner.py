@@ -16,6 +16,7 @@ engine the reference delegates to its vLLM containers (SURVEY.md §2.3
 from __future__ import annotations
 
 import os
+from array import array
 from typing import Dict, List, Optional, Tuple
 
 import numpy as np
@@ -29,6 +30,9 @@ from fusioninfer_amd.models.registry import build_model
 import fusioninfer_amd.ops as ops_mod
 
 _DECODE_BUCKETS = [1, 2, 4, 8, 16, 24, 32, 48, 64, 96, 128, 160, 192, 224, 256, 320, 384, 448, 512]
+
+# array and numpy types of the step inputs' dtypes
+_HOST_TYPES = {torch.int32: ("i", np.int32), torch.int64: ("q", np.int64)}
 
 
 class ModelRunner:
@@ -157,6 +161,47 @@ class ModelRunner:
             for _ in range(self.model.num_local_layers)
         ]
 
+    # ------------------------------------------------------------ inputs
+    def _to_device(self, arrays):
+        """A step's host arrays as device tensors, in one copy: dict of
+        name -> (values, torch.int32 or torch.int64), lists or arrays.
+
+        A prompt step of 8765 tokens made eleven tensors by torch.tensor
+        from lists, 0.44 ms of host time for each long one, and as many
+        synchronous copies; the GPU idled through about a millisecond."""
+        parts, total = {}, 0
+        for name, (values, dtype) in arrays.items():
+            values = self._host_array(values, dtype)
+            parts[name] = (total, values, dtype)
+            total += -(-values.nbytes // 16) * 16
+        host = torch.empty(total, dtype=torch.uint8, pin_memory=self.is_cuda)
+        flat = host.numpy()
+        for at, values, _ in parts.values():
+            flat[at: at + values.nbytes] = values.reshape(-1).view(np.uint8)
+        dev = host.to(self.device, non_blocking=True)
+        return {
+            name: dev[at: at + values.nbytes].view(dtype).view(values.shape)
+            for name, (at, values, dtype) in parts.items()
+        }
+
+    @staticmethod
+    def _host_array(values, dtype):
+        code, np_type = _HOST_TYPES[dtype]
+        if isinstance(values, list):
+            # array reads a list of ints three times as fast as torch
+            values = np.frombuffer(array(code, values), dtype=np_type) \
+                if values else np.empty(0, dtype=np_type)
+        return np.ascontiguousarray(values, dtype=np_type)
+
+    @staticmethod
+    def _block_table(bts, width: int = 0):
+        """Block lists as int32 rows, filled up with zeros."""
+        width = max(width, max((len(b) for b in bts), default=0), 1)
+        table = np.zeros((len(bts), width), dtype=np.int32)
+        for i, b in enumerate(bts):
+            table[i, : len(b)] = b
+        return table
+
     # ------------------------------------------------------------ prefill
     def build_prefill_payload(
         self,
@@ -234,21 +279,27 @@ class ModelRunner:
         S = len(lens)
         cu = np.zeros(S + 1, dtype=np.int32)
         np.cumsum(np.asarray(lens, dtype=np.int32), out=cu[1:])
-        width = max(max((len(b) for b in bts), default=1), 1)
-        bt_np = np.zeros((S, width), dtype=np.int32)
-        for i, b in enumerate(bts):
-            bt_np[i, : len(b)] = b
-        meta.seq_cu = torch.from_numpy(cu).to(dev)
-        meta.row_seq = torch.from_numpy(
-            np.repeat(np.arange(S, dtype=np.int32), lens)).to(dev)
-        meta.seq_bt = torch.from_numpy(bt_np).to(dev)
-        meta.seq_slots = torch.tensor(slots, dtype=torch.int32, device=dev)
-        meta.max_seq_rows = max(lens, default=0)
-        if prefill_payload is not None and prefill_payload["new_lens"]:
+        arrays = {
+            "seq_cu": (cu, torch.int32),
+            "row_seq": (np.repeat(np.arange(S, dtype=np.int32), lens),
+                        torch.int32),
+            "seq_bt": (self._block_table(bts), torch.int32),
+            "seq_slots": (slots, torch.int32),
+        }
+        prompts = prefill_payload is not None and prefill_payload["new_lens"]
+        if prompts:
             from fusioninfer_amd.ops import seqmix
 
-            meta.seq_tiles = seqmix.build_attention_tiles(
-                prefill_payload["new_lens"], device=dev)
+            tile_seq, tile_row0, covered = seqmix.build_attention_tiles(
+                prefill_payload["new_lens"])
+            arrays["tile_seq"] = (tile_seq.numpy(), torch.int32)
+            arrays["tile_row0"] = (tile_row0.numpy(), torch.int32)
+        t = self._to_device(arrays)
+        meta.seq_cu, meta.row_seq = t["seq_cu"], t["row_seq"]
+        meta.seq_bt, meta.seq_slots = t["seq_bt"], t["seq_slots"]
+        meta.max_seq_rows = max(lens, default=0)
+        if prompts:
+            meta.seq_tiles = (t["tile_seq"], t["tile_row0"], covered)
             meta.prefill_spans = list(zip(
                 prefill_payload["new_lens"], prefill_payload["total_lens"],
                 prefill_payload["bt"]))
@@ -296,49 +347,44 @@ class ModelRunner:
             return self._forward_and_logits(ids, meta, logits_idx)
 
     def _prefill_inputs(self, payload):
-        dev = self.device
         cu = payload["cu"]
         tile_rows = ops_mod.prefill_tile_rows(payload["new_lens"])
         tile_seq, tile_row0 = ops_mod.build_prefill_tiles(
-            payload["new_lens"], device=dev, rows=tile_rows
+            payload["new_lens"], rows=tile_rows
         )
-        meta = AttnMetadata(
-            num_prefill_tokens=cu[-1],
-            num_decode_tokens=0,
-            positions=torch.tensor(
-                payload["positions"], dtype=torch.int32, device=dev
-            ),
-            slot_mapping=torch.tensor(
-                payload["slots"], dtype=torch.int32, device=dev
-            ),
-            cu_seqlens=torch.tensor(cu, dtype=torch.int32, device=dev),
-            tile_seq=tile_seq,
-            tile_rows=tile_rows,
-            tile_row0=tile_row0,
-            prefill_block_tables=torch.tensor(
-                payload["bt"], dtype=torch.int32, device=dev
-            ),
-            prefill_seq_lens_k=torch.tensor(
-                payload["total_lens"], dtype=torch.int32, device=dev
-            ),
-        )
-        meta.lora = self._lora_batch(payload, None)
-        self._seq_meta(meta, payload, None)
-        ids = torch.tensor(payload["ids"], dtype=torch.long, device=dev)
         if payload.get("logits_rows") is not None:
             # spec-decode verification asks for explicit rows (every draft
             # position, not just chunk ends)
-            logits_idx = torch.tensor(
-                payload["logits_rows"], dtype=torch.long, device=dev
-            )
+            rows = list(payload["logits_rows"])
         else:
             sample = payload.get("sample") or [True] * (len(cu) - 1)
-            logits_idx = torch.tensor(
-                [c - 1 for c, smp in zip(cu[1:], sample) if smp],
-                dtype=torch.long,
-                device=dev,
-            )
-        return ids, meta, logits_idx
+            rows = [c - 1 for c, smp in zip(cu[1:], sample) if smp]
+        t = self._to_device({
+            "ids": (payload["ids"], torch.long),
+            "positions": (payload["positions"], torch.int32),
+            "slots": (payload["slots"], torch.int32),
+            "cu": (cu, torch.int32),
+            "tile_seq": (tile_seq.numpy(), torch.int32),
+            "tile_row0": (tile_row0.numpy(), torch.int32),
+            "bt": (self._block_table(payload["bt"]), torch.int32),
+            "total_lens": (payload["total_lens"], torch.int32),
+            "rows": (rows, torch.long),
+        })
+        meta = AttnMetadata(
+            num_prefill_tokens=cu[-1],
+            num_decode_tokens=0,
+            positions=t["positions"],
+            slot_mapping=t["slots"],
+            cu_seqlens=t["cu"],
+            tile_seq=t["tile_seq"],
+            tile_rows=tile_rows,
+            tile_row0=t["tile_row0"],
+            prefill_block_tables=t["bt"],
+            prefill_seq_lens_k=t["total_lens"],
+        )
+        meta.lora = self._lora_batch(payload, None)
+        self._seq_meta(meta, payload, None)
+        return t["ids"], meta, t["rows"]
 
     # ------------------------------------------- PP microbatch pipelining
     def _split_prefill_payload(self, payload, min_mb_tokens: int = 256):
@@ -612,82 +658,83 @@ class ModelRunner:
             return self.run_decode(d)
         if not d["ids"]:
             return self.run_prefill(payload)
-        dev = self.device
         cu = payload["cu"]
         np_ = cu[-1]
         nd = len(d["ids"])
         tile_rows = ops_mod.prefill_tile_rows(payload["new_lens"])
         tile_seq, tile_row0 = ops_mod.build_prefill_tiles(
-            payload["new_lens"], device=dev, rows=tile_rows
-        )
-        max_blocks = max(len(b) for b in d["bt"])
-        dbt_np = np.zeros((nd, max_blocks), dtype=np.int32)
-        for i, ids in enumerate(d["bt"]):
-            dbt_np[i, : len(ids)] = ids
-        dbt = torch.from_numpy(dbt_np)
-        meta = AttnMetadata(
-            num_prefill_tokens=np_,
-            num_decode_tokens=nd,
-            positions=torch.tensor(
-                payload["positions"] + d["positions"],
-                dtype=torch.int32, device=dev,
-            ),
-            slot_mapping=torch.tensor(
-                payload["slots"] + d["slots"], dtype=torch.int32, device=dev
-            ),
-            cu_seqlens=torch.tensor(cu, dtype=torch.int32, device=dev),
-            tile_seq=tile_seq,
-            tile_rows=tile_rows,
-            tile_row0=tile_row0,
-            prefill_block_tables=torch.tensor(
-                payload["bt"], dtype=torch.int32, device=dev
-            ),
-            prefill_seq_lens_k=torch.tensor(
-                payload["total_lens"], dtype=torch.int32, device=dev
-            ),
-            block_tables=dbt.to(dev),
-            seq_lens=torch.tensor(d["lens"], dtype=torch.int32, device=dev),
-        )
-        meta.lora = self._lora_batch(payload, d, np_=np_)
-        self._seq_meta(meta, payload, d)
-        ids = torch.tensor(
-            payload["ids"] + d["ids"], dtype=torch.long, device=dev
+            payload["new_lens"], rows=tile_rows
         )
         if payload.get("logits_rows") is not None:
             # prompt_logprobs asks for explicit rows (prompt positions
             # plus the standard sampling rows); the engine re-maps them
-            logits_idx = torch.tensor(
-                payload["logits_rows"], dtype=torch.long, device=dev
-            )
+            rows = list(payload["logits_rows"])
         else:
             # logits rows: completing prefill chunks first, then every
             # decode row
-            pf_idx = [
-                c - 1 for c, smp in zip(cu[1:], payload["sample"]) if smp
-            ]
-            logits_idx = torch.tensor(
-                pf_idx + list(range(np_, np_ + nd)), dtype=torch.long,
-                device=dev,
-            )
+            rows = [c - 1 for c, smp in zip(cu[1:], payload["sample"]) if smp]
+            rows += range(np_, np_ + nd)
+        t = self._to_device({
+            "ids": (payload["ids"] + d["ids"], torch.long),
+            "positions": (payload["positions"] + d["positions"], torch.int32),
+            "slots": (payload["slots"] + d["slots"], torch.int32),
+            "cu": (cu, torch.int32),
+            "tile_seq": (tile_seq.numpy(), torch.int32),
+            "tile_row0": (tile_row0.numpy(), torch.int32),
+            "bt": (self._block_table(payload["bt"]), torch.int32),
+            "total_lens": (payload["total_lens"], torch.int32),
+            "decode_bt": (self._block_table(d["bt"]), torch.int32),
+            "lens": (d["lens"], torch.int32),
+            "rows": (rows, torch.long),
+        })
+        meta = AttnMetadata(
+            num_prefill_tokens=np_,
+            num_decode_tokens=nd,
+            positions=t["positions"],
+            slot_mapping=t["slots"],
+            cu_seqlens=t["cu"],
+            tile_seq=t["tile_seq"],
+            tile_rows=tile_rows,
+            tile_row0=t["tile_row0"],
+            prefill_block_tables=t["bt"],
+            prefill_seq_lens_k=t["total_lens"],
+            block_tables=t["decode_bt"],
+            seq_lens=t["lens"],
+        )
+        meta.lora = self._lora_batch(payload, d, np_=np_)
+        self._seq_meta(meta, payload, d)
+        ids, logits_idx = t["ids"], t["rows"]
         with torch.no_grad():
             return self._forward_and_logits(ids, meta, logits_idx)
 
     # ------------------------------------------------------------ decode
     def _alloc_static(self, max_bs: int) -> None:
         dev = self.device
+        # the per-row inputs lie in one buffer, which one copy fills; ids
+        # come last, since they may be on the device already
+        self._static_rows = {"positions": (torch.int32, 0),
+                             "slots": (torch.int32, -1),
+                             "seq_lens": (torch.int32, 1)}
+        if self.uses_state_slots:
+            self._static_rows["state_slots"] = (torch.int32, -1)
+        self._static_rows["ids"] = (torch.long, 0)
+        unit = -(-max_bs // 4) * 16       # bytes of max_bs int32, padded
+        total = sum(unit * (dt.itemsize // 4)
+                    for dt, _ in self._static_rows.values())
+        self._static_buf = torch.zeros(total, dtype=torch.uint8, device=dev)
         self._static = {
-            "ids": torch.zeros(max_bs, dtype=torch.long, device=dev),
-            "positions": torch.zeros(max_bs, dtype=torch.int32, device=dev),
-            "slots": torch.full((max_bs,), -1, dtype=torch.int32, device=dev),
             "block_tables": torch.zeros(
                 (max_bs, self.max_blocks_per_seq), dtype=torch.int32, device=dev
             ),
-            "seq_lens": torch.ones(max_bs, dtype=torch.int32, device=dev),
         }
+        at = 0
+        for name, (dt, fill) in self._static_rows.items():
+            self._static[name] = self._static_buf[
+                at: at + max_bs * dt.itemsize].view(dt)
+            self._static[name].fill_(fill)
+            at += unit * (dt.itemsize // 4)
         if self.uses_state_slots:
             # every decode row is its own one-row group
-            self._static["state_slots"] = torch.full(
-                (max_bs,), -1, dtype=torch.int32, device=dev)
             self._static["seq_cu"] = torch.arange(
                 max_bs + 1, dtype=torch.int32, device=dev)
             self._static["row_seq"] = torch.arange(
@@ -760,43 +807,32 @@ class ModelRunner:
     def _fill_decode_inputs(self, payload, bs: int) -> None:
         n = len(payload["lens"])
         st = self._static
-        if payload["ids"] is not None:
-            st["ids"][:n].copy_(
-                torch.tensor(payload["ids"], dtype=torch.long),
-                non_blocking=True,
-            )
-        st["positions"][:n].copy_(
-            torch.tensor(payload["positions"], dtype=torch.int32),
-            non_blocking=True,
-        )
-        st["slots"][:n].copy_(
-            torch.tensor(payload["slots"], dtype=torch.int32),
-            non_blocking=True,
-        )
-        st["seq_lens"][:n].copy_(
-            torch.tensor(payload["lens"], dtype=torch.int32), non_blocking=True
-        )
-        # numpy row fill: a per-row torch.tensor loop cost 2-4 ms/step at
-        # batch 256 (measured with FI_STEP_TIMING)
-        bt_np = np.zeros((n, self.max_blocks_per_seq), dtype=np.int32)
-        for i, ids in enumerate(payload["bt"]):
-            bt_np[i, : len(ids)] = ids
-        st["block_tables"][:n].copy_(
-            torch.from_numpy(bt_np), non_blocking=True
-        )
+        # padding rows: decode block 0, pos 0, len 1, slot -1
+        given = {"positions": payload["positions"], "slots": payload["slots"],
+                 "seq_lens": payload["lens"], "ids": payload["ids"]}
         if self.uses_state_slots:
-            st["state_slots"][:n].copy_(
-                torch.tensor(payload["state_slots"], dtype=torch.int32),
-                non_blocking=True,
-            )
-            if bs > n:
-                st["state_slots"][n:bs].fill_(-1)
-        if bs > n:  # padding rows: decode block 0, pos 0, len 1, slot -1
-            st["ids"][n:bs].zero_()
-            st["positions"][n:bs].zero_()
-            st["slots"][n:bs].fill_(-1)
-            st["seq_lens"][n:bs].fill_(1)
-            st["block_tables"][n:bs].zero_()
+            given["state_slots"] = payload["state_slots"]
+        # a few kilobytes: the copy out of pageable memory starts sooner than
+        # one that the DMA engine fetches (one row 898 us a step against 909)
+        host = torch.empty(self._static_buf.shape, dtype=torch.uint8)
+        flat = host.numpy()
+        base = self._static_buf.data_ptr()
+        end = 0
+        for name, (dt, fill) in self._static_rows.items():
+            at = st[name].data_ptr() - base
+            if given[name] is None:       # ids, already on the device
+                st[name][n:bs].zero_()
+                continue
+            end = at + st[name].numel() * dt.itemsize
+            rows = flat[at: end].view(_HOST_TYPES[dt][1])
+            rows[:n] = self._host_array(given[name], dt)
+            rows[n:] = fill
+        self._static_buf[:end].copy_(host[:end], non_blocking=True)
+        # the columns in use; what an earlier step left behind them belongs
+        # to no context of this one
+        table = self._block_table(payload["bt"] + [[]] * (bs - n))
+        st["block_tables"][:bs, : table.shape[1]].copy_(
+            torch.from_numpy(table), non_blocking=True)
 
     def run_decode_device_ids(self, payload, ids_dev: torch.Tensor):
         """Graph-replay decode with ON-DEVICE input ids: the pipelined
