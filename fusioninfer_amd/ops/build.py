@@ -33,7 +33,8 @@ SOURCES = [
     "cache.hip",
     "paged_attention.hip",
     "prefill_attention.hip",
-    "skinny_gemm.hip", "part_gemm.hip",
+    "skinny_gemm.hip",
+    "part_gemm.hip",
 ]
 
 MOE_SOURCES = [
@@ -41,7 +42,8 @@ MOE_SOURCES = [
     "moe_gemm.hip",
     "moe_tile.hip",
     "moe_plain.hip",
-    "moe_router.hip", "moe_stream.hip",
+    "moe_router.hip",
+    "moe_stream.hip",
 ]
 
 

@@ -43,6 +43,9 @@ void launch_skinny_gemm(u16*, const u16*, const u16*, const u16*, int, int,
 int64_t part_gemm_floats(int, int, int);
 void launch_part_gemm(u16*, float*, const u16*, const u16*, const u16*, int,
                       int, int, int64_t, int64_t, bool, hipStream_t);
+void launch_part_gemm_fp8(u16*, float*, const unsigned char*, const float*,
+                          const unsigned char*, const float*, int, int, int,
+                          int64_t, int64_t, hipStream_t);
 
 }  // namespace fi
 
@@ -437,6 +440,40 @@ void few_rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
                        silu_mul, current_stream());
 }
 
+// out [M, N] bf16 = (x [M, K] * x_scales) @ (w [N, K] * w_scales)^T, e4m3
+void few_rows_gemm_fp8(at::Tensor out, at::Tensor x, at::Tensor x_scales,
+                       at::Tensor w, at::Tensor w_scales) {
+  CHECK_BF16_CUDA(out);
+  TORCH_CHECK(x.is_cuda() && w.is_cuda() &&
+              x.scalar_type() == at::kFloat8_e4m3fn &&
+              w.scalar_type() == at::kFloat8_e4m3fn);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2);
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(M >= 1 && M <= 256 && w.size(1) == K && K % 256 == 0 && K > 0 &&
+                  N > 0 && N % 16 == 0 && K <= (1 << 24) && N <= (1 << 24),
+              "few_rows_gemm_fp8: unsupported sizes");
+  TORCH_CHECK(out.size(0) == M && out.size(1) == N && out.stride(1) == 1 &&
+              out.stride(0) % 4 == 0);
+  TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % 16 == 0 &&
+              x.stride(0) <= (1 << 22) && w.is_contiguous());
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0);
+  TORCH_CHECK(x_scales.is_cuda() && x_scales.scalar_type() == at::kFloat &&
+              x_scales.is_contiguous() && x_scales.numel() == M &&
+              w_scales.is_cuda() && w_scales.scalar_type() == at::kFloat &&
+              w_scales.is_contiguous() && w_scales.numel() == N);
+  at::Tensor pieces = at::empty({fi::part_gemm_floats(M, N, K / 2)},
+                                x.options().dtype(at::kFloat));
+  fi::launch_part_gemm_fp8(
+      bf16_ptr(out), pieces.data_ptr<float>(),
+      static_cast<const unsigned char*>(x.data_ptr()),
+      x_scales.data_ptr<float>(),
+      static_cast<const unsigned char*>(w.data_ptr()),
+      w_scales.data_ptr<float>(), M, N, K, x.stride(0), out.stride(0),
+      current_stream());
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -458,6 +495,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gather_kv_blocks", &gather_kv_blocks, "pack KV blocks for PD send");
   m.def("scatter_kv_blocks", &scatter_kv_blocks, "unpack KV blocks from PD recv");
   m.def("few_rows_gemm", &few_rows_gemm, "x W^T for up to 256 rows of x");
+  m.def("few_rows_gemm_fp8", &few_rows_gemm_fp8,
+        "x W^T for up to 256 rows of e4m3 x with scales per row");
   m.def("paged_attention_decode", &paged_attention_decode,
         "paged decode attention");
   m.def("prefill_attention", &prefill_attention, "varlen causal MFMA prefill");

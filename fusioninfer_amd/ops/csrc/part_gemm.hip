@@ -27,6 +27,11 @@
 // 26 / 37 / 66 / 53; 151936, 4096 211 (5880) / 238 / 266 / 391 against 264 /
 // 262 / 279 / 350.
 
+//
+// FP8: the same kernel on e4m3 rows, 1 to 128 of them. 24576 x 4096 at 1 / 32
+// / 64 rows 20.0 (5040) / 19.3 / 24.3 us, the library's GEMM 30.8 / 24.4 /
+// 25.9; 4096 x 12288 14.2 (3550) / 14.5 / 19.4 against 21.1 / 20.5 / 24.1.
+
 #include "common.h"
 
 namespace fi {
@@ -96,14 +101,22 @@ FI_DEV int w_fragment(int wn, int rf) {
   return rf < h ? wn * h + rf : S::TN / 32 + wn * h + rf - h;
 }
 
+// FP8: the scales of the rows of x and of W
+struct Scales {
+  const float* x;
+  const float* w;
+};
+
 // results n4 .. n4+3 of row m; SILU_MUL: of gate values g and up values u
-template <bool SILU_MUL>
-FI_DEV void store4(u16* out, const u16* bias, const floatx4& g,
-                   const floatx4& u, int m, int n, int64_t out_stride) {
+template <bool SILU_MUL, bool FP8>
+FI_DEV void store4(u16* out, const u16* bias, const Scales& scales,
+                   const floatx4& g, const floatx4& u, int m, int n,
+                   int64_t out_stride) {
   bf16x4 o;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     float v = g[r];
+    if (FP8) v *= scales.x[m] * scales.w[n + r];
     if (SILU_MUL)
       v = v / (1.f + __expf(-v)) * u[r];
     else if (bias)
@@ -113,12 +126,15 @@ FI_DEV void store4(u16* out, const u16* bias, const floatx4& g,
   *reinterpret_cast<bf16x4*>(out + m * out_stride + n) = o;
 }
 
-template <class S, bool SILU_MUL>
+// FP8: e4m3 values, two to a u16 everywhere (K and strides too); a chunk of 16
+// goes through two products, in the same order for W and x
+template <class S, bool SILU_MUL, bool FP8>
 __global__ __launch_bounds__(S::kWaves * kWaveSize)
 void part_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
                       const u16* __restrict__ x, const u16* __restrict__ w,
-                      const u16* __restrict__ bias, const int M, const int N,
-                      const int K, const int64_t x_stride,
+                      const u16* __restrict__ bias, const Scales scales,
+                      const int M, const int N, const int K,
+                      const int64_t x_stride,
                       const int64_t out_stride, const int tiles,
                       const int unit) {
   constexpr int LW = S::LW, LX = S::LX, RF = S::RF, CF = S::CF;
@@ -268,9 +284,20 @@ void part_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
 #pragma unroll
         for (int f = 0; f < RF; ++f)
 #pragma unroll
-          for (int c = 0; c < CF; ++c)
-            acc[f][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                a[f], b[c], acc[f][c], 0, 0, 0);
+          for (int c = 0; c < CF; ++c) {
+            if constexpr (FP8) {
+              typedef __attribute__((ext_vector_type(2))) long long i64x2;
+              const i64x2 a8 = __builtin_bit_cast(i64x2, a[f]);
+              const i64x2 b8 = __builtin_bit_cast(i64x2, b[c]);
+#pragma unroll
+              for (int i = 0; i < 2; ++i)
+                acc[f][c] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
+                    a8[i], b8[i], acc[f][c], 0, 0, 0);
+            } else {
+              acc[f][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  a[f], b[c], acc[f][c], 0, 0, 0);
+            }
+          }
       }
       if (++wslot == S::RW) wslot = 0;
       if (++xslot == S::RX) xslot = 0;
@@ -284,9 +311,9 @@ void part_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
         for (int c = 0; c < CF; ++c) {
           const int m = (wm * CF + c) * 16 + (lane & 15);
           if (m < M && n < (SILU_MUL ? N / 2 : N))
-            store4<SILU_MUL>(out, bias, acc[f][c],
-                             acc[SILU_MUL ? f + RF / 2 : f][c], m, n,
-                             out_stride);
+            store4<SILU_MUL, FP8>(out, bias, scales, acc[f][c],
+                                  acc[SILU_MUL ? f + RF / 2 : f][c], m, n,
+                                  out_stride);
         }
       }
     } else {
@@ -306,13 +333,14 @@ void part_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
 
 // One row of workgroups per border between parts; the first border inside a
 // tile sums its pieces.
-template <class S, bool SILU_MUL>
+template <class S, bool SILU_MUL, bool FP8>
 __global__ __launch_bounds__(256)
 void part_gemm_join_kernel(u16* __restrict__ out,
                            const floatx4* __restrict__ pieces,
-                           const u16* __restrict__ bias, const int M,
-                           const int N, const int K, const int64_t out_stride,
-                           const int tiles, const int parts) {
+                           const u16* __restrict__ bias, const Scales scales,
+                           const int M, const int N, const int K,
+                           const int64_t out_stride, const int tiles,
+                           const int parts) {
   constexpr int RF = S::RF, CF = S::CF;
   constexpr int kUse = SILU_MUL ? RF / 2 : RF;   // fragments with results
   const int SK = K / S::KS;
@@ -354,7 +382,7 @@ void part_gemm_join_kernel(u16* __restrict__ out,
         if (SILU_MUL) u += us[i];
       }
   }
-  store4<SILU_MUL>(out, bias, g, u, m, n, out_stride);
+  store4<SILU_MUL, FP8>(out, bias, scales, g, u, m, n, out_stride);
 }
 
 // How a shape cuts [N, K] up and what that takes by what limits it here: a
@@ -392,21 +420,22 @@ Plan plan_of(int N, int K) {
   return a.us <= b.us ? a : b;
 }
 
-template <class S, bool SILU_MUL>
+template <class S, bool SILU_MUL, bool FP8>
 void launch_part(const Plan& pl, u16* out, float* pieces, const u16* x,
-                 const u16* w, const u16* bias, int M, int N, int K,
-                 int64_t x_stride, int64_t out_stride, hipStream_t stream) {
+                 const u16* w, const u16* bias, const Scales& scales, int M,
+                 int N, int K, int64_t x_stride, int64_t out_stride,
+                 hipStream_t stream) {
   auto* p = reinterpret_cast<floatx4*>(pieces);
-  hipLaunchKernelGGL((part_gemm_kernel<S, SILU_MUL>), dim3(pl.parts),
+  hipLaunchKernelGGL((part_gemm_kernel<S, SILU_MUL, FP8>), dim3(pl.parts),
                      dim3(S::kWaves * kWaveSize), 0, stream, out, p, x, w,
-                     bias, M, N, K, x_stride, out_stride, pl.tiles,
+                     bias, scales, M, N, K, x_stride, out_stride, pl.tiles,
                      pl.split ? 1 : K / S::KS);
   if (!pl.split || pl.parts == 1) return;
-  hipLaunchKernelGGL((part_gemm_join_kernel<S, SILU_MUL>),
+  hipLaunchKernelGGL((part_gemm_join_kernel<S, SILU_MUL, FP8>),
                      dim3(pl.parts - 1,
                           S::kPiece / (SILU_MUL ? 2 : 1) / 256),
-                     dim3(256), 0, stream, out, p, bias, M, N, K, out_stride,
-                     pl.tiles, pl.parts);
+                     dim3(256), 0, stream, out, p, bias, scales, M, N, K,
+                     out_stride, pl.tiles, pl.parts);
 }
 
 // Row classes and their shapes: tiles of 96 rows where the chip takes them
@@ -461,11 +490,25 @@ void launch_part_gemm(u16* out, float* pieces, const u16* x, const u16* w,
   with_shape(M, N, K, [&](auto shape, const Plan& pl) {
     using S = decltype(shape);
     if (silu_mul)
-      launch_part<S, true>(pl, out, pieces, x, w, bias, M, N, K, x_stride,
-                           out_stride, stream);
+      launch_part<S, true, false>(pl, out, pieces, x, w, bias, Scales{}, M, N,
+                                  K, x_stride, out_stride, stream);
     else
-      launch_part<S, false>(pl, out, pieces, x, w, bias, M, N, K, x_stride,
-                            out_stride, stream);
+      launch_part<S, false, false>(pl, out, pieces, x, w, bias, Scales{}, M,
+                                   N, K, x_stride, out_stride, stream);
+  });
+}
+
+// e4m3 x and W with a scale per row each; K a multiple of 256
+void launch_part_gemm_fp8(u16* out, float* pieces, const unsigned char* x,
+                          const float* x_scales, const unsigned char* w,
+                          const float* w_scales, int M, int N, int K,
+                          int64_t x_stride, int64_t out_stride,
+                          hipStream_t stream) {
+  with_shape(M, N, K / 2, [&](auto shape, const Plan& pl) {
+    launch_part<decltype(shape), false, true>(
+        pl, out, pieces, reinterpret_cast<const u16*>(x),
+        reinterpret_cast<const u16*>(w), nullptr, Scales{x_scales, w_scales},
+        M, N, K / 2, x_stride / 2, out_stride, stream);
   });
 }
 

@@ -55,13 +55,9 @@ def fp8_linear(x, w_fp8: torch.Tensor, w_scale: torch.Tensor):
     else:
         x_fp8, x_scale = None, None  # CPU: keep the bf16 tensor
     if x_fp8 is not None and x_fp8.is_cuda:
-        return torch._scaled_mm(
-            x_fp8,
-            w_fp8.t(),  # [I, O], column-major view of the row-major weight
-            scale_a=x_scale.unsqueeze(1),
-            scale_b=w_scale.unsqueeze(0),
-            out_dtype=torch.bfloat16,
-        )
+        from fusioninfer_amd import ops
+
+        return ops.linear_fp8(x_fp8, x_scale, w_fp8, w_scale)
     # CPU reference path (tests): dequantize and matmul in fp32
     if x_fp8 is not None:  # tuple input on CPU
         x = x_fp8.float() * x_scale.unsqueeze(1).float()

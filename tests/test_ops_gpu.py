@@ -912,6 +912,45 @@ def test_linear_in_parts(rows, n, k, bias):
                 <= want.abs() * 2 ** -8 + 1e-3 * k ** 0.5).all()
 
 
+@pytest.mark.parametrize("rows", [1, 32, 33, 64, 65, 128, 129, 256])
+@pytest.mark.parametrize("n,k", [
+    (16, 256),           # one ragged tile, one or two stages
+    (4128, 2560),        # cut tiles, a ragged last one
+    (288, 16384),        # a tile in many pieces
+    (24608, 512),        # whole tiles and one more
+])
+def test_linear_fp8_in_parts(rows, n, k):
+    """e4m3 rows with scales against a float64 product; one bf16 rounding of
+    the result (2^-9 relative), fp32 sums and two scale products."""
+    g = torch.Generator().manual_seed(n + k + rows)
+    f8 = torch.float8_e4m3fn
+    w = torch.randn(n, k, generator=g).to(f8).to(DEV)
+    x = torch.randn(rows, 2 * k, generator=g).to(f8).to(DEV)[:, k:]
+    ws = torch.rand(n, generator=g).to(DEV) + 0.5
+    xs = torch.rand(rows, generator=g).to(DEV) + 0.5
+    out = torch.empty(rows, n, dtype=torch.bfloat16, device=DEV)
+    ops._C.few_rows_gemm_fp8(out, x, xs, w, ws)
+    want = (x.double() @ w.double().T) * xs.double()[:, None] * ws.double()
+    assert ((out.double() - want).abs()
+            <= want.abs() * 2 ** -8 + 3e-4 * k ** 0.5).all()
+
+
+def test_linear_fp8_takes_parts_by_size():
+    """The sizes that stream and those of the library give the same."""
+    f8 = torch.float8_e4m3fn
+    for rows, n, k, streams in [(1, 4096, 4096, True), (64, 4096, 4096, False),
+                                (64, 2048, 8192, True), (3, 64, 256, False),
+                                (200, 4096, 8192, False)]:
+        assert ops._streams_fp8(rows, n, k) == streams
+        x = torch.randn(rows, k, device=DEV).to(f8)
+        w = torch.randn(n, k, device=DEV).to(f8)
+        xs = torch.rand(rows, device=DEV) + 0.5
+        ws = torch.rand(n, device=DEV) + 0.5
+        want = (x.double() @ w.double().T) * xs.double()[:, None] * ws.double()
+        err = (ops.linear_fp8(x, xs, w, ws).double() - want).abs()
+        assert (err <= want.abs() * 2 ** -8 + 3e-4 * k ** 0.5).all()
+
+
 def test_linear_takes_parts_by_size():
     """The sizes that stream and those that stay with the library give the
     same product."""
