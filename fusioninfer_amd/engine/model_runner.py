@@ -9,8 +9,7 @@ eager; batches with live LoRA adapters also run eager. Payloads are plain
 host lists so the TP driver can broadcast them to worker ranks.
 
 Capability parity: the execution layer of the continuous-batching
-engine the reference delegates to its vLLM containers (SURVEY.md §2.3
-"Continuous-batching scheduler + paged KV cache").
+engine the reference delegates to its vLLM containers.
 """
 
 from __future__ import annotations

@@ -169,7 +169,7 @@ class MoEMLP(nn.Module):
     remote expert contribute nothing locally and the per-layer all-reduce
     — the same one the dense row-parallel convention already requires —
     sums expert outputs across ranks (allreduce-combine EP; all-to-all
-    dispatch is the multi-node variant, SURVEY.md §5.8). Expert weights
+    dispatch is the multi-node variant). Expert weights
     are drawn from per-(layer, expert) seeds so the same engine seed
     yields identical experts under any EP layout."""
 
@@ -660,7 +660,7 @@ class DecoderLayer(nn.Module):
 class CausalLM(nn.Module):
     """The full model: embedding -> N decoder layers -> final norm -> lm_head.
 
-    Pipeline parallelism (SURVEY.md §2.4): stage r holds a contiguous slice
+    Pipeline parallelism: stage r holds a contiguous slice
     of the layers; the first stage owns the embedding, the last the final
     norm + lm_head. Random init draws every module from a per-module seed
     derived from the caller's seed, so the SAME seed produces the SAME

@@ -30,7 +30,7 @@
 // -> 35 (4.6); one of 301 12.0 -> 10.1, one of 8000 19.5 -> 15.0.
 //
 // Capability parity: the paged-attention decode the reference delegates to
-// its vLLM containers (SURVEY.md §2.3 "Paged-attention decode kernel").
+// its vLLM containers.
 
 #include "common.h"
 

@@ -46,7 +46,7 @@
 // col = lane&31.
 //
 // Capability parity: the paged-attention prefill the reference delegates
-// to vLLM (SURVEY.md §2.3).
+// to vLLM.
 #pragma once
 
 #include "common.h"

@@ -5,11 +5,10 @@ bytes — decode-time GEMMs are weight-bandwidth-bound, so fp8 weights pay
 there directly. Enabled per-engine with `--quantization fp8`: projection
 weights are stored fp8 with per-output-channel scales; activations are
 dynamically quantized per-token; the GEMM is hipBLASLt fp8 via
-torch._scaled_mm with bf16 output. The flagship benchmark stays bf16
+ops.linear_fp8 with bf16 output. The flagship benchmark stays bf16
 (BASELINE dtype contract); fp8 is an opt-in serving mode.
 
-Note: gfx950 fp8 is OCP e4m3fn — NOT the MI300X fnuz variant
-(guide cdna_hip_programming.md §4).
+Note: gfx950 fp8 is OCP e4m3fn — NOT the MI300X fnuz variant.
 """
 
 from __future__ import annotations

@@ -1,7 +1,7 @@
 """GPU numerics tests: every HIP kernel vs the PyTorch fp32 reference.
 
-Mirrors the reference's test strategy tier 1 (table-driven unit tests,
-SURVEY.md §4) applied to the data plane: each op is compared against
+Mirrors the reference's test strategy tier 1 (table-driven unit tests)
+applied to the data plane: each op is compared against
 ops/reference.py on random inputs.
 """
 
@@ -265,7 +265,7 @@ def test_prefill_attention(head_dim, seq_lens, hq, hk):
 
 def test_prefill_attention_spiked_scores():
     """Force large per-tile max jumps so online-softmax rescale paths fire
-    (guide §5.4 rule 26: bounded random data never exercises them)."""
+    (bounded random data never exercises them)."""
     torch.manual_seed(4)
     L, hq, hk, D = 256, 2, 2, 128
     q = torch.randn(L, hq, D, dtype=torch.bfloat16, device=DEV)
