@@ -219,6 +219,19 @@ FI_DEV __attribute__((ext_vector_type(4))) short lds_read_tr4(
 #endif
 }
 
+// A softmax weight for the bf16 matrix cores without loss: three terms of
+// eight bits each, by truncation, add up to the fp32 value. No term is 0, so
+// that an infinite operand stays what it is; 2^-126 of a finite one is nothing.
+FI_DEV void split_weight(float p, u16 (&terms)[3]) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    p = fmaxf(p, 0x1p-126f);
+    const u32 top = __float_as_uint(p) & 0xffff0000u;
+    terms[i] = static_cast<u16>(top >> 16);
+    p -= __uint_as_float(top);
+  }
+}
+
 template <int NWAVES>
 FI_DEV float block_reduce_max(float wave_val, float* scratch) {
   const int wave = threadIdx.x / kWaveSize;

@@ -18,16 +18,23 @@
 //   O^T[dim, head] += V^T P^T         A = V through the transposing LDS
 //                                     read, B = P as the scores' registers
 //                                     already hold it (the order of the
-//                                     tokens within a step is theirs)
+//                                     tokens within a step is theirs), in
+//                                     three bf16 terms that are the fp32 P
 // A lane keeps one head's statistics; e4m3 rows are converted exactly after
-// the LDS read. 96 KB in flight and a few hundred cycles of work per 8 KB
-// step leave memory as the only bound.
+// the LDS read. 96 KB in flight and some hundred cycles of work per 8 KB
+// step leave memory as the bound of long contexts. P in one bf16 term is 0.4
+// us less for one of 301 tokens, 1 to 2 % of the bf16 contexts below and 2 us
+// of the e4m3 ones; its weights have 8 bits where the sum they are divided by
+// has 24.
+// Where a context is cut depends on the lengths of all contexts of the
+// launch, and so do the last bits of the fp32 sums: a row of one batch can
+// differ by a bf16 rounding from the same row among other neighbours.
 //
 // Measured at 32 query heads, D 128, both kernels, us (TB/s of K/V), before
-// -> now: 256 contexts of 1024-1279 tokens, 8 K/V heads 278 (4.3) -> 207
-// (5.8); 6 of 20-32 thousand 168 (3.9) -> 109 (6.0); 13 of 70-4100 42 -> 25;
-// 64 of 512-2048 e4m3 101 (1.6) -> 34 (4.7), with 4 K/V heads bf16 58 (2.7)
-// -> 35 (4.6); one of 301 12.0 -> 10.1, one of 8000 19.5 -> 15.0.
+// -> now: 256 contexts of 1024-1279 tokens, 8 K/V heads 278 (4.3) -> 212
+// (5.7); 6 of 20-32 thousand 168 (3.9) -> 110 (6.0); 13 of 70-4100 42 -> 26;
+// 64 of 512-2048 e4m3 101 (1.6) -> 36 (4.4), with 4 K/V heads bf16 58 (2.7)
+// -> 36 (4.4); one of 301 12.0 -> 10.5, one of 8000 19.5 -> 15.4.
 //
 // Capability parity: the paged-attention decode the reference delegates to
 // its vLLM containers.
@@ -198,6 +205,7 @@ struct DecShape {
   static constexpr int kRowB = D * (FP8 ? 1 : 2);
   // pages of a step: 8 KB of K and V together (4 KB for the smallest rows)
   static constexpr int PP = kRowB == 256 ? 1 : 2;
+  static_assert(!FP8 || PP == 2, "byte transposes take two pages");
 };
 
 template <int D, bool FP8>
@@ -424,7 +432,7 @@ void paged_attn_decode_kernel(const DecodeArgs p) {
           for (int r = 0; r < 4; ++r) o_acc[dt][r] *= alpha;
       }
       const float mc = m_row * c;
-      u16 pb[PP * 4];
+      short4v pb[3][PP];       // the weights' terms, per page
 #pragma unroll
       for (int pg = 0; pg < PP; ++pg)
 #pragma unroll
@@ -432,34 +440,41 @@ void paged_attn_decode_kernel(const DecodeArgs p) {
           const float e =
               __builtin_amdgcn_exp2f(fmaf(s[pg][r], c, -mc));
           l_row += e;
-          pb[pg * 4 + r] = f32_to_bf16(e);
+          u16 terms[3];
+          split_weight(e, terms);
+#pragma unroll
+          for (int x = 0; x < 3; ++x)
+            pb[x][pg][r] = static_cast<short>(terms[x]);
         }
+      // term by term over all columns, so that no product waits for the one
+      // before it; a single page's first two terms share a 32-deep product
+      short8 a_v[DT];
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
-        if constexpr (PP == 1) {
-          const short4v b = {static_cast<short>(pb[0]),
-                             static_cast<short>(pb[1]),
-                             static_cast<short>(pb[2]),
-                             static_cast<short>(pb[3])};
-          o_acc[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
-              lds_read_tr4(vb + v_off[dt]), b, o_acc[dt], 0, 0, 0);
+        if constexpr (FP8) {
+          a_v[dt] = fp8_to_bf16(lds_read_tr8(vb + v_off[dt]));
         } else {
-          const short8 b = {
-              static_cast<short>(pb[0]), static_cast<short>(pb[1]),
-              static_cast<short>(pb[2]), static_cast<short>(pb[3]),
-              static_cast<short>(pb[4]), static_cast<short>(pb[5]),
-              static_cast<short>(pb[6]), static_cast<short>(pb[7])};
-          short8 a;
-          if constexpr (FP8) {
-            a = fp8_to_bf16(lds_read_tr8(vb + v_off[dt]));
-          } else {
-            const short4v x = lds_read_tr4(vb + v_off[dt]);
-            const short4v y = lds_read_tr4(vb + v_off[dt] + kPage * kRowB);
-            a = short8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
-          }
-          o_acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              a, b, o_acc[dt], 0, 0, 0);
+          const short4v x = lds_read_tr4(vb + v_off[dt]);
+          const short4v y = PP == 1
+              ? x : lds_read_tr4(vb + v_off[dt] + kPage * kRowB);
+          a_v[dt] = short8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
         }
+      }
+#pragma unroll
+      for (int x = 0; x < (PP == 1 ? 1 : 3); ++x) {
+        const short4v u = pb[x][0], v = PP == 1 ? pb[1][0] : pb[x][PP - 1];
+        const short8 b = {u[0], u[1], u[2], u[3], v[0], v[1], v[2], v[3]};
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+          o_acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              a_v[dt], b, o_acc[dt], 0, 0, 0);
+      }
+      if (PP == 1) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+          o_acc[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+              short4v{a_v[dt][0], a_v[dt][1], a_v[dt][2], a_v[dt][3]},
+              pb[2][0], o_acc[dt], 0, 0, 0);
       }
       if (++ring_slot == kRing) ring_slot = 0;
       ++at.step;
@@ -533,8 +548,8 @@ void paged_attn_join_kernel(const DecodeArgs p, const int heads) {
   float m = kNegInf, l = 0.f, o[V];
 #pragma unroll
   for (int j = 0; j < V; ++j) o[j] = 0.f;
-  // `count` pieces from s0 on, loads first; fewer there: the first again,
-  // with weight 0
+  // `count` pieces from s0 on, loads first; where there are fewer the first
+  // again, as zeros (it may hold infinities) of weight 0
   auto add = [&](int s0, auto count) {
     constexpr int N = decltype(count)::value;
     float pm[N], pl[N], x[N][V];
@@ -551,8 +566,10 @@ void paged_attn_join_kernel(const DecodeArgs p, const int heads) {
         pl[i] = 0.f;
       }
 #pragma unroll
-      for (int j = 0; j < V; ++j)
+      for (int j = 0; j < V; ++j) {
         x[i][j] = p.piece_o[piece * D + lane * V + j];
+        if (!there) x[i][j] = 0.f;
+      }
     }
     float mx = m;
 #pragma unroll

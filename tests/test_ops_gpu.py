@@ -429,6 +429,75 @@ def test_paged_attention_decode_parts(group, hk, lens, scale_by, head_dim,
         off, k_cache, v_cache, bt.to(DEV), sl.to(DEV), scale))
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("group", [1, 4, 8])
+def test_paged_attention_decode_weights_are_fp32(group, head_dim, fp8):
+    """The last value row takes back what the others add up to, so that the
+    sum is far smaller than its terms: a weight of eight bits is off by 2^-9
+    of a term. Bound: the bf16 result's 2^-8 of itself, and 1e-5 of the terms
+    for fp32 scores of 128 products (2^-24 of their 80 or so each) and exp2."""
+    g = torch.Generator().manual_seed(17)
+    bs, hk, lens = 16, 2, [2, 3, 7, 16, 17, 33]
+    cache = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    S, blocks = len(lens), -(-max(lens) // bs)
+    scale = 1.0 / math.sqrt(head_dim)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g).to(cache).double()
+
+    q = torch.randn(S, hk, 1, head_dim, generator=g).to(torch.bfloat16)
+    q = q.expand(-1, -1, group, -1).reshape(S, hk * group, head_dim)
+    k_cache = rnd(S * blocks, hk, bs, head_dim)
+    v_cache = rnd(S * blocks, hk, bs, head_dim)
+    bt = torch.arange(S * blocks, dtype=torch.int32).view(S, blocks)
+    want = torch.empty(S, hk * group, head_dim, dtype=torch.float64)
+    size = torch.empty_like(want)
+    for i, n in enumerate(lens):
+        rows = slice(i * blocks, (i + 1) * blocks)
+        for h in range(hk):
+            k = k_cache[rows, h].reshape(-1, head_dim)[:n]
+            v = v_cache[rows, h].reshape(-1, head_dim)[:n].clone()
+            p = torch.softmax(k @ q[i, h * group].double() * scale, 0)
+            v[-1] = (-(p[:-1] @ v[:-1]) / p[-1]).clamp(-400, 400).to(
+                cache).double()
+            v_cache[i * blocks + (n - 1) // bs, h, (n - 1) % bs] = v[-1]
+            want[i, h * group:(h + 1) * group] = p @ v
+            size[i, h * group:(h + 1) * group] = p @ v.abs()
+    out = ops.paged_attention_decode(
+        q.to(DEV), k_cache.to(cache).to(DEV), v_cache.to(cache).to(DEV),
+        bt.to(DEV), torch.tensor(lens, dtype=torch.int32, device=DEV), scale)
+    err = (out.cpu().double() - want).abs()
+    assert (err <= 2 ** -8 * want.abs() + 1e-5 * size).all(), \
+        (err / size).max()
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_paged_attention_decode_infinite_values(head_dim):
+    """An infinite value makes its column infinite and no other, also where
+    it stands in the context's last row."""
+    bs, lens = 16, [1, 5, 16, 40]
+    S, blocks = len(lens), 3
+    g = torch.Generator().manual_seed(3)
+    q = torch.randn(S, 4, head_dim, generator=g).to(torch.bfloat16)
+    k_cache = torch.randn(S * blocks, 1, bs, head_dim, generator=g).to(q.dtype)
+    v_cache = torch.randn(S * blocks, 1, bs, head_dim, generator=g).to(q.dtype)
+    for i, n in enumerate(lens):
+        v_cache[i * blocks + (n - 1) // bs, 0, (n - 1) % bs, 7] = math.inf
+        v_cache[i * blocks, 0, 0, 9] = -math.inf
+    bt = torch.arange(S * blocks, dtype=torch.int32).view(S, blocks)
+    sl = torch.tensor(lens, dtype=torch.int32)
+    scale = 1.0 / math.sqrt(head_dim)
+    out = ops.paged_attention_decode(q.to(DEV), k_cache.to(DEV),
+                                     v_cache.to(DEV), bt.to(DEV), sl.to(DEV),
+                                     scale).cpu()
+    want = ref.paged_attention_decode(q, k_cache, v_cache, bt, sl, scale)
+    assert (out[..., 7] == math.inf).all() and (out[..., 9] == -math.inf).all()
+    rest = torch.ones(head_dim, dtype=torch.bool)
+    rest[[7, 9]] = False
+    assert_close_bf16(out[..., rest], want[..., rest])
+
+
 # ------------------------------------------------------------ fp8 KV cache
 
 def _fp8_cache(t):
