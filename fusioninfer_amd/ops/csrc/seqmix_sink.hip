@@ -363,13 +363,10 @@ __global__ __launch_bounds__(256) void sink_attention_span_kernel(
     short8 w[3];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      float rest = sc[2 * st + i / 4][i % 4];
+      u16 terms[3];
+      split_weight(sc[2 * st + i / 4][i % 4], terms);
 #pragma unroll
-      for (int x = 0; x < 3; ++x) {
-        const u16 b = f32_to_bf16(rest);
-        w[x][i] = static_cast<short>(b);
-        rest -= bf16_to_f32(b);
-      }
+      for (int x = 0; x < 3; ++x) w[x][i] = static_cast<short>(terms[x]);
     }
     const int row = st * 32 + g4 * 4 + (c16 >> 2);
     const unsigned char* vr = vals + row * kRowB + (lane & 1) * 8;

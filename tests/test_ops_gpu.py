@@ -1243,3 +1243,32 @@ def test_sink_attention_spans(DK, DV, heads, groups, block, window, keep,
                     og[i, h * DV:(h + 1) * DV].double())
             err = (got[i, h].cpu().double() - want).abs()
             assert (err <= want.abs() * 2 ** -8 + 2e-5).all(), (i, h)
+
+
+@pytest.mark.parametrize("DK,DV", [(128, 128), (288, 256)])
+def test_sink_attention_spans_infinite_values(DK, DV):
+    """An infinite value makes its column infinite and no other."""
+    from fusioninfer_amd.ops import seqmix
+
+    g = torch.Generator().manual_seed(DK)
+    ctx, block = [1, 17, 300], 16
+    need = [-(-c // block) for c in ctx]
+    table = torch.zeros(len(ctx), max(need), dtype=torch.int32)
+    for i, n in enumerate(need):
+        table[i, :n] = torch.arange(n) + sum(need[:i])
+    q = torch.randn(len(ctx), 4, DK, generator=g).bfloat16()
+    k = torch.randn(sum(need), 1, block, DK, generator=g).bfloat16()
+    v = torch.randn(sum(need), 1, block, DV, generator=g).bfloat16()
+    for i, c in enumerate(ctx):
+        v[table[i, (c - 1) // block], 0, (c - 1) % block, 7] = math.inf
+        v[table[i, 0], 0, 0, 9] = -math.inf
+    got = seqmix.sink_paged_attention(
+        q.to(DEV), k.to(DEV), v.to(DEV), table.to(DEV),
+        torch.arange(len(ctx), dtype=torch.int32, device=DEV),
+        torch.tensor(ctx, dtype=torch.int32, device=DEV) - 1,
+        DK ** -0.5).view(len(ctx), 4, DV).cpu()
+    assert (got[..., 7] == math.inf).all()
+    assert (got[..., 9] == -math.inf).all()
+    rest = torch.ones(DV, dtype=torch.bool)
+    rest[[7, 9]] = False
+    assert got[..., rest].isfinite().all()
