@@ -36,7 +36,7 @@ void prefill_attn_join_kernel(const PrefillArgs p) {
 #pragma unroll
     for (int g = 0; g < kGroup; ++g) {
       const int s = s0 + g;
-      const bool there = s < cut.z;  // otherwise the first again, weight 0
+      const bool there = s < cut.z;  // otherwise the first again, as zeros
       const int64_t piece =
           static_cast<int64_t>(there ? s * 2 + (s == slot ? 1 : 0)
                                      : slot * 2 + 1) * kWaves + qwave;
@@ -44,7 +44,10 @@ void prefill_attn_join_kernel(const PrefillArgs p) {
       if (!there) ml[g] = make_float2(kPNegInf, 0.f);
       const float* src = p.piece_o + piece * 32 * D + part * kRegs * 64 + lane;
 #pragma unroll
-      for (int r = 0; r < kRegs; ++r) x[g][r] = src[r * 64];
+      for (int r = 0; r < kRegs; ++r) {
+        x[g][r] = src[r * 64];
+        if (!there) x[g][r] = 0.f;     // it may hold infinities
+      }
     }
     float mx = m;
 #pragma unroll

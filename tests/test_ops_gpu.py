@@ -1272,3 +1272,28 @@ def test_sink_attention_spans_infinite_values(DK, DV):
     rest = torch.ones(DV, dtype=torch.bool)
     rest[[7, 9]] = False
     assert got[..., rest].isfinite().all()
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_prefill_attention_parts_infinite_values(head_dim):
+    """Cut K/V ranges: an infinite value makes its column infinite and no
+    other, whichever piece it is in."""
+    bs, ctx, n = 16, 2100, 3
+    g = torch.Generator().manual_seed(4)
+    blocks = -(-ctx // bs)
+    q = torch.randn(n, 8, head_dim, generator=g).bfloat16()
+    k = torch.randn(blocks, 2, bs, head_dim, generator=g).bfloat16()
+    v = torch.randn(blocks, 2, bs, head_dim, generator=g).bfloat16()
+    v[0, :, 3, 5] = math.inf
+    v[70, :, 0, 6] = -math.inf
+    out = ops.prefill_attention_paged(
+        q.to(DEV), k.to(DEV), v.to(DEV),
+        torch.arange(blocks, dtype=torch.int32, device=DEV)[None],
+        torch.tensor([0, n], dtype=torch.int32, device=DEV),
+        torch.tensor([ctx], dtype=torch.int32, device=DEV),
+        head_dim ** -0.5).cpu()
+    assert (out[..., 5] == math.inf).all()
+    assert (out[..., 6] == -math.inf).all()
+    rest = torch.ones(head_dim, dtype=torch.bool)
+    rest[[5, 6]] = False
+    assert out[..., rest].isfinite().all()
