@@ -113,7 +113,10 @@ PrefillPlan plan_prefill_attn(int ntiles, int tile_rows, int num_q_heads,
   const double fill = blocks / 256.0;
   const double idle = fill < 1.0 ? 1.0 - std::min(1.0, 1.4 * fill)
                                  : std::ceil(fill) - 1.04 * fill;
-  if (2 * static_cast<int64_t>(new_rows) > max_k_len || idle * tiles <= 26)
+  // A workgroup's rows lie within one entry of the tile table: the split
+  // form's 256 (one head per workgroup) do not fit into entries of 128.
+  if (pl.rows > tile_rows ||
+      2 * static_cast<int64_t>(new_rows) > max_k_len || idle * tiles <= 26)
     return layout(false);
   // parts of at least eight tiles, in whole rounds over the XCDs
   pl.slots = static_cast<int>(std::min<int64_t>(

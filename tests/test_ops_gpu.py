@@ -371,6 +371,28 @@ def test_prefill_attention_row_blocks_and_parts(hq, hk, ctx_lens, new_lens,
     assert_close_bf16(out.cpu(), want, atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("hq,hk", [(2, 2), (3, 1)])
+def test_prefill_attention_one_head_per_workgroup_small_entries(hq, hk):
+    """4099 new rows make the tile table's entries 128 rows; with one head
+    per workgroup a row still belongs to one workgroup: the same bits every
+    time. Bound as above."""
+    g = torch.Generator().manual_seed(8)
+    D, new, past = 64, 4099, 8205
+    blocks = -(-(new + past) // 16)
+    assert ops.prefill_tile_rows([new]) == 128
+    q = torch.randn(new, hq, D, generator=g).bfloat16().to(DEV)
+    k = torch.randn(blocks, hk, 16, D, generator=g).bfloat16().to(DEV)
+    v = torch.randn(blocks, hk, 16, D, generator=g).bfloat16().to(DEV)
+    bt = torch.randperm(blocks, generator=g).int()[None].to(DEV)
+    cu = torch.tensor([0, new], dtype=torch.int32, device=DEV)
+    lens = torch.tensor([new + past], dtype=torch.int32, device=DEV)
+    outs = [ops.prefill_attention_paged(q, k, v, bt, cu, lens, D ** -0.5)
+            for _ in range(3)]
+    want = ref.prefill_attention_paged(q, k, v, bt, cu, lens, D ** -0.5)
+    assert_close_bf16(outs[0], want, atol=2e-2, rtol=2e-2)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("head_dim", [64, 128])
 @pytest.mark.parametrize(
