@@ -354,6 +354,7 @@ void part_gemm_join_kernel(u16* __restrict__ out,
   const int lane = i % kWaveSize;
   const int c = i / kWaveSize % CF, f = i / kWaveSize / CF % kUse;
   const int wave = i / kWaveSize / CF / kUse;
+  if (wave >= S::kWaves) return;                 // the last block's rest
   const int wn = wave / S::WM, wm = wave % S::WM;
   const int m = (wm * CF + c) * 16 + (lane & 15);
   const int n = tile * (SILU_MUL ? S::TN / 2 : S::TN) +
@@ -433,7 +434,7 @@ void launch_part(const Plan& pl, u16* out, float* pieces, const u16* x,
   if (!pl.split || pl.parts == 1) return;
   hipLaunchKernelGGL((part_gemm_join_kernel<S, SILU_MUL, FP8>),
                      dim3(pl.parts - 1,
-                          S::kPiece / (SILU_MUL ? 2 : 1) / 256),
+                          ceil_div(S::kPiece / (SILU_MUL ? 2 : 1), 256)),
                      dim3(256), 0, stream, out, p, bias, scales, M, N, K,
                      out_stride, pl.tiles, pl.parts);
 }

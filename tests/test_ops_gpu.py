@@ -1003,6 +1003,23 @@ def test_linear_in_parts(rows, n, k, bias):
                 <= want.abs() * 2 ** -8 + 1e-3 * k ** 0.5).all()
 
 
+@pytest.mark.parametrize("rows", [17, 32])
+def test_linear_silu_mul_in_parts_of_96_rows(rows):
+    """One tile of 96 rows in many pieces, whose kept third of a wave's
+    results fills one and a half blocks of the join. x is scaled so that the
+    products are of size one: a bf16 rounding of the result (2^-9 relative)
+    and fp32 sums (16 and 256 additions of 2^-24 each, a few of that)."""
+    g = torch.Generator().manual_seed(rows)
+    n, k = 96, 1 << 17
+    w = torch.randn(n, k, generator=g).to(torch.bfloat16).to(DEV)
+    x = (torch.randn(rows, k, generator=g) / 256).to(torch.bfloat16).to(DEV)
+    assert ops._skinny_ok(x, w, 32, True)
+    prod = x.double() @ w.double().T
+    want = torch.nn.functional.silu(prod[:, : n // 2]) * prod[:, n // 2:]
+    err = (ops.linear_silu_mul(x, w).double() - want).abs()
+    assert (err <= want.abs() * 2 ** -8 + 1e-4).all()
+
+
 @pytest.mark.parametrize("rows", [1, 32, 33, 64, 65, 128, 129, 256])
 @pytest.mark.parametrize("n,k", [
     (16, 256),           # one ragged tile, one or two stages
