@@ -287,6 +287,19 @@ void scatter_kv_blocks(at::Tensor staging, at::Tensor k_cache,
       block_elems, current_stream());
 }
 
+// What 16-byte pieces are copied from straight to LDS starts on their grid:
+// the tensor itself or a copy.
+at::Tensor dma_whole(const at::Tensor& t) {
+  if (reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0) return t;
+  return t.clone(at::MemoryFormat::Contiguous);
+}
+
+// and so does every row, at 32-bit byte offsets within a tile of 64
+at::Tensor dma_rows(const at::Tensor& t) {
+  if (t.stride(0) % 8 == 0 && t.stride(0) <= (1 << 24)) return dma_whole(t);
+  return t.clone(at::MemoryFormat::Contiguous);
+}
+
 void paged_attention_decode(at::Tensor out, at::Tensor q, at::Tensor k_cache,
                             at::Tensor v_cache, at::Tensor block_tables,
                             at::Tensor seq_lens, double scale) {
@@ -310,10 +323,9 @@ void paged_attention_decode(at::Tensor out, at::Tensor q, at::Tensor k_cache,
               "decode attention takes head sizes 64 and 128 and 1, 2, 4 or 8 "
               "query heads per K/V head");
   if (num_seqs == 0) return;
-  // query rows are copied in 16-byte pieces
-  if (q.stride(0) % 8 != 0 ||
-      reinterpret_cast<uintptr_t>(q.data_ptr()) % 16 != 0)
-    q = q.clone(at::MemoryFormat::Contiguous);
+  q = dma_rows(q);
+  k_cache = dma_whole(k_cache);
+  v_cache = dma_whole(v_cache);
   at::Tensor pieces = at::empty(
       {fi::decode_piece_floats(num_seqs, num_kv_heads, head_dim,
                                num_heads / num_kv_heads)},
@@ -351,6 +363,8 @@ void prefill_attention(at::Tensor out, at::Tensor q, at::Tensor k,
   TORCH_CHECK(q.stride(2) == 1 && q.stride(1) == head_dim);
   TORCH_CHECK(k.stride(2) == 1 && k.stride(1) == head_dim);
   TORCH_CHECK(v.stride(2) == 1 && v.stride(1) == head_dim);
+  k = dma_rows(k);
+  v = dma_rows(v);
   const fi::PrefillPlan pl = fi::plan_prefill_attn(
       tile_seq.size(0), tile_rows, num_q_heads, num_kv_heads, q.size(0),
       k.size(0));
@@ -387,6 +401,8 @@ void prefill_attention_paged(at::Tensor out, at::Tensor q, at::Tensor k_cache,
   const int num_kv_heads = k_cache.size(1);
   TORCH_CHECK(k_cache.size(2) == 16, "cache block_size must be 16");
   TORCH_CHECK(q.stride(2) == 1 && q.stride(1) == head_dim);
+  k_cache = dma_whole(k_cache);
+  v_cache = dma_whole(v_cache);
   const fi::PrefillPlan pl = fi::plan_prefill_attn(
       tile_seq.size(0), tile_rows, num_q_heads, num_kv_heads, q.size(0),
       block_tables.size(1) * 16);

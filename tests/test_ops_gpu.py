@@ -263,6 +263,46 @@ def test_prefill_attention(head_dim, seq_lens, hq, hk):
     assert_close_bf16(out.cpu(), expected, atol=3e-2, rtol=3e-2)
 
 
+def _shifted(t, by):
+    """t's values in a tensor that starts `by` elements off the grid."""
+    flat = torch.empty(t.numel() + by, dtype=t.dtype, device=t.device)
+    return flat[by:].view(t.shape).copy_(t)
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("pad,by", [(4, 0), (8, 1), (1, 3)])
+def test_attention_rows_off_the_16_byte_grid(head_dim, pad, by):
+    """K, V and caches whose rows or start lie off the grid of the 16-byte
+    copies give the bits that the same values on the grid give."""
+    g = torch.Generator().manual_seed(head_dim + pad)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g).to(torch.bfloat16).to(DEV)
+
+    T, hk, w = 130, 2, 2 * head_dim
+    q, k, v = rnd(T, 4, head_dim), rnd(T, hk, head_dim), rnd(T, hk, head_dim)
+    cu = torch.tensor([0, 33, T], dtype=torch.int32, device=DEV)
+    wide = _shifted(torch.cat([k.view(T, w), v.view(T, w), rnd(T, pad)], 1),
+                    by)
+    scale = head_dim ** -0.5
+    assert torch.equal(
+        ops.prefill_attention(q, k, v, cu, scale),
+        ops.prefill_attention(q, wide[:, :w].view(T, hk, head_dim),
+                              wide[:, w:2 * w].view(T, hk, head_dim), cu,
+                              scale))
+    kc, vc = rnd(9, hk, 16, head_dim), rnd(9, hk, 16, head_dim)
+    off = _shifted(kc, by), _shifted(vc, by)
+    bt = torch.randperm(9, generator=g).int()[None].to(DEV)
+    lens = torch.tensor([140], dtype=torch.int32, device=DEV)
+    one = torch.tensor([0, 1], dtype=torch.int32, device=DEV)
+    assert torch.equal(
+        ops.paged_attention_decode(q[:1], kc, vc, bt, lens, scale),
+        ops.paged_attention_decode(q[:1], *off, bt, lens, scale))
+    assert torch.equal(
+        ops.prefill_attention_paged(q[:1], kc, vc, bt, one, lens, scale),
+        ops.prefill_attention_paged(q[:1], *off, bt, one, lens, scale))
+
+
 def test_prefill_attention_spiked_scores():
     """Force large per-tile max jumps so online-softmax rescale paths fire
     (bounded random data never exercises them)."""
