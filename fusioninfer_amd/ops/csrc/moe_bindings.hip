@@ -93,10 +93,6 @@ void moe_gemm(at::Tensor out, at::Tensor a, at::Tensor b_packed,
   TORCH_CHECK(expert_ids.size(0) >= PM / block_m);
   if (mode != 0) TORCH_CHECK(sorted_ids.size(0) >= PM);
   if (mode == 0) TORCH_CHECK(a.size(0) >= PM);
-  // 32-bit byte offsets into the rows and into one expert's weights
-  TORCH_CHECK(a.numel() < (int64_t(1) << 31) &&
-              b_packed.numel() / std::max<int64_t>(b_packed.size(0), 1) <
-                  (int64_t(1) << 31), "moe_gemm: operands over 4 GB");
   fi::launch_moe_gemm(bf16_ptr(out), bf16_cptr(a),
                       bf16_cptr(b_packed), sorted_ids.data_ptr<int>(),
                       expert_ids.data_ptr<int>(), n_valid.data_ptr<int>(),

@@ -28,7 +28,8 @@ namespace fi {
 void launch_moe_tile(u16*, const u16*, const u16*, const int*, const int*,
                      const int*, int, int, int, int, int, float, hipStream_t);
 void launch_moe_stream(u16*, const u16*, const u16*, const int*, const int*,
-                       const int*, int, int, int, int, float, hipStream_t);
+                       const int*, int, int, int, int, int, float,
+                       hipStream_t);
 
 namespace {
 
@@ -250,13 +251,18 @@ void launch_moe_gemm(u16* out, const u16* a, const u16* b,
                      const int* n_valid, int max_mtiles, int rows, int K,
                      int N, int block_m, int mode, float limit,
                      hipStream_t stream) {
-  if (block_m == 16) {
+  // The tiles read gathered rows and one expert's weights at 32-bit byte
+  // offsets; operands beyond those go through the streaming kernel, which
+  // takes a block of 128 rows as eight of 16.
+  const int64_t limit32 = int64_t(1) << 31;      // bf16 values in 4 GB
+  const int NB = mode == 1 || mode == 3 ? 2 * N : N;
+  if (block_m == 16 || static_cast<int64_t>(K) * NB >= limit32 ||
+      (mode != 0 && static_cast<int64_t>(rows) * K >= limit32))
     launch_moe_stream(out, a, b, sorted_ids, expert_ids, n_valid, max_mtiles,
-                      K, N, mode, limit, stream);
-  } else {  // block_m == 128
+                      block_m == 16 ? 0 : 3, K, N, mode, limit, stream);
+  else
     launch_moe_tile(out, a, b, sorted_ids, expert_ids, n_valid, max_mtiles,
                     rows, K, N, mode, limit, stream);
-  }
 }
 
 void launch_moe_gemm_fp8(u16* out, const unsigned char* a,

@@ -11,7 +11,9 @@
 // registers from one unit to the next (KEEP) where the slice fits: rows read
 // again for every 16 columns cost half the weights' traffic between L2 and
 // the CUs, which ends at about 10 TB/s. The waves' sums meet in LDS, one
-// barrier per unit, one wave after the other writing the result.
+// barrier per unit, one wave after the other writing the result. All rows and
+// weights are addressed in 64 bits: blocks of 128 rows whose operands are too
+// large for the tiles' 32-bit offsets come here as eight of 16.
 //
 // The fragments of the weights are the first operand, so a lane ends with
 // four neighbouring columns of one row.
@@ -50,9 +52,9 @@ void moe_stream_kernel(
     const u16* __restrict__ a,          // MODE 0: act [PM, K]; else x [T, K]
     const u16* __restrict__ b,          // [E][K/32][NB/16][64][8] bf16
     const int* __restrict__ sorted_ids, // [PM] token row per padded slot
-    const int* __restrict__ expert_ids, // [PM/16] local expert per block
-    const int* __restrict__ n_valid,    // device scalar: blocks in use
-    const int K, const int N, const float limit) {
+    const int* __restrict__ expert_ids, // local expert of 16 << per rows
+    const int* __restrict__ n_valid,    // device scalar: those in use
+    const int per, const int K, const int N, const float limit) {
   constexpr bool GATE_UP = MODE == 1 || MODE == 3;
   constexpr int NF = GATE_UP ? 2 * COLS : COLS;   // fragments per step
   __shared__ floatx4 sums[2][kStreamWaves][NF][kWaveSize];
@@ -60,11 +62,11 @@ void moe_stream_kernel(
   const int lane = threadIdx.x % kWaveSize;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
   const int per_block = N / (16 * COLS);          // units of a row block
-  const int units = *n_valid * per_block;
-  const int per = units / gridDim.x, rem = units % gridDim.x;
+  const int units = (*n_valid << per) * per_block;
+  const int each = units / gridDim.x, rem = units % gridDim.x;
   const int part = blockIdx.x;
-  const int lo = part * per + min(part, rem);
-  const int hi = lo + per + (part < rem ? 1 : 0);
+  const int lo = part * each + min(part, rem);
+  const int hi = lo + each + (part < rem ? 1 : 0);
   if (lo >= hi) return;
 
   const int NB16 = (GATE_UP ? 2 * N : N) / 16;
@@ -90,7 +92,7 @@ void moe_stream_kernel(
     const int slot = m * 16 + (lane & 15);
     const int row = MODE != 0 ? sorted_ids[slot] : slot;
     a_row = a + static_cast<int64_t>(row) * K + (lane >> 4) * 8;
-    b_e = b + static_cast<int64_t>(expert_ids[m]) * steps * NB16 * 512 +
+    b_e = b + static_cast<int64_t>(expert_ids[m >> per]) * steps * NB16 * 512 +
           lane * 8;
   };
   auto load_rows = [&](short8* v, int s0) {
@@ -220,15 +222,15 @@ void moe_stream_kernel(
 template <int MODE>
 void launch_stream(u16* out, const u16* a, const u16* b,
                    const int* sorted_ids, const int* expert_ids,
-                   const int* n_valid, int blocks, int K, int N, float limit,
-                   hipStream_t stream) {
+                   const int* n_valid, int blocks, int per, int K, int N,
+                   float limit, hipStream_t stream) {
   constexpr bool gate = MODE == 1 || MODE == 3;
   const int span = ceil_div(K / 32, kStreamWaves);   // steps per wave
-  const int units = blocks * (N / 16);               // at the most
+  const int units = (blocks << per) * (N / 16);      // at the most
   auto run = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(std::min(units, 256)),
                        dim3(kStreamWaves * kWaveSize), 0, stream, out, a, b,
-                       sorted_ids, expert_ids, n_valid, K, N, limit);
+                       sorted_ids, expert_ids, n_valid, per, K, N, limit);
   };
   // sixteen loads together, fewer where K gives a wave only two or three
   // steps (K = 512, 16 experts of 1536 columns: 2 steps by 32 columns 7.0 us
@@ -247,14 +249,15 @@ void launch_stream(u16* out, const u16* a, const u16* b,
 
 }  // namespace
 
-// row blocks of 16, K a multiple of 32, N of 64
+// row blocks of 16 << per rows, K a multiple of 32, N of 64
 void launch_moe_stream(u16* out, const u16* a, const u16* b,
                        const int* sorted_ids, const int* expert_ids,
-                       const int* n_valid, int blocks, int K, int N, int mode,
-                       float limit, hipStream_t stream) {
+                       const int* n_valid, int blocks, int per, int K, int N,
+                       int mode, float limit, hipStream_t stream) {
   auto* f = mode == 0 ? &launch_stream<0> : mode == 1 ? &launch_stream<1>
       : mode == 2 ? &launch_stream<2> : &launch_stream<3>;
-  f(out, a, b, sorted_ids, expert_ids, n_valid, blocks, K, N, limit, stream);
+  f(out, a, b, sorted_ids, expert_ids, n_valid, blocks, per, K, N, limit,
+    stream);
 }
 
 }  // namespace fi

@@ -1214,6 +1214,51 @@ def check_moe_gemm(k, n, gate_up, act, bm):
         assert (err <= y.abs() * 2 ** -8 + slack).all(), m
 
 
+@pytest.mark.parametrize("bm", [16, 128])
+@pytest.mark.parametrize("act,gate_up", [(None, True), ("relu_sq", False)])
+def test_moe_gemm_rows_over_4_gb(bm, act, gate_up):
+    """Gathered rows at both ends of 2^31 values and more; bound as above."""
+    g = torch.Generator().manual_seed(bm)
+    T, k, n = (1 << 20) + 64, 2048, 64
+    x = torch.empty(T, k, dtype=torch.bfloat16, device=DEV)
+    ids = torch.cat([torch.arange(64), torch.arange(T - 64, T)])
+    ids = ids[torch.randperm(128, generator=g)].int().to(DEV)
+    x[:64] = torch.randn(64, k, generator=g).to(x.dtype).to(DEV)
+    x[-64:] = torch.randn(64, k, generator=g).to(x.dtype).to(DEV)
+    w = torch.randn(1, k, 2 * n if gate_up else n, generator=g)
+    w = (w / 32).to(x.dtype).to(DEV)
+    out = torch.empty(128, n, dtype=x.dtype, device=DEV)
+    ops.moe_gemm(out, x, ops.pack_moe_weights(w), ids,
+                 torch.zeros(128 // bm, dtype=torch.int32, device=DEV),
+                 torch.tensor([128 // bm], dtype=torch.int32, device=DEV), bm,
+                 gate_up, act, 0.0)
+    y = x[ids.long()].double() @ w[0].double()
+    y = torch.nn.functional.silu(y[:, :n]) * y[:, n:] if gate_up \
+        else y.clamp(min=0).square()
+    assert ((out.double() - y).abs() <= y.abs() * 2 ** -8 + 1e-4).all()
+
+
+@pytest.mark.parametrize("bm", [16, 128])
+def test_moe_gemm_expert_of_4_gb(bm):
+    """An expert of 2^31 values: its first and last fragments are found."""
+    g = torch.Generator().manual_seed(bm)
+    k, n = 1 << 15, 1 << 16
+    part = torch.randn(2, 32, 16, generator=g).bfloat16().to(DEV)
+    b = torch.zeros(1, k // 32, n // 16, 64, 8, dtype=torch.bfloat16,
+                    device=DEV)
+    b[0, 0, 0], b[0, -1, -1] = ops.pack_moe_weights(part)[:, 0, 0]
+    a = torch.randn(128, k, generator=g).bfloat16().to(DEV)
+    out = torch.empty(128, n, dtype=torch.bfloat16, device=DEV)
+    ops.moe_gemm(out, a, b, torch.zeros(128, dtype=torch.int32, device=DEV),
+                 torch.zeros(128 // bm, dtype=torch.int32, device=DEV),
+                 torch.tensor([128 // bm], dtype=torch.int32, device=DEV), bm,
+                 False, None, 0.0)
+    for got, y in ((out[:, :16], a[:, :32].double() @ part[0].double()),
+                   (out[:, -16:], a[:, -32:].double() @ part[1].double())):
+        assert ((got.double() - y).abs() <= y.abs() * 2 ** -8 + 1e-4).all()
+    assert not out[:, 16:-16].any()
+
+
 # --------------------------- attention with sink, gate and window, bf16 rows
 
 
