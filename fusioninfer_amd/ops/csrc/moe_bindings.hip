@@ -93,6 +93,9 @@ void moe_gemm(at::Tensor out, at::Tensor a, at::Tensor b_packed,
   TORCH_CHECK(expert_ids.size(0) >= PM / block_m);
   if (mode != 0) TORCH_CHECK(sorted_ids.size(0) >= PM);
   if (mode == 0) TORCH_CHECK(a.size(0) >= PM);
+  // rows go to LDS by DMA in 16-byte pieces
+  if (block_m == 128 && reinterpret_cast<uintptr_t>(a.data_ptr()) % 16 != 0)
+    a = a.clone();
   fi::launch_moe_gemm(bf16_ptr(out), bf16_cptr(a),
                       bf16_cptr(b_packed), sorted_ids.data_ptr<int>(),
                       expert_ids.data_ptr<int>(), n_valid.data_ptr<int>(),

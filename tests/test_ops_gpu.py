@@ -1259,6 +1259,26 @@ def test_moe_gemm_expert_of_4_gb(bm):
     assert not out[:, 16:-16].any()
 
 
+@pytest.mark.parametrize("bm", [16, 128])
+@pytest.mark.parametrize("gate_up", [True, False])
+def test_moe_gemm_rows_off_the_16_byte_grid(bm, gate_up):
+    """Rows that start off the grid give the bits of rows on it."""
+    g = torch.Generator().manual_seed(bm)
+    x = torch.randn(128, 256, generator=g).bfloat16().to(DEV)
+    w = ops.pack_moe_weights(
+        torch.randn(1, 256, 256, generator=g).bfloat16().to(DEV))
+    ids = torch.randperm(128, generator=g).int().to(DEV)
+    outs = []
+    for a in (x, _shifted(x, 3)):
+        outs.append(torch.empty(128, 128 if gate_up else 256, dtype=x.dtype,
+                                device=DEV))
+        ops.moe_gemm(outs[-1], a, w, ids,
+                     torch.zeros(128 // bm, dtype=torch.int32, device=DEV),
+                     torch.tensor([128 // bm], dtype=torch.int32, device=DEV),
+                     bm, gate_up)
+    assert torch.equal(*outs)
+
+
 # --------------------------- attention with sink, gate and window, bf16 rows
 
 
