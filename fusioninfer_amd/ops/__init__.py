@@ -132,6 +132,7 @@ def linear(x: torch.Tensor, w: torch.Tensor,
     that, anything else is the library's GEMM."""
     if _skinny_ok(x, w, 16) and (bias is None or (
             bias.dtype == torch.bfloat16 and bias.is_contiguous()
+            and bias.shape == w.shape[:1]    # others broadcast: the library
             and not (torch.is_grad_enabled() and bias.requires_grad))):
         out = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype,
                           device=x.device)

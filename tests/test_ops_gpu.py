@@ -1138,6 +1138,20 @@ def test_skinny_linear_leaves_other_calls_to_the_library():
     assert x.grad is not None
 
 
+@pytest.mark.parametrize("rows", [4, 64])
+@pytest.mark.parametrize("shape", [(1,), (), ("rows", 1), (1, 64),
+                                   ("rows", 64)])
+def test_linear_bias_that_broadcasts(rows, shape):
+    """A bias of another shape than [N] gives what torch gives."""
+    def rnd(*shape):
+        return torch.randn(shape, device=DEV).to(torch.bfloat16)
+
+    x, w = rnd(rows, 256), rnd(64, 256)
+    b = rnd(*[rows if d == "rows" else d for d in shape])
+    torch.testing.assert_close(ops.linear(x, w, b),
+                               torch.nn.functional.linear(x, w, b))
+
+
 # ------------------------------------------------- grouped GEMM, 128 rows
 
 
