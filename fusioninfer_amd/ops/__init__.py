@@ -13,6 +13,7 @@ import math
 from typing import Optional
 
 import torch
+from torch.autograd import forward_ad
 
 from fusioninfer_amd.ops import reference as ref
 
@@ -104,13 +105,34 @@ def _streams(M: int, N: int, K: int, silu_mul: bool = False) -> bool:
                           or silu_mul and 224 < -(-N // 96) <= 256)
 
 
-def _skinny_ok(x, w, unit: int, silu_mul: bool = False) -> bool:
-    """Whether x W^T can run on the streaming kernels: few bf16 rows, whole
-    128-value stages of K, whole tiles of N, 16-byte aligned rows, nothing
-    to differentiate. A family that builds only its own extension keeps the
-    library's GEMM."""
+def _memory_alone(*tensors: torch.Tensor) -> bool:
+    """Whether a call is about its operands' memory and nothing else. The
+    kernels see no tracing or compilation, functional transform, dispatch or
+    autocast mode, tensor subclass, gradient or tangent; torch's own
+    operations carry all of them."""
     return (
-        _C is not None and x.is_cuda and w.is_cuda and x.dim() == 2 and w.dim() == 2
+        not torch.compiler.is_compiling() and not torch._C._is_tracing()
+        and torch._C._functorch.maybe_current_level() is None
+        and forward_ad._current_level < 0
+        and torch._C._len_torch_dispatch_stack() == 0
+        and not torch.overrides.has_torch_function(tensors)
+        and not torch.is_autocast_enabled("cuda")
+        and all(type(t) in (torch.Tensor, torch.nn.Parameter)
+                for t in tensors)
+        and not (torch.is_grad_enabled()
+                 and any(t.requires_grad for t in tensors))
+    )
+
+
+def _skinny_ok(x, w, unit: int, silu_mul: bool = False, bias=None) -> bool:
+    """Whether x W^T (+ bias) can run on the streaming kernels: few bf16
+    rows, whole 128-value stages of K, whole tiles of N, 16-byte aligned
+    rows, a bias of [N], an eager call without gradients. A family that
+    builds only its own extension keeps the library's GEMM."""
+    return (
+        _C is not None
+        and _memory_alone(*((x, w) if bias is None else (x, w, bias)))
+        and x.is_cuda and w.is_cuda and x.dim() == 2 and w.dim() == 2
         and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
         and 1 <= x.shape[0] <= PART_ROWS
         and x.shape[1] == w.shape[1] and 0 < x.shape[1] <= 1 << 24
@@ -121,8 +143,9 @@ def _skinny_ok(x, w, unit: int, silu_mul: bool = False) -> bool:
         and _streams(x.shape[0], w.shape[0], x.shape[1], silu_mul)
         and w.is_contiguous()
         and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-        and not (torch.is_grad_enabled()
-                 and (x.requires_grad or w.requires_grad))
+        and (bias is None or (
+            bias.dtype == torch.bfloat16 and bias.is_contiguous()
+            and bias.shape == w.shape[:1]))
     )
 
 
@@ -130,10 +153,7 @@ def linear(x: torch.Tensor, w: torch.Tensor,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x W^T (+ bias): a few bf16 rows stream W once through the kernels for
     that, anything else is the library's GEMM."""
-    if _skinny_ok(x, w, 16) and (bias is None or (
-            bias.dtype == torch.bfloat16 and bias.is_contiguous()
-            and bias.shape == w.shape[:1]    # others broadcast: the library
-            and not (torch.is_grad_enabled() and bias.requires_grad))):
+    if _skinny_ok(x, w, 16, bias=bias):
         out = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype,
                           device=x.device)
         _C.few_rows_gemm(out, x, w, bias, False)

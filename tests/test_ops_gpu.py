@@ -1139,6 +1139,55 @@ def test_skinny_linear_leaves_other_calls_to_the_library():
 
 
 @pytest.mark.parametrize("rows", [4, 64])
+def test_linear_under_transforms_and_modes(rows):
+    """Batching, tangents, traces, operator modes and autocast reach the
+    product of a linear layer as they reach torch's."""
+    from torch.autograd import forward_ad
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils.flop_counter import FlopCounterMode
+
+    F = torch.nn.functional
+
+    def rnd(*shape):
+        return torch.randn(shape, device=DEV).to(torch.bfloat16)
+
+    x, t, w, b = rnd(rows, 256), rnd(rows, 256), rnd(64, 256), rnd(64)
+    batch = rnd(3, rows, 256)
+
+    def tangent(linear):
+        with forward_ad.dual_level():
+            out = linear(forward_ad.make_dual(x, t), w, b)
+            return forward_ad.unpack_dual(out).tangent
+
+    def flops(linear):
+        with FlopCounterMode(display=False) as count:
+            linear(x, w, b)
+        return torch.tensor(count.get_total_flops())
+
+    def autocast(linear):
+        with torch.autocast("cuda", torch.float16):
+            return linear(x, w, b)
+
+    for way in (
+        lambda f: torch.vmap(lambda v: f(v, w, b))(batch),
+        lambda f: torch.func.jvp(lambda v: f(v, w, b), (x,), (t,))[1],
+        lambda f: torch.func.grad(lambda v: f(v, w, b).sum())(x),
+        lambda f: make_fx(lambda v: f(v, w, b))(x)(t),
+        lambda f: torch.jit.trace(lambda v: f(v, w, b), x)(t),
+        tangent, flops, autocast,
+    ):
+        torch.testing.assert_close(way(ops.linear), way(F.linear))
+
+    class Named(torch.Tensor):
+        pass
+
+    assert type(ops.linear(x.as_subclass(Named), w)) is Named
+    x.requires_grad_()
+    ops.linear(x, w).sum().backward()
+    assert x.grad is not None
+
+
+@pytest.mark.parametrize("rows", [4, 64])
 @pytest.mark.parametrize("shape", [(1,), (), ("rows", 1), (1, 64),
                                    ("rows", 64)])
 def test_linear_bias_that_broadcasts(rows, shape):
