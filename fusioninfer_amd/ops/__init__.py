@@ -124,6 +124,14 @@ def _memory_alone(*tensors: torch.Tensor) -> bool:
     )
 
 
+def _on_current_gpu(*tensors: torch.Tensor) -> bool:
+    """Whether all lie on the GPU that a launch goes to; torch's operations
+    follow their operands or refuse a mixture."""
+    d = tensors[0].device
+    return (d.type == "cuda" and all(t.device == d for t in tensors[1:])
+            and d.index == torch.cuda.current_device())
+
+
 def _skinny_ok(x, w, unit: int, silu_mul: bool = False, bias=None) -> bool:
     """Whether x W^T (+ bias) can run on the streaming kernels: few bf16
     rows, whole 128-value stages of K, whole tiles of N, 16-byte aligned
@@ -132,7 +140,8 @@ def _skinny_ok(x, w, unit: int, silu_mul: bool = False, bias=None) -> bool:
     return (
         _C is not None
         and _memory_alone(*((x, w) if bias is None else (x, w, bias)))
-        and x.is_cuda and w.is_cuda and x.dim() == 2 and w.dim() == 2
+        and _on_current_gpu(*((x, w) if bias is None else (x, w, bias)))
+        and x.dim() == 2 and w.dim() == 2
         and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
         and 1 <= x.shape[0] <= PART_ROWS
         and x.shape[1] == w.shape[1] and 0 < x.shape[1] <= 1 << 24
@@ -185,7 +194,8 @@ def linear_fp8(x: torch.Tensor, x_scales: torch.Tensor, w: torch.Tensor,
                w_scales: torch.Tensor) -> torch.Tensor:
     """(x * x_scales) (w * w_scales)^T in bf16 on the GPU: x [M, K] and w
     [N, K] e4m3, a scale per row each."""
-    if (_C is not None and x.dim() == 2 and w.dim() == 2
+    if (_C is not None and _on_current_gpu(x, x_scales, w, w_scales)
+            and x.dim() == 2 and w.dim() == 2
             and x.dtype == w.dtype == torch.float8_e4m3fn
             and x.shape[0] >= 1 and x.shape[1] == w.shape[1]
             and x.shape[1] % 256 == 0 and w.shape[0] % 16 == 0

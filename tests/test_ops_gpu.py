@@ -1138,6 +1138,29 @@ def test_skinny_linear_leaves_other_calls_to_the_library():
     assert x.grad is not None
 
 
+def test_linear_elsewhere_than_on_the_current_gpu(monkeypatch):
+    """Operands of another GPU than the current one, or of two places, are
+    torch's to follow or refuse."""
+    f8 = torch.float8_e4m3fn
+    x = torch.randn(4, 4096, device=DEV).to(torch.bfloat16)
+    w = torch.randn(4096, 4096, device=DEV).to(torch.bfloat16)
+    b = torch.zeros(4096, dtype=torch.bfloat16)
+    assert ops._skinny_ok(x, w, 16)
+    with pytest.raises(RuntimeError, match="same device"):
+        ops.linear(x, w.cpu())
+    with pytest.raises(RuntimeError, match="same device"):
+        ops.linear(x, w, b)
+    calls = []
+    for name in ("few_rows_gemm", "few_rows_gemm_fp8"):
+        monkeypatch.setattr(ops._C, name, lambda *a: calls.append(a))
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    assert torch.equal(ops.linear(x, w), torch.nn.functional.linear(x, w))
+    ops.linear_silu_mul(x, w)
+    ops.linear_fp8(x.to(f8), torch.ones(4, device=DEV), w.to(f8),
+                   torch.ones(4096, device=DEV))
+    assert not calls
+
+
 @pytest.mark.parametrize("rows", [4, 64])
 def test_linear_under_transforms_and_modes(rows):
     """Batching, tangents, traces, operator modes and autocast reach the
