@@ -80,6 +80,19 @@ class MergedColumnParallelLinear(nn.Module):
         return ops.linear(x, self.weight, self.bias)
 
 
+def weight_alone(layer: nn.Module) -> bool:
+    """Whether calling a MergedColumnParallelLinear is x W^T and nothing
+    else, so that a kernel that goes on from there may take its place: no
+    bias, no forward of another class or set on the instance, no hook."""
+    return (
+        type(layer) is MergedColumnParallelLinear and layer.bias is None
+        and "forward" not in vars(layer)
+        and not (layer._forward_hooks or layer._forward_pre_hooks
+                 or layer._backward_hooks or layer._backward_pre_hooks)
+        and not torch.nn.modules.module._has_any_global_hook()
+    )
+
+
 class RowParallelLinear(nn.Module):
     """Y = X W^T with W sharded along the input dim; all-reduce on forward."""
 

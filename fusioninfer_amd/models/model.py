@@ -23,6 +23,7 @@ from fusioninfer_amd.distributed.layers import (
     MergedColumnParallelLinear,
     ReplicatedLinear,
     RowParallelLinear,
+    weight_alone,
 )
 from fusioninfer_amd.engine.metadata import AttnMetadata
 
@@ -155,8 +156,10 @@ class MLP(nn.Module):
             return self.down_proj.forward_with_lora(
                 ops.silu_and_mul(gu), lora, self.layer_idx, "down"
             )
-        return self.down_proj(
-            ops.linear_silu_mul(x, self.gate_up_proj.weight))
+        if weight_alone(self.gate_up_proj):
+            return self.down_proj(
+                ops.linear_silu_mul(x, self.gate_up_proj.weight))
+        return self.down_proj(ops.silu_and_mul(self.gate_up_proj(x)))
 
 
 class MoEMLP(nn.Module):
