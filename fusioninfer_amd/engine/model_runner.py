@@ -187,9 +187,13 @@ class ModelRunner:
     def _host_array(values, dtype):
         code, np_type = _HOST_TYPES[dtype]
         if isinstance(values, list):
-            # array reads a list of ints three times as fast as torch
-            values = np.frombuffer(array(code, values), dtype=np_type) \
-                if values else np.empty(0, dtype=np_type)
+            # array reads a list of ints three times as fast as torch, which
+            # takes whatever else counts as a number
+            try:
+                values = np.frombuffer(array(code, values), dtype=np_type) \
+                    if values else np.empty(0, dtype=np_type)
+            except TypeError:
+                values = torch.tensor(values, dtype=dtype).numpy()
         return np.ascontiguousarray(values, dtype=np_type)
 
     @staticmethod

@@ -30,6 +30,16 @@ def test_to_device_keeps_values_types_and_shapes(runner):
         assert v.is_contiguous() and v.data_ptr() % 16 == 0
 
 
+def test_to_device_takes_what_a_tensor_takes(runner):
+    """Token ids that a client sent as 7.0, scalars of torch and numpy."""
+    for values in ([3, 7.0, True], [torch.tensor(5), 2], [np.float32(4), 1],
+                   [[1, 2], [3, 4]]):
+        t = runner._to_device({"a": (values, torch.long),
+                               "b": (values, torch.int32)})
+        want = torch.tensor(values, dtype=torch.long)
+        assert torch.equal(t["a"], want) and torch.equal(t["b"], want.int())
+
+
 def test_values_out_of_range_are_refused(runner):
     with pytest.raises(OverflowError):
         runner._to_device({"a": ([2 ** 31], torch.int32)})
