@@ -32,7 +32,7 @@ def test_to_device_keeps_values_types_and_shapes(runner):
 
 def test_to_device_takes_what_a_tensor_takes(runner):
     """Token ids that a client sent as 7.0, scalars of torch and numpy."""
-    for values in ([3, 7.0, True], [torch.tensor(5), 2], [np.float32(4), 1],
+    for values in ([3, 7.0, True], [torch.tensor(5), 2], [np.int64(4), 1.0],
                    [[1, 2], [3, 4]]):
         t = runner._to_device({"a": (values, torch.long),
                                "b": (values, torch.int32)})
