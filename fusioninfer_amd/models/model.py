@@ -494,8 +494,8 @@ class MoEMLP(nn.Module):
         - pos [T*topk] int32: padded slot per assignment (-1 = non-local)
         """
         if topi.is_cuda:
-            # one fused kernel instead of this ~12-op torch composition
-            # (same contract; within-expert slot order is arrival order,
+            # one or two launches instead of this ~12-op torch composition
+            # (same contract; the slot order within an expert is another,
             # which is output-invariant — see ops.moe_align)
             return ops.moe_align(topi, self.e_start, self.e_end, block_m)
         T, k = topi.shape

@@ -635,12 +635,12 @@ def moe_block_rows(assignments: int, experts: int, ff: int,
 
 
 def moe_align(topi: torch.Tensor, e_start: int, e_end: int, block_m: int):
-    """Single-kernel device-side block alignment of expert assignments
-    (GPU only; MoEMLP._moe_align's torch composition is the CPU
-    reference and the semantic oracle). Within-expert slot order is
-    arrival order rather than stable order — downstream results are
-    bit-identical either way (each row's K-loop and the pos-gathered
-    combine don't depend on the slot). Returns
+    """Device-side block alignment of expert assignments (GPU only;
+    MoEMLP._moe_align's torch composition is the CPU reference and the
+    semantic oracle): one launch up to 4096 assignments, two with scratch
+    counts above. The order of the slots within an expert is unspecified and
+    may differ from run to run; results do not depend on it (a row's K loop
+    is the same in every slot, the combine gathers by pos). Returns
     (sorted_ids [PM], expert_ids [PM/bm], n_valid [1], pos [T*k], PM)."""
     C = _moe_native()
     T, k = topi.shape

@@ -341,7 +341,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_combine", &moe_combine,
         "weighted top-k combine of expert outputs (deterministic)");
   m.def("moe_align", &moe_align,
-        "single-kernel block alignment of expert assignments "
+        "block alignment of expert assignments without host synchronisation "
         "(vLLM moe_align_block_size analog)");
   m.def("moe_router_logits", &moe_router_logits,
         "fp32 router logits of a few bf16 rows");

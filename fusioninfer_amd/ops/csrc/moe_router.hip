@@ -14,7 +14,8 @@
 //    the launch).
 //  * moe_align: token assignments sorted by expert, every expert's segment
 //    padded to block_m rows, without host synchronisation and with static
-//    shapes. Within-expert slot order is arrival order: the grouped GEMM
+//    shapes. The order within an expert is that in which its atomic
+//    counter was reached, different from run to run: the grouped GEMM
 //    computes each row the same wherever it sits and the combine gathers by
 //    pos. Up to kAlignOne assignments one workgroup does it all in LDS;
 //    more are counted and placed by up to 64 workgroups in two launches
