@@ -297,7 +297,9 @@ def rope_qk_norm_(
     k_weight: Optional[torch.Tensor] = None,
     eps: float = 1e-6,
 ):
-    """Fused optional per-head RMSNorm + NeoX RoPE, in-place. Returns (q, k)."""
+    """Fused optional per-head RMSNorm + NeoX RoPE, in-place. Returns (q, k).
+    The models here call rope_qk_norm_cache_, which on the CPU comes back to
+    this; on the GPU this form is there for callers without a paged cache."""
     if q.is_cuda:
         _require_native()
         _C.rope_qk_norm(

@@ -167,7 +167,9 @@ def test_reshape_and_cache():
 def test_rope_qk_norm_cache(T, Hq, Hk, D, pad, fp8):
     """One kernel against the two it stands for: q, both caches, bit for bit
     what rope_qk_norm_ and reshape_and_cache leave, rows of negative slots
-    left out."""
+    left out. And against the fp32 oracle: one bf16 rounding each (2^-9, 2^-8
+    of an ulp that falls the other way) and 1e-5 for fp32 sums; a cached row
+    as bf16 rounds it, in e4m3 with its scale at most one step (2^-3) off."""
     torch.manual_seed(2)
     qkv = torch.randn(T, (Hq + 2 * Hk) * D + pad, device=DEV,
                       dtype=torch.bfloat16)[:, pad:]
@@ -182,6 +184,10 @@ def test_rope_qk_norm_cache(T, Hq, Hk, D, pad, fp8):
               for _ in range(4)]
     cut = lambda t: (t[:, :Hq * D], t[:, Hq * D:(Hq + Hk) * D],
                      t[:, (Hq + Hk) * D:])
+    want_q, want_k = ref.rope_qk_norm(
+        *(t.cpu().float().view(T, -1, D) for t in cut(qkv)[:2]),
+        positions.cpu().long(), cos_sin.cpu(), qw.cpu().float(), None)
+    want_v = cut(qkv)[2].cpu().float().view(T, Hk, D)
     q, k, v = cut(qkv.clone())
     ops.rope_qk_norm_(q, k, positions, cos_sin, Hq, Hk, D, qw, None)
     ops.reshape_and_cache(k.contiguous(), v.contiguous(), *caches[:2], slots,
@@ -193,6 +199,16 @@ def test_rope_qk_norm_cache(T, Hq, Hk, D, pad, fp8):
     for a, b in zip(caches[:2], caches[2:]):
         assert a.float().abs().sum() > 0
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+    assert_close_bf16(got.cpu().view(T, Hq, D), want_q, atol=1e-5,
+                      rtol=2 ** -8)
+    kept = (slots >= 0).cpu()
+    at = slots[slots >= 0].cpu().long()
+    for cache, want, inv in ((caches[2], want_k, 1 / 3.),
+                             (caches[3], want_v, 1 / 4.)):
+        row = cache.cpu().float()[at // 16, :, at % 16]
+        want = want[kept] * (inv if fp8 else 1.0)
+        assert_close_bf16(row, want, atol=2 ** -9 if fp8 else 1e-5,
+                          rtol=2 ** -3 if fp8 else 2 ** -8)
 
 
 def test_kv_block_gather_scatter_roundtrip():
