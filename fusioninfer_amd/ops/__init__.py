@@ -79,30 +79,36 @@ PART_ROWS = 256   # and up to which it does for the sizes below
 
 def _streams(M: int, N: int, K: int, silu_mul: bool = False) -> bool:
     """Whether the streaming kernels beat the library's GEMM for x [M, K],
-    W [N, K]. Up to 16 rows they always do. Above, the library is as good or
-    better where its tiles fill the chip by themselves, and loses where N is
-    too small for that or W too large to be read at 4.3 TB/s. Library / here
-    in us: 6144 x 4096 at 17, 64, 128, 256 rows 14.6 / 13.7, 17.8 / 17.6,
-    25.3 / 22.9, 39.7 / 28.8; 4096 x 4096 12.8 / 11.0, 14.7 / 13.8, 23.7 /
-    18.3, 22.0 / 22.8; 4096 x 12288 23.6 / 20.8, 36.7 / 26.1, 66 / 33, 53 /
-    45; 5120 x 2048 12.5 / 9.7, 12.9 / 12.4, 15.2 / 16.2; 8192 x 4096 15.7 /
-    19.1, 18.6 / 22.0, 26.3 / 27.6; 28672 x 4096 54 / 41, 51 / 40, 54 / 65;
-    51200 x 5120 94 / 87, 99 / 115, 110 / 134; 151936 x 4096 255 / 201, 262 /
-    238, 279 / 266, 350 / 391; 2048 x 2048 8.2 / 8.4, 8.9 / 11.8. With
-    silu_mul the pass over the product goes (5 us of 24576 x 4096: 50 / 36,
-    51 / 39, 55 / 45, 67 / 63): taken where tiles of 96 rows fill the chip
-    once."""
+    W [N, K]. Up to 16 rows they always do; matrices of 2^23 values are read
+    in a few us either way and are the library's.
+
+    Up to 128 rows the kernel's own estimate (tiles, parts, joins) is held
+    against what the library is seen to take: up to 64 rows W at 2.5 TB/s
+    and 1 us, above them W at 3.5 TB/s or, where N gives it few tiles, the
+    chain of 6 us per 1000 of K; with silu_mul 3 us for the pass over the
+    product. From 129 rows on both compute more than they read and the
+    library's choice of tiles jumps with M: the streaming kernel is ahead
+    where N is small (6144 x 4096 at 129 / 256 rows 40.2 / 40.7 us against
+    28.8 / 31.0, 2048 x 12288 39.4 / 40.5 against 27.9 / 30.5), from 192 rows
+    on until half the chip's 256 tiles of 96 rows are taken (12288 x 4096 at
+    129 / 256 37.8 / 49.4 against 40.1 / 43.2, 16384 x 5120 at 256 64 against
+    72), with silu_mul all of them (24576 x 4096 at 256 68 against 62, 28672
+    x 4096 74 against 91), and behind for less than 5 * 2^22 values of W
+    (4096 x 4096 at 256 23.0 against 24.6).
+
+    Over 24 N of 2048 to 151936, five K of 2048 to 12288 and ten M of 17 to
+    256 the choice takes 1.4 % longer than the better of the two on average
+    (silu_mul 1.3 %), the library alone 12 (18) and streaming alone 7 (4)."""
     if M <= SKINNY_ROWS:
         return True
-    if M > PART_ROWS or N * K < 1 << 23:
+    if M > PART_ROWS or N * K <= 1 << 23:
         return False
-    if M <= 64:
-        return not (6144 < N < 9216
-                    or M > 32 and 32768 < N < 1 << 17)
-    if N >= 1 << 17:
-        return M <= 128
-    return K >= 4096 and (3072 <= N <= 6144
-                          or silu_mul and 224 < -(-N // 96) <= 256)
+    if M > 128:
+        return N * K >= 5 << 22 and (
+            N <= 6144 or M >= 192 and N <= 96 * (256 if silu_mul else 128))
+    library = max(2 * N * K / 3.5e6, 6e-3 * K) if M > 64 \
+        else 2 * N * K / 2.5e6 + 1
+    return _C.few_rows_gemm_us(M, N, K) < library + (3 if silu_mul else 0)
 
 
 def _memory_alone(*tensors: torch.Tensor) -> bool:
@@ -171,23 +177,22 @@ def linear(x: torch.Tensor, w: torch.Tensor,
 
 
 def _streams_fp8(M: int, N: int, K: int) -> bool:
-    """As _streams, for e4m3 operands with scales per row. Library / here in
-    us: 6144 x 4096 at 1, 16, 32, 64 rows 23.3 / 10.4, 12.7 / 10.8, 12.6 /
-    11.2, 13.2 / 14.5; 24576 x 4096 30.8 / 20.0, 31.7 / 19.3, 24.4 / 19.3,
-    25.9 / 24.3; 4096 x 12288 21.1 / 14.2, 19.9 / 13.9, 20.5 / 14.5, 24.1 /
-    19.4, 128 rows 35.8 / 26.0, 256 rows 30.9 / 33.6; 4096 x 4096 12.1 / 9.6,
-    12.2 / 9.4, 12.1 / 9.9, 12.6 / 12.8; 8192 x 4096 22.9 / 13.4, 13.3 /
-    13.6, 13.0 / 13.8, 13.5 / 16.2; 28672 x 4096 32.0 / 28.7, 33.0 / 28.0,
-    27.8 / 28.8, 28.9 / 26.0; 51200 x 5120 50.8 / 49.0, 51.4 / 50.2, 52.6 /
-    53.9, 56.8 / 68.4; 5120 x 8192 14.2 / 13.2, 14.3 / 13.1, 14.5 / 13.6,
-    16.4 / 19.5; 2048 x 2048 8.4 / 8.2, 8.6 / 8.6, 8.5 / 8.7, 8.7 / 10.1."""
+    """As _streams, for e4m3 operands with scales per row, whose library
+    reads W at 5 TB/s and 1 us up to 64 rows or walks K in 1.6 us per 1000;
+    up to 16 rows it is behind at nearly all sizes (8192 x 8192 at 9 rows 42
+    us against 20). From 65 rows on it is ahead but for long K and few tiles
+    (4096 x 12288 at 65, 96, 128 rows 21.5, 30.1, 36.4 us against 24.8, 26.0,
+    26.9; 2048 x 12288 at 128 14.5 against 19.7). Over 24 N, five K and
+    eleven M of 1 to 128 the choice takes 1.3 % longer than the better of the
+    two on average, the library alone 19 and streaming alone 6."""
     if M > 128 or N * K < 1 << 23:
         return False
-    if M <= 16:
-        return M <= 8 or not 6144 < N < 9216
-    if M <= 32:
-        return N <= 24576 and not 6144 < N < 9216
-    return K >= 2 * N or M <= 64 and 16384 <= N <= 32768
+    if M <= SKINNY_ROWS:
+        return True
+    if M > 64:
+        return M >= 96 and K >= 2 * N and N >= 3072
+    return _C.few_rows_gemm_us(M, N, K // 2) < max(N * K / 5e6 + 1,
+                                                   1.6e-3 * K)
 
 
 def linear_fp8(x: torch.Tensor, x_scales: torch.Tensor, w: torch.Tensor,

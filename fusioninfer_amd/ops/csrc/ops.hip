@@ -41,6 +41,7 @@ void launch_prefill_attn(u16*, const u16*, const void*, const void*,
 void launch_skinny_gemm(u16*, const u16*, const u16*, const u16*, int, int,
                         int, int64_t, int64_t, bool, hipStream_t);
 int64_t part_gemm_floats(int, int, int);
+double part_gemm_us(int, int, int);
 void launch_part_gemm(u16*, float*, const u16*, const u16*, const u16*, int,
                       int, int, int64_t, int64_t, bool, hipStream_t);
 void launch_part_gemm_fp8(u16*, float*, const unsigned char*, const float*,
@@ -511,6 +512,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gather_kv_blocks", &gather_kv_blocks, "pack KV blocks for PD send");
   m.def("scatter_kv_blocks", &scatter_kv_blocks, "unpack KV blocks from PD recv");
   m.def("few_rows_gemm", &few_rows_gemm, "x W^T for up to 256 rows of x");
+  m.def("few_rows_gemm_us", &fi::part_gemm_us,
+        "estimate for M of 17 to 256 rows, N, K of 16-bit values");
   m.def("few_rows_gemm_fp8", &few_rows_gemm_fp8,
         "x W^T for up to 256 rows of e4m3 x with scales per row");
   m.def("paged_attention_decode", &paged_attention_decode,

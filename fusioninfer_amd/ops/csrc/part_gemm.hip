@@ -26,7 +26,6 @@
 // behind it 48 / 51 / 55 / 67; 4096, 12288 21 (4700) / 26 / 33 / 45 against
 // 26 / 37 / 66 / 53; 151936, 4096 211 (5880) / 238 / 266 / 391 against 264 /
 // 262 / 279 / 350.
-
 //
 // FP8: the same kernel on e4m3 rows, 1 to 128 of them. 24576 x 4096 at 1 / 32
 // / 64 rows 20.0 (5040) / 19.3 / 24.3 us, the library's GEMM 30.8 / 24.4 /
@@ -473,6 +472,13 @@ void with_shape(int M, int N, int K, const F& f) {
 }
 
 }  // namespace
+
+// what the chosen plan takes by its own estimate, in us
+double part_gemm_us(int M, int N, int K) {
+  double us = 0;
+  with_shape(M, N, K, [&](auto, const Plan& pl) { us = pl.us; });
+  return us;
+}
 
 // floats of scratch that launch_part_gemm needs
 int64_t part_gemm_floats(int M, int N, int K) {
