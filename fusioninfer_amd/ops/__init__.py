@@ -79,35 +79,42 @@ PART_ROWS = 256   # and up to which it does for the sizes below
 
 def _streams(M: int, N: int, K: int, silu_mul: bool = False) -> bool:
     """Whether the streaming kernels beat the library's GEMM for x [M, K],
-    W [N, K]. Up to 16 rows they always do; matrices of 2^23 values are read
-    in a few us either way and are the library's.
+    W [N, K]. Up to 16 rows they always do; matrices of less than 2^23
+    values, and K below 2048 up to N 8192, take a few us either way and stay
+    with the library.
 
     Up to 128 rows the kernel's own estimate (tiles, parts, joins) is held
     against what the library is seen to take: up to 64 rows W at 2.5 TB/s
-    and 1 us, above them W at 3.5 TB/s or, where N gives it few tiles, the
-    chain of 6 us per 1000 of K; with silu_mul 3 us for the pass over the
-    product. From 129 rows on both compute more than they read and the
-    library's choice of tiles jumps with M: the streaming kernel is ahead
-    where N is small (6144 x 4096 at 129 / 256 rows 40.2 / 40.7 us against
-    28.8 / 31.0, 2048 x 12288 39.4 / 40.5 against 27.9 / 30.5), from 192 rows
-    on until half the chip's 256 tiles of 96 rows are taken (12288 x 4096 at
-    129 / 256 37.8 / 49.4 against 40.1 / 43.2, 16384 x 5120 at 256 64 against
-    72), with silu_mul all of them (24576 x 4096 at 256 68 against 62, 28672
-    x 4096 74 against 91), and behind for less than 5 * 2^22 values of W
-    (4096 x 4096 at 256 23.0 against 24.6).
+    and 4 us, above them 4 us and W at 4 TB/s or, where N gives it few tiles,
+    the chain of 7 us per 1000 of K; with silu_mul 3 us more for the pass
+    over the product. (Where that errs most: 14336 x 5120 at 64 rows streams
+    in 38.2 us, the library takes 32.4.)
 
-    Over 24 N of 2048 to 151936, five K of 2048 to 12288 and ten M of 17 to
-    256 the choice takes 1.4 % longer than the better of the two on average
-    (silu_mul 1.3 %), the library alone 12 (18) and streaming alone 7 (4)."""
+    From 129 rows on both compute more than they read and the library's
+    choice of tiles jumps with M. The streaming kernel is ahead where N is
+    small (6144 x 4096 at 129 / 256 rows 28.1 / 30.1 us, the library 39.4 /
+    40.0; 2048 x 12288 27.9 / 30.2 and 39.0 / 39.9), from 192 rows on until
+    half the chip's 256 tiles of 96 rows are taken (12288 x 4096 at 129 / 256
+    41.7 / 44.1 and 38.3 / 49.5; 16384 x 5120 at 256 71 and 65), and behind
+    for less than 5 * 2^22 values of W (4096 x 4096 at 256 23.6 and 22.5).
+    With silu_mul it is ahead until all 256 are (24576 x 4096 at 256 62 and
+    69, 28672 x 4096 90 and 75).
+
+    Weights that no cache holds (4 GB of them in turn), 24 N of 2048 to
+    151936, eight K of 512 to 12288, ten M of 17 to 256: this choice takes
+    1.5 % longer than the better of the two on average (silu_mul 1.6 %), the
+    library alone 14 (25), streaming alone 5 (3)."""
     if M <= SKINNY_ROWS:
         return True
-    if M > PART_ROWS or N * K <= 1 << 23:
+    if M > PART_ROWS or N * K < 1 << 23 or K < 2048 and N <= 8192:
         return False
     if M > 128:
-        return N * K >= 5 << 22 and (
-            N <= 6144 or M >= 192 and N <= 96 * (256 if silu_mul else 128))
-    library = max(2 * N * K / 3.5e6, 6e-3 * K) if M > 64 \
-        else 2 * N * K / 2.5e6 + 1
+        if silu_mul:
+            return N <= 96 * 256
+        return N * K >= 5 << 22 and (N <= 6144
+                                     or M >= 192 and N <= 96 * 128)
+    library = 4 + (2 * N * K / 2.5e6 if M <= 64
+                   else max(2 * N * K / 4e6, 7e-3 * K))
     return _C.few_rows_gemm_us(M, N, K) < library + (3 if silu_mul else 0)
 
 
@@ -177,22 +184,23 @@ def linear(x: torch.Tensor, w: torch.Tensor,
 
 
 def _streams_fp8(M: int, N: int, K: int) -> bool:
-    """As _streams, for e4m3 operands with scales per row, whose library
-    reads W at 5 TB/s and 1 us up to 64 rows or walks K in 1.6 us per 1000;
-    up to 16 rows it is behind at nearly all sizes (8192 x 8192 at 9 rows 42
-    us against 20). From 65 rows on it is ahead but for long K and few tiles
-    (4096 x 12288 at 65, 96, 128 rows 21.5, 30.1, 36.4 us against 24.8, 26.0,
-    26.9; 2048 x 12288 at 128 14.5 against 19.7). Over 24 N, five K and
-    eleven M of 1 to 128 the choice takes 1.3 % longer than the better of the
-    two on average, the library alone 19 and streaming alone 6."""
+    """As _streams, for e4m3 operands with scales per row. Up to 16 rows the
+    library is behind at nearly all sizes (8192 x 8192 at 9 rows 43 us, 20
+    here); up to 64 rows it takes W at 4.5 TB/s and 5 us or 2 us per 1000 of
+    K (6144 x 4096 at 64 13.1 and 14.5, 4096 x 12288 23.7 and 19.6). From 65
+    rows on it is ahead but for long K and few tiles (4096 x 12288 at 65, 96,
+    128 rows 20.6, 29.8, 35.8 and 23.5, 24.9, 25.9; 2048 x 12288 at 128 17.6
+    and 18.8). Over the same N and K and eleven M of 1 to 128 this choice
+    takes 1.9 % longer than the better of the two on average, the library
+    alone 22, streaming alone 5."""
     if M > 128 or N * K < 1 << 23:
         return False
     if M <= SKINNY_ROWS:
         return True
     if M > 64:
         return M >= 96 and K >= 2 * N and N >= 3072
-    return _C.few_rows_gemm_us(M, N, K // 2) < max(N * K / 5e6 + 1,
-                                                   1.6e-3 * K)
+    return _C.few_rows_gemm_us(M, N, K // 2) < max(N * K / 4.5e6 + 5,
+                                                   2e-3 * K)
 
 
 def linear_fp8(x: torch.Tensor, x_scales: torch.Tensor, w: torch.Tensor,
