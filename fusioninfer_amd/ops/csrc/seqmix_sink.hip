@@ -936,6 +936,9 @@ bool launch_sink_attention_tiles(A* out, const A* q, const A* k_cache,
                            block_size, scale, window, keep_first, s))
       return true;
   }
+  // bf16 of 64 and 128 values: only for what launch_equal_sizes leaves,
+  // tensors off its 16-byte grid and value rows of another length; fp32 of
+  // these sizes always.
   // head pairs (HP_ == 2) need an even number of heads per key/value head
   const bool pairs = (H / G) % 2 == 0;
 #define FI_TILE(K_, V_, BNB, BNF, QS_, HP_)                                    \

@@ -1432,6 +1432,36 @@ def test_sink_attention_row_tiles(D, heads, groups, block, window, keep,
     assert err <= 2 ** -8 * v.float().abs().max()
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("off", ["q", "k", "v"])
+def test_sink_attention_row_tiles_off_the_16_byte_grid(D, off):
+    """Tensors that start 8 bytes off the grid take the tiles that stage
+    through registers; bound as above, against the rows on the grid: both
+    round weights and results to bf16 once."""
+    from fusioninfer_amd.ops import seqmix
+
+    g = torch.Generator().manual_seed(D)
+    new, past, block = [1, 70, 200], [40, 0, 61], 16
+    need = [-(-(a + b) // block) for a, b in zip(new, past)]
+    table = torch.zeros(3, max(need), dtype=torch.int32)
+    for i, n in enumerate(need):
+        table[i, :n] = torch.arange(n) + sum(need[:i])
+    T = sum(new)
+    x = {n: torch.randn(*shape, generator=g).bfloat16().to(DEV) for n, shape in
+         (("q", (T, 4, D)), ("k", (sum(need), 2, block, D)),
+          ("v", (sum(need), 2, block, D)))}
+    cu = torch.tensor([0, *torch.tensor(new).cumsum(0)], dtype=torch.int32)
+    rows = torch.cat([torch.full((n,), i) for i, n in enumerate(new)]).int()
+    pos = torch.cat([torch.arange(p, p + n) for n, p in zip(new, past)]).int()
+    outs = [seqmix.sink_paged_attention(
+        t["q"], t["k"], t["v"], table.to(DEV), rows.to(DEV), pos.to(DEV),
+        D ** -0.5, seq_cu=cu.to(DEV),
+        tiles=seqmix.build_attention_tiles(new, device=DEV))
+        for t in (x, dict(x, **{off: _shifted(x[off], 4)}))]
+    err = (outs[0].float() - outs[1].float()).abs().max()
+    assert err <= 2 * 2 ** -8 * x["v"].float().abs().max()
+
+
 @pytest.mark.parametrize("DK,DV", [(64, 64), (128, 128), (192, 128),
                                    (288, 256)])
 @pytest.mark.parametrize("heads,groups,block,window,keep,gate", [
