@@ -75,6 +75,7 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
 
 SKINNY_ROWS = 16  # rows of x up to which a GEMM always streams W
 PART_ROWS = 256   # and up to which it does for the sizes below
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 def _streams(M: int, N: int, K: int, silu_mul: bool = False) -> bool:
@@ -118,31 +119,33 @@ def _streams(M: int, N: int, K: int, silu_mul: bool = False) -> bool:
     return _C.few_rows_gemm_us(M, N, K) < library + (3 if silu_mul else 0)
 
 
-def _memory_alone(*tensors: torch.Tensor) -> bool:
+def _memory_alone(x, w, bias) -> bool:
     """Whether a call is about its operands' memory and nothing else. The
-    kernels see no tracing or compilation, functional transform, dispatch or
-    autocast mode, tensor subclass, gradient or tangent; torch's own
-    operations carry all of them."""
+    kernels see no compilation, functional transform, operator or autocast
+    mode, tensor subclass, gradient or tangent (nor a trace); torch's own
+    operations carry all of them. A microsecond: it runs at every call."""
     return (
-        not torch.compiler.is_compiling() and not torch._C._is_tracing()
-        and torch._C._functorch.maybe_current_level() is None
+        type(x) in _PLAIN and type(w) in _PLAIN
+        and (bias is None or type(bias) in _PLAIN)
+        and not (torch.is_grad_enabled() and (
+            x.requires_grad or w.requires_grad
+            or bias is not None and bias.requires_grad))
         and forward_ad._current_level < 0
+        and torch._C._functorch.maybe_current_level() is None
         and torch._C._len_torch_dispatch_stack() == 0
-        and not torch.overrides.has_torch_function(tensors)
+        and torch._C._len_torch_function_stack() == 0
         and not torch.is_autocast_enabled("cuda")
-        and all(type(t) in (torch.Tensor, torch.nn.Parameter)
-                for t in tensors)
-        and not (torch.is_grad_enabled()
-                 and any(t.requires_grad for t in tensors))
+        and not torch.compiler.is_compiling()
     )
 
 
-def _on_current_gpu(*tensors: torch.Tensor) -> bool:
+def _on_current_gpu(x, w, *others) -> bool:
     """Whether all lie on the GPU that a launch goes to; torch's operations
     follow their operands or refuse a mixture."""
-    d = tensors[0].device
-    return (d.type == "cuda" and all(t.device == d for t in tensors[1:])
-            and d.index == torch.cuda.current_device())
+    d = x.get_device()
+    return (0 <= d == w.get_device() and all(t.get_device() == d
+                                             for t in others)
+            and d == torch.cuda.current_device())
 
 
 def _skinny_ok(x, w, unit: int, silu_mul: bool = False, bias=None) -> bool:
@@ -151,12 +154,12 @@ def _skinny_ok(x, w, unit: int, silu_mul: bool = False, bias=None) -> bool:
     rows, a bias of [N], an eager call without gradients. A family that
     builds only its own extension keeps the library's GEMM."""
     return (
-        _C is not None
-        and _memory_alone(*((x, w) if bias is None else (x, w, bias)))
-        and _on_current_gpu(*((x, w) if bias is None else (x, w, bias)))
-        and x.dim() == 2 and w.dim() == 2
+        _C is not None and not torch._C._is_tracing()
+        and x.dim() == 2 and w.dim() == 2 and 1 <= x.shape[0] <= PART_ROWS
+        and _memory_alone(x, w, bias)
+        and (_on_current_gpu(x, w) if bias is None
+             else _on_current_gpu(x, w, bias))
         and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
-        and 1 <= x.shape[0] <= PART_ROWS
         and x.shape[1] == w.shape[1] and 0 < x.shape[1] <= 1 << 24
         and x.shape[1] % 128 == 0
         and 0 < w.shape[0] <= 1 << 24 and w.shape[0] % unit == 0
@@ -207,10 +210,10 @@ def linear_fp8(x: torch.Tensor, x_scales: torch.Tensor, w: torch.Tensor,
                w_scales: torch.Tensor) -> torch.Tensor:
     """(x * x_scales) (w * w_scales)^T in bf16 on the GPU: x [M, K] and w
     [N, K] e4m3, a scale per row each."""
-    if (_C is not None and _on_current_gpu(x, x_scales, w, w_scales)
-            and x.dim() == 2 and w.dim() == 2
+    if (_C is not None and x.dim() == 2 and w.dim() == 2
+            and 1 <= x.shape[0] <= 128 and x.shape[1] == w.shape[1]
+            and _on_current_gpu(x, w, x_scales, w_scales)
             and x.dtype == w.dtype == torch.float8_e4m3fn
-            and x.shape[0] >= 1 and x.shape[1] == w.shape[1]
             and x.shape[1] % 256 == 0 and w.shape[0] % 16 == 0
             and 0 < x.shape[1] <= 1 << 24 and 0 < w.shape[0] <= 1 << 24
             and _streams_fp8(x.shape[0], w.shape[0], x.shape[1])
