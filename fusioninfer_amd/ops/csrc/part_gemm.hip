@@ -389,7 +389,10 @@ void part_gemm_join_kernel(u16* __restrict__ out,
 // CU's share of HBM (25 GB/s), its share of what L2 delivers (39 GB/s, W and
 // x together), and, where tiles are cut, 5 us for the second kernel and the
 // way of the pieces through memory. Whole tiles on an uneven number of CUs
-// against even parts with a join comes out of the same sum.
+// against even parts with a join comes out of the same sum, and so does the
+// caller's choice between this kernel and the library: up to 128 rows nine
+// in ten sizes take 0.9 to 1.25 times the estimate (e4m3 1.0 to 1.6), above
+// them 0.75 to 0.9.
 struct Plan {
   int tiles = 0, parts = 0;
   bool split = false;
