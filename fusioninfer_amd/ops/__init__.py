@@ -174,14 +174,66 @@ def _skinny_ok(x, w, unit: int, silu_mul: bool = False, bias=None) -> bool:
     )
 
 
+def _tiles(M: int, N: int, K: int, silu_mul: bool = False) -> bool:
+    """Whether the kernel of 256 x 256 tiles beats the library's GEMM for
+    more than 256 rows. On whole rounds of tiles both reach 1.4 to 1.55
+    PFLOP/s; the kernel cuts what is left over into even pieces, where the
+    library's choice of tiles takes up to twice as long (4099 rows, 4096 x
+    12288: 312 us here, 619; 24576 x 4096 580 and 690; 2700 1.22 times). The
+    kernel's own estimate is held against 8 us and 1.2 PFLOP/s, or the chain
+    of 7 us per 1000 of K; with silu_mul the pass over the product is added,
+    which the kernel has in its epilogue (7600 rows, 24576 x 4096 1041 us
+    here, 1135). Over 504 sizes this takes 2.6 % longer than the better of
+    the two, the library alone 4.8 (up to 98), the kernel alone 11.
+
+    Where both operands together outgrow the memory-side cache and rows are
+    longer than 16 KB the library is ahead more often than not (7600 rows,
+    4096 x 12288 533 us, 627 here)."""
+    if K > 8192 and (M + N) * K > 1 << 27:
+        return False
+    library = max(8 + 2 * M * N * K / 1.2e9, 7e-3 * K)
+    if silu_mul:
+        library += 3 * M * N / 5e6
+    return _C.many_rows_gemm_us(M, N, K) < library
+
+
+def _tiles_ok(x, w, unit: int, silu_mul: bool = False, bias=None) -> bool:
+    """As _skinny_ok, for the rows above: whole 64-value stages of K."""
+    return (
+        _C is not None and not torch._C._is_tracing()
+        and x.dim() == 2 and w.dim() == 2 and x.shape[0] > PART_ROWS
+        and _memory_alone(x, w, bias)
+        and (_on_current_gpu(x, w) if bias is None
+             else _on_current_gpu(x, w, bias))
+        and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+        and x.shape[1] == w.shape[1] and 128 <= x.shape[1] <= 1 << 22
+        and x.shape[1] % 64 == 0 and x.shape[0] <= 1 << 20
+        and 0 < w.shape[0] <= 1 << 20 and w.shape[0] % unit == 0
+        and x.stride(1) == 1 and x.stride(0) % 8 == 0
+        and x.shape[1] <= x.stride(0) <= 1 << 22
+        and _tiles(x.shape[0], w.shape[0], x.shape[1], silu_mul)
+        and w.is_contiguous()
+        and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+        and (bias is None or (
+            bias.dtype == torch.bfloat16 and bias.is_contiguous()
+            and bias.shape == w.shape[:1] and bias.data_ptr() % 16 == 0))
+    )
+
+
 def linear(x: torch.Tensor, w: torch.Tensor,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x W^T (+ bias): a few bf16 rows stream W once through the kernels for
-    that, anything else is the library's GEMM."""
+    that, many rows go by tiles where the library's GEMM leaves the chip
+    idle, anything else is the library's."""
     if _skinny_ok(x, w, 16, bias=bias):
         out = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype,
                           device=x.device)
         _C.few_rows_gemm(out, x, w, bias, False)
+        return out
+    if _tiles_ok(x, w, 16, bias=bias):
+        out = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype,
+                          device=x.device)
+        _C.many_rows_gemm(out, x, w, bias, False)
         return out
     return torch.nn.functional.linear(x, w, bias)
 
@@ -235,12 +287,17 @@ def linear_fp8(x: torch.Tensor, x_scales: torch.Tensor, w: torch.Tensor,
 
 
 def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """silu(x G^T) * (x U^T) with w = [G; U]; few rows in one kernel, whose
-    gate and up values are not rounded in between."""
+    """silu(x G^T) * (x U^T) with w = [G; U]; in one kernel where linear has
+    one, whose gate and up values are not rounded in between."""
     if _skinny_ok(x, w, 32, True):
         out = torch.empty((x.shape[0], w.shape[0] // 2), dtype=x.dtype,
                           device=x.device)
         _C.few_rows_gemm(out, x, w, None, True)
+        return out
+    if _tiles_ok(x, w, 32, True):
+        out = torch.empty((x.shape[0], w.shape[0] // 2), dtype=x.dtype,
+                          device=x.device)
+        _C.many_rows_gemm(out, x, w, None, True)
         return out
     return silu_and_mul(linear(x, w))
 

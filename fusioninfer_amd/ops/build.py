@@ -35,6 +35,7 @@ SOURCES = [
     "prefill_attention.hip",
     "skinny_gemm.hip",
     "part_gemm.hip",
+    "tile_gemm.hip",
 ]
 
 MOE_SOURCES = [

@@ -47,6 +47,10 @@ void launch_part_gemm(u16*, float*, const u16*, const u16*, const u16*, int,
 void launch_part_gemm_fp8(u16*, float*, const unsigned char*, const float*,
                           const unsigned char*, const float*, int, int, int,
                           int64_t, int64_t, hipStream_t);
+int64_t tile_gemm_floats(int, int, int);
+double tile_gemm_us(int, int, int);
+void launch_tile_gemm(u16*, float*, const u16*, const u16*, const u16*, int,
+                      int, int, int64_t, int64_t, bool, hipStream_t);
 
 }  // namespace fi
 
@@ -457,6 +461,41 @@ void few_rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
                        silu_mul, current_stream());
 }
 
+// the same for more rows, by tiles of 256 x 256
+void many_rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
+                    c10::optional<at::Tensor> bias, bool silu_mul) {
+  CHECK_BF16_CUDA(out);
+  CHECK_BF16_CUDA(x);
+  CHECK_BF16_CUDA(w);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2);
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(M >= 1 && M <= (1 << 24) && w.size(1) == K && K % 64 == 0 &&
+                  K >= 128 && N > 0 && N % (silu_mul ? 32 : 16) == 0 &&
+                  K <= (1 << 22) && N <= (1 << 24) &&
+                  (M + 255) / 256 * ((N + 255) / 256) <= (1 << 24),
+              "many_rows_gemm: unsupported sizes");
+  TORCH_CHECK(out.size(0) == M && out.size(1) == (silu_mul ? N / 2 : N));
+  TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % 8 == 0 && x.stride(0) >= K &&
+              x.stride(0) <= (1 << 22) && w.is_contiguous() &&
+              out.stride(1) == 1 && out.stride(0) % 8 == 0);
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0);
+  const u16* b = nullptr;
+  if (bias.has_value()) {
+    TORCH_CHECK(!silu_mul && bias->is_cuda() &&
+                bias->scalar_type() == at::kBFloat16 &&
+                bias->is_contiguous() && bias->numel() == N &&
+                reinterpret_cast<uintptr_t>(bias->data_ptr()) % 16 == 0);
+    b = bf16_cptr(*bias);
+  }
+  at::Tensor pieces = at::empty({fi::tile_gemm_floats(M, N, K)},
+                                x.options().dtype(at::kFloat));
+  fi::launch_tile_gemm(bf16_ptr(out), pieces.data_ptr<float>(), bf16_cptr(x),
+                       bf16_cptr(w), b, M, N, K, x.stride(0), out.stride(0),
+                       silu_mul, current_stream());
+}
+
 // out [M, N] bf16 = (x [M, K] * x_scales) @ (w [N, K] * w_scales)^T, e4m3
 void few_rows_gemm_fp8(at::Tensor out, at::Tensor x, at::Tensor x_scales,
                        at::Tensor w, at::Tensor w_scales) {
@@ -514,6 +553,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("few_rows_gemm", &few_rows_gemm, "x W^T for up to 256 rows of x");
   m.def("few_rows_gemm_us", &fi::part_gemm_us,
         "estimate for M of 17 to 256 rows, N, K of 16-bit values");
+  m.def("many_rows_gemm", &many_rows_gemm, "x W^T by tiles of 256 x 256");
+  m.def("many_rows_gemm_us", &fi::tile_gemm_us, "estimate for M, N, K");
   m.def("few_rows_gemm_fp8", &few_rows_gemm_fp8,
         "x W^T for up to 256 rows of e4m3 x with scales per row");
   m.def("paged_attention_decode", &paged_attention_decode,

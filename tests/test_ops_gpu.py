@@ -1059,6 +1059,58 @@ def test_linear_in_parts(rows, n, k, bias):
                 <= want.abs() * 2 ** -8 + 1e-3 * k ** 0.5).all()
 
 
+@pytest.mark.parametrize("rows", [1, 255, 257, 1029])
+@pytest.mark.parametrize("n,k,bias", [
+    (16, 128, True),        # one ragged tile, two stages, whole
+    (288, 192, False),      # three stages: not to be cut
+    (4128, 1024, True),     # cut tiles, a ragged last one
+    (288, 16384, False),    # 16 pieces, every other tile begins half way
+    (65568, 128, False),    # whole rounds of tiles and a rest
+])
+def test_linear_by_tiles(rows, n, k, bias):
+    """Tiles of 256 x 256 against a float64 product; one bf16 rounding of the
+    result (2^-9 relative) and fp32 sums of k products. Rows that are not of
+    the result stay as they were."""
+    g = torch.Generator().manual_seed(n + k + rows)
+    w = torch.randn(n, k, generator=g).to(torch.bfloat16).to(DEV)
+    b = torch.randn(n, generator=g).to(torch.bfloat16).to(DEV) if bias \
+        else None
+    x = torch.randn(rows, 2 * k, generator=g).to(torch.bfloat16).to(DEV)[:, k:]
+    out = torch.full((rows + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops._C.many_rows_gemm(out[:rows], x, w, b, False)
+    prod = x.double() @ w.double().T
+    want = prod + (0.0 if b is None else b.double())
+    assert ((out[:rows].double() - want).abs()
+            <= want.abs() * 2 ** -8 + 1e-4 * k ** 0.5).all()
+    assert (out[rows] == 7.0).all()
+    if n % 32 == 0 and not bias:
+        out = torch.full((rows + 1, n // 2), 7.0, dtype=torch.bfloat16,
+                         device=DEV)
+        ops._C.many_rows_gemm(out[:rows], x, w, None, True)
+        want = torch.nn.functional.silu(prod[:, : n // 2]) * prod[:, n // 2:]
+        assert ((out[:rows].double() - want).abs()
+                <= want.abs() * 2 ** -8 + 1e-3 * k ** 0.5).all()
+        assert (out[rows] == 7.0).all()
+
+
+def test_linear_takes_tiles():
+    """Whole rounds with every other tile begun half way and a cut rest, as
+    ops.linear chooses it; what it refuses goes to the library."""
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(4099, 12288, generator=g).to(torch.bfloat16).to(DEV)
+    w = torch.randn(4096, 12288, generator=g).to(torch.bfloat16).to(DEV)
+    assert ops._tiles_ok(x, w, 16)
+    want = x.double() @ w.double().T
+    assert ((ops.linear(x, w).double() - want).abs()
+            <= want.abs() * 2 ** -8 + 1e-4 * 12288 ** 0.5).all()
+    x, w = x[:, :4096], w[:, :4096].contiguous()
+    for other in (x[:, 1:129], x.T, x.float(), x[:256]):
+        assert not ops._tiles_ok(other, w[:, :other.shape[1]].contiguous(), 16)
+    assert ops._tiles_ok(x, w, 16) and not ops._tiles_ok(x, w.T, 16)
+    with torch.enable_grad():
+        assert not ops._tiles_ok(x, w.clone().requires_grad_(), 16)
+
+
 @pytest.mark.parametrize("rows", [17, 32])
 def test_linear_silu_mul_in_parts_of_96_rows(rows):
     """One tile of 96 rows in many pieces, whose kept third of a wave's
