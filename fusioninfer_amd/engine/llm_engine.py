@@ -1066,8 +1066,14 @@ class LLMEngine:
             at = {r: r for r in range(len(decode))}
         else:
             at = {r: i for i, r in enumerate(rows)}
-        out = logits.float()[[at[r] for r in asked]] if asked else \
-            logits.float()[:0]
+        # an index that is a list would be copied to the GPU synchronously,
+        # and the host would stand still until this step is over
+        picked = [at[r] for r in asked]
+        if picked == list(range(logits.shape[0])):
+            out = logits.to(torch.float32, copy=True)
+        else:
+            out = logits.float()[self.runner._to_device(
+                {"rows": (picked, torch.long)})["rows"]]
         for seq in prefill + decode:
             seq.num_computed_tokens = seq.num_prompt_tokens
         self.num_prefilled_tokens += sum(chunks) + len(decode)
