@@ -194,7 +194,7 @@ def _tiles(M: int, N: int, K: int, silu_mul: bool = False) -> bool:
     library = max(8 + 2 * M * N * K / 1.2e9, 7e-3 * K)
     if silu_mul:
         library += 3 * M * N / 5e6
-    return _C.many_rows_gemm_us(M, N, K) < library
+    return _C.many_rows_gemm_us(M, N, 2 * K) < library
 
 
 def _tiles_ok(x, w, unit: int, silu_mul: bool = False, bias=None) -> bool:
@@ -258,6 +258,40 @@ def _streams_fp8(M: int, N: int, K: int) -> bool:
                                                    2e-3 * K)
 
 
+def _tiles_fp8(M: int, N: int, K: int) -> bool:
+    """As _tiles, for e4m3 operands: the kernel's own estimate against 6 us
+    and 2.2 PFLOP/s, or 18 us and 2 us per 1000 of K above 8192 (4096 x 4096
+    at 1024 rows 36.6 us here, the library 23.0; at 8192 100.4 and 102.8;
+    4096 x 12288 at 4099 153 and 268). Over twelve N and K and up to 17 M of
+    257 to 8192 this takes 2.4 % longer than the better of the two, the
+    library alone 8.9 (up to 75), the kernel alone 8.7."""
+    return _C.many_rows_gemm_us(M, N, K) < max(
+        6 + 2 * M * N * K / 2.2e9, 18 + 2e-3 * max(0, K - 8192))
+
+
+def _tiles_fp8_ok(x, x_scales, w, w_scales) -> bool:
+    """As _tiles_ok, for e4m3 operands with a scale per row each."""
+    return (
+        _C is not None and not torch._C._is_tracing()
+        and x.dim() == 2 and w.dim() == 2 and x.shape[0] > PART_ROWS
+        and _memory_alone(x, w, x_scales) and type(w_scales) in _PLAIN
+        and _on_current_gpu(x, w, x_scales, w_scales)
+        and x.dtype == w.dtype == torch.float8_e4m3fn
+        and x.shape[1] == w.shape[1] and 256 <= x.shape[1] <= 1 << 22
+        and x.shape[1] % 128 == 0 and x.shape[0] <= 1 << 20
+        and 0 < w.shape[0] <= 1 << 20 and w.shape[0] % 16 == 0
+        and x.stride(1) == 1 and x.stride(0) % 16 == 0
+        and x.shape[1] <= x.stride(0) <= 1 << 22
+        and _tiles_fp8(x.shape[0], w.shape[0], x.shape[1])
+        and w.is_contiguous()
+        and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+        and x_scales.dtype == w_scales.dtype == torch.float32
+        and x_scales.is_contiguous() and w_scales.is_contiguous()
+        and x_scales.shape == x.shape[:1] and w_scales.shape == w.shape[:1]
+        and w_scales.data_ptr() % 16 == 0
+    )
+
+
 def linear_fp8(x: torch.Tensor, x_scales: torch.Tensor, w: torch.Tensor,
                w_scales: torch.Tensor) -> torch.Tensor:
     """(x * x_scales) (w * w_scales)^T in bf16 on the GPU: x [M, K] and w
@@ -279,6 +313,11 @@ def linear_fp8(x: torch.Tensor, x_scales: torch.Tensor, w: torch.Tensor,
         out = torch.empty((x.shape[0], w.shape[0]), dtype=torch.bfloat16,
                           device=x.device)
         _C.few_rows_gemm_fp8(out, x, x_scales, w, w_scales)
+        return out
+    if _tiles_fp8_ok(x, x_scales, w, w_scales):
+        out = torch.empty((x.shape[0], w.shape[0]), dtype=torch.bfloat16,
+                          device=x.device)
+        _C.many_rows_gemm_fp8(out, x, x_scales, w, w_scales)
         return out
     return torch._scaled_mm(
         x, w.t(),  # column-major view of the row-major weight

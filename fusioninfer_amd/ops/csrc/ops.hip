@@ -51,6 +51,9 @@ int64_t tile_gemm_floats(int, int, int);
 double tile_gemm_us(int, int, int);
 void launch_tile_gemm(u16*, float*, const u16*, const u16*, const u16*, int,
                       int, int, int64_t, int64_t, bool, hipStream_t);
+void launch_tile_gemm_fp8(u16*, float*, const unsigned char*, const float*,
+                          const unsigned char*, const float*, int, int, int,
+                          int64_t, int64_t, hipStream_t);
 
 }  // namespace fi
 
@@ -489,7 +492,7 @@ void many_rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
                 reinterpret_cast<uintptr_t>(bias->data_ptr()) % 16 == 0);
     b = bf16_cptr(*bias);
   }
-  at::Tensor pieces = at::empty({fi::tile_gemm_floats(M, N, K)},
+  at::Tensor pieces = at::empty({fi::tile_gemm_floats(M, N, 2 * K)},
                                 x.options().dtype(at::kFloat));
   fi::launch_tile_gemm(bf16_ptr(out), pieces.data_ptr<float>(), bf16_cptr(x),
                        bf16_cptr(w), b, M, N, K, x.stride(0), out.stride(0),
@@ -530,6 +533,43 @@ void few_rows_gemm_fp8(at::Tensor out, at::Tensor x, at::Tensor x_scales,
       current_stream());
 }
 
+// the same for more rows, by tiles of 256 x 256
+void many_rows_gemm_fp8(at::Tensor out, at::Tensor x, at::Tensor x_scales,
+                        at::Tensor w, at::Tensor w_scales) {
+  CHECK_BF16_CUDA(out);
+  TORCH_CHECK(x.is_cuda() && w.is_cuda() &&
+              x.scalar_type() == at::kFloat8_e4m3fn &&
+              w.scalar_type() == at::kFloat8_e4m3fn);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2);
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(M >= 1 && M <= (1 << 24) && w.size(1) == K && K % 128 == 0 &&
+                  K >= 256 && N > 0 && N % 16 == 0 && K <= (1 << 22) &&
+                  N <= (1 << 24) &&
+                  (M + 255) / 256 * ((N + 255) / 256) <= (1 << 24),
+              "many_rows_gemm_fp8: unsupported sizes");
+  TORCH_CHECK(out.size(0) == M && out.size(1) == N);
+  TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % 16 == 0 && x.stride(0) >= K &&
+              x.stride(0) <= (1 << 22) && w.is_contiguous() &&
+              out.stride(1) == 1 && out.stride(0) % 8 == 0);
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0);
+  TORCH_CHECK(x_scales.is_cuda() && x_scales.scalar_type() == at::kFloat &&
+              x_scales.is_contiguous() && x_scales.numel() == M &&
+              w_scales.is_cuda() && w_scales.scalar_type() == at::kFloat &&
+              w_scales.is_contiguous() && w_scales.numel() == N &&
+              reinterpret_cast<uintptr_t>(w_scales.data_ptr()) % 16 == 0);
+  at::Tensor pieces = at::empty({fi::tile_gemm_floats(M, N, K)},
+                                x.options().dtype(at::kFloat));
+  fi::launch_tile_gemm_fp8(
+      bf16_ptr(out), pieces.data_ptr<float>(),
+      static_cast<const unsigned char*>(x.data_ptr()),
+      x_scales.data_ptr<float>(),
+      static_cast<const unsigned char*>(w.data_ptr()),
+      w_scales.data_ptr<float>(), M, N, K, x.stride(0), out.stride(0),
+      current_stream());
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -554,7 +594,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("few_rows_gemm_us", &fi::part_gemm_us,
         "estimate for M of 17 to 256 rows, N, K of 16-bit values");
   m.def("many_rows_gemm", &many_rows_gemm, "x W^T by tiles of 256 x 256");
-  m.def("many_rows_gemm_us", &fi::tile_gemm_us, "estimate for M, N, K");
+  m.def("many_rows_gemm_us", &fi::tile_gemm_us,
+        "estimate for M, N, bytes of a row of K");
+  m.def("many_rows_gemm_fp8", &many_rows_gemm_fp8,
+        "x W^T by tiles of 256 x 256, e4m3 with scales per row");
   m.def("few_rows_gemm_fp8", &few_rows_gemm_fp8,
         "x W^T for up to 256 rows of e4m3 x with scales per row");
   m.def("paged_attention_decode", &paged_attention_decode,

@@ -1,5 +1,6 @@
-// y = x W^T for more than 256 rows of x (prompts): bf16 operands, fp32
-// accumulation, W [N, K] row-major. Bound by the matrix cores.
+// y = x W^T for more than 256 rows of x (prompts): bf16 operands, or e4m3
+// with a scale per row of either, fp32 accumulation, W [N, K] row-major.
+// Bound by the matrix cores.
 //
 // 256 persistent workgroups, one per CU, take tiles of 256 rows of x by 256
 // rows of W. Four waves hold 128 x 128 results each (256 registers), which
@@ -22,8 +23,8 @@
 // Rows lie in LDS as eight chunks of 16 bytes, chunk c of row r at c ^ key(r):
 // the 16 lanes that LDS serves together then touch all its banks (no
 // conflicts counted), and a DMA still reads whole lines of eight rows.
-// MFMA 16x16x32 with A = W, B = x; the W rows of a fragment pair are dealt so
-// that a lane ends with eight neighbouring outputs of one row of x.
+// bf16: MFMA 16x16x32 with A = W, B = x; the W rows of a fragment pair are
+// dealt so that a lane ends with eight neighbouring outputs of one row of x.
 //
 // What whole rounds of 256 tiles leave over is cut along K into equal pieces
 // (tile_plan), which a second kernel sums in a fixed order.
@@ -33,6 +34,13 @@
 // CUs meet on few memory channels (8192 x 4096 x 12288: 1.28 PFLOP/s, with K
 // of 12160 or 12416 1.49); there every other column tile starts half way
 // along K (1.41).
+//
+// e4m3: the same bytes in the same places, so a stage is 128 of K. MFMA
+// 32x32x64 (four times a bf16 product's time, eight times its work), a lane
+// has two chunks of a row; scales are applied in the epilogue. 8192 rows, us
+// (PFLOP/s), the library's GEMM and this: 4096 x 12288 288 (2.86) and 271
+// (3.04), 24576 x 4096 636 (2.59) and 589 (2.80); where the library's tiles
+// leave the chip idle, 4099 rows, 4096 x 12288: 268 (1.54) and 153 (2.70).
 //
 // SILU_MUL: the first half of a tile's W rows are gate rows and the second
 // the up rows that go with them; a wave holds both.
@@ -45,9 +53,13 @@ namespace {
 
 typedef __attribute__((ext_vector_type(8))) short short8;
 typedef __attribute__((ext_vector_type(4))) float floatx4;
+typedef __attribute__((ext_vector_type(16))) float floatx16;
+typedef __attribute__((ext_vector_type(4))) int intx4;
+typedef __attribute__((ext_vector_type(8))) int intx8;
 
-constexpr int kTile = 256, kChip = 256, kKS = 64;
-constexpr int kHalfB = kTile * kKS * 2;   // one operand's part of a stage
+constexpr int kTile = 256, kChip = 256;
+constexpr int kRowB = 128;                // of a row in a stage
+constexpr int kHalfB = kTile * kRowB;     // one operand's part of a stage
 constexpr int kStageB = 2 * kHalfB;
 constexpr int kPiece = kTile * kTile / 4;  // float4
 
@@ -109,6 +121,13 @@ FI_DEV void mfma(floatx4& acc, const short8& w, const short8& x) {
                : "v"(w), "v"(x));
 #endif
 }
+FI_DEV void mfma(floatx16& acc, const intx8& w, const intx8& x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("v_mfma_f32_32x32x64_f8f6f4 %0, %1, %2, %0"
+               : "+a"(acc)
+               : "v"(w), "v"(x));
+#endif
+}
 FI_DEV float acc_of(float a) {
   float v = a;
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -119,6 +138,12 @@ FI_DEV float acc_of(float a) {
 FI_DEV floatx4 acc_of(const floatx4& a) {
   return floatx4{acc_of(a[0]), acc_of(a[1]), acc_of(a[2]), acc_of(a[3])};
 }
+// four of a lane's results of a wave's fragment
+FI_DEV floatx4 quad_of(const floatx4& a, int) { return acc_of(a); }
+FI_DEV floatx4 quad_of(const floatx16& a, int g) {
+  return floatx4{acc_of(a[4 * g]), acc_of(a[4 * g + 1]), acc_of(a[4 * g + 2]),
+                 acc_of(a[4 * g + 3])};
+}
 FI_DEV void settle() {
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
@@ -128,24 +153,63 @@ FI_DEV void sync_waves() {
   asm volatile("" ::: "memory");
 }
 
-// W row (of the tile) of fragment f's row 0 in wave column wn; row i of the
-// fragment lies (i >> 2) * 8 + (i & 3) further on
-template <bool SILU_MUL>
-FI_DEV constexpr int w_row(int f) {
-  return SILU_MUL ? (f >> 2) * 128 + (f >> 1 & 1) * 32 + (f & 1) * 4
-                  : (f >> 1) * 32 + (f & 1) * 4;
-}
+// What the operands' type decides. A fragment is kRows rows of either operand
+// by half a stage of K; a lane has kChunks chunks of a row of it and kQuads
+// times four results of a product.
+//
+// w_row: W row (of the tile) of fragment f's row 0 in wave column wn; w_at:
+// how much further on row i of the fragment lies. A lane's results are then
+// neighbouring outputs of one row of x: eight of a fragment pair (bf16), 16
+// of a fragment (e4m3).
+template <bool FP8>
+struct Kind {
+  using Elem = u16;
+  using Frag = short8;
+  using Acc = floatx4;
+  static constexpr int kRows = 16, kChunks = 1, kQuads = 1;
+  static constexpr int w_row(int f, bool silu_mul) {
+    return silu_mul ? (f >> 2) * 128 + (f >> 1 & 1) * 32 + (f & 1) * 4
+                    : (f >> 1) * 32 + (f & 1) * 4;
+  }
+  FI_DEV static int w_at(int i) { return (i >> 2) * 8 + (i & 3); }
+  // three bits of W's row that tell a fragment's rows of one parity apart
+  FI_DEV static u32 w_key(int r) { return (r >> 1 & 1) | (r >> 3 & 3) << 1; }
+  FI_DEV static void put(Frag& f, int, const short8& v) { f = v; }
+};
+template <>
+struct Kind<true> {
+  using Elem = unsigned char;
+  using Frag = intx8;
+  using Acc = floatx16;
+  static constexpr int kRows = 32, kChunks = 2, kQuads = 4;
+  static constexpr int w_row(int f, bool) { return f * 32; }
+  FI_DEV static int w_at(int i) {
+    return (i >> 2 & 1) * 16 + (i >> 3) * 4 + (i & 3);
+  }
+  FI_DEV static u32 w_key(int r) { return (r >> 1 & 3) | (r >> 4 & 1) << 2; }
+  FI_DEV static void put(Frag& f, int chunk, const short8& v) {
+    const intx4 q = __builtin_bit_cast(intx4, v);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f[chunk * 4 + i] = q[i];
+  }
+};
 
 // what becomes of the products: nothing, + bias, silu(gate) * up
 enum { PLAIN, BIAS, SILU };
 
-// eight outputs of a row of x: fragments a, b; SILU: of gate values, the up
-// values that go with them in u, v
-template <int MODE>
-FI_DEV void store8(u16* to, const u16* bias, const floatx4& a,
-                   const floatx4& b, const floatx4& u, const floatx4& v) {
+// eight outputs of a row of x: sums a, b; SILU: of gate values, the up values
+// that go with them in u, v. FP8: times xs, the row's scale, and the scales
+// of W's rows at ws.
+template <int MODE, bool FP8>
+FI_DEV void store8(u16* to, const u16* bias, floatx4 a, floatx4 b,
+                   const floatx4& u, const floatx4& v, float xs,
+                   const floatx4* ws) {
   bf16x8 o, add;
   if (MODE == BIAS) add = *reinterpret_cast<const bf16x8*>(bias);
+  if (FP8) {
+    a *= xs * ws[0];
+    b *= xs * ws[1];
+  }
 #pragma unroll
   for (int r = 0; r < 8; ++r) {
     float y = r < 4 ? a[r] : b[r - 4];
@@ -157,22 +221,27 @@ FI_DEV void store8(u16* to, const u16* bias, const floatx4& a,
   *reinterpret_cast<bf16x8*>(to) = o;
 }
 
-template <int MODE>
+template <int MODE, bool FP8>
 __global__ __launch_bounds__(256, 1)
 void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
-                      const u16* __restrict__ x, const u16* __restrict__ w,
-                      const u16* __restrict__ bias, const int M, const int N,
-                      const int K, const int64_t x_stride,
+                      const typename Kind<FP8>::Elem* __restrict__ x,
+                      const typename Kind<FP8>::Elem* __restrict__ w,
+                      const u16* __restrict__ bias,
+                      const float* __restrict__ x_scales,
+                      const float* __restrict__ w_scales, const int M,
+                      const int N, const int K, const int64_t x_stride,
                       const int64_t out_stride, const TilePlan plan,
                       const int turn) {
+  using T = Kind<FP8>;
   constexpr bool SILU_MUL = MODE == SILU;
+  constexpr int kElemB = sizeof(typename T::Elem);
   __shared__ __attribute__((aligned(1024))) unsigned char smem[2 * kStageB];
   const u32 lds0 = static_cast<u32>(reinterpret_cast<uintptr_t>(
       (__attribute__((address_space(3))) unsigned char*)smem));
   const int lane = threadIdx.x % kWaveSize;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
   const int wm = wave >> 1, wn = wave & 1;
-  const int SK = K / kKS;
+  const int SK = K * kElemB / kRowB;
   // out columns of a tile, and all of them
   constexpr int kCols = SILU_MUL ? kTile / 2 : kTile;
   const int cols = SILU_MUL ? N / 2 : N;
@@ -207,11 +276,11 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
 
   // ---- requests: DMA j of a wave brings eight rows, group wave + 4 j of the
   // tile; lane l chunk (l % 8) ^ key of one of them
-  const u32 ab = static_cast<u32>(x_stride) * 2, wb = K * 2;
+  const u32 ab = static_cast<u32>(x_stride) * kElemB, wb = K * kElemB;
   const u32 a_voff = (lane >> 3) * ab +
                      (((lane & 7) ^ ((lane >> 4) | ((wave & 1) << 2))) << 4);
   const u32 b_voff = (lane >> 3) * wb +
-                     (((lane & 7) ^ (((lane >> 4) & 1) | (wave << 1))) << 4);
+                     (((lane & 7) ^ T::w_key(wave * 8 + (lane >> 3))) << 4);
   u32x4 da, db, dc;             // x rows, first and second half of W's rows
   int ru = 0, rs = 0, rend = 0, rlo = 0, left = 0;
   auto aim = [&] {
@@ -245,7 +314,10 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
     b_soff = wave * 8 * wb + rs * 128;
   };
   seek();
-  auto m0_of = [&](int j) { set_m0(rdst + j * 4096); };
+  auto m0_of = [&](int j) {
+    set_m0(rdst + j * 4096);
+    if (FP8) asm volatile("s_nop 0");   // no product lies in between
+  };
   auto load_of = [&](int j) {
     if (j < 8) load_lds(da, a_voff, a_soff + j * a_step);
     else if (j < 12) load_lds(db, b_voff, b_soff + (j - 8) * b_step);
@@ -258,22 +330,38 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
     seek();
   };
 
-  // ---- fragment reads: row lane & 15, chunk 4 half + (lane >> 4)
-  const int i16 = lane & 15, q = lane >> 4;
-  const u32 a_rd = (wm * 128 + i16) * 128 + ((q ^ (i16 >> 1)) << 4);
+  // ---- fragment reads: row lane % kRows, from chunk 4 half + q on; the i-th
+  // of eight
+  constexpr int kRows = T::kRows, kChunks = T::kChunks, kFrags = 8 / kChunks;
+  const int ir = lane % kRows, q = lane / kRows * kChunks;
+  const u32 a_rd = (wm * 128 + ir) * kRowB + ((q ^ (ir >> 1 & 7)) << 4);
   const u32 b_rd = kHalfB +
-      (wn * (SILU_MUL ? 64 : 128) + (i16 >> 2) * 8 + (i16 & 3)) * 128 +
-      ((q ^ ((i16 >> 1 & 1) | (i16 >> 2) << 1)) << 4);
-  auto rda = [&](int buf, int half, int mi) {
-    return *reinterpret_cast<const short8*>(
-        smem + buf * kStageB + (a_rd ^ (half * 64)) + mi * 2048);
+                   (wn * (SILU_MUL ? 64 : 128) + T::w_at(ir)) * kRowB +
+                   ((q ^ T::w_key(T::w_at(ir))) << 4);
+  using Frag = typename T::Frag;
+  auto rda = [&](Frag (&to)[kFrags], int buf, int half, int i) {
+    const int mi = i / kChunks, c = i % kChunks;
+    T::put(to[mi], c, *reinterpret_cast<const short8*>(
+        smem + buf * kStageB + (a_rd ^ (half * 64 + c * 16)) +
+        mi * kRows * kRowB));
   };
-  auto rdb = [&](int buf, int half, int f) {
-    return *reinterpret_cast<const short8*>(
-        smem + buf * kStageB + (b_rd ^ (half * 64)) + w_row<SILU_MUL>(f) * 128);
+  auto rdb = [&](Frag (&to)[kFrags], int buf, int half, int i) {
+    const int f = i / kChunks, c = i % kChunks;
+    T::put(to[f], c, *reinterpret_cast<const short8*>(
+        smem + buf * kStageB + (b_rd ^ (half * 64 + c * 16)) +
+        T::w_row(f, SILU_MUL) * kRowB));
   };
-  short8 a0[8], b0[8], a1[8], b1[8];
-  floatx4 acc[8][8];
+  Frag a0[kFrags], b0[kFrags], a1[kFrags], b1[kFrags];
+  typename T::Acc acc[kFrags][kFrags];
+  // place i of 64 in a half stage: a product, in e4m3 every fourth time (it
+  // takes as long as four)
+  auto product = [&](int i, const Frag (&b)[kFrags], const Frag (&a)[kFrags]) {
+    constexpr int kEach = 64 / (kFrags * kFrags);
+    if (i % kEach == 0)
+      mfma(acc[i / kEach / kFrags][i / kEach % kFrags],
+           b[i / kEach % kFrags], a[i / kEach / kFrags]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
 
   for (int k = 0; k < 2; ++k) {
 #pragma unroll
@@ -288,8 +376,8 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
   sync_waves();
 #pragma unroll
   for (int f = 0; f < 8; ++f) {
-    b0[f] = rdb(0, 0, f);
-    a0[f] = rda(0, 0, f);
+    rdb(b0, 0, 0, f);
+    rda(a0, 0, 0, f);
   }
   int buf = 0;
   constexpr int kFree = 40, kEarly = 6;  // MFMAs up to the first barrier, DMAs
@@ -297,11 +385,9 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
   auto stage = [&] {
 #pragma unroll
     for (int i = 0; i < 64; ++i) {
-      const int mi = i >> 3, f = i & 7;
-      mfma(acc[mi][f], b0[f], a0[mi]);
-      __builtin_amdgcn_sched_barrier(0);
-      if (i < 16 && i % 2 == 0) b1[i / 2] = rdb(buf, 1, i / 2);
-      if (i >= 16 && i < 32 && i % 2 == 0) a1[i / 2 - 8] = rda(buf, 1, i / 2 - 8);
+      product(i, b0, a0);
+      if (i < 16 && i % 2 == 0) rdb(b1, buf, 1, i / 2);
+      if (i >= 16 && i < 32 && i % 2 == 0) rda(a1, buf, 1, i / 2 - 8);
       if (i == kFree) {
         // all waves hold the stage in registers
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -321,11 +407,12 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
     buf ^= 1;
 #pragma unroll
     for (int i = 0; i < 64; ++i) {
-      const int mi = i >> 3, f = i & 7;
-      mfma(acc[mi][f], b1[f], a1[mi]);
-      __builtin_amdgcn_sched_barrier(0);
-      if (i % 4 == 0 && i < 32) b0[i / 4] = rdb(buf, 0, i / 4);
-      if (i % 4 == 0 && i >= 32) a0[i / 4 - 8] = rda(buf, 0, i / 4 - 8);
+      product(i, b1, a1);
+      // (e4m3: the last a few of its longer products before they are used)
+      constexpr int kGap = FP8 ? 3 : 4;
+      if (i % kGap == 0 && i < 8 * kGap) rdb(b0, buf, 0, i / kGap);
+      if (i % kGap == 0 && i >= 8 * kGap && i < 16 * kGap)
+        rda(a0, buf, 0, i / kGap - 8);
       if (i / 4 < 16 - kEarly) {
         if (i % 4 == 1) m0_of(kEarly + i / 4);
         if (i % 4 == 2) load_of(kEarly + i / 4);
@@ -337,9 +424,9 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
 
   for (int u = 0; u < units; ++u) {
 #pragma unroll
-    for (int mi = 0; mi < 8; ++mi)
+    for (int mi = 0; mi < kFrags; ++mi)
 #pragma unroll
-      for (int f = 0; f < 8; ++f) acc[mi][f] = {0.f, 0.f, 0.f, 0.f};
+      for (int f = 0; f < kFrags; ++f) acc[mi][f] = typename T::Acc(0.f);
     settle();
     const Unit t = unit(u);
     for (int s = 0; s < t.count; ++s) stage();
@@ -350,24 +437,57 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
     asm volatile("" : "+v"(l));
     const int row0 = t.m * kTile + wm * 128;
     if (t.count == SK) {
-      const int row1 = row0 + (l & 15);
-      const int col1 = t.n * kCols + wn * (kCols / 2) + (l >> 4) * 8;
+      const int row1 = row0 + l % kRows;
+      const int col1 = t.n * kCols + wn * (kCols / 2) +
+                       l / kRows * (FP8 ? 16 : 8);
       u16* to = out + row1 * out_stride + col1;
       const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+      // eight outputs at a time: 16 columns on per fragment (pairs of them in
+      // bf16, halves of them in e4m3)
+      constexpr int kEights = SILU_MUL ? 4 : 8;
+      // scales, all of them before the first store and waited for on every
+      // path: a load behind a store waits for it too, and one that may still
+      // be under way at the next stage would make that wait for all DMAs
+      float xs[4] = {};
+      floatx4 ws[16] = {};
+      if (FP8) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) xs[i] = x_scales[min(row1 + i * 32, M - 1)];
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          ws[i] = reinterpret_cast<const floatx4*>(
+              w_scales + min(col1 + i / 4 * 32, cols - 16))[i % 4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(xs[i]));
+#pragma unroll
+        for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(ws[i]));
+      }
       auto store = [&](bool inside) {
 #pragma unroll
-        for (int mi = 0; mi < 8; ++mi) {
-          if (inside || row1 + mi * 16 < M) {
+        for (int mi = 0; mi < kFrags; ++mi) {
+          if (inside || row1 + mi * kRows < M) {
 #pragma unroll
-            for (int f = 0; f < (SILU_MUL ? 4 : 8); f += 2)
-              if (inside || col1 + f * 16 < cols)
-                store8<MODE>(to + f * 16,
-                             MODE == BIAS ? bias + col1 + f * 16 : nullptr,
-                             acc_of(acc[mi][f]), acc_of(acc[mi][f + 1]),
-                             SILU_MUL ? acc_of(acc[mi][(f + 4) % 8]) : zero,
-                             SILU_MUL ? acc_of(acc[mi][(f + 5) % 8]) : zero);
+            for (int i = 0; i < kEights; i += 2) {
+              if (inside || col1 + i * 16 < cols) {
+                const u16* add = MODE == BIAS ? bias + col1 + i * 16 : nullptr;
+                if constexpr (FP8) {
+#pragma unroll
+                  for (int e = 0; e < 2; ++e)
+                    store8<MODE, FP8>(to + i * 16 + e * 8, nullptr,
+                                      quad_of(acc[mi][i / 2], 2 * e),
+                                      quad_of(acc[mi][i / 2], 2 * e + 1), zero,
+                                      zero, xs[mi], &ws[i * 2 + e * 2]);
+                } else {
+                  store8<MODE, FP8>(
+                      to + i * 16, add, acc_of(acc[mi][i]),
+                      acc_of(acc[mi][i + 1]),
+                      SILU_MUL ? acc_of(acc[mi][(i + 4) % 8]) : zero,
+                      SILU_MUL ? acc_of(acc[mi][(i + 5) % 8]) : zero, 0.f, ws);
+                }
+              }
+            }
           }
-          to += 16 * out_stride;
+          to += kRows * out_stride;
         }
       };
       if (t.m * kTile + kTile <= M && t.n * kCols + kCols <= cols)
@@ -378,12 +498,15 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
       floatx4* p = pieces + static_cast<int64_t>(place) * kPiece +
                    wave * 64 * kWaveSize + l;
 #pragma unroll
-      for (int mi = 0; mi < 8; ++mi) {
-        if (row0 + mi * 16 < M) {
+      for (int mi = 0; mi < kFrags; ++mi) {
+        if (row0 + mi * kRows < M) {
 #pragma unroll
-          for (int f = 0; f < 8; ++f) p[f * kWaveSize] = acc_of(acc[mi][f]);
+          for (int f = 0; f < kFrags; ++f)
+#pragma unroll
+            for (int g = 0; g < T::kQuads; ++g)
+              p[(f * T::kQuads + g) * kWaveSize] = quad_of(acc[mi][f], g);
         }
-        p += 8 * kWaveSize;
+        p += kFrags * T::kQuads * kWaveSize;
       }
     }
   }
@@ -393,30 +516,40 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
 
 // Sums the pieces of the cut tiles: blockIdx.y is the tile, a thread takes
 // eight outputs.
-template <int MODE>
+template <int MODE, bool FP8>
 __global__ __launch_bounds__(256)
 void tile_gemm_join_kernel(u16* __restrict__ out,
                            const floatx4* __restrict__ pieces,
-                           const u16* __restrict__ bias, const int M,
+                           const u16* __restrict__ bias,
+                           const float* __restrict__ x_scales,
+                           const float* __restrict__ w_scales, const int M,
                            const int N, const int64_t out_stride,
                            const TilePlan plan) {
+  using T = Kind<FP8>;
   constexpr bool SILU_MUL = MODE == SILU;
   constexpr int kCols = SILU_MUL ? kTile / 2 : kTile;
   const int cols = SILU_MUL ? N / 2 : N;
-  constexpr int kPairs = SILU_MUL ? 2 : 4;
+  constexpr int kFrags = 8 / T::kChunks, kQuads = kFrags * T::kQuads;
+  // pairs of quads of a wave's row of fragments (SILU: of its gate half)
+  constexpr int kPairs = kQuads / (SILU_MUL ? 4 : 2);
   const int i = blockIdx.x * 256 + threadIdx.x;
-  const int lane = i % kWaveSize, f = i / kWaveSize % kPairs * 2;
-  const int mi = i / kWaveSize / kPairs % 8, wave = i / kWaveSize / kPairs / 8;
+  const int lane = i % kWaveSize, pair = i / kWaveSize % kPairs;
+  const int mi = i / kWaveSize / kPairs % kFrags;
+  const int wave = i / kWaveSize / kPairs / kFrags;
   const Tile tile = tile_at(plan, plan.whole * kChip + blockIdx.y);
   const int m = tile.m, n = tile.n;
-  const int row = m * kTile + (wave >> 1) * 128 + mi * 16 + (lane & 15);
-  const int col = n * kCols + (wave & 1) * (kCols / 2) + f * 16 +
-                  (lane >> 4) * 8;
+  const int row = m * kTile + (wave >> 1) * 128 + mi * T::kRows +
+                  lane % T::kRows;
+  const int col = n * kCols + (wave & 1) * (kCols / 2) +
+                  (FP8 ? (pair >> 1) * 32 + lane / T::kRows * 16 +
+                             (pair & 1) * 8
+                       : pair * 32 + lane / T::kRows * 8);
   if (row >= M || col >= cols) return;
   constexpr int kOps = SILU_MUL ? 4 : 2;
   floatx4 s[4];
-  const floatx4* p = pieces + static_cast<int64_t>(blockIdx.y) * kPiece +
-                     ((wave * 8 + mi) * 8 + f) * kWaveSize + lane;
+  const floatx4* p =
+      pieces + static_cast<int64_t>(blockIdx.y) * kPiece +
+      ((wave * kFrags + mi) * kQuads + pair * 2) * kWaveSize + lane;
   const int64_t next = static_cast<int64_t>(plan.rest) * kPiece;
   for (int c = 0; c < plan.cut; c += 4) {
     floatx4 v[4][kOps];
@@ -425,22 +558,25 @@ void tile_gemm_join_kernel(u16* __restrict__ out,
 #pragma unroll
       for (int o = 0; o < kOps; ++o)
         v[k][o] = p[min(c + k, plan.cut - 1) * next +
-                    ((o & 1) + (o >> 1) * 4) * kWaveSize];
+                    ((o & 1) + (o >> 1) * (kQuads / 2)) * kWaveSize];
 #pragma unroll
     for (int k = 0; k < 4; ++k)
       if (c + k < plan.cut)
 #pragma unroll
         for (int o = 0; o < kOps; ++o) s[o] = c + k ? s[o] + v[k][o] : v[k][o];
   }
-  store8<MODE>(out + row * out_stride + col,
-               MODE == BIAS ? bias + col : nullptr, s[0], s[1],
-               s[SILU_MUL ? 2 : 0], s[SILU_MUL ? 3 : 1]);
+  store8<MODE, FP8>(out + row * out_stride + col,
+                    MODE == BIAS ? bias + col : nullptr, s[0], s[1],
+                    s[SILU_MUL ? 2 : 0], s[SILU_MUL ? 3 : 1],
+                    FP8 ? x_scales[row] : 0.f,
+                    reinterpret_cast<const floatx4*>(w_scales + col));
 }
 
-// A stage takes 1.42 us; a piece costs 0.06 us of the way through memory and
+// A stage takes 1.42 us (e4m3 too); a piece costs 0.06 us of the way through memory and
 // all of them 4 us for the second kernel. (504 sizes of 512 to 8192 rows and
 // 14 N and K: 0.98 of what is measured on average, 0.7 to 1.13.)
-TilePlan tile_plan(int M, int N, int K) {
+// KB: bytes of a row
+TilePlan tile_plan(int M, int N, int KB) {
   constexpr double kStage = 1.42;
   TilePlan p;
   p.mt = ceil_div(M, kTile);
@@ -448,7 +584,7 @@ TilePlan tile_plan(int M, int N, int K) {
   const int64_t tiles = static_cast<int64_t>(p.mt) * p.nt;
   p.whole = static_cast<int>(tiles / kChip);
   p.rest = static_cast<int>(tiles % kChip);
-  const int SK = K / kKS;
+  const int SK = KB / kRowB;
   p.cut = 1;
   double least = p.rest ? SK * kStage : 0;
   // two stages a piece at least: that many are requested ahead
@@ -464,14 +600,33 @@ TilePlan tile_plan(int M, int N, int K) {
   return p;
 }
 
+template <int MODE, bool FP8>
+void launch(u16* out, float* pieces, const typename Kind<FP8>::Elem* x,
+            const typename Kind<FP8>::Elem* w, const u16* bias,
+            const float* x_scales, const float* w_scales, int M, int N, int K,
+            int64_t x_stride, int64_t out_stride, hipStream_t stream) {
+  const int KB = K * static_cast<int>(sizeof(typename Kind<FP8>::Elem));
+  const TilePlan p = tile_plan(M, N, KB);
+  auto* pc = reinterpret_cast<floatx4*>(pieces);
+  const int turn = KB > 16384 && KB % 4096 == 0 ? 1 : 0;
+  hipLaunchKernelGGL((tile_gemm_kernel<MODE, FP8>), dim3(kChip), dim3(256), 0,
+                     stream, out, pc, x, w, bias, x_scales, w_scales, M, N, K,
+                     x_stride, out_stride, p, turn);
+  if (p.cut > 1)
+    hipLaunchKernelGGL((tile_gemm_join_kernel<MODE, FP8>),
+                       dim3(MODE == SILU ? 16 : 32, p.rest), dim3(256), 0,
+                       stream, out, pc, bias, x_scales, w_scales, M, N,
+                       out_stride, p);
+}
+
 }  // namespace
 
 // by its own estimate, in us
-double tile_gemm_us(int M, int N, int K) { return tile_plan(M, N, K).us; }
+double tile_gemm_us(int M, int N, int KB) { return tile_plan(M, N, KB).us; }
 
 // floats of scratch that launch_tile_gemm needs
-int64_t tile_gemm_floats(int M, int N, int K) {
-  const TilePlan p = tile_plan(M, N, K);
+int64_t tile_gemm_floats(int M, int N, int KB) {
+  const TilePlan p = tile_plan(M, N, KB);
   return p.cut > 1 ? static_cast<int64_t>(p.rest) * p.cut * kPiece * 4 : 0;
 }
 
@@ -479,22 +634,25 @@ int64_t tile_gemm_floats(int M, int N, int K) {
 void launch_tile_gemm(u16* out, float* pieces, const u16* x, const u16* w,
                       const u16* bias, int M, int N, int K, int64_t x_stride,
                       int64_t out_stride, bool silu_mul, hipStream_t stream) {
-  const TilePlan p = tile_plan(M, N, K);
-  auto* pc = reinterpret_cast<floatx4*>(pieces);
-  const int turn = K > 8192 && K % 2048 == 0 ? 1 : 0;
-  auto launch = [&](auto mode) {
-    constexpr int MODE = decltype(mode)::value;
-    hipLaunchKernelGGL((tile_gemm_kernel<MODE>), dim3(kChip), dim3(256), 0,
-                       stream, out, pc, x, w, bias, M, N, K, x_stride,
-                       out_stride, p, turn);
-    if (p.cut > 1)
-      hipLaunchKernelGGL((tile_gemm_join_kernel<MODE>),
-                         dim3(MODE == SILU ? 16 : 32, p.rest), dim3(256), 0,
-                         stream, out, pc, bias, M, N, out_stride, p);
-  };
-  if (silu_mul) launch(std::integral_constant<int, SILU>{});
-  else if (bias) launch(std::integral_constant<int, BIAS>{});
-  else launch(std::integral_constant<int, PLAIN>{});
+  if (silu_mul)
+    launch<SILU, false>(out, pieces, x, w, bias, nullptr, nullptr, M, N, K,
+                        x_stride, out_stride, stream);
+  else if (bias)
+    launch<BIAS, false>(out, pieces, x, w, bias, nullptr, nullptr, M, N, K,
+                        x_stride, out_stride, stream);
+  else
+    launch<PLAIN, false>(out, pieces, x, w, bias, nullptr, nullptr, M, N, K,
+                         x_stride, out_stride, stream);
+}
+
+// e4m3: K a multiple of 128 and 256 at least
+void launch_tile_gemm_fp8(u16* out, float* pieces, const unsigned char* x,
+                          const float* x_scales, const unsigned char* w,
+                          const float* w_scales, int M, int N, int K,
+                          int64_t x_stride, int64_t out_stride,
+                          hipStream_t stream) {
+  launch<PLAIN, true>(out, pieces, x, w, nullptr, x_scales, w_scales, M, N, K,
+                      x_stride, out_stride, stream);
 }
 
 }  // namespace fi

@@ -4,8 +4,8 @@ gfx950 runs OCP fp8 MFMA at ~2x the bf16 rate and halves weight-read
 bytes — decode-time GEMMs are weight-bandwidth-bound, so fp8 weights pay
 there directly. Enabled per-engine with `--quantization fp8`: projection
 weights are stored fp8 with per-output-channel scales; activations are
-dynamically quantized per-token; the GEMM (ops.linear_fp8: a HIP kernel
-for few rows, hipBLASLt above) gives bf16. The flagship benchmark stays bf16
+dynamically quantized per-token; the GEMM (ops.linear_fp8: HIP kernels for
+few rows and for many, hipBLASLt between) gives bf16. The flagship benchmark stays bf16
 (BASELINE dtype contract); fp8 is an opt-in serving mode.
 
 Note: gfx950 fp8 is OCP e4m3fn — NOT the MI300X fnuz variant.

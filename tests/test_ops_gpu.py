@@ -1151,6 +1151,52 @@ def test_linear_fp8_in_parts(rows, n, k):
             <= want.abs() * 2 ** -8 + 3e-4 * k ** 0.5).all()
 
 
+@pytest.mark.parametrize("rows", [1, 31, 255, 257, 1029])
+@pytest.mark.parametrize("n,k", [
+    (16, 256),           # one ragged tile, two stages, whole
+    (288, 384),          # three stages: not to be cut
+    (4128, 2048),        # cut tiles, a ragged last one
+    (288, 32768),        # 16 pieces, every other tile begins half way
+    (65568, 256),        # whole rounds of tiles and a rest
+])
+def test_linear_fp8_by_tiles(rows, n, k):
+    """e4m3 tiles of 256 x 256 against a float64 product: one bf16 rounding of
+    the result (2^-9 relative), fp32 sums and two scale products. Rows that
+    are not of the result stay as they were."""
+    g = torch.Generator().manual_seed(n + k + rows)
+    f8 = torch.float8_e4m3fn
+    w = torch.randn(n, k, generator=g).to(f8).to(DEV)
+    x = torch.randn(rows, 2 * k, generator=g).to(f8).to(DEV)[:, k:]
+    ws = torch.rand(n, generator=g).to(DEV) + 0.5
+    xs = torch.rand(rows, generator=g).to(DEV) + 0.5
+    out = torch.full((rows + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops._C.many_rows_gemm_fp8(out[:rows], x, xs, w, ws)
+    want = (x.double() @ w.double().T) * xs.double()[:, None] * ws.double()
+    assert ((out[:rows].double() - want).abs()
+            <= want.abs() * 2 ** -8 + 3e-4 * k ** 0.5).all()
+    assert (out[rows] == 7.0).all()
+
+
+def test_linear_fp8_takes_tiles():
+    """What the tiles take and what they leave to the library."""
+    f8 = torch.float8_e4m3fn
+    x = torch.randn(4099, 4096, device=DEV).to(f8)
+    w = torch.randn(4096, 4096, device=DEV).to(f8)
+    xs = torch.rand(4099, device=DEV) + 0.5
+    ws = torch.rand(4097, device=DEV) + 0.5
+    assert ops._tiles_fp8_ok(x, xs, w, ws[:4096])
+    for refused in ((x[:256], xs[:256], w, ws[:4096]),
+                    (x[:1024], xs[:1024], w, ws[:4096]),
+                    (x, xs, w, ws[1:]), (x, xs[:, None], w, ws[:4096]),
+                    (x[:, 8:4040], xs, w[:, 8:4040], ws[:4096]),
+                    (x.cpu(), xs.cpu(), w.cpu(), ws[:4096].cpu())):
+        assert not ops._tiles_fp8_ok(*refused)
+    want = (x.double() @ w.double().T) * xs.double()[:, None]
+    for s in (ws[:4096], ws[1:]):
+        err = (ops.linear_fp8(x, xs, w, s).double() - want * s.double()).abs()
+        assert (err <= (want * s.double()).abs() * 2 ** -8 + 0.02).all()
+
+
 def test_linear_fp8_takes_parts_by_size():
     """The sizes that stream and those of the library give the same."""
     f8 = torch.float8_e4m3fn
