@@ -42,6 +42,7 @@ MOE_SOURCES = [
     "moe_bindings.hip",
     "moe_gemm.hip",
     "moe_tile.hip",
+    "moe_wide.hip",
     "moe_plain.hip",
     "moe_router.hip",
     "moe_stream.hip",
@@ -71,7 +72,7 @@ EXTENSIONS = {
     "core": ("_C", SOURCES, ["common.h", "prefill_kernel.h", "tile_engine.h"]),
     "seqmix": ("_C_seqmix", SEQMIX_SOURCES, ["common.h", "seqmix.h", "seqmix_bind.h",
                 "seqmix_hyper.h", "seqmix_scan.h", "prefill_kernel.h"]),
-    "moe": ("_C_moe", MOE_SOURCES, ["common.h", "seqmix.h"]),
+    "moe": ("_C_moe", MOE_SOURCES, ["common.h", "seqmix.h", "tile_engine.h"]),
 }
 
 

@@ -13,8 +13,9 @@
 namespace fi {
 
 void launch_moe_gemm(u16*, const u16*, const u16*, const int*, const int*,
-                     const int*, int, int, int, int, int, int, float,
+                     const int*, int, int, int, int, int, int, int, float,
                      hipStream_t);
+bool wide_tiles(int, int, int, int, int);
 void launch_moe_route_grouped(const float*, const float*, float*, int*, int,
                               int, int, int, int, hipStream_t);
 void launch_moe_route_corrected(const float*, int64_t, const float*, float*,
@@ -99,7 +100,7 @@ void moe_gemm(at::Tensor out, at::Tensor a, at::Tensor b_packed,
   fi::launch_moe_gemm(bf16_ptr(out), bf16_cptr(a),
                       bf16_cptr(b_packed), sorted_ids.data_ptr<int>(),
                       expert_ids.data_ptr<int>(), n_valid.data_ptr<int>(),
-                      PM / block_m, a.size(0), K, N,
+                      PM / block_m, b_packed.size(0), a.size(0), K, N,
                       static_cast<int>(block_m), static_cast<int>(mode),
                       static_cast<float>(limit), current_stream());
 }
@@ -333,6 +334,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_gemm", &moe_gemm,
         "grouped MFMA GEMM over block-aligned expert segments "
         "(gate_up=true fuses the SwiGLU epilogue)");
+  m.def("moe_gemm_wide", &fi::wide_tiles,
+        "whether moe_gemm takes wide tiles for so many blocks of 128 rows, "
+        "experts, K, N, mode");
   m.def("moe_gemm_fp8", &moe_gemm_fp8,
         "grouped fp8 (e4m3) MFMA GEMM with per-row/per-channel dequant "
         "epilogue (gate_up=true fuses SwiGLU)");

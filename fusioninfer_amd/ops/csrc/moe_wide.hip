@@ -1,0 +1,325 @@
+// Grouped MFMA GEMM for long expert segments (128-row blocks, prompts) whose K
+// is a multiple of 64. Bound by the matrix cores.
+//
+// 256 persistent workgroups, one per CU, take tiles of 128 rows by 512 columns
+// of the expert's B (256 gate and the same 256 up columns where the epilogue
+// joins them). Four waves side by side hold 128 x 128 results each, so a
+// fragment read from LDS feeds eight MFMAs; the form with 128 x 256 tiles, two
+// workgroups per CU and B in registers loads half as much again per product
+// (48 bytes a cycle and CU, of 64 that the first-level cache delivers; here
+// 40).
+//
+// A stage is 64 of K: 128 gathered rows of 128 bytes, and 64 of B's packed
+// fragments (1 KB each), 80 KB in all; two of them are kept, all of a CU's
+// LDS. As in the dense kernel of 256 x 256 tiles a stage is used in two halves:
+// the second half's fragments are read while the first is multiplied, then
+// the stage's place is free and the stage after the next is requested into
+// it. Every MFMA is followed by at most one other instruction, in an order
+// that is pinned. The DMAs run on over the borders of tiles; the rows' ids
+// come through the scalar cache, since a vector load would wait for all DMAs
+// in front of it.
+//
+// LDS: 16-byte chunk c of row r sits at c ^ (r >> 1 & 7); B's fragments lie as
+// they are packed, in odd ones columns c at c ^ 4. MFMA operands are B, A; a
+// pair of fragments (32 columns) is read so that a lane ends with eight
+// neighbouring columns of a row: column (i >> 2) * 8 + (i & 3) + 4 p of the
+// pair is row i of product p.
+//
+// Workgroups of one XCD take a contiguous run of tiles, eight row blocks by
+// all column tiles at a time.
+//
+// A stage takes 1.4 us; a tile's end about 8, most of it until its results
+// have left (the stages after the first wait for them). Measured, us (TFLOP/s
+// of the real rows), 128 x 256 tiles and these: 8765 rows, 128 experts, top 8,
+// 2048 x 768: gate|up 456 (968) and 432 (1020), down 308 (717) and 266 (831);
+// 8192 rows, 64 experts, top 6, 2048 x 1408: 554 (1024) and 548, down 324 and
+// 284 (997); 8192 rows, 8 experts, top 2, 4096 x 6144 gate|up 1447 (1139) and
+// 1330 (1240).
+
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+
+#include "tile_engine.h"
+
+namespace fi {
+
+namespace {
+
+constexpr int kWideM = 128, kChip = 256;
+constexpr int kRowsB = kWideM * 128, kWaveB = 16 * 1024;  // A's, a wave's B
+constexpr int kWideStageB = kRowsB + 4 * kWaveB;
+constexpr int kRunRows = 8;                               // row blocks of a run
+
+template <int MODE>
+__global__ __launch_bounds__(256, 1) void moe_wide_kernel(
+    u16* __restrict__ out,              // [PM, N]
+    const u16* __restrict__ a,          // gathered x [T, K]; MODE 0 [PM, K]
+    const u16* __restrict__ b,          // [E][K/32][NB/16][64][8]
+    const int* __restrict__ sorted_ids, // [PM]
+    const int* __restrict__ expert_ids, // [PM/128]
+    const int* __restrict__ n_valid, const int K, const int N, const int NT,
+    const u32 a_bytes, const float limit) {
+  constexpr bool GATE_UP = MODE == 1 || MODE == 3;
+  __shared__ __attribute__((aligned(1024))) unsigned char
+      smem[2 * kWideStageB];
+  const u32 lds0 = static_cast<u32>(reinterpret_cast<uintptr_t>(
+      (__attribute__((address_space(3))) unsigned char*)smem));
+  const int lane = threadIdx.x % kWaveSize;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+  const int SK = K / 64;
+
+  // tiles of this workgroup: `first`, and every 32nd after it
+  const int nv = const_ints(n_valid)[0];
+  const int total = nv * NT, per = (total + 7) / 8;
+  const int run0 = (blockIdx.x & 7) * per;
+  const int first = run0 + (blockIdx.x >> 3);
+  const int end = min(run0 + per, total);
+  if (first >= end) return;
+  constexpr int kNext = kChip / 8;
+  struct Place {
+    int m, n;
+  };
+  auto place_of = [&](int at) {
+    const int m0 = at / (kRunRows * NT) * kRunRows;
+    const int rows = min(kRunRows, nv - m0);
+    const int in = at - m0 * NT;
+    const int n = in / rows;
+    return Place{m0 + in - n * rows, n};
+  };
+
+  // ---- requests: DMAs 0 to 3 bring eight rows of A each, the others a
+  // fragment of this wave's B
+  const int NB16 = (GATE_UP ? 2 * N : N) / 16;
+  const u32 b_step = static_cast<u32>(NB16) * 1024;   // 32 of K
+  constexpr int kOwn = GATE_UP ? 4 : 8;   // fragments apart from up's
+  const u32 up = N / 16 * 1024u;
+  u32 a_voff[4];
+  const u32 b_voff[2] = {lane * 16u, (lane ^ 4) * 16u};
+  u32x4 da, db;
+  int rat = first, left = 0;
+  u32 a_soff = 0, b_soff = 0, b_col[kOwn];
+  auto aim = [&] {
+    a_soff = b_soff = 0;
+    if (rat >= end) {           // past the end the last tile's beginning again
+      left = 1 << 30;
+      return;
+    }
+    const Place t = place_of(rat);
+    rat += kNext;
+    int ids[32];
+    if (MODE != 0) {
+      const auto from = const_ints(sorted_ids + t.m * kWideM + wave * 32);
+#pragma unroll
+      for (int i = 0; i < 32; ++i) ids[i] = from[i];
+      // in scalar registers, or the choice by lane becomes a vector load
+#pragma unroll
+      for (int i = 0; i < 32; ++i) asm volatile("" : "+s"(ids[i]));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      int row = wave * 32 + i * 8 + (lane >> 3);
+      if (MODE != 0) {
+        row = ids[i * 8];
+#pragma unroll
+        for (int r = 1; r < 8; ++r)
+          row = (lane >> 3) == r ? ids[i * 8 + r] : row;
+      }
+      a_voff[i] = static_cast<u32>(row) * (K * 2) +
+                  (((lane & 7) ^ (lane >> 4 | (i & 1) << 2)) << 4);
+    }
+    da = MODE != 0 ? uniform_descriptor(a, a_bytes)
+                   : uniform_descriptor(
+                         a + static_cast<int64_t>(t.m) * kWideM * K,
+                         kWideM * K * 2);
+    const int e = const_ints(expert_ids)[t.m];
+    db = uniform_descriptor(
+        b + static_cast<int64_t>(e) * (K / 32) * NB16 * 512,
+        K / 32 * b_step);
+#pragma unroll
+    for (int f = 0; f < kOwn; ++f)
+      b_col[f] = min((t.n * 4 + wave) * kOwn + f, N / 16 - 1) * 1024;
+    left = SK;
+  };
+  aim();
+  u32 rbuf = lds0;
+  auto m0_of = [&](int j) {
+    set_m0(j < 4 ? rbuf + wave * 4096 + j * 1024
+                 : rbuf + kRowsB + wave * kWaveB + (j - 4) * 1024);
+  };
+  auto load_of = [&](int j) {
+    if (j < 4) {
+      load_lds(da, a_voff[j], a_soff);
+    } else {
+      const int f = (j - 4) % 8, half = (j - 4) / 8;
+      load_lds(db, b_voff[f & 1],
+               b_soff + half * b_step + b_col[f % kOwn] +
+                   (f >= kOwn ? up : 0));
+    }
+  };
+  auto requested = [&] {
+    rbuf = 2 * lds0 + kWideStageB - rbuf;
+    a_soff += 128;
+    b_soff += 2 * b_step;
+    if (--left == 0) aim();
+  };
+
+  // ---- fragment reads: A row lane & 15, chunk 4 half + (lane >> 4)
+  const int i16 = lane & 15, q = lane >> 4;
+  const u32 a_rd = i16 * 128 + ((q ^ (i16 >> 1)) << 4);
+  const u32 b_rd = kRowsB + wave * kWaveB + (i16 >> 3) * 1024 +
+                   (q * 16 + (i16 >> 2 & 1) * 8 + (i16 >> 3) * 4 + (i16 & 3)) *
+                       16;
+  auto rda = [&](u32 buf, int half, int mi) {
+    return *reinterpret_cast<const short8*>(
+        smem + buf + (a_rd ^ (half * 64)) + mi * 2048);
+  };
+  auto rdb = [&](u32 buf, int half, int f) {
+    return *reinterpret_cast<const short8*>(
+        smem + buf + (b_rd ^ ((f & 1) * 64)) + half * 8192 + (f >> 1) * 2048);
+  };
+  short8 a0[8], b0[8], a1[8], b1[8];
+  floatx4 acc[8][8];
+
+  for (int k = 0; k < 2; ++k) {
+#pragma unroll
+    for (int j = 0; j < 20; ++j) {
+      m0_of(j);
+      asm volatile("s_nop 4");
+      load_of(j);
+    }
+    requested();
+  }
+  asm volatile("s_waitcnt vmcnt(20)" ::: "memory");
+  sync_waves();
+#pragma unroll
+  for (int f = 0; f < 8; ++f) {
+    b0[f] = rdb(0, 0, f);
+    a0[f] = rda(0, 0, f);
+  }
+  u32 buf = 0;
+  constexpr int kCols = GATE_UP ? 64 : 128;   // of a wave
+  constexpr int kStores = kCols / 4;          // of a tile
+  constexpr int kFree = 40, kEarly = 6;  // MFMAs up to the first barrier, DMAs
+                                         // between the two
+  // `behind`: stores that follow the DMAs that are waited for
+  auto stage = [&](auto first, bool behind) {
+#pragma unroll
+    for (int i = 0; i < 64; ++i) {
+      const int mi = i >> 3, f = i & 7;
+      if (first) mfma_first(acc[mi][f], b0[f], a0[mi]);
+      else mfma(acc[mi][f], b0[f], a0[mi]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (i < 16 && i % 2 == 0) b1[i / 2] = rdb(buf, 1, i / 2);
+      if (i >= 16 && i < 32 && i % 2 == 0)
+        a1[i / 2 - 8] = rda(buf, 1, i / 2 - 8);
+      if (i == kFree) {
+        // all waves hold the stage in registers
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        sync_waves();
+      }
+      const int j = i - kFree - 1;
+      if (j >= 0 && j < 2 * kEarly) {
+        if (j % 2 == 0) m0_of(j / 2);
+        else load_of(j / 2);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // the next stage has landed: this wave's DMAs but the youngest, and
+    // after the barrier all waves'
+    if (first && behind)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kEarly + kStores) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kEarly) : "memory");
+    sync_waves();
+    buf = kWideStageB - buf;
+#pragma unroll
+    for (int i = 0; i < 64; ++i) {
+      const int mi = i >> 3, f = i & 7;
+      mfma(acc[mi][f], b1[f], a1[mi]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (i % 4 == 0 && i < 32) b0[i / 4] = rdb(buf, 0, i / 4);
+      if (i % 4 == 0 && i >= 32) a0[i / 4 - 8] = rda(buf, 0, i / 4 - 8);
+      if (i / 4 < 20 - kEarly) {
+        if (i % 4 == 1) m0_of(kEarly + i / 4);
+        if (i % 4 == 2) load_of(kEarly + i / 4);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    requested();
+  };
+
+  bool behind = false;
+  for (int at = first; at < end; at += kNext) {
+    stage(std::true_type{}, behind);
+    for (int s = 1; s < SK; ++s) stage(std::false_type{}, false);
+    settle();
+    const Place t = place_of(at);
+    // (from a fresh copy of the lane, or the addresses would be kept in
+    // registers that the loop needs)
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    const int col = t.n * 4 * kCols + wave * kCols + (l >> 4) * 8;
+    u16* to = out +
+              static_cast<int64_t>(t.m * kWideM + (l & 15)) * N + col;
+    auto store = [&](bool inside) {
+#pragma unroll
+      for (int mi = 0; mi < 8; ++mi) {
+#pragma unroll
+        for (int f = 0; f < kCols / 16; f += 2) {
+          if (inside || col + f * 16 < N) {
+            bf16x8 o;
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+              const floatx4 g = acc_of(acc[mi][f + p]);
+              floatx4 u = g;
+              if (GATE_UP) u = acc_of(acc[mi][(f + p + 4) % 8]);
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                float v = g[r];
+                if (MODE == 3) {
+                  const float gt = fminf(v, limit);
+                  const float up1 = fminf(fmaxf(u[r], -limit), limit);
+                  v = (gt / (1.f + __expf(-1.702f * gt))) * (up1 + 1.f);
+                } else if (MODE == 1) {
+                  v = fast_silu(v) * u[r];
+                } else if (MODE == 2) {
+                  v = fmaxf(v, 0.f);
+                  v *= v;
+                }
+                o.h[p * 4 + r] = f32_to_bf16(v);
+              }
+            }
+            *reinterpret_cast<bf16x8*>(to + f * 16) = o;
+          }
+        }
+        to += static_cast<int64_t>(16) * N;
+      }
+    };
+    behind = (t.n + 1) * 4 * kCols <= N;
+    if (behind) store(true);
+    else store(false);
+  }
+  // no DMA may land in LDS that is no longer this workgroup's
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+}  // namespace
+
+void launch_moe_wide(u16* out, const u16* a, const u16* b,
+                     const int* sorted_ids, const int* expert_ids,
+                     const int* n_valid, int rows, int K, int N, int mode,
+                     float limit, hipStream_t stream) {
+  const int nt = ceil_div(N, mode == 1 || mode == 3 ? 256 : 512);
+#define FI_WIDE(M)                                                           \
+  hipLaunchKernelGGL((moe_wide_kernel<M>), dim3(kChip), dim3(256), 0,        \
+                     stream, out, a, b, sorted_ids, expert_ids, n_valid, K,  \
+                     N, nt, static_cast<u32>(rows) * (K * 2), limit)
+  if (mode == 1) FI_WIDE(1);
+  else if (mode == 2) FI_WIDE(2);
+  else if (mode == 3) FI_WIDE(3);
+  else FI_WIDE(0);
+#undef FI_WIDE
+}
+
+}  // namespace fi

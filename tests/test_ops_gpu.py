@@ -1354,6 +1354,22 @@ def test_moe_gemm_row_blocks_of_128(k, n, gate_up, act):
     check_moe_gemm(k, n, gate_up, act, 128)
 
 
+@pytest.mark.parametrize("k", [128, 192, 1088])
+@pytest.mark.parametrize("n,gate_up,act", [
+    (2880, True, None),         # ragged last tile and wave, one round
+    (7744, True, "clamped_glu"),  # two rounds
+    (5760, False, "relu_sq"),
+    (5760, False, None),
+    (15488, False, None),
+])
+def test_moe_gemm_wide_tiles(k, n, gate_up, act):
+    mode = 3 if act == "clamped_glu" else 1 if gate_up else 2 if act else 0
+    # as many blocks and experts as the check has
+    assert ops._moe_native().moe_gemm_wide(18, 7, k, n, mode)
+    assert not ops._moe_native().moe_gemm_wide(18, 7, k + 32, n, mode)
+    check_moe_gemm(k, n, gate_up, act, 128)
+
+
 @pytest.mark.parametrize("k", [32, 224, 512, 768, 1024, 2080, 2624])
 @pytest.mark.parametrize("n,gate_up,act", [
     (64, True, None), (320, True, "clamped_glu"), (192, False, "relu_sq"),
