@@ -84,7 +84,7 @@ __host__ __device__ __forceinline__ constexpr int ceil_div(int a, int b) {
 // and whether K/V ranges are cut into equal parts.
 struct PrefillPlan {
   int waves, hpb, rows, sub, nq, slots;
-  bool split;
+  bool split, pair;
 };
 
 // pack 8 f32 into 8 OCP-e4m3 bytes (two u32 words) via v_cvt_pk_fp8_f32

@@ -31,7 +31,7 @@ int64_t decode_piece_floats(int, int, int, int);
 void launch_paged_attn_decode(u16*, const u16*, const void*, const void*,
                               const int*, const int*, int, int64_t, int, int,
                               int, int, float, bool, float*, hipStream_t);
-PrefillPlan plan_prefill_attn(int, int, int, int, int, int);
+PrefillPlan plan_prefill_attn(int, int, int, int, int, int, int, bool);
 int64_t prefill_piece_floats(const PrefillPlan&, int);
 void launch_prefill_attn(u16*, const u16*, const void*, const void*,
                          const int*, const int*, const int*, const int*,
@@ -375,7 +375,7 @@ void prefill_attention(at::Tensor out, at::Tensor q, at::Tensor k,
   v = dma_rows(v);
   const fi::PrefillPlan pl = fi::plan_prefill_attn(
       tile_seq.size(0), tile_rows, num_q_heads, num_kv_heads, q.size(0),
-      k.size(0));
+      k.size(0), head_dim, false);
   at::Tensor pieces = prefill_pieces(pl, q);
   fi::launch_prefill_attn(
       bf16_ptr(out), bf16_cptr(q), bf16_cptr(k), bf16_cptr(v),
@@ -413,7 +413,7 @@ void prefill_attention_paged(at::Tensor out, at::Tensor q, at::Tensor k_cache,
   v_cache = dma_whole(v_cache);
   const fi::PrefillPlan pl = fi::plan_prefill_attn(
       tile_seq.size(0), tile_rows, num_q_heads, num_kv_heads, q.size(0),
-      block_tables.size(1) * 16);
+      block_tables.size(1) * 16, head_dim, fp8);
   at::Tensor pieces = prefill_pieces(pl, q);
   fi::launch_prefill_attn(
       bf16_ptr(out), bf16_cptr(q), k_cache.data_ptr(), v_cache.data_ptr(),

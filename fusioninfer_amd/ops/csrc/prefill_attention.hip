@@ -1,7 +1,7 @@
 // Prefill attention: the join of cut query tiles, the plan of a launch and
 // the launch itself.
 
-#include "prefill_kernel.h"
+#include "prefill_pair.h"
 
 #include <cmath>
 
@@ -92,12 +92,21 @@ void prefill_attn_join_kernel(const PrefillArgs p) {
 // 16 rows behind 2000: 47 / 33; 1024 behind 1024: 53 / 61; 1024 behind 8192:
 // 217 / 178; 4099 behind 16384: 1448 / 1250; 4096 behind 16384 (exactly two
 // rounds): 1190 / 1224; 2048 from the start: 57 / 100.
+//
+// The split form with 64 query vectors per wave (`pair`) takes 0.92 of the
+// time per tile, but 15 us more for its longer pipeline and the tiles that go
+// step by step: it is ahead from parts of 128 tiles on (8 query heads, 4 K/V
+// heads, 1024 rows behind 8192, parts of 17: 79 us, 94 with pairs; 32 and 8,
+// 700 + 33 + 1200 behind 6000, parts of 120: 240 and 250; 1000 behind 30000,
+// parts of 242: 519 and 489).
 PrefillPlan plan_prefill_attn(int ntiles, int tile_rows, int num_q_heads,
-                              int num_kv_heads, int new_rows, int max_k_len) {
+                              int num_kv_heads, int new_rows, int max_k_len,
+                              int head_dim, bool fp8) {
   const int group = num_q_heads / num_kv_heads;
   auto layout = [&](bool split) {
     PrefillPlan pl;
     pl.split = split;
+    pl.pair = false;
     pl.waves = attn_waves(split);
     pl.hpb = group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1);
     pl.rows = pl.waves * 32 / pl.hpb;
@@ -111,8 +120,10 @@ PrefillPlan plan_prefill_attn(int ntiles, int tile_rows, int num_q_heads,
                          (num_q_heads / pl.hpb);
   const int64_t tiles = ceil_div(max_k_len, kKVTile);
   const double fill = blocks / 256.0;
+  pl.pair = head_dim == 128 && !fp8 && fill * tiles >= 128;
   const double idle = fill < 1.0 ? 1.0 - std::min(1.0, 1.4 * fill)
-                                 : std::ceil(fill) - 1.04 * fill;
+                                 : std::ceil(fill) -
+                                       (pl.pair ? 0.96 : 1.04) * fill;
   // A workgroup's rows lie within one entry of the tile table: the split
   // form's 256 (one head per workgroup) do not fit into entries of 128.
   if (pl.rows > tile_rows ||
@@ -173,8 +184,12 @@ void launch_prefill_attn(u16* out, const u16* q, const void* k, const void* v,
 #define FI_PF_LAUNCH(DD, PP, F8)                                              \
   do {                                                                        \
     if (pl.split) {                                                           \
-      hipLaunchKernelGGL((prefill_attn_kernel<DD, PP, F8, true>),             \
-                         dim3(pl.slots), block, 0, stream, a);                \
+      if (PP && pl.pair)                                                      \
+        hipLaunchKernelGGL((prefill_pair_kernel<4>), dim3(pl.slots),          \
+                           dim3(4 * kWaveSize), 0, stream, a);                \
+      else                                                                    \
+        hipLaunchKernelGGL((prefill_attn_kernel<DD, PP, F8, true>),           \
+                           dim3(pl.slots), block, 0, stream, a);              \
       hipLaunchKernelGGL((prefill_attn_join_kernel<DD, PP>),                  \
                          dim3(pl.slots, pl.waves),                            \
                          dim3(DD / 16 * kWaveSize), 0, stream, a);            \

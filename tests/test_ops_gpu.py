@@ -427,6 +427,53 @@ def test_prefill_attention_row_blocks_and_parts(hq, hk, ctx_lens, new_lens,
     assert_close_bf16(out.cpu(), want, atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("scale_by", [1.0, -1.0, 8.0])
+@pytest.mark.parametrize("hq,hk", [
+    (64, 16),    # four heads per workgroup
+    (64, 32),    # two
+    (64, 64),    # one
+])
+def test_prefill_attention_long_parts(hq, hk, scale_by):
+    """Parts of more than 128 K/V tiles (two groups of queries per wave):
+    odd rows, a portion of 33 and one whose end lies within a tile, maxima
+    that jump late, against float64. Bound: P and the output are rounded to
+    bf16 (2^-9 each) and |v| stays below 6, hence 2.4e-2."""
+    g = torch.Generator().manual_seed(hq + hk)
+    new_lens, ctx_lens, D = [901, 33], [9001, 8064], 128
+    need = [-(-c // 16) for c in ctx_lens]
+    perm = (torch.randperm(sum(need), generator=g) + 1).int()
+    bt = torch.zeros(len(need), max(need), dtype=torch.int32)
+    for i, row in enumerate(perm.split(need)):
+        bt[i, :need[i]] = row
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g).to(torch.bfloat16).to(DEV)
+
+    q = rnd(sum(new_lens), hq, D)
+    kc, vc = rnd(sum(need) + 1, hk, 16, D), rnd(sum(need) + 1, hk, 16, D)
+    kc[int(bt[0, 300]), :, 5] *= 3.0     # a key that outweighs those before
+    for c in (kc, vc):                   # behind the end: never read
+        c[int(bt[0, need[0] - 1]), :, ctx_lens[0] % 16:] = float("nan")
+    cu = torch.tensor([0, 901, 934], dtype=torch.int32, device=DEV)
+    lens = torch.tensor(ctx_lens, dtype=torch.int32, device=DEV)
+    scale = scale_by / math.sqrt(D)
+    out = ops.prefill_attention_paged(q, kc, vc, bt.to(DEV), cu, lens, scale)
+    at = 0
+    for i, (n, c) in enumerate(zip(new_lens, ctx_lens)):
+        rows = bt[i, :need[i]].long().to(DEV)
+        hide = torch.arange(c, device=DEV) > torch.arange(
+            c - n, c, device=DEV)[:, None]
+        for h in range(0, hq, 7):
+            k = kc[rows, h * hk // hq].reshape(-1, D)[:c].double()
+            v = vc[rows, h * hk // hq].reshape(-1, D)[:c].double()
+            s = (q[at:at + n, h].double() @ k.T) * scale
+            s = s.masked_fill(hide, -math.inf)
+            want = torch.softmax(s, 1) @ v
+            err = (out[at:at + n, h].double() - want).abs()
+            assert (err <= 2.4e-2).all(), (i, h, err.max())
+        at += n
+
+
 @pytest.mark.parametrize("hq,hk", [(2, 2), (3, 1)])
 def test_prefill_attention_one_head_per_workgroup_small_entries(hq, hk):
     """4099 new rows make the tile table's entries 128 rows; with one head
