@@ -48,17 +48,42 @@ FI_DEV u16 f32_to_bf16(float f) {
   return c.u;
 }
 
-// Wave-wide reductions (64 lanes).
-FI_DEV float wave_reduce_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+template <int CTRL>
+FI_DEV float dpp_move(float x) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL,
+                                         0xF, 0xF, true));
+}
+
+// Wave-wide reductions (64 lanes, all of them active), by exchanges with the
+// lane 32, 16, 8, 4, 2 and 1 away. They stay among the registers: six of them
+// through LDS, as __shfl_xor has them, take 700 cycles. Swapping a register
+// with itself leaves either half's (row's) value in one of two; after the
+// exchange over 8 lanes a row has period 8, so a rotation by 4 reaches the
+// lane 4 away.
+template <class Op>
+FI_DEV float wave_reduce(float v, Op op) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto h = __builtin_amdgcn_permlane32_swap(
+      __float_as_int(v), __float_as_int(v), false, false);
+  v = op(__int_as_float(h[0]), __int_as_float(h[1]));
+  const auto r = __builtin_amdgcn_permlane16_swap(
+      __float_as_int(v), __float_as_int(v), false, false);
+  v = op(__int_as_float(r[0]), __int_as_float(r[1]));
+  v = op(v, dpp_move<0x128>(v));   // row_ror:8
+  v = op(v, dpp_move<0x124>(v));   // row_ror:4
+  v = op(v, dpp_move<0x4E>(v));    // quad_perm [2,3,0,1]
+  v = op(v, dpp_move<0xB1>(v));    // quad_perm [1,0,3,2]
+#endif
   return v;
 }
 
+FI_DEV float wave_reduce_sum(float v) {
+  return wave_reduce(v, [](float a, float b) { return a + b; });
+}
+
 FI_DEV float wave_reduce_max(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-  return v;
+  return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Block-wide sum over NWAVES waves (each wave passes its wave-reduced value

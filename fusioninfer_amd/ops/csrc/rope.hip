@@ -69,6 +69,8 @@ __global__ __launch_bounds__(kRopeWaves * kWaveSize) void rope_qk_norm_kernel(
   const int kv = head - num_q_heads;             // K heads, then V heads
   const bool is_v = CACHE && kv >= num_kv_heads;
 
+  // (requested here, not at its use behind the sums)
+  const int slot = CACHE ? cache.slots[token] : 0;
   const u16* row = is_q ? q + token * q_stride + head * D
       : is_v ? v + token * v_stride + (kv - num_kv_heads) * D
              : k + token * k_stride + kv * D;
@@ -93,7 +95,13 @@ __global__ __launch_bounds__(kRopeWaves * kWaveSize) void rope_qk_norm_kernel(
 #pragma unroll
       for (int i = 0; i < 8; ++i) sum += x[i] * x[i];
 #pragma unroll
-      for (int off = L / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+      for (int off = L / 2; off > 0; off >>= 1) {
+        if (off == 8) sum += dpp_move<0x128>(sum);       // row_ror:8
+        else if (off == 4 && L == 16) sum += dpp_move<0x124>(sum);  // :4
+        else if (off == 2) sum += dpp_move<0x4E>(sum);
+        else if (off == 1) sum += dpp_move<0xB1>(sum);
+        else sum += __shfl_xor(sum, off);
+      }
       const float inv_rms = rsqrtf(sum / D + eps);
 #pragma unroll
       for (int i = 0; i < 8; ++i) x[i] *= inv_rms * wf[i];
@@ -102,7 +110,8 @@ __global__ __launch_bounds__(kRopeWaves * kWaveSize) void rope_qk_norm_kernel(
     const float sign = e < D / 2 ? -1.f : 1.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const float other = __shfl_xor(x[i], L / 2);
+      const float other = L == 16 ? dpp_move<0x128>(x[i])
+                                  : __shfl_xor(x[i], L / 2);
       x[i] = x[i] * c[i / 4][i % 4] + sign * other * s[i / 4][i % 4];
     }
   }
@@ -116,7 +125,6 @@ __global__ __launch_bounds__(kRopeWaves * kWaveSize) void rope_qk_norm_kernel(
     *reinterpret_cast<u32x4_any*>(const_cast<u16*>(row) + e) = bits;
     return;
   }
-  const int slot = cache.slots[token];
   if (slot < 0) return;              // padding
   const int h = is_v ? kv - num_kv_heads : kv;
   const int64_t dst =

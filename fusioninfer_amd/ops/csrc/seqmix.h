@@ -88,13 +88,6 @@ FI_DEV void block_reduce_sum2_256(float& a, float& b, float* scratch) {
   b = scratch[4] + scratch[5] + scratch[6] + scratch[7];
 }
 
-template <int CTRL>
-FI_DEV float dpp_move(float x) {
-  return __builtin_bit_cast(
-      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL,
-                                         0xF, 0xF, true));
-}
-
 // sum over groups of SL adjacent lanes (a power of two up to 64); every
 // lane of a group ends with the total
 template <int SL>

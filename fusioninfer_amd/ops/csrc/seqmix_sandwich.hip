@@ -31,16 +31,22 @@ __global__ __launch_bounds__(256) void norm_residual_norm_kernel(
   A* orow = out + t * W;
   float dummy = 0.f, sq = 0.f;
   if constexpr (NCH > 0) {
-    float v[NCH][4], r[NCH][4];
+    // few rows take the time of one chain: both weights are requested with
+    // the row, the stream is written behind the sums (a barrier waits for
+    // what has been stored)
+    float v[NCH][4], r[NCH][4], wp[NCH][4], wn[NCH][4];
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
       const int i = (c * 256 + threadIdx.x) * 4;
       if (i < W) {
         ldv<A, 4>(yr + i, v[c]);
         ldv<float, 4>(rr + i, r[c]);
+        ldv<float, 4>(w_post + i, wp[c]);
+        ldv<float, 4>(w_next + i, wn[c]);
       } else {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) v[c][k] = r[c][k] = 0.f;
+        for (int k = 0; k < 4; ++k)
+          v[c][k] = r[c][k] = wp[c][k] = wn[c][k] = 0.f;
       }
 #pragma unroll
       for (int k = 0; k < 4; ++k) sq += v[c][k] * v[c][k];
@@ -52,14 +58,11 @@ __global__ __launch_bounds__(256) void norm_residual_norm_kernel(
     for (int c = 0; c < NCH; ++c) {
       const int i = (c * 256 + threadIdx.x) * 4;
       if (i >= W) continue;
-      float w4[4];
-      ldv<float, 4>(w_post + i, w4);
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        r[c][k] += v[c][k] * s1 * w4[k];
+        r[c][k] += v[c][k] * s1 * wp[c][k];
         sq += r[c][k] * r[c][k];
       }
-      stv<float, 4>(rr + i, r[c]);
     }
     block_reduce_sum2_256(sq, dummy, scratch);
     const float s2 = rsqrtf(sq / W + eps);
@@ -67,11 +70,10 @@ __global__ __launch_bounds__(256) void norm_residual_norm_kernel(
     for (int c = 0; c < NCH; ++c) {
       const int i = (c * 256 + threadIdx.x) * 4;
       if (i >= W) continue;
-      float w4[4];
-      ldv<float, 4>(w_next + i, w4);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) w4[k] *= r[c][k] * s2;
-      stv<A, 4>(orow + i, w4);
+      for (int k = 0; k < 4; ++k) wn[c][k] *= r[c][k] * s2;
+      stv<A, 4>(orow + i, wn[c]);
+      stv<float, 4>(rr + i, r[c]);
     }
   } else {
     for (int i = threadIdx.x; i < W; i += 256) {
