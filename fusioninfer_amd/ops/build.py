@@ -80,27 +80,13 @@ def extension_path(ext: str) -> str:
     return os.path.join(OPS_DIR, EXTENSIONS[ext][0] + ".so")
 
 
-def build(verbose: bool = True, force: bool = False) -> str:
-    """The core extension (kept as the historical entry point)."""
-    return build_extension("core", verbose=verbose, force=force)
-
-
-def build_extension(ext: str, verbose: bool = True,
-                    force: bool = False) -> str:
+def compile_command(mod_name: str):
+    """hipcc, and the command line that compiles a source of an extension."""
     import torch
     from torch.utils import cpp_extension as ce
 
-    mod_name, sources, headers = EXTENSIONS[ext]
-    so_path = extension_path(ext)
-    srcs = [os.path.join(CSRC, s) for s in sources]
-    hdrs = [os.path.join(CSRC, h) for h in headers]
-    if not force and os.path.exists(so_path):
-        so_mtime = os.path.getmtime(so_path)
-        if all(os.path.getmtime(f) < so_mtime for f in srcs + hdrs):
-            return so_path
     hipcc = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "bin", "hipcc")
-    torch_lib = ce.library_paths()[0]
-    common = [
+    return hipcc, [
         hipcc,
         "--offload-arch=gfx950",
         "-O3",
@@ -117,6 +103,27 @@ def build_extension(ext: str, verbose: bool = True,
         f"-I{sysconfig.get_paths()['include']}",
         f"-I{CSRC}",
     ]
+
+
+def build(verbose: bool = True, force: bool = False) -> str:
+    """The core extension (kept as the historical entry point)."""
+    return build_extension("core", verbose=verbose, force=force)
+
+
+def build_extension(ext: str, verbose: bool = True,
+                    force: bool = False) -> str:
+    from torch.utils import cpp_extension as ce
+
+    mod_name, sources, headers = EXTENSIONS[ext]
+    so_path = extension_path(ext)
+    srcs = [os.path.join(CSRC, s) for s in sources]
+    hdrs = [os.path.join(CSRC, h) for h in headers]
+    if not force and os.path.exists(so_path):
+        so_mtime = os.path.getmtime(so_path)
+        if all(os.path.getmtime(f) < so_mtime for f in srcs + hdrs):
+            return so_path
+    hipcc, common = compile_command(mod_name)
+    torch_lib = ce.library_paths()[0]
     out = None if verbose else subprocess.DEVNULL
 
     def run(cmd):

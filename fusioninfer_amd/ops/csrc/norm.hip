@@ -1,11 +1,21 @@
 // RMSNorm kernels (bf16, fp32 accumulation) for CDNA4.
 //
 // Capability parity: the fused rmsnorm+residual epilogue the reference
-// delegates to its vLLM containers (SURVEY.md §2.3 "RMSNorm ... fused ops").
+// delegates to its vLLM containers.
 //
 // One 256-thread workgroup per token row; bf16x8 vector loads (16 B/lane);
 // row held in registers between the sum-of-squares pass and the scale pass
-// (template ITERS gives compile-time register indexing — guide §5.4 rule 20).
+// (template ITERS gives compile-time register indexing).
+//
+// Few rows (a decode step) take the time of one chain of loads, sums and
+// stores: the weight is requested with the row (AHEAD), the new residual is
+// written behind the sums. Many rows are bound by memory, and what the weight
+// takes of the registers costs workgroups in flight. us a call, the weight and
+// the residual in the plain order and this (residual added, bf16 out): 4096
+// wide, 1 row 2.6 and 2.3, 64 rows 2.9 and 2.5, 1024 7.2 and 7.1, 4099 22.2
+// and 22.1; 16384 wide, 1 row 5.2 and 3.9, 64 rows 6.6 and 5.3. (Back to back
+// on a quiet card; in a decode step of 8 layers, 900 us, the difference is
+// within what two runs differ by.)
 
 #include "common.h"
 
@@ -16,8 +26,9 @@ namespace fi {
 // `out_scales` — the fused epilogue for the fp8 serving mode (the normalized
 // row only feeds a fp8 GEMM there, so the bf16 intermediate is never
 // materialized).
-template <int ITERS, bool FUSED_ADD, bool FP8_OUT>
-__global__ void rms_norm_kernel(
+// AHEAD: the weight is requested with the row, not behind the sums.
+template <int ITERS, bool FUSED_ADD, bool FP8_OUT, bool AHEAD>
+__global__ __launch_bounds__(256) void rms_norm_kernel(
     void* __restrict__ out_p,       // [T, H] bf16 (FP8_OUT: u8 e4m3)
     float* __restrict__ out_scales, // [T] (FP8_OUT only; else nullptr)
     const u16* __restrict__ in,     // [T, H]  (FUSED_ADD: the just-computed layer output x)
@@ -29,27 +40,34 @@ __global__ void rms_norm_kernel(
   const int tid = threadIdx.x;
   const int64_t base = static_cast<int64_t>(row) * hidden;
 
-  // Few rows (a decode step) take the time of one chain of loads, sums and
-  // stores: the weight is requested with the row, the new residual is written
-  // after the sum, since a barrier waits for what has been stored. (With
-  // reductions among registers and the cache slot of rope requested early, a
-  // step of eight layers: 901 -> 891 us at one row, 1735 -> 1717 at six with
-  // long contexts.)
+  constexpr int kRowsAtOnce = 2048;       // eight workgroups a CU
   float vals[ITERS][8];
   bf16x8 wt[ITERS];
   float sumsq = 0.f;
+  // the new residual is written behind the sums, whose barriers would wait
+  // for it; with more rows than the chip holds at once it goes out before,
+  // beside other rows' loads
+  const bool late = AHEAD && gridDim.x <= kRowsAtOnce;
+  auto keep = [&](int it) {
+    const int col = (it * blockDim.x + tid) * 8;
+    bf16x8 nr;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) nr.h[j] = f32_to_bf16(vals[it][j]);
+    *reinterpret_cast<bf16x8*>(residual + base + col) = nr;
+  };
 
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
     const int col = (it * blockDim.x + tid) * 8;
     if (col < hidden) {
       bf16x8 v = *reinterpret_cast<const bf16x8*>(in + base + col);
-      wt[it] = *reinterpret_cast<const bf16x8*>(weight + col);
+      if (AHEAD) wt[it] = *reinterpret_cast<const bf16x8*>(weight + col);
       if (FUSED_ADD) {
         bf16x8 r = *reinterpret_cast<const bf16x8*>(residual + base + col);
 #pragma unroll
         for (int j = 0; j < 8; ++j)
           vals[it][j] = bf16_to_f32(v.h[j]) + bf16_to_f32(r.h[j]);
+        if (!late) keep(it);
       } else {
 #pragma unroll
         for (int j = 0; j < 8; ++j) vals[it][j] = bf16_to_f32(v.h[j]);
@@ -63,26 +81,27 @@ __global__ void rms_norm_kernel(
   sumsq = wave_reduce_sum(sumsq);
   sumsq = block_reduce_sum<4>(sumsq, scratch);
   const float inv_rms = rsqrtf(sumsq / hidden + eps);
-  auto keep = [&](int it) {
-    const int col = (it * blockDim.x + tid) * 8;
-    bf16x8 nr;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) nr.h[j] = f32_to_bf16(vals[it][j]);
-    *reinterpret_cast<bf16x8*>(residual + base + col) = nr;
+  auto weight_of = [&](int it) {
+    return AHEAD ? wt[it]
+                 : *reinterpret_cast<const bf16x8*>(
+                       weight + (it * blockDim.x + tid) * 8);
   };
 
   if (FP8_OUT) {
-    // normalize into registers, then a second block reduce for the row
-    // absmax -> per-row scale -> pack via v_cvt_pk_fp8_f32
+    // a second block reduce for the row absmax of the normalized values ->
+    // per-row scale -> pack via v_cvt_pk_fp8_f32
     float amax = 0.f;
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
       const int col = (it * blockDim.x + tid) * 8;
       if (col < hidden) {
+        const bf16x8 w = weight_of(it);
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          amax = fmaxf(amax, fabsf(vals[it][j] * inv_rms *
-                                   bf16_to_f32(wt[it].h[j])));
+        for (int j = 0; j < 8; ++j) {
+          const float y = vals[it][j] * inv_rms * bf16_to_f32(w.h[j]);
+          amax = fmaxf(amax, fabsf(y));
+          if (!AHEAD) vals[it][j] = y;
+        }
       }
     }
     __shared__ float scratch_max[4];
@@ -98,13 +117,17 @@ __global__ void rms_norm_kernel(
       if (col < hidden) {
         float sv[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          sv[j] = vals[it][j] * inv_rms * bf16_to_f32(wt[it].h[j]) * inv_scale;
+        for (int j = 0; j < 8; ++j) {
+          const float y = AHEAD ? vals[it][j] * inv_rms *
+                                      bf16_to_f32(wt[it].h[j])
+                                : vals[it][j];
+          sv[j] = y * inv_scale;
+        }
         u32 packed[2];
         pack_fp8x8(sv, packed);
         *reinterpret_cast<u32*>(out8 + base + col) = packed[0];
         *reinterpret_cast<u32*>(out8 + base + col + 4) = packed[1];
-        if (FUSED_ADD) keep(it);
+        if (FUSED_ADD && late) keep(it);
       }
     }
   } else {
@@ -113,13 +136,13 @@ __global__ void rms_norm_kernel(
     for (int it = 0; it < ITERS; ++it) {
       const int col = (it * blockDim.x + tid) * 8;
       if (col < hidden) {
+        const bf16x8 w = weight_of(it);
         bf16x8 o;
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-          o.h[j] =
-              f32_to_bf16(vals[it][j] * inv_rms * bf16_to_f32(wt[it].h[j]));
+          o.h[j] = f32_to_bf16(vals[it][j] * inv_rms * bf16_to_f32(w.h[j]));
         *reinterpret_cast<bf16x8*>(out + base + col) = o;
-        if (FUSED_ADD) keep(it);
+        if (FUSED_ADD && late) keep(it);
       }
     }
   }
@@ -131,11 +154,21 @@ void launch_rms_norm(void* out, float* out_scales, const u16* in,
                      int hidden, hipStream_t stream) {
   dim3 grid(tokens), block(256);
   const int iters = ceil_div(hidden, 256 * 8);
+  // With the weight ahead of the sums rows of more than 12288 values take 126
+  // to 169 registers instead of 70 to 96: half the workgroups in flight. 1024
+  // rows of 16384, residual added, e4m3 out: 28.9 us, and 20.2 behind them;
+  // 14336 18.9 and 17.4. Up to 12288 the two differ by 2 % either way.
+  constexpr int kAlwaysAhead = 6;
+#define FI_LAUNCH(N, AHEAD)                                                  \
+  hipLaunchKernelGGL((rms_norm_kernel<N, FUSED_ADD, FP8_OUT, AHEAD>), grid,  \
+                     block, 0, stream, out, out_scales, in, residual,        \
+                     weight, eps, hidden)
 #define FI_CASE(N)                                                           \
   case N:                                                                    \
-    hipLaunchKernelGGL((rms_norm_kernel<N, FUSED_ADD, FP8_OUT>), grid,       \
-                       block, 0, stream, out, out_scales, in, residual,      \
-                       weight, eps, hidden);                                 \
+    if (N <= kAlwaysAhead || tokens <= 256)                                  \
+      FI_LAUNCH(N, true);                                                    \
+    else                                                                     \
+      FI_LAUNCH(N, N <= kAlwaysAhead);                                       \
     break;
   switch (iters) {
     FI_CASE(1)
@@ -151,6 +184,7 @@ void launch_rms_norm(void* out, float* out_scales, const u16* in,
       abort();
   }
 #undef FI_CASE
+#undef FI_LAUNCH
 }
 
 template void launch_rms_norm<true, false>(void*, float*, const u16*, u16*,

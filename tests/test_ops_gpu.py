@@ -49,6 +49,40 @@ def test_fused_add_rms_norm(tokens, hidden):
     assert_close_bf16(out.cpu(), x_ref)
 
 
+@pytest.mark.parametrize("hidden", [12288, 12296, 14344, 16384])
+@pytest.mark.parametrize("tokens", [1, 256, 257, 2048, 2049])
+def test_norms_of_wide_rows(tokens, hidden):
+    """Where the weight is requested and the residual is written changes at
+    257 and 2049 rows and above 12288 values."""
+    g = torch.Generator(DEV).manual_seed(tokens + hidden)
+    x, res = (torch.randn(tokens, hidden, dtype=torch.bfloat16, device=DEV,
+                          generator=g) for _ in range(2))
+    w = torch.randn(hidden, dtype=torch.bfloat16, device=DEV, generator=g)
+
+    def normed(rows):
+        rows = rows.float()
+        return rows * torch.rsqrt(rows.square().mean(-1, keepdim=True)
+                                  + 1e-6) * w.float()
+
+    def near_fp8(f8, scales, exact):
+        # half a step of e4m3 is 2^-4 of a value, and 2^-10 of the scale
+        # where values are small
+        err = (f8.float() * scales[:, None] - exact).abs()
+        assert (err <= exact.abs() / 16 + scales[:, None] / 512).all()
+
+    exact = normed(x)
+    assert_close_bf16(ops.rms_norm(x, w, 1e-6), exact)
+    near_fp8(*ops.rms_norm_fp8(x, w, 1e-6), exact)
+    total = x.float() + res.float()
+    exact = normed(total)
+    f8, scales, new = ops.fused_add_rms_norm_fp8(x, res.clone(), w, 1e-6)
+    assert torch.equal(new, total.bfloat16())
+    near_fp8(f8, scales, exact)
+    out, new = ops.fused_add_rms_norm(x, res, w, 1e-6)
+    assert torch.equal(new, total.bfloat16())
+    assert_close_bf16(out, exact)
+
+
 @pytest.mark.parametrize("tokens,inter", [(7, 12288), (64, 512)])
 def test_silu_and_mul(tokens, inter):
     x = torch.randn(tokens, 2 * inter, dtype=torch.bfloat16, device=DEV)
