@@ -41,6 +41,7 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(
   const int64_t base = static_cast<int64_t>(row) * hidden;
 
   constexpr int kRowsAtOnce = 2048;       // eight workgroups a CU
+  constexpr int kSecondFirst = ITERS > 1;
   float vals[ITERS][8];
   bf16x8 wt[ITERS];
   float sumsq = 0.f;
@@ -72,8 +73,14 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(
 #pragma unroll
         for (int j = 0; j < 8; ++j) vals[it][j] = bf16_to_f32(v.h[j]);
       }
+      // in an order that is written out: left to the compiler, which of the
+      // first two squares is rounded before it is added changes with what
+      // surrounds the loop, and outputs with it
 #pragma unroll
-      for (int j = 0; j < 8; ++j) sumsq += vals[it][j] * vals[it][j];
+      for (int j = 0; j < 8; ++j) {
+        const float x = vals[it][it == 0 && j < 2 ? j ^ kSecondFirst : j];
+        sumsq = fmaf(x, x, sumsq);
+      }
     }
   }
 

@@ -83,6 +83,32 @@ def test_norms_of_wide_rows(tokens, hidden):
     assert_close_bf16(out, exact)
 
 
+@pytest.mark.parametrize("hidden", [1024, 2048, 2056, 4096, 16384])
+def test_norm_order_of_the_first_squares(hidden):
+    """A thread adds its squares by fma, of the first two the second comes
+    first (the first in rows of up to 2048 values): the same two values
+    further on, in that order, give the same bits, and in the other order
+    they do not always."""
+    rows = 4096
+    g = torch.Generator(DEV).manual_seed(hidden)
+    x, res = (torch.randn(rows, 2, dtype=torch.bfloat16, device=DEV,
+                          generator=g) for _ in range(2))
+    w = torch.ones(hidden, dtype=torch.bfloat16, device=DEV)
+
+    def scales_and_rows(*at):
+        a, b = (torch.zeros(rows, hidden, dtype=torch.bfloat16, device=DEV)
+                for _ in range(2))
+        a[:, list(at)], b[:, list(at)] = x, res
+        scales = ops.fused_add_rms_norm_fp8(a, b.clone(), w, 0.0)[1]
+        return scales, ops.fused_add_rms_norm(a, b, w, 0.0)[0][:, list(at)]
+
+    first, first_rows = scales_and_rows(0, 1)
+    same, same_rows = scales_and_rows(*((2, 3) if hidden <= 2048 else (3, 2)))
+    other, _ = scales_and_rows(*((3, 2) if hidden <= 2048 else (2, 3)))
+    assert torch.equal(first, same) and torch.equal(first_rows, same_rows)
+    assert not torch.equal(first, other)
+
+
 @pytest.mark.parametrize("tokens,inter", [(7, 12288), (64, 512)])
 def test_silu_and_mul(tokens, inter):
     x = torch.randn(tokens, 2 * inter, dtype=torch.bfloat16, device=DEV)
