@@ -31,10 +31,10 @@
 // A stage takes 1.4 us; a tile's end about 8, most of it until its results
 // have left (the stages after the first wait for them). Measured, us (TFLOP/s
 // of the real rows), 128 x 256 tiles and these: 8765 rows, 128 experts, top 8,
-// 2048 x 768: gate|up 456 (968) and 432 (1020), down 308 (717) and 266 (831);
-// 8192 rows, 64 experts, top 6, 2048 x 1408: 554 (1024) and 548, down 324 and
-// 284 (997); 8192 rows, 8 experts, top 2, 4096 x 6144 gate|up 1447 (1139) and
-// 1330 (1240).
+// 2048 x 768: gate|up 467 (945) and 445 (992), down 308 (717) and 266 (831);
+// 8192 rows, 64 experts, top 6, 2048 x 1408: 544 (1040) and 549, down 324 and
+// 284 (997); 8192 rows, 8 experts, top 2, 4096 x 6144 gate|up 1385 (1190) and
+// 1324 (1245).
 
 #include <hip/hip_runtime.h>
 
@@ -282,7 +282,7 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
                   const float up1 = fminf(fmaxf(u[r], -limit), limit);
                   v = (gt / (1.f + __expf(-1.702f * gt))) * (up1 + 1.f);
                 } else if (MODE == 1) {
-                  v = fast_silu(v) * u[r];
+                  v = silu(v) * u[r];
                 } else if (MODE == 2) {
                   v = fmaxf(v, 0.f);
                   v *= v;

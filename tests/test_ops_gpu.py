@@ -1200,6 +1200,35 @@ def test_linear_by_tiles(rows, n, k, bias):
         assert (out[rows] == 7.0).all()
 
 
+def test_silu_by_tiles_of_far_gates():
+    """Gates down to where 1 + exp(-gate) leaves fp32, infinite ones and NaN,
+    against float64: exp of fp32 is off by |gate| 2^-23, the result has one
+    bf16 rounding. (A product with a zero carries a row's infinity into all
+    of its sums, so each kind has a column of x to itself.)"""
+    n, k = 512, 128
+    gates = torch.linspace(-88.5, 88.5, n // 2 - 4).bfloat16()
+    gates = torch.cat([gates, torch.tensor([-1e30, -200.0, 0.0, 1e38])
+                       .bfloat16()])
+    w = torch.zeros(n, k, dtype=torch.bfloat16)
+    w[: n // 2, 0] = gates
+    w[n // 2:, 0] = 2.0 ** 100
+    w[: n // 2, 1] = w[n // 2:, 2] = 1.0
+    x = torch.zeros(300, k, dtype=torch.bfloat16)
+    x[:290, 0] = 1.0
+    x[290:292, 1], x[292:294, 1] = float("inf"), float("-inf")
+    x[294:296, 1] = float("nan")
+    x[290:296, 2] = 1.0
+    out = torch.empty(300, n // 2, dtype=torch.bfloat16, device=DEV)
+    ops._C.many_rows_gemm(out, x.to(DEV), w.to(DEV), None, True)
+    got = out.double().cpu()
+    g = gates.double()
+    want = g / (1 + torch.exp(-g)) * 2.0 ** 100
+    err = (got[:290, :-4] - want[:-4]).abs()
+    assert (err <= want[:-4].abs() * (2 ** -8 + 89 * 2 ** -23)).all()
+    assert (got[:290, -4:-1] == 0).all() and got[:290, -1].isinf().all()
+    assert got[290:296].isnan().all()
+
+
 def test_linear_takes_tiles():
     """Whole rounds with every other tile begun half way and a cut rest, as
     ops.linear chooses it; what it refuses goes to the library."""
@@ -1475,6 +1504,31 @@ def test_moe_gemm_wide_tiles(k, n, gate_up, act):
     assert ops._moe_native().moe_gemm_wide(18, 7, k, n, mode)
     assert not ops._moe_native().moe_gemm_wide(18, 7, k + 32, n, mode)
     check_moe_gemm(k, n, gate_up, act, 128)
+
+
+def test_moe_gemm_wide_tiles_are_the_narrow_ones():
+    """Blocks of 128 rows have the same bits whether there are enough of them
+    for wide tiles or not; gates reach to where 1 + exp(-gate) leaves fp32."""
+    g = torch.Generator().manual_seed(11)
+    experts, k, n, T = 4, 128, 2880, 2000
+    x = torch.randn(T, k, generator=g).bfloat16()
+    x[::3] *= 8
+    w = torch.randn(experts, k, 2 * n, generator=g).bfloat16()
+    topi = torch.randint(0, experts, (T, 1), generator=g).int().to(DEV)
+    sid, eid, nv, pos, PM = ops.moe_align(topi, 0, experts, 128)
+    x, b = x.to(DEV), ops.pack_moe_weights(w.to(DEV))
+    out = torch.zeros(PM, n, dtype=torch.bfloat16, device=DEV)
+    blocks = int(nv)
+    wide = ops._moe_native().moe_gemm_wide
+    assert wide(PM // 128, experts, k, n, 1) and not wide(4, experts, k, n, 1)
+    ops.moe_gemm(out, x, b, sid, eid, nv, 128, True, None, 3.0)
+    few = torch.zeros_like(out)
+    for m in range(0, blocks, 4):
+        count = min(4, blocks - m)
+        rows = slice(m * 128, (m + count) * 128)
+        ops.moe_gemm(few[rows], x, b, sid[rows], eid[m:m + count],
+                     torch.full_like(nv, count), 128, True, None, 3.0)
+    assert torch.equal(out, few)
 
 
 @pytest.mark.parametrize("k", [32, 224, 512, 768, 1024, 2080, 2624])
