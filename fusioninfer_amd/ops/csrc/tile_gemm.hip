@@ -206,18 +206,28 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
   };
 
   // ---- requests: DMA j of a wave brings eight rows, group wave + 4 j of the
-  // tile; lane l chunk (l % 8) ^ key of one of them
+  // tile; lane l chunk (l % 8) ^ key of one of them. The row is in the vector
+  // offset and the place along K in the scalar one, which so never reaches
+  // past a descriptor's end: rows past it are cut off by the vector offset
+  // alone (the bound that it is held against is the size less the scalar
+  // offset, and need not be right where that is negative).
   const u32 ab = static_cast<u32>(x_stride) * kElemB, wb = K * kElemB;
-  const u32 a_voff = (lane >> 3) * ab +
-                     (((lane & 7) ^ ((lane >> 4) | ((wave & 1) << 2))) << 4);
-  const u32 b_voff = (lane >> 3) * wb +
-                     (((lane & 7) ^ T::w_key(wave * 8 + (lane >> 3))) << 4);
+  u32 a_voff[8], b_voff[4];
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    a_voff[j] = ((wave + 4 * j) * 8 + (lane >> 3)) * ab +
+                (((lane & 7) ^ ((lane >> 4) | ((wave & 1) << 2))) << 4);
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    b_voff[j] = ((wave + 4 * j) * 8 + (lane >> 3)) * wb +
+                (((lane & 7) ^ T::w_key(wave * 8 + (lane >> 3))) << 4);
   u32x4 da, db, dc;             // x rows, first and second half of W's rows
+  constexpr int kPast = 1 << 30;
   int ru = 0, rs = 0, rend = 0, rlo = 0, left = 0;
   auto aim = [&] {
     if (ru == units) {          // past the end nothing is read
       da[2] = db[2] = dc[2] = 0;
-      left = 1 << 30;
+      left = kPast;
       return;
     }
     const Unit t = unit(ru++);
@@ -229,30 +239,29 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
     const int end1 = SILU_MUL ? N : cols;
     db = uniform_descriptor(w + static_cast<int64_t>(n0) * K,
                        min(kTile / 2, cols - n0) * wb);
-    dc = uniform_descriptor(w + static_cast<int64_t>(min(n1, end1)) * K,
-                       max(0, min(kTile / 2, end1 - n1)) * wb);
+    if (n1 < end1)
+      dc = uniform_descriptor(w + static_cast<int64_t>(n1) * K,
+                              min(kTile / 2, end1 - n1) * wb);
+    else
+      dc = db;                  // nobody uses these columns
     rlo = t.lo;
     rend = t.lo + t.count;
     rs = t.lo + t.rot;
     left = t.count;
   };
   aim();
-  const u32 a_step = 32 * ab, b_step = 32 * wb;   // four groups of eight rows
   u32 rdst = lds0 + wave * 1024;
-  u32 a_soff = 0, b_soff = 0;
-  auto seek = [&] {
-    a_soff = wave * 8 * ab + rs * 128;
-    b_soff = wave * 8 * wb + rs * 128;
-  };
+  u32 soff = 0;
+  auto seek = [&] { soff = left > kPast / 2 ? 0 : rs * kRowB; };
   seek();
   auto m0_of = [&](int j) {
     set_m0(rdst + j * 4096);
     if (FP8) asm volatile("s_nop 0");   // no product lies in between
   };
   auto load_of = [&](int j) {
-    if (j < 8) load_lds(da, a_voff, a_soff + j * a_step);
-    else if (j < 12) load_lds(db, b_voff, b_soff + (j - 8) * b_step);
-    else load_lds(dc, b_voff, b_soff + (j - 12) * b_step);
+    if (j < 8) load_lds(da, a_voff[j], soff);
+    else if (j < 12) load_lds(db, b_voff[j - 8], soff);
+    else load_lds(dc, b_voff[j - 12], soff);
   };
   auto requested = [&] {
     rdst ^= kStageB;

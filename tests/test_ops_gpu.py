@@ -1200,6 +1200,30 @@ def test_linear_by_tiles(rows, n, k, bias):
         assert (out[rows] == 7.0).all()
 
 
+@pytest.mark.parametrize("rows,n,k", [
+    (257, 144, 128),      # one row and 16 columns over; two stages
+    (264, 16, 1024),      # eight rows over, half a tile of W without a row
+    (513, 272, 4096),     # cut tiles, one row and 16 columns over
+])
+def test_linear_by_tiles_reads_its_operands_alone(rows, n, k):
+    """What lies behind the last row of either operand has no part in the
+    result."""
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, k, generator=g).bfloat16().to(DEV)
+    w = torch.randn(n, k, generator=g).bfloat16().to(DEV)
+    xn, wn = (torch.full((512 + t.shape[0], k), float("nan"),
+                         dtype=torch.bfloat16, device=DEV) for t in (x, w))
+    xn[:rows], wn[:n] = x, w
+    out, same = (torch.empty(rows, n, dtype=torch.bfloat16, device=DEV)
+                 for _ in range(2))
+    ops._C.many_rows_gemm(out, x, w, None, False)
+    ops._C.many_rows_gemm(same, xn[:rows], wn[:n], None, False)
+    assert torch.equal(out, same)
+    want = x.double() @ w.double().T
+    assert ((out.double() - want).abs()
+            <= want.abs() * 2 ** -8 + 1e-4 * k ** 0.5).all()
+
+
 def test_silu_by_tiles_of_far_gates():
     """Gates down to where 1 + exp(-gate) leaves fp32, infinite ones and NaN,
     against float64: exp of fp32 is off by |gate| 2^-23, the result has one
