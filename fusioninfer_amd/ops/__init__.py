@@ -179,16 +179,19 @@ def _tiles(M: int, N: int, K: int, silu_mul: bool = False) -> bool:
     more than 256 rows. On whole rounds of tiles both reach 1.4 to 1.55
     PFLOP/s; the kernel cuts what is left over into even pieces, where the
     library's choice of tiles takes up to twice as long (4099 rows, 4096 x
-    12288: 312 us here, 619; 24576 x 4096 580 and 690; 2700 1.22 times). The
-    kernel's own estimate is held against 8 us and 1.2 PFLOP/s, or the chain
-    of 7 us per 1000 of K; with silu_mul the pass over the product is added,
-    which the kernel has in its epilogue (7600 rows, 24576 x 4096 1041 us
-    here, 1135). Over 504 sizes this takes 2.6 % longer than the better of
-    the two, the library alone 4.8 (up to 98), the kernel alone 11.
+    12288: 281 us here, 614; 24576 x 4096 572 and 695; 2700 rows 380 and
+    471). The kernel's own estimate is held against 8 us and 1.2 PFLOP/s, or
+    the chain of 7 us per 1000 of K; with silu_mul the pass over the product
+    is added, which the kernel has in its epilogue (7600 rows, 24576 x 4096
+    1020 us here, 1127). Over 504 sizes this took 2.6 % longer than the better
+    of the two, the library alone 4.8 (up to 98), the kernel alone 11 (before
+    rows of x and W went by the vector offset, which made the kernel up to an
+    eighth faster where K is long).
 
     Where both operands together outgrow the memory-side cache and rows are
-    longer than 16 KB the library is ahead more often than not (7600 rows,
-    4096 x 12288 533 us, 627 here)."""
+    longer than 16 KB the two are even or the library is ahead (4096 x 12288
+    at 7600 rows 519 us, 525 here, at 8192 530 and 528; 8192 x 14336 at 6000
+    900 and 1008)."""
     if K > 8192 and (M + N) * K > 1 << 27:
         return False
     library = max(8 + 2 * M * N * K / 1.2e9, 7e-3 * K)
@@ -261,8 +264,8 @@ def _streams_fp8(M: int, N: int, K: int) -> bool:
 def _tiles_fp8(M: int, N: int, K: int) -> bool:
     """As _tiles, for e4m3 operands: the kernel's own estimate against 6 us
     and 2.2 PFLOP/s, or 18 us and 2 us per 1000 of K above 8192 (4096 x 4096
-    at 1024 rows 36.6 us here, the library 23.0; at 8192 100.4 and 102.8;
-    4096 x 12288 at 4099 153 and 268). Over twelve N and K and up to 17 M of
+    at 1024 rows 38 us here, the library 28; at 8192 100 and 111; 4096 x
+    12288 at 4099 151 and 270). Over twelve N and K and up to 17 M of
     257 to 8192 this takes 2.4 % longer than the better of the two, the
     library alone 8.9 (up to 75), the kernel alone 8.7."""
     return _C.many_rows_gemm_us(M, N, K) < max(

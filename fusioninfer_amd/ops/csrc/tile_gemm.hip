@@ -31,18 +31,18 @@
 // What whole rounds of 256 tiles leave over is cut along K into equal pieces
 // (tile_plan), which a second kernel sums in a fixed order.
 //
-// Where both operands are larger than the 256 MB memory-side cache and rows
-// are a multiple of 4 KB and longer than 16 KB, reads of the same K by all
-// CUs meet on few memory channels (8192 x 4096 x 12288: 1.28 PFLOP/s, with K
-// of 12160 or 12416 1.49); there every other column tile starts half way
-// along K (1.41).
+// Where rows are a multiple of 4 KB, reads of the same K by all CUs meet on few
+// memory channels. With rows longer than 16 KB every other column tile starts
+// half way along K: bf16, 4096 x 12288 at 4099, 6000 and 7600 rows 294, 437 and
+// 540 us, so 285, 428 and 526 (at 1024 rows 90 and 91); K 10240 the same either
+// way; e4m3, 8192 x 32768 at 2700 rows 569 and 542, K 20480 the same.
 //
 // e4m3: the same bytes in the same places, so a stage is 128 of K. MFMA
 // 32x32x64 (four times a bf16 product's time, eight times its work), a lane
 // has two chunks of a row; scales are applied in the epilogue. 8192 rows, us
-// (PFLOP/s), the library's GEMM and this: 4096 x 12288 288 (2.86) and 271
-// (3.04), 24576 x 4096 636 (2.59) and 589 (2.80); where the library's tiles
-// leave the chip idle, 4099 rows, 4096 x 12288: 268 (1.54) and 153 (2.70).
+// (PFLOP/s), the library's GEMM and this: 4096 x 12288 281 (2.93) and 265
+// (3.12), 24576 x 4096 633 (2.60) and 574 (2.87); where the library's tiles
+// leave the chip idle, 4099 rows, 4096 x 12288: 270 (1.53) and 151 (2.73).
 //
 // SILU_MUL: the first half of a tile's W rows are gate rows and the second
 // the up rows that go with them; a wave holds both.
