@@ -31,7 +31,7 @@ int64_t decode_piece_floats(int, int, int, int);
 void launch_paged_attn_decode(u16*, const u16*, const void*, const void*,
                               const int*, const int*, int, int64_t, int, int,
                               int, int, float, bool, float*, hipStream_t);
-PrefillPlan plan_prefill_attn(int, int, int, int, int, int, int, bool);
+PrefillPlan plan_prefill_attn(int, int, int, int, int, int, bool);
 int64_t prefill_piece_floats(const PrefillPlan&, int);
 void launch_prefill_attn(u16*, const u16*, const void*, const void*,
                          const int*, const int*, const int*, const int*,
@@ -346,6 +346,22 @@ void paged_attention_decode(at::Tensor out, at::Tensor q, at::Tensor k_cache,
       pieces.data_ptr<float>(), current_stream());
 }
 
+// whether the kernel with two groups of queries per wave takes the operands
+bool prefill_pairs(int head_dim, bool paged, bool fp8) {
+  return paged && head_dim == 128 && !fp8;
+}
+
+// a call's choice: cut K/V ranges, two groups of queries per wave, parts
+std::tuple<bool, bool, int> prefill_plan(int tiles, int tile_rows,
+                                         int num_q_heads, int num_kv_heads,
+                                         int new_rows, int max_k_len,
+                                         int head_dim, bool paged, bool fp8) {
+  const fi::PrefillPlan pl = fi::plan_prefill_attn(
+      tiles, tile_rows, num_q_heads, num_kv_heads, new_rows, max_k_len,
+      prefill_pairs(head_dim, paged, fp8));
+  return {pl.split, pl.pair, pl.slots};
+}
+
 // room for the pieces of cut query tiles
 at::Tensor prefill_pieces(const fi::PrefillPlan& pl, const at::Tensor& q) {
   if (!pl.split) return at::Tensor();
@@ -375,7 +391,7 @@ void prefill_attention(at::Tensor out, at::Tensor q, at::Tensor k,
   v = dma_rows(v);
   const fi::PrefillPlan pl = fi::plan_prefill_attn(
       tile_seq.size(0), tile_rows, num_q_heads, num_kv_heads, q.size(0),
-      k.size(0), head_dim, false);
+      k.size(0), prefill_pairs(head_dim, false, false));
   at::Tensor pieces = prefill_pieces(pl, q);
   fi::launch_prefill_attn(
       bf16_ptr(out), bf16_cptr(q), bf16_cptr(k), bf16_cptr(v),
@@ -390,7 +406,7 @@ void prefill_attention_paged(at::Tensor out, at::Tensor q, at::Tensor k_cache,
                              at::Tensor v_cache, at::Tensor tile_seq,
                              at::Tensor tile_row0, at::Tensor cu_seqlens,
                              at::Tensor block_tables, at::Tensor seq_lens_k,
-                             double scale, int64_t tile_rows) {
+                             double scale, int64_t tile_rows, bool pairs) {
   TORCH_CHECK(tile_rows == 128 || tile_rows == 256,
               "tile_rows must be 128 or 256");
   CHECK_BF16_CUDA(out);
@@ -413,7 +429,7 @@ void prefill_attention_paged(at::Tensor out, at::Tensor q, at::Tensor k_cache,
   v_cache = dma_whole(v_cache);
   const fi::PrefillPlan pl = fi::plan_prefill_attn(
       tile_seq.size(0), tile_rows, num_q_heads, num_kv_heads, q.size(0),
-      block_tables.size(1) * 16, head_dim, fp8);
+      block_tables.size(1) * 16, pairs && prefill_pairs(head_dim, true, fp8));
   at::Tensor pieces = prefill_pieces(pl, q);
   fi::launch_prefill_attn(
       bf16_ptr(out), bf16_cptr(q), k_cache.data_ptr(), v_cache.data_ptr(),
@@ -604,5 +620,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "paged decode attention");
   m.def("prefill_attention", &prefill_attention, "varlen causal MFMA prefill");
   m.def("prefill_attention_paged", &prefill_attention_paged,
-        "varlen causal MFMA prefill over the paged cache (context attention)");
+        "varlen causal MFMA prefill over the paged cache (context attention)",
+        py::arg("out"), py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),
+        py::arg("tile_seq"), py::arg("tile_row0"), py::arg("cu_seqlens"),
+        py::arg("block_tables"), py::arg("seq_lens_k"), py::arg("scale"),
+        py::arg("tile_rows"), py::arg("pairs") = true);
+  m.def("prefill_plan", &prefill_plan,
+        "(split, two groups of queries per wave, parts) for tiles, tile_rows, "
+        "query heads, K/V heads, new rows, longest K/V range, head_dim, paged, "
+        "fp8");
 }

@@ -98,10 +98,11 @@ void prefill_attn_join_kernel(const PrefillArgs p) {
 // step by step: it is ahead from parts of 128 tiles on (8 query heads, 4 K/V
 // heads, 1024 rows behind 8192, parts of 17: 79 us, 94 with pairs; 32 and 8,
 // 700 + 33 + 1200 behind 6000, parts of 120: 240 and 250; 1000 behind 30000,
-// parts of 242: 519 and 489).
+// parts of 242: 519 and 489). `pairs`: whether that kernel takes the operands,
+// bf16 rows of 128 in a paged cache.
 PrefillPlan plan_prefill_attn(int ntiles, int tile_rows, int num_q_heads,
                               int num_kv_heads, int new_rows, int max_k_len,
-                              int head_dim, bool fp8) {
+                              bool pairs) {
   const int group = num_q_heads / num_kv_heads;
   auto layout = [&](bool split) {
     PrefillPlan pl;
@@ -120,7 +121,7 @@ PrefillPlan plan_prefill_attn(int ntiles, int tile_rows, int num_q_heads,
                          (num_q_heads / pl.hpb);
   const int64_t tiles = ceil_div(max_k_len, kKVTile);
   const double fill = blocks / 256.0;
-  pl.pair = head_dim == 128 && !fp8 && fill * tiles >= 128;
+  pl.pair = pairs && fill * tiles >= 128;
   const double idle = fill < 1.0 ? 1.0 - std::min(1.0, 1.4 * fill)
                                  : std::ceil(fill) -
                                        (pl.pair ? 0.96 : 1.04) * fill;
@@ -184,7 +185,7 @@ void launch_prefill_attn(u16* out, const u16* q, const void* k, const void* v,
 #define FI_PF_LAUNCH(DD, PP, F8)                                              \
   do {                                                                        \
     if (pl.split) {                                                           \
-      if (PP && pl.pair)                                                      \
+      if (DD == 128 && PP && !F8 && pl.pair)                                  \
         hipLaunchKernelGGL((prefill_pair_kernel<4>), dim3(pl.slots),          \
                            dim3(4 * kWaveSize), 0, stream, a);                \
       else                                                                    \

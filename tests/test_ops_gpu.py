@@ -497,7 +497,8 @@ def test_prefill_attention_long_parts(hq, hk, scale_by):
     """Parts of more than 128 K/V tiles (two groups of queries per wave):
     odd rows, a portion of 33 and one whose end lies within a tile, maxima
     that jump late, against float64. Bound: P and the output are rounded to
-    bf16 (2^-9 each) and |v| stays below 6, hence 2.4e-2."""
+    bf16 (2^-9 each) and |v| stays below 6, hence 2.4e-2. One group per wave
+    over the same parts gives the same bits."""
     g = torch.Generator().manual_seed(hq + hk)
     new_lens, ctx_lens, D = [901, 33], [9001, 8064], 128
     need = [-(-c // 16) for c in ctx_lens]
@@ -518,6 +519,16 @@ def test_prefill_attention_long_parts(hq, hk, scale_by):
     lens = torch.tensor(ctx_lens, dtype=torch.int32, device=DEV)
     scale = scale_by / math.sqrt(D)
     out = ops.prefill_attention_paged(q, kc, vc, bt.to(DEV), cu, lens, scale)
+    tile_rows = ops.prefill_tile_rows(new_lens)
+    tiles = ops.build_prefill_tiles(new_lens, device=DEV, rows=tile_rows)
+    plan = (tiles[0].shape[0], tile_rows, hq, hk, len(q), bt.shape[1] * 16, D,
+            True)
+    assert ops._C.prefill_plan(*plan, False)[:2] == (True, True)
+    assert ops._C.prefill_plan(*plan, True)[:2] == (True, False)
+    alone = torch.empty_like(out)
+    ops._C.prefill_attention_paged(alone, q, kc, vc, *tiles, cu, bt.to(DEV),
+                                   lens, scale, tile_rows, pairs=False)
+    assert torch.equal(out, alone)
     at = 0
     for i, (n, c) in enumerate(zip(new_lens, ctx_lens)):
         rows = bt[i, :need[i]].long().to(DEV)
