@@ -1184,6 +1184,9 @@ def test_linear_in_parts(rows, n, k, bias):
     (4128, 1024, True),     # cut tiles, a ragged last one
     (288, 16384, False),    # 16 pieces, every other tile begins half way
     (65568, 128, False),    # whole rounds of tiles and a rest
+    (65568, 128, True),
+    (33056, 1024, False),   # whole rounds, the rest cut (257, 1029 rows)
+    (33056, 1024, True),
 ])
 def test_linear_by_tiles(rows, n, k, bias):
     """Tiles of 256 x 256 against a float64 product; one bf16 rounding of the
@@ -1235,6 +1238,38 @@ def test_linear_by_tiles_reads_its_operands_alone(rows, n, k):
             <= want.abs() * 2 ** -8 + 1e-4 * k ** 0.5).all()
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+def test_linear_by_tiles_carries_what_is_not_finite(fp8):
+    """An infinity or NaN reaches its row or column as in float64, and no
+    other; across a tile's border too."""
+    rows, n, k = 300, 528, 512
+    g = torch.Generator().manual_seed(k)
+    x = torch.randn(rows, k, generator=g)
+    w = torch.randn(n, k, generator=g)
+    x[7, 3], x[299, 511] = float("nan"), float("nan")
+    w[255, 5], w[520, 0] = float("nan"), float("nan")
+    if fp8:
+        f8 = torch.float8_e4m3fn
+        x, w = x.to(f8).to(DEV), w.to(f8).to(DEV)
+        xs, ws = torch.ones(rows, device=DEV), torch.ones(n, device=DEV)
+        xs[100], ws[300] = float("inf"), float("inf")
+        out = torch.empty(rows, n, dtype=torch.bfloat16, device=DEV)
+        ops._C.many_rows_gemm_fp8(out, x, xs, w, ws)
+        want = (x.double() @ w.double().T) * xs.double()[:, None] * ws.double()
+    else:
+        x[100, 0], w[300, 7] = float("inf"), float("-inf")
+        x, w = x.bfloat16().to(DEV), w.bfloat16().to(DEV)
+        out = torch.empty(rows, n, dtype=torch.bfloat16, device=DEV)
+        ops._C.many_rows_gemm(out, x, w, None, False)
+        want = x.double() @ w.double().T
+    assert torch.equal(out.isnan(), want.isnan())
+    assert torch.equal(out.isposinf(), want.isposinf())
+    assert torch.equal(out.isneginf(), want.isneginf())
+    err = (out.double() - want).abs()[want.isfinite()]
+    assert (err <= want[want.isfinite()].abs() * 2 ** -8
+            + 3e-4 * k ** 0.5).all()
+
+
 def test_silu_by_tiles_of_far_gates():
     """Gates down to where 1 + exp(-gate) leaves fp32, infinite ones and NaN,
     against float64: exp of fp32 is off by |gate| 2^-23, the result has one
@@ -1275,9 +1310,11 @@ def test_linear_takes_tiles():
     assert ((ops.linear(x, w).double() - want).abs()
             <= want.abs() * 2 ** -8 + 1e-4 * 12288 ** 0.5).all()
     x, w = x[:, :4096], w[:, :4096].contiguous()
-    for other in (x[:, 1:129], x.T, x.float(), x[:256]):
+    for other in (x[:, 1:129], x.float(), x[:256]):
         assert not ops._tiles_ok(other, w[:, :other.shape[1]].contiguous(), 16)
     assert ops._tiles_ok(x, w, 16) and not ops._tiles_ok(x, w.T, 16)
+    square = x[:4096].contiguous()
+    assert ops._tiles_ok(square, w, 16) and not ops._tiles_ok(square.T, w, 16)
     with torch.enable_grad():
         assert not ops._tiles_ok(x, w.clone().requires_grad_(), 16)
 
@@ -1329,6 +1366,7 @@ def test_linear_fp8_in_parts(rows, n, k):
     (4128, 2048),        # cut tiles, a ragged last one
     (288, 32768),        # 16 pieces, every other tile begins half way
     (65568, 256),        # whole rounds of tiles and a rest
+    (33056, 2048),       # whole rounds, the rest cut (257, 1029 rows)
 ])
 def test_linear_fp8_by_tiles(rows, n, k):
     """e4m3 tiles of 256 x 256 against a float64 product: one bf16 rounding of
@@ -1531,6 +1569,8 @@ def test_moe_gemm_row_blocks_of_128(k, n, gate_up, act):
     (7744, True, "clamped_glu"),  # two rounds
     (5760, False, "relu_sq"),
     (5760, False, None),
+    (7744, True, None),
+    (15488, False, "relu_sq"),
     (15488, False, None),
 ])
 def test_moe_gemm_wide_tiles(k, n, gate_up, act):
@@ -1539,6 +1579,42 @@ def test_moe_gemm_wide_tiles(k, n, gate_up, act):
     assert ops._moe_native().moe_gemm_wide(18, 7, k, n, mode)
     assert not ops._moe_native().moe_gemm_wide(18, 7, k + 32, n, mode)
     check_moe_gemm(k, n, gate_up, act, 128)
+
+
+@pytest.mark.parametrize("n,gate_up,act", [
+    (2880, True, None), (5760, False, "relu_sq"), (5760, False, None)])
+def test_moe_gemm_wide_tiles_carry_what_is_not_finite(n, gate_up, act):
+    """A row's infinity or NaN stays in the row, an expert's in the expert's
+    column."""
+    g = torch.Generator().manual_seed(n)
+    experts, k, T = 7, 128, 2000
+    mode = 1 if gate_up else 2 if act else 0
+    x = torch.randn(T, k, generator=g)
+    w = torch.randn(experts, k, 2 * n if gate_up else n, generator=g)
+    x[5, 1], x[700, 0], x[1999, 127] = (float(v) for v in ("nan", "inf",
+                                                           "-inf"))
+    w[2, 9, n - 1] = float("nan")
+    topi = (torch.arange(T) % experts).int()[:, None].to(DEV)
+    sid, eid, nv, pos, PM = ops.moe_align(topi, 0, experts, 128)
+    assert ops._moe_native().moe_gemm_wide(PM // 128, experts, k, n, mode)
+    x, w = x.bfloat16().to(DEV), w.bfloat16().to(DEV)
+    ids = sid.long()
+    gathered = torch.where((ids < T)[:, None], x[ids.clamp(max=T - 1)], 0)
+    out = torch.empty(PM, n, dtype=torch.bfloat16, device=DEV)
+    ops.moe_gemm(out, x if mode else gathered, ops.pack_moe_weights(w), sid,
+                 eid, nv, 128, gate_up, act, 3.0)
+    for m in range(int(nv)):
+        at = slice(m * 128, (m + 1) * 128)
+        live = ids[at] < T
+        y = gathered[at][live].double() @ w[int(eid[m])].double()
+        if gate_up:
+            y = torch.nn.functional.silu(y[:, :n]) * y[:, n:]
+        elif act:
+            # (the kernel's maximum takes the number that is none for zero)
+            y = torch.where(y.isnan(), 0, y).clamp(min=0).square()
+        got = out[at][live].double()
+        assert torch.equal(got.isnan(), y.isnan()), m
+        assert torch.equal(got.isinf(), y.isinf()), m
 
 
 def test_moe_gemm_wide_tiles_are_the_narrow_ones():
