@@ -35,6 +35,7 @@
 #include <utility>
 
 #include "prefill_kernel.h"
+#include "tile_engine.h"
 
 namespace fi {
 
@@ -44,12 +45,7 @@ FI_DEV void each_place(F&& f, std::integer_sequence<int, I...>) {
   (f(std::integral_constant<int, I>{}), ...);
 }
 
-FI_DEV void pair_m0(u32 lds) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("s_mov_b32 m0, %0" ::"s"(lds) : "memory");
-#endif
-}
-// 16 bytes per lane to LDS at m0 + 16 lane; pair_m0 lies at least one
+// 16 bytes per lane to LDS at m0 + 16 lane; set_m0 lies at least one
 // instruction ahead
 FI_DEV void pair_load(const void* base, u32 offset) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -63,7 +59,7 @@ FI_DEV void pair_load(const void* base, u32 offset) {
 // registers; O += V^T P: results in accumulation registers. In asm, so that
 // each has one place (from the builtins the compiler moves a third of them
 // back and forth). The wait states between a product and other instructions
-// on its registers are kept by distance, or by settle_pair().
+// on its registers are kept by distance, or by settle().
 FI_DEV void qk_first(floatx16& s, const short8& k, const short8& q) {
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0"
@@ -85,13 +81,6 @@ FI_DEV void pv(floatx16& o, const short8& v, const short8& w) {
                : "v"(v), "v"(w));
 #endif
 }
-FI_DEV float result_of(float a) {
-  float v = a;
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(a));
-#endif
-  return v;
-}
 FI_DEV void clear_result(float& a) {
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("v_accvgpr_write_b32 %0, 0" : "=a"(a));
@@ -112,10 +101,6 @@ FI_DEV floatx2 move(floatx2 from) {
   asm volatile("v_mov_b64 %0, %1" : "=v"(to) : "v"(from));
 #endif
   return to;
-}
-FI_DEV void settle_pair() {
-  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
 }
 FI_DEV void pin() { __builtin_amdgcn_sched_barrier(0); }
 
@@ -225,7 +210,7 @@ void prefill_pair_kernel(const PrefillArgs p) {
       limit = t.k_len - 1 - min(min(tile, tb - 1) * 4 + wave, last_blk) * 16;
     };
     auto m0_of = [&](int i) {
-      pair_m0(dst + (i & 1) * kBufs * kTileB + (i >> 1) * 1024);
+      set_m0(dst + (i & 1) * kBufs * kTileB + (i >> 1) * 1024);
     };
     auto load_of = [&](int i) {
       const int r = (i >> 1) * 4 + lane / kChunk;  // row of the wave
@@ -460,7 +445,7 @@ void prefill_pair_kernel(const PrefillArgs p) {
       asm volatile("" ::: "memory");
       aim(tile + kBufs - 1, __builtin_amdgcn_readfirstlane(ids), sbuf);
       stage_all();
-      settle_pair();
+      settle();
 #pragma unroll
       for (int g = 0; g < kGroups; ++g) {
         const int r0 = row0 + g * 32;
@@ -488,7 +473,7 @@ void prefill_pair_kernel(const PrefillArgs p) {
             w.h[j] = f32_to_bf16(e);
           }
           const short8 wk = __builtin_bit_cast(short8, w);
-          settle_pair();
+          settle();
 #pragma unroll
           for (int cb = 0; cb < CB; ++cb)
             pv(o_acc[g][cb], read_v(vbuf, kc * 4 + cb), wk);
@@ -532,7 +517,7 @@ void prefill_pair_kernel(const PrefillArgs p) {
     }
 
     // ---- epilogue ----
-    settle_pair();
+    settle();
     const bool whole = ta == 0 && tb == t.work;
     const int piece = slot * 2 + (ta > 0 ? 0 : 1);
 #pragma unroll
@@ -551,7 +536,7 @@ void prefill_pair_kernel(const PrefillArgs p) {
               bf16x4 w;
 #pragma unroll
               for (int j = 0; j < 4; ++j)
-                w.h[j] = f32_to_bf16(result_of(o_acc[g][cb][r + j]) * inv);
+                w.h[j] = f32_to_bf16(acc_of(o_acc[g][cb][r + j]) * inv);
               *reinterpret_cast<bf16x4*>(orow + cb * 32 + crow(r, hi1)) = w;
             }
         }
@@ -563,7 +548,7 @@ void prefill_pair_kernel(const PrefillArgs p) {
         for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
           for (int r = 0; r < 16; ++r)
-            o[(cb * 16 + r) * 64] = result_of(o_acc[g][cb][r]);
+            o[(cb * 16 + r) * 64] = acc_of(o_acc[g][cb][r]);
         reinterpret_cast<float2*>(p.piece_ml)[at * 64 + lane] =
             make_float2(m_row[g], l_row[g]);
       }
