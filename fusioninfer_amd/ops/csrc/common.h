@@ -1,8 +1,8 @@
 // Common device helpers for FusionInfer-AMD CDNA4 (gfx950) kernels.
 //
-// Design notes (see /opt/skills/guides/cdna_hip_programming.md):
+// Design notes:
 //  * wave64 everywhere; block sizes are multiples of 64.
-//  * bf16 loads are ALWAYS vectorized (short4/short8 reinterpret, G13).
+//  * bf16 loads are ALWAYS vectorized (short4/short8 reinterpret).
 //  * bf16<->f32 via bit ops (RNE) — matches hardware v_cvt rounding.
 #pragma once
 

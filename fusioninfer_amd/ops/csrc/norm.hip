@@ -13,9 +13,9 @@
 // takes of the registers costs workgroups in flight. us a call, the weight and
 // the residual in the plain order and this (residual added, bf16 out): 4096
 // wide, 1 row 2.6 and 2.3, 64 rows 2.9 and 2.5, 1024 7.2 and 7.1, 4099 22.2
-// and 22.1; 16384 wide, 1 row 5.2 and 3.9, 64 rows 6.6 and 5.3. (Back to back
-// on a quiet card; in a decode step of 8 layers, 900 us, the difference is
-// within what two runs differ by.)
+// and 22.1; 16384 wide, 1 row 5.2 and 3.9, 64 rows 6.6 and 5.3. A step of eight
+// layers, with sums by exchanges among registers and rope's cache slot requested
+// early: 897 and 890 us at one row, 1723 and 1708 at six with long contexts.
 
 #include "common.h"
 

@@ -24,10 +24,12 @@
 // prefill_attn_kernel, bit for bit.
 //
 // Measured, us, eight waves of one group and this (32 query heads, 8 K/V
-// heads): 4099 rows behind 16384 1253 -> 1162 (1.06 PFLOP/s), 6000 behind
-// 14000 1717 -> 1563, 1000 behind 30000 529 -> 494. Matrix cores busy 56 % of
-// the time at the 2.05 GHz that the card holds here; vector instructions
-// issue for 53 %, waits take 19 %.
+// heads), repeated alone: 4099 rows behind 16384 1231 -> 1132 (1.09 PFLOP/s),
+// 6000 behind 14000 1651 -> 1534, 1000 behind 30000 520 -> 484; behind an idle
+// card, or between the linear layers of a step, at a lower clock, 4099 rows take
+// 1210 to 1320. Matrix cores busy 56 % of the time at 2.05 GHz; vector
+// instructions issue for 53 %, waits take 19 %. (Twelve registers are spilled,
+// outside the overlapped form.)
 
 #pragma once
 

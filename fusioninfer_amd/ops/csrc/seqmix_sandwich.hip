@@ -33,7 +33,8 @@ __global__ __launch_bounds__(256) void norm_residual_norm_kernel(
   if constexpr (NCH > 0) {
     // few rows take the time of one chain: both weights are requested with
     // the row, the stream is written behind the sums (a barrier waits for
-    // what has been stored)
+    // what has been stored). Before and so, us: 2048 wide, 1 row 3.1 and 2.5,
+    // 4099 rows 17.7 and 15.9; 8192 wide 5.6 and 4.4, 89 and 84.5.
     float v[NCH][4], r[NCH][4], wp[NCH][4], wn[NCH][4];
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
