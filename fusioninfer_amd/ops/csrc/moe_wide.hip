@@ -199,7 +199,9 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
   }
   u32 buf = 0;
   constexpr int kCols = GATE_UP ? 64 : 128;   // of a wave
-  constexpr int kStores = kCols / 4;          // of a tile
+  // of a tile, at least: 16 bytes are one instruction or more, and a wait that
+  // counts too few is only longer
+  constexpr int kStores = kCols / 4;
   constexpr int kFree = 40, kEarly = 6;  // MFMAs up to the first barrier, DMAs
                                          // between the two
   // `behind`: stores that follow the DMAs that are waited for

@@ -325,7 +325,9 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
   int buf = 0;
   constexpr int kFree = 40, kEarly = 6;  // MFMAs up to the first barrier, DMAs
                                          // between the two
-  constexpr int kStores = SILU_MUL ? 16 : 32;  // of a whole tile
+  // of a whole tile, at least: 16 bytes are one instruction or more, and a
+  // wait that counts too few is only longer
+  constexpr int kStores = SILU_MUL ? 16 : 32;
   // `behind`: that many follow the DMAs that are waited for
   auto stage = [&](auto first, bool behind) {
 #pragma unroll
