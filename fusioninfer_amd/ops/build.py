@@ -1,7 +1,7 @@
 """In-tree build of the CDNA4 HIP extension (gfx950 only, no hipify).
 
 Drives hipcc directly — no CUDA compatibility layer, no JIT cache: the
-resulting ``_C.so`` lives next to this file so the gpurun snapshot carries it.
+resulting ``_C.so`` lives next to this file so a copy of the tree carries it.
 
 Three extensions, so that a model family compiles only what it runs:
 
