@@ -89,31 +89,28 @@ def _streams(M: int, N: int, K: int, silu_mul: bool = False) -> bool:
     and 4 us, above them 4 us and W at 4 TB/s or, where N gives it few tiles,
     the chain of 7 us per 1000 of K; with silu_mul 3 us more for the pass
     over the product. (Where that errs most: 14336 x 5120 at 64 rows streams
-    in 38.2 us, the library takes 32.4.)
+    in 38 us, the library takes 32.)
 
-    From 129 rows on both compute more than they read and the library's
-    choice of tiles jumps with M. The streaming kernel is ahead where N is
-    small (6144 x 4096 at 129 / 256 rows 28.1 / 30.1 us, the library 39.4 /
-    40.0; 2048 x 12288 27.9 / 30.2 and 39.0 / 39.9), from 192 rows on until
-    half the chip's 256 tiles of 96 rows are taken (12288 x 4096 at 129 / 256
-    41.7 / 44.1 and 38.3 / 49.5; 16384 x 5120 at 256 71 and 65), and behind
-    for less than 5 * 2^22 values of W (4096 x 4096 at 256 23.6 and 22.5).
-    With silu_mul it is ahead until all 256 are (24576 x 4096 at 256 62 and
-    69, 28672 x 4096 90 and 75).
+    From 129 rows on both compute more than they read. The library's choice
+    of tiles jumps with M and N there, and streaming is ahead but for few
+    values of W (2048 x 4096 at 192 rows 20.2 us, the library 16.1; 3072 x
+    5120 24.8 and 41.6; 4096 x 4096 at 256 24.2 and 22.0; 6144 x 4096 29 and
+    40), short rows (49152 x 1024 at 256 40 and 31) and N at which the
+    library's tiles fill the chip exactly (49152 x 4096 at 256 125 and 107).
 
-    Weights that no cache holds (4 GB of them in turn), 24 N of 2048 to
-    151936, eight K of 512 to 12288, ten M of 17 to 256: this choice takes
-    1.5 % longer than the better of the two on average (silu_mul 1.6 %), the
-    library alone 14 (25), streaming alone 5 (3)."""
+    Weights that no cache holds, launched from a graph, 15 N of 2048 to
+    151936, eight K of 512 to 12288: this choice takes 0.8 to 2.1 % longer
+    than the better of the two up to 128 rows, 1.9 to 3.1 % at 160 to 256;
+    the library alone 11 to 27, streaming alone 0.4 to 4. With silu_mul 0.2
+    to 1.7 %, the library alone 14 to 29."""
     if M <= SKINNY_ROWS:
         return True
     if M > PART_ROWS or N * K < 1 << 23 or K < 2048 and N <= 8192:
         return False
     if M > 128:
         if silu_mul:
-            return N <= 96 * 256
-        return N * K >= 5 << 22 and (N <= 6144
-                                     or M >= 192 and N <= 96 * 128)
+            return K >= 2048 or N <= 96 * 256
+        return K >= 2048 and N * K >= (3 << 22 if M <= 192 else 5 << 22)
     library = 4 + (2 * N * K / 2.5e6 if M <= 64
                    else max(2 * N * K / 4e6, 7e-3 * K))
     return _C.few_rows_gemm_us(M, N, K) < library + (3 if silu_mul else 0)
@@ -242,18 +239,18 @@ def linear(x: torch.Tensor, w: torch.Tensor,
 
 
 def _streams_fp8(M: int, N: int, K: int) -> bool:
-    """As _streams, for e4m3 operands with scales per row. Up to 16 rows the
-    library is behind at nearly all sizes (8192 x 8192 at 9 rows 43 us, 20
-    here); up to 64 rows it takes W at 4.5 TB/s and 5 us or 2 us per 1000 of
-    K (6144 x 4096 at 64 13.1 and 14.5, 4096 x 12288 23.7 and 19.6). From 65
-    rows on it is ahead but for long K and few tiles (4096 x 12288 at 65, 96,
-    128 rows 20.6, 29.8, 35.8 and 23.5, 24.9, 25.9; 2048 x 12288 at 128 17.6
-    and 18.8). Over the same N and K and eleven M of 1 to 128 this choice
-    takes 1.9 % longer than the better of the two on average, the library
-    alone 22, streaming alone 5."""
+    """As _streams, for e4m3 operands with scales per row. Up to 32 rows the
+    library is behind at nearly all sizes (24576 x 4096 at 32 rows 24 us, 20
+    here; 8192 x 8192 20 and 24.8); up to 64 rows it takes W at 4.5 TB/s and 5
+    us or 2 us per 1000 of K (6144 x 4096 at 64 13.1 and 15, 4096 x 12288 23.5
+    and 19.7). From 65 rows on it is ahead but for long K and few tiles (4096
+    x 12288 at 96 and 128 rows 20 and 27, here 17 and 20). Ten N and six K,
+    launched from a graph: this choice takes 0.7 to 2.7 % longer than the
+    better of the two up to 64 rows (the library alone 8 to 32, streaming
+    alone 0.7 to 3.1), 0.2 % at 96 and 128."""
     if M > 128 or N * K < 1 << 23:
         return False
-    if M <= SKINNY_ROWS:
+    if M <= 32:
         return True
     if M > 64:
         return M >= 96 and K >= 2 * N and N >= 3072

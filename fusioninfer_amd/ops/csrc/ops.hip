@@ -40,7 +40,7 @@ void launch_prefill_attn(u16*, const u16*, const void*, const void*,
                          hipStream_t);
 void launch_skinny_gemm(u16*, const u16*, const u16*, const u16*, int, int,
                         int, int64_t, int64_t, bool, hipStream_t);
-int64_t part_gemm_floats(int, int, int);
+int64_t part_gemm_floats(int, int, int, bool);
 double part_gemm_us(int, int, int);
 void launch_part_gemm(u16*, float*, const u16*, const u16*, const u16*, int,
                       int, int, int64_t, int64_t, bool, hipStream_t);
@@ -473,7 +473,7 @@ void few_rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
                            current_stream());
     return;
   }
-  at::Tensor pieces = at::empty({fi::part_gemm_floats(M, N, K)},
+  at::Tensor pieces = at::empty({fi::part_gemm_floats(M, N, K, false)},
                                 x.options().dtype(at::kFloat));
   fi::launch_part_gemm(bf16_ptr(out), pieces.data_ptr<float>(), bf16_cptr(x),
                        bf16_cptr(w), b, M, N, K, x.stride(0), out.stride(0),
@@ -538,7 +538,7 @@ void few_rows_gemm_fp8(at::Tensor out, at::Tensor x, at::Tensor x_scales,
               x_scales.is_contiguous() && x_scales.numel() == M &&
               w_scales.is_cuda() && w_scales.scalar_type() == at::kFloat &&
               w_scales.is_contiguous() && w_scales.numel() == N);
-  at::Tensor pieces = at::empty({fi::part_gemm_floats(M, N, K / 2)},
+  at::Tensor pieces = at::empty({fi::part_gemm_floats(M, N, K / 2, true)},
                                 x.options().dtype(at::kFloat));
   fi::launch_part_gemm_fp8(
       bf16_ptr(out), pieces.data_ptr<float>(),

@@ -17,28 +17,39 @@
 // outputs of one row of x. SILU_MUL: the first half of a tile's rows are gate
 // rows and the second the up rows that go with them; a wave holds both.
 //
-// What L2 delivers to the CUs, W and x together, ends at about 10 TB/s (x
-// requests of 16 KB per CU in flight or 64 made no difference, nor did other
-// row strides of x); hence tiles at least as tall as x has rows, taller where
-// N allows. The second kernel of a cut product costs 4.7 us at the least.
-// Measured, us (GB/s of W) at 32 / 64 / 128 / 256 rows: N 24576, K 4096 with
-// silu 31.4 (6410) / 34.5 / 44.6 / 64, the library's GEMM and the pass
-// behind it 48 / 51 / 55 / 67; 4096, 12288 21 (4700) / 26 / 33 / 45 against
-// 26 / 37 / 66 / 53; 151936, 4096 211 (5880) / 238 / 266 / 391 against 264 /
-// 262 / 279 / 350.
+// What bounds it, from DMAs alone without products: a CU has at most some 41
+// KB on the way and gets its data in the order asked for, so x, which comes
+// from L2, waits behind W, which comes from HBM; both together arrive at 55 to
+// 60 KB/us per CU (x alone at 130, W alone at 26, which is what HBM gives to 256
+// CUs), whatever the depth of the rings. Hence tiles at least as tall as x has
+// rows, taller where N allows. The second kernel of a cut product costs 4.7 us
+// at the least, and results leave by stores that the next stages' waits count
+// (151936 x 4096 at 64 rows 243 us, and 249).
 //
-// FP8: the same kernel on e4m3 rows, 1 to 128 of them. 24576 x 4096 at 1 / 32
-// / 64 rows 20.0 (5040) / 19.3 / 24.3 us, the library's GEMM 30.8 / 24.4 /
-// 25.9; 4096 x 12288 14.2 (3550) / 14.5 / 19.4 against 21.1 / 20.5 / 24.1.
+// From 129 rows on the fragment reads would be the bound, a wave of 32 x 64
+// results reading as much as it multiplies: there four waves hold a tile's rows
+// of W by a quarter of x (part_gemm_ahead_kernel), read the fragments of half a
+// stage during the products of the other half, and cross one barrier a stage.
+// Before and now at 192 rows: 24576 x 4096 with silu 57 and 50 us, 4096 x 12288
+// 43 and 38, 8192 x 8192 55 and 42; at 256 63 and 59, 45 and 43.5, 56 and 49;
+// 151936 x 4096 at 256 446 and 345, the library 358.
+//
+// Measured, us (GB/s of W) at 32 / 64 / 128 / 256 rows: N 24576, K 4096 with
+// silu 32.4 (6210) / 33.8 / 44.2 / 59, the library's GEMM and the pass behind it
+// 49 / 49 / 53 / 69; 4096, 12288 23 (4380) / 26 / 33 / 44 against 27 / 37 / 67 /
+// 55; 151936, 2048 109 (5710) / 128 / 153 / 188 against 145 / 150 / 166 / 212.
+//
+// FP8: the same kernel on e4m3 rows, 1 to 128 of them. 24576 x 4096 at 16 / 32
+// / 64 rows 19.8 (5090) / 19.9 / 23.5 us, the library's GEMM 30.1 / 25.7 /
+// 26.7; 4096 x 12288 15.0 (3350) / 15.8 / 19.7 against 19.3 / 20.5 / 24.4.
 
-#include "common.h"
+#include <type_traits>
+
+#include "tile_engine.h"
 
 namespace fi {
 
 namespace {
-
-typedef __attribute__((ext_vector_type(8))) short short8;
-typedef __attribute__((ext_vector_type(4))) float floatx4;
 
 template <int N>
 FI_DEV void wait_vm() {
@@ -85,11 +96,18 @@ struct PartShape {
   static constexpr int LW = TN / kRowsPerDma / kWLoaders;
   static constexpr int LX = MB / kRowsPerDma / kXLoaders;
   static constexpr int kPiece = TN * MB / 4;  // float4
+  static constexpr bool kAhead = false;
   static_assert(RF % 2 == 0 && TN / 2 % kRowsPerDma == 0);
   static_assert(LW * kRowsPerDma * kWLoaders == TN &&
                 LX * kRowsPerDma * kXLoaders == MB);
   static_assert(RW * kWB + RX * kXB <= 160 * 1024 && RW >= 2 && RW <= 7 &&
                 RX >= 2 && RX <= 7);
+};
+
+// the same for part_gemm_ahead_kernel: four waves of RF x CF fragments
+template <int RF, int CF, int RW, int RX>
+struct AheadShape : PartShape<1, RF, 4, CF, 64, RW, RX, 2> {
+  static constexpr bool kAhead = true;
 };
 
 // fragment of W rows (of the tile) that wave column wn holds as its rf-th
@@ -244,7 +262,9 @@ void part_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
     fr[kk] = frow * S::kRowB +
              (((kk * 4 + (lane >> 4)) ^ frow) & (S::kChunks - 1)) * 16;
 
-  int wslot = 0, xslot = 0, pos = lo;
+  // results on their way out are behind the DMAs that the next stages wait for
+  constexpr int kStores = (SILU_MUL ? RF / 2 : RF) * CF;
+  int wslot = 0, xslot = 0, pos = lo, behind = 0;
   while (pos < hi) {
     const int tile = pos / SK;
     const int begin = tile * SK, end = begin + SK;
@@ -258,10 +278,18 @@ void part_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
     for (; pos < stop; ++pos) {
       // this wave's share of the stage has landed; after the barrier all
       // shares have, and every wave is done with the slot read last
-      if (loads_w)
-        wait_stages<LW, S::RW - 2>(issued - pos - 1);
-      else
-        wait_stages<LX, S::RX - 2>(issued - pos - 1);
+      if (loads_w) {
+        if (behind > 0 && issued - pos > S::RW - 2)
+          wait_vm<(S::RW - 2) * LW + kStores>();
+        else
+          wait_stages<LW, S::RW - 2>(issued - pos - 1);
+      } else {
+        if (behind > 0 && issued - pos > S::RX - 2)
+          wait_vm<(S::RX - 2) * LX + kStores>();
+        else
+          wait_stages<LX, S::RX - 2>(issued - pos - 1);
+      }
+      --behind;
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
@@ -315,6 +343,12 @@ void part_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
                                   out_stride);
         }
       }
+      // stage pos + RW - 2 has been requested before the stores
+      behind = 0;
+      if ((wm * CF + CF - 1) * 16 < M &&
+          (tile + 1) * (SILU_MUL ? S::TN / 2 : S::TN) <=
+              (SILU_MUL ? N / 2 : N))
+        behind = (loads_w ? S::RW : S::RX) - 1;
     } else {
       // a part holds at most two pieces: the end of a tile that an earlier
       // part began (0) and the start of one that goes on (1)
@@ -326,8 +360,257 @@ void part_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
 #pragma unroll
         for (int c = 0; c < CF; ++c)
           p[(f * CF + c) * kWaveSize] = acc[f][c];
+      behind = (loads_w ? S::RW : S::RX) - 1;
     }
   }
+}
+
+// Four waves that read ahead, each a tile's rows of W by a quarter of x; two
+// load W, two x (LOADS_W). Each MFMA is followed by at most one read or DMA, in
+// an order that is pinned: one wave per SIMD hides nothing by itself. While the
+// first half of a stage (32 of K) is multiplied the fragments of the second are
+// read; with them in registers, and the next stage landed, the barrier frees the
+// stage's place, and the second half's products cover the reads of the next
+// stage's first half and half of the DMAs into the free place.
+template <class S, bool SILU_MUL, bool LOADS_W>
+FI_DEV void run_ahead(u16* __restrict__ out, floatx4* __restrict__ pieces,
+                      const u16* __restrict__ x, const u16* __restrict__ w,
+                      const u16* __restrict__ bias, const int M, const int N,
+                      const int K, const int64_t x_stride,
+                      const int64_t out_stride, const int tiles,
+                      const int unit, unsigned char* smem, const int wave,
+                      const int lane) {
+  constexpr int RF = S::RF, CF = S::CF;
+  constexpr int R = LOADS_W ? S::RW : S::RX, L = LOADS_W ? S::LW : S::LX;
+  constexpr int kLoaders = LOADS_W ? S::kWLoaders : S::kXLoaders;
+  constexpr int kSlotB = LOADS_W ? S::kWB : S::kXB;
+  const int SK = K / S::KS;
+  const Cut cut(tiles * SK / unit, gridDim.x, unit);
+  const int lo = cut.start(blockIdx.x), hi = cut.start(blockIdx.x + 1);
+  const int lwave = LOADS_W ? wave : wave - S::kWLoaders;
+
+  // ---- requests: DMA j of a wave brings eight rows, group kLoaders j + lwave;
+  // lane l chunk (l % 8) ^ key of one of them. The row is in the vector
+  // offset, the place along K in the scalar one; rows past the descriptor's
+  // end come as zeros.
+  const u32 ring = static_cast<u32>(reinterpret_cast<uintptr_t>(
+                       (__attribute__((address_space(3))) unsigned char*)
+                           smem)) +
+                   (LOADS_W ? 0 : S::RW * S::kWB) + lwave * 1024;
+  const u32 row_b = LOADS_W ? K * 2 : static_cast<u32>(x_stride) * 2;
+  u32 voff[L];
+#pragma unroll
+  for (int j = 0; j < L; ++j) {
+    const int half = LOADS_W && SILU_MUL ? L / 2 : L;
+    const int g = j * kLoaders + lwave;
+    const int r = (j % half * kLoaders + lwave) * 8 + (lane >> 3);
+    voff[j] = (LOADS_W ? r : min(r, M - 1)) * row_b +
+              (((lane & 7) ^ ((lane >> 4) | ((g & 1) << 2))) << 4);
+  }
+  u32x4 d0{}, d1{};
+  u32 soff = 0;
+  int rt = lo / SK, issued = lo, rs = 0, ra = 0, rb = 0, left = 0;
+  constexpr int kPast = 1 << 30;
+  auto seek = [&] { soff = left > kPast / 2 ? 0 : rs * S::kRowB; };
+  auto enter = [&] {
+    if (issued >= hi) {           // past the end nothing is read
+      d0[2] = d1[2] = 0;
+      left = kPast;
+      return;
+    }
+    ra = max(lo - rt * SK, 0);
+    rb = max(min(hi - rt * SK, SK), ra + 1);
+    rs = ra + static_cast<int>(blockIdx.x / 8) % (rb - ra);
+    left = rb - ra;
+    if (LOADS_W) {
+      const int n0 = rt * (SILU_MUL ? S::TN / 2 : S::TN);
+      const int cols = SILU_MUL ? N / 2 : N;
+      const u32 bytes = min(SILU_MUL ? S::TN / 2 : S::TN, cols - n0) * row_b;
+      d0 = uniform_descriptor(w + static_cast<int64_t>(n0) * K, bytes);
+      if (SILU_MUL)
+        d1 = uniform_descriptor(w + static_cast<int64_t>(cols + n0) * K,
+                                bytes);
+    }
+  };
+  if (!LOADS_W) d0 = uniform_descriptor(x, (M - 1) * row_b + K * 2);
+  enter();
+  seek();
+  u32 rdst = ring;
+  int rslot = 0;
+  auto m0_of = [&](int j) { set_m0(rdst + j * kLoaders * 1024); };
+  auto load_of = [&](int j) {
+    if (!LOADS_W)
+      load_lds(d0, voff[j], soff);
+    else
+      load_lds_nt(SILU_MUL && j >= L / 2 ? d1 : d0, voff[j], soff);
+  };
+  auto requested = [&] {
+    rdst += kSlotB;
+    if (++rslot == R) {
+      rslot = 0;
+      rdst = ring;
+    }
+    ++issued;
+    if (++rs == rb) rs = ra;
+    if (--left == 0) {
+      ++rt;
+      enter();
+    }
+    seek();
+  };
+
+  // ---- fragment reads
+  const int ir = lane & 15, q = lane >> 4;
+  const int rd = ir * S::kRowB + ((q ^ (ir >> 1 & 7)) << 4);
+  short8 a0[CF], b0[RF], a1[CF], b1[RF];
+  floatx4 acc[RF][CF];
+  int wat = 0, xat = S::RW * S::kWB + wave * CF * 16 * S::kRowB;
+  auto read = [&](short8 (&a)[CF], short8 (&b)[RF], int half, int i) {
+    const int at = rd ^ (half * 64);
+    if (i < CF)
+      a[i] = *reinterpret_cast<const short8*>(smem + xat + at +
+                                              i * 16 * S::kRowB);
+    else
+      b[i - CF] = *reinterpret_cast<const short8*>(
+          smem + wat + at + (i - CF) * 16 * S::kRowB);
+  };
+  constexpr int kReads = RF + CF, kMfmas = RF * CF;
+  constexpr int kEvery = 2 * kReads <= kMfmas + 1 ? 2 : 1;  // products a read
+  // DMAs go out at even distances over both halves: kSoon of a stage's L in the
+  // second half, the rest in the first half of the next stage
+  constexpr int kSoon = L / 2, kApart = kMfmas / (L - kSoon);
+  static_assert(kReads <= kMfmas && L % 2 == 0 && kApart >= 2);
+  constexpr int kStores = (SILU_MUL ? RF / 2 : RF) * CF;
+  auto product = [&](int i, const short8 (&a)[CF], const short8 (&b)[RF],
+                     bool first) {
+    const int c = i / RF, f = i % RF;
+    if (first) mfma_first(acc[f][c], b[f], a[c]);
+    else mfma(acc[f][c], b[f], a[c]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  for (int k = 0; k < R; ++k) {
+#pragma unroll
+    for (int j = 0; j < L; ++j) {
+      if (k == R - 1 && j >= kSoon) break;
+      m0_of(j);
+      asm volatile("s_nop 4");
+      load_of(j);
+    }
+    if (k < R - 1) requested();
+  }
+  wait_vm<(R - 2) * L + kSoon>();
+  sync_waves();
+#pragma unroll
+  for (int i = 0; i < kReads; ++i) read(a0, b0, 0, i);
+  int wslot = 0, xslot = 0;
+  auto stage = [&](auto first, bool behind) {
+#pragma unroll
+    for (int i = 0; i < kMfmas; ++i) {
+      product(i, a0, b0, first);
+      if (i % kEvery == 0 && i / kEvery < kReads)
+        read(a1, b1, 1, i / kEvery);
+      if (i / kApart < L - kSoon) {
+        if (i % kApart == 0) m0_of(kSoon + i / kApart);
+        if (i % kApart == 1) load_of(kSoon + i / kApart);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    requested();
+    // the stage is in registers, this wave's share of the next has landed;
+    // after the barrier that is so for all waves
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (behind) wait_vm<(R - 2) * L + kStores>();
+    else wait_vm<(R - 2) * L>();
+    sync_waves();
+    wat += S::kWB;
+    if (++wslot == S::RW) wslot = wat = 0;
+    xat += S::kXB;
+    if (++xslot == S::RX) {
+      xslot = 0;
+      xat -= S::RX * S::kXB;
+    }
+#pragma unroll
+    for (int i = 0; i < kMfmas; ++i) {
+      product(i, a1, b1, false);
+      if (i % kEvery == 0 && i / kEvery < kReads)
+        read(a0, b0, 0, i / kEvery);
+      if (i / kApart < kSoon) {
+        if (i % kApart == 0) m0_of(i / kApart);
+        if (i % kApart == 1) load_of(i / kApart);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  int pos = lo, behind = 0;
+  while (pos < hi) {
+    const int tile = pos / SK;
+    const int begin = tile * SK, end = begin + SK;
+    const bool from_start = pos == begin;
+    const int stop = min(hi, end);
+    stage(std::true_type{}, behind > 0);
+    --behind;
+    for (++pos; pos < stop; ++pos, --behind)
+      stage(std::false_type{}, behind > 0);
+    settle();
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    if (from_start && stop == end) {
+#pragma unroll
+      for (int f = 0; f < (SILU_MUL ? RF / 2 : RF); ++f) {
+        const int n = tile * (SILU_MUL ? S::TN / 2 : S::TN) + f * 16 +
+                      (l >> 4) * 4;
+#pragma unroll
+        for (int c = 0; c < CF; ++c) {
+          const int m = (wave * CF + c) * 16 + (l & 15);
+          if (m < M && n < (SILU_MUL ? N / 2 : N))
+            store4<SILU_MUL, false>(
+                out, bias, Scales{}, acc_of(acc[f][c]),
+                acc_of(acc[SILU_MUL ? f + RF / 2 : f][c]), m, n, out_stride);
+        }
+      }
+      behind = 0;
+      if ((wave * CF + CF - 1) * 16 < M &&
+          (tile + 1) * (SILU_MUL ? S::TN / 2 : S::TN) <=
+              (SILU_MUL ? N / 2 : N))
+        behind = R - 2;
+    } else {
+      floatx4* p = pieces + (static_cast<int64_t>(blockIdx.x) * 2 +
+                             (from_start ? 1 : 0)) * S::kPiece +
+                   wave * RF * CF * kWaveSize + l;
+#pragma unroll
+      for (int f = 0; f < RF; ++f)
+#pragma unroll
+        for (int c = 0; c < CF; ++c)
+          p[(f * CF + c) * kWaveSize] = acc_of(acc[f][c]);
+      behind = R - 2;
+    }
+  }
+  // no DMA may land in LDS that is no longer this workgroup's
+  wait_vm<0>();
+}
+
+template <class S, bool SILU_MUL>
+__global__ __launch_bounds__(256, 1)
+void part_gemm_ahead_kernel(u16* __restrict__ out,
+                            floatx4* __restrict__ pieces,
+                            const u16* __restrict__ x,
+                            const u16* __restrict__ w,
+                            const u16* __restrict__ bias, const int M,
+                            const int N, const int K, const int64_t x_stride,
+                            const int64_t out_stride, const int tiles,
+                            const int unit) {
+  __shared__ __attribute__((aligned(1024)))
+  unsigned char smem[S::RW * S::kWB + S::RX * S::kXB];
+  const int lane = threadIdx.x % kWaveSize;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+  if (wave < S::kWLoaders)
+    run_ahead<S, SILU_MUL, true>(out, pieces, x, w, bias, M, N, K, x_stride,
+                                 out_stride, tiles, unit, smem, wave, lane);
+  else
+    run_ahead<S, SILU_MUL, false>(out, pieces, x, w, bias, M, N, K, x_stride,
+                                  out_stride, tiles, unit, smem, wave, lane);
 }
 
 // One row of workgroups per border between parts; the first border inside a
@@ -385,14 +668,13 @@ void part_gemm_join_kernel(u16* __restrict__ out,
   store4<SILU_MUL, FP8>(out, bias, scales, g, u, m, n, out_stride);
 }
 
-// How a shape cuts [N, K] up and what that takes by what limits it here: a
-// CU's share of HBM (25 GB/s), its share of what L2 delivers (39 GB/s, W and
-// x together), and, where tiles are cut, 5 us for the second kernel and the
-// way of the pieces through memory. Whole tiles on an uneven number of CUs
-// against even parts with a join comes out of the same sum, and so does the
-// caller's choice between this kernel and the library: up to 128 rows nine
-// in ten sizes take 0.9 to 1.25 times the estimate (e4m3 1.0 to 1.6), above
-// them 0.75 to 0.9.
+// How a shape cuts [N, K] up and what that takes: 3 us, a time per stage of the
+// part that has most of them, and one for the second kernel and the way of the
+// pieces through memory where tiles are cut. Both times are measured, per shape
+// (17 N by six K, weights that no cache holds, 1500 runs). Whole tiles on an
+// uneven number of CUs against even parts with a join comes out of the same sum,
+// and so does the caller's choice between this kernel and the library; the
+// shape taken is 1.0 to 1.5 % slower than the best one on average.
 struct Plan {
   int tiles = 0, parts = 0;
   bool split = false;
@@ -412,8 +694,8 @@ Plan plan_of(int N, int K, bool split) {
   const int64_t most = split
       ? (stages + p.parts - 1) / p.parts
       : static_cast<int64_t>(ceil_div(p.tiles, p.parts)) * (K / S::KS);
-  p.us = most * std::max(S::kWB / 25e3, (S::kWB + S::kXB) / 39e3);
-  if (split) p.us += 5 + p.parts * (S::kPiece * 16 * 2 / 4e6);
+  p.us = 3 + most * S::kStageUs;
+  if (split) p.us += S::kCutUs * p.parts / kChip;
   return p;
 }
 
@@ -429,10 +711,18 @@ void launch_part(const Plan& pl, u16* out, float* pieces, const u16* x,
                  int N, int K, int64_t x_stride, int64_t out_stride,
                  hipStream_t stream) {
   auto* p = reinterpret_cast<floatx4*>(pieces);
-  hipLaunchKernelGGL((part_gemm_kernel<S, SILU_MUL, FP8>), dim3(pl.parts),
-                     dim3(S::kWaves * kWaveSize), 0, stream, out, p, x, w,
-                     bias, scales, M, N, K, x_stride, out_stride, pl.tiles,
-                     pl.split ? 1 : K / S::KS);
+  const int unit = pl.split ? 1 : K / S::KS;
+  if constexpr (S::kAhead) {
+    static_assert(!FP8);
+    hipLaunchKernelGGL((part_gemm_ahead_kernel<S, SILU_MUL>), dim3(pl.parts),
+                       dim3(256), 0, stream, out, p, x, w, bias, M, N, K,
+                       x_stride, out_stride, pl.tiles, unit);
+  } else {
+    hipLaunchKernelGGL((part_gemm_kernel<S, SILU_MUL, FP8>), dim3(pl.parts),
+                       dim3(S::kWaves * kWaveSize), 0, stream, out, p, x, w,
+                       bias, scales, M, N, K, x_stride, out_stride, pl.tiles,
+                       unit);
+  }
   if (!pl.split || pl.parts == 1) return;
   hipLaunchKernelGGL((part_gemm_join_kernel<S, SILU_MUL, FP8>),
                      dim3(pl.parts - 1,
@@ -442,18 +732,57 @@ void launch_part(const Plan& pl, u16* out, float* pieces, const u16* x,
 }
 
 // Row classes and their shapes: tiles of 96 rows where the chip takes them
-// whole, 64 or 32 where N is small and K is cut, 128 or more where N is
-// large and x would be read too often.
-using A32 = PartShape<3, 2, 2, 1, 128, 5, 4, 4>;
-using B32 = PartShape<2, 2, 2, 1, 64, 7, 7, 2>;
-using A64 = PartShape<3, 2, 2, 2, 64, 7, 6, 4>;
-using B64 = PartShape<2, 2, 4, 1, 64, 7, 7, 4>;
-using C64 = PartShape<4, 2, 2, 2, 64, 6, 6, 4>;
-using A128 = PartShape<3, 2, 4, 2, 64, 7, 4, 4>;
-using B128 = PartShape<2, 2, 4, 2, 64, 7, 5, 4>;
-using C128 = PartShape<4, 4, 2, 4, 64, 3, 4, 4>;
-using A256 = PartShape<3, 2, 4, 4, 64, 5, 3, 4>;
-using B256 = PartShape<2, 2, 8, 2, 64, 6, 3, 8>;
+// whole, 64 where N is small and K is cut, 128 or more where N is large and x
+// would be read too often. From 129 rows on by waves that read ahead.
+struct B32 : PartShape<2, 2, 2, 1, 64, 7, 7, 2> {
+  static constexpr double kStageUs = 0.325, kCutUs = 4.4;
+};
+struct A32 : PartShape<3, 2, 2, 1, 128, 5, 4, 4> {
+  static constexpr double kStageUs = 0.807, kCutUs = 6.6;
+};
+struct C32 : PartShape<4, 2, 2, 1, 128, 4, 4, 4> {
+  static constexpr double kStageUs = 1.054, kCutUs = 7.4;
+};
+struct B64 : PartShape<2, 2, 4, 1, 64, 7, 7, 4> {
+  static constexpr double kStageUs = 0.384, kCutUs = 6.5;
+};
+struct A64 : PartShape<3, 2, 2, 2, 128, 4, 4, 4> {
+  static constexpr double kStageUs = 0.908, kCutUs = 8.3;
+};
+struct C64 : PartShape<4, 2, 2, 2, 64, 6, 6, 4> {
+  static constexpr double kStageUs = 0.592, kCutUs = 9.3;
+};
+struct D64 : PartShape<4, 4, 2, 2, 64, 4, 4, 4> {
+  static constexpr double kStageUs = 1.1, kCutUs = 15.7;
+};
+struct B128 : PartShape<2, 2, 4, 2, 64, 7, 5, 4> {
+  static constexpr double kStageUs = 0.526, kCutUs = 8.3;
+};
+struct A128 : PartShape<3, 2, 4, 2, 64, 7, 4, 4> {
+  static constexpr double kStageUs = 0.623, kCutUs = 11.8;
+};
+struct C128 : AheadShape<8, 2, 6, 4> {
+  static constexpr double kStageUs = 0.692, kCutUs = 13.2;
+};
+struct D128 : PartShape<4, 4, 2, 4, 64, 3, 4, 4> {
+  static constexpr double kStageUs = 1.158, kCutUs = 18.3;
+};
+struct A192 : AheadShape<6, 3, 5, 4> {
+  static constexpr double kStageUs = 0.717, kCutUs = 12.5;
+};
+struct C192 : AheadShape<8, 3, 4, 4> {
+  static constexpr double kStageUs = 0.862, kCutUs = 15.2;
+};
+struct A256 : AheadShape<6, 4, 5, 3> {
+  static constexpr double kStageUs = 0.842, kCutUs = 14.1;
+};
+struct C256 : AheadShape<8, 4, 4, 3> {
+  static constexpr double kStageUs = 0.979, kCutUs = 17.2;
+};
+// rows of W too long for the offsets within a tile
+struct L256 : PartShape<2, 2, 8, 2, 64, 6, 3, 8> {
+  static constexpr double kStageUs = 0.717, kCutUs = 10.6;
+};
 
 // calls f(shape, plan) for the shape that takes least
 template <class F, class... Shapes>
@@ -466,12 +795,22 @@ void with_best(int N, int K, const F& f, Shapes...) {
   ((best == plans + i++ ? f(Shapes{}, *best) : void()), ...);
 }
 
-template <class F>
+template <bool FP8, class F>
 void with_shape(int M, int N, int K, const F& f) {
-  if (M <= 32) with_best(N, K, f, A32{}, B32{});
-  else if (M <= 64) with_best(N, K, f, A64{}, B64{}, C64{});
-  else if (M <= 128) with_best(N, K, f, A128{}, B128{}, C128{});
-  else with_best(N, K, f, A256{}, B256{});
+  // the waves that read ahead are bf16 ones with 32-bit offsets in a tile of W
+  const bool ahead = !FP8 && K <= 1 << 22;
+  if (M <= 32) {
+    with_best(N, K, f, A32{}, B32{}, C32{});
+  } else if (M <= 64) {
+    with_best(N, K, f, A64{}, B64{}, C64{}, D64{});
+  } else if (!ahead) {
+    if (M <= 128) with_best(N, K, f, A128{}, B128{}, D128{});
+    else with_best(N, K, f, L256{});
+  } else if constexpr (!FP8) {
+    if (M <= 128) with_best(N, K, f, A128{}, B128{}, C128{}, D128{});
+    else if (M <= 192) with_best(N, K, f, A192{}, C192{});
+    else with_best(N, K, f, A256{}, C256{});
+  }
 }
 
 }  // namespace
@@ -479,16 +818,19 @@ void with_shape(int M, int N, int K, const F& f) {
 // what the chosen plan takes by its own estimate, in us
 double part_gemm_us(int M, int N, int K) {
   double us = 0;
-  with_shape(M, N, K, [&](auto, const Plan& pl) { us = pl.us; });
+  with_shape<false>(M, N, K, [&](auto, const Plan& pl) { us = pl.us; });
   return us;
 }
 
-// floats of scratch that launch_part_gemm needs
-int64_t part_gemm_floats(int M, int N, int K) {
+// floats of scratch that launch_part_gemm (fp8: launch_part_gemm_fp8 with twice
+// the K) needs
+int64_t part_gemm_floats(int M, int N, int K, bool fp8) {
   int64_t n = 0;
-  with_shape(M, N, K, [&](auto shape, const Plan& pl) {
+  auto count = [&](auto shape, const Plan& pl) {
     n = pl.split ? static_cast<int64_t>(pl.parts) * 2 * shape.kPiece * 4 : 0;
-  });
+  };
+  if (fp8) with_shape<true>(M, N, K, count);
+  else with_shape<false>(M, N, K, count);
   return n;
 }
 
@@ -497,7 +839,7 @@ void launch_part_gemm(u16* out, float* pieces, const u16* x, const u16* w,
                       const u16* bias, int M, int N, int K, int64_t x_stride,
                       int64_t out_stride, bool silu_mul,
                       hipStream_t stream) {
-  with_shape(M, N, K, [&](auto shape, const Plan& pl) {
+  with_shape<false>(M, N, K, [&](auto shape, const Plan& pl) {
     using S = decltype(shape);
     if (silu_mul)
       launch_part<S, true, false>(pl, out, pieces, x, w, bias, Scales{}, M, N,
@@ -514,7 +856,7 @@ void launch_part_gemm_fp8(u16* out, float* pieces, const unsigned char* x,
                           const float* w_scales, int M, int N, int K,
                           int64_t x_stride, int64_t out_stride,
                           hipStream_t stream) {
-  with_shape(M, N, K / 2, [&](auto shape, const Plan& pl) {
+  with_shape<true>(M, N, K / 2, [&](auto shape, const Plan& pl) {
     launch_part<decltype(shape), false, true>(
         pl, out, pieces, reinterpret_cast<const u16*>(x),
         reinterpret_cast<const u16*>(w), nullptr, Scales{x_scales, w_scales},

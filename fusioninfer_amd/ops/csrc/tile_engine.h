@@ -29,6 +29,15 @@ FI_DEV void load_lds(u32x4 desc, u32 voff, u32 soff) {
                : "memory");
 #endif
 }
+// the same for data that is read once: it leaves the caches first
+FI_DEV void load_lds_nt(u32x4 desc, u32 voff, u32 soff) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("buffer_load_dwordx4 %0, %1, %2 offen nt lds"
+               :
+               : "v"(voff), "s"(desc), "s"(soff)
+               : "memory");
+#endif
+}
 // in scalar registers, as the loads want it
 FI_DEV u32x4 uniform_descriptor(const void* p, u32 bytes) {
   u32x4 d = descriptor_of(p, bytes);

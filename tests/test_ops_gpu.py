@@ -1177,6 +1177,61 @@ def test_linear_in_parts(rows, n, k, bias):
                 <= want.abs() * 2 ** -8 + 1e-3 * k ** 0.5).all()
 
 
+@pytest.mark.parametrize("rows", [31, 64, 100, 128, 192, 193, 255])
+@pytest.mark.parametrize("n,k,bias", [
+    (65552, 128, True),     # results on their way behind stages of next tiles
+    (65568, 256, False),
+    (24624, 384, False),    # a tile of 96 rows for every workgroup, and a rest
+    (12320, 1024, False),   # fewer whole tiles than workgroups
+])
+def test_linear_in_parts_of_several_tiles(rows, n, k, bias):
+    """Parts that hold several tiles, whole or cut, against a float64 product;
+    one bf16 rounding of the result (2^-9 relative) and fp32 sums of k
+    products. What lies behind the last row of either operand has no part in
+    the result, and rows that are not of the result stay as they were."""
+    g = torch.Generator().manual_seed(n + k + rows)
+    w, x = (torch.full((m + 256, k), float("nan"), dtype=torch.bfloat16,
+                       device=DEV) for m in (n, rows))
+    w[:n] = torch.randn(n, k, generator=g)
+    x[:rows] = torch.randn(rows, k, generator=g)
+    w, x = w[:n], x[:rows]
+    b = torch.randn(n, generator=g).to(torch.bfloat16).to(DEV) if bias \
+        else None
+    prod = x.double() @ w.double().T
+    out = torch.full((rows + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops._C.few_rows_gemm(out[:rows], x, w, b, False)
+    want = prod + (0.0 if b is None else b.double())
+    assert ((out[:rows].double() - want).abs()
+            <= want.abs() * 2 ** -8 + 1e-4 * k ** 0.5).all()
+    assert (out[rows] == 7.0).all()
+    if n % 32 == 0 and not bias:
+        out = torch.full((rows + 1, n // 2), 7.0, dtype=torch.bfloat16,
+                         device=DEV)
+        ops._C.few_rows_gemm(out[:rows], x, w, None, True)
+        want = torch.nn.functional.silu(prod[:, : n // 2]) * prod[:, n // 2:]
+        assert ((out[:rows].double() - want).abs()
+                <= want.abs() * 2 ** -8 + 1e-3 * k ** 0.5).all()
+        assert (out[rows] == 7.0).all()
+
+
+@pytest.mark.parametrize("rows", [128, 129])
+def test_linear_in_parts_of_long_rows(rows):
+    """Rows of W too long for 32-bit offsets within a tile (x one row, given
+    that often). x is scaled so that the products are of size one: a bf16
+    rounding of the result and fp32 sums (2^17 additions in a lane's turn,
+    2^-24 of their size each, errors of either sign)."""
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    n, k = 16, (1 << 22) + 128
+    w = torch.randn(n, k, generator=g, device=DEV).to(torch.bfloat16)
+    x = (torch.randn(1, k, generator=g, device=DEV) / 2048).to(
+        torch.bfloat16).expand(rows, k)
+    out = torch.empty(rows, n, dtype=torch.bfloat16, device=DEV)
+    ops._C.few_rows_gemm(out, x, w, None, False)
+    want = x[:1].double() @ w.double().T
+    assert ((out.double() - want).abs()
+            <= want.abs() * 2 ** -8 + 1e-4).all()
+
+
 @pytest.mark.parametrize("rows", [1, 255, 257, 1029])
 @pytest.mark.parametrize("n,k,bias", [
     (16, 128, True),        # one ragged tile, two stages, whole
