@@ -112,6 +112,24 @@ struct PrefillPlan {
   bool split, pair;
 };
 
+// v / (1 + exp(-v)), the bits of the division (all 2^32 values compared) in
+// half its instructions: with one wave per SIMD an epilogue hides none of
+// them. A reciprocal (of a quarter of the divisor, since those below the normal
+// range come out as zero), the quotient, its remainder times the reciprocal
+// added, infinities and NaN put right. (The reciprocal alone, a unit off in
+// the last place, saves 1 % of a GEMM: 24576 x 4096 at 8192 rows 1084 us, and
+// 1095.)
+FI_DEV float silu(float v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float e = __expf(-v), d = 1.f + e;
+  const float r = __builtin_amdgcn_rcpf(fmaf(e, 0.25f, 0.25f)) * 0.25f;
+  const float q = v * r;
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, v), r, q), d, v);
+#else
+  return 0.f;
+#endif
+}
+
 // pack 8 f32 into 8 OCP-e4m3 bytes (two u32 words) via v_cvt_pk_fp8_f32
 FI_DEV void pack_fp8x8(const float* v, unsigned int out[2]) {
 #if defined(__HIP_DEVICE_COMPILE__)

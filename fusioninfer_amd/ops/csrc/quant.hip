@@ -40,7 +40,7 @@ __global__ void row_quant_fp8_kernel(
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const float gf = bf16_to_f32(g.h[j]);
-          vals[it][j] = gf / (1.f + __expf(-gf)) * bf16_to_f32(u.h[j]);
+          vals[it][j] = silu(gf) * bf16_to_f32(u.h[j]);
         }
       } else {
         bf16x8 v = *reinterpret_cast<const bf16x8*>(in + in_row + col);
@@ -68,10 +68,8 @@ __global__ void row_quant_fp8_kernel(
       for (int j = 0; j < 8; ++j) sv[j] = vals[it][j] * inv_scale;
       u32 packed[2];
       pack_fp8x8(sv, packed);
-      *reinterpret_cast<u32*>(out + static_cast<int64_t>(row) * cols + col) =
-          packed[0];
-      *reinterpret_cast<u32*>(out + static_cast<int64_t>(row) * cols + col + 4) =
-          packed[1];
+      *reinterpret_cast<uint2*>(out + static_cast<int64_t>(row) * cols + col) =
+          make_uint2(packed[0], packed[1]);
     }
   }
 }

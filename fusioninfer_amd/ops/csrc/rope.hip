@@ -6,10 +6,12 @@
 // elements, so D / 8 lanes hold a head and a wave four heads (D = 128) or
 // eight (64) of one token; the rotate-half partner is D / 16 lanes away in
 // the same row of 16 lanes, and the norm's sum is three or four exchanges
-// within it. One wave per (token, head) with two elements per lane and a
-// second kernel for the cache took 87 + 9 us at 8765 tokens, 32 + 2 * 4
-// heads of 128; this takes 41 us (4.4 TB/s). cos/sin come from a table (f32
-// [P, D], cos | sin): sines computed here would make it bound by the VALU.
+// within it. A workgroup is one token; every load is requested before anything
+// waits for one. cos/sin come from a table (f32 [P, D], cos | sin): sines
+// computed here would make it bound by the VALU. us at 32 + 2 * 8 heads of 128,
+// loads as they are needed and a rolled loop for the sum, and this: 64 tokens
+// 3.2 and 2.8, 1024 7.7 and 6.0, 4099 19.7 and 16.0 (6.3 TB/s), 8765 44.6 and
+// 37.7; e4m3 cache, 8765 43.8 and 37.9.
 //
 // Capability parity: RoPE / qk-norm epilogue and cache write the reference
 // delegates to vLLM.
@@ -24,15 +26,32 @@ namespace {
 typedef u32 u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
-constexpr int kRopeWaves = 4;
+constexpr int kRopeWaves = 16;      // of a workgroup, at most
 
-FI_DEV void load8(const u16* p, float v[8]) {
-  const u32x4_any w = *reinterpret_cast<const u32x4_any*>(p);
+FI_DEV u32x4_any load8(const u16* p) {
+  return *reinterpret_cast<const u32x4_any*>(p);
+}
+FI_DEV void unpack8(const u32x4_any& w, float v[8]) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     v[2 * i] = bf16_to_f32(static_cast<u16>(w[i] & 0xffff));
     v[2 * i + 1] = bf16_to_f32(static_cast<u16>(w[i] >> 16));
   }
+}
+
+// sum over the L lanes of a head, by exchanges with the lane 8 (L = 16), 4, 2
+// and 1 away
+template <int L>
+FI_DEV float head_sum(float s) {
+  if constexpr (L == 16) {
+    s += dpp_move<0x128>(s);         // row_ror:8
+    s += dpp_move<0x124>(s);         // row_ror:4
+  } else {
+    s += __shfl_xor(s, 4);
+  }
+  s += dpp_move<0x4E>(s);            // quad_perm [2,3,0,1]
+  s += dpp_move<0xB1>(s);            // quad_perm [1,0,3,2]
+  return s;
 }
 
 struct CacheRows {
@@ -43,7 +62,8 @@ struct CacheRows {
   float k_inv_scale, v_inv_scale;  // fp8 only
 };
 
-template <int D, bool CACHE, bool FP8>
+// UNITS: times four heads (D = 128) or eight (64) that a wave takes of a token
+template <int D, bool CACHE, bool FP8, int UNITS>
 __global__ __launch_bounds__(kRopeWaves * kWaveSize) void rope_qk_norm_kernel(
     u16* __restrict__ q,             // [T, Hq*D] rows, stride q_stride
     u16* __restrict__ k,             // [T, Hk*D] rows, stride k_stride
@@ -53,119 +73,132 @@ __global__ __launch_bounds__(kRopeWaves * kWaveSize) void rope_qk_norm_kernel(
     const u16* __restrict__ k_weight,  // [D] or nullptr
     const float* __restrict__ cos_sin,  // [P, D]
     const int* __restrict__ positions,  // [T]
-    const int tokens, const int num_q_heads, const int num_kv_heads,
-    const int groups,                // waves per token
+    const int num_q_heads, const int num_kv_heads,
     const float eps, const CacheRows cache) {
   constexpr int L = D / 8;           // lanes per head
+  constexpr int H = kWaveSize / L;   // heads at a time
   const int lane = threadIdx.x % kWaveSize;
-  const u32 unit = __builtin_amdgcn_readfirstlane(
-      blockIdx.x * kRopeWaves + threadIdx.x / kWaveSize);
-  const int token = unit / groups;
-  if (token >= tokens) return;
-  const int head = (unit - token * groups) * (kWaveSize / L) + lane / L;
-  if (head >= num_q_heads + (CACHE ? 2 : 1) * num_kv_heads) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+  const int token = blockIdx.x;
+  const int heads = num_q_heads + (CACHE ? 2 : 1) * num_kv_heads;
+  const int head0 = (blockIdx.y * kRopeWaves + wave) * (H * UNITS) + lane / L;
   const int e = (lane % L) * 8;      // first element of this lane
-  const bool is_q = head < num_q_heads;
-  const int kv = head - num_q_heads;             // K heads, then V heads
-  const bool is_v = CACHE && kv >= num_kv_heads;
 
-  // (requested here, not at its use behind the sums)
+  // all loads are requested before anything waits for one of them
   const int slot = CACHE ? cache.slots[token] : 0;
-  const u16* row = is_q ? q + token * q_stride + head * D
-      : is_v ? v + token * v_stride + (kv - num_kv_heads) * D
-             : k + token * k_stride + kv * D;
-  float x[8];
-  load8(row + e, x);
+  const int position = positions[token];
+  u32x4_any raw[UNITS], wr[UNITS];
+  f32x4_any c[2], s[2];
+  auto row_of = [&](int head) {
+    const int kv = head - num_q_heads;           // K heads, then V heads
+    return head < num_q_heads ? q + token * q_stride + head * D
+        : CACHE && kv >= num_kv_heads
+            ? v + token * v_stride + (kv - num_kv_heads) * D
+            : k + token * k_stride + kv * D;
+  };
+#pragma unroll
+  for (int u = 0; u < UNITS; ++u)
+    // heads past the last one repeat it
+    raw[u] = load8(row_of(min(head0 + u * H, heads - 1)) + e);
+  auto weight_of = [&](int head) {
+    return head < num_q_heads ? q_weight : k_weight;
+  };
+#pragma unroll
+  for (int u = 0; u < UNITS; ++u) {
+    const u16* w = weight_of(head0 + u * H);
+    wr[u] = load8((w != nullptr ? w : reinterpret_cast<const u16*>(cos_sin)) + e);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const int pair = e % (D / 2);      // rotary pair of the first element
+  const float* cs = cos_sin + static_cast<int64_t>(position) * D + pair;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    c[i] = *reinterpret_cast<const f32x4_any*>(cs + 4 * i);
+    s[i] = *reinterpret_cast<const f32x4_any*>(cs + D / 2 + 4 * i);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const float sign = e < D / 2 ? -1.f : 1.f;
 
-  if (!is_v) {
-    const int pair = e % (D / 2);    // rotary pair of the first element
-    const float* cs = cos_sin + static_cast<int64_t>(positions[token]) * D +
-                      pair;
-    f32x4_any c[2], s[2];
+  // (no branch around what a load feeds: the compiler would move the load into
+  // it, behind the waits for the others)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      c[i] = *reinterpret_cast<const f32x4_any*>(cs + 4 * i);
-      s[i] = *reinterpret_cast<const f32x4_any*>(cs + D / 2 + 4 * i);
-    }
-    const u16* w = is_q ? q_weight : k_weight;
-    if (w != nullptr) {
-      float wf[8];
-      load8(w + e, wf);
-      float sum = 0.f;
+  for (int u = 0; u < UNITS; ++u) {
+    const int head = head0 + u * H;
+    const bool is_q = head < num_q_heads;
+    const int kv = head - num_q_heads;
+    const bool is_v = CACHE && kv >= num_kv_heads;
+    const bool normed = weight_of(head) != nullptr;
+    float x[8], wf[8], sum = 0.f;
+    unpack8(raw[u], x);
+    unpack8(wr[u], wf);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) sum += x[i] * x[i];
+    for (int i = 0; i < 8; ++i) sum += x[i] * x[i];
+    sum = head_sum<L>(sum);
+    const float inv_rms = rsqrtf(sum / D + eps);
 #pragma unroll
-      for (int off = L / 2; off > 0; off >>= 1) {
-        if (off == 8) sum += dpp_move<0x128>(sum);       // row_ror:8
-        else if (off == 4 && L == 16) sum += dpp_move<0x124>(sum);  // :4
-        else if (off == 2) sum += dpp_move<0x4E>(sum);
-        else if (off == 1) sum += dpp_move<0xB1>(sum);
-        else sum += __shfl_xor(sum, off);
-      }
-      const float inv_rms = rsqrtf(sum / D + eps);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) x[i] *= inv_rms * wf[i];
-    }
+    for (int i = 0; i < 8; ++i) x[i] = normed ? x[i] * (inv_rms * wf[i]) : x[i];
     // x1' = x1 cos - x2 sin in the first half, x2' = x2 cos + x1 sin
-    const float sign = e < D / 2 ? -1.f : 1.f;
+    u32x4_any bits;
+    u16 y[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const float other = L == 16 ? dpp_move<0x128>(x[i])
                                   : __shfl_xor(x[i], L / 2);
-      x[i] = x[i] * c[i / 4][i % 4] + sign * other * s[i / 4][i % 4];
+      y[i] = f32_to_bf16(x[i] * c[i / 4][i % 4] +
+                         sign * other * s[i / 4][i % 4]);
     }
-  }
-
-  u32x4_any bits;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-    bits[i] = static_cast<u32>(f32_to_bf16(x[2 * i])) |
-              (static_cast<u32>(f32_to_bf16(x[2 * i + 1])) << 16);
-  if (!CACHE || is_q) {
-    *reinterpret_cast<u32x4_any*>(const_cast<u16*>(row) + e) = bits;
-    return;
-  }
-  if (slot < 0) return;              // padding
-  const int h = is_v ? kv - num_kv_heads : kv;
-  const int64_t dst =
-      ((static_cast<int64_t>(slot / cache.block_size) * num_kv_heads + h) *
-           cache.block_size + slot % cache.block_size) * D + e;
-  void* to = is_v ? cache.v : cache.k;
-  if (FP8) {
-    // the row as bf16 holds it, clamped to e4m3's largest value: the
-    // conversion makes NaN of what lies beyond
-    const float inv = is_v ? cache.v_inv_scale : cache.k_inv_scale;
-    float f[8];
+    for (int i = 0; i < 4; ++i)
+      bits[i] = is_v ? raw[u][i]
+                     : static_cast<u32>(y[2 * i]) |
+                           (static_cast<u32>(y[2 * i + 1]) << 16);
+    if (head >= heads) continue;
+    if (!CACHE || is_q) {
+      *reinterpret_cast<u32x4_any*>(const_cast<u16*>(row_of(head)) + e) = bits;
+      continue;
+    }
+    if (slot < 0) continue;          // padding
+    const int h = is_v ? kv - num_kv_heads : kv;
+    const int64_t dst =
+        ((static_cast<int64_t>(slot / cache.block_size) * num_kv_heads + h) *
+             cache.block_size + slot % cache.block_size) * D + e;
+    void* to = is_v ? cache.v : cache.k;
+    if (FP8) {
+      // the row as bf16 holds it, clamped to e4m3's largest value: the
+      // conversion makes NaN of what lies beyond
+      const float inv = is_v ? cache.v_inv_scale : cache.k_inv_scale;
+      float f[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      f[i] = fminf(fmaxf(bf16_to_f32(static_cast<u16>(
-                             bits[i / 2] >> (16 * (i % 2)))) * inv,
-                         -448.f), 448.f);
-    u32 packed[2];
-    pack_fp8x8(f, packed);
-    *reinterpret_cast<uint2*>(static_cast<unsigned char*>(to) + dst) =
-        make_uint2(packed[0], packed[1]);
-  } else {
-    *reinterpret_cast<u32x4_any*>(static_cast<u16*>(to) + dst) = bits;
+      for (int i = 0; i < 8; ++i)
+        f[i] = fminf(fmaxf(bf16_to_f32(static_cast<u16>(
+                               bits[i / 2] >> (16 * (i % 2)))) * inv,
+                           -448.f), 448.f);
+      u32 packed[2];
+      pack_fp8x8(f, packed);
+      *reinterpret_cast<uint2*>(static_cast<unsigned char*>(to) + dst) =
+          make_uint2(packed[0], packed[1]);
+    } else {
+      *reinterpret_cast<u32x4_any*>(static_cast<u16*>(to) + dst) = bits;
+    }
   }
 }
 
-template <int D>
+template <int D, int UNITS>
 void launch_rope(u16* q, u16* k, const u16* v, int64_t q_stride,
                  int64_t k_stride, int64_t v_stride, const u16* q_weight,
                  const u16* k_weight, const float* cos_sin,
                  const int* positions, int tokens, int hq, int hk, float eps,
                  const CacheRows& cache, bool fp8, hipStream_t stream) {
-  const int groups = ceil_div(hq + (v ? 2 : 1) * hk, kWaveSize / (D / 8));
-  const int64_t units = static_cast<int64_t>(tokens) * groups;
-  if (units == 0) return;
-  auto kernel = !v ? &rope_qk_norm_kernel<D, false, false>
-      : fp8 ? &rope_qk_norm_kernel<D, true, true>
-            : &rope_qk_norm_kernel<D, true, false>;
-  hipLaunchKernelGGL(kernel, dim3((units + kRopeWaves - 1) / kRopeWaves),
-                     dim3(kRopeWaves * kWaveSize), 0, stream, q, k, v,
-                     q_stride, k_stride, v_stride, q_weight, k_weight,
-                     cos_sin, positions, tokens, hq, hk, groups, eps, cache);
+  if (tokens == 0) return;
+  const int waves = ceil_div(hq + (v ? 2 : 1) * hk,
+                             kWaveSize / (D / 8) * UNITS);
+  auto kernel = !v ? &rope_qk_norm_kernel<D, false, false, UNITS>
+      : fp8 ? &rope_qk_norm_kernel<D, true, true, UNITS>
+            : &rope_qk_norm_kernel<D, true, false, UNITS>;
+  hipLaunchKernelGGL(kernel, dim3(tokens, ceil_div(waves, kRopeWaves)),
+                     dim3(std::min(waves, kRopeWaves) * kWaveSize), 0, stream,
+                     q, k, v, q_stride, k_stride, v_stride, q_weight,
+                     k_weight, cos_sin, positions, hq, hk, eps, cache);
 }
 
 }  // namespace
@@ -182,14 +215,22 @@ void launch_rope_qk_norm(u16* q, u16* k, const u16* v, int64_t q_stride,
                          hipStream_t stream) {
   const CacheRows cache{k_cache, v_cache, slots, block_size, k_inv_scale,
                         v_inv_scale};
-  if (head_dim == 128)
-    launch_rope<128>(q, k, v, q_stride, k_stride, v_stride, q_weight,
-                     k_weight, cos_sin, positions, tokens, num_q_heads,
-                     num_kv_heads, eps, cache, fp8, stream);
-  else
-    launch_rope<64>(q, k, v, q_stride, k_stride, v_stride, q_weight,
-                    k_weight, cos_sin, positions, tokens, num_q_heads,
-                    num_kv_heads, eps, cache, fp8, stream);
+  // from 1024 tokens on a wave takes twice the heads: cos, sin and weights once,
+  // twice the loads on the way (8765 tokens, 32 + 2 * 8 heads of 128: 48 us with
+  // one unit, 38 with two; 512 tokens 4.1 and 4.5)
+  const bool many = tokens >= 1024;
+#define FI_ROPE(D, U)                                                          \
+  launch_rope<D, U>(q, k, v, q_stride, k_stride, v_stride, q_weight, k_weight, \
+                    cos_sin, positions, tokens, num_q_heads, num_kv_heads,     \
+                    eps, cache, fp8, stream)
+  if (head_dim == 128) {
+    if (many) FI_ROPE(128, 2);
+    else FI_ROPE(128, 1);
+  } else {
+    if (many) FI_ROPE(64, 2);
+    else FI_ROPE(64, 1);
+  }
+#undef FI_ROPE
 }
 
 }  // namespace fi

@@ -100,23 +100,6 @@ FI_DEV void settle() {
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
 }
-// v / (1 + exp(-v)), the bits of the division (all 2^32 values compared) in
-// half its instructions: with one wave per SIMD an epilogue hides none of
-// them. A reciprocal (of a quarter of the divisor, since those below the normal
-// range come out as zero), the quotient, its remainder times the reciprocal
-// added, infinities and NaN put right. (The reciprocal alone, a unit off in
-// the last place, saves 1 % of a GEMM: 24576 x 4096 at 8192 rows 1084 us, and
-// 1095.)
-FI_DEV float silu(float v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const float e = __expf(-v), d = 1.f + e;
-  const float r = __builtin_amdgcn_rcpf(fmaf(e, 0.25f, 0.25f)) * 0.25f;
-  const float q = v * r;
-  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, v), r, q), d, v);
-#else
-  return 0.f;
-#endif
-}
 FI_DEV void sync_waves() {
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");

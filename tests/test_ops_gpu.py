@@ -271,6 +271,49 @@ def test_rope_qk_norm_cache(T, Hq, Hk, D, pad, fp8):
                           rtol=2 ** -3 if fp8 else 2 ** -8)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("Hq,Hk,D", [
+    (5, 1, 128),     # a wave's second unit is partly, or not at all, there
+    (72, 4, 128),    # more heads than a workgroup's waves take
+    (33, 3, 64),
+])
+def test_rope_qk_norm_cache_of_many_tokens(Hq, Hk, D, fp8):
+    """Many tokens, two units of heads per wave, are bit for bit what the same
+    tokens in shorter calls are; q against the fp32 oracle, one bf16 rounding
+    (2^-8: of an ulp that falls the other way) and 1e-5 for fp32 sums."""
+    torch.manual_seed(3)
+    T = 1027
+    qkv = torch.randn(T, (Hq + 2 * Hk) * D, device=DEV, dtype=torch.bfloat16)
+    cos_sin = ops.compute_cos_sin_cache(D, 512, 10000.0).to(DEV)
+    positions = torch.randint(0, 512, (T,), dtype=torch.int32, device=DEV)
+    qw, kw = torch.randn(2, D, device=DEV).to(torch.bfloat16)
+    slots = torch.randperm(1040, device=DEV)[:T].to(torch.int32)
+    slots[700] = -1
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    caches = [torch.zeros(65, Hk, 16, D, device=DEV).to(dt) for _ in range(4)]
+
+    def run(x, rows, k_cache, v_cache):
+        q, k, v = x[rows].split([Hq * D, Hk * D, Hk * D], dim=1)
+        ops.rope_qk_norm_cache_(q, k, v, positions[rows], cos_sin, k_cache,
+                                v_cache, slots[rows], Hq, qw, kw, 1e-6,
+                                1 / 3., 1 / 4.)
+
+    whole, parts = qkv.clone(), qkv.clone()
+    run(whole, slice(0, T), *caches[:2])
+    run(parts, slice(0, 500), *caches[2:])
+    run(parts, slice(500, T), *caches[2:])
+    assert torch.equal(whole, parts)
+    for a, b in zip(caches[:2], caches[2:]):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+    want, _ = ref.rope_qk_norm(
+        qkv[:, :Hq * D].cpu().float().view(T, Hq, D),
+        qkv[:, Hq * D:(Hq + Hk) * D].cpu().float().view(T, Hk, D),
+        positions.cpu().long(), cos_sin.cpu(), qw.cpu().float(),
+        kw.cpu().float())
+    assert_close_bf16(whole[:, :Hq * D].cpu().view(T, Hq, D), want,
+                      atol=1e-5, rtol=2 ** -8)
+
+
 def test_kv_block_gather_scatter_roundtrip():
     Hk, D, bs, nblocks = 2, 128, 16, 20
     k_cache = torch.randn(nblocks, Hk, bs, D, dtype=torch.bfloat16, device=DEV)
