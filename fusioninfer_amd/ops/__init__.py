@@ -86,10 +86,12 @@ def _streams(M: int, N: int, K: int, silu_mul: bool = False) -> bool:
 
     Up to 128 rows the kernel's own estimate (tiles, parts, joins) is held
     against what the library is seen to take: up to 64 rows W at 2.5 TB/s
-    and 4 us, above them 4 us and W at 4 TB/s or, where N gives it few tiles,
+    and 6 us, above them 5 us and W at 4 TB/s or, where N gives it few tiles,
     the chain of 7 us per 1000 of K; with silu_mul 3 us more for the pass
     over the product. (Where that errs most: 14336 x 5120 at 64 rows streams
-    in 38 us, the library takes 32.)
+    in 38 us, the library takes 32. Where the two are even, 5120 x 2048 and
+    2048 x 4096 at 64 rows 13.5 and 13.8 us, 12.9 and 14.2, a step of four such
+    layers takes 10 us less with streaming.)
 
     From 129 rows on both compute more than they read. The library's choice
     of tiles jumps with M and N there, and streaming is ahead but for few
@@ -99,7 +101,7 @@ def _streams(M: int, N: int, K: int, silu_mul: bool = False) -> bool:
     library's tiles fill the chip exactly (49152 x 4096 at 256 125 and 107).
 
     Weights that no cache holds, launched from a graph, 15 N of 2048 to
-    151936, eight K of 512 to 12288: this choice takes 0.8 to 2.1 % longer
+    151936, eight K of 512 to 12288: this choice takes 0.7 to 1.9 % longer
     than the better of the two up to 128 rows, 1.9 to 3.1 % at 160 to 256;
     the library alone 11 to 27, streaming alone 0.4 to 4. With silu_mul 0.2
     to 1.7 %, the library alone 14 to 29."""
@@ -111,8 +113,8 @@ def _streams(M: int, N: int, K: int, silu_mul: bool = False) -> bool:
         if silu_mul:
             return K >= 2048 or N <= 96 * 256
         return K >= 2048 and N * K >= (3 << 22 if M <= 192 else 5 << 22)
-    library = 4 + (2 * N * K / 2.5e6 if M <= 64
-                   else max(2 * N * K / 4e6, 7e-3 * K))
+    library = (6 + 2 * N * K / 2.5e6 if M <= 64
+               else 5 + max(2 * N * K / 4e6, 7e-3 * K))
     return _C.few_rows_gemm_us(M, N, K) < library + (3 if silu_mul else 0)
 
 
