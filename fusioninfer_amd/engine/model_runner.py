@@ -488,15 +488,22 @@ class ModelRunner:
         driver. PP: activations flow stage-to-stage with p2p send/recv
         (xGMI under RCCL); the last stage computes logits over the sampled
         rows and ships them back to rank 0. Middle stages return an empty
-        placeholder."""
+        placeholder. logits_idx None: every row is sampled."""
         import fusioninfer_amd.distributed.parallel_state as ps
 
         V = self.cfg.model.vocab_size
         if ps.pp_world_size() == 1:
-            hidden = self.model(ids, meta, self.kv_caches)
+            if logits_idx is None:
+                return self.model.compute_logits(
+                    self.model(ids, meta, self.kv_caches))
+            if getattr(self.model, "takes_rows", False):
+                hidden = self.model(ids, meta, self.kv_caches,
+                                    rows=logits_idx)
+            else:
+                hidden = self.model(ids, meta, self.kv_caches)[logits_idx]
             if logits_idx.numel() == 0:
                 return hidden.new_empty((0, V))
-            return self.model.compute_logits(hidden[logits_idx])
+            return self.model.compute_logits(hidden)
         T = ids.shape[0]
         H = self.cfg.model.hidden_size
         dt = torch.bfloat16
@@ -517,11 +524,13 @@ class ModelRunner:
                 ps.pp_send_next(h2)
                 ps.pp_send_next(r2)
         last = ps.pp_world_size() - 1
-        S = int(logits_idx.numel())
+        S = T if logits_idx is None else int(logits_idx.numel())
         if ps.pp_rank() == last:
             if S == 0:
                 return torch.empty((0, V), dtype=dt, device=self.device)
-            logits = self.model.compute_logits(final[logits_idx])
+            if logits_idx is not None:
+                final = final[logits_idx]
+            logits = self.model.compute_logits(final)
             ps.pp_send_to(logits, 0)
             return logits
         if ps.pp_rank() == 0:
@@ -760,10 +769,7 @@ class ModelRunner:
             meta.seq_bt = s["block_tables"][:bs]
             meta.seq_slots = s["state_slots"][:bs]
             meta.max_seq_rows = 1
-        return self._forward_and_logits(
-            s["ids"][:bs], meta,
-            torch.arange(bs, dtype=torch.long, device=self.device),
-        )
+        return self._forward_and_logits(s["ids"][:bs], meta, None)
 
     def capture_decode_graphs(self) -> None:
         import fusioninfer_amd.distributed.parallel_state as ps

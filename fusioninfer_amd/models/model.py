@@ -627,12 +627,16 @@ class DecoderLayer(nn.Module):
         self.eps = cfg.rms_norm_eps
         self.fp8 = cfg.quantization == "fp8"
 
-    def forward(self, hidden, residual, meta, kv_cache, cos_sin):
+    def forward(self, hidden, residual, meta, kv_cache, cos_sin,
+                keep_hidden: bool = True):
+        """keep_hidden: where residual is None the stream begins as a copy of
+        hidden; otherwise hidden itself becomes it, for a caller that has no
+        other use of it."""
         if self.fp8:
             # fused epilogues: the norms emit (fp8, per-row scale) directly
             # into the fp8 GEMMs — the bf16 normalized row never hits HBM
             if residual is None:
-                residual = hidden.clone()
+                residual = hidden.clone() if keep_hidden else hidden
                 x = ops.rms_norm_fp8(hidden, self.input_norm_weight, self.eps)
             else:
                 f8, sc, residual = ops.fused_add_rms_norm_fp8(
@@ -646,7 +650,7 @@ class DecoderLayer(nn.Module):
             hidden = self.mlp((f8, sc))
             return hidden, residual
         if residual is None:
-            residual = hidden.clone()
+            residual = hidden.clone() if keep_hidden else hidden
             hidden = ops.rms_norm(hidden, self.input_norm_weight, self.eps)
         else:
             hidden, residual = ops.fused_add_rms_norm(
@@ -662,6 +666,7 @@ class DecoderLayer(nn.Module):
 
 class CausalLM(nn.Module):
     """The full model: embedding -> N decoder layers -> final norm -> lm_head.
+    ``forward`` takes the rows whose final state is wanted.
 
     Pipeline parallelism: stage r holds a contiguous slice
     of the layers; the first stage owns the embedding, the last the final
@@ -669,6 +674,8 @@ class CausalLM(nn.Module):
     derived from the caller's seed, so the SAME seed produces the SAME
     weights regardless of the PP/TP layout (stages skip modules without
     desyncing the stream; TP ranks still slice identical full matrices)."""
+
+    takes_rows = True
 
     def __init__(self, cfg: ModelConfig):
         super().__init__()
@@ -730,14 +737,22 @@ class CausalLM(nn.Module):
         kv_caches,                   # list of (k_cache, v_cache) per LOCAL layer
         hidden: torch.Tensor = None,     # PP stages > 0: received activations
         residual: torch.Tensor = None,
+        rows: torch.Tensor = None,   # whose final state is wanted; None: all
     ):
         if self.pp_first:
             hidden = self.embed_tokens[input_ids]
             residual = None
         for layer, kv in zip(self.layers, kv_caches):
-            hidden, residual = layer(hidden, residual, meta, kv, self.cos_sin)
+            hidden, residual = layer(hidden, residual, meta, kv, self.cos_sin,
+                                     keep_hidden=not self.pp_first)
         if not self.pp_last:
             return hidden, residual
+        if rows is not None:
+            if rows.numel() == 0:
+                return hidden.new_empty((0, hidden.shape[1]))
+            hidden = hidden[rows]
+            if residual is not None:
+                residual = residual[rows]
         hidden, _ = ops.fused_add_rms_norm(
             hidden, residual, self.final_norm_weight, self.cfg.rms_norm_eps
         )
