@@ -80,17 +80,29 @@ class MergedColumnParallelLinear(nn.Module):
         return ops.linear(x, self.weight, self.bias)
 
 
-def weight_alone(layer: nn.Module) -> bool:
+def unhooked(layer: nn.Module) -> bool:
+    """No forward set on the instance, no hook."""
+    return not (
+        "forward" in vars(layer)
+        or layer._forward_hooks or layer._forward_pre_hooks
+        or layer._backward_hooks or layer._backward_pre_hooks
+        or torch.nn.modules.module._has_any_global_hook()
+    )
+
+
+def weight_alone(layer: nn.Module, bias: bool = False) -> bool:
     """Whether calling a MergedColumnParallelLinear is x W^T and nothing
     else, so that a kernel that goes on from there may take its place: no
-    bias, no forward of another class or set on the instance, no hook."""
-    return (
-        type(layer) is MergedColumnParallelLinear and layer.bias is None
-        and "forward" not in vars(layer)
-        and not (layer._forward_hooks or layer._forward_pre_hooks
-                 or layer._backward_hooks or layer._backward_pre_hooks)
-        and not torch.nn.modules.module._has_any_global_hook()
-    )
+    bias (or, asked for, one), no forward of another class or set on the
+    instance, no hook."""
+    return (type(layer) is MergedColumnParallelLinear
+            and (bias or layer.bias is None) and unhooked(layer))
+
+
+def product_alone(layer: nn.Module) -> bool:
+    """The same of a RowParallelLinear that has nothing to sum over ranks."""
+    return (type(layer) is RowParallelLinear and ps.tp_world_size() == 1
+            and unhooked(layer))
 
 
 class RowParallelLinear(nn.Module):

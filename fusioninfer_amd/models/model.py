@@ -23,6 +23,8 @@ from fusioninfer_amd.distributed.layers import (
     MergedColumnParallelLinear,
     ReplicatedLinear,
     RowParallelLinear,
+    product_alone,
+    unhooked,
     weight_alone,
 )
 from fusioninfer_amd.engine.metadata import AttnMetadata
@@ -77,8 +79,16 @@ class Attention(nn.Module):
         meta: AttnMetadata,
         kv_cache,  # (k_cache, v_cache) [B, Hk, bs, D]
         cos_sin: torch.Tensor,
-    ) -> torch.Tensor:
-        qkv = self.qkv_proj(x)
+        norm_behind: torch.Tensor = None,
+    ):
+        """x may be the rows of a residual stream: the result is added to it,
+        and its rows before the norm of norm_behind come back."""
+        stream = x if isinstance(x, ops.StreamRows) else None
+        if stream is not None:
+            qkv = ops.stream_linear(x, self.qkv_proj.weight,
+                                    self.qkv_proj.bias)
+        else:
+            qkv = self.qkv_proj(x)
         if meta.lora is not None:
             meta.lora.apply(self.layer_idx, "qkv", x, qkv)
         q = qkv[:, : self.q_size]
@@ -129,6 +139,9 @@ class Attention(nn.Module):
             )
         if vs != 1.0:
             out *= vs
+        if stream is not None:
+            return ops.stream_add_(stream.stream, out, self.o_proj.weight,
+                                   norm_behind, self.eps)
         if meta.lora is not None:
             return self.o_proj.forward_with_lora(out, meta.lora,
                                                  self.layer_idx, "o")
@@ -627,11 +640,45 @@ class DecoderLayer(nn.Module):
         self.eps = cfg.rms_norm_eps
         self.fp8 = cfg.quantization == "fp8"
 
+    def _streams(self, x, meta) -> bool:
+        """Whether the norms go into the linear layers on both sides of them
+        and the sums into those in front: few rows, whose kernels do both, and
+        linear layers that are products and nothing else."""
+        return (x.is_cuda and ops.stream_rows_ok(*x.shape)
+                and type(self.mlp) is MLP and not self.fp8
+                and meta.lora is None and ps.pp_world_size() == 1
+                and unhooked(self.self_attn) and unhooked(self.mlp)
+                and weight_alone(self.self_attn.qkv_proj, bias=True)
+                and product_alone(self.self_attn.o_proj)
+                and weight_alone(self.mlp.gate_up_proj)
+                and product_alone(self.mlp.down_proj))
+
     def forward(self, hidden, residual, meta, kv_cache, cos_sin,
-                keep_hidden: bool = True):
+                keep_hidden: bool = True, norm_behind: torch.Tensor = None):
         """keep_hidden: where residual is None the stream begins as a copy of
         hidden; otherwise hidden itself becomes it, for a caller that has no
-        other use of it."""
+        other use of it.
+
+        What is still to be added to the stream comes back first. A layer that
+        adds by itself gives the stream's rows before the norm of norm_behind
+        instead, or None without one, and the stream in fp32."""
+        rows = hidden if isinstance(hidden, ops.StreamRows) else None
+        if self._streams(hidden if residual is None else residual, meta):
+            if rows is None:
+                if hidden is None:
+                    hidden = residual
+                elif residual is not None:
+                    hidden = residual.float() + hidden
+                rows = ops.stream_begin(hidden, self.input_norm_weight,
+                                        self.eps)
+            rows = self.self_attn(rows, meta, kv_cache, cos_sin,
+                                  self.post_norm_weight)
+            act = ops.stream_linear_silu_mul(rows,
+                                             self.mlp.gate_up_proj.weight)
+            return ops.stream_add_(rows.stream, act, self.mlp.down_proj.weight,
+                                   norm_behind, self.eps), rows.stream
+        if rows is not None or hidden is None:
+            hidden, residual = residual.to(self.input_norm_weight.dtype), None
         if self.fp8:
             # fused epilogues: the norms emit (fp8, per-row scale) directly
             # into the fp8 GEMMs — the bf16 normalized row never hits HBM
@@ -742,17 +789,21 @@ class CausalLM(nn.Module):
         if self.pp_first:
             hidden = self.embed_tokens[input_ids]
             residual = None
-        for layer, kv in zip(self.layers, kv_caches):
+        norms = [layer.input_norm_weight for layer in self.layers[1:]] + [None]
+        for layer, kv, norm in zip(self.layers, kv_caches, norms):
             hidden, residual = layer(hidden, residual, meta, kv, self.cos_sin,
-                                     keep_hidden=not self.pp_first)
+                                     keep_hidden=not self.pp_first,
+                                     norm_behind=norm)
         if not self.pp_last:
             return hidden, residual
         if rows is not None:
             if rows.numel() == 0:
-                return hidden.new_empty((0, hidden.shape[1]))
-            hidden = hidden[rows]
-            if residual is not None:
-                residual = residual[rows]
+                return residual.new_empty((0, residual.shape[1]))
+            hidden = None if hidden is None else hidden[rows]
+            residual = residual[rows]
+        if hidden is None:
+            return ops.stream_norm(residual, self.final_norm_weight,
+                                   self.cfg.rms_norm_eps)
         hidden, _ = ops.fused_add_rms_norm(
             hidden, residual, self.final_norm_weight, self.cfg.rms_norm_eps
         )

@@ -112,6 +112,21 @@ struct PrefillPlan {
   bool split, pair;
 };
 
+// What the kernel for few rows does beside out = x W^T, by what is not null.
+// squares_in [parts][16]: rows of x are divided by the root mean square that
+// these have as sums of squares of K values. add: the product is added to it,
+// fp32, in place of out; with norm scaled [M, N] gets the sums times norm, and
+// squares_out [N / 16][16] their squares.
+struct SkinnyExtra {
+  const float* squares_in = nullptr;
+  int parts = 0;
+  float eps = 0.f;
+  float* add = nullptr;
+  const u16* norm = nullptr;
+  u16* scaled = nullptr;
+  float* squares_out = nullptr;
+};
+
 // v / (1 + exp(-v)), the bits of the division (all 2^32 values compared) in
 // half its instructions: with one wave per SIMD an epilogue hides none of
 // them. A reciprocal (of a quarter of the divisor, since those below the normal

@@ -27,11 +27,13 @@ namespace fi {
 // row only feeds a fp8 GEMM there, so the bf16 intermediate is never
 // materialized).
 // AHEAD: the weight is requested with the row, not behind the sums.
-template <int ITERS, bool FUSED_ADD, bool FP8_OUT, bool AHEAD>
+// F32_IN: the rows of `in` are fp32.
+template <int ITERS, bool FUSED_ADD, bool FP8_OUT, bool AHEAD,
+          bool F32_IN = false>
 __global__ __launch_bounds__(256) void rms_norm_kernel(
     void* __restrict__ out_p,       // [T, H] bf16 (FP8_OUT: u8 e4m3)
     float* __restrict__ out_scales, // [T] (FP8_OUT only; else nullptr)
-    const u16* __restrict__ in,     // [T, H]  (FUSED_ADD: the just-computed layer output x)
+    const void* __restrict__ in_p,  // [T, H]  (FUSED_ADD: the just-computed layer output x)
     u16* __restrict__ residual,     // [T, H]  in/out (FUSED_ADD only; else nullptr)
     const u16* __restrict__ weight, // [H]
     const float eps,
@@ -40,6 +42,7 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(
   const int tid = threadIdx.x;
   const int64_t base = static_cast<int64_t>(row) * hidden;
 
+  const u16* in = static_cast<const u16*>(in_p);
   constexpr int kRowsAtOnce = 2048;       // eight workgroups a CU
   constexpr int kSecondFirst = ITERS > 1;
   float vals[ITERS][8];
@@ -61,7 +64,14 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(
   for (int it = 0; it < ITERS; ++it) {
     const int col = (it * blockDim.x + tid) * 8;
     if (col < hidden) {
-      bf16x8 v = *reinterpret_cast<const bf16x8*>(in + base + col);
+      typedef __attribute__((ext_vector_type(8))) float floatx8;
+      bf16x8 v;
+      floatx8 vf;
+      if (F32_IN)
+        vf = *reinterpret_cast<const floatx8*>(
+            static_cast<const float*>(in_p) + base + col);
+      else
+        v = *reinterpret_cast<const bf16x8*>(in + base + col);
       if (AHEAD) wt[it] = *reinterpret_cast<const bf16x8*>(weight + col);
       if (FUSED_ADD) {
         bf16x8 r = *reinterpret_cast<const bf16x8*>(residual + base + col);
@@ -71,7 +81,8 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(
         if (!late) keep(it);
       } else {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) vals[it][j] = bf16_to_f32(v.h[j]);
+        for (int j = 0; j < 8; ++j)
+          vals[it][j] = F32_IN ? vf[j] : bf16_to_f32(v.h[j]);
       }
       // in an order that is written out: left to the compiler, which of the
       // first two squares is rounded before it is added changes with what
@@ -155,8 +166,8 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(
   }
 }
 
-template <bool FUSED_ADD, bool FP8_OUT>
-void launch_rms_norm(void* out, float* out_scales, const u16* in,
+template <bool FUSED_ADD, bool FP8_OUT, bool F32_IN = false>
+void launch_norm(void* out, float* out_scales, const void* in,
                      u16* residual, const u16* weight, float eps, int tokens,
                      int hidden, hipStream_t stream) {
   dim3 grid(tokens), block(256);
@@ -167,9 +178,9 @@ void launch_rms_norm(void* out, float* out_scales, const u16* in,
   // 14336 18.9 and 17.4. Up to 12288 the two differ by 2 % either way.
   constexpr int kAlwaysAhead = 6;
 #define FI_LAUNCH(N, AHEAD)                                                  \
-  hipLaunchKernelGGL((rms_norm_kernel<N, FUSED_ADD, FP8_OUT, AHEAD>), grid,  \
-                     block, 0, stream, out, out_scales, in, residual,        \
-                     weight, eps, hidden)
+  hipLaunchKernelGGL(                                                        \
+      (rms_norm_kernel<N, FUSED_ADD, FP8_OUT, AHEAD, F32_IN>), grid, block,  \
+      0, stream, out, out_scales, in, residual, weight, eps, hidden)
 #define FI_CASE(N)                                                           \
   case N:                                                                    \
     if (N <= kAlwaysAhead || tokens <= 256)                                  \
@@ -194,6 +205,21 @@ void launch_rms_norm(void* out, float* out_scales, const u16* in,
 #undef FI_LAUNCH
 }
 
+template <bool FUSED_ADD, bool FP8_OUT>
+void launch_rms_norm(void* out, float* out_scales, const u16* in,
+                     u16* residual, const u16* weight, float eps, int tokens,
+                     int hidden, hipStream_t stream) {
+  launch_norm<FUSED_ADD, FP8_OUT>(out, out_scales, in, residual, weight, eps,
+                                  tokens, hidden, stream);
+}
+
+void launch_stream_norm(u16* out, const float* in, const u16* weight,
+                        float eps, int tokens, int hidden,
+                        hipStream_t stream) {
+  launch_norm<false, false, true>(out, nullptr, in, nullptr, weight, eps,
+                                  tokens, hidden, stream);
+}
+
 template void launch_rms_norm<true, false>(void*, float*, const u16*, u16*,
                                            const u16*, float, int, int,
                                            hipStream_t);
@@ -206,5 +232,51 @@ template void launch_rms_norm<true, true>(void*, float*, const u16*, u16*,
 template void launch_rms_norm<false, true>(void*, float*, const u16*, u16*,
                                            const u16*, float, int, int,
                                            hipStream_t);
+
+// stream = x in fp32, scaled = x times weight, squares[row] = their sum
+template <class X>
+__global__ __launch_bounds__(256) void stream_begin_kernel(
+    float* __restrict__ stream, u16* __restrict__ scaled,
+    float* __restrict__ squares, const X* __restrict__ x,
+    const u16* __restrict__ weight, const int hidden) {
+  typedef __attribute__((ext_vector_type(8))) float floatx8;
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * hidden;
+  float sum = 0.f;
+  for (int col = threadIdx.x * 8; col < hidden; col += 256 * 8) {
+    floatx8 v;
+    if constexpr (sizeof(X) == 4) {
+      v = *reinterpret_cast<const floatx8*>(x + base + col);
+    } else {
+      const bf16x8 h = *reinterpret_cast<const bf16x8*>(x + base + col);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = bf16_to_f32(h.h[j]);
+    }
+    const bf16x8 g = *reinterpret_cast<const bf16x8*>(weight + col);
+    bf16x8 y;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      y.h[j] = f32_to_bf16(v[j] * bf16_to_f32(g.h[j]));
+      sum = fmaf(v[j], v[j], sum);
+    }
+    *reinterpret_cast<floatx8*>(stream + base + col) = v;
+    *reinterpret_cast<bf16x8*>(scaled + base + col) = y;
+  }
+  __shared__ float scratch[4];
+  sum = block_reduce_sum<4>(wave_reduce_sum(sum), scratch);
+  if (threadIdx.x == 0) squares[blockIdx.x] = sum;
+}
+
+template <class X>
+void launch_stream_begin(float* stream, u16* scaled, float* squares,
+                         const X* x, const u16* weight, int rows, int hidden,
+                         hipStream_t s) {
+  hipLaunchKernelGGL(stream_begin_kernel<X>, dim3(rows), dim3(256), 0, s,
+                     stream, scaled, squares, x, weight, hidden);
+}
+
+template void launch_stream_begin<u16>(float*, u16*, float*, const u16*,
+                                       const u16*, int, int, hipStream_t);
+template void launch_stream_begin<float>(float*, u16*, float*, const float*,
+                                         const u16*, int, int, hipStream_t);
 
 }  // namespace fi

@@ -38,8 +38,14 @@ void launch_prefill_attn(u16*, const u16*, const void*, const void*,
                          const int*, int, int64_t, int64_t, int64_t, int, int,
                          int, float, bool, const PrefillPlan&, float*,
                          hipStream_t);
-void launch_skinny_gemm(u16*, const u16*, const u16*, const u16*, int, int,
-                        int, int64_t, int64_t, bool, hipStream_t);
+void launch_skinny_gemm(u16*, const u16*, const u16*, const u16*,
+                        const SkinnyExtra&, int, int, int, int64_t, int64_t,
+                        bool, hipStream_t);
+void launch_stream_norm(u16*, const float*, const u16*, float, int, int,
+                        hipStream_t);
+template <class X>
+void launch_stream_begin(float*, u16*, float*, const X*, const u16*, int, int,
+                         hipStream_t);
 int64_t part_gemm_floats(int, int, int, bool);
 double part_gemm_us(int, int, int);
 void launch_part_gemm(u16*, float*, const u16*, const u16*, const u16*, int,
@@ -92,6 +98,28 @@ void rms_norm(at::Tensor out, at::Tensor input, at::Tensor weight, double eps) {
                                     nullptr, bf16_cptr(weight),
                                     static_cast<float>(eps), tokens, hidden,
                                     current_stream());
+}
+
+// of fp32 rows
+void stream_norm(at::Tensor out, at::Tensor input, at::Tensor weight,
+                 double eps) {
+  CHECK_BF16_CUDA(out);
+  CHECK_BF16_CUDA(weight);
+  TORCH_CHECK(input.is_cuda() && input.scalar_type() == at::kFloat &&
+              input.is_contiguous() && out.is_contiguous() &&
+              weight.is_contiguous() && input.dim() == 2 &&
+              out.sizes() == input.sizes());
+  const int hidden = input.size(1);
+  TORCH_CHECK(hidden > 0 && hidden % 8 == 0 && hidden <= 16384 &&
+                  weight.numel() == hidden,
+              "stream_norm: unsupported sizes");
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(input.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(weight.data_ptr()) % 16 == 0);
+  if (input.numel() == 0) return;
+  fi::launch_stream_norm(bf16_ptr(out), input.data_ptr<float>(),
+                         bf16_cptr(weight), static_cast<float>(eps),
+                         input.size(0), hidden, current_stream());
 }
 
 void fused_add_rms_norm(at::Tensor input, at::Tensor residual,
@@ -441,15 +469,16 @@ void prefill_attention_paged(at::Tensor out, at::Tensor q, at::Tensor k_cache,
       pl.split ? pieces.data_ptr<float>() : nullptr, current_stream());
 }
 
-// out [M, N] (silu_mul: [M, N / 2]) = x [M, K] @ w [N, K]^T (+ bias)
-void few_rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
-                 c10::optional<at::Tensor> bias, bool silu_mul) {
-  CHECK_BF16_CUDA(out);
-  CHECK_BF16_CUDA(x);
+void check_few_rows(const at::Tensor& out, const at::Tensor& x,
+                    const at::Tensor& w, bool silu_mul, int64_t most,
+                    at::ScalarType out_type = at::kBFloat16,
+                    at::ScalarType x_type = at::kBFloat16) {
+  TORCH_CHECK(out.is_cuda() && out.scalar_type() == out_type &&
+              x.is_cuda() && x.scalar_type() == x_type);
   CHECK_BF16_CUDA(w);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2);
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
-  TORCH_CHECK(M >= 1 && M <= 256 && w.size(1) == K && K % 128 == 0 &&
+  TORCH_CHECK(M >= 1 && M <= most && w.size(1) == K && K % 128 == 0 &&
                   K > 0 && N > 0 && N % (silu_mul ? 32 : 16) == 0 &&
                   K <= (1 << 24) && N <= (1 << 24),
               "few_rows_gemm: unsupported sizes");
@@ -459,17 +488,28 @@ void few_rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
               out.stride(1) == 1 && out.stride(0) % 4 == 0);
   TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
               reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 &&
-              reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0);
-  const u16* b = nullptr;
-  if (bias.has_value()) {
-    TORCH_CHECK(!silu_mul && bias->is_cuda() &&
-                bias->scalar_type() == at::kBFloat16 &&
-                bias->is_contiguous() && bias->numel() == N);
-    b = bf16_cptr(*bias);
-  }
+              reinterpret_cast<uintptr_t>(out.data_ptr()) %
+                      (4 * out.element_size()) == 0);
+}
+
+const u16* check_bias(const c10::optional<at::Tensor>& bias, int64_t N,
+                      bool silu_mul) {
+  if (!bias.has_value()) return nullptr;
+  TORCH_CHECK(!silu_mul && bias->is_cuda() &&
+              bias->scalar_type() == at::kBFloat16 && bias->is_contiguous() &&
+              bias->numel() == N);
+  return bf16_cptr(*bias);
+}
+
+// out [M, N] (silu_mul: [M, N / 2]) = x [M, K] @ w [N, K]^T (+ bias)
+void few_rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
+                   c10::optional<at::Tensor> bias, bool silu_mul) {
+  check_few_rows(out, x, w, silu_mul, 256);
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  const u16* b = check_bias(bias, N, silu_mul);
   if (M <= 16) {
-    fi::launch_skinny_gemm(bf16_ptr(out), bf16_cptr(x), bf16_cptr(w), b, M, N,
-                           K, x.stride(0), out.stride(0), silu_mul,
+    fi::launch_skinny_gemm(bf16_ptr(out), bf16_cptr(x), bf16_cptr(w), b, {}, M,
+                           N, K, x.stride(0), out.stride(0), silu_mul,
                            current_stream());
     return;
   }
@@ -478,6 +518,90 @@ void few_rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
   fi::launch_part_gemm(bf16_ptr(out), pieces.data_ptr<float>(), bf16_cptr(x),
                        bf16_cptr(w), b, M, N, K, x.stride(0), out.stride(0),
                        silu_mul, current_stream());
+}
+
+// the same of up to 16 rows of x, divided by the root mean square that squares
+// [parts, 16] are the sums of
+void few_rows_scaled_gemm(at::Tensor out, at::Tensor x, at::Tensor squares,
+                          double eps, at::Tensor w,
+                          c10::optional<at::Tensor> bias, bool silu_mul) {
+  check_few_rows(out, x, w, silu_mul, 16);
+  TORCH_CHECK(squares.is_cuda() && squares.scalar_type() == at::kFloat &&
+              squares.dim() == 2 && squares.size(0) >= 1 &&
+              squares.size(0) <= (1 << 20) && squares.size(1) == 16 &&
+              squares.is_contiguous() &&
+              reinterpret_cast<uintptr_t>(squares.data_ptr()) % 16 == 0);
+  fi::SkinnyExtra extra;
+  extra.squares_in = squares.data_ptr<float>();
+  extra.parts = squares.size(0);
+  extra.eps = static_cast<float>(eps);
+  fi::launch_skinny_gemm(bf16_ptr(out), bf16_cptr(x), bf16_cptr(w),
+                         check_bias(bias, w.size(0), silu_mul), extra,
+                         x.size(0), w.size(0), x.size(1), x.stride(0),
+                         out.stride(0), silu_mul, current_stream());
+}
+
+void check_stream(const at::Tensor& stream, const at::Tensor& norm,
+                  const at::Tensor& scaled, const at::Tensor& squares,
+                  int64_t parts) {
+  const int64_t M = stream.size(0), N = stream.size(1);
+  CHECK_BF16_CUDA(norm);
+  CHECK_BF16_CUDA(scaled);
+  TORCH_CHECK(M <= 16 && N % 16 == 0 && norm.is_contiguous() &&
+              norm.numel() == N && scaled.is_contiguous() &&
+              scaled.sizes() == stream.sizes() && squares.is_cuda() &&
+              squares.scalar_type() == at::kFloat && squares.is_contiguous() &&
+              squares.dim() == 2 && squares.size(0) == parts &&
+              squares.size(1) == 16);
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(norm.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(scaled.data_ptr()) % 16 == 0);
+}
+
+// stream [M, N] fp32 += x [M, K] @ w [N, K]^T, up to 16 rows; with norm also
+// scaled [M, N] = stream times norm, squares [N / 16, 16] of the rows
+void few_rows_gemm_add(at::Tensor stream, at::Tensor x, at::Tensor w,
+                       c10::optional<at::Tensor> norm,
+                       c10::optional<at::Tensor> scaled,
+                       c10::optional<at::Tensor> squares) {
+  check_few_rows(stream, x, w, false, 16, at::kFloat);
+  fi::SkinnyExtra extra;
+  extra.add = stream.data_ptr<float>();
+  TORCH_CHECK(norm.has_value() == scaled.has_value() &&
+              norm.has_value() == squares.has_value());
+  if (norm.has_value()) {
+    check_stream(stream, *norm, *scaled, *squares, w.size(0) / 16);
+    extra.norm = bf16_cptr(*norm);
+    extra.scaled = bf16_ptr(*scaled);
+    extra.squares_out = squares->data_ptr<float>();
+  }
+  fi::launch_skinny_gemm(nullptr, bf16_cptr(x), bf16_cptr(w), nullptr, extra,
+                         x.size(0), w.size(0), x.size(1), x.stride(0),
+                         stream.stride(0), false, current_stream());
+}
+
+// stream [M, N] = rows (bf16 or fp32), scaled and squares [1, 16] as above
+void stream_begin(at::Tensor stream, at::Tensor scaled, at::Tensor squares,
+                  at::Tensor rows, at::Tensor norm) {
+  TORCH_CHECK(stream.is_cuda() && stream.scalar_type() == at::kFloat &&
+              stream.dim() == 2 && stream.size(0) >= 1 &&
+              stream.is_contiguous() && rows.is_cuda() &&
+              rows.is_contiguous() && rows.sizes() == stream.sizes() &&
+              stream.size(1) > 0 && stream.size(1) <= (1 << 24) &&
+              reinterpret_cast<uintptr_t>(stream.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(rows.data_ptr()) % 16 == 0);
+  check_stream(stream, norm, scaled, squares, 1);
+  const int M = stream.size(0), N = stream.size(1);
+  if (rows.scalar_type() == at::kFloat) {
+    fi::launch_stream_begin(stream.data_ptr<float>(), bf16_ptr(scaled),
+                            squares.data_ptr<float>(),
+                            static_cast<const float*>(rows.data_ptr()), bf16_cptr(norm), M, N,
+                            current_stream());
+  } else {
+    CHECK_BF16_CUDA(rows);
+    fi::launch_stream_begin(stream.data_ptr<float>(), bf16_ptr(scaled),
+                            squares.data_ptr<float>(), bf16_cptr(rows),
+                            bf16_cptr(norm), M, N, current_stream());
+  }
 }
 
 // the same for more rows, by tiles of 256 x 256
@@ -590,6 +714,7 @@ void many_rows_gemm_fp8(at::Tensor out, at::Tensor x, at::Tensor x_scales,
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rms_norm", &rms_norm, "RMSNorm (bf16, fp32 accum)");
+  m.def("stream_norm", &stream_norm, "RMSNorm (fp32 to bf16)");
   m.def("fused_add_rms_norm", &fused_add_rms_norm,
         "in-place residual add + RMSNorm");
   m.def("silu_and_mul", &silu_and_mul, "fused SiLU-mul");
@@ -607,6 +732,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gather_kv_blocks", &gather_kv_blocks, "pack KV blocks for PD send");
   m.def("scatter_kv_blocks", &scatter_kv_blocks, "unpack KV blocks from PD recv");
   m.def("few_rows_gemm", &few_rows_gemm, "x W^T for up to 256 rows of x");
+  m.def("few_rows_scaled_gemm", &few_rows_scaled_gemm,
+        "linear layer of up to 16 rows over their root mean square");
+  m.def("few_rows_gemm_add", &few_rows_gemm_add,
+        "fp32 stream += linear layer of up to 16 rows, and the next norm");
+  m.def("stream_begin", &stream_begin, "fp32 stream of rows, the next norm");
   m.def("few_rows_gemm_us", &fi::part_gemm_us,
         "estimate for M of 17 to 256 rows, N, K of 16-bit values");
   m.def("many_rows_gemm", &many_rows_gemm, "x W^T by tiles of 256 x 256");

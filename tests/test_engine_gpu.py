@@ -398,3 +398,23 @@ def test_gpu_embeddings():
     vs = eng.embed([[5, 6, 7] * 10, [9, 8] * 12])
     assert abs(sum(x * x for x in vs[0]) - 1.0) < 1e-2
     assert vs[0] != vs[1]
+
+
+def test_layers_with_and_without_a_stream():
+    """Few rows: a layer whose parts are hooked takes its norms and sums one by
+    one, next to layers that do not, and the hook sees each call. The states
+    differ by roundings to bf16, eleven a layer of 2^-9 each."""
+    eng = make_engine(enforce_eager=True)
+    prompt = [[5, 6, 7] * 5]
+    want = torch.tensor(eng.embed(prompt)[0])
+    layers = eng.runner.model.layers
+    for hooked in ([1], [0, 2], [3], [0, 1, 2, 3]):
+        seen = []
+        hooks = [
+            layers[i].self_attn.o_proj.register_forward_hook(
+                lambda *_, i=i: seen.append(i)) for i in hooked]
+        got = torch.tensor(eng.embed(prompt)[0])
+        for h in hooks:
+            h.remove()
+        assert seen == hooked
+        assert (got - want).norm() <= len(layers) * 11 * 2 ** -9

@@ -1257,6 +1257,86 @@ def test_linear_in_parts_of_several_tiles(rows, n, k, bias):
         assert (out[rows] == 7.0).all()
 
 
+@pytest.mark.parametrize("rows", [1, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("n,k,parts,bias", [
+    (16, 128, 1, True),        # one tile; most waves without a stage
+    (2576, 1152, 127, False),  # tiles of 16 rows, parts short of a round
+    (6176, 384, 129, True),    # of 32, and one over
+    (24640, 512, 32, False),   # several tiles for some workgroups
+    (12320, 2048, 300, False),
+])
+def test_linear_of_stream_rows(rows, n, k, parts, bias):
+    """Rows divided by the root mean square that parts add up to, against
+    float64; the result is rounded to bf16 once (2^-9 relative) and the sums
+    of k products are fp32. What the parts hold for rows beyond x, and what
+    lies behind any operand's last row, has no part in the result."""
+    g = torch.Generator().manual_seed(n + k + rows)
+    w, x = (torch.full((m + 32, k), float("nan"), dtype=torch.bfloat16,
+                       device=DEV) for m in (n, rows))
+    w[:n] = torch.randn(n, k, generator=g)
+    x[:rows] = torch.randn(rows, k, generator=g)
+    w, x = w[:n], x[:rows]
+    sq = torch.full((parts + 16, 16), float("nan"), device=DEV)
+    sq[:parts, :rows] = torch.rand(parts, rows, generator=g).to(DEV) * k / parts
+    sq = sq[:parts]
+    b = torch.randn(n, generator=g).to(torch.bfloat16).to(DEV) if bias \
+        else None
+    inv = (sq[:, :rows].double().sum(0) / k + 0.5).rsqrt()[:, None]
+    prod = x.double() @ w.double().T * inv
+    out = torch.full((rows + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops._C.few_rows_scaled_gemm(out[:rows], x, sq, 0.5, w, b, False)
+    want = prod + (0.0 if b is None else b.double())
+    assert ((out[:rows].double() - want).abs()
+            <= want.abs() * 2 ** -8 + 1e-4 * k ** 0.5).all()
+    assert (out[rows] == 7.0).all()
+    if n % 32 == 0 and not bias:
+        out = torch.full((rows + 1, n // 2), 7.0, dtype=torch.bfloat16,
+                         device=DEV)
+        ops._C.few_rows_scaled_gemm(out[:rows], x, sq, 0.5, w, None, True)
+        want = torch.nn.functional.silu(prod[:, : n // 2]) * prod[:, n // 2:]
+        assert ((out[:rows].double() - want).abs()
+                <= want.abs() * 2 ** -8 + 1e-3 * k ** 0.5).all()
+        assert (out[rows] == 7.0).all()
+
+
+@pytest.mark.parametrize("rows", [1, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("n,k", [(128, 128), (2560, 1152), (4224, 256),
+                                 (6272, 384), (16384, 128)])
+def test_stream_add(rows, n, k):
+    """The sums keep fp32: off by the sums of k products alone; the rows for
+    the norm are theirs, bit by bit, and the squares add up in any order (n
+    roundings at most). Its norm, in one pass, has one rounding to bf16."""
+    g = torch.Generator().manual_seed(n + k + rows)
+    w = torch.randn(n, k, generator=g).to(torch.bfloat16).to(DEV)
+    x = torch.randn(rows, k, generator=g).to(torch.bfloat16).to(DEV)
+    norm = torch.randn(n, generator=g).to(torch.bfloat16).to(DEV)
+    begun = torch.randn(rows, n, generator=g).to(torch.bfloat16).to(DEV)
+    first = ops.stream_begin(begun, norm, 1e-6)
+    stream = first.stream
+    for r in (first, ops.stream_begin(stream, norm, 1e-6)):
+        assert torch.equal(r.stream, begun.float())
+        assert torch.equal(r.scaled, begun * norm)
+        torch.testing.assert_close(
+            r.squares.sum(0)[:rows].double(),
+            begun.double().square().sum(1), rtol=n * 2.0 ** -24, atol=0)
+    want = stream.double() + x.double() @ w.double().T
+    without = stream.clone()
+    assert ops.stream_add_(without, x, w) is None
+    r = ops.stream_add_(stream, x, w, norm, 1e-6)
+    assert r.stream is stream and torch.equal(stream, without)
+    assert ((stream.double() - want).abs()
+            <= want.abs() * 2 ** -23 + 1e-4 * k ** 0.5).all()
+    assert torch.equal(r.scaled, (stream * norm.float()).to(torch.bfloat16))
+    assert r.squares.shape == (n // 16, 16)
+    torch.testing.assert_close(
+        r.squares.sum(0)[:rows].double(), stream.double().square().sum(1),
+        rtol=n * 2.0 ** -24, atol=0)
+    want = (stream.double() * norm.double()
+            * (stream.double().square().mean(1, keepdim=True) + 1e-6).rsqrt())
+    assert ((ops.stream_norm(stream, norm, 1e-6).double() - want).abs()
+            <= want.abs() * 2 ** -8).all()
+
+
 @pytest.mark.parametrize("rows", [128, 129])
 def test_linear_in_parts_of_long_rows(rows):
     """Rows of W too long for 32-bit offsets within a tile (x one row, given
