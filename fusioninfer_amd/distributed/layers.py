@@ -80,13 +80,15 @@ class MergedColumnParallelLinear(nn.Module):
         return ops.linear(x, self.weight, self.bias)
 
 
-def unhooked(layer: nn.Module) -> bool:
-    """No forward set on the instance, no hook."""
-    return not (
-        "forward" in vars(layer)
-        or layer._forward_hooks or layer._forward_pre_hooks
-        or layer._backward_hooks or layer._backward_pre_hooks
-        or torch.nn.modules.module._has_any_global_hook()
+def unhooked(layer: nn.Module, fp8: bool = False) -> bool:
+    """No hook, and no forward set on the instance (fp8: but the conversion's
+    own)."""
+    fwd = vars(layer).get("forward")
+    return (
+        (getattr(fwd, "product_of", None) is layer if fp8 else fwd is None)
+        and not (layer._forward_hooks or layer._forward_pre_hooks
+                 or layer._backward_hooks or layer._backward_pre_hooks)
+        and not torch.nn.modules.module._has_any_global_hook()
     )
 
 
@@ -99,10 +101,30 @@ def weight_alone(layer: nn.Module, bias: bool = False) -> bool:
             and (bias or layer.bias is None) and unhooked(layer))
 
 
-def product_alone(layer: nn.Module) -> bool:
+def product_alone(layer: nn.Module, fp8: bool = False) -> bool:
     """The same of a RowParallelLinear that has nothing to sum over ranks."""
     return (type(layer) is RowParallelLinear and ps.tp_world_size() == 1
-            and unhooked(layer))
+            and unhooked(layer, fp8))
+
+
+def add_norm(layer: nn.Module, x, residual: torch.Tensor,
+             weight: torch.Tensor, eps: float, fp8: bool):
+    """The layer, its sum with the residual and the norm behind that: (rows,
+    residual), in the fp8 mode ((rows, scales), residual)."""
+    if not fp8:
+        if product_alone(layer):
+            return ops.linear_add_rms_norm(x, layer.weight, residual, weight,
+                                           eps)
+        return ops.fused_add_rms_norm(layer(x), residual, weight, eps)
+    if residual.is_cuda and product_alone(layer, fp8=True):
+        if not isinstance(x, tuple):
+            x = ops.quant_fp8_rows(x)
+        return ops.linear_fp8_add_rms_norm(*x, layer.weight,
+                                           layer.weight_scale, residual,
+                                           weight, eps)
+    f8, scales, residual = ops.fused_add_rms_norm_fp8(layer(x), residual,
+                                                      weight, eps)
+    return (f8, scales), residual
 
 
 class RowParallelLinear(nn.Module):

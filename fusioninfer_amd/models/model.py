@@ -23,6 +23,7 @@ from fusioninfer_amd.distributed.layers import (
     MergedColumnParallelLinear,
     ReplicatedLinear,
     RowParallelLinear,
+    add_norm,
     product_alone,
     unhooked,
     weight_alone,
@@ -51,6 +52,7 @@ class Attention(nn.Module):
         self.k_scale = 1.0
         self.v_scale = 1.0
         self.eps = cfg.rms_norm_eps
+        self.fp8 = cfg.quantization == "fp8"
         hidden = cfg.hidden_size
         self.qkv_proj = MergedColumnParallelLinear(
             hidden,
@@ -79,10 +81,12 @@ class Attention(nn.Module):
         meta: AttnMetadata,
         kv_cache,  # (k_cache, v_cache) [B, Hk, bs, D]
         cos_sin: torch.Tensor,
+        residual: torch.Tensor = None,
         norm_behind: torch.Tensor = None,
     ):
-        """x may be the rows of a residual stream: the result is added to it,
-        and its rows before the norm of norm_behind come back."""
+        """With the residual and the norm behind: what add_norm gives. x may
+        be the rows of a residual stream: the result is added to it, and its
+        rows before the norm of norm_behind come back."""
         stream = x if isinstance(x, ops.StreamRows) else None
         if stream is not None:
             qkv = ops.stream_linear(x, self.qkv_proj.weight,
@@ -142,6 +146,9 @@ class Attention(nn.Module):
         if stream is not None:
             return ops.stream_add_(stream.stream, out, self.o_proj.weight,
                                    norm_behind, self.eps)
+        if residual is not None:
+            return add_norm(self.o_proj, out, residual, norm_behind, self.eps,
+                            self.fp8)
         if meta.lora is not None:
             return self.o_proj.forward_with_lora(out, meta.lora,
                                                  self.layer_idx, "o")
@@ -160,19 +167,22 @@ class MLP(nn.Module):
         self.inter_per_rank = cfg.intermediate_size // ps.tp_world_size()
 
     def forward(self, x, lora=None) -> torch.Tensor:
-        if self.fp8:
-            # fused SwiGLU + fp8 row quant straight into the fp8 down_proj
-            return self.down_proj(ops.silu_and_mul_fp8(self.gate_up_proj(x)))
-        if lora is not None:
+        if lora is not None and not self.fp8:
             gu = self.gate_up_proj(x)
             lora.apply(self.layer_idx, "gate_up", x, gu)
             return self.down_proj.forward_with_lora(
                 ops.silu_and_mul(gu), lora, self.layer_idx, "down"
             )
+        return self.down_proj(self.activation(x))
+
+    def activation(self, x):
+        """What down_proj takes."""
+        if self.fp8:
+            # fused SwiGLU + fp8 row quant straight into the fp8 down_proj
+            return ops.silu_and_mul_fp8(self.gate_up_proj(x))
         if weight_alone(self.gate_up_proj):
-            return self.down_proj(
-                ops.linear_silu_mul(x, self.gate_up_proj.weight))
-        return self.down_proj(ops.silu_and_mul(self.gate_up_proj(x)))
+            return ops.linear_silu_mul(x, self.gate_up_proj.weight)
+        return ops.silu_and_mul(self.gate_up_proj(x))
 
 
 class MoEMLP(nn.Module):
@@ -660,26 +670,29 @@ class DecoderLayer(nn.Module):
         other use of it.
 
         What is still to be added to the stream comes back first. A layer that
-        adds by itself gives the stream's rows before the norm of norm_behind
-        instead, or None without one, and the stream in fp32."""
+        adds by itself gives the rows behind the norm of norm_behind instead;
+        for few rows the stream's rows before it, or None without one, and the
+        stream in fp32."""
         rows = hidden if isinstance(hidden, ops.StreamRows) else None
         if self._streams(hidden if residual is None else residual, meta):
             if rows is None:
-                if hidden is None:
+                if hidden is None or isinstance(hidden, ops.NormedRows):
                     hidden = residual
                 elif residual is not None:
                     hidden = residual.float() + hidden
                 rows = ops.stream_begin(hidden, self.input_norm_weight,
                                         self.eps)
             rows = self.self_attn(rows, meta, kv_cache, cos_sin,
-                                  self.post_norm_weight)
+                                  norm_behind=self.post_norm_weight)
             act = ops.stream_linear_silu_mul(rows,
                                              self.mlp.gate_up_proj.weight)
             return ops.stream_add_(rows.stream, act, self.mlp.down_proj.weight,
                                    norm_behind, self.eps), rows.stream
         if rows is not None or hidden is None:
             hidden, residual = residual.to(self.input_norm_weight.dtype), None
-        if self.fp8:
+        if isinstance(hidden, ops.NormedRows):
+            x = hidden.x
+        elif self.fp8:
             # fused epilogues: the norms emit (fp8, per-row scale) directly
             # into the fp8 GEMMs — the bf16 normalized row never hits HBM
             if residual is None:
@@ -690,25 +703,34 @@ class DecoderLayer(nn.Module):
                     hidden, residual, self.input_norm_weight, self.eps
                 )
                 x = (f8, sc)
-            hidden = self.self_attn(x, meta, kv_cache, cos_sin)
-            f8, sc, residual = ops.fused_add_rms_norm_fp8(
-                hidden, residual, self.post_norm_weight, self.eps
-            )
-            hidden = self.mlp((f8, sc))
-            return hidden, residual
-        if residual is None:
+        elif residual is None:
             residual = hidden.clone() if keep_hidden else hidden
-            hidden = ops.rms_norm(hidden, self.input_norm_weight, self.eps)
+            x = ops.rms_norm(hidden, self.input_norm_weight, self.eps)
         else:
-            hidden, residual = ops.fused_add_rms_norm(
+            x, residual = ops.fused_add_rms_norm(
                 hidden, residual, self.input_norm_weight, self.eps
             )
-        hidden = self.self_attn(hidden, meta, kv_cache, cos_sin)
-        hidden, residual = ops.fused_add_rms_norm(
-            hidden, residual, self.post_norm_weight, self.eps
-        )
-        hidden = self.mlp(hidden, lora=meta.lora)
-        return hidden, residual
+        if meta.lora is None and unhooked(self.self_attn):
+            x, residual = self.self_attn(x, meta, kv_cache, cos_sin, residual,
+                                         self.post_norm_weight)
+        else:
+            hidden = self.self_attn(x, meta, kv_cache, cos_sin)
+            if self.fp8:
+                f8, sc, residual = ops.fused_add_rms_norm_fp8(
+                    hidden, residual, self.post_norm_weight, self.eps
+                )
+                x = (f8, sc)
+            else:
+                x, residual = ops.fused_add_rms_norm(
+                    hidden, residual, self.post_norm_weight, self.eps
+                )
+        if (norm_behind is not None and type(self.mlp) is MLP
+                and meta.lora is None and unhooked(self.mlp)):
+            x, residual = add_norm(self.mlp.down_proj, self.mlp.activation(x),
+                                   residual, norm_behind, self.eps, self.fp8)
+            return ops.NormedRows(x), residual
+        return (self.mlp(x) if self.fp8
+                else self.mlp(x, lora=meta.lora)), residual
 
 
 class CausalLM(nn.Module):

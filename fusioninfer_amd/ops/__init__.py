@@ -294,24 +294,32 @@ def _tiles_fp8_ok(x, x_scales, w, w_scales) -> bool:
     )
 
 
+def _few_rows_fp8_ok(x, x_scales, w, w_scales) -> bool:
+    """As _skinny_ok, for e4m3 operands with a scale per row each: whole
+    256-value stages of K."""
+    return (
+        _C is not None and x.dim() == 2 and w.dim() == 2
+        and 1 <= x.shape[0] <= 128 and x.shape[1] == w.shape[1]
+        and _on_current_gpu(x, w, x_scales, w_scales)
+        and x.dtype == w.dtype == torch.float8_e4m3fn
+        and x.shape[1] % 256 == 0 and w.shape[0] % 16 == 0
+        and 0 < x.shape[1] <= 1 << 24 and 0 < w.shape[0] <= 1 << 24
+        and _streams_fp8(x.shape[0], w.shape[0], x.shape[1])
+        and x.stride(1) == 1 and x.stride(0) % 16 == 0
+        and x.stride(0) <= 1 << 22 and w.is_contiguous()
+        and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+        and x_scales.dtype == w_scales.dtype == torch.float32
+        and x_scales.is_contiguous() and w_scales.is_contiguous()
+        and x_scales.shape == x.shape[:1]
+        and w_scales.shape == w.shape[:1]
+    )
+
+
 def linear_fp8(x: torch.Tensor, x_scales: torch.Tensor, w: torch.Tensor,
                w_scales: torch.Tensor) -> torch.Tensor:
     """(x * x_scales) (w * w_scales)^T in bf16 on the GPU: x [M, K] and w
     [N, K] e4m3, a scale per row each."""
-    if (_C is not None and x.dim() == 2 and w.dim() == 2
-            and 1 <= x.shape[0] <= 128 and x.shape[1] == w.shape[1]
-            and _on_current_gpu(x, w, x_scales, w_scales)
-            and x.dtype == w.dtype == torch.float8_e4m3fn
-            and x.shape[1] % 256 == 0 and w.shape[0] % 16 == 0
-            and 0 < x.shape[1] <= 1 << 24 and 0 < w.shape[0] <= 1 << 24
-            and _streams_fp8(x.shape[0], w.shape[0], x.shape[1])
-            and x.stride(1) == 1 and x.stride(0) % 16 == 0
-            and x.stride(0) <= 1 << 22 and w.is_contiguous()
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and x_scales.dtype == w_scales.dtype == torch.float32
-            and x_scales.is_contiguous() and w_scales.is_contiguous()
-            and x_scales.shape == x.shape[:1]
-            and w_scales.shape == w.shape[:1]):
+    if _few_rows_fp8_ok(x, x_scales, w, w_scales):
         out = torch.empty((x.shape[0], w.shape[0]), dtype=torch.bfloat16,
                           device=x.device)
         _C.few_rows_gemm_fp8(out, x, x_scales, w, w_scales)
@@ -433,6 +441,38 @@ def stream_add_(stream: torch.Tensor, x: torch.Tensor, w: torch.Tensor,
     return rows
 
 
+class NormedRows(NamedTuple):
+    """Rows behind their norm; of the fp8 mode with a scale each."""
+
+    x: object
+
+
+def _norm_ok(residual, weight, rows: int, columns: int) -> bool:
+    return (
+        type(residual) in _PLAIN and type(weight) in _PLAIN
+        and residual.dtype == weight.dtype == torch.bfloat16
+        and residual.get_device() == weight.get_device()
+        == torch.cuda.current_device()
+        and residual.shape == (rows, columns) and weight.shape == (columns,)
+        and residual.is_contiguous() and weight.is_contiguous()
+        and residual.data_ptr() % 8 == 0 and weight.data_ptr() % 8 == 0
+    )
+
+
+def linear_add_rms_norm(x: torch.Tensor, w: torch.Tensor,
+                        residual: torch.Tensor, weight: torch.Tensor,
+                        eps: float):
+    """fused_add_rms_norm(linear(x, w), residual, weight, eps); 17 to 256 rows,
+    where pieces of the product are summed by a second kernel, leave that one
+    added and normed."""
+    if (SKINNY_ROWS < x.shape[0] <= PART_ROWS and _skinny_ok(x, w, 16)
+            and _norm_ok(residual, weight, x.shape[0], w.shape[0])):
+        out = torch.empty_like(residual)
+        if _C.few_rows_gemm_norm(out, x, w, residual, weight, eps):
+            return out, residual
+    return fused_add_rms_norm(linear(x, w), residual, weight, eps)
+
+
 # ------------------------------------------------------- fp8 fused epilogues
 #
 # The fp8 serving mode quantizes activations per-token for torch._scaled_mm;
@@ -460,6 +500,23 @@ def fused_add_rms_norm_fp8(x, residual, weight, eps: float):
         _C.fused_add_rms_norm_fp8(out, scales, x, residual, weight, eps)
         return out, scales, residual
     return ref.fused_add_rms_norm_fp8(x, residual, weight, eps)
+
+
+def linear_fp8_add_rms_norm(x: torch.Tensor, x_scales: torch.Tensor,
+                            w: torch.Tensor, w_scales: torch.Tensor,
+                            residual: torch.Tensor, weight: torch.Tensor,
+                            eps: float):
+    """As linear_add_rms_norm, in e4m3: ((rows, scales), residual)."""
+    if (_few_rows_fp8_ok(x, x_scales, w, w_scales)
+            and _norm_ok(residual, weight, x.shape[0], w.shape[0])):
+        out = torch.empty(residual.shape, dtype=x.dtype, device=x.device)
+        scales = torch.empty_like(x_scales)
+        if _C.few_rows_gemm_norm_fp8(out, scales, x, x_scales, w, w_scales,
+                                     residual, weight, eps):
+            return (out, scales), residual
+    out, scales, residual = fused_add_rms_norm_fp8(
+        linear_fp8(x, x_scales, w, w_scales), residual, weight, eps)
+    return (out, scales), residual
 
 
 def silu_and_mul_fp8(x: torch.Tensor):

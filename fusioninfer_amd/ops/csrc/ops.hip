@@ -48,6 +48,9 @@ void launch_stream_begin(float*, u16*, float*, const X*, const u16*, int, int,
                          hipStream_t);
 int64_t part_gemm_floats(int, int, int, bool);
 double part_gemm_us(int, int, int);
+bool launch_part_gemm_norm(void*, float*, u16*, const u16*, float, float*,
+                           const u16*, const float*, const u16*, const float*,
+                           int, int, int, int64_t, hipStream_t);
 void launch_part_gemm(u16*, float*, const u16*, const u16*, const u16*, int,
                       int, int, int64_t, int64_t, bool, hipStream_t);
 void launch_part_gemm_fp8(u16*, float*, const unsigned char*, const float*,
@@ -639,29 +642,36 @@ void many_rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
                        silu_mul, current_stream());
 }
 
-// out [M, N] bf16 = (x [M, K] * x_scales) @ (w [N, K] * w_scales)^T, e4m3
-void few_rows_gemm_fp8(at::Tensor out, at::Tensor x, at::Tensor x_scales,
-                       at::Tensor w, at::Tensor w_scales) {
-  CHECK_BF16_CUDA(out);
+void check_few_rows_fp8(const at::Tensor& x, const at::Tensor& x_scales,
+                        const at::Tensor& w, const at::Tensor& w_scales,
+                        int64_t most) {
   TORCH_CHECK(x.is_cuda() && w.is_cuda() &&
               x.scalar_type() == at::kFloat8_e4m3fn &&
               w.scalar_type() == at::kFloat8_e4m3fn);
-  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2);
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
-  TORCH_CHECK(M >= 1 && M <= 256 && w.size(1) == K && K % 256 == 0 && K > 0 &&
+  TORCH_CHECK(M >= 1 && M <= most && w.size(1) == K && K % 256 == 0 && K > 0 &&
                   N > 0 && N % 16 == 0 && K <= (1 << 24) && N <= (1 << 24),
               "few_rows_gemm_fp8: unsupported sizes");
-  TORCH_CHECK(out.size(0) == M && out.size(1) == N && out.stride(1) == 1 &&
-              out.stride(0) % 4 == 0);
   TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % 16 == 0 &&
               x.stride(0) <= (1 << 22) && w.is_contiguous());
   TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
-              reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 &&
-              reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0);
+              reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0);
   TORCH_CHECK(x_scales.is_cuda() && x_scales.scalar_type() == at::kFloat &&
               x_scales.is_contiguous() && x_scales.numel() == M &&
               w_scales.is_cuda() && w_scales.scalar_type() == at::kFloat &&
               w_scales.is_contiguous() && w_scales.numel() == N);
+}
+
+// out [M, N] bf16 = (x [M, K] * x_scales) @ (w [N, K] * w_scales)^T, e4m3
+void few_rows_gemm_fp8(at::Tensor out, at::Tensor x, at::Tensor x_scales,
+                       at::Tensor w, at::Tensor w_scales) {
+  check_few_rows_fp8(x, x_scales, w, w_scales, 256);
+  CHECK_BF16_CUDA(out);
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(out.dim() == 2 && out.size(0) == M && out.size(1) == N &&
+              out.stride(1) == 1 && out.stride(0) % 4 == 0 &&
+              reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0);
   at::Tensor pieces = at::empty({fi::part_gemm_floats(M, N, K / 2, true)},
                                 x.options().dtype(at::kFloat));
   fi::launch_part_gemm_fp8(
@@ -671,6 +681,65 @@ void few_rows_gemm_fp8(at::Tensor out, at::Tensor x, at::Tensor x_scales,
       static_cast<const unsigned char*>(w.data_ptr()),
       w_scales.data_ptr<float>(), M, N, K, x.stride(0), out.stride(0),
       current_stream());
+}
+
+void check_norm(const at::Tensor& out, const at::Tensor& residual,
+                const at::Tensor& norm, int64_t M, int64_t N) {
+  CHECK_BF16_CUDA(residual);
+  CHECK_BF16_CUDA(norm);
+  TORCH_CHECK(out.dim() == 2 && out.size(0) == M && out.size(1) == N &&
+              out.is_contiguous() && residual.sizes() == out.sizes() &&
+              residual.is_contiguous() && norm.is_contiguous() &&
+              norm.numel() == N);
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0 &&
+              reinterpret_cast<uintptr_t>(residual.data_ptr()) % 8 == 0 &&
+              reinterpret_cast<uintptr_t>(norm.data_ptr()) % 8 == 0);
+}
+
+// residual [M, N] += x [M, K] @ w [N, K]^T, out [M, N] = its rms norm times
+// norm; false, with nothing done, where the kernels for that are not chosen
+bool few_rows_gemm_norm(at::Tensor out, at::Tensor x, at::Tensor w,
+                        at::Tensor residual, at::Tensor norm, double eps) {
+  check_few_rows(out, x, w, false, 256);
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  check_norm(out, residual, norm, M, N);
+  const auto run = [&](float* pieces) {
+    return M > 16 &&
+           fi::launch_part_gemm_norm(
+               out.data_ptr(), nullptr, bf16_ptr(residual), bf16_cptr(norm),
+               static_cast<float>(eps), pieces, bf16_cptr(x), nullptr,
+               bf16_cptr(w), nullptr, M, N, K, x.stride(0), current_stream());
+  };
+  if (!run(nullptr)) return false;
+  at::Tensor pieces = at::empty({fi::part_gemm_floats(M, N, K, false)},
+                                x.options().dtype(at::kFloat));
+  return run(pieces.data_ptr<float>());
+}
+
+// the same with e4m3 operands and rows out, a scale per row each
+bool few_rows_gemm_norm_fp8(at::Tensor out, at::Tensor out_scales,
+                            at::Tensor x, at::Tensor x_scales, at::Tensor w,
+                            at::Tensor w_scales, at::Tensor residual,
+                            at::Tensor norm, double eps) {
+  check_few_rows_fp8(x, x_scales, w, w_scales, 128);
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(out.is_cuda() && out.scalar_type() == at::kFloat8_e4m3fn &&
+              out_scales.is_cuda() &&
+              out_scales.scalar_type() == at::kFloat &&
+              out_scales.is_contiguous() && out_scales.numel() == M);
+  check_norm(out, residual, norm, M, N);
+  const auto run = [&](float* pieces) {
+    return fi::launch_part_gemm_norm(
+        out.data_ptr(), out_scales.data_ptr<float>(), bf16_ptr(residual),
+        bf16_cptr(norm), static_cast<float>(eps), pieces,
+        static_cast<const u16*>(x.data_ptr()), x_scales.data_ptr<float>(),
+        static_cast<const u16*>(w.data_ptr()), w_scales.data_ptr<float>(), M,
+        N, K / 2, x.stride(0) / 2, current_stream());
+  };
+  if (!run(nullptr)) return false;
+  at::Tensor pieces = at::empty({fi::part_gemm_floats(M, N, K / 2, true)},
+                                x.options().dtype(at::kFloat));
+  return run(pieces.data_ptr<float>());
 }
 
 // the same for more rows, by tiles of 256 x 256
@@ -744,6 +813,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "estimate for M, N, bytes of a row of K");
   m.def("many_rows_gemm_fp8", &many_rows_gemm_fp8,
         "x W^T by tiles of 256 x 256, e4m3 with scales per row");
+  m.def("few_rows_gemm_norm", &few_rows_gemm_norm,
+        "residual += x W^T and its norm, or false");
+  m.def("few_rows_gemm_norm_fp8", &few_rows_gemm_norm_fp8,
+        "the same with e4m3 operands and rows out");
   m.def("few_rows_gemm_fp8", &few_rows_gemm_fp8,
         "x W^T for up to 256 rows of e4m3 x with scales per row");
   m.def("paged_attention_decode", &paged_attention_decode,

@@ -39,6 +39,14 @@
 // 49 / 49 / 53 / 69; 4096, 12288 23 (4380) / 26 / 33 / 44 against 27 / 37 / 67 /
 // 55; 151936, 2048 109 (5710) / 128 / 153 / 188 against 145 / 150 / 166 / 212.
 //
+// Where a norm follows, the second kernel does the sum with the residual and
+// the norm too (part_gemm_norm_kernel): a launch of 3 to 5 us less, and the
+// product is not rounded before the sum. us, product and norm / both in one, at
+// 43 / 64 / 128 / 256 rows: 4096 x 4096 17.5, 18.2, 23.3, 29.4 / 15.7, 16.2, 20.8,
+// 28.3; 4096 x 12288 28.7, 30.0, 36.7, 47.4 / 27.0, 29.0, 36.0, 45.9; e4m3 at 64
+// rows 16.4 / 14.2 and 23.6 / 21.5. A step of eight layers at 256 rows 3360 ->
+// 3333 us.
+//
 // FP8: the same kernel on e4m3 rows, 1 to 128 of them. 24576 x 4096 at 16 / 32
 // / 64 rows 19.8 (5090) / 19.9 / 23.5 us, the library's GEMM 30.1 / 25.7 /
 // 26.7; 4096 x 12288 15.0 (3350) / 15.8 / 19.7 against 19.3 / 20.5 / 24.4.
@@ -124,6 +132,21 @@ struct Scales {
   const float* w;
 };
 
+// Where a piece has a lane's results of a fragment: fragment by fragment of a
+// wave, or, with ROWS, for a kernel that sums whole rows. There rows of the tile
+// follow one another; from 129 rows of x on, where that kernel has workgroups
+// enough and the product is held up by its stores, 16 columns of all rows do: a
+// wave's store is 1 KB in one, not 16 times 64 bytes. (Both kernels, 4096 x 4096
+// at 43 / 192 / 256 rows: 15.7 / 25.3 / 30.0 us with rows, 16.4 / 24.4 / 27.7
+// with columns.)
+template <class S, bool ROWS>
+FI_DEV int in_piece(int wave, int wn, int wm, int f, int c, int lane) {
+  if (!ROWS) return ((wave * S::RF + f) * S::CF + c) * kWaveSize + lane;
+  const int m = (wm * S::CF + c) * 16 + (lane & 15), nf = wn * S::RF + f;
+  return S::kAhead ? (nf * S::MB + m) * 4 + (lane >> 4)
+                   : m * (S::TN / 4) + nf * 4 + (lane >> 4);
+}
+
 // results n4 .. n4+3 of row m; SILU_MUL: of gate values g and up values u
 template <bool SILU_MUL, bool FP8>
 FI_DEV void store4(u16* out, const u16* bias, const Scales& scales,
@@ -145,7 +168,7 @@ FI_DEV void store4(u16* out, const u16* bias, const Scales& scales,
 
 // FP8: e4m3 values, two to a u16 everywhere (K and strides too); a chunk of 16
 // goes through two products, in the same order for W and x
-template <class S, bool SILU_MUL, bool FP8>
+template <class S, bool SILU_MUL, bool FP8, bool ROWS>
 __global__ __launch_bounds__(S::kWaves * kWaveSize)
 void part_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
                       const u16* __restrict__ x, const u16* __restrict__ w,
@@ -329,7 +352,7 @@ void part_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
       if (++wslot == S::RW) wslot = 0;
       if (++xslot == S::RX) xslot = 0;
     }
-    if (from_start && stop == end) {
+    if (!ROWS && from_start && stop == end) {
 #pragma unroll
       for (int f = 0; f < (SILU_MUL ? RF / 2 : RF); ++f) {
         const int n = tile * (SILU_MUL ? S::TN / 2 : S::TN) +
@@ -353,13 +376,12 @@ void part_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
       // a part holds at most two pieces: the end of a tile that an earlier
       // part began (0) and the start of one that goes on (1)
       floatx4* p = pieces + (static_cast<int64_t>(blockIdx.x) * 2 +
-                             (from_start ? 1 : 0)) * S::kPiece +
-                   wave * RF * CF * kWaveSize + lane;
+                             (from_start ? 1 : 0)) * S::kPiece;
 #pragma unroll
       for (int f = 0; f < RF; ++f)
 #pragma unroll
         for (int c = 0; c < CF; ++c)
-          p[(f * CF + c) * kWaveSize] = acc[f][c];
+          p[in_piece<S, ROWS>(wave, wn, wm, f, c, lane)] = acc[f][c];
       behind = (loads_w ? S::RW : S::RX) - 1;
     }
   }
@@ -372,7 +394,7 @@ void part_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
 // read; with them in registers, and the next stage landed, the barrier frees the
 // stage's place, and the second half's products cover the reads of the next
 // stage's first half and half of the DMAs into the free place.
-template <class S, bool SILU_MUL, bool LOADS_W>
+template <class S, bool SILU_MUL, bool ROWS, bool LOADS_W>
 FI_DEV void run_ahead(u16* __restrict__ out, floatx4* __restrict__ pieces,
                       const u16* __restrict__ x, const u16* __restrict__ w,
                       const u16* __restrict__ bias, const int M, const int N,
@@ -556,7 +578,7 @@ FI_DEV void run_ahead(u16* __restrict__ out, floatx4* __restrict__ pieces,
     settle();
     int l = lane;
     asm volatile("" : "+v"(l));
-    if (from_start && stop == end) {
+    if (!ROWS && from_start && stop == end) {
 #pragma unroll
       for (int f = 0; f < (SILU_MUL ? RF / 2 : RF); ++f) {
         const int n = tile * (SILU_MUL ? S::TN / 2 : S::TN) + f * 16 +
@@ -577,13 +599,12 @@ FI_DEV void run_ahead(u16* __restrict__ out, floatx4* __restrict__ pieces,
         behind = R - 2;
     } else {
       floatx4* p = pieces + (static_cast<int64_t>(blockIdx.x) * 2 +
-                             (from_start ? 1 : 0)) * S::kPiece +
-                   wave * RF * CF * kWaveSize + l;
+                             (from_start ? 1 : 0)) * S::kPiece;
 #pragma unroll
       for (int f = 0; f < RF; ++f)
 #pragma unroll
         for (int c = 0; c < CF; ++c)
-          p[(f * CF + c) * kWaveSize] = acc_of(acc[f][c]);
+          p[in_piece<S, ROWS>(wave, 0, wave, f, c, l)] = acc_of(acc[f][c]);
       behind = R - 2;
     }
   }
@@ -591,7 +612,7 @@ FI_DEV void run_ahead(u16* __restrict__ out, floatx4* __restrict__ pieces,
   wait_vm<0>();
 }
 
-template <class S, bool SILU_MUL>
+template <class S, bool SILU_MUL, bool ROWS>
 __global__ __launch_bounds__(256, 1)
 void part_gemm_ahead_kernel(u16* __restrict__ out,
                             floatx4* __restrict__ pieces,
@@ -606,11 +627,13 @@ void part_gemm_ahead_kernel(u16* __restrict__ out,
   const int lane = threadIdx.x % kWaveSize;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
   if (wave < S::kWLoaders)
-    run_ahead<S, SILU_MUL, true>(out, pieces, x, w, bias, M, N, K, x_stride,
-                                 out_stride, tiles, unit, smem, wave, lane);
+    run_ahead<S, SILU_MUL, ROWS, true>(out, pieces, x, w, bias, M, N, K,
+                                       x_stride, out_stride, tiles, unit, smem,
+                                       wave, lane);
   else
-    run_ahead<S, SILU_MUL, false>(out, pieces, x, w, bias, M, N, K, x_stride,
-                                  out_stride, tiles, unit, smem, wave, lane);
+    run_ahead<S, SILU_MUL, ROWS, false>(out, pieces, x, w, bias, M, N, K,
+                                        x_stride, out_stride, tiles, unit,
+                                        smem, wave, lane);
 }
 
 // One row of workgroups per border between parts; the first border inside a
@@ -668,6 +691,109 @@ void part_gemm_join_kernel(u16* __restrict__ out,
   store4<SILU_MUL, FP8>(out, bias, scales, g, u, m, n, out_stride);
 }
 
+// The second kernel where a norm follows: a workgroup sums a row's pieces, adds
+// the residual, writes it back and leaves the normed row, as bf16 or (OUT8)
+// as e4m3 with the row's scale. Bound by the way of the pieces through memory,
+// all of a thread's on their way at once; 256 rows of 4096 take 7.8 us, the sum
+// of pieces alone 6.8 and the norm 4.4. Every tile is in pieces, none of which is more
+// than a tile long: the first piece of a tile is its part's start of one, the
+// others are ends.
+template <class S, bool FP8, bool OUT8, int THREADS, int ITERS>
+__global__ __launch_bounds__(THREADS)
+void part_gemm_norm_kernel(void* __restrict__ out, float* __restrict__ out_scales,
+                           const floatx4* __restrict__ pieces,
+                           u16* __restrict__ residual,
+                           const u16* __restrict__ norm, const float eps,
+                           const Scales scales, const int M, const int N,
+                           const int K, const int tiles, const int parts) {
+  const int SK = K / S::KS;
+  const Cut cut(tiles * SK, parts, 1);
+  // two rows that share the lines of the pieces go to the same XCD, whose turn
+  // comes every eight workgroups
+  const int xcd = blockIdx.x % 8, turn = blockIdx.x / 8;
+  const int m = S::kAhead ? (turn / 2 * 8 + xcd) * 2 + turn % 2
+                          : static_cast<int>(blockIdx.x);
+  if (m >= M) return;
+  const int64_t row = static_cast<int64_t>(m) * N;
+  const BufferRsrc from = buffer_of(pieces, parts * 2 * S::kPiece * 16u);
+  floatx4 v[ITERS];
+  bf16x4 weight[ITERS];
+  float squares = 0.f;
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int n = (it * THREADS + static_cast<int>(threadIdx.x)) * 4;
+    v[it] = {0.f, 0.f, 0.f, 0.f};
+    if (n < N) {
+      weight[it] = *reinterpret_cast<const bf16x4*>(norm + n);
+      const bf16x4 r = *reinterpret_cast<const bf16x4*>(residual + row + n);
+      const int tile = n / S::TN;
+      const int first = cut.holder(tile * SK);
+      const int last = cut.holder(tile * SK + SK - 1);
+      const int of = n % S::TN;        // the tile's column
+      const u32 at = S::kAhead ? (of / 16 * S::MB + m) * 64 + of % 16 * 4
+                               : (m * S::TN + of) * 4;
+      constexpr int kAtOnce = 8;
+      for (int q = first; q <= last; q += kAtOnce) {
+        floatx4 got[kAtOnce];
+#pragma unroll
+        for (int i = 0; i < kAtOnce; ++i)   // beyond the last: zeros, no fetch
+          got[i] = __builtin_bit_cast(floatx4, buffer_load16(
+              from, q + i > last ? ~0u
+                                 : at + ((q + i) * 2 + (q + i == first)) *
+                                            (S::kPiece * 16u), 0));
+#pragma unroll
+        for (int i = 0; i < kAtOnce; ++i) v[it] += got[i];
+      }
+      bf16x4 sum;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (FP8) v[it][j] *= scales.x[m] * scales.w[n + j];
+        v[it][j] += bf16_to_f32(r.h[j]);
+        sum.h[j] = f32_to_bf16(v[it][j]);
+        squares = fmaf(v[it][j], v[it][j], squares);
+      }
+      *reinterpret_cast<bf16x4*>(residual + row + n) = sum;
+    }
+  }
+  __shared__ float scratch[2][THREADS / kWaveSize];
+  squares = block_reduce_sum<THREADS / kWaveSize>(wave_reduce_sum(squares),
+                                                  scratch[0]);
+  const float inv_rms = rsqrtf(squares / N + eps);
+  float most = 0.f;
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int n = (it * THREADS + static_cast<int>(threadIdx.x)) * 4;
+    if (n >= N) continue;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[it][j] *= inv_rms * bf16_to_f32(weight[it].h[j]);
+      most = fmaxf(most, fabsf(v[it][j]));
+    }
+    if (!OUT8) {
+      bf16x4 o;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o.h[j] = f32_to_bf16(v[it][j]);
+      *reinterpret_cast<bf16x4*>(static_cast<u16*>(out) + row + n) = o;
+    }
+  }
+  if (!OUT8) return;
+  most = block_reduce_max<THREADS / kWaveSize>(wave_reduce_max(most),
+                                               scratch[1]);
+  const float scale = fmaxf(most, 1e-8f) / 448.0f, inv = 1.f / scale;
+  if (threadIdx.x == 0) out_scales[m] = scale;
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int n = (it * THREADS + static_cast<int>(threadIdx.x)) * 4;
+    if (n >= N) continue;
+    float o[8] = {v[it][0] * inv, v[it][1] * inv, v[it][2] * inv,
+                  v[it][3] * inv};
+    u32 packed[2];
+    pack_fp8x8(o, packed);
+    *reinterpret_cast<u32*>(static_cast<unsigned char*>(out) + row + n) =
+        packed[0];
+  }
+}
+
 // How a shape cuts [N, K] up and what that takes: 3 us, a time per stage of the
 // part that has most of them, and one for the second kernel and the way of the
 // pieces through memory where tiles are cut. Both times are measured, per shape
@@ -705,25 +831,36 @@ Plan plan_of(int N, int K) {
   return a.us <= b.us ? a : b;
 }
 
+template <class S, bool SILU_MUL, bool FP8, bool ROWS>
+void launch_products(const Plan& pl, u16* out, float* pieces, const u16* x,
+                     const u16* w, const u16* bias, const Scales& scales,
+                     int M, int N, int K, int64_t x_stride, int64_t out_stride,
+                     hipStream_t stream) {
+  auto* p = reinterpret_cast<floatx4*>(pieces);
+  const int unit = pl.split ? 1 : K / S::KS;
+  if constexpr (S::kAhead) {
+    static_assert(!FP8);
+    hipLaunchKernelGGL((part_gemm_ahead_kernel<S, SILU_MUL, ROWS>),
+                       dim3(pl.parts), dim3(256), 0, stream, out, p, x, w,
+                       bias, M, N, K, x_stride, out_stride, pl.tiles, unit);
+  } else {
+    hipLaunchKernelGGL((part_gemm_kernel<S, SILU_MUL, FP8, ROWS>),
+                       dim3(pl.parts), dim3(S::kWaves * kWaveSize), 0, stream,
+                       out, p, x, w, bias, scales, M, N, K, x_stride,
+                       out_stride, pl.tiles, unit);
+  }
+}
+
 template <class S, bool SILU_MUL, bool FP8>
 void launch_part(const Plan& pl, u16* out, float* pieces, const u16* x,
                  const u16* w, const u16* bias, const Scales& scales, int M,
                  int N, int K, int64_t x_stride, int64_t out_stride,
                  hipStream_t stream) {
-  auto* p = reinterpret_cast<floatx4*>(pieces);
-  const int unit = pl.split ? 1 : K / S::KS;
-  if constexpr (S::kAhead) {
-    static_assert(!FP8);
-    hipLaunchKernelGGL((part_gemm_ahead_kernel<S, SILU_MUL>), dim3(pl.parts),
-                       dim3(256), 0, stream, out, p, x, w, bias, M, N, K,
-                       x_stride, out_stride, pl.tiles, unit);
-  } else {
-    hipLaunchKernelGGL((part_gemm_kernel<S, SILU_MUL, FP8>), dim3(pl.parts),
-                       dim3(S::kWaves * kWaveSize), 0, stream, out, p, x, w,
-                       bias, scales, M, N, K, x_stride, out_stride, pl.tiles,
-                       unit);
-  }
+  launch_products<S, SILU_MUL, FP8, false>(pl, out, pieces, x, w, bias, scales,
+                                           M, N, K, x_stride, out_stride,
+                                           stream);
   if (!pl.split || pl.parts == 1) return;
+  auto* p = reinterpret_cast<const floatx4*>(pieces);
   hipLaunchKernelGGL((part_gemm_join_kernel<S, SILU_MUL, FP8>),
                      dim3(pl.parts - 1,
                           ceil_div(S::kPiece / (SILU_MUL ? 2 : 1), 256)),
@@ -862,6 +999,49 @@ void launch_part_gemm_fp8(u16* out, float* pieces, const unsigned char* x,
         reinterpret_cast<const u16*>(w), nullptr, Scales{x_scales, w_scales},
         M, N, K / 2, x_stride / 2, out_stride, stream);
   });
+}
+
+// The product of 17 to 256 rows (e4m3: 1 to 128), its sum with the residual and
+// the norm behind, N up to 16384. Whether that is done, which it is where the
+// second kernel runs anyway and no part holds more than a tile; if not, nothing
+// is. x_scales: e4m3 operands, sizes in pairs of values, and e4m3 rows out.
+bool launch_part_gemm_norm(void* out, float* out_scales, u16* residual,
+                           const u16* norm, float eps, float* pieces,
+                           const u16* x, const float* x_scales, const u16* w,
+                           const float* w_scales, int M, int N, int K,
+                           int64_t x_stride, hipStream_t stream) {
+  bool done = false;
+  auto run = [&](auto shape, const Plan& pl, auto fp8) {
+    using S = decltype(shape);
+    constexpr bool kFp8 = decltype(fp8)::value;
+    if (!pl.split || pl.tiles >= pl.parts || N > 16384) return;
+    done = true;
+    if (pieces == nullptr) return;
+    const Scales scales{x_scales, w_scales};
+    launch_products<S, false, kFp8, true>(pl, nullptr, pieces, x, w, nullptr,
+                                          scales, M, N, K, x_stride, 0,
+                                          stream);
+    auto* p = reinterpret_cast<const floatx4*>(pieces);
+#define FI_NORM(THREADS, ITERS)                                               \
+  hipLaunchKernelGGL((part_gemm_norm_kernel<S, kFp8, kFp8, THREADS, ITERS>),  \
+                     dim3(ceil_div(M, 16) * 16), dim3(THREADS), 0, stream,    \
+                     out, out_scales, p, residual, norm, eps, scales, M, N,   \
+                     K, pl.tiles, pl.parts)
+    if (N <= 2048) FI_NORM(512, 1);
+    else if (N <= 4096) FI_NORM(1024, 1);
+    else if (N <= 8192) FI_NORM(1024, 2);
+    else FI_NORM(1024, 4);
+#undef FI_NORM
+  };
+  if (x_scales != nullptr)
+    with_shape<true>(M, N, K, [&](auto shape, const Plan& pl) {
+      run(shape, pl, std::true_type{});
+    });
+  else
+    with_shape<false>(M, N, K, [&](auto shape, const Plan& pl) {
+      run(shape, pl, std::false_type{});
+    });
+  return done;
 }
 
 }  // namespace fi

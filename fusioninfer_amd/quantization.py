@@ -96,4 +96,5 @@ def _make_fp8_forward(m):
             out = ps.tp_all_reduce(out)
         return out
 
+    fwd.product_of = m
     return fwd

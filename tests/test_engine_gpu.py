@@ -13,9 +13,11 @@ from fusioninfer_amd.models.registry import get_model_config
 pytestmark = pytest.mark.gpu
 
 
-def make_engine(enforce_eager, num_blocks=512, max_seqs=16):
+def make_engine(enforce_eager, num_blocks=512, max_seqs=16, fp8=False):
     mc = get_model_config("Qwen3-0.6B")
     mc.num_layers = 4
+    if fp8:
+        mc.quantization = "fp8"
     cfg = EngineConfig(
         model=mc,
         cache=CacheConfig(num_gpu_blocks=num_blocks),
@@ -400,12 +402,15 @@ def test_gpu_embeddings():
     assert vs[0] != vs[1]
 
 
-def test_layers_with_and_without_a_stream():
-    """Few rows: a layer whose parts are hooked takes its norms and sums one by
-    one, next to layers that do not, and the hook sees each call. The states
-    differ by roundings to bf16, eleven a layer of 2^-9 each."""
-    eng = make_engine(enforce_eager=True)
-    prompt = [[5, 6, 7] * 5]
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("length", [15, 42])
+def test_layers_whose_norms_are_apart(length, fp8):
+    """A layer whose parts are hooked takes its norms and sums one by one, next
+    to layers that have them in the linear layers' kernels, and the hook sees
+    each call. The states differ by roundings to bf16, eleven a layer of 2^-9
+    each, in the fp8 mode by four to e4m3 of 2^-4."""
+    eng = make_engine(enforce_eager=True, fp8=fp8)
+    prompt = [[5, 6, 7] * (length // 3)]
     want = torch.tensor(eng.embed(prompt)[0])
     layers = eng.runner.model.layers
     for hooked in ([1], [0, 2], [3], [0, 1, 2, 3]):
@@ -417,4 +422,5 @@ def test_layers_with_and_without_a_stream():
         for h in hooks:
             h.remove()
         assert seen == hooked
-        assert (got - want).norm() <= len(layers) * 11 * 2 ** -9
+        bound = 11 * 2 ** -9 + (4 * 2 ** -4 if fp8 else 0)
+        assert (got - want).norm() <= len(layers) * bound

@@ -1337,6 +1337,69 @@ def test_stream_add(rows, n, k):
             <= want.abs() * 2 ** -8).all()
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("rows", [17, 32, 33, 64, 65, 128, 129, 192, 193, 256])
+@pytest.mark.parametrize("n,k", [
+    (4096, 4096), (2064, 4608),   # a tile that is not full
+    (1040, 512),                  # few parts, fewer stages in each
+    (8208, 1024), (12304, 256),
+    (16400, 256),                 # rows longer than the kernel takes
+])
+def test_linear_in_parts_and_norm(rows, n, k, fp8):
+    """The sum of a residual and a product in parts, and its norm, against
+    float64: fp32 sums of k products; the sum and the normed row are rounded to
+    bf16 once (2^-9 relative), or the row to e4m3 (2^-4, 2^-10 of the scale
+    where it is smallest). Nothing is written behind the last row, nor anything
+    at all where another way is taken."""
+    if fp8 and rows > 128:
+        pytest.skip("more rows than the e4m3 kernels take")
+    g = torch.Generator().manual_seed(n + k + rows)
+    x = torch.randn(rows, k, generator=g).to(torch.bfloat16).to(DEV)
+    w = torch.randn(n, k, generator=g).to(torch.bfloat16).to(DEV)
+    norm = torch.randn(n, generator=g).to(torch.bfloat16).to(DEV)
+    old = (torch.randn(rows + 1, n, generator=g) * k ** 0.5).to(
+        torch.bfloat16).to(DEV)
+    residual = old.clone()
+    if fp8:
+        x, xs = ops.quant_fp8_rows(x)
+        w, ws = w.to(torch.float8_e4m3fn), torch.rand(n, generator=g).to(DEV)
+        prod = (x.double() * xs.double()[:, None]) @ (
+            w.double() * ws.double()[:, None]).T
+        out = torch.ones(rows + 1, n, device=DEV).to(x.dtype)
+        scales = torch.full((rows + 1,), 7.0, device=DEV)
+        done = ops._C.few_rows_gemm_norm_fp8(
+            out[:rows], scales[:rows], x, xs, w, ws, residual[:rows], norm,
+            1e-6)
+        got = out[:rows].double() * scales[:rows].double()[:, None]
+        assert scales[rows] == 7.0 and (out[rows].float() == 1.0).all()
+    else:
+        prod = x.double() @ w.double().T
+        out = torch.full((rows + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+        done = ops._C.few_rows_gemm_norm(out[:rows], x, w, residual[:rows],
+                                         norm, 1e-6)
+        got = out[:rows].double()
+        assert (out[rows] == 7.0).all()
+    if not done:
+        # (so few values, or so many tiles, that one kernel does)
+        assert (n, k) in ((1040, 512), (8208, 1024), (12304, 256),
+                          (16400, 256)) and torch.equal(residual, old)
+        return
+    assert n <= 16384 and torch.equal(residual[rows], old[rows])
+    want = prod + old[:rows].double()
+    err = 1e-4 * k ** 0.5
+    assert ((residual[:rows].double() - want).abs()
+            <= want.abs() * 2 ** -8 + err).all()
+    inv = (want.square().mean(1, keepdim=True) + 1e-6).rsqrt()
+    want = want * inv * norm.double()
+    err = err * inv * norm.double().abs()
+    if fp8:
+        bound = want.abs() * (2 ** -4 + 2 ** -8) + err + (
+            scales[:rows].double()[:, None] * 2 ** -10)
+    else:
+        bound = want.abs() * 2 ** -8 + err
+    assert ((got - want).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("rows", [128, 129])
 def test_linear_in_parts_of_long_rows(rows):
     """Rows of W too long for 32-bit offsets within a tile (x one row, given
