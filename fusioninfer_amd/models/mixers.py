@@ -103,8 +103,9 @@ from fusioninfer_amd.distributed.layers import (
     MergedColumnParallelLinear,
     ReplicatedLinear,
     RowParallelLinear,
+    unhooked,
 )
-from fusioninfer_amd.ops import linear, seqmix
+from fusioninfer_amd.ops import linear, linear_gelu, seqmix
 
 
 @dataclasses.dataclass
@@ -1147,10 +1148,16 @@ class PlainMLP(nn.Module):
             raise ValueError(f"unsupported activation {act!r}")
         self.ff = ff
         self._act = acts[act]
+        self._gelu = act == "gelu_tanh"
         self.up_proj = ReplicatedLinear(width, ff, dtype=dtype)
         self.down_proj = RowParallelLinear(ff, width, dtype=dtype)
 
     def forward(self, x):
+        if (self._gelu and type(self.up_proj) is ReplicatedLinear
+                and unhooked(self.up_proj)):
+            act = linear_gelu(x, self.up_proj.weight)
+            if act is not None:
+                return self.down_proj(act)
         return self.down_proj(self._act(self.up_proj(x)))
 
 

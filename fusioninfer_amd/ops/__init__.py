@@ -351,6 +351,20 @@ def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return silu_and_mul(linear(x, w))
 
 
+def linear_gelu(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
+    """gelu(x W^T), the tanh form, where a kernel for few rows or many has it
+    in its epilogue; else None. (A pass of its own is a launch of 2.5 us for few
+    rows and 33 us for 7100 of 6144. Four layers with four prompts of 1.8
+    thousand tokens and eight tokens each: 5540 us, and 5410.)"""
+    few = x.dim() == 2 and x.shape[0] <= SKINNY_ROWS
+    if not (_skinny_ok(x, w, 16) if few else _tiles_ok(x, w, 16)):
+        return None
+    out = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype, device=x.device)
+    (_C.few_rows_gemm if few else _C.many_rows_gemm)(out, x, w, None, False,
+                                                     True)
+    return out
+
+
 class StreamRows(NamedTuple):
     """Rows of a residual stream on their way into its norm. scaled [M, K] is
     stream times weight, the columns of squares [parts, 16] add up to the sums

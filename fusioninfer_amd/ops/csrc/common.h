@@ -116,7 +116,7 @@ struct PrefillPlan {
 // squares_in [parts][16]: rows of x are divided by the root mean square that
 // these have as sums of squares of K values. add: the product is added to it,
 // fp32, in place of out; with norm scaled [M, N] gets the sums times norm, and
-// squares_out [N / 16][16] their squares.
+// squares_out [N / 16][16] their squares. gelu: of the product.
 struct SkinnyExtra {
   const float* squares_in = nullptr;
   int parts = 0;
@@ -125,24 +125,31 @@ struct SkinnyExtra {
   const u16* norm = nullptr;
   u16* scaled = nullptr;
   float* squares_out = nullptr;
+  bool gelu = false;
 };
 
-// v / (1 + exp(-v)), the bits of the division (all 2^32 values compared) in
+// v / (1 + e), the bits of the division (all 2^32 values of silu compared) in
 // half its instructions: with one wave per SIMD an epilogue hides none of
 // them. A reciprocal (of a quarter of the divisor, since those below the normal
 // range come out as zero), the quotient, its remainder times the reciprocal
 // added, infinities and NaN put right. (The reciprocal alone, a unit off in
 // the last place, saves 1 % of a GEMM: 24576 x 4096 at 8192 rows 1084 us, and
 // 1095.)
-FI_DEV float silu(float v) {
+FI_DEV float over_one_plus(float v, float e) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  const float e = __expf(-v), d = 1.f + e;
+  const float d = 1.f + e;
   const float r = __builtin_amdgcn_rcpf(fmaf(e, 0.25f, 0.25f)) * 0.25f;
   const float q = v * r;
   return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, v), r, q), d, v);
 #else
   return 0.f;
 #endif
+}
+FI_DEV float silu(float v) { return over_one_plus(v, __expf(-v)); }
+// the tanh form: 0.5 (1 + tanh(a)) is 1 / (1 + exp(-2 a))
+FI_DEV float gelu(float v) {
+  return over_one_plus(
+      v, __expf(-1.5957691216057308f * (v + 0.044715f * v * v * v)));
 }
 
 // pack 8 f32 into 8 OCP-e4m3 bytes (two u32 words) via v_cvt_pk_fp8_f32

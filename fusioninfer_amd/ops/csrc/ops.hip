@@ -59,7 +59,7 @@ void launch_part_gemm_fp8(u16*, float*, const unsigned char*, const float*,
 int64_t tile_gemm_floats(int, int, int);
 double tile_gemm_us(int, int, int);
 void launch_tile_gemm(u16*, float*, const u16*, const u16*, const u16*, int,
-                      int, int, int64_t, int64_t, bool, hipStream_t);
+                      int, int, int64_t, int64_t, bool, bool, hipStream_t);
 void launch_tile_gemm_fp8(u16*, float*, const unsigned char*, const float*,
                           const unsigned char*, const float*, int, int, int,
                           int64_t, int64_t, hipStream_t);
@@ -504,15 +504,19 @@ const u16* check_bias(const c10::optional<at::Tensor>& bias, int64_t N,
   return bf16_cptr(*bias);
 }
 
-// out [M, N] (silu_mul: [M, N / 2]) = x [M, K] @ w [N, K]^T (+ bias)
+// out [M, N] (silu_mul: [M, N / 2]) = x [M, K] @ w [N, K]^T (+ bias); of up to
+// 16 rows its gelu
 void few_rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
-                   c10::optional<at::Tensor> bias, bool silu_mul) {
-  check_few_rows(out, x, w, silu_mul, 256);
+                   c10::optional<at::Tensor> bias, bool silu_mul, bool gelu) {
+  check_few_rows(out, x, w, silu_mul, gelu ? 16 : 256);
+  TORCH_CHECK(!gelu || !(silu_mul || bias.has_value()));
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
   const u16* b = check_bias(bias, N, silu_mul);
   if (M <= 16) {
-    fi::launch_skinny_gemm(bf16_ptr(out), bf16_cptr(x), bf16_cptr(w), b, {}, M,
-                           N, K, x.stride(0), out.stride(0), silu_mul,
+    fi::SkinnyExtra extra;
+    extra.gelu = gelu;
+    fi::launch_skinny_gemm(bf16_ptr(out), bf16_cptr(x), bf16_cptr(w), b, extra,
+                           M, N, K, x.stride(0), out.stride(0), silu_mul,
                            current_stream());
     return;
   }
@@ -609,7 +613,8 @@ void stream_begin(at::Tensor stream, at::Tensor scaled, at::Tensor squares,
 
 // the same for more rows, by tiles of 256 x 256
 void many_rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
-                    c10::optional<at::Tensor> bias, bool silu_mul) {
+                    c10::optional<at::Tensor> bias, bool silu_mul, bool gelu) {
+  TORCH_CHECK(!gelu || !(silu_mul || bias.has_value()));
   CHECK_BF16_CUDA(out);
   CHECK_BF16_CUDA(x);
   CHECK_BF16_CUDA(w);
@@ -639,7 +644,7 @@ void many_rows_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
                                 x.options().dtype(at::kFloat));
   fi::launch_tile_gemm(bf16_ptr(out), pieces.data_ptr<float>(), bf16_cptr(x),
                        bf16_cptr(w), b, M, N, K, x.stride(0), out.stride(0),
-                       silu_mul, current_stream());
+                       silu_mul, gelu, current_stream());
 }
 
 void check_few_rows_fp8(const at::Tensor& x, const at::Tensor& x_scales,
@@ -800,7 +805,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("reshape_and_cache", &reshape_and_cache, "scatter K/V into paged cache");
   m.def("gather_kv_blocks", &gather_kv_blocks, "pack KV blocks for PD send");
   m.def("scatter_kv_blocks", &scatter_kv_blocks, "unpack KV blocks from PD recv");
-  m.def("few_rows_gemm", &few_rows_gemm, "x W^T for up to 256 rows of x");
+  m.def("few_rows_gemm", &few_rows_gemm, "x W^T for up to 256 rows of x",
+        py::arg("out"), py::arg("x"), py::arg("w"), py::arg("bias"),
+        py::arg("silu_mul"), py::arg("gelu") = false);
   m.def("few_rows_scaled_gemm", &few_rows_scaled_gemm,
         "linear layer of up to 16 rows over their root mean square");
   m.def("few_rows_gemm_add", &few_rows_gemm_add,
@@ -808,7 +815,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("stream_begin", &stream_begin, "fp32 stream of rows, the next norm");
   m.def("few_rows_gemm_us", &fi::part_gemm_us,
         "estimate for M of 17 to 256 rows, N, K of 16-bit values");
-  m.def("many_rows_gemm", &many_rows_gemm, "x W^T by tiles of 256 x 256");
+  m.def("many_rows_gemm", &many_rows_gemm, "x W^T by tiles of 256 x 256",
+        py::arg("out"), py::arg("x"), py::arg("w"), py::arg("bias"),
+        py::arg("silu_mul"), py::arg("gelu") = false);
   m.def("many_rows_gemm_us", &fi::tile_gemm_us,
         "estimate for M, N, bytes of a row of K");
   m.def("many_rows_gemm_fp8", &many_rows_gemm_fp8,

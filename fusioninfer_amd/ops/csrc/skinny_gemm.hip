@@ -58,7 +58,7 @@ FI_DEV void wait_vm() {
 }
 
 // what becomes of the product
-enum { PLAIN, SCALED, ADD };
+enum { PLAIN, SCALED, ADD, GELU };
 
 FI_DEV void sync_waves() {
   __builtin_amdgcn_s_barrier();
@@ -298,6 +298,8 @@ void skinny_gemm_kernel(void* __restrict__ out_p, const u16* __restrict__ x,
           float v = sum[0][r];
           if (SILU_MUL)
             v = v / (1.f + __expf(-v)) * sum[1][r];
+          else if (MODE == GELU)
+            v = gelu(v);
           else if (bias)
             v += bf16_to_f32(bias[n + r]);
           o.h[r] = f32_to_bf16(v);
@@ -356,6 +358,9 @@ void launch_skinny_gemm(u16* out, const u16* x, const u16* w, const u16* bias,
   } else if (extra.add != nullptr) {
     if (wide) FI_SK_WIDE(false, ADD);
     else FI_SK_NARROW(ADD);
+  } else if (extra.gelu) {
+    if (wide) FI_SK_WIDE(false, GELU);
+    else FI_SK_NARROW(GELU);
   } else {
     if (silu_mul) FI_SK_WIDE(true, PLAIN);
     else if (wide) FI_SK_WIDE(false, PLAIN);

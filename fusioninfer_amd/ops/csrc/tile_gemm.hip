@@ -45,7 +45,8 @@
 // leave the chip idle, 4099 rows, 4096 x 12288: 270 (1.53) and 151 (2.73).
 //
 // SILU_MUL: the first half of a tile's W rows are gate rows and the second
-// the up rows that go with them; a wave holds both.
+// the up rows that go with them; a wave holds both. GELU: of the fp32 sums; a
+// pass over 7100 rows of 6144 that took 33 us beside a product of 150.
 
 #include <type_traits>
 
@@ -125,8 +126,8 @@ struct Kind<true> {
   }
 };
 
-// what becomes of the products: nothing, + bias, silu(gate) * up
-enum { PLAIN, BIAS, SILU };
+// what becomes of the products: nothing, + bias, silu(gate) * up, gelu
+enum { PLAIN, BIAS, SILU, GELU };
 
 // eight outputs of a row of x: sums a, b; SILU: of gate values, the up values
 // that go with them in u, v. FP8: times xs, the row's scale, and the scales
@@ -146,6 +147,7 @@ FI_DEV void store8(u16* to, const u16* bias, floatx4 a, floatx4 b,
     float y = r < 4 ? a[r] : b[r - 4];
     if (MODE == SILU)
       y = silu(y) * (r < 4 ? u[r] : v[r - 4]);
+    if (MODE == GELU) y = gelu(y);
     if (MODE == BIAS) y += bf16_to_f32(add.h[r]);
     o.h[r] = f32_to_bf16(y);
   }
@@ -582,8 +584,12 @@ int64_t tile_gemm_floats(int M, int N, int KB) {
 // K a multiple of 64 and 128 at least, N of 16 (32 with silu_mul)
 void launch_tile_gemm(u16* out, float* pieces, const u16* x, const u16* w,
                       const u16* bias, int M, int N, int K, int64_t x_stride,
-                      int64_t out_stride, bool silu_mul, hipStream_t stream) {
-  if (silu_mul)
+                      int64_t out_stride, bool silu_mul, bool gelu,
+                      hipStream_t stream) {
+  if (gelu)
+    launch<GELU, false>(out, pieces, x, w, bias, nullptr, nullptr, M, N, K,
+                        x_stride, out_stride, stream);
+  else if (silu_mul)
     launch<SILU, false>(out, pieces, x, w, bias, nullptr, nullptr, M, N, K,
                         x_stride, out_stride, stream);
   else if (bias)

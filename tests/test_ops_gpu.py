@@ -1400,6 +1400,35 @@ def test_linear_in_parts_and_norm(rows, n, k, fp8):
     assert ((got - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("rows,n,k", [
+    (1, 6144, 2048), (4, 16, 128), (5, 2064, 384), (8, 6176, 384),
+    (9, 24640, 256), (16, 1040, 1152),
+    (257, 528, 256),       # a tile and a row, the last columns of a tile
+    (300, 4096, 2048),     # tiles in pieces
+    (2304, 8192, 320),     # whole rounds and a rest
+])
+def test_linear_gelu(rows, n, k):
+    """The tanh form of gelu of a product against float64: its slope is below
+    1.13, the product's sums are fp32, the result has one rounding to bf16."""
+    g = torch.Generator().manual_seed(n + k + rows)
+    w, x = (torch.full((m + 256, k), float("nan"), dtype=torch.bfloat16,
+                       device=DEV) for m in (n, rows))
+    w[:n] = torch.randn(n, k, generator=g) * k ** -0.5 * 3
+    x[:rows] = torch.randn(rows, k, generator=g)
+    w, x = w[:n], x[:rows]
+    out = torch.full((rows + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+    kernel = ops._C.few_rows_gemm if rows <= 16 else ops._C.many_rows_gemm
+    kernel(out[:rows], x, w, None, False, True)
+    want = torch.nn.functional.gelu(x.double() @ w.double().T,
+                                    approximate="tanh")
+    assert ((out[:rows].double() - want).abs()
+            <= want.abs() * 2 ** -8 + 1e-4).all()
+    assert (out[rows] == 7.0).all()
+    taken = ops.linear_gelu(x, w)
+    assert taken is None or torch.equal(taken, out[:rows])
+    assert taken is not None or rows > 16
+
+
 @pytest.mark.parametrize("rows", [128, 129])
 def test_linear_in_parts_of_long_rows(rows):
     """Rows of W too long for 32-bit offsets within a tile (x one row, given
