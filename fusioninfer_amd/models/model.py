@@ -561,10 +561,12 @@ class MoEMLP(nn.Module):
         n_valid = tile_cum[-1:].int()
         return sorted_ids[:PM].contiguous(), expert_ids, n_valid, pos, PM
 
-    def _forward_grouped(self, x: torch.Tensor) -> torch.Tensor:
+    def _forward_grouped(self, x: torch.Tensor, norm=None):
         """GPU path: hand-written grouped MFMA GEMM over block-aligned
         expert segments with fused SwiGLU, then a deterministic weighted
-        combine. No host syncs — MoE decode is hipGraph-capturable."""
+        combine. No host syncs — MoE decode is hipGraph-capturable.
+        norm: (residual, weight, eps) of the norm behind, where nothing is to
+        be summed over ranks; gives (rows, residual)."""
         T, H = x.shape
         E_local = self.e_end - self.e_start
         if x.is_cuda:
@@ -587,8 +589,11 @@ class MoEMLP(nn.Module):
         y = torch.empty(PM, H, dtype=x.dtype, device=x.device)
         ops.moe_gemm(y, act, dn_packed, sorted_ids, expert_ids, n_valid,
                      block_m, gate_up=False)
+        topv = topv.reshape(-1).float().contiguous()
+        if norm is not None:
+            return ops.moe_combine_norm(y, pos, topv, *norm)
         out = torch.empty(T, H, dtype=x.dtype, device=x.device)
-        ops.moe_combine(out, y, pos, topv.reshape(-1).float().contiguous())
+        ops.moe_combine(out, y, pos, topv)
         return ps.tp_all_reduce(out)
 
     def forward(self, x: torch.Tensor, lora=None) -> torch.Tensor:
@@ -728,6 +733,12 @@ class DecoderLayer(nn.Module):
                 and meta.lora is None and unhooked(self.mlp)):
             x, residual = add_norm(self.mlp.down_proj, self.mlp.activation(x),
                                    residual, norm_behind, self.eps, self.fp8)
+            return ops.NormedRows(x), residual
+        if (norm_behind is not None and type(self.mlp) is MoEMLP
+                and not self.fp8 and x.is_cuda and ps.tp_world_size() == 1
+                and unhooked(self.mlp)):
+            x, residual = self.mlp._forward_grouped(
+                x, (residual, norm_behind, self.eps))
             return ops.NormedRows(x), residual
         return (self.mlp(x) if self.fp8
                 else self.mlp(x, lora=meta.lora)), residual

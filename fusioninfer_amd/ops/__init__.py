@@ -1049,4 +1049,22 @@ def moe_combine(out, y, pos, w):
     return ref.moe_combine(out, y, pos, w)
 
 
+def moe_combine_norm(y, pos, w, residual, weight, eps: float):
+    """residual += the rows of moe_combine and the norm behind that, in one
+    pass: (rows, residual)."""
+    T, H = residual.shape
+    if (residual.dtype == y.dtype == weight.dtype == torch.bfloat16
+            and H % 8 == 0 and H <= 8192 and y.is_contiguous()
+            and residual.is_contiguous() and weight.is_contiguous()
+            and residual.is_cuda
+            and (residual.data_ptr() | weight.data_ptr() | y.data_ptr()) % 16
+            == 0):
+        out = torch.empty_like(residual)
+        _moe_native().moe_combine_norm(out, residual, weight, eps, y, pos, w)
+        return out, residual
+    out = torch.empty((T, H), dtype=y.dtype, device=y.device)
+    return fused_add_rms_norm(moe_combine(out, y, pos, w), residual, weight,
+                              eps)
+
+
 compute_cos_sin_cache = ref.compute_cos_sin_cache

@@ -34,6 +34,9 @@ void launch_moe_router_topk(const float*, float*, int*, int, int, int,
                             bool, hipStream_t);
 void launch_moe_route(const float*, float*, int*, int, int, int, bool, bool,
                       float, hipStream_t);
+void launch_moe_combine_norm(u16*, u16*, const u16*, float, const u16*,
+                             const int*, const float*, int, int, int,
+                             hipStream_t);
 template <typename A>
 void launch_moe_combine(A*, const A*, const int*, const float*, int, int,
                         int, hipStream_t);
@@ -162,6 +165,33 @@ void moe_combine(at::Tensor out, at::Tensor y, at::Tensor pos, at::Tensor w) {
     fi::launch_moe_combine<float>(out.data_ptr<float>(), y.data_ptr<float>(),
                                   pos.data_ptr<int>(), w.data_ptr<float>(), T,
                                   topk, H, current_stream());
+}
+
+// residual [T, H] += the combined rows, out = its rms norm times norm
+void moe_combine_norm(at::Tensor out, at::Tensor residual, at::Tensor norm,
+                      double eps, at::Tensor y, at::Tensor pos, at::Tensor w) {
+  for (const at::Tensor& t : {out, residual, norm, y})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::kBFloat16 &&
+                t.is_contiguous() &&
+                reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0);
+  TORCH_CHECK(pos.is_cuda() && pos.scalar_type() == at::kInt &&
+              pos.is_contiguous());
+  TORCH_CHECK(w.is_cuda() && w.scalar_type() == at::kFloat &&
+              w.is_contiguous());
+  TORCH_CHECK(out.dim() == 2 && y.dim() == 2 &&
+              out.sizes() == residual.sizes());
+  const int T = out.size(0), H = out.size(1);
+  TORCH_CHECK(y.size(1) == H && norm.numel() == H && H > 0 && H % 8 == 0 &&
+                  H <= 8192,
+              "moe_combine_norm: unsupported sizes");
+  if (T == 0) return;
+  const int topk = pos.numel() / T;
+  TORCH_CHECK(pos.numel() == T * topk && w.numel() == T * topk);
+  fi::launch_moe_combine_norm(bf16_ptr(out), bf16_ptr(residual),
+                              bf16_cptr(norm), static_cast<float>(eps),
+                              bf16_cptr(y), pos.data_ptr<int>(),
+                              w.data_ptr<float>(), T, topk, H,
+                              current_stream());
 }
 
 void moe_gemm_plain(at::Tensor out, at::Tensor a, at::Tensor w,
@@ -342,6 +372,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "epilogue (gate_up=true fuses SwiGLU)");
   m.def("moe_gemm_plain", &moe_gemm_plain,
         "grouped GEMM for any sizes, bf16 or fp32 operands");
+  m.def("moe_combine_norm", &moe_combine_norm,
+        "weighted sum of expert rows, residual and norm");
   m.def("moe_combine", &moe_combine,
         "weighted top-k combine of expert outputs (deterministic)");
   m.def("moe_align", &moe_align,

@@ -416,7 +416,94 @@ __global__ __launch_bounds__(256) void moe_combine_vec_kernel(
   *reinterpret_cast<Vec*>(out + static_cast<int64_t>(t) * H + c) = o;
 }
 
+// The same of bf16 rows with the residual added and the norm behind that: a
+// workgroup has a token, the sums stay fp32 until the norm. Bound by memory
+// like the one above, and two passes less over the tokens. (Four layers: 8765
+// tokens 5260 -> 5222 us, 64 tokens 1332 -> 1320; the norm alone takes 25 and 2.7
+// us a layer.)
+template <int ITERS>
+__global__ __launch_bounds__(256) void moe_combine_norm_kernel(
+    u16* __restrict__ out, u16* __restrict__ residual,
+    const u16* __restrict__ norm, const float eps, const u16* __restrict__ y,
+    const int* __restrict__ pos, const float* __restrict__ w, const int topk,
+    const int H) {
+  constexpr int kAhead = 8;
+  const int t = blockIdx.x;
+  const int64_t row = static_cast<int64_t>(t) * H;
+  float acc[ITERS][8];
+  bf16x8 g[ITERS];
+  float squares = 0.f;
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int c = (it * 256 + static_cast<int>(threadIdx.x)) * 8;
+    if (c < H) {
+      const bf16x8 old = *reinterpret_cast<const bf16x8*>(residual + row + c);
+      g[it] = *reinterpret_cast<const bf16x8*>(norm + c);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[it][j] = 0.f;
+      for (int k0 = 0; k0 < topk; k0 += kAhead) {
+        bf16x8 r[kAhead];
+        float wk[kAhead];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+          const int k = k0 + i;
+          const int p = k < topk ? pos[t * topk + k] : -1;
+          wk[i] = 0.f;
+          r[i] = bf16x8{};
+          if (p >= 0) {
+            wk[i] = w[t * topk + k];
+            r[i] = *reinterpret_cast<const bf16x8*>(
+                y + static_cast<int64_t>(p) * H + c);
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i)
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            acc[it][j] += wk[i] * bf16_to_f32(r[i].h[j]);
+      }
+      bf16x8 sum;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        acc[it][j] += bf16_to_f32(old.h[j]);
+        squares = fmaf(acc[it][j], acc[it][j], squares);
+        sum.h[j] = f32_to_bf16(acc[it][j]);
+      }
+      *reinterpret_cast<bf16x8*>(residual + row + c) = sum;
+    }
+  }
+  __shared__ float scratch[4];
+  squares = block_reduce_sum<4>(wave_reduce_sum(squares), scratch);
+  const float inv_rms = rsqrtf(squares / H + eps);
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int c = (it * 256 + static_cast<int>(threadIdx.x)) * 8;
+    if (c < H) {
+      bf16x8 o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        o.h[j] =
+            f32_to_bf16(acc[it][j] * inv_rms * bf16_to_f32(g[it].h[j]));
+      *reinterpret_cast<bf16x8*>(out + row + c) = o;
+    }
+  }
+}
+
 }  // namespace
+
+// H a multiple of 8, up to 8192
+void launch_moe_combine_norm(u16* out, u16* residual, const u16* norm,
+                             float eps, const u16* y, const int* pos,
+                             const float* w, int tokens, int topk, int H,
+                             hipStream_t stream) {
+#define FI_CN(ITERS)                                                          \
+  hipLaunchKernelGGL(moe_combine_norm_kernel<ITERS>, dim3(tokens), dim3(256), \
+                     0, stream, out, residual, norm, eps, y, pos, w, topk, H)
+  if (H <= 2048) FI_CN(1);
+  else if (H <= 4096) FI_CN(2);
+  else FI_CN(4);
+#undef FI_CN
+}
 
 void launch_moe_route(const float* logits, float* topv, int* topi, int T,
                       int E, int k, bool sigmoid, bool renorm, float scale,

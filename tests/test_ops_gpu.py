@@ -1157,6 +1157,38 @@ def test_moe_combine_widths(T, top, H, dtype):
     assert (err <= want.abs() * half + 1e-5).all()
 
 
+@pytest.mark.parametrize("T,top,H", [(1, 1, 8), (3, 8, 2048), (64, 9, 2056),
+                                     (5, 4, 4096), (2, 16, 8192),
+                                     (300, 8, 264), (4, 2, 8200)])
+def test_moe_combine_norm(T, top, H):
+    """The combined rows, the residual and the norm behind: fp32 sums of top
+    products and one rounding to bf16 each (2^-9 relative)."""
+    g = torch.Generator().manual_seed(T + top + H)
+    y = torch.randn(T * top + 5, H, generator=g).to(torch.bfloat16)
+    pos = torch.randperm(T * top + 5, generator=g)[: T * top].int()
+    pos[::7] = -1
+    w = torch.rand(T * top, generator=g)
+    old = torch.randn(T, H, generator=g).to(torch.bfloat16)
+    norm = torch.randn(H, generator=g).to(torch.bfloat16)
+    rows = y.double()[pos.clamp(min=0).long()] * (pos >= 0).double()[:, None]
+    combined = (rows * w.double()[:, None]).view(T, top, H).sum(1)
+    want = combined + old.double()
+    out, res = ops.moe_combine_norm(y.to(DEV), pos.to(DEV), w.to(DEV),
+                                    old.to(DEV), norm.to(DEV), 1e-6)
+    # wider rows go through two kernels: the combined ones are rounded
+    # between, by 2^-9 of themselves, which the sum with the residual keeps
+    err = (top + 1) * 2 ** -21 + (0 if H <= 8192
+                                  else combined.abs() * 2 ** -9)
+    assert ((res.cpu().double() - want).abs()
+            <= want.abs() * 2 ** -8 + 2 * err).all()
+    inv = (want.square().mean(1, keepdim=True) + 1e-6).rsqrt()
+    want = want * inv * norm.double()
+    assert ((out.cpu().double() - want).abs()
+            <= want.abs() * 2 ** -8 + 2 * err * inv * norm.double().abs()
+            ).all()
+
+
+
 # ------------------------------------------------------------ skinny GEMM
 
 
