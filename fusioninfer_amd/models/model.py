@@ -88,33 +88,38 @@ class Attention(nn.Module):
         be the rows of a residual stream: the result is added to it, and its
         rows before the norm of norm_behind come back."""
         stream = x if isinstance(x, ops.StreamRows) else None
-        if stream is not None:
-            qkv = ops.stream_linear(x, self.qkv_proj.weight,
-                                    self.qkv_proj.bias)
-        else:
-            qkv = self.qkv_proj(x)
-        if meta.lora is not None:
-            meta.lora.apply(self.layer_idx, "qkv", x, qkv)
-        q = qkv[:, : self.q_size]
-        k = qkv[:, self.q_size : self.q_size + self.kv_size]
-        v = qkv[:, self.q_size + self.kv_size :]
         k_cache, v_cache = kv_cache
         fp8_kv = k_cache.dtype == torch.float8_e4m3fn
         ks = self.k_scale if fp8_kv else 1.0
         vs = self.v_scale if fp8_kv else 1.0
-        ops.rope_qk_norm_cache_(
-            q, k, v, meta.positions, cos_sin, k_cache, v_cache,
-            meta.slot_mapping, self.num_heads, self.q_norm_weight,
-            self.k_norm_weight, self.eps, 1.0 / ks, 1.0 / vs,
-        )
+        rope = (meta.positions, cos_sin, k_cache, v_cache, meta.slot_mapping,
+                self.num_heads, self.q_norm_weight, self.k_norm_weight,
+                self.eps, 1.0 / ks, 1.0 / vs)
+        q = None
+        if (stream is None and meta.lora is None and not self.fp8 and x.is_cuda
+                and weight_alone(self.qkv_proj, bias=True)):
+            q = ops.linear_rope_qk_norm_cache(
+                x, self.qkv_proj.weight, self.qkv_proj.bias, *rope)
+        if q is None:
+            if stream is not None:
+                qkv = ops.stream_linear(x, self.qkv_proj.weight,
+                                        self.qkv_proj.bias)
+            else:
+                qkv = self.qkv_proj(x)
+            if meta.lora is not None:
+                meta.lora.apply(self.layer_idx, "qkv", x, qkv)
+            q = qkv[:, : self.q_size]
+            ops.rope_qk_norm_cache_(
+                q, qkv[:, self.q_size : self.q_size + self.kv_size],
+                qkv[:, self.q_size + self.kv_size :], *rope)
         # K's dequant scale folds EXACTLY into the softmax scalar:
         # scale*(Q . ks*K8) == (scale*ks)*(Q . K8); V's is a linear
         # post-multiply on the attention output (applied below).
         scale = self.scale * ks
 
-        T = qkv.shape[0]
+        T = q.shape[0]
         np_, nd = meta.num_prefill_tokens, meta.num_decode_tokens
-        out = torch.empty(T, self.q_size, dtype=qkv.dtype, device=qkv.device)
+        out = torch.empty(T, self.q_size, dtype=q.dtype, device=q.device)
         if np_ > 0:
             # context attention over the paged cache (the new tokens' K/V
             # were just written above); cached prefixes are never recomputed

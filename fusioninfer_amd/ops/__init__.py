@@ -612,6 +612,33 @@ def rope_qk_norm_cache_(q, k, v, positions, cos_sin, k_cache, v_cache,
     return q
 
 
+def linear_rope_qk_norm_cache(x, w, bias, positions, cos_sin, k_cache, v_cache,
+                              slot_mapping, num_q_heads: int,
+                              q_weight: Optional[torch.Tensor] = None,
+                              k_weight: Optional[torch.Tensor] = None,
+                              eps: float = 1e-6, k_inv_scale: float = 1.0,
+                              v_inv_scale: float = 1.0):
+    """rope_qk_norm_cache_ of linear(x, w, bias)'s queries, keys and values
+    [T, (Hq | Hk | Hk) * D], where one kernel sums the pieces of 17 to 128 rows'
+    product and goes on; else None. Returns q. (us, product and rope apart and
+    so, 6144 x 4096 at 20, 43, 64 and 128 rows: 17.9, 20.2, 21.2, 28.6 and 17.7,
+    19.8, 20.8, 27.5; from there on the way of the pieces takes what the launch
+    did, 33.1 and 33.6 at 256. A prompt of 43 tokens, whose launches the host
+    does not keep up with: 1029 and 1017.)"""
+    if not (SKINNY_ROWS < x.shape[0] <= 128
+            and _skinny_ok(x, w, 16, bias=bias)
+            and k_cache.shape[3] in (64, 128)
+            and w.shape[0] == (num_q_heads + 2 * k_cache.shape[1])
+            * k_cache.shape[3]):
+        return None
+    q = torch.empty((x.shape[0], num_q_heads * k_cache.shape[3]),
+                    dtype=x.dtype, device=x.device)
+    return q if _C.few_rows_gemm_rope(
+        q, x, w, bias, q_weight, k_weight, cos_sin, positions, k_cache,
+        v_cache, slot_mapping, num_q_heads, eps, k_inv_scale, v_inv_scale,
+    ) else None
+
+
 # ---------------------------------------------------------------- kv cache
 
 def reshape_and_cache(k, v, k_cache, v_cache, slot_mapping,

@@ -112,6 +112,23 @@ struct PrefillPlan {
   bool split, pair;
 };
 
+// Heads of a projection's rows that are normed per head, rotated and kept in the
+// paged cache [num_blocks, Hk, block_size, head_dim].
+struct RopeArgs {
+  const u16* q_weight;    // [head_dim] or nullptr
+  const u16* k_weight;
+  const float* cos_sin;   // [P, head_dim], cos | sin
+  const int* positions;   // [T]
+  int num_q_heads, num_kv_heads, head_dim;
+  float eps;
+  void* k_cache;
+  void* v_cache;
+  const int* slots;       // [T], negative: the row is not kept
+  int block_size;
+  bool fp8;
+  float k_inv_scale, v_inv_scale;
+};
+
 // What the kernel for few rows does beside out = x W^T, by what is not null.
 // squares_in [parts][16]: rows of x are divided by the root mean square that
 // these have as sums of squares of K values. add: the product is added to it,

@@ -51,6 +51,9 @@ double part_gemm_us(int, int, int);
 bool launch_part_gemm_norm(void*, float*, u16*, const u16*, float, float*,
                            const u16*, const float*, const u16*, const float*,
                            int, int, int, int64_t, hipStream_t);
+bool launch_part_gemm_rope(u16*, const RopeArgs&, const u16*, float*,
+                           const u16*, const u16*, int, int, int, int64_t,
+                           hipStream_t);
 void launch_part_gemm(u16*, float*, const u16*, const u16*, const u16*, int,
                       int, int, int64_t, int64_t, bool, hipStream_t);
 void launch_part_gemm_fp8(u16*, float*, const unsigned char*, const float*,
@@ -688,6 +691,67 @@ void few_rows_gemm_fp8(at::Tensor out, at::Tensor x, at::Tensor x_scales,
       current_stream());
 }
 
+// (x [M, K] @ w [N, K]^T + bias) as heads: queries normed and rotated to q [M,
+// num_q_heads * D], K and V rows to the cache; false, with nothing done, where
+// the kernels for that are not chosen
+bool few_rows_gemm_rope(at::Tensor q, at::Tensor x, at::Tensor w,
+                        c10::optional<at::Tensor> bias,
+                        c10::optional<at::Tensor> q_weight,
+                        c10::optional<at::Tensor> k_weight,
+                        at::Tensor cos_sin, at::Tensor positions,
+                        at::Tensor k_cache, at::Tensor v_cache,
+                        at::Tensor slot_mapping, int64_t num_q_heads,
+                        double eps, double k_inv_scale, double v_inv_scale) {
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  const int64_t Hk = k_cache.size(1), D = k_cache.size(3);
+  CHECK_BF16_CUDA(q);
+  CHECK_BF16_CUDA(x);
+  CHECK_BF16_CUDA(w);
+  const bool fp8 = cache_is_fp8(k_cache);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && M >= 1 && M <= 256 &&
+              w.size(1) == K && K > 0 && K % 128 == 0 && K <= (1 << 24) &&
+              N > 0 && N % 16 == 0 && N <= (1 << 24) && x.stride(1) == 1 &&
+              x.stride(0) % 8 == 0 && x.stride(0) <= (1 << 22) &&
+              w.is_contiguous() &&
+              reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0);
+  TORCH_CHECK((D == 64 || D == 128) && num_q_heads >= 1 &&
+              N == (num_q_heads + 2 * Hk) * D && q.dim() == 2 &&
+              q.size(0) == M && q.size(1) == num_q_heads * D &&
+              q.is_contiguous());
+  TORCH_CHECK(cos_sin.scalar_type() == at::kFloat && cos_sin.is_cuda() &&
+              cos_sin.size(-1) == D && positions.is_cuda() &&
+              positions.scalar_type() == at::kInt && positions.numel() >= M &&
+              slot_mapping.is_cuda() &&
+              slot_mapping.scalar_type() == at::kInt &&
+              slot_mapping.numel() >= M);
+  TORCH_CHECK(k_cache.is_contiguous() && v_cache.is_contiguous() &&
+              v_cache.sizes() == k_cache.sizes() &&
+              v_cache.scalar_type() == k_cache.scalar_type());
+  for (const auto& t : {q_weight, k_weight})
+    TORCH_CHECK(!t || (t->is_cuda() && t->scalar_type() == at::kBFloat16 &&
+                       t->is_contiguous() && t->numel() == D));
+  fi::RopeArgs rope{
+      q_weight ? bf16_cptr(*q_weight) : nullptr,
+      k_weight ? bf16_cptr(*k_weight) : nullptr,
+      cos_sin.data_ptr<float>(), positions.data_ptr<int>(),
+      static_cast<int>(num_q_heads), static_cast<int>(Hk),
+      static_cast<int>(D), static_cast<float>(eps), k_cache.data_ptr(),
+      v_cache.data_ptr(), slot_mapping.data_ptr<int>(),
+      static_cast<int>(k_cache.size(2)), fp8,
+      static_cast<float>(k_inv_scale), static_cast<float>(v_inv_scale)};
+  const u16* b = check_bias(bias, N, false);
+  const auto run = [&](float* pieces) {
+    return M > 16 && fi::launch_part_gemm_rope(
+                         bf16_ptr(q), rope, b, pieces, bf16_cptr(x),
+                         bf16_cptr(w), M, N, K, x.stride(0), current_stream());
+  };
+  if (!run(nullptr)) return false;
+  at::Tensor pieces = at::empty({fi::part_gemm_floats(M, N, K, false)},
+                                x.options().dtype(at::kFloat));
+  return run(pieces.data_ptr<float>());
+}
+
 void check_norm(const at::Tensor& out, const at::Tensor& residual,
                 const at::Tensor& norm, int64_t M, int64_t N) {
   CHECK_BF16_CUDA(residual);
@@ -822,6 +886,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "estimate for M, N, bytes of a row of K");
   m.def("many_rows_gemm_fp8", &many_rows_gemm_fp8,
         "x W^T by tiles of 256 x 256, e4m3 with scales per row");
+  m.def("few_rows_gemm_rope", &few_rows_gemm_rope,
+        "heads of x W^T to q and the cache, or false");
   m.def("few_rows_gemm_norm", &few_rows_gemm_norm,
         "residual += x W^T and its norm, or false");
   m.def("few_rows_gemm_norm_fp8", &few_rows_gemm_norm_fp8,

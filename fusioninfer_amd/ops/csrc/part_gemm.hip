@@ -53,9 +53,13 @@
 
 #include <type_traits>
 
+#include "pieces.h"
 #include "tile_engine.h"
 
 namespace fi {
+
+void launch_rope_of_pieces(u16*, const PieceRows&, const RopeArgs&, int,
+                           hipStream_t);
 
 namespace {
 
@@ -63,19 +67,6 @@ template <int N>
 FI_DEV void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
-
-// parts of `total` units of `unit` stages over `n` workgroups
-struct Cut {
-  int per, rem, unit;
-  FI_DEV Cut(int total, int n, int unit)
-      : per(total / n), rem(total % n), unit(unit) {}
-  FI_DEV int start(int i) const { return (i * per + min(i, rem)) * unit; }
-  // the part that holds a stage (unit 1)
-  FI_DEV int holder(int stage) const {
-    const int wide = rem * (per + 1);
-    return stage < wide ? stage / (per + 1) : rem + (stage - wide) / per;
-  }
-};
 
 // at most `stages` stages of L DMAs each of this wave are still on the way
 template <int L, int MAX>
@@ -692,30 +683,19 @@ void part_gemm_join_kernel(u16* __restrict__ out,
 }
 
 // The second kernel where a norm follows: a workgroup sums a row's pieces, adds
-// the residual, writes it back and leaves the normed row, as bf16 or (OUT8)
-// as e4m3 with the row's scale. Bound by the way of the pieces through memory,
-// all of a thread's on their way at once; 256 rows of 4096 take 7.8 us, the sum
-// of pieces alone 6.8 and the norm 4.4. Every tile is in pieces, none of which is more
-// than a tile long: the first piece of a tile is its part's start of one, the
-// others are ends.
-template <class S, bool FP8, bool OUT8, int THREADS, int ITERS>
+// the residual, writes it back and leaves the normed row, as bf16 or (FP8) as
+// e4m3 with the row's scale. Bound by the way of the pieces through memory,
+// all of a thread's on their way at once; 256 rows of 4096 take 7.8 us,
+// the sum of pieces alone 6.8 and the norm 4.4.
+template <bool FP8, int THREADS, int ITERS>
 __global__ __launch_bounds__(THREADS)
 void part_gemm_norm_kernel(void* __restrict__ out, float* __restrict__ out_scales,
-                           const floatx4* __restrict__ pieces,
-                           u16* __restrict__ residual,
+                           const PieceRows pieces, u16* __restrict__ residual,
                            const u16* __restrict__ norm, const float eps,
-                           const Scales scales, const int M, const int N,
-                           const int K, const int tiles, const int parts) {
-  const int SK = K / S::KS;
-  const Cut cut(tiles * SK, parts, 1);
-  // two rows that share the lines of the pieces go to the same XCD, whose turn
-  // comes every eight workgroups
-  const int xcd = blockIdx.x % 8, turn = blockIdx.x / 8;
-  const int m = S::kAhead ? (turn / 2 * 8 + xcd) * 2 + turn % 2
-                          : static_cast<int>(blockIdx.x);
+                           const Scales scales, const int M, const int N) {
+  const int m = piece_row(pieces.columns);
   if (m >= M) return;
   const int64_t row = static_cast<int64_t>(m) * N;
-  const BufferRsrc from = buffer_of(pieces, parts * 2 * S::kPiece * 16u);
   floatx4 v[ITERS];
   bf16x4 weight[ITERS];
   float squares = 0.f;
@@ -726,21 +706,12 @@ void part_gemm_norm_kernel(void* __restrict__ out, float* __restrict__ out_scale
     if (n < N) {
       weight[it] = *reinterpret_cast<const bf16x4*>(norm + n);
       const bf16x4 r = *reinterpret_cast<const bf16x4*>(residual + row + n);
-      const int tile = n / S::TN;
-      const int first = cut.holder(tile * SK);
-      const int last = cut.holder(tile * SK + SK - 1);
-      const int of = n % S::TN;        // the tile's column
-      const u32 at = S::kAhead ? (of / 16 * S::MB + m) * 64 + of % 16 * 4
-                               : (m * S::TN + of) * 4;
       constexpr int kAtOnce = 8;
-      for (int q = first; q <= last; q += kAtOnce) {
+      for (PieceReader p(pieces, m, n); p.next <= p.last; p.next += kAtOnce) {
         floatx4 got[kAtOnce];
 #pragma unroll
-        for (int i = 0; i < kAtOnce; ++i)   // beyond the last: zeros, no fetch
-          got[i] = __builtin_bit_cast(floatx4, buffer_load16(
-              from, q + i > last ? ~0u
-                                 : at + ((q + i) * 2 + (q + i == first)) *
-                                            (S::kPiece * 16u), 0));
+        for (int i = 0; i < kAtOnce; ++i)
+          got[i] = __builtin_bit_cast(floatx4, p.get(i, 0));
 #pragma unroll
         for (int i = 0; i < kAtOnce; ++i) v[it] += got[i];
       }
@@ -769,14 +740,14 @@ void part_gemm_norm_kernel(void* __restrict__ out, float* __restrict__ out_scale
       v[it][j] *= inv_rms * bf16_to_f32(weight[it].h[j]);
       most = fmaxf(most, fabsf(v[it][j]));
     }
-    if (!OUT8) {
+    if (!FP8) {
       bf16x4 o;
 #pragma unroll
       for (int j = 0; j < 4; ++j) o.h[j] = f32_to_bf16(v[it][j]);
       *reinterpret_cast<bf16x4*>(static_cast<u16*>(out) + row + n) = o;
     }
   }
-  if (!OUT8) return;
+  if (!FP8) return;
   most = block_reduce_max<THREADS / kWaveSize>(wave_reduce_max(most),
                                                scratch[1]);
   const float scale = fmaxf(most, 1e-8f) / 448.0f, inv = 1.f / scale;
@@ -1001,37 +972,27 @@ void launch_part_gemm_fp8(u16* out, float* pieces, const unsigned char* x,
   });
 }
 
-// The product of 17 to 256 rows (e4m3: 1 to 128), its sum with the residual and
-// the norm behind, N up to 16384. Whether that is done, which it is where the
-// second kernel runs anyway and no part holds more than a tile; if not, nothing
-// is. x_scales: e4m3 operands, sizes in pairs of values, and e4m3 rows out.
-bool launch_part_gemm_norm(void* out, float* out_scales, u16* residual,
-                           const u16* norm, float eps, float* pieces,
-                           const u16* x, const float* x_scales, const u16* w,
-                           const float* w_scales, int M, int N, int K,
-                           int64_t x_stride, hipStream_t stream) {
+// The products of 17 to 256 rows (e4m3: 1 to 128) in pieces, and then sum(where
+// they are). Whether that is done, which it is where the pieces are summed by a
+// second kernel anyway and no part holds more than a tile; if not, or without
+// scratch, nothing is. x_scales: e4m3 operands, sizes in pairs of values.
+template <class F>
+bool in_pieces(float* pieces, const u16* x, const float* x_scales,
+               const u16* w, const float* w_scales, const u16* bias, int M,
+               int N, int K, int64_t x_stride, hipStream_t stream,
+               const F& sum) {
   bool done = false;
   auto run = [&](auto shape, const Plan& pl, auto fp8) {
     using S = decltype(shape);
     constexpr bool kFp8 = decltype(fp8)::value;
-    if (!pl.split || pl.tiles >= pl.parts || N > 16384) return;
+    if (!pl.split || pl.tiles >= pl.parts) return;
     done = true;
     if (pieces == nullptr) return;
-    const Scales scales{x_scales, w_scales};
-    launch_products<S, false, kFp8, true>(pl, nullptr, pieces, x, w, nullptr,
-                                          scales, M, N, K, x_stride, 0,
-                                          stream);
-    auto* p = reinterpret_cast<const floatx4*>(pieces);
-#define FI_NORM(THREADS, ITERS)                                               \
-  hipLaunchKernelGGL((part_gemm_norm_kernel<S, kFp8, kFp8, THREADS, ITERS>),  \
-                     dim3(ceil_div(M, 16) * 16), dim3(THREADS), 0, stream,    \
-                     out, out_scales, p, residual, norm, eps, scales, M, N,   \
-                     K, pl.tiles, pl.parts)
-    if (N <= 2048) FI_NORM(512, 1);
-    else if (N <= 4096) FI_NORM(1024, 1);
-    else if (N <= 8192) FI_NORM(1024, 2);
-    else FI_NORM(1024, 4);
-#undef FI_NORM
+    launch_products<S, false, kFp8, true>(
+        pl, nullptr, pieces, x, w, nullptr, Scales{x_scales, w_scales}, M, N,
+        K, x_stride, 0, stream);
+    sum(PieceRows{pieces, bias, S::TN, K / S::KS, pl.tiles, pl.parts, S::MB,
+                  S::kAhead});
   };
   if (x_scales != nullptr)
     with_shape<true>(M, N, K, [&](auto shape, const Plan& pl) {
@@ -1042,6 +1003,48 @@ bool launch_part_gemm_norm(void* out, float* out_scales, u16* residual,
       run(shape, pl, std::false_type{});
     });
   return done;
+}
+
+// residual += x W^T and the norm behind, N up to 16384
+bool launch_part_gemm_norm(void* out, float* out_scales, u16* residual,
+                           const u16* norm, float eps, float* pieces,
+                           const u16* x, const float* x_scales, const u16* w,
+                           const float* w_scales, int M, int N, int K,
+                           int64_t x_stride, hipStream_t stream) {
+  if (N > 16384) return false;
+  return in_pieces(
+      pieces, x, x_scales, w, w_scales, nullptr, M, N, K, x_stride, stream,
+      [&](const PieceRows& rows) {
+        const dim3 grid(ceil_div(M, 16) * 16);
+#define FI_NORM(FP8, THREADS, ITERS)                                          \
+  hipLaunchKernelGGL((part_gemm_norm_kernel<FP8, THREADS, ITERS>), grid,      \
+                     dim3(THREADS), 0, stream, out, out_scales, rows,         \
+                     residual, norm, eps, Scales{x_scales, w_scales}, M, N)
+#define FI_NORM_N(FP8)                                                        \
+  if (N <= 2048) FI_NORM(FP8, 512, 1);                                        \
+  else if (N <= 4096) FI_NORM(FP8, 1024, 1);                                  \
+  else if (N <= 8192) FI_NORM(FP8, 1024, 2);                                  \
+  else FI_NORM(FP8, 1024, 4)
+        if (x_scales != nullptr) {
+          FI_NORM_N(true);
+        } else {
+          FI_NORM_N(false);
+        }
+#undef FI_NORM_N
+#undef FI_NORM
+      });
+}
+
+// x W^T + bias as heads of 64 or 128: queries normed and rotated to q, K and V
+// rows to the paged cache
+bool launch_part_gemm_rope(u16* q, const RopeArgs& rope, const u16* bias,
+                           float* pieces, const u16* x, const u16* w, int M,
+                           int N, int K, int64_t x_stride,
+                           hipStream_t stream) {
+  return in_pieces(pieces, x, nullptr, w, nullptr, bias, M, N, K, x_stride,
+                   stream, [&](const PieceRows& rows) {
+                     launch_rope_of_pieces(q, rows, rope, M, stream);
+                   });
 }
 
 }  // namespace fi

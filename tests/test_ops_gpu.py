@@ -1461,6 +1461,75 @@ def test_linear_gelu(rows, n, k):
     assert taken is not None or rows > 16
 
 
+@pytest.mark.parametrize("rows", [17, 43, 64, 65, 129, 193, 256])
+@pytest.mark.parametrize("hq,hk,d,k,bias,norm,fp8", [
+    (32, 8, 128, 4096, False, True, False),
+    (32, 4, 128, 2048, True, False, True),
+    (14, 2, 64, 3584, True, True, False),
+    (9, 1, 64, 512, False, False, True),     # heads that fill no wave
+    (70, 5, 128, 1024, False, True, False),  # two workgroups a token
+])
+def test_linear_in_parts_to_heads(rows, hq, hk, d, k, bias, norm, fp8):
+    """Queries, keys and values of a product in parts, normed, rotated and in
+    the cache, against float64: fp32 sums of k products, which the norm scales,
+    each result rounded to bf16 once (2^-9 relative), to e4m3 once more (2^-4,
+    2^-10 where it is smallest). Rows without a slot are not kept."""
+    g = torch.Generator().manual_seed(rows + hq + d + k)
+    n, bs = (hq + 2 * hk) * d, 16
+    x = torch.randn(rows, k, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(n, k, generator=g) * k ** -0.5).to(torch.bfloat16).to(DEV)
+    b = torch.randn(n, generator=g).to(torch.bfloat16).to(DEV) if bias \
+        else None
+    qw, kw = (torch.rand(2, d, generator=g) + 0.5).to(torch.bfloat16).to(DEV) \
+        if norm else (None, None)
+    pos = torch.randint(0, 500, (rows,), generator=g).int().to(DEV)
+    cs = ops.compute_cos_sin_cache(d, 512, 1e4).to(DEV)
+    blocks = rows // bs + 3
+    slots = torch.randperm(blocks * bs, generator=g)[:rows].int()
+    slots[::9] = -1
+    kc, vc = (torch.zeros(blocks, hk, bs, d, device=DEV).to(
+        torch.float8_e4m3fn if fp8 else torch.bfloat16) for _ in range(2))
+    q = torch.full((rows + 1, hq * d), 7.0, dtype=torch.bfloat16, device=DEV)
+    done = ops._C.few_rows_gemm_rope(
+        q[:rows], x, w, b, qw, kw, cs, pos, kc, vc, slots.to(DEV), hq, 1e-6,
+        0.5, 2.0)
+    assert (q[rows] == 7.0).all()
+    if not done:
+        assert k <= 1024 and not kc.float().any() and (q == 7.0).all()
+        return
+    heads = x.double() @ w.double().T + (0.0 if b is None else b.double())
+    heads = heads.view(rows, hq + 2 * hk, d)
+    err = torch.full_like(heads, 1e-5)
+    if norm:
+        inv = (heads.square().mean(-1, keepdim=True) + 1e-6).rsqrt()
+        wt = torch.cat([qw.expand(hq, d), kw.expand(hk, d),
+                        torch.ones_like(kw).expand(hk, d)]).double()
+        inv[:, hq + hk:] = 1.0
+        heads, err = heads * inv * wt, 4 * err * inv * wt
+    c, s = (t.double()[:, None] for t in cs[pos.long()].chunk(2, dim=-1))
+    x1, x2 = heads.chunk(2, dim=-1)
+    turned = torch.cat([x1 * c - x2 * s, x2 * c + x1 * s], -1)
+    err = 2 * err.amax(-1, keepdim=True).expand_as(err)
+    got, want = q[:rows].view(rows, hq, d).double(), turned[:, :hq]
+    assert ((got - want).abs() <= want.abs() * 2 ** -8 + err[:, :hq]).all()
+    kept = (slots >= 0).nonzero()[:, 0].to(DEV)
+    at = slots.to(DEV)[kept].long()
+    for cache, want, e, scale in (
+            (kc, turned[:, hq:hq + hk], err[:, hq:hq + hk], 0.5),
+            (vc, heads[:, hq + hk:], err[:, hq + hk:], 2.0)):
+        got = cache[at // bs, :, at % bs].double()
+        want, e = want[kept], e[kept]
+        bound = want.abs() * 2 ** -8 + e
+        if fp8:
+            want, bound = want * scale, bound * scale
+            bound = bound + want.abs() * 2 ** -4 + 2.0 ** -10
+        assert ((got - want).abs() <= bound).all()
+        rest = torch.ones(blocks * bs, dtype=torch.bool, device=DEV)
+        rest[at] = False
+        rest = rest.nonzero()[:, 0]
+        assert not cache[rest // bs, :, rest % bs].float().any()
+
+
 @pytest.mark.parametrize("rows", [128, 129])
 def test_linear_in_parts_of_long_rows(rows):
     """Rows of W too long for 32-bit offsets within a tile (x one row, given
