@@ -222,6 +222,22 @@ def _tiles_ok(x, w, unit: int, silu_mul: bool = False, bias=None) -> bool:
     )
 
 
+def _one_row_of_tiles(x, w, bias=None) -> bool:
+    """Whether 129 to 256 rows that stream go by tiles of 256 x 256 for it: wide
+    W, where the chip has whole rounds of those, by the two kernels' own
+    estimates. 151936 x 4096 at 129 and 256 rows 300 and 349 us in parts, 258
+    and 302 so; 98304 x 3072 at 256 174 and 169; 40960 x 5120 at 256, where the
+    estimates are even, 141 and 144; from K 8192 on the tiles wait for memory
+    (49152 x 8192 at 256 216 and 294). 14 N, seven K, three numbers of rows: 0.9
+    % above the better one on average, parts alone 3.1."""
+    M, N, K = x.shape[0], w.shape[0], w.shape[1]
+    return (
+        M > 128 and 40960 <= N <= 1 << 20 and K < 8192 and x.stride(0) >= K
+        and (bias is None or bias.data_ptr() % 16 == 0)
+        and _C.many_rows_gemm_us(M, N, 2 * K) < _C.few_rows_gemm_us(M, N, K)
+    )
+
+
 def linear(x: torch.Tensor, w: torch.Tensor,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x W^T (+ bias): a few bf16 rows stream W once through the kernels for
@@ -230,7 +246,10 @@ def linear(x: torch.Tensor, w: torch.Tensor,
     if _skinny_ok(x, w, 16, bias=bias):
         out = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype,
                           device=x.device)
-        _C.few_rows_gemm(out, x, w, bias, False)
+        if _one_row_of_tiles(x, w, bias):
+            _C.many_rows_gemm(out, x, w, bias, False)
+        else:
+            _C.few_rows_gemm(out, x, w, bias, False)
         return out
     if _tiles_ok(x, w, 16, bias=bias):
         out = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype,
@@ -341,7 +360,10 @@ def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if _skinny_ok(x, w, 32, True):
         out = torch.empty((x.shape[0], w.shape[0] // 2), dtype=x.dtype,
                           device=x.device)
-        _C.few_rows_gemm(out, x, w, None, True)
+        if _one_row_of_tiles(x, w):
+            _C.many_rows_gemm(out, x, w, None, True)
+        else:
+            _C.few_rows_gemm(out, x, w, None, True)
         return out
     if _tiles_ok(x, w, 32, True):
         out = torch.empty((x.shape[0], w.shape[0] // 2), dtype=x.dtype,

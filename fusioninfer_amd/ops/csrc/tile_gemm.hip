@@ -35,7 +35,11 @@
 // memory channels. With rows longer than 16 KB every other column tile starts
 // half way along K: bf16, 4096 x 12288 at 4099, 6000 and 7600 rows 294, 437 and
 // 540 us, so 285, 428 and 526 (at 1024 rows 90 and 91); K 10240 the same either
-// way; e4m3, 8192 x 32768 at 2700 rows 569 and 542, K 20480 the same.
+// way; e4m3, 8192 x 32768 at 2700 rows 569 and 542, K 20480 the same. Where x is
+// one or two tiles tall no two CUs (or only two) read the same of W, and
+// columns start at 32 places: 151936 x 4096 at 256 rows 320 and 296, 65536 x 4096
+// 151 and 122, 24576 x 4096 with silu at 300 98 and 88. (The same at 1024 rows
+// 177 and 174, 4096 x 12288 at 4099 300 and 317.)
 //
 // e4m3: the same bytes in the same places, so a stage is 128 of K. MFMA
 // 32x32x64 (four times a bf16 product's time, eight times its work), a lane
@@ -203,7 +207,7 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
     const Tile tile = tile_at(plan, at);
     t.m = tile.m;
     t.n = tile.n;
-    t.rot = (t.n & 1) * turn * t.count / 2;
+    t.rot = t.n % turn * t.count / turn;
     return t;
   };
 
@@ -559,7 +563,8 @@ void launch(u16* out, float* pieces, const typename Kind<FP8>::Elem* x,
   const int KB = K * static_cast<int>(sizeof(typename Kind<FP8>::Elem));
   const TilePlan p = tile_plan(M, N, KB);
   auto* pc = reinterpret_cast<floatx4*>(pieces);
-  const int turn = KB > 16384 && KB % 4096 == 0 ? 1 : 0;
+  // the places along K that column tiles start at
+  const int turn = p.mt <= 2 ? 32 : KB > 16384 && KB % 4096 == 0 ? 2 : 1;
   hipLaunchKernelGGL((tile_gemm_kernel<MODE, FP8>), dim3(kChip), dim3(256), 0,
                      stream, out, pc, x, w, bias, x_scales, w_scales, M, N, K,
                      x_stride, out_stride, p, turn);

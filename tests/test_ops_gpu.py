@@ -1690,6 +1690,43 @@ def test_linear_takes_tiles():
         assert not ops._tiles_ok(x, w.clone().requires_grad_(), 16)
 
 
+@pytest.mark.parametrize("rows", [129, 192, 255, 256, 511])
+@pytest.mark.parametrize("n,k,bias", [(49184, 2048, True), (151936, 192, False),
+                                      (66560, 1344, False)])
+def test_linear_by_one_or_two_rows_of_tiles(rows, n, k, bias):
+    """Tiles that begin at 32 places along K, fewer stages than places among
+    them, against a float64 product; one bf16 rounding and fp32 sums."""
+    g = torch.Generator().manual_seed(n + k + rows)
+    w, x = (torch.full((m + 256, k), float("nan"), dtype=torch.bfloat16,
+                       device=DEV) for m in (n, rows))
+    w[:n] = torch.randn(n, k, generator=g)
+    x[:rows] = torch.randn(rows, k, generator=g)
+    w, x = w[:n], x[:rows]
+    b = torch.randn(n, generator=g).to(torch.bfloat16).to(DEV) if bias \
+        else None
+    prod = x.double() @ w.double().T
+    out = torch.full((rows + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops._C.many_rows_gemm(out[:rows], x, w, b, False)
+    want = prod + (0.0 if b is None else b.double())
+    assert ((out[:rows].double() - want).abs()
+            <= want.abs() * 2 ** -8 + 1e-4 * k ** 0.5).all()
+    assert (out[rows] == 7.0).all()
+    if rows <= 256 and k == 2048:
+        assert ops._one_row_of_tiles(x, w, b)
+        assert torch.equal(ops.linear(x, w, b), out[:rows])
+        assert not ops._one_row_of_tiles(x[:128], w, b)
+        assert not ops._one_row_of_tiles(x[:1].expand(rows, k), w, b)
+        assert not ops._one_row_of_tiles(x, w[:4096], None)
+    if n % 32 == 0 and not bias:
+        out = torch.full((rows + 1, n // 2), 7.0, dtype=torch.bfloat16,
+                         device=DEV)
+        ops._C.many_rows_gemm(out[:rows], x, w, None, True)
+        want = torch.nn.functional.silu(prod[:, : n // 2]) * prod[:, n // 2:]
+        assert ((out[:rows].double() - want).abs()
+                <= want.abs() * 2 ** -8 + 1e-3 * k ** 0.5).all()
+        assert (out[rows] == 7.0).all()
+
+
 @pytest.mark.parametrize("rows", [17, 32])
 def test_linear_silu_mul_in_parts_of_96_rows(rows):
     """One tile of 96 rows in many pieces, whose kept third of a wave's
