@@ -16,10 +16,24 @@ namespace fi {
 
 constexpr float kFp8Max = 448.0f;
 
-// one 256-thread workgroup per row; row held in registers between the
-// absmax pass and the convert pass (ITERS = ceil(cols / 2048))
-template <int ITERS, bool SILU_MUL>
-__global__ void row_quant_fp8_kernel(
+template <bool ONCE>
+FI_DEV bf16x8 load8(const u16* p) {
+  const u32x4* from = reinterpret_cast<const u32x4*>(p);
+  return __builtin_bit_cast(
+      bf16x8, ONCE ? __builtin_nontemporal_load(from) : *from);
+}
+
+// One workgroup per row, which it holds in registers between the absmax pass and
+// the convert pass: 256 threads up to 4096 columns, up to 1024 beyond, eight
+// columns each, once or twice. Few rows take the time of one chain from load to
+// store, which is the shorter the more threads share it; many are bound by
+// memory. ONCE: what is read and written goes past the caches, for more than the
+// memory-side one holds. us, 12288 columns of silu(gate) * up, 256 threads of six
+// vectors each, and this: 1 row 4.3 and 3.2, 64 rows 4.8 and 3.6, 1000 11.6 and
+// 11.6, 8000 95 and 87, with ONCE 74 (6.6 TB/s; at 2000 rows, 98 MB, 20 either
+// way). 4096 columns as they are: 8000 rows 15.2, with 512 threads 15.9.
+template <int ITERS, bool SILU_MUL, bool ONCE>
+__global__ __launch_bounds__(1024) void row_quant_fp8_kernel(
     unsigned char* __restrict__ out,   // [T, cols] fp8
     float* __restrict__ out_scales,    // [T]
     const u16* __restrict__ in,        // [T, cols] bf16 (SILU_MUL: [T, 2*cols])
@@ -35,15 +49,15 @@ __global__ void row_quant_fp8_kernel(
     const int col = (it * blockDim.x + tid) * 8;
     if (col < cols) {
       if (SILU_MUL) {
-        bf16x8 g = *reinterpret_cast<const bf16x8*>(in + in_row + col);
-        bf16x8 u = *reinterpret_cast<const bf16x8*>(in + in_row + cols + col);
+        const bf16x8 g = load8<ONCE>(in + in_row + col);
+        const bf16x8 u = load8<ONCE>(in + in_row + cols + col);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const float gf = bf16_to_f32(g.h[j]);
           vals[it][j] = silu(gf) * bf16_to_f32(u.h[j]);
         }
       } else {
-        bf16x8 v = *reinterpret_cast<const bf16x8*>(in + in_row + col);
+        const bf16x8 v = load8<ONCE>(in + in_row + col);
 #pragma unroll
         for (int j = 0; j < 8; ++j) vals[it][j] = bf16_to_f32(v.h[j]);
       }
@@ -52,9 +66,12 @@ __global__ void row_quant_fp8_kernel(
     }
   }
 
-  __shared__ float scratch[4];
+  __shared__ float scratch[16];
   amax = wave_reduce_max(amax);
-  amax = block_reduce_max<4>(amax, scratch);
+  if (tid % kWaveSize == 0) scratch[tid / kWaveSize] = amax;
+  __syncthreads();
+  for (int i = 0; i < static_cast<int>(blockDim.x) / kWaveSize; ++i)
+    amax = fmaxf(amax, scratch[i]);
   const float scale = fmaxf(amax, 1e-8f) / kFp8Max;
   const float inv_scale = 1.f / scale;
   if (tid == 0) out_scales[row] = scale;
@@ -68,8 +85,11 @@ __global__ void row_quant_fp8_kernel(
       for (int j = 0; j < 8; ++j) sv[j] = vals[it][j] * inv_scale;
       u32 packed[2];
       pack_fp8x8(sv, packed);
-      *reinterpret_cast<uint2*>(out + static_cast<int64_t>(row) * cols + col) =
-          make_uint2(packed[0], packed[1]);
+      auto* to = reinterpret_cast<uint64_t*>(
+          out + static_cast<int64_t>(row) * cols + col);
+      const uint64_t both = static_cast<uint64_t>(packed[1]) << 32 | packed[0];
+      if (ONCE) __builtin_nontemporal_store(both, to);
+      else *to = both;
     }
   }
 }
@@ -77,26 +97,26 @@ __global__ void row_quant_fp8_kernel(
 template <bool SILU_MUL>
 void launch_row_quant_fp8(unsigned char* out, float* scales, const u16* in,
                           int rows, int cols, hipStream_t stream) {
-  dim3 grid(rows), block(256);
-  const int iters = ceil_div(cols, 256 * 8);
-#define FI_QCASE(N)                                                        \
-  case N:                                                                  \
-    hipLaunchKernelGGL((row_quant_fp8_kernel<N, SILU_MUL>), grid, block, 0, \
-                       stream, out, scales, in, cols);                     \
-    break;
-  switch (iters) {
-    FI_QCASE(1)
-    FI_QCASE(2)
-    FI_QCASE(3)
-    FI_QCASE(4)
-    FI_QCASE(5)
-    FI_QCASE(6)
-    FI_QCASE(7)
-    FI_QCASE(8)
-    default:
-      abort();
+  if (cols > 16384) abort();     // more than two vectors of 1024 threads
+  const int vectors = ceil_div(cols, 8);
+  const int iters = cols <= 2048 ? 1 : cols <= 4096 ? 2 : ceil_div(cols, 8192);
+  const int threads =
+      cols <= 4096 ? 256
+                   : ceil_div(ceil_div(vectors, iters), kWaveSize) * kWaveSize;
+  // 256 MB of memory-side cache
+  const bool once = static_cast<int64_t>(rows) * cols * (SILU_MUL ? 4 : 2) >
+                    int64_t{256} << 20;
+#define FI_QUANT(N, ONCE)                                                     \
+  hipLaunchKernelGGL((row_quant_fp8_kernel<N, SILU_MUL, ONCE>), dim3(rows),   \
+                     dim3(threads), 0, stream, out, scales, in, cols)
+  if (iters == 1) {
+    if (once) FI_QUANT(1, true);
+    else FI_QUANT(1, false);
+  } else {
+    if (once) FI_QUANT(2, true);
+    else FI_QUANT(2, false);
   }
-#undef FI_QCASE
+#undef FI_QUANT
 }
 
 template void launch_row_quant_fp8<true>(unsigned char*, float*, const u16*,

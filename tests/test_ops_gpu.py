@@ -172,6 +172,33 @@ def test_quant_fp8_rows(tokens, cols):
     _assert_fp8_close(f8, sc, ef8, esc, exact=x.cpu())
 
 
+@pytest.mark.parametrize("cols", [2056, 4096, 4104, 8192, 8200, 12288, 16384])
+@pytest.mark.parametrize("silu_mul", [False, True])
+def test_quant_fp8_of_rows_of_all_lengths(cols, silu_mul):
+    """One or two vectors a thread, workgroups of all sizes, and the loads and
+    stores for more than the caches hold give the bits of short calls; those
+    are within half a step of e4m3 (2^-4 relative, 2^-10 of the scale) and fp32
+    roundings of silu of the exact rows, the largest of which is 448."""
+    width = cols * (2 if silu_mul else 1)
+    call = ops.silu_and_mul_fp8 if silu_mul else ops.quant_fp8_rows
+    rows = (1 << 27) // width + 3        # of 2 bytes: more than 256 MB
+    x = torch.randn(rows, width, device=DEV, dtype=torch.bfloat16)
+    f8, sc = call(x)
+    for part in (slice(0, 1), slice(1, 34), slice(rows - 40, rows)):
+        g8, gs = call(x[part])
+        assert torch.equal(g8.view(torch.uint8), f8[part].view(torch.uint8))
+        assert torch.equal(gs, sc[part])
+    want = x[-40:].double()
+    if silu_mul:
+        want = torch.nn.functional.silu(want[:, :cols]) * want[:, cols:]
+    scale = want.abs().amax(1) / 448
+    torch.testing.assert_close(sc[-40:].double(), scale, rtol=2 ** -18, atol=0)
+    got = f8[-40:].double() * sc[-40:].double()[:, None]
+    assert ((got - want).abs() <= want.abs() * (2 ** -4 + 2 ** -18)
+            + scale[:, None] * 2 ** -10).all()
+
+
+
 @pytest.mark.parametrize("qk_norm", [True, False])
 @pytest.mark.parametrize("head_dim", [64, 128])
 def test_rope_qk_norm(qk_norm, head_dim):
