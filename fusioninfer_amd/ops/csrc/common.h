@@ -100,6 +100,9 @@ FI_DEV float block_reduce_sum(float wave_val, float* scratch) {
   return total;
 }
 
+// more than the memory-side cache holds: what is read once better goes past it
+inline bool beyond_caches(int64_t bytes) { return bytes > int64_t{256} << 20; }
+
 __host__ __device__ __forceinline__ constexpr int ceil_div(int a, int b) {
   return (a + b - 1) / b;
 }

@@ -375,8 +375,9 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(
 // Rows of whole 16-byte vectors: a thread takes one vector of a token, all
 // of its experts' rows are requested before the first is used. Bound by
 // reading the rows (8765 tokens, top 8, width 2048: 287 MB and 36 MB out,
-// 172 us with one value per thread, 61 now).
-template <typename A>
+// 172 us with one value per thread, 61 so). ONCE: the rows go past the caches,
+// for more of them than the memory-side one holds.
+template <typename A, bool ONCE>
 __global__ __launch_bounds__(256) void moe_combine_vec_kernel(
     A* __restrict__ out, const A* __restrict__ y, const int* __restrict__ pos,
     const float* __restrict__ w, const int topk, const int H) {
@@ -401,8 +402,10 @@ __global__ __launch_bounds__(256) void moe_combine_vec_kernel(
       r[i] = Vec{};
       if (p >= 0) {
         wk[i] = w[t * topk + k];
-        r[i] = *reinterpret_cast<const Vec*>(
+        const u32x4* from = reinterpret_cast<const u32x4*>(
             y + static_cast<int64_t>(p) * H + c);
+        r[i] = __builtin_bit_cast(
+            Vec, ONCE ? __builtin_nontemporal_load(from) : *from);
       }
     }
 #pragma unroll
@@ -420,8 +423,9 @@ __global__ __launch_bounds__(256) void moe_combine_vec_kernel(
 // workgroup has a token, the sums stay fp32 until the norm. Bound by memory
 // like the one above, and two passes less over the tokens. (Four layers: 8765
 // tokens 5260 -> 5222 us, 64 tokens 1332 -> 1320; the norm alone takes 25 and 2.7
-// us a layer.)
-template <int ITERS>
+// us a layer.) 8765 tokens, top 8, width 2048: 71 us, with ONCE 63; 4000 tokens
+// 28 and 29. No load is behind a branch: 64 tokens 3.5 us with, 3.0 without.
+template <int ITERS, bool ONCE>
 __global__ __launch_bounds__(256) void moe_combine_norm_kernel(
     u16* __restrict__ out, u16* __restrict__ residual,
     const u16* __restrict__ norm, const float eps, const u16* __restrict__ y,
@@ -447,14 +451,13 @@ __global__ __launch_bounds__(256) void moe_combine_norm_kernel(
 #pragma unroll
         for (int i = 0; i < kAhead; ++i) {
           const int k = k0 + i;
-          const int p = k < topk ? pos[t * topk + k] : -1;
-          wk[i] = 0.f;
-          r[i] = bf16x8{};
-          if (p >= 0) {
-            wk[i] = w[t * topk + k];
-            r[i] = *reinterpret_cast<const bf16x8*>(
-                y + static_cast<int64_t>(p) * H + c);
-          }
+          const int at = t * topk + min(k, topk - 1);
+          const int p = k < topk ? pos[at] : -1;
+          const u32x4* from = reinterpret_cast<const u32x4*>(
+              y + static_cast<int64_t>(max(p, 0)) * H + c);
+          const u32x4 got = ONCE ? __builtin_nontemporal_load(from) : *from;
+          wk[i] = p >= 0 ? w[at] : 0.f;
+          r[i] = __builtin_bit_cast(bf16x8, p >= 0 ? got : u32x4{0, 0, 0, 0});
         }
 #pragma unroll
         for (int i = 0; i < kAhead; ++i)
@@ -496,9 +499,14 @@ void launch_moe_combine_norm(u16* out, u16* residual, const u16* norm,
                              float eps, const u16* y, const int* pos,
                              const float* w, int tokens, int topk, int H,
                              hipStream_t stream) {
+  const bool once = beyond_caches(static_cast<int64_t>(tokens) * topk * H * 2);
 #define FI_CN(ITERS)                                                          \
-  hipLaunchKernelGGL(moe_combine_norm_kernel<ITERS>, dim3(tokens), dim3(256), \
-                     0, stream, out, residual, norm, eps, y, pos, w, topk, H)
+  do {                                                                        \
+    auto kernel = once ? &moe_combine_norm_kernel<ITERS, true>                \
+                       : &moe_combine_norm_kernel<ITERS, false>;              \
+    hipLaunchKernelGGL(kernel, dim3(tokens), dim3(256), 0, stream, out,       \
+                       residual, norm, eps, y, pos, w, topk, H);              \
+  } while (0)
   if (H <= 2048) FI_CN(1);
   else if (H <= 4096) FI_CN(2);
   else FI_CN(4);
@@ -563,9 +571,12 @@ void launch_moe_combine(A* out, const A* y, const int* pos, const float* w,
       (reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(y)) %
           16 == 0;
   if (vec) {
-    hipLaunchKernelGGL(moe_combine_vec_kernel<A>,
-                       dim3(tokens, ceil_div(H / V, 256)), dim3(256), 0,
-                       stream, out, y, pos, w, topk, H);
+    auto kernel = beyond_caches(static_cast<int64_t>(tokens) * topk * H *
+                                static_cast<int64_t>(sizeof(A)))
+                      ? &moe_combine_vec_kernel<A, true>
+                      : &moe_combine_vec_kernel<A, false>;
+    hipLaunchKernelGGL(kernel, dim3(tokens, ceil_div(H / V, 256)), dim3(256),
+                       0, stream, out, y, pos, w, topk, H);
     return;
   }
   const dim3 grid(ceil_div(H, 256), tokens);

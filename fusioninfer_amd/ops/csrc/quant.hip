@@ -103,9 +103,8 @@ void launch_row_quant_fp8(unsigned char* out, float* scales, const u16* in,
   const int threads =
       cols <= 4096 ? 256
                    : ceil_div(ceil_div(vectors, iters), kWaveSize) * kWaveSize;
-  // 256 MB of memory-side cache
-  const bool once = static_cast<int64_t>(rows) * cols * (SILU_MUL ? 4 : 2) >
-                    int64_t{256} << 20;
+  const bool once = beyond_caches(static_cast<int64_t>(rows) * cols *
+                                  (SILU_MUL ? 4 : 2));
 #define FI_QUANT(N, ONCE)                                                     \
   hipLaunchKernelGGL((row_quant_fp8_kernel<N, SILU_MUL, ONCE>), dim3(rows),   \
                      dim3(threads), 0, stream, out, scales, in, cols)

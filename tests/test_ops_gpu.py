@@ -1215,6 +1215,32 @@ def test_moe_combine_norm(T, top, H):
             ).all()
 
 
+def test_moe_combine_past_the_caches():
+    """More rows than the memory-side cache holds give the bits of the same
+    tokens in shorter calls; what rows that nobody has hold does not matter."""
+    T, top, H = 8200, 8, 2048
+    y = torch.randn(T * top, H, device=DEV, dtype=torch.bfloat16)
+    y[0] = float("nan")
+    pos = torch.randperm(T * top, device=DEV).int()
+    pos[pos == 0] = -1
+    pos[::11] = -1
+    w = torch.rand(T * top, device=DEV)
+    old, norm = (torch.randn(n, H, device=DEV, dtype=torch.bfloat16)
+                 for n in (T, 1))
+    out, res = ops.moe_combine_norm(y, pos, w, old.clone(), norm[0], 1e-6)
+    plain = ops.moe_combine(torch.empty_like(old), y, pos, w)
+    assert out.isfinite().all() and plain.isfinite().all()
+    for a in (0, 4000, T - 7):
+        b = min(a + 500, T)
+        cut = slice(a * top, b * top)
+        o, r = ops.moe_combine_norm(y, pos[cut], w[cut], old[a:b].clone(),
+                                    norm[0], 1e-6)
+        assert torch.equal(o, out[a:b]) and torch.equal(r, res[a:b])
+        assert torch.equal(ops.moe_combine(torch.empty_like(o), y, pos[cut],
+                                           w[cut]), plain[a:b])
+
+
+
 
 # ------------------------------------------------------------ skinny GEMM
 
