@@ -50,7 +50,6 @@ typedef __attribute__((ext_vector_type(8))) short short8;
 typedef __attribute__((ext_vector_type(4))) float floatx4;
 
 constexpr int kStageK = 128;          // values of K per stage
-constexpr int kFragB = 16 * kStageK * 2;  // 16 rows of a stage
 
 template <int N>
 FI_DEV void wait_vm() {
@@ -105,8 +104,9 @@ FI_DEV floatx4 sum_of_parts(const float* squares, int parts, int lane) {
   return sum;
 }
 
-// XR: DMAs for the rows of x per stage, four rows each
-template <int NW, int RF, int XR, int R, bool SILU_MUL, int MODE>
+// XR: DMAs for the rows of x per stage, four rows each. WR: rows of W of a
+// fragment; eight leave half of a product unused.
+template <int NW, int RF, int XR, int R, bool SILU_MUL, int MODE, int WR = 16>
 __global__ __launch_bounds__((NW + (MODE == SCALED)) * kWaveSize)
 void skinny_gemm_kernel(void* __restrict__ out_p, const u16* __restrict__ x,
                         const u16* __restrict__ w,
@@ -120,8 +120,10 @@ void skinny_gemm_kernel(void* __restrict__ out_p, const u16* __restrict__ x,
   static_assert(MODE != ADD || !SILU_MUL);
   using Out = std::conditional_t<MODE == ADD, float, u16>;
   Out* out = static_cast<Out*>(out_p);
+  static_assert(WR == 16 || (WR == 8 && RF == 1 && MODE == PLAIN));
+  constexpr int kFragB = WR * kStageK * 2;       // rows of W of a stage
   constexpr int kStageB = RF * kFragB + XR * 1024;
-  constexpr int kLoads = RF * 4 + XR;            // DMAs of a stage
+  constexpr int kLoads = RF * (WR / 4) + XR;     // DMAs of a stage
   constexpr int kScratch = NW * RF * kWaveSize;  // float4
   constexpr int kRingB = NW * R * kStageB;
   constexpr int kSquaresB = MODE == SCALED ? 64 : 0;
@@ -136,7 +138,7 @@ void skinny_gemm_kernel(void* __restrict__ out_p, const u16* __restrict__ x,
 
   const int lane = threadIdx.x % kWaveSize;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
-  const int tiles = (SILU_MUL ? N / 2 : N) / (SILU_MUL ? 16 : 16 * RF);
+  const int tiles = (SILU_MUL ? N / 2 : N) / (SILU_MUL ? 16 : WR * RF);
   const int stages = K / kStageK;
   const int s_lo = wave * stages / NW, s_hi = (wave + 1) * stages / NW;
 
@@ -148,9 +150,9 @@ void skinny_gemm_kernel(void* __restrict__ out_p, const u16* __restrict__ x,
 
   // per-lane source offsets: DMA j copies rows 4j..4j+3, lane l chunk
   // (l & 15) ^ row of row 4j + (l >> 4) to its place l & 15
-  u32 w_off[4], x_off[XR];
+  u32 w_off[WR / 4], x_off[XR];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < WR / 4; ++j) {
     const int row = 4 * j + (lane >> 4);
     w_off[j] = static_cast<u32>(row * K + ((lane & 15) ^ row) * 8) * 2;
   }
@@ -167,7 +169,7 @@ void skinny_gemm_kernel(void* __restrict__ out_p, const u16* __restrict__ x,
 #pragma unroll
   for (int kk = 0; kk < 4; ++kk) {
     const int c = kk * 4 + (lane >> 4);
-    wr[kk] = row * 256 + ((c ^ row) & 15) * 16;
+    wr[kk] = (row & (WR - 1)) * 256 + ((c ^ (row & (WR - 1))) & 15) * 16;
     xr[kk] = RF * kFragB + xrow * 256 + ((c ^ xrow) & 15) * 16;
   }
 
@@ -199,10 +201,10 @@ void skinny_gemm_kernel(void* __restrict__ out_p, const u16* __restrict__ x,
 #pragma unroll
     for (int f = 0; f < RF; ++f) {
       const int64_t r0 = SILU_MUL ? it * 16 + f * (N / 2)
-                                  : (it * RF + f) * 16;
+                                  : (it * RF + f) * WR;
       const u16* src = w + r0 * K + is * kStageK;
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < WR / 4; ++j)
         dma_to_lds16_nt(dst + f * kFragB + j * 1024, src, w_off[j]);
     }
 #pragma unroll
@@ -222,8 +224,9 @@ void skinny_gemm_kernel(void* __restrict__ out_p, const u16* __restrict__ x,
   for (int t = 0; t < mine; ++t) {
     const int tile = blockIdx.x + t * gridDim.x;
     const int m = lane & 15, n4 = (lane >> 4) * 4;
-    const bool mine_to_store = wave < (SILU_MUL ? 1 : RF) && m < M;
-    const int n = (SILU_MUL ? tile : tile * RF + wave) * 16 + n4;
+    const bool mine_to_store =
+        wave < (SILU_MUL ? 1 : RF) && m < M && (WR == 16 || n4 < WR);
+    const int n = (SILU_MUL ? tile : tile * RF + wave) * WR + n4;
     // (requested here: at its use nothing else would be on its way)
     floatx4 old;
     bf16x4 g;
@@ -321,8 +324,8 @@ void launch_skinny_gemm(u16* out, const u16* x, const u16* w, const u16* bias,
                         const SkinnyExtra& extra, int M, int N, int K,
                         int64_t x_stride, int64_t out_stride, bool silu_mul,
                         hipStream_t stream) {
-#define FI_SK(NW, RF, XR, R, S, MODE)                                         \
-  hipLaunchKernelGGL((skinny_gemm_kernel<NW, RF, XR, R, S, MODE>),            \
+#define FI_SK(NW, RF, XR, R, S, MODE, ...)                                    \
+  hipLaunchKernelGGL((skinny_gemm_kernel<NW, RF, XR, R, S, MODE, ##__VA_ARGS__>), \
                      dim3(grid), dim3((NW + (MODE == SCALED)) * kWaveSize),   \
                      0, stream,                                               \
                      MODE == ADD ? static_cast<void*>(extra.add) : out, x, w, \
@@ -337,7 +340,14 @@ void launch_skinny_gemm(u16* out, const u16* x, const u16* w, const u16* bias,
   // 4096 32.0 / 31.6; 6144, 4096 9.6 / 11.2; 4096, 4096 9.3 / 7.7; 4096,
   // 12288 23.3 / 17.8; at M = 16 33.4 / 37.9, 12.1 / 14.2, 11.3 / 9.3.
   const bool wide = silu_mul || (N % 32 == 0 && N >= 6144);
-  const int tiles = silu_mul ? N / 32 : (wide ? N / 32 : N / 16);
+  // where tiles of 16 rows fill half of the chip at most, twice as many of eight
+  // have two thirds of the bytes each on their way for half as long. us at M = 1
+  // / 4 / 16: 2048, 6144 8.2 / 9.0 / 10.9 and 6.7 / 6.9 / 9.5; 2048, 2048 4.0 /
+  // 4.2 / 4.7 and 3.7 / 3.8 / 4.2; 256, 4096 4.5 / 4.8 / 6.2 and 3.7 / 3.9 / 5.2
+  const bool plain = extra.squares_in == nullptr && extra.add == nullptr &&
+                     !extra.gelu && !silu_mul;
+  const bool few = plain && N <= 2048;
+  const int tiles = silu_mul || wide ? N / 32 : few ? N / 8 : N / 16;
   const int grid = std::min(tiles, 256);
 #define FI_SK_WIDE(S, MODE)                                                   \
   do {                                                                        \
@@ -364,7 +374,10 @@ void launch_skinny_gemm(u16* out, const u16* x, const u16* w, const u16* bias,
   } else {
     if (silu_mul) FI_SK_WIDE(true, PLAIN);
     else if (wide) FI_SK_WIDE(false, PLAIN);
-    else FI_SK_NARROW(PLAIN);
+    else if (!few) FI_SK_NARROW(PLAIN);
+    else if (M <= 4) FI_SK(8, 1, 1, 4, false, PLAIN, 8);
+    else if (M <= 8) FI_SK(8, 1, 2, 4, false, PLAIN, 8);
+    else FI_SK(8, 1, 4, 3, false, PLAIN, 8);
   }
 #undef FI_SK_NARROW
 #undef FI_SK_WIDE

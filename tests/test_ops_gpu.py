@@ -1343,6 +1343,30 @@ def test_linear_in_parts_of_several_tiles(rows, n, k, bias):
 
 
 @pytest.mark.parametrize("rows", [1, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("n,k,bias", [
+    (16, 128, False), (16, 1152, True), (2032, 256, True), (2048, 6144, False),
+    (2064, 384, True),      # the first that goes by tiles of 16 rows again
+])
+def test_linear_by_tiles_of_eight_rows(rows, n, k, bias):
+    """Against float64: fp32 sums of k products, one bf16 rounding (2^-9
+    relative). What lies behind the last row of either operand has no part."""
+    g = torch.Generator().manual_seed(n + k + rows)
+    w, x = (torch.full((m + 32, k), float("nan"), dtype=torch.bfloat16,
+                       device=DEV) for m in (n, rows))
+    w[:n] = torch.randn(n, k, generator=g)
+    x[:rows] = torch.randn(rows, k, generator=g)
+    w, x = w[:n], x[:rows]
+    b = torch.randn(n, generator=g).to(torch.bfloat16).to(DEV) if bias \
+        else None
+    out = torch.full((rows + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops._C.few_rows_gemm(out[:rows], x, w, b, False)
+    want = x.double() @ w.double().T + (0.0 if b is None else b.double())
+    assert ((out[:rows].double() - want).abs()
+            <= want.abs() * 2 ** -8 + 1e-4 * k ** 0.5).all()
+    assert (out[rows] == 7.0).all()
+
+
+@pytest.mark.parametrize("rows", [1, 4, 5, 8, 9, 16])
 @pytest.mark.parametrize("n,k,parts,bias", [
     (16, 128, 1, True),        # one tile; most waves without a stage
     (2576, 1152, 127, False),  # tiles of 16 rows, parts short of a round
