@@ -674,17 +674,19 @@ class DecoderLayer(nn.Module):
                 and product_alone(self.mlp.down_proj))
 
     def forward(self, hidden, residual, meta, kv_cache, cos_sin,
-                keep_hidden: bool = True, norm_behind: torch.Tensor = None):
+                keep_hidden: bool = True, norm_behind: torch.Tensor = None,
+                stream: bool = False):
         """keep_hidden: where residual is None the stream begins as a copy of
         hidden; otherwise hidden itself becomes it, for a caller that has no
         other use of it.
 
-        What is still to be added to the stream comes back first. A layer that
-        adds by itself gives the rows behind the norm of norm_behind instead;
-        for few rows the stream's rows before it, or None without one, and the
-        stream in fp32."""
+        What is still to be added to the stream comes back first. With
+        norm_behind a layer that adds by itself gives the rows behind that norm
+        instead; of few rows, with stream, the stream's rows before it, or None
+        without one, and the stream in fp32."""
         rows = hidden if isinstance(hidden, ops.StreamRows) else None
-        if self._streams(hidden if residual is None else residual, meta):
+        if stream and self._streams(hidden if residual is None else residual,
+                                    meta):
             if rows is None:
                 if hidden is None or isinstance(hidden, ops.NormedRows):
                     hidden = residual
@@ -827,11 +829,20 @@ class CausalLM(nn.Module):
         if self.pp_first:
             hidden = self.embed_tokens[input_ids]
             residual = None
+        # whoever looks at layers from outside sees them pass rows and residual
+        apart = (torch.nn.modules.module._has_any_global_hook()
+                 or any("forward" in vars(layer) or layer._forward_hooks
+                        or layer._forward_pre_hooks for layer in self.layers))
         norms = [layer.input_norm_weight for layer in self.layers[1:]] + [None]
         for layer, kv, norm in zip(self.layers, kv_caches, norms):
-            hidden, residual = layer(hidden, residual, meta, kv, self.cos_sin,
-                                     keep_hidden=not self.pp_first,
-                                     norm_behind=norm)
+            if apart:
+                hidden, residual = layer(hidden, residual, meta, kv,
+                                         self.cos_sin)
+            else:
+                hidden, residual = layer(
+                    hidden, residual, meta, kv, self.cos_sin,
+                    keep_hidden=not self.pp_first, norm_behind=norm,
+                    stream=True)
         if not self.pp_last:
             return hidden, residual
         if rows is not None:

@@ -424,3 +424,13 @@ def test_layers_whose_norms_are_apart(length, fp8):
         assert seen == hooked
         bound = 11 * 2 ** -9 + (4 * 2 ** -4 if fp8 else 0)
         assert (got - want).norm() <= len(layers) * bound
+    # from outside a layer passes rows and residual, as ever
+    seen = []
+    hook = layers[1].register_forward_hook(
+        lambda _, args, out: seen.extend([*args[:2], *out]))
+    got = torch.tensor(eng.embed(prompt)[0])
+    hook.remove()
+    assert len(seen) == 4 and all(
+        type(t) is torch.Tensor and t.dtype == torch.bfloat16
+        and t.shape[0] == length for t in seen)
+    assert (got - want).norm() <= len(layers) * bound
