@@ -829,11 +829,12 @@ class CausalLM(nn.Module):
         if self.pp_first:
             hidden = self.embed_tokens[input_ids]
             residual = None
-        # whoever looks at layers from outside sees them pass rows and residual
-        apart = (torch.nn.modules.module._has_any_global_hook()
-                 or any("forward" in vars(layer) or layer._forward_hooks
-                        or layer._forward_pre_hooks for layer in self.layers))
-        norms = [layer.input_norm_weight for layer in self.layers[1:]] + [None]
+        # whoever looks at layers from outside, or stands in the place of one,
+        # sees them pass rows and residual
+        apart = not all(type(layer) is DecoderLayer and unhooked(layer)
+                        for layer in self.layers)
+        norms = [None if apart else layer.input_norm_weight
+                 for layer in self.layers[1:]] + [None]
         for layer, kv, norm in zip(self.layers, kv_caches, norms):
             if apart:
                 hidden, residual = layer(hidden, residual, meta, kv,

@@ -1,0 +1,76 @@
+"""The decoder model with parts that are not its own: whatever stands in a
+layer's or an attention's place is called with rows, residual, metadata, cache
+and angles (an attention without the residual), as the model's own modules can
+be, and nothing else is asked of it."""
+
+import pytest
+import torch
+from torch import nn
+
+from fusioninfer_amd.config import CacheConfig, EngineConfig, SchedulerConfig
+from fusioninfer_amd.engine.llm_engine import LLMEngine
+from fusioninfer_amd.models.registry import get_model_config
+
+PROMPT = [3, 1, 4, 1, 5, 9, 2, 6, 5]
+
+
+def make_engine(name="tiny-qwen3", layers=3, quantization=None):
+    mc = get_model_config(name)
+    mc.num_layers = layers
+    mc.quantization = quantization
+    return LLMEngine(EngineConfig(
+        model=mc, cache=CacheConfig(num_gpu_blocks=64),
+        scheduler=SchedulerConfig(max_num_seqs=4, max_num_batched_tokens=256,
+                                  max_model_len=128)), device="cpu")
+
+
+def states(eng, **kw):
+    """Of all rows, from the model itself."""
+    seen = []
+    forward = type(eng.runner.model).forward
+
+    class Seen(type(eng.runner.model)):
+        def forward(self, ids, meta, caches):
+            seen.append(forward(self, ids, meta, caches, **kw))
+            return seen[-1]
+
+    model, eng.runner.model.__class__ = type(eng.runner.model), Seen
+    try:
+        eng.embed([PROMPT])
+    finally:
+        eng.runner.model.__class__ = model
+    return seen[0]
+
+
+class Inside(nn.Module):
+    """Calls the layer, or the attention, in whose place it stands."""
+
+    def __init__(self, inner):
+        super().__init__()
+        self.inner = inner
+        self.calls = 0
+
+    def forward(self, *args):
+        self.calls += 1
+        return self.inner(*args)
+
+
+class LayerInside(Inside):
+    def forward(self, hidden, residual, meta, kv_cache, cos_sin):
+        return super().forward(hidden, residual, meta, kv_cache, cos_sin)
+
+
+CONFIGS = [("tiny-qwen3", None), ("tiny-qwen3", "fp8"),
+           ("tiny-qwen3-moe", None)]
+
+
+@pytest.mark.parametrize("name,quantization", CONFIGS)
+@pytest.mark.parametrize("places", [[0], [1], [2], [0, 1, 2]])
+def test_module_in_a_layers_place(name, quantization, places):
+    eng = make_engine(name, quantization=quantization)
+    want = states(eng)
+    layers = eng.runner.model.layers
+    for i in places:
+        layers[i] = LayerInside(layers[i])
+    assert torch.equal(states(eng), want)
+    assert all(layers[i].calls == 1 for i in places)
