@@ -660,6 +660,11 @@ class DecoderLayer(nn.Module):
         self.eps = cfg.rms_norm_eps
         self.fp8 = cfg.quantization == "fp8"
 
+    def _attention_alone(self) -> bool:
+        """Whether the attention is the model's own and nobody looks at its
+        calls, so that it may be given the residual too."""
+        return type(self.self_attn) is Attention and unhooked(self.self_attn)
+
     def _streams(self, x, meta) -> bool:
         """Whether the norms go into the linear layers on both sides of them
         and the sums into those in front: few rows, whose kernels do both, and
@@ -667,7 +672,7 @@ class DecoderLayer(nn.Module):
         return (x.is_cuda and ops.stream_rows_ok(*x.shape)
                 and type(self.mlp) is MLP and not self.fp8
                 and meta.lora is None and ps.pp_world_size() == 1
-                and unhooked(self.self_attn) and unhooked(self.mlp)
+                and self._attention_alone() and unhooked(self.mlp)
                 and weight_alone(self.self_attn.qkv_proj, bias=True)
                 and product_alone(self.self_attn.o_proj)
                 and weight_alone(self.mlp.gate_up_proj)
@@ -722,7 +727,7 @@ class DecoderLayer(nn.Module):
             x, residual = ops.fused_add_rms_norm(
                 hidden, residual, self.input_norm_weight, self.eps
             )
-        if meta.lora is None and unhooked(self.self_attn):
+        if meta.lora is None and self._attention_alone():
             x, residual = self.self_attn(x, meta, kv_cache, cos_sin, residual,
                                          self.post_norm_weight)
         else:

@@ -74,3 +74,20 @@ def test_module_in_a_layers_place(name, quantization, places):
         layers[i] = LayerInside(layers[i])
     assert torch.equal(states(eng), want)
     assert all(layers[i].calls == 1 for i in places)
+
+
+class AttentionInside(Inside):
+    def forward(self, x, meta, kv_cache, cos_sin):
+        return super().forward(x, meta, kv_cache, cos_sin)
+
+
+@pytest.mark.parametrize("name,quantization", CONFIGS)
+@pytest.mark.parametrize("places", [[0], [1, 2]])
+def test_module_in_an_attentions_place(name, quantization, places):
+    eng = make_engine(name, quantization=quantization)
+    want = states(eng)
+    layers = eng.runner.model.layers
+    for i in places:
+        layers[i].self_attn = AttentionInside(layers[i].self_attn)
+    assert torch.equal(states(eng), want)
+    assert all(layers[i].self_attn.calls == 1 for i in places)
