@@ -838,16 +838,18 @@ class CausalLM(nn.Module):
         # sees them pass rows and residual
         apart = not all(type(layer) is DecoderLayer and unhooked(layer)
                         for layer in self.layers)
-        norms = [None if apart else layer.input_norm_weight
-                 for layer in self.layers[1:]] + [None]
-        for layer, kv, norm in zip(self.layers, kv_caches, norms):
+        # (as many layers as there are caches)
+        run = list(zip(self.layers, kv_caches))
+        for i, (layer, kv) in enumerate(run):
             if apart:
                 hidden, residual = layer(hidden, residual, meta, kv,
                                          self.cos_sin)
             else:
                 hidden, residual = layer(
                     hidden, residual, meta, kv, self.cos_sin,
-                    keep_hidden=not self.pp_first, norm_behind=norm,
+                    keep_hidden=not self.pp_first,
+                    norm_behind=(run[i + 1][0].input_norm_weight
+                                 if i + 1 < len(run) else None),
                     stream=True)
         if not self.pp_last:
             return hidden, residual

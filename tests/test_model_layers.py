@@ -24,14 +24,14 @@ def make_engine(name="tiny-qwen3", layers=3, quantization=None):
                                   max_model_len=128)), device="cpu")
 
 
-def states(eng, **kw):
-    """Of all rows, from the model itself."""
+def states(eng, caches=None):
+    """Of all rows, from the model itself; of the first caches' layers."""
     seen = []
     forward = type(eng.runner.model).forward
 
     class Seen(type(eng.runner.model)):
-        def forward(self, ids, meta, caches):
-            seen.append(forward(self, ids, meta, caches, **kw))
+        def forward(self, ids, meta, kv_caches):
+            seen.append(forward(self, ids, meta, kv_caches[:caches]))
             return seen[-1]
 
     model, eng.runner.model.__class__ = type(eng.runner.model), Seen
@@ -91,3 +91,14 @@ def test_module_in_an_attentions_place(name, quantization, places):
         layers[i].self_attn = AttentionInside(layers[i].self_attn)
     assert torch.equal(states(eng), want)
     assert all(layers[i].self_attn.calls == 1 for i in places)
+
+
+@pytest.mark.parametrize("name,quantization", CONFIGS)
+@pytest.mark.parametrize("caches", [1, 2])
+def test_state_after_the_first_layers(name, quantization, caches):
+    """The caches say how many layers run, and the last norm is behind the
+    last of these: as in a model whose other layers are not there."""
+    eng = make_engine(name, quantization=quantization)
+    got = states(eng, caches)
+    eng.runner.model.layers = eng.runner.model.layers[:caches]
+    assert torch.equal(got, states(eng))
