@@ -767,8 +767,6 @@ class CausalLM(nn.Module):
     weights regardless of the PP/TP layout (stages skip modules without
     desyncing the stream; TP ranks still slice identical full matrices)."""
 
-    takes_rows = True
-
     def __init__(self, cfg: ModelConfig):
         super().__init__()
         self.cfg = cfg
@@ -817,6 +815,12 @@ class CausalLM(nn.Module):
             rope_scaling=cfg.rope_scaling,
         )
         self.register_buffer("cos_sin", cos_sin, persistent=False)
+
+    @property
+    def takes_rows(self) -> bool:
+        """Whether a call is this class's forward and nobody looks at it, so
+        that it may be given the rows that are wanted."""
+        return type(self).forward is CausalLM.forward and unhooked(self)
 
     @property
     def num_local_layers(self) -> int:

@@ -9,6 +9,7 @@ from torch import nn
 
 from fusioninfer_amd.config import CacheConfig, EngineConfig, SchedulerConfig
 from fusioninfer_amd.engine.llm_engine import LLMEngine
+from fusioninfer_amd.engine.sequence import SamplingParams
 from fusioninfer_amd.models.registry import get_model_config
 
 PROMPT = [3, 1, 4, 1, 5, 9, 2, 6, 5]
@@ -102,3 +103,34 @@ def test_state_after_the_first_layers(name, quantization, caches):
     got = states(eng, caches)
     eng.runner.model.layers = eng.runner.model.layers[:caches]
     assert torch.equal(got, states(eng))
+
+
+def test_models_forward_as_ever():
+    """A forward without the rows to give, of a class of its own or set on the
+    model, serves; whoever hooks the model sees the state of all rows."""
+    eng = make_engine()
+    model = eng.runner.model
+    cls = type(model)
+    seen = []
+
+    def tokens():
+        return eng.generate([PROMPT], SamplingParams(max_tokens=3))[0] \
+            .output_token_ids
+
+    def forward(self, ids, meta, kv_caches):
+        seen.append(cls.forward(self, ids, meta, kv_caches).shape)
+        return cls.forward(self, ids, meta, kv_caches)
+
+    want = tokens()
+    model.__class__ = type("Own", (cls,), {"forward": forward})
+    assert tokens() == want
+    model.__class__ = cls
+    model.forward = lambda *args: forward(model, *args)
+    assert tokens() == want
+    del model.forward
+    hook = model.register_forward_hook(
+        lambda _, args, out: seen.append(out.shape))
+    assert tokens() == want
+    hook.remove()
+    width = model.cfg.hidden_size
+    assert seen == 3 * [(len(PROMPT), width), (1, width), (1, width)]
