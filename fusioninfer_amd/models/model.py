@@ -859,7 +859,8 @@ class CausalLM(nn.Module):
             return hidden, residual
         if rows is not None:
             if rows.numel() == 0:
-                return residual.new_empty((0, residual.shape[1]))
+                return self.final_norm_weight.new_empty(
+                    (0, residual.shape[1]))
             hidden = None if hidden is None else hidden[rows]
             residual = residual[rows]
         if hidden is None:

@@ -10,6 +10,7 @@ from torch import nn
 from fusioninfer_amd.config import CacheConfig, EngineConfig, SchedulerConfig
 from fusioninfer_amd.engine.llm_engine import LLMEngine
 from fusioninfer_amd.engine.sequence import SamplingParams
+from fusioninfer_amd.models.model import DecoderLayer
 from fusioninfer_amd.models.registry import get_model_config
 
 PROMPT = [3, 1, 4, 1, 5, 9, 2, 6, 5]
@@ -134,3 +135,23 @@ def test_models_forward_as_ever():
     hook.remove()
     width = model.cfg.hidden_size
     assert seen == 3 * [(len(PROMPT), width), (1, width), (1, width)]
+
+
+@pytest.mark.parametrize("stream", [False, True])
+def test_no_row_wanted(stream, monkeypatch):
+    """Nothing, in the model's type, of a stream that is kept in fp32 too."""
+    eng = make_engine()
+    model = eng.runner.model
+    if stream:
+        monkeypatch.setattr(
+            DecoderLayer, "forward",
+            lambda self, hidden, residual, *_, **__: (None, (
+                hidden if residual is None else residual).float()))
+    else:
+        monkeypatch.setattr(
+            DecoderLayer, "forward",
+            lambda self, hidden, residual, *_, **__: (hidden, hidden))
+    got = model(torch.tensor(PROMPT), None, eng.runner.kv_caches,
+                rows=torch.empty(0, dtype=torch.long))
+    assert got.shape == (0, model.cfg.hidden_size)
+    assert got.dtype == torch.bfloat16
