@@ -1103,7 +1103,7 @@ def moe_combine_norm(y, pos, w, residual, weight, eps: float):
     pass: (rows, residual)."""
     T, H = residual.shape
     if (residual.dtype == y.dtype == weight.dtype == torch.bfloat16
-            and H % 8 == 0 and H <= 8192 and y.is_contiguous()
+            and H % 8 == 0 and H <= 8192 and len(y) > 0 and y.is_contiguous()
             and residual.is_contiguous() and weight.is_contiguous()
             and residual.is_cuda
             and (residual.data_ptr() | weight.data_ptr() | y.data_ptr()) % 16

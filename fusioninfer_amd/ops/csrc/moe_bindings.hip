@@ -185,6 +185,8 @@ void moe_combine_norm(at::Tensor out, at::Tensor residual, at::Tensor norm,
                   H <= 8192,
               "moe_combine_norm: unsupported sizes");
   if (T == 0) return;
+  // the kernel reads row 0 for an expert that is not there
+  TORCH_CHECK(y.size(0) > 0, "moe_combine_norm: no rows");
   const int topk = pos.numel() / T;
   TORCH_CHECK(pos.numel() == T * topk && w.numel() == T * topk);
   fi::launch_moe_combine_norm(bf16_ptr(out), bf16_ptr(residual),

@@ -1215,6 +1215,18 @@ def test_moe_combine_norm(T, top, H):
             ).all()
 
 
+def test_moe_combine_norm_of_no_rows():
+    """No expert has a row for any token: the residual alone, and its norm."""
+    g = torch.Generator().manual_seed(5)
+    old = torch.randn(3, 64, generator=g).bfloat16().to(DEV)
+    norm = torch.randn(64, generator=g).bfloat16().to(DEV)
+    out, res = ops.moe_combine_norm(
+        old[:0], torch.full((3, 2), -1, dtype=torch.int32, device=DEV),
+        torch.ones(6, device=DEV), old.clone(), norm, 1e-6)
+    assert torch.equal(res, old)
+    assert torch.equal(out, ops.rms_norm(old, norm, 1e-6))
+
+
 def test_moe_combine_past_the_caches():
     """More rows than the memory-side cache holds give the bits of the same
     tokens in shorter calls; what rows that nobody has hold does not matter."""
