@@ -251,7 +251,8 @@ __global__ __launch_bounds__(256) void stream_begin_kernel(
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[j] = bf16_to_f32(h.h[j]);
     }
-    const bf16x8 g = *reinterpret_cast<const bf16x8*>(weight + col);
+    bf16x8 g;
+    __builtin_memcpy(&g, weight + col, sizeof(g));   // on any grid
     bf16x8 y;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {

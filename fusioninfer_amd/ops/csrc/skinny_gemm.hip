@@ -232,7 +232,8 @@ void skinny_gemm_kernel(void* __restrict__ out_p, const u16* __restrict__ x,
     bf16x4 g;
     if (MODE == ADD && mine_to_store) {
       old = *reinterpret_cast<const floatx4*>(out + m * out_stride + n);
-      if (norm != nullptr) g = *reinterpret_cast<const bf16x4*>(norm + n);
+      if (norm != nullptr)
+        __builtin_memcpy(&g, norm + n, sizeof(g));   // on any grid
     }
     floatx4 acc[RF];
 #pragma unroll

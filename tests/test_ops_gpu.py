@@ -1458,6 +1458,32 @@ def test_stream_add(rows, n, k):
             <= want.abs() * 2 ** -8).all()
 
 
+@pytest.mark.parametrize("offset", [1, 2, 4, 7])
+def test_stream_norms_weight_on_any_grid(offset):
+    """A norm's weight may begin anywhere, as in rms_norm: the bits are those
+    of a weight on the 16-byte grid."""
+    g = torch.Generator().manual_seed(offset)
+    n, k, rows = 2576, 256, 5
+    w = torch.randn(n, k, generator=g).to(torch.bfloat16).to(DEV)
+    x = torch.randn(rows, k, generator=g).to(torch.bfloat16).to(DEV)
+    begun = torch.randn(rows, n, generator=g).to(torch.bfloat16).to(DEV)
+    flat = torch.randn(n + 8, generator=g).to(torch.bfloat16).to(DEV)
+    norm = flat[offset:offset + n]
+
+    def run(weight):
+        first = ops.stream_begin(begun, weight, 1e-6)
+        got = [first.scaled.clone(), first.squares[:, :rows].clone()]
+        then = ops.stream_add_(first.stream, x, w, weight, 1e-6)
+        return [*got, then.scaled, then.squares[:, :rows], then.stream,
+                ops.stream_norm(then.stream, weight, 1e-6)]
+
+    assert norm.data_ptr() % 16 != 0
+    for a, b in zip(run(norm), run(norm.clone())):
+        assert torch.equal(a, b)
+    assert torch.equal(ops.rms_norm(begun, norm, 1e-6),
+                       ops.rms_norm(begun, norm.clone(), 1e-6))
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("rows", [17, 32, 33, 64, 65, 128, 129, 192, 193, 256])
 @pytest.mark.parametrize("n,k", [
