@@ -1484,32 +1484,41 @@ def test_stream_norms_weight_on_any_grid(offset):
                        ops.rms_norm(begun, norm.clone(), 1e-6))
 
 
-@pytest.mark.parametrize("fp8", [False, True])
-@pytest.mark.parametrize("rows", [17, 32, 33, 64, 65, 128, 129, 192, 193, 256])
-@pytest.mark.parametrize("n,k", [
-    (4096, 4096), (2064, 4608),   # a tile that is not full
-    (1040, 512),                  # few parts, fewer stages in each
-    (8208, 1024), (12304, 256),
-    (16400, 256),                 # rows longer than the kernel takes
+@pytest.mark.parametrize("fp8,rows", [
+    (fp8, rows) for rows in (1, 16, 17, 32, 33, 64, 65, 128, 129, 192, 193,
+                             256) for fp8 in (False, True)
+    if rows <= 128 or not fp8])
+@pytest.mark.parametrize("n,k,most,most_fp8", [
+    (4096, 4096, 256, 128),
+    (2064, 4608, 256, 128),    # a tile that is not full
+    (1040, 512, 256, 32),      # few parts, fewer stages in each
+    (5136, 5120, 256, 128),    # two turns of a workgroup along a row
+    (8208, 8192, 256, 128), (12304, 8192, 256, 128),   # four
+    (16384, 8192, 256, 0),     # the longest row; of e4m3 by whole tiles
+    (16400, 8192, 0, 0),       # longer than the kernel takes, if cut
+    (8208, 1024, 0, 0),        # whole tiles
 ])
-def test_linear_in_parts_and_norm(rows, n, k, fp8):
+def test_linear_in_parts_and_norm(rows, n, k, most, most_fp8, fp8):
     """The sum of a residual and a product in parts, and its norm, against
     float64: fp32 sums of k products; the sum and the normed row are rounded to
     bf16 once (2^-9 relative), or the row to e4m3 (2^-4, 2^-10 of the scale
     where it is smallest). Nothing is written behind the last row, nor anything
-    at all where another way is taken."""
-    if fp8 and rows > 128:
-        pytest.skip("more rows than the e4m3 kernels take")
-    g = torch.Generator().manual_seed(n + k + rows)
-    x = torch.randn(rows, k, generator=g).to(torch.bfloat16).to(DEV)
-    w = torch.randn(n, k, generator=g).to(torch.bfloat16).to(DEV)
-    norm = torch.randn(n, generator=g).to(torch.bfloat16).to(DEV)
-    old = (torch.randn(rows + 1, n, generator=g) * k ** 0.5).to(
-        torch.bfloat16).to(DEV)
+    at all where another way is taken: of more than `most` rows, of up to 16 in
+    bf16."""
+    g = torch.Generator(device=DEV).manual_seed(n + k + rows)
+
+    def randn(*shape):
+        return torch.randn(*shape, generator=g, device=DEV)
+
+    x = randn(rows, k).to(torch.bfloat16)
+    w = randn(n, k).to(torch.bfloat16)
+    norm = randn(n).to(torch.bfloat16)
+    old = (randn(rows + 1, n) * k ** 0.5).to(torch.bfloat16)
     residual = old.clone()
     if fp8:
         x, xs = ops.quant_fp8_rows(x)
-        w, ws = w.to(torch.float8_e4m3fn), torch.rand(n, generator=g).to(DEV)
+        w, ws = w.to(torch.float8_e4m3fn), torch.rand(n, generator=g,
+                                                      device=DEV)
         prod = (x.double() * xs.double()[:, None]) @ (
             w.double() * ws.double()[:, None]).T
         out = torch.ones(rows + 1, n, device=DEV).to(x.dtype)
@@ -1526,12 +1535,11 @@ def test_linear_in_parts_and_norm(rows, n, k, fp8):
                                          norm, 1e-6)
         got = out[:rows].double()
         assert (out[rows] == 7.0).all()
+    assert done == (rows <= most_fp8 if fp8 else 16 < rows <= most)
     if not done:
-        # (so few values, or so many tiles, that one kernel does)
-        assert (n, k) in ((1040, 512), (8208, 1024), (12304, 256),
-                          (16400, 256)) and torch.equal(residual, old)
+        assert torch.equal(residual, old)
         return
-    assert n <= 16384 and torch.equal(residual[rows], old[rows])
+    assert torch.equal(residual[rows], old[rows])
     want = prod + old[:rows].double()
     err = 1e-4 * k ** 0.5
     assert ((residual[:rows].double() - want).abs()
@@ -1576,23 +1584,27 @@ def test_linear_gelu(rows, n, k):
     assert taken is not None or rows > 16
 
 
-@pytest.mark.parametrize("rows", [17, 43, 64, 65, 129, 193, 256])
-@pytest.mark.parametrize("hq,hk,d,k,bias,norm,fp8", [
-    (32, 8, 128, 4096, False, True, False),
-    (32, 4, 128, 2048, True, False, True),
-    (14, 2, 64, 3584, True, True, False),
-    (9, 1, 64, 512, False, False, True),     # heads that fill no wave
-    (70, 5, 128, 1024, False, True, False),  # two workgroups a token
+@pytest.mark.parametrize("rows", [16, 17, 43, 64, 65, 129, 193, 256])
+@pytest.mark.parametrize("hq,hk,d,k,bias,norm,fp8,cut", [
+    (32, 8, 128, 4096, False, True, False, True),
+    (32, 4, 128, 2048, True, False, True, True),
+    (14, 2, 64, 3584, True, True, False, True),
+    (9, 1, 64, 512, False, False, True, True),     # heads that fill no wave
+    (70, 5, 128, 8192, False, True, False, True),  # two workgroups a token
+    (70, 5, 128, 8192, True, True, True, True),
+    (70, 5, 128, 1024, False, True, False, False),   # whole tiles
 ])
-def test_linear_in_parts_to_heads(rows, hq, hk, d, k, bias, norm, fp8):
+def test_linear_in_parts_to_heads(rows, hq, hk, d, k, bias, norm, fp8, cut):
     """Queries, keys and values of a product in parts, normed, rotated and in
     the cache, against float64: fp32 sums of k products, which the norm scales,
     each result rounded to bf16 once (2^-9 relative), to e4m3 once more (2^-4,
-    2^-10 where it is smallest). Rows without a slot are not kept."""
+    2^-10 where it is smallest). Rows without a slot are not kept. Of up to 16
+    rows, or where the product is not cut, nothing is done."""
     g = torch.Generator().manual_seed(rows + hq + d + k)
     n, bs = (hq + 2 * hk) * d, 16
     x = torch.randn(rows, k, generator=g).to(torch.bfloat16).to(DEV)
-    w = (torch.randn(n, k, generator=g) * k ** -0.5).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(n, k, device=DEV, generator=torch.Generator(
+        device=DEV).manual_seed(k)) * k ** -0.5).to(torch.bfloat16)
     b = torch.randn(n, generator=g).to(torch.bfloat16).to(DEV) if bias \
         else None
     qw, kw = (torch.rand(2, d, generator=g) + 0.5).to(torch.bfloat16).to(DEV) \
@@ -1609,8 +1621,10 @@ def test_linear_in_parts_to_heads(rows, hq, hk, d, k, bias, norm, fp8):
         q[:rows], x, w, b, qw, kw, cs, pos, kc, vc, slots.to(DEV), hq, 1e-6,
         0.5, 2.0)
     assert (q[rows] == 7.0).all()
+    assert done == (cut and rows > 16)
     if not done:
-        assert k <= 1024 and not kc.float().any() and (q == 7.0).all()
+        assert not kc.float().any() and not vc.float().any()
+        assert (q == 7.0).all()
         return
     heads = x.double() @ w.double().T + (0.0 if b is None else b.double())
     heads = heads.view(rows, hq + 2 * hk, d)
