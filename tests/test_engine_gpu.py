@@ -4,6 +4,7 @@ on the real HIP kernels with a small Qwen3-architecture model."""
 import pytest
 import torch
 
+import fusioninfer_amd.ops as ops
 from fusioninfer_amd.config import CacheConfig, EngineConfig, SchedulerConfig
 from fusioninfer_amd.engine.block_manager import BlockManager
 from fusioninfer_amd.engine.llm_engine import LLMEngine
@@ -13,11 +14,9 @@ from fusioninfer_amd.models.registry import get_model_config
 pytestmark = pytest.mark.gpu
 
 
-def make_engine(enforce_eager, num_blocks=512, max_seqs=16, fp8=False):
+def make_engine(enforce_eager, num_blocks=512, max_seqs=16):
     mc = get_model_config("Qwen3-0.6B")
     mc.num_layers = 4
-    if fp8:
-        mc.quantization = "fp8"
     cfg = EngineConfig(
         model=mc,
         cache=CacheConfig(num_gpu_blocks=num_blocks),
@@ -402,35 +401,251 @@ def test_gpu_embeddings():
     assert vs[0] != vs[1]
 
 
+def make_wide_engine(layers=2, fp8=False, fp8_kv=False, bias=False,
+                     enforce_eager=True):
+    """Widths at which steps of 17 rows and more have their norms and rotation
+    in the linear layers' second kernels; weights of norms, biases and scales
+    of the cache that no two places share."""
+    mc = get_model_config("Qwen3-8B")
+    mc.num_layers, mc.vocab_size = layers, 2048
+    mc.attention_bias, mc.qk_norm = bias, not bias
+    mc.quantization = "fp8" if fp8 else None
+    eng = LLMEngine(EngineConfig(
+        model=mc,
+        cache=CacheConfig(num_gpu_blocks=128,
+                          kv_cache_dtype="fp8" if fp8_kv else "auto"),
+        scheduler=SchedulerConfig(
+            max_num_seqs=4, max_num_batched_tokens=512, max_model_len=256),
+        seed=7, enforce_eager=enforce_eager,
+    ), device="cuda:0")
+    g = torch.Generator(device="cuda:0").manual_seed(11)
+    for name, p in eng.runner.model.named_parameters():
+        if name.endswith("norm_weight"):
+            p.data.copy_(1 + 0.5 * torch.rand(
+                p.shape, generator=g, device=p.device))
+        elif name.endswith("bias"):
+            p.data.normal_(generator=g)
+    for layer in eng.runner.model.layers if fp8_kv else ():
+        layer.self_attn.k_scale, layer.self_attn.v_scale = 0.25, 0.5
+    return eng
+
+
+def states_of(eng, ids):
+    """Of all rows behind the last norm, in a step of one prompt."""
+    runner = eng.runner
+    bm = BlockManager(runner.num_gpu_blocks, eng.cfg.cache.block_size)
+    seq = Sequence("s", ids, SamplingParams())
+    bm.allocate(seq)
+    tokens, meta, _ = runner._prefill_inputs(
+        runner.build_prefill_payload([seq], bm))
+    with torch.no_grad():
+        return runner.model(tokens, meta, runner.kv_caches)
+
+
+def exact_states(model, ids):
+    """The same in float64 by torch alone, nothing rounded on the way."""
+    cfg, rows = model.cfg, len(ids)
+
+    def norm(x, weight):
+        return (x * (x.square().mean(-1, keepdim=True)
+                     + cfg.rms_norm_eps).rsqrt() * weight.double())
+
+    def linear(x, layer):
+        w = layer.weight.double()
+        if hasattr(layer, "weight_scale"):
+            w = w * layer.weight_scale.double()[:, None]
+        y = x @ w.T
+        bias = getattr(layer, "bias", None)
+        return y if bias is None else y + bias.double()
+
+    cos, sin = (t[:, None] for t in
+                model.cos_sin[:rows].double().chunk(2, dim=-1))
+
+    def turn(x):
+        a, b = x.chunk(2, dim=-1)
+        return torch.cat([a * cos - b * sin, b * cos + a * sin], -1)
+
+    x = model.embed_tokens[torch.tensor(ids, device="cuda:0")].double()
+    late = torch.ones(rows, rows, device="cuda:0").triu(1).bool()
+    for layer in model.layers:
+        a = layer.self_attn
+        qkv = linear(norm(x, layer.input_norm_weight), a.qkv_proj)
+        q, k, v = (t.view(rows, -1, a.head_dim) for t in qkv.split(
+            [a.q_size, a.kv_size, a.kv_size], -1))
+        if a.q_norm_weight is not None:
+            q, k = norm(q, a.q_norm_weight), norm(k, a.k_norm_weight)
+        out = torch.empty_like(q)
+        k = turn(k)
+        for h, qh in enumerate(turn(q).unbind(1)):
+            group = h * a.num_kv_heads // a.num_heads
+            scores = (qh @ k[:, group].T * a.scale).masked_fill(
+                late, float("-inf"))
+            out[:, h] = scores.softmax(-1) @ v[:, group]
+        x = x + linear(out.flatten(1), a.o_proj)
+        gate, up = linear(norm(x, layer.post_norm_weight),
+                          layer.mlp.gate_up_proj).chunk(2, -1)
+        x = x + linear(torch.nn.functional.silu(gate) * up,
+                       layer.mlp.down_proj)
+    return norm(x, model.final_norm_weight)
+
+
+def distance(got, want):
+    assert got.dtype == torch.bfloat16
+    return float((got.double() - want).norm() / want.norm())
+
+
+def one_after_another(call):
+    """What call gives while a hook looks at every module, so that no kernel
+    does the work of two."""
+    hook = torch.nn.modules.module.register_module_forward_hook(
+        lambda *_: None)
+    try:
+        return call()
+    finally:
+        hook.remove()
+
+
+def rounding_bound(layers, fp8, fp8_kv=False):
+    """Of a state's distance from float64: eleven roundings to bf16 a layer of
+    2^-9 at most, added up, and beside them four to e4m3 of 2^-4, in an e4m3
+    cache two, of either sign and so by their squares."""
+    return layers * 11 * 2 ** -9 + (
+        layers * (4 * fp8 + 2 * fp8_kv)) ** 0.5 * 2 ** -4
+
+
+@pytest.mark.parametrize("rows,fp8,fp8_kv,bias,taken", [
+    (1, False, False, False, {"few_rows_scaled_gemm": 4,
+                              "few_rows_gemm_add": 4}),
+    (16, False, False, True, {"few_rows_scaled_gemm": 4,
+                              "few_rows_gemm_add": 4}),
+    (16, False, True, False, {"few_rows_scaled_gemm": 4,
+                              "few_rows_gemm_add": 4}),
+    (17, False, False, False, {"few_rows_gemm_rope": 2,
+                               "few_rows_gemm_norm": 3}),
+    (43, False, True, False, {"few_rows_gemm_rope": 2,
+                              "few_rows_gemm_norm": 3}),
+    (128, False, True, True, {"few_rows_gemm_rope": 2,
+                              "few_rows_gemm_norm": 3}),
+    (1, True, False, False, {"few_rows_gemm_norm_fp8": 3}),
+    (16, True, True, False, {"few_rows_gemm_norm_fp8": 3}),
+    (32, True, False, True, {"few_rows_gemm_norm_fp8": 3}),
+    (43, True, False, False, {"few_rows_gemm_norm_fp8": 1}),
+    (100, True, False, False, {"few_rows_gemm_norm_fp8": 1}),
+])
+def test_layers_with_norms_in_their_products(rows, fp8, fp8_kv, bias, taken,
+                                             monkeypatch):
+    """Two layers by the kernels that go on from a product, which are counted
+    where they did (the last layer's down projection has no norm behind it),
+    against float64: no further from it than one kernel after another, which is
+    what a hook everywhere gives, but for the scatter of the roundings that one
+    of the two has (a quarter for one row, a twentieth for more). A norm's
+    weight in the wrong places alone is 0.15 off, which adds to the roundings
+    by squares: 0.2 where these are most, 0.13 in e4m3 with its cache."""
+    eng = make_wide_engine(fp8=fp8, fp8_kv=fp8_kv, bias=bias)
+    model = eng.runner.model
+    ids = [(7 * i + 3) % 2048 for i in range(rows)]
+    want = exact_states(model, ids)
+
+    def error():
+        return distance(states_of(eng, ids), want)
+
+    count = dict.fromkeys(("few_rows_scaled_gemm", "few_rows_gemm_add",
+                           "few_rows_gemm_rope", "few_rows_gemm_norm",
+                           "few_rows_gemm_norm_fp8"), 0)
+
+    def counted(name, kernel):
+        def call(*args):
+            done = kernel(*args)
+            count[name] += done is None or done
+            return done
+        return call
+
+    for name in count:
+        monkeypatch.setattr(ops._C, name, counted(name, getattr(ops._C, name)))
+    fused = error()
+    assert {k: n for k, n in count.items() if n} == taken
+    apart = one_after_another(error)
+    assert {k: n for k, n in count.items() if n} == taken
+    assert apart <= rounding_bound(2, fp8, fp8_kv)
+    most = 1.25 if rows == 1 else 1.05
+    assert fused <= most * apart
+    weight = model.layers[1].post_norm_weight
+    weight.data.copy_(weight.data.roll(1))
+    assert error() > 1.25 * most * apart
+
+
+def test_layers_of_which_some_stream_in_a_graph():
+    """A layer with a hook between two that keep the residual stream in fp32:
+    replays of a captured step, other work between them, give the bits of the
+    same step run eagerly; and those of a graph without the hook differ."""
+    eng = make_wide_engine(layers=3, bias=True, enforce_eager=False)
+    runner = eng.runner
+    bm = BlockManager(runner.num_gpu_blocks, eng.cfg.cache.block_size)
+    seqs = []
+    for i in range(3):
+        seq = Sequence(f"s{i}", list(range(20 + i, 60 + 7 * i)),
+                       SamplingParams())
+        bm.allocate(seq)
+        logits = runner.execute_prefill([seq], bm)
+        seq.output_token_ids = [int(logits.argmax(-1)[0])]
+        bm.append_slot(seq)
+        seqs.append(seq)
+
+    def step(n):
+        return runner.execute_decode(seqs[:n], bm).clone()
+
+    whole = {n: step(n) for n in (1, 2)}
+    hook = runner.model.layers[1].self_attn.register_forward_hook(
+        lambda *_: None)
+    runner.capture_decode_graphs()
+    first = {n: step(n) for n in (1, 2)}
+    graphs, runner._graphs = runner._graphs, {}
+    eager = {n: step(n) for n in (1, 2)}
+    runner._graphs = graphs
+    again = {n: step(n) for n in (2, 1)}
+    hook.remove()
+    for n in (1, 2):
+        assert torch.equal(first[n], eager[n])
+        assert torch.equal(again[n], eager[n])
+        assert not torch.equal(first[n], whole[n])
+        assert (first[n].float() - whole[n].float()).norm() \
+            <= 0.03 * whole[n].float().norm()
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("length", [15, 42])
 def test_layers_whose_norms_are_apart(length, fp8):
     """A layer whose parts are hooked takes its norms and sums one by one, next
     to layers that have them in the linear layers' kernels, and the hook sees
-    each call. The states differ by roundings to bf16, eleven a layer of 2^-9
-    each, in the fp8 mode by four to e4m3 of 2^-4."""
-    eng = make_engine(enforce_eager=True, fp8=fp8)
-    prompt = [[5, 6, 7] * (length // 3)]
-    want = torch.tensor(eng.embed(prompt)[0])
+    each call. However they are mixed, the states are no further from float64
+    than one kernel after another, but for the scatter of roundings (a tenth);
+    with a norm's weight in the wrong places they are."""
+    eng = make_wide_engine(layers=4, fp8=fp8)
     layers = eng.runner.model.layers
-    for hooked in ([1], [0, 2], [3], [0, 1, 2, 3]):
+    ids = [(7 * i + 3) % 2048 for i in range(length)]
+    want = exact_states(eng.runner.model, ids)
+    apart = one_after_another(lambda: distance(states_of(eng, ids), want))
+    assert apart <= rounding_bound(4, fp8)
+    for hooked in ([], [1], [0, 2], [3], [0, 1, 2, 3]):
         seen = []
         hooks = [
             layers[i].self_attn.o_proj.register_forward_hook(
                 lambda *_, i=i: seen.append(i)) for i in hooked]
-        got = torch.tensor(eng.embed(prompt)[0])
+        got = states_of(eng, ids)
         for h in hooks:
             h.remove()
         assert seen == hooked
-        bound = 11 * 2 ** -9 + (4 * 2 ** -4 if fp8 else 0)
-        assert (got - want).norm() <= len(layers) * bound
+        assert distance(got, want) <= 1.1 * apart
     # from outside a layer passes rows and residual, as ever
     seen = []
     hook = layers[1].register_forward_hook(
         lambda _, args, out: seen.extend([*args[:2], *out]))
-    got = torch.tensor(eng.embed(prompt)[0])
+    got = states_of(eng, ids)
     hook.remove()
     assert len(seen) == 4 and all(
         type(t) is torch.Tensor and t.dtype == torch.bfloat16
         and t.shape[0] == length for t in seen)
-    assert (got - want).norm() <= len(layers) * bound
+    assert distance(got, want) <= 1.1 * apart
+    weight = layers[1].post_norm_weight
+    weight.data.copy_(weight.data.roll(1))
+    assert distance(states_of(eng, ids), want) > 1.25 * 1.1 * apart
