@@ -85,37 +85,76 @@ def _streams(M: int, N: int, K: int, silu_mul: bool = False) -> bool:
     with the library.
 
     Up to 128 rows the kernel's own estimate (tiles, parts, joins) is held
-    against what the library is seen to take: up to 64 rows W at 2.5 TB/s
-    and 6 us, above them 5 us and W at 4 TB/s or, where N gives it few tiles,
-    the chain of 7 us per 1000 of K; with silu_mul 3 us more for the pass
-    over the product. (Where that errs most: 14336 x 5120 at 64 rows streams
-    in 38 us, the library takes 32. Where the two are even, 5120 x 2048 and
-    2048 x 4096 at 64 rows 13.5 and 13.8 us, 12.9 and 14.2, a step of four such
-    layers takes 10 us less with streaming.)
+    against what the library is seen to take: up to 64 rows W at 3.2 TB/s or
+    4.2 us per 1000 of K, and 4.4 us, above them 3.6 TB/s or 3.8 us, and 8;
+    with silu_mul 3 us or 1.2 more for the pass over the product. (Where that
+    errs most: 12288 x 2560 at 128 rows streams in 26.4 us, the library takes
+    23.2.)
 
-    From 129 rows on both compute more than they read. The library's choice
-    of tiles jumps with M and N there, and streaming is ahead but for few
-    values of W (2048 x 4096 at 192 rows 20.2 us, the library 16.1; 3072 x
-    5120 24.8 and 41.6; 4096 x 4096 at 256 24.2 and 22.0; 6144 x 4096 29 and
-    40), short rows (49152 x 1024 at 256 40 and 31) and N at which the
-    library's tiles fill the chip exactly (49152 x 4096 at 256 125 and 107).
-
-    Weights that no cache holds, launched from a graph, 15 N of 2048 to
-    151936, eight K of 512 to 12288: this choice takes 0.7 to 1.9 % longer
-    than the better of the two up to 128 rows, 1.9 to 3.1 % at 160 to 256;
-    the library alone 11 to 27, streaming alone 0.4 to 4. With silu_mul 0.2
-    to 1.7 %, the library alone 14 to 29."""
+    Weights that no cache holds, launched from a graph, 20 N of 1024 to
+    151936, eleven K of 1024 to 14336: with _streams_many this choice takes
+    0.7 to 1.7 % longer than the best of the library, parts in any shape and
+    tiles up to 128 rows, 1.7 to 2.0 % at 144 to 192 and 3.4 to 3.8 at 224
+    and 256; the library alone 13 to 22. With silu_mul 0.8 to 1.0 % and 2.3
+    to 3.9, the library alone 18 to 32."""
     if M <= SKINNY_ROWS:
         return True
     if M > PART_ROWS or N * K < 1 << 23 or K < 2048 and N <= 8192:
         return False
     if M > 128:
-        if silu_mul:
-            return K >= 2048 or N <= 96 * 256
-        return K >= 2048 and N * K >= (3 << 22 if M <= 192 else 5 << 22)
-    library = (6 + 2 * N * K / 2.5e6 if M <= 64
-               else 5 + max(2 * N * K / 4e6, 7e-3 * K))
-    return _C.few_rows_gemm_us(M, N, K) < library + (3 if silu_mul else 0)
+        return _streams_many(M, N, K, silu_mul)
+    if M <= 64:
+        library = 4.4 + max(2 * N * K / 3.2e6, 4.2e-3 * K) + 3 * silu_mul
+    else:
+        library = 8 + max(2 * N * K / 3.6e6, 3.8e-3 * K) + 1.2 * silu_mul
+    return _C.few_rows_gemm_us(M, N, K) < library
+
+
+def _streams_many(M: int, N: int, K: int, silu_mul: bool) -> bool:
+    """_streams from 129 rows on. There both compute more than they read, and
+    the library's choice of tiles jumps with M, N and K, so the lines are where
+    one of the two is ahead for good (us, the library and here). N above 2^15:
+    the library, but for one row of tiles where _one_row says so and W beyond
+    2^16 (57344 x 8192 at 160 and 256 rows 183 and 226, 217 and 260; 40960 x
+    4096 at 256 93 and 108; 151936 x 4096 at 256 361 and 303). Few values of W,
+    short rows and N 12289 to 16384: the library (2048 x 4096 at 192 16.0 and
+    21.0, 4096 x 2048 at 256 13.7 and 20.2, 16384 x 2560 at 144 28.6 and 32.9);
+    what it has tiles for at few rows too: up to 144 (8192 x 2048 15.7 and
+    21.1, 6144 x 4096 39.6 and 24.4), up to 160 (3072 x 4096 16.6 and 21.2, 4096
+    x 4096 27.2 and 21.6). With silu_mul here: the pass over the product costs
+    the library 3 to 10."""
+    if K < 2048 and (N > 96 * 256 or not silu_mul):
+        return False
+    if N > 1 << 15:
+        return not (N <= 1 << 16 and K >= 8192) and (
+            silu_mul or N > 1 << 16 or _one_row(M, N, K, silu_mul))
+    if silu_mul:
+        return True
+    if N * K < 3 << 22 or 12288 < N <= 1 << 14 and N * K <= 3 << 24:
+        return False
+    if M > 192:
+        return N * K >= 5 << 22 and K > 2048
+    if M > 160 or K >= 6144:
+        return True
+    if M > 144:
+        return N > 1 << 14 or K >= 2560 and N * K >= 1 << 24
+    return N >= 12288 or N <= 6144 and N * K >= 1 << 24
+
+
+def _one_row(M: int, N: int, K: int, silu_mul: bool) -> bool:
+    """Of 129 to 256 rows, whether one row of 256 x 256 tiles is ahead of
+    parts, by the two kernels' own estimates: wide W, where the chip has whole
+    rounds of tiles (151936 x 4096 at 160 and 256 rows 306 and 343 us in parts,
+    273 and 300 so). Up to 2^16 long K is the library's: 57344 x 4096 at 256
+    rows 117 us here, 116 there, 57344 x 5120 at 160 139 and 126; with silu_mul
+    40960 x 2048 at 256 52, the library 61, in parts 59."""
+    if N <= 1 << 16:
+        ok = N >= (40960 if silu_mul else 49152) and (
+            K <= 4096 or silu_mul and N >= 57344 and K < 8192)
+    else:
+        ok = N <= 1 << 20 and K < 8192
+    return ok and (_C.many_rows_gemm_us(M, N, 2 * K)
+                   < _C.few_rows_gemm_us(M, N, K))
 
 
 def _memory_alone(x, w, bias) -> bool:
@@ -222,19 +261,13 @@ def _tiles_ok(x, w, unit: int, silu_mul: bool = False, bias=None) -> bool:
     )
 
 
-def _one_row_of_tiles(x, w, bias=None) -> bool:
-    """Whether 129 to 256 rows that stream go by tiles of 256 x 256 for it: wide
-    W, where the chip has whole rounds of those, by the two kernels' own
-    estimates. 151936 x 4096 at 129 and 256 rows 300 and 349 us in parts, 258
-    and 302 so; 98304 x 3072 at 256 174 and 169; 40960 x 5120 at 256, where the
-    estimates are even, 141 and 144; from K 8192 on the tiles wait for memory
-    (49152 x 8192 at 256 216 and 294). 14 N, seven K, three numbers of rows: 0.9
-    % above the better one on average, parts alone 3.1."""
+def _one_row_of_tiles(x, w, bias=None, silu_mul: bool = False) -> bool:
+    """Whether 129 to 256 rows that stream go by tiles of 256 x 256 for it."""
     M, N, K = x.shape[0], w.shape[0], w.shape[1]
     return (
-        M > 128 and 40960 <= N <= 1 << 20 and K < 8192 and x.stride(0) >= K
+        M > 128 and x.stride(0) >= K
         and (bias is None or bias.data_ptr() % 16 == 0)
-        and _C.many_rows_gemm_us(M, N, 2 * K) < _C.few_rows_gemm_us(M, N, K)
+        and _one_row(M, N, K, silu_mul)
     )
 
 
@@ -260,23 +293,25 @@ def linear(x: torch.Tensor, w: torch.Tensor,
 
 
 def _streams_fp8(M: int, N: int, K: int) -> bool:
-    """As _streams, for e4m3 operands with scales per row. Up to 32 rows the
-    library is behind at nearly all sizes (24576 x 4096 at 32 rows 24 us, 20
-    here; 8192 x 8192 20 and 24.8); up to 64 rows it takes W at 4.5 TB/s and 5
-    us or 2 us per 1000 of K (6144 x 4096 at 64 13.1 and 15, 4096 x 12288 23.5
-    and 19.7). From 65 rows on it is ahead but for long K and few tiles (4096
-    x 12288 at 96 and 128 rows 20 and 27, here 17 and 20). Ten N and six K,
-    launched from a graph: this choice takes 0.7 to 2.7 % longer than the
-    better of the two up to 64 rows (the library alone 8 to 32, streaming
-    alone 0.7 to 3.1), 0.2 % at 96 and 128."""
+    """As _streams, for e4m3 operands with scales per row. Up to 16 rows the
+    library is behind at nearly all sizes (24576 x 4096 at 16 rows 30 us, 19
+    here); up to 64 rows it takes W at 4.7 TB/s and 7.8 us or 2.2 us per 1000
+    of K (6144 x 4096 at 64 13.5 and 14.8, 4096 x 12288 24.2 and 18.0), and
+    less for few values of W (2560 x 4096 9.4 and 11.7). From 65 rows on it
+    is ahead but for long K and few tiles (4096 x 12288 at 96 and 128 rows 30
+    and 36, here 24 and 25). Twelve N and eleven K, launched from a graph:
+    this choice takes 0.3 to 1.7 % longer than the best of the two up to 96
+    rows (the library alone 10 to 48), 2.0 at 128."""
     if M > 128 or N * K < 1 << 23:
         return False
-    if M <= 32:
+    if M <= SKINNY_ROWS:
         return True
     if M > 64:
         return M >= 96 and K >= 2 * N and N >= 3072
-    return _C.few_rows_gemm_us(M, N, K // 2) < max(N * K / 4.5e6 + 5,
-                                                   2e-3 * K)
+    if M > 32 and N * K < 3 << 22:
+        return False
+    return _C.few_rows_gemm_us(M, N, K, True) < max(7.8 + N * K / 4.7e6,
+                                                    0.6 + 2.2e-3 * K)
 
 
 def _tiles_fp8(M: int, N: int, K: int) -> bool:
@@ -360,7 +395,7 @@ def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if _skinny_ok(x, w, 32, True):
         out = torch.empty((x.shape[0], w.shape[0] // 2), dtype=x.dtype,
                           device=x.device)
-        if _one_row_of_tiles(x, w):
+        if _one_row_of_tiles(x, w, silu_mul=True):
             _C.many_rows_gemm(out, x, w, None, True)
         else:
             _C.few_rows_gemm(out, x, w, None, True)

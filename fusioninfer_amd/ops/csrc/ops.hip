@@ -47,7 +47,7 @@ template <class X>
 void launch_stream_begin(float*, u16*, float*, const X*, const u16*, int, int,
                          hipStream_t);
 int64_t part_gemm_floats(int, int, int, bool);
-double part_gemm_us(int, int, int);
+double part_gemm_us(int, int, int, bool);
 bool launch_part_gemm_norm(void*, float*, u16*, const u16*, float, float*,
                            const u16*, const float*, const u16*, const float*,
                            int, int, int, int64_t, hipStream_t);
@@ -878,7 +878,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "fp32 stream += linear layer of up to 16 rows, and the next norm");
   m.def("stream_begin", &stream_begin, "fp32 stream of rows, the next norm");
   m.def("few_rows_gemm_us", &fi::part_gemm_us,
-        "estimate for M of 17 to 256 rows, N, K of 16-bit values");
+        "estimate for M of 17 to 256 rows (e4m3: 1 to 128), N, K", py::arg("M"),
+        py::arg("N"), py::arg("K"), py::arg("fp8") = false);
   m.def("many_rows_gemm", &many_rows_gemm, "x W^T by tiles of 256 x 256",
         py::arg("out"), py::arg("x"), py::arg("w"), py::arg("bias"),
         py::arg("silu_mul"), py::arg("gelu") = false);

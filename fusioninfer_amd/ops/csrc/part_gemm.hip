@@ -24,20 +24,23 @@
 // CUs), whatever the depth of the rings. Hence tiles at least as tall as x has
 // rows, taller where N allows. The second kernel of a cut product costs 4.7 us
 // at the least, and results leave by stores that the next stages' waits count
-// (151936 x 4096 at 64 rows 243 us, and 249).
+// (8192 to 12288 x 1024 to 2048 at 17 to 128 rows 0.5 to 1.5 % less; where HBM is
+// the bound nothing, 151936 x 4096 at 64 rows 249 us in whole tiles, 236 cut).
 //
-// From 129 rows on the fragment reads would be the bound, a wave of 32 x 64
-// results reading as much as it multiplies: there four waves hold a tile's rows
-// of W by a quarter of x (part_gemm_ahead_kernel), read the fragments of half a
-// stage during the products of the other half, and cross one barrier a stage.
+// From 129 rows on, and below where tiles have 128 rows, the fragment reads
+// would be the bound, a wave of 32 x 64 results reading as much as it
+// multiplies: there four waves hold a tile's rows of W by a quarter of x
+// (part_gemm_ahead_kernel), read the fragments of half a stage during the
+// products of the other half, and cross one barrier a stage.
 // Before and now at 192 rows: 24576 x 4096 with silu 57 and 50 us, 4096 x 12288
 // 43 and 38, 8192 x 8192 55 and 42; at 256 63 and 59, 45 and 43.5, 56 and 49;
 // 151936 x 4096 at 256 446 and 345, the library 358.
 //
 // Measured, us (GB/s of W) at 32 / 64 / 128 / 256 rows: N 24576, K 4096 with
-// silu 32.4 (6210) / 33.8 / 44.2 / 59, the library's GEMM and the pass behind it
-// 49 / 49 / 53 / 69; 4096, 12288 23 (4380) / 26 / 33 / 44 against 27 / 37 / 67 /
-// 55; 151936, 2048 109 (5710) / 128 / 153 / 188 against 145 / 150 / 166 / 212.
+// silu 33.4 (6030) / 33.9 / 44.3 / 58, the library's GEMM and the pass behind it
+// 48 / 49 / 53 / 70; 4096, 12288 21 (4780) / 26 / 33 / 42 against 26 / 37 / 66 /
+// 55; 151936, 2048 109 (5690) / 129 / 151 / 192 against 146 / 153 / 168 / 212 (at
+// 256 rows 176 by tiles of 256 x 256).
 //
 // Where a norm follows, the second kernel does the sum with the residual and
 // the norm too (part_gemm_norm_kernel): a launch of 3 to 5 us less, and the
@@ -48,9 +51,10 @@
 // 3333 us.
 //
 // FP8: the same kernel on e4m3 rows, 1 to 128 of them. 24576 x 4096 at 16 / 32
-// / 64 rows 19.8 (5090) / 19.9 / 23.5 us, the library's GEMM 30.1 / 25.7 /
-// 26.7; 4096 x 12288 15.0 (3350) / 15.8 / 19.7 against 19.3 / 20.5 / 24.4.
+// / 64 rows 19.3 (5210) / 19.9 / 22.7 us, the library's GEMM 30.0 / 25.3 /
+// 26.4; 4096 x 12288 13.9 (3630) / 14.5 / 18.0 against 19.2 / 20.3 / 24.2.
 
+#include <cmath>
 #include <type_traits>
 
 #include "pieces.h"
@@ -95,7 +99,7 @@ struct PartShape {
   static constexpr int LW = TN / kRowsPerDma / kWLoaders;
   static constexpr int LX = MB / kRowsPerDma / kXLoaders;
   static constexpr int kPiece = TN * MB / 4;  // float4
-  static constexpr bool kAhead = false;
+  static constexpr bool kAhead = false, kCuts = true;
   static_assert(RF % 2 == 0 && TN / 2 % kRowsPerDma == 0);
   static_assert(LW * kRowsPerDma * kWLoaders == TN &&
                 LX * kRowsPerDma * kXLoaders == MB);
@@ -772,41 +776,58 @@ void part_gemm_norm_kernel(void* __restrict__ out, float* __restrict__ out_scale
   }
 }
 
-// How a shape cuts [N, K] up and what that takes: 3 us, a time per stage of the
-// part that has most of them, and one for the second kernel and the way of the
-// pieces through memory where tiles are cut. Both times are measured, per shape
-// (17 N by six K, weights that no cache holds, 1500 runs). Whole tiles on an
-// uneven number of CUs against even parts with a join comes out of the same sum,
-// and so does the caller's choice between this kernel and the library; the
-// shape taken is 1.0 to 1.5 % slower than the best one on average.
+// us of a shape: a stage while few CUs stream and while all do, where HBM has its
+// say; what whole tiles take beside their stages; what cut ones do beside those
+// and 3 us, the second kernel and the way of the pieces through memory.
+struct Times {
+  double whole, cut, lone, full;
+};
+
+// How a shape cuts [N, K] up and what that takes by its times, which are
+// measured (20 N by eleven K, weights that no cache holds, plain, with silu and
+// e4m3, 10000 runs). Whole tiles on an uneven number of CUs against even parts
+// with a join comes out of the same sum, and so does the caller's choice between
+// this kernel and the library. Of what the best shape takes the one taken takes
+// 0.5 to 0.6 % more on average, 20 at most (65536 x 2048 with silu at 17 rows), and
+// the sum is 7 % off (one rate of a stage, whether few CUs stream or all: 1.3 %
+// more, 27 at most, and 13 % off).
 struct Plan {
   int tiles = 0, parts = 0;
   bool split = false;
   double us = 0;
 };
 
+// stage: by how much this kind of operands makes a stage longer
 template <class S>
-Plan plan_of(int N, int K, bool split) {
+Plan plan_of(int N, int K, bool split, double stage) {
   constexpr int kChip = 256;
+  constexpr Times us = S::kUs;
   Plan p;
   p.tiles = ceil_div(N, S::TN);
-  const int64_t stages = static_cast<int64_t>(p.tiles) * (K / S::KS);
   p.split = split;
+  const int64_t of_tile = K / S::KS, stages = p.tiles * of_tile;
   // two stages at least, so that the ring has something to run ahead on
   p.parts = static_cast<int>(
       std::min<int64_t>(kChip, split ? (stages + 1) / 2 : p.tiles));
-  const int64_t most = split
-      ? (stages + p.parts - 1) / p.parts
-      : static_cast<int64_t>(ceil_div(p.tiles, p.parts)) * (K / S::KS);
-  p.us = 3 + most * S::kStageUs;
-  if (split) p.us += S::kCutUs * p.parts / kChip;
+  // rounds that all CUs take part in, and the last one
+  const int rounds = split ? 1 : ceil_div(p.tiles, kChip);
+  const int64_t most = split ? (stages + p.parts - 1) / p.parts : of_tile;
+  const double busy =
+      (split ? p.parts : p.tiles - (rounds - 1) * kChip) / double{kChip};
+  const double shared = us.full * busy;
+  const double last = std::sqrt(std::sqrt(
+      us.lone * us.lone * us.lone * us.lone + shared * shared * shared * shared));
+  p.us = stage * ((rounds - 1) * most * us.full + most * last) +
+         (split ? 3 + us.cut * busy : us.whole);
   return p;
 }
 
 template <class S>
-Plan plan_of(int N, int K) {
-  const Plan a = plan_of<S>(N, K, false), b = plan_of<S>(N, K, true);
-  return a.us <= b.us ? a : b;
+Plan plan_of(int N, int K, double stage) {
+  const Plan whole = plan_of<S>(N, K, false, stage);
+  if (!S::kCuts) return whole;
+  const Plan cut = plan_of<S>(N, K, true, stage);
+  return whole.us <= cut.us ? whole : cut;
 }
 
 template <class S, bool SILU_MUL, bool FP8, bool ROWS>
@@ -837,72 +858,81 @@ void launch_part(const Plan& pl, u16* out, float* pieces, const u16* x,
   launch_products<S, SILU_MUL, FP8, false>(pl, out, pieces, x, w, bias, scales,
                                            M, N, K, x_stride, out_stride,
                                            stream);
-  if (!pl.split || pl.parts == 1) return;
-  auto* p = reinterpret_cast<const floatx4*>(pieces);
-  hipLaunchKernelGGL((part_gemm_join_kernel<S, SILU_MUL, FP8>),
-                     dim3(pl.parts - 1,
-                          ceil_div(S::kPiece / (SILU_MUL ? 2 : 1), 256)),
-                     dim3(256), 0, stream, out, p, bias, scales, M, N, K,
-                     out_stride, pl.tiles, pl.parts);
+  if constexpr (S::kCuts) {
+    if (!pl.split || pl.parts == 1) return;
+    auto* p = reinterpret_cast<const floatx4*>(pieces);
+    hipLaunchKernelGGL((part_gemm_join_kernel<S, SILU_MUL, FP8>),
+                       dim3(pl.parts - 1,
+                            ceil_div(S::kPiece / (SILU_MUL ? 2 : 1), 256)),
+                       dim3(256), 0, stream, out, p, bias, scales, M, N, K,
+                       out_stride, pl.tiles, pl.parts);
+  }
 }
 
 // Row classes and their shapes: tiles of 96 rows where the chip takes them
 // whole, 64 where N is small and K is cut, 128 or more where N is large and x
-// would be read too often. From 129 rows on by waves that read ahead.
+// would be read too often. Waves that read ahead are ahead of the others from
+// 129 rows on, and at 65 to 128 where tiles of 128 rows are.
 struct B32 : PartShape<2, 2, 2, 1, 64, 7, 7, 2> {
-  static constexpr double kStageUs = 0.325, kCutUs = 4.4;
+  static constexpr Times kUs{4.7, 3.7, 0.242, 0.303};
 };
+// (cut, these two are next to never the best, and far off where parts begin in
+// step: 10240 x 12288 at 17 rows 44 us with tiles of 64 rows, 56 with 128)
 struct A32 : PartShape<3, 2, 2, 1, 128, 5, 4, 4> {
-  static constexpr double kStageUs = 0.807, kCutUs = 6.6;
+  static constexpr Times kUs{4.8, 0, 0.555, 0.929};
+  static constexpr bool kCuts = false;
 };
 struct C32 : PartShape<4, 2, 2, 1, 128, 4, 4, 4> {
-  static constexpr double kStageUs = 1.054, kCutUs = 7.4;
+  static constexpr Times kUs{4.6, 0, 0.652, 1.21};
+  static constexpr bool kCuts = false;
 };
 struct B64 : PartShape<2, 2, 4, 1, 64, 7, 7, 4> {
-  static constexpr double kStageUs = 0.384, kCutUs = 6.5;
+  static constexpr Times kUs{5.8, 5.9, 0.277, 0.361};
 };
 struct A64 : PartShape<3, 2, 2, 2, 128, 4, 4, 4> {
-  static constexpr double kStageUs = 0.908, kCutUs = 8.3;
+  static constexpr Times kUs{6.3, 7.3, 0.617, 1.009};
 };
 struct C64 : PartShape<4, 2, 2, 2, 64, 6, 6, 4> {
-  static constexpr double kStageUs = 0.592, kCutUs = 9.3;
+  static constexpr Times kUs{6.2, 7.7, 0.412, 0.669};
 };
 struct D64 : PartShape<4, 4, 2, 2, 64, 4, 4, 4> {
-  static constexpr double kStageUs = 1.1, kCutUs = 15.7;
+  static constexpr Times kUs{5.3, 12, 0.812, 1.239};
 };
 struct B128 : PartShape<2, 2, 4, 2, 64, 7, 5, 4> {
-  static constexpr double kStageUs = 0.526, kCutUs = 8.3;
+  static constexpr Times kUs{7.2, 8.3, 0.367, 0.448};
 };
 struct A128 : PartShape<3, 2, 4, 2, 64, 7, 4, 4> {
-  static constexpr double kStageUs = 0.623, kCutUs = 11.8;
+  static constexpr Times kUs{7.7, 10.8, 0.461, 0.584};
 };
 struct C128 : AheadShape<8, 2, 6, 4> {
-  static constexpr double kStageUs = 0.692, kCutUs = 13.2;
+  static constexpr Times kUs{7.9, 10.7, 0.483, 0.759};
 };
 struct D128 : PartShape<4, 4, 2, 4, 64, 3, 4, 4> {
-  static constexpr double kStageUs = 1.158, kCutUs = 18.3;
+  static constexpr Times kUs{8.9, 16.6, 1.04, 1.348};
 };
 struct A192 : AheadShape<6, 3, 5, 4> {
-  static constexpr double kStageUs = 0.717, kCutUs = 12.5;
+  static constexpr Times kUs{6.3, 11.3, 0.563, 0.701};
 };
 struct C192 : AheadShape<8, 3, 4, 4> {
-  static constexpr double kStageUs = 0.862, kCutUs = 15.2;
+  static constexpr Times kUs{6, 13.1, 0.668, 0.911};
 };
 struct A256 : AheadShape<6, 4, 5, 3> {
-  static constexpr double kStageUs = 0.842, kCutUs = 14.1;
+  static constexpr Times kUs{7.1, 12.4, 0.665, 0.839};
 };
 struct C256 : AheadShape<8, 4, 4, 3> {
-  static constexpr double kStageUs = 0.979, kCutUs = 17.2;
+  static constexpr Times kUs{6.8, 14.6, 0.778, 1.075};
 };
-// rows of W too long for the offsets within a tile
-struct L256 : PartShape<2, 2, 8, 2, 64, 6, 3, 8> {
-  static constexpr double kStageUs = 0.717, kCutUs = 10.6;
+// for few tiles with few stages each (10240 x 2048 with silu at 256 rows 25 us, by
+// waves that read ahead 29), and rows of W too long for the others' offsets
+// within a tile
+struct B256 : PartShape<2, 2, 8, 2, 64, 6, 3, 8> {
+  static constexpr Times kUs{6.3, 11, 0.576, 0.672};
 };
 
 // calls f(shape, plan) for the shape that takes least
 template <class F, class... Shapes>
-void with_best(int N, int K, const F& f, Shapes...) {
-  const Plan plans[] = {plan_of<Shapes>(N, K)...};
+void with_best(int N, int K, double stage, const F& f, Shapes...) {
+  const Plan plans[] = {plan_of<Shapes>(N, K, stage)...};
   const Plan* best = plans;
   for (const Plan& p : plans)
     if (p.us < best->us) best = &p;
@@ -910,30 +940,35 @@ void with_best(int N, int K, const F& f, Shapes...) {
   ((best == plans + i++ ? f(Shapes{}, *best) : void()), ...);
 }
 
+// A stage of e4m3 has twice the products on the same bytes: the longer the more
+// rows of x there are.
 template <bool FP8, class F>
 void with_shape(int M, int N, int K, const F& f) {
   // the waves that read ahead are bf16 ones with 32-bit offsets in a tile of W
   const bool ahead = !FP8 && K <= 1 << 22;
+  const double stage = !FP8 ? 1 : M <= 32 ? 1.03 : M <= 64 ? 1.08 : 1.24;
   if (M <= 32) {
-    with_best(N, K, f, A32{}, B32{}, C32{});
+    with_best(N, K, stage, f, A32{}, B32{}, C32{});
   } else if (M <= 64) {
-    with_best(N, K, f, A64{}, B64{}, C64{}, D64{});
+    with_best(N, K, stage, f, A64{}, B64{}, C64{}, D64{});
   } else if (!ahead) {
-    if (M <= 128) with_best(N, K, f, A128{}, B128{}, D128{});
-    else with_best(N, K, f, L256{});
+    if (M <= 128) with_best(N, K, stage, f, A128{}, B128{}, D128{});
+    else with_best(N, K, stage, f, B256{});
   } else if constexpr (!FP8) {
-    if (M <= 128) with_best(N, K, f, A128{}, B128{}, C128{}, D128{});
-    else if (M <= 192) with_best(N, K, f, A192{}, C192{});
-    else with_best(N, K, f, A256{}, C256{});
+    if (M <= 128) with_best(N, K, stage, f, A128{}, B128{}, C128{}, D128{});
+    else if (M <= 192) with_best(N, K, stage, f, A192{}, C192{});
+    else with_best(N, K, stage, f, A256{}, B256{}, C256{});
   }
 }
 
 }  // namespace
 
 // what the chosen plan takes by its own estimate, in us
-double part_gemm_us(int M, int N, int K) {
+double part_gemm_us(int M, int N, int K, bool fp8) {
   double us = 0;
-  with_shape<false>(M, N, K, [&](auto, const Plan& pl) { us = pl.us; });
+  auto take = [&](auto, const Plan& pl) { us = pl.us; };
+  if (fp8) with_shape<true>(M, N, K / 2, take);
+  else with_shape<false>(M, N, K, take);
   return us;
 }
 
@@ -992,14 +1027,16 @@ bool in_pieces(float* pieces, const u16* x, const float* x_scales,
   auto run = [&](auto shape, const Plan& pl, auto fp8) {
     using S = decltype(shape);
     constexpr bool kFp8 = decltype(fp8)::value;
-    if (!pl.split || pl.tiles >= pl.parts) return;
-    done = true;
-    if (pieces == nullptr) return;
-    launch_products<S, false, kFp8, true>(
-        pl, nullptr, pieces, x, w, nullptr, Scales{x_scales, w_scales}, M, N,
-        K, x_stride, 0, stream);
-    sum(PieceRows{pieces, bias, S::TN, K / S::KS, pl.tiles, pl.parts, S::MB,
-                  S::kAhead});
+    if constexpr (S::kCuts) {
+      if (!pl.split || pl.tiles >= pl.parts) return;
+      done = true;
+      if (pieces == nullptr) return;
+      launch_products<S, false, kFp8, true>(
+          pl, nullptr, pieces, x, w, nullptr, Scales{x_scales, w_scales}, M, N,
+          K, x_stride, 0, stream);
+      sum(PieceRows{pieces, bias, S::TN, K / S::KS, pl.tiles, pl.parts, S::MB,
+                    S::kAhead});
+    }
   };
   if (x_scales != nullptr)
     with_shape<true>(M, N, K, [&](auto shape, const Plan& pl) {

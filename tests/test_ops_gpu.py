@@ -1488,23 +1488,23 @@ def test_stream_norms_weight_on_any_grid(offset):
     (fp8, rows) for rows in (1, 16, 17, 32, 33, 64, 65, 128, 129, 192, 193,
                              256) for fp8 in (False, True)
     if rows <= 128 or not fp8])
-@pytest.mark.parametrize("n,k,most,most_fp8", [
-    (4096, 4096, 256, 128),
-    (2064, 4608, 256, 128),    # a tile that is not full
-    (1040, 512, 256, 32),      # few parts, fewer stages in each
-    (5136, 5120, 256, 128),    # two turns of a workgroup along a row
-    (8208, 8192, 256, 128), (12304, 8192, 256, 128),   # four
-    (16384, 8192, 256, 0),     # the longest row; of e4m3 by whole tiles
-    (16400, 8192, 0, 0),       # longer than the kernel takes, if cut
-    (8208, 1024, 0, 0),        # whole tiles
+@pytest.mark.parametrize("n,k,cut,cut_fp8", [
+    (4096, 4096, 17, 1),
+    (2064, 4608, 17, 1),      # a tile that is not full
+    (1040, 512, 17, 1),       # few parts, fewer stages in each
+    (5136, 5120, 17, 1),      # two turns of a workgroup along a row
+    (8208, 8192, 17, 1), (12304, 12288, 17, 1),   # four
+    (16384, 16384, 33, 33),   # the longest row
+    (16400, 16384, 257, 129),  # longer than the kernel takes, if cut
+    (8208, 1024, 257, 129),   # whole tiles
 ])
-def test_linear_in_parts_and_norm(rows, n, k, most, most_fp8, fp8):
+def test_linear_in_parts_and_norm(rows, n, k, cut, cut_fp8, fp8):
     """The sum of a residual and a product in parts, and its norm, against
     float64: fp32 sums of k products; the sum and the normed row are rounded to
     bf16 once (2^-9 relative), or the row to e4m3 (2^-4, 2^-10 of the scale
     where it is smallest). Nothing is written behind the last row, nor anything
-    at all where another way is taken: of more than `most` rows, of up to 16 in
-    bf16."""
+    at all where another way is taken: of fewer rows than those from which on
+    the product is cut and summed so."""
     g = torch.Generator(device=DEV).manual_seed(n + k + rows)
 
     def randn(*shape):
@@ -1535,7 +1535,7 @@ def test_linear_in_parts_and_norm(rows, n, k, most, most_fp8, fp8):
                                          norm, 1e-6)
         got = out[:rows].double()
         assert (out[rows] == 7.0).all()
-    assert done == (rows <= most_fp8 if fp8 else 16 < rows <= most)
+    assert done == (rows >= (cut_fp8 if fp8 else cut))
     if not done:
         assert torch.equal(residual, old)
         return
