@@ -99,7 +99,7 @@ struct PartShape {
   static constexpr int LW = TN / kRowsPerDma / kWLoaders;
   static constexpr int LX = MB / kRowsPerDma / kXLoaders;
   static constexpr int kPiece = TN * MB / 4;  // float4
-  static constexpr bool kAhead = false, kCuts = true;
+  static constexpr bool kAhead = false, kCuts = true, kColumns = false;
   static_assert(RF % 2 == 0 && TN / 2 % kRowsPerDma == 0);
   static_assert(LW * kRowsPerDma * kWLoaders == TN &&
                 LX * kRowsPerDma * kXLoaders == MB);
@@ -110,7 +110,7 @@ struct PartShape {
 // the same for part_gemm_ahead_kernel: four waves of RF x CF fragments
 template <int RF, int CF, int RW, int RX>
 struct AheadShape : PartShape<1, RF, 4, CF, 64, RW, RX, 2> {
-  static constexpr bool kAhead = true;
+  static constexpr bool kAhead = true, kColumns = 4 * CF * 16 > 128;
 };
 
 // fragment of W rows (of the tile) that wave column wn holds as its rf-th
@@ -129,16 +129,17 @@ struct Scales {
 
 // Where a piece has a lane's results of a fragment: fragment by fragment of a
 // wave, or, with ROWS, for a kernel that sums whole rows. There rows of the tile
-// follow one another; from 129 rows of x on, where that kernel has workgroups
-// enough and the product is held up by its stores, 16 columns of all rows do: a
-// wave's store is 1 KB in one, not 16 times 64 bytes. (Both kernels, 4096 x 4096
-// at 43 / 192 / 256 rows: 15.7 / 25.3 / 30.0 us with rows, 16.4 / 24.4 / 27.7
-// with columns.)
+// follow one another; in shapes for more than 128 rows of x, where that kernel
+// has workgroups enough and the product is held up by its stores, 16 columns of
+// all rows do (kColumns): a wave's store is 1 KB in one, not 16 times 64 bytes.
+// (Both kernels with rows / columns: 4096 x 4096 at 43 rows 15.7 / 16.4 us, at 192
+// 25.3 / 24.4, at 256 30.0 / 27.7; 4096 x 12288 at 65 and 128 rows, waves that
+// read ahead too, 30.4 and 33.8 / 31.2 and 34.2.)
 template <class S, bool ROWS>
 FI_DEV int in_piece(int wave, int wn, int wm, int f, int c, int lane) {
   if (!ROWS) return ((wave * S::RF + f) * S::CF + c) * kWaveSize + lane;
   const int m = (wm * S::CF + c) * 16 + (lane & 15), nf = wn * S::RF + f;
-  return S::kAhead ? (nf * S::MB + m) * 4 + (lane >> 4)
+  return S::kColumns ? (nf * S::MB + m) * 4 + (lane >> 4)
                    : m * (S::TN / 4) + nf * 4 + (lane >> 4);
 }
 
@@ -1035,7 +1036,7 @@ bool in_pieces(float* pieces, const u16* x, const float* x_scales,
           pl, nullptr, pieces, x, w, nullptr, Scales{x_scales, w_scales}, M, N,
           K, x_stride, 0, stream);
       sum(PieceRows{pieces, bias, S::TN, K / S::KS, pl.tiles, pl.parts, S::MB,
-                    S::kAhead});
+                    S::kColumns});
     }
   };
   if (x_scales != nullptr)
