@@ -669,6 +669,19 @@ def rope_qk_norm_cache_(q, k, v, positions, cos_sin, k_cache, v_cache,
     return q
 
 
+def _rope_in_one(M: int, N: int, K: int) -> bool:
+    """Whether the kernel that sums the pieces of a product and goes on with
+    its heads is ahead of two. Its reads of pieces wait for one another where a
+    token has many heads, or a tile many pieces. (us, product and rope apart
+    and so: 6144 x 4096 at 43, 64 and 128 rows 20.2, 21.2, 28.6 and 19.8, 20.8,
+    27.5, at 256 33.1 and 33.6; 5120 x 8192 at 65 29.5 and 32.6; 8192 x 4096 at
+    128 28.5 and 30.0; 10240 x 4096 at 65 29.2 and 31.9. Eleven kinds of heads,
+    seven K, eight numbers of rows: 1.4 % less than two kernels with this rule,
+    0.6 % always in one, with 14 % more at worst. A prompt of 43 tokens, whose
+    launches the host does not keep up with: 1029 and 1017.)"""
+    return N <= 6144 and K <= (8192 if M <= 64 else 6144)
+
+
 def linear_rope_qk_norm_cache(x, w, bias, positions, cos_sin, k_cache, v_cache,
                               slot_mapping, num_q_heads: int,
                               q_weight: Optional[torch.Tensor] = None,
@@ -677,12 +690,9 @@ def linear_rope_qk_norm_cache(x, w, bias, positions, cos_sin, k_cache, v_cache,
                               v_inv_scale: float = 1.0):
     """rope_qk_norm_cache_ of linear(x, w, bias)'s queries, keys and values
     [T, (Hq | Hk | Hk) * D], where one kernel sums the pieces of 17 to 128 rows'
-    product and goes on; else None. Returns q. (us, product and rope apart and
-    so, 6144 x 4096 at 20, 43, 64 and 128 rows: 17.9, 20.2, 21.2, 28.6 and 17.7,
-    19.8, 20.8, 27.5; from there on the way of the pieces takes what the launch
-    did, 33.1 and 33.6 at 256. A prompt of 43 tokens, whose launches the host
-    does not keep up with: 1029 and 1017.)"""
+    product and goes on; else None. Returns q."""
     if not (SKINNY_ROWS < x.shape[0] <= 128
+            and _rope_in_one(x.shape[0], w.shape[0], x.shape[1])
             and _skinny_ok(x, w, 16, bias=bias)
             and k_cache.shape[3] in (64, 128)
             and w.shape[0] == (num_q_heads + 2 * k_cache.shape[1])

@@ -62,6 +62,17 @@ def test_choice_e4m3(rows, n, k, want):
     assert ops._streams_fp8(rows, n, k) == want
 
 
+@pytest.mark.parametrize("rows,n,k,want", [
+    (17, 6144, 4096, True), (128, 6144, 4096, True),   # 28.6 apart, 27.5
+    (64, 5120, 8192, True),
+    (65, 5120, 8192, False),      # 29.5, 32.6
+    (128, 8192, 4096, False),     # 28.5, 30.0
+    (64, 10240, 4096, False),
+])
+def test_choice_of_heads_from_pieces(rows, n, k, want):
+    assert ops._rope_in_one(rows, n, k) == want
+
+
 def test_estimates_grow():
     """With either size of W, whatever the shape of a tile is."""
     for rows in (17, 33, 65, 129, 193):
