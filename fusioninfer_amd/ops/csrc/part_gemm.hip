@@ -44,11 +44,11 @@
 //
 // Where a norm follows, the second kernel does the sum with the residual and
 // the norm too (part_gemm_norm_kernel): a launch of 3 to 5 us less, and the
-// product is not rounded before the sum. us, product and norm / both in one, at
-// 43 / 64 / 128 / 256 rows: 4096 x 4096 17.5, 18.2, 23.3, 29.4 / 15.7, 16.2, 20.8,
-// 28.3; 4096 x 12288 28.7, 30.0, 36.7, 47.4 / 27.0, 29.0, 36.0, 45.9; e4m3 at 64
-// rows 16.4 / 14.2 and 23.6 / 21.5. A step of eight layers at 256 rows 3360 ->
-// 3333 us.
+// product is not rounded before the sum. us in a graph, product and norm / both
+// in one, at 43 / 64 / 128 / 256 rows: 4096 x 4096 16.3, 17.0, 21.8, 28.5 / 14.6,
+// 15.1, 19.7, 27.1; 4096 x 12288 27.5, 28.8, 35.5, 45.7 / 25.9, 27.7, 33.9, 43.9;
+// e4m3 at 64 rows 16.4 / 14.2 and 23.6 / 21.5. (At 256 rows the library takes
+// 4096 x 4096 and its norm in 26.4.)
 //
 // FP8: the same kernel on e4m3 rows, 1 to 128 of them. 24576 x 4096 at 16 / 32
 // / 64 rows 19.3 (5210) / 19.9 / 22.7 us, the library's GEMM 30.0 / 25.3 /
