@@ -24,29 +24,32 @@ FI_DEV bf16x8 load8(const u16* p) {
 }
 
 // One workgroup per row, which it holds in registers between the absmax pass and
-// the convert pass: 256 threads up to 4096 columns, up to 1024 beyond, eight
-// columns each, once or twice. Few rows take the time of one chain from load to
-// store, which is the shorter the more threads share it; many are bound by
-// memory. ONCE: what is read and written goes past the caches, for more than the
-// memory-side one holds. us, 12288 columns of silu(gate) * up, 256 threads of six
-// vectors each, and this: 1 row 4.3 and 3.2, 64 rows 4.8 and 3.6, 1000 11.6 and
-// 11.6, 8000 95 and 87, with ONCE 74 (6.6 TB/s; at 2000 rows, 98 MB, 20 either
-// way). 4096 columns as they are: 8000 rows 15.2, with 512 threads 15.9.
-template <int ITERS, bool SILU_MUL, bool ONCE>
-__global__ __launch_bounds__(1024) void row_quant_fp8_kernel(
+// the convert pass, eight columns a thread at a time. THREADS 256, or 0: of the
+// launch, up to 1024. Few rows take the time of one chain from load to store,
+// which is the shorter the more threads share it; many are bound by memory, and
+// more of them are in flight the smaller they are. ONCE: what is read and
+// written goes past the caches, for more than the memory-side one holds. us,
+// 12288 columns of silu(gate) * up, 256 threads of six vectors each, and up to
+// 1024: 1 row 4.3 and 3.2, 64 rows 4.8 and 3.6, 1000 11.6 and 11.6, 8000 95 and 87,
+// with ONCE 74 (6.6 TB/s; at 2000 rows, 98 MB, 20 either way). 5120 columns as
+// they are: 16 rows 2.5 and 2.4, 1000 3.5 and 4.5, 8000 19 and 22.4.
+template <int THREADS, int ITERS, bool SILU_MUL, bool ONCE>
+__global__ __launch_bounds__(THREADS ? THREADS : 1024)
+void row_quant_fp8_kernel(
     unsigned char* __restrict__ out,   // [T, cols] fp8
     float* __restrict__ out_scales,    // [T]
     const u16* __restrict__ in,        // [T, cols] bf16 (SILU_MUL: [T, 2*cols])
     const int cols) {
   const int row = blockIdx.x;
   const int tid = threadIdx.x;
+  const int threads = THREADS ? THREADS : static_cast<int>(blockDim.x);
   const int64_t in_row = static_cast<int64_t>(row) * (SILU_MUL ? 2 * cols : cols);
 
   float vals[ITERS][8];
   float amax = 0.f;
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
-    const int col = (it * blockDim.x + tid) * 8;
+    const int col = (it * threads + tid) * 8;
     if (col < cols) {
       if (SILU_MUL) {
         const bf16x8 g = load8<ONCE>(in + in_row + col);
@@ -68,17 +71,21 @@ __global__ __launch_bounds__(1024) void row_quant_fp8_kernel(
 
   __shared__ float scratch[16];
   amax = wave_reduce_max(amax);
-  if (tid % kWaveSize == 0) scratch[tid / kWaveSize] = amax;
-  __syncthreads();
-  for (int i = 0; i < static_cast<int>(blockDim.x) / kWaveSize; ++i)
-    amax = fmaxf(amax, scratch[i]);
+  if (THREADS) {
+    amax = block_reduce_max<THREADS / kWaveSize>(amax, scratch);
+  } else {
+    if (tid % kWaveSize == 0) scratch[tid / kWaveSize] = amax;
+    __syncthreads();
+    for (int i = 0; i < threads / kWaveSize; ++i)
+      amax = fmaxf(amax, scratch[i]);
+  }
   const float scale = fmaxf(amax, 1e-8f) / kFp8Max;
   const float inv_scale = 1.f / scale;
   if (tid == 0) out_scales[row] = scale;
 
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
-    const int col = (it * blockDim.x + tid) * 8;
+    const int col = (it * threads + tid) * 8;
     if (col < cols) {
       float sv[8];
 #pragma unroll
@@ -98,22 +105,33 @@ template <bool SILU_MUL>
 void launch_row_quant_fp8(unsigned char* out, float* scales, const u16* in,
                           int rows, int cols, hipStream_t stream) {
   if (cols > 16384) abort();     // more than two vectors of 1024 threads
-  const int vectors = ceil_div(cols, 8);
-  const int iters = cols <= 2048 ? 1 : cols <= 4096 ? 2 : ceil_div(cols, 8192);
+  const bool wide = cols > (SILU_MUL ? 6144 : 10240) ||
+                    (cols > 4096 && rows <= (SILU_MUL ? 512 : 256));
+  const int iters = ceil_div(cols, wide ? 8192 : 2048);
   const int threads =
-      cols <= 4096 ? 256
-                   : ceil_div(ceil_div(vectors, iters), kWaveSize) * kWaveSize;
+      wide ? ceil_div(ceil_div(ceil_div(cols, 8), iters), kWaveSize) * kWaveSize
+           : 256;
   const bool once = beyond_caches(static_cast<int64_t>(rows) * cols *
                                   (SILU_MUL ? 4 : 2));
-#define FI_QUANT(N, ONCE)                                                     \
-  hipLaunchKernelGGL((row_quant_fp8_kernel<N, SILU_MUL, ONCE>), dim3(rows),   \
-                     dim3(threads), 0, stream, out, scales, in, cols)
-  if (iters == 1) {
-    if (once) FI_QUANT(1, true);
-    else FI_QUANT(1, false);
-  } else {
-    if (once) FI_QUANT(2, true);
-    else FI_QUANT(2, false);
+#define FI_QUANT(THREADS, N)                                                  \
+  do {                                                                        \
+    auto kernel = once ? &row_quant_fp8_kernel<THREADS, N, SILU_MUL, true>    \
+                       : &row_quant_fp8_kernel<THREADS, N, SILU_MUL, false>;  \
+    hipLaunchKernelGGL(kernel, dim3(rows), dim3(threads), 0, stream, out,     \
+                       scales, in, cols);                                     \
+  } while (0)
+  if (wide) {
+    if (iters == 1) FI_QUANT(0, 1);
+    else FI_QUANT(0, 2);
+  } else if (iters <= 1) {
+    FI_QUANT(256, 1);
+  } else if (iters == 2) {
+    FI_QUANT(256, 2);
+  } else if (iters == 3) {
+    FI_QUANT(256, 3);
+  } else if constexpr (!SILU_MUL) {
+    if (iters == 4) FI_QUANT(256, 4);
+    else FI_QUANT(256, 5);
   }
 #undef FI_QUANT
 }
