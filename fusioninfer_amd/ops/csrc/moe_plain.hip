@@ -425,8 +425,11 @@ __global__ __launch_bounds__(256) void moe_combine_vec_kernel(
 // tokens 5260 -> 5222 us, 64 tokens 1332 -> 1320; the norm alone takes 25 and 2.7
 // us a layer.) 8765 tokens, top 8, width 2048: 71 us, with ONCE 63; 4000 tokens
 // 28 and 29. No load is behind a branch: 64 tokens 3.5 us with, 3.0 without.
-template <int ITERS, bool ONCE>
-__global__ __launch_bounds__(256) void moe_combine_norm_kernel(
+// THREADS: of the workgroup; 1024 from 4097 columns on, where vectors of a thread
+// one after another take longer than the two kernels for few tokens (64 tokens,
+// top 16, width 8192 7.4 us in two, 10.3 in one with 256).
+template <int THREADS, int ITERS, bool ONCE>
+__global__ __launch_bounds__(THREADS) void moe_combine_norm_kernel(
     u16* __restrict__ out, u16* __restrict__ residual,
     const u16* __restrict__ norm, const float eps, const u16* __restrict__ y,
     const int* __restrict__ pos, const float* __restrict__ w, const int topk,
@@ -439,7 +442,7 @@ __global__ __launch_bounds__(256) void moe_combine_norm_kernel(
   float squares = 0.f;
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
-    const int c = (it * 256 + static_cast<int>(threadIdx.x)) * 8;
+    const int c = (it * THREADS + static_cast<int>(threadIdx.x)) * 8;
     if (c < H) {
       const bf16x8 old = *reinterpret_cast<const bf16x8*>(residual + row + c);
       g[it] = *reinterpret_cast<const bf16x8*>(norm + c);
@@ -475,12 +478,13 @@ __global__ __launch_bounds__(256) void moe_combine_norm_kernel(
       *reinterpret_cast<bf16x8*>(residual + row + c) = sum;
     }
   }
-  __shared__ float scratch[4];
-  squares = block_reduce_sum<4>(wave_reduce_sum(squares), scratch);
+  __shared__ float scratch[THREADS / kWaveSize];
+  squares = block_reduce_sum<THREADS / kWaveSize>(wave_reduce_sum(squares),
+                                                  scratch);
   const float inv_rms = rsqrtf(squares / H + eps);
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
-    const int c = (it * 256 + static_cast<int>(threadIdx.x)) * 8;
+    const int c = (it * THREADS + static_cast<int>(threadIdx.x)) * 8;
     if (c < H) {
       bf16x8 o;
 #pragma unroll
@@ -500,16 +504,16 @@ void launch_moe_combine_norm(u16* out, u16* residual, const u16* norm,
                              const float* w, int tokens, int topk, int H,
                              hipStream_t stream) {
   const bool once = beyond_caches(static_cast<int64_t>(tokens) * topk * H * 2);
-#define FI_CN(ITERS)                                                          \
+#define FI_CN(THREADS, ITERS)                                                 \
   do {                                                                        \
-    auto kernel = once ? &moe_combine_norm_kernel<ITERS, true>                \
-                       : &moe_combine_norm_kernel<ITERS, false>;              \
-    hipLaunchKernelGGL(kernel, dim3(tokens), dim3(256), 0, stream, out,       \
+    auto kernel = once ? &moe_combine_norm_kernel<THREADS, ITERS, true>       \
+                       : &moe_combine_norm_kernel<THREADS, ITERS, false>;     \
+    hipLaunchKernelGGL(kernel, dim3(tokens), dim3(THREADS), 0, stream, out,   \
                        residual, norm, eps, y, pos, w, topk, H);              \
   } while (0)
-  if (H <= 2048) FI_CN(1);
-  else if (H <= 4096) FI_CN(2);
-  else FI_CN(4);
+  if (H <= 2048) FI_CN(256, 1);
+  else if (H <= 4096) FI_CN(256, 2);
+  else FI_CN(1024, 1);
 #undef FI_CN
 }
 
