@@ -6,12 +6,13 @@
 // elements, so D / 8 lanes hold a head and a wave four heads (D = 128) or
 // eight (64) of one token; the rotate-half partner is D / 16 lanes away in
 // the same row of 16 lanes, and the norm's sum is three or four exchanges
-// within it. A workgroup is one token; every load is requested before anything
-// waits for one. cos/sin come from a table (f32 [P, D], cos | sin): sines
-// computed here would make it bound by the VALU. us at 32 + 2 * 8 heads of 128,
-// loads as they are needed and a rolled loop for the sum, and this: 64 tokens
-// 3.2 and 2.8, 1024 7.7 and 6.0, 4099 19.7 and 16.0 (6.3 TB/s), 8765 44.6 and
-// 37.7; e4m3 cache, 8765 43.8 and 37.9.
+// within it. A workgroup is one token, or four waves of one where there are
+// few; every load is requested before anything waits for one. cos/sin come from
+// a table (f32 [P, D], cos | sin): sines computed here would make it bound by
+// the VALU. us at 32 + 2 * 8 heads of 128, loads as they are needed and a
+// rolled loop for the sum, and this: 64 tokens 2.9 and 2.5, 1024 7.7 and 6.0,
+// 4099 19.7 and 16.0 (6.3 TB/s), 8765 44.6 and 37.7; e4m3 cache, 8765 43.8 and
+// 37.9.
 //
 // Capability parity: RoPE / qk-norm epilogue and cache write the reference
 // delegates to vLLM.
@@ -66,8 +67,11 @@ struct CacheRows {
 // PIECES: the rows are sums of pieces (+ bias) of a product that is cut, a
 // launch and a pass over them less; results of q go to q. Bound by the way of
 // the pieces through memory as their sum alone is: 64 rows, 32 + 2 * 8 heads of
-// 128, 5.8 us, the sum 4.6 and the rest 4.0 (256 rows 9.4, 6.7 and 4.2).
-template <int D, bool CACHE, bool FP8, int UNITS, bool PIECES>
+// 128, 5.8 us with 16 waves a workgroup, 1.1 less with four; the sum alone 4.6
+// and the rest 4.0 (256 rows 9.4, 6.7 and 4.2).
+// NORM: there is a weight for q or k. (Without one a sum that nobody reads
+// costs a launch for few tokens 0.2 to 0.5 us of 2.3.)
+template <int D, bool CACHE, bool FP8, int UNITS, bool PIECES, bool NORM>
 __global__ __launch_bounds__(kRopeWaves * kWaveSize) void rope_qk_norm_kernel(
     u16* __restrict__ q,             // [T, Hq*D] rows, stride q_stride
     u16* __restrict__ k,             // [T, Hk*D] rows, stride k_stride
@@ -89,7 +93,8 @@ __global__ __launch_bounds__(kRopeWaves * kWaveSize) void rope_qk_norm_kernel(
                            : static_cast<int>(blockIdx.x);
   if (PIECES && token >= tokens) return;
   const int heads = num_q_heads + (CACHE ? 2 : 1) * num_kv_heads;
-  const int head0 = (blockIdx.y * kRopeWaves + wave) * (H * UNITS) + lane / L;
+  const int waves = blockDim.x / kWaveSize;
+  const int head0 = (blockIdx.y * waves + wave) * (H * UNITS) + lane / L;
   const int e = (lane % L) * 8;      // first element of this lane
 
   // all loads are requested before anything waits for one of them
@@ -124,10 +129,13 @@ __global__ __launch_bounds__(kRopeWaves * kWaveSize) void rope_qk_norm_kernel(
   auto weight_of = [&](int head) {
     return head < num_q_heads ? q_weight : k_weight;
   };
+  if constexpr (NORM) {
 #pragma unroll
-  for (int u = 0; u < UNITS; ++u) {
-    const u16* w = weight_of(head0 + u * H);
-    wr[u] = load8((w != nullptr ? w : reinterpret_cast<const u16*>(cos_sin)) + e);
+    for (int u = 0; u < UNITS; ++u) {
+      const u16* w = weight_of(head0 + u * H);
+      wr[u] =
+          load8((w != nullptr ? w : reinterpret_cast<const u16*>(cos_sin)) + e);
+    }
   }
   __builtin_amdgcn_sched_barrier(0);
   const int pair = e % (D / 2);      // rotary pair of the first element
@@ -148,8 +156,7 @@ __global__ __launch_bounds__(kRopeWaves * kWaveSize) void rope_qk_norm_kernel(
     const bool is_q = head < num_q_heads;
     const int kv = head - num_q_heads;
     const bool is_v = CACHE && kv >= num_kv_heads;
-    const bool normed = weight_of(head) != nullptr;
-    float x[8], wf[8], sum = 0.f;
+    float x[8];
     if constexpr (PIECES) {
       unpack8(add, x);
       for (;;) {
@@ -172,13 +179,18 @@ __global__ __launch_bounds__(kRopeWaves * kWaveSize) void rope_qk_norm_kernel(
     } else {
       unpack8(raw[u], x);
     }
-    unpack8(wr[u], wf);
+    if constexpr (NORM) {
+      const bool normed = weight_of(head) != nullptr;
+      float wf[8], sum = 0.f;
+      unpack8(wr[u], wf);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) sum += x[i] * x[i];
-    sum = head_sum<L>(sum);
-    const float inv_rms = rsqrtf(sum / D + eps);
+      for (int i = 0; i < 8; ++i) sum += x[i] * x[i];
+      sum = head_sum<L>(sum);
+      const float inv_rms = rsqrtf(sum / D + eps);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) x[i] = normed ? x[i] * (inv_rms * wf[i]) : x[i];
+      for (int i = 0; i < 8; ++i)
+        x[i] = normed ? x[i] * (inv_rms * wf[i]) : x[i];
+    }
     // x1' = x1 cos - x2 sin in the first half, x2' = x2 cos + x1 sin
     u32x4_any bits;
     u16 y[8];
@@ -225,7 +237,15 @@ __global__ __launch_bounds__(kRopeWaves * kWaveSize) void rope_qk_norm_kernel(
   }
 }
 
-template <int D, int UNITS>
+// of a workgroup, for so many of a token: few tokens are spread over more CUs
+// (us with 16 waves and with four, 32 + 2 * 8 heads of 128: 64 tokens 2.8 and
+// 2.5, 128 2.95 and 2.66, 256 3.15 and 3.05; of pieces, product and all, 6144 x
+// 4096: 17 rows 17.0 and 15.5, 128 26.3 and 25.6)
+int waves_of(int waves, int tokens) {
+  return std::min(waves, tokens <= 256 ? 4 : kRopeWaves);
+}
+
+template <int D, int UNITS, bool NORM>
 void launch_rope(u16* q, u16* k, const u16* v, int64_t q_stride,
                  int64_t k_stride, int64_t v_stride, const u16* q_weight,
                  const u16* k_weight, const float* cos_sin,
@@ -234,29 +254,29 @@ void launch_rope(u16* q, u16* k, const u16* v, int64_t q_stride,
   if (tokens == 0) return;
   const int waves = ceil_div(hq + (v ? 2 : 1) * hk,
                              kWaveSize / (D / 8) * UNITS);
-  auto kernel = !v ? &rope_qk_norm_kernel<D, false, false, UNITS, false>
-      : fp8 ? &rope_qk_norm_kernel<D, true, true, UNITS, false>
-            : &rope_qk_norm_kernel<D, true, false, UNITS, false>;
-  hipLaunchKernelGGL(kernel, dim3(tokens, ceil_div(waves, kRopeWaves)),
-                     dim3(std::min(waves, kRopeWaves) * kWaveSize), 0, stream,
-                     q, k, v, q_stride, k_stride, v_stride, q_weight,
-                     k_weight, cos_sin, positions, hq, hk, eps, cache,
-                     PieceRows{}, tokens);
+  auto kernel = !v ? &rope_qk_norm_kernel<D, false, false, UNITS, false, NORM>
+      : fp8 ? &rope_qk_norm_kernel<D, true, true, UNITS, false, NORM>
+            : &rope_qk_norm_kernel<D, true, false, UNITS, false, NORM>;
+  const int at_once = waves_of(waves, tokens);
+  hipLaunchKernelGGL(kernel, dim3(tokens, ceil_div(waves, at_once)),
+                     dim3(at_once * kWaveSize), 0, stream, q, k, v, q_stride,
+                     k_stride, v_stride, q_weight, k_weight, cos_sin,
+                     positions, hq, hk, eps, cache, PieceRows{}, tokens);
 }
 
-template <int D>
+template <int D, bool NORM>
 void launch_of_pieces(u16* q, const PieceRows& pieces, const RopeArgs& a,
                       int tokens, hipStream_t stream) {
   const CacheRows cache{a.k_cache, a.v_cache, a.slots, a.block_size,
                         a.k_inv_scale, a.v_inv_scale};
   const int waves = ceil_div(a.num_q_heads + 2 * a.num_kv_heads,
                              kWaveSize / (D / 8));
-  auto kernel = a.fp8 ? &rope_qk_norm_kernel<D, true, true, 1, true>
-                      : &rope_qk_norm_kernel<D, true, false, 1, true>;
+  auto kernel = a.fp8 ? &rope_qk_norm_kernel<D, true, true, 1, true, NORM>
+                      : &rope_qk_norm_kernel<D, true, false, 1, true, NORM>;
+  const int at_once = waves_of(waves, tokens);
   hipLaunchKernelGGL(
-      kernel,
-      dim3(ceil_div(tokens, 16) * 16, ceil_div(waves, kRopeWaves)),
-      dim3(std::min(waves, kRopeWaves) * kWaveSize), 0, stream, q, nullptr,
+      kernel, dim3(ceil_div(tokens, 16) * 16, ceil_div(waves, at_once)),
+      dim3(at_once * kWaveSize), 0, stream, q, nullptr,
       nullptr, static_cast<int64_t>(a.num_q_heads) * D, 0, 0, a.q_weight,
       a.k_weight, a.cos_sin, a.positions, a.num_q_heads, a.num_kv_heads,
       a.eps, cache, pieces, tokens);
@@ -276,21 +296,30 @@ void launch_rope_qk_norm(u16* q, u16* k, const u16* v, int64_t q_stride,
                          hipStream_t stream) {
   const CacheRows cache{k_cache, v_cache, slots, block_size, k_inv_scale,
                         v_inv_scale};
-  // from 1024 tokens on a wave takes twice the heads: cos, sin and weights once,
-  // twice the loads on the way (8765 tokens, 32 + 2 * 8 heads of 128: 48 us with
-  // one unit, 38 with two; 512 tokens 4.1 and 4.5)
-  const bool many = tokens >= 1024;
-#define FI_ROPE(D, U)                                                          \
-  launch_rope<D, U>(q, k, v, q_stride, k_stride, v_stride, q_weight, k_weight, \
-                    cos_sin, positions, tokens, num_q_heads, num_kv_heads,     \
-                    eps, cache, fp8, stream)
+  // from 2^22 values on a wave takes twice the heads: cos, sin and weights
+  // once, twice the loads on the way (8765 tokens, 32 + 2 * 8 heads of 128: 48
+  // us with one unit, 38 with two; 512 tokens 4.1 and 4.5; 1000 tokens of 64 + 2
+  // * 8 heads without a norm 9.8 and 8.9)
+  const bool many = static_cast<int64_t>(tokens) * head_dim *
+                        (num_q_heads + (v ? 2 : 1) * num_kv_heads) >= 1 << 22;
+  const bool norm = q_weight != nullptr || k_weight != nullptr;
+#define FI_ROPE(D, U, NORM)                                                    \
+  launch_rope<D, U, NORM>(q, k, v, q_stride, k_stride, v_stride, q_weight,     \
+                          k_weight, cos_sin, positions, tokens, num_q_heads,   \
+                          num_kv_heads, eps, cache, fp8, stream)
+#define FI_ROPE_N(D, U)                                                        \
+  do {                                                                         \
+    if (norm) FI_ROPE(D, U, true);                                             \
+    else FI_ROPE(D, U, false);                                                 \
+  } while (0)
   if (head_dim == 128) {
-    if (many) FI_ROPE(128, 2);
-    else FI_ROPE(128, 1);
+    if (many) FI_ROPE_N(128, 2);
+    else FI_ROPE_N(128, 1);
   } else {
-    if (many) FI_ROPE(64, 2);
-    else FI_ROPE(64, 1);
+    if (many) FI_ROPE_N(64, 2);
+    else FI_ROPE_N(64, 1);
   }
+#undef FI_ROPE_N
 #undef FI_ROPE
 }
 
@@ -298,8 +327,11 @@ void launch_rope_qk_norm(u16* q, u16* k, const u16* v, int64_t q_stride,
 // pieces; head_dim 64 or 128
 void launch_rope_of_pieces(u16* q, const PieceRows& pieces, const RopeArgs& a,
                            int tokens, hipStream_t stream) {
-  if (a.head_dim == 128) launch_of_pieces<128>(q, pieces, a, tokens, stream);
-  else launch_of_pieces<64>(q, pieces, a, tokens, stream);
+  const bool norm = a.q_weight != nullptr || a.k_weight != nullptr;
+  auto launch = a.head_dim == 128
+      ? (norm ? &launch_of_pieces<128, true> : &launch_of_pieces<128, false>)
+      : (norm ? &launch_of_pieces<64, true> : &launch_of_pieces<64, false>);
+  launch(q, pieces, a, tokens, stream);
 }
 
 }  // namespace fi

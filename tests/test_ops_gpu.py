@@ -299,25 +299,29 @@ def test_rope_qk_norm_cache(T, Hq, Hk, D, pad, fp8):
 
 
 @pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("norm", [False, True])
 @pytest.mark.parametrize("Hq,Hk,D", [
     (5, 1, 128),     # a wave's second unit is partly, or not at all, there
     (72, 4, 128),    # more heads than a workgroup's waves take
     (33, 3, 64),
 ])
-def test_rope_qk_norm_cache_of_many_tokens(Hq, Hk, D, fp8):
-    """Many tokens, two units of heads per wave, are bit for bit what the same
-    tokens in shorter calls are; q against the fp32 oracle, one bf16 rounding
+def test_rope_qk_norm_cache_of_many_tokens(Hq, Hk, D, norm, fp8):
+    """Many tokens, from 2^22 values on two units of heads per wave, are bit
+    for bit what the same tokens in shorter calls are, of up to 256 of them
+    with four waves a workgroup; q against the fp32 oracle, one bf16 rounding
     (2^-8: of an ulp that falls the other way) and 1e-5 for fp32 sums."""
     torch.manual_seed(3)
-    T = 1027
+    T = -(-2 ** 22 // ((Hq + 2 * Hk) * D))
     qkv = torch.randn(T, (Hq + 2 * Hk) * D, device=DEV, dtype=torch.bfloat16)
     cos_sin = ops.compute_cos_sin_cache(D, 512, 10000.0).to(DEV)
     positions = torch.randint(0, 512, (T,), dtype=torch.int32, device=DEV)
-    qw, kw = torch.randn(2, D, device=DEV).to(torch.bfloat16)
-    slots = torch.randperm(1040, device=DEV)[:T].to(torch.int32)
-    slots[700] = -1
+    qw, kw = torch.randn(2, D, device=DEV).to(torch.bfloat16) if norm \
+        else (None, None)
+    blocks = T // 16 + 2
+    slots = torch.randperm(blocks * 16, device=DEV)[:T].to(torch.int32)
+    slots[300] = -1
     dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
-    caches = [torch.zeros(65, Hk, 16, D, device=DEV).to(dt) for _ in range(4)]
+    caches = [torch.zeros(blocks, Hk, 16, D, device=DEV).to(dt) for _ in range(4)]
 
     def run(x, rows, k_cache, v_cache):
         q, k, v = x[rows].split([Hq * D, Hk * D, Hk * D], dim=1)
@@ -327,16 +331,16 @@ def test_rope_qk_norm_cache_of_many_tokens(Hq, Hk, D, fp8):
 
     whole, parts = qkv.clone(), qkv.clone()
     run(whole, slice(0, T), *caches[:2])
-    run(parts, slice(0, 500), *caches[2:])
-    run(parts, slice(500, T), *caches[2:])
+    run(parts, slice(0, 256), *caches[2:])
+    run(parts, slice(256, T), *caches[2:])
     assert torch.equal(whole, parts)
     for a, b in zip(caches[:2], caches[2:]):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
     want, _ = ref.rope_qk_norm(
         qkv[:, :Hq * D].cpu().float().view(T, Hq, D),
         qkv[:, Hq * D:(Hq + Hk) * D].cpu().float().view(T, Hk, D),
-        positions.cpu().long(), cos_sin.cpu(), qw.cpu().float(),
-        kw.cpu().float())
+        positions.cpu().long(), cos_sin.cpu(),
+        *(w.cpu().float() if norm else None for w in (qw, kw)))
     assert_close_bf16(whole[:, :Hq * D].cpu().view(T, Hq, D), want,
                       atol=1e-5, rtol=2 ** -8)
 
