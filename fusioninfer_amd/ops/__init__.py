@@ -672,14 +672,14 @@ def rope_qk_norm_cache_(q, k, v, positions, cos_sin, k_cache, v_cache,
 def _rope_in_one(M: int, N: int, K: int) -> bool:
     """Whether the kernel that sums the pieces of a product and goes on with
     its heads is ahead of two. Its reads of pieces wait for one another where a
-    token has many heads, or a tile many pieces. (us, product and rope apart
-    and so: 6144 x 4096 at 43, 64 and 128 rows 20.2, 21.2, 28.6 and 19.8, 20.8,
-    27.5, at 256 33.1 and 33.6; 5120 x 8192 at 65 29.5 and 32.6; 8192 x 4096 at
-    128 28.5 and 30.0; 10240 x 4096 at 65 29.2 and 31.9. Eleven kinds of heads,
-    seven K, eight numbers of rows: 1.4 % less than two kernels with this rule,
-    0.6 % always in one, with 14 % more at worst. A prompt of 43 tokens, whose
-    launches the host does not keep up with: 1029 and 1017.)"""
-    return N <= 6144 and K <= (8192 if M <= 64 else 6144)
+    tile has many pieces, or many rows many heads. (us, product and rope apart
+    and so: 6144 x 4096 at 43, 64 and 128 rows 19.4, 20.2, 26.5 and 18.5, 19.7,
+    25.6, 10240 x 4096 at 64 27.5 and 27.0, at 65 29.1 and 31.4; 5120 x 8192 at
+    64 27.1 and 26.1, at 65 29.3 and 31.2; 8192 x 4096 at 128 28.3 and 29.1; 256
+    rows of 6144 x 4096, with 16 waves a workgroup, 33.1 and 33.6. Eleven kinds
+    of heads, seven K, eight numbers of rows: 3.3 % less than two kernels with
+    this rule, 3.5 % always in one, with 10 % more at worst.)"""
+    return K <= 8192 if M <= 64 else N <= 6144 and K <= 6144
 
 
 def linear_rope_qk_norm_cache(x, w, bias, positions, cos_sin, k_cache, v_cache,

@@ -63,11 +63,11 @@ def test_choice_e4m3(rows, n, k, want):
 
 
 @pytest.mark.parametrize("rows,n,k,want", [
-    (17, 6144, 4096, True), (128, 6144, 4096, True),   # 28.6 apart, 27.5
-    (64, 5120, 8192, True),
-    (65, 5120, 8192, False),      # 29.5, 32.6
-    (128, 8192, 4096, False),     # 28.5, 30.0
-    (64, 10240, 4096, False),
+    (17, 6144, 4096, True), (128, 6144, 4096, True),   # 26.5 apart, 25.6
+    (64, 5120, 8192, True), (64, 5120, 12288, False),
+    (65, 5120, 8192, False),      # 29.3, 31.2
+    (128, 8192, 4096, False),     # 28.3, 29.1
+    (64, 10240, 4096, True), (65, 10240, 4096, False),   # 29.1, 31.4
 ])
 def test_choice_of_heads_from_pieces(rows, n, k, want):
     assert ops._rope_in_one(rows, n, k) == want
