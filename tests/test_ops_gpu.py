@@ -172,10 +172,11 @@ def test_quant_fp8_rows(tokens, cols):
     _assert_fp8_close(f8, sc, ef8, esc, exact=x.cpu())
 
 
-@pytest.mark.parametrize("cols", [2056, 4096, 4104, 8192, 8200, 12288, 16384])
+@pytest.mark.parametrize("cols", [2056, 4096, 4104, 6144, 6152, 8192, 8200, 10240,
+                                  10248, 12288, 16384])
 @pytest.mark.parametrize("silu_mul", [False, True])
 def test_quant_fp8_of_rows_of_all_lengths(cols, silu_mul):
-    """One or two vectors a thread, workgroups of all sizes, and the loads and
+    """One to five vectors a thread, workgroups of all sizes, and the loads and
     stores for more than the caches hold give the bits of short calls; those
     are within half a step of e4m3 (2^-4 relative, 2^-10 of the scale) and fp32
     roundings of silu of the exact rows, the largest of which is 448."""
@@ -184,7 +185,8 @@ def test_quant_fp8_of_rows_of_all_lengths(cols, silu_mul):
     rows = (1 << 27) // width + 3        # of 2 bytes: more than 256 MB
     x = torch.randn(rows, width, device=DEV, dtype=torch.bfloat16)
     f8, sc = call(x)
-    for part in (slice(0, 1), slice(1, 34), slice(rows - 40, rows)):
+    for part in (slice(0, 1), slice(1, 34), slice(34, 634),
+                 slice(rows - 40, rows)):
         g8, gs = call(x[part])
         assert torch.equal(g8.view(torch.uint8), f8[part].view(torch.uint8))
         assert torch.equal(gs, sc[part])
@@ -1189,7 +1191,7 @@ def test_moe_combine_widths(T, top, H, dtype):
 
 
 @pytest.mark.parametrize("T,top,H", [(1, 1, 8), (3, 8, 2048), (64, 9, 2056),
-                                     (5, 4, 4096), (2, 16, 8192),
+                                     (5, 4, 4096), (5, 4, 4104), (2, 16, 8192),
                                      (300, 8, 264), (4, 2, 8200)])
 def test_moe_combine_norm(T, top, H):
     """The combined rows, the residual and the norm behind: fp32 sums of top
