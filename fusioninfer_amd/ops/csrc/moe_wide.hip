@@ -20,15 +20,21 @@
 // in front of it.
 //
 // LDS: 16-byte chunk c of row r sits at c ^ (r >> 1 & 7); B's fragments lie as
-// they are packed, in odd ones columns c at c ^ 4. MFMA operands are B, A; a
-// pair of fragments (32 columns) is read so that a lane ends with eight
-// neighbouring columns of a row: column (i >> 2) * 8 + (i & 3) + 4 p of the
-// pair is row i of product p.
+// they are packed, in the f-th columns c at c ^ f. MFMA operands are A, B; B is
+// read so that lane i of 16 has column 8 i + f of a wave's in product f: eight
+// neighbouring columns of a row (of each four rows; joined ones four), beside
+// those of the next lane.
 //
 // Workgroups of one XCD take a contiguous run of tiles, eight row blocks by
 // all column tiles at a time.
 //
-// A stage takes 1.4 us; a tile's end about 8, most of it until its results
+// Results leave in that order because a CU takes stores 64 bytes of neighbouring
+// lanes at a time: 128 KB in 0.9 us so (8 bytes a lane 1.7), in 3.5 where a lane's
+// 16 bytes are another row than the next one's (all CUs at once: 5.7 either way).
+// 8100 rows, 128 experts, top 8, 2048 x 768: down 251 and 240 us, gate|up 414 and
+// 416; 4000 rows 152 and 146.
+//
+// A stage takes 1.4 to 1.7 us; a tile's end 5 to 7, most of it until its results
 // have left (the stages after the first wait for them). Measured, us (TFLOP/s
 // of the real rows), 128 x 256 tiles and these: 8765 rows, 128 experts, top 8,
 // 2048 x 768: gate|up 467 (945) and 445 (992), down 308 (717) and 266 (831);
@@ -95,7 +101,6 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
   constexpr int kOwn = GATE_UP ? 4 : 8;   // fragments apart from up's
   const u32 up = N / 16 * 1024u;
   u32 a_voff[4];
-  const u32 b_voff[2] = {lane * 16u, (lane ^ 4) * 16u};
   u32x4 da, db;
   int rat = first, left = 0;
   u32 a_soff = 0, b_soff = 0, b_col[kOwn];
@@ -152,7 +157,7 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
       load_lds(da, a_voff[j], a_soff);
     } else {
       const int f = (j - 4) % 8, half = (j - 4) / 8;
-      load_lds(db, b_voff[f & 1],
+      load_lds(db, (lane ^ f) * 16u,
                b_soff + half * b_step + b_col[f % kOwn] +
                    (f >= kOwn ? up : 0));
     }
@@ -167,16 +172,16 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
   // ---- fragment reads: A row lane & 15, chunk 4 half + (lane >> 4)
   const int i16 = lane & 15, q = lane >> 4;
   const u32 a_rd = i16 * 128 + ((q ^ (i16 >> 1)) << 4);
-  const u32 b_rd = kRowsB + wave * kWaveB + (i16 >> 3) * 1024 +
-                   (q * 16 + (i16 >> 2 & 1) * 8 + (i16 >> 3) * 4 + (i16 & 3)) *
-                       16;
+  constexpr int kEach = GATE_UP ? 4 : 8;   // of a lane's columns in a row
+  const u32 b_rd = kRowsB + wave * kWaveB + i16 * kEach / 16 * 1024 +
+                   (q * 16 + ((i16 * kEach & 15) | i16 * kEach / 16)) * 16;
   auto rda = [&](u32 buf, int half, int mi) {
     return *reinterpret_cast<const short8*>(
         smem + buf + (a_rd ^ (half * 64)) + mi * 2048);
   };
   auto rdb = [&](u32 buf, int half, int f) {
     return *reinterpret_cast<const short8*>(
-        smem + buf + (b_rd ^ ((f & 1) * 64)) + half * 8192 + (f >> 1) * 2048);
+        smem + buf + (b_rd ^ (f * 16)) + half * 8192 + f / kEach * 4096);
   };
   short8 a0[8], b0[8], a1[8], b1[8];
   floatx4 acc[8][8];
@@ -199,9 +204,9 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
   }
   u32 buf = 0;
   constexpr int kCols = GATE_UP ? 64 : 128;   // of a wave
-  // of a tile, at least: 16 bytes are one instruction or more, and a wait that
-  // counts too few is only longer
-  constexpr int kStores = kCols / 4;
+  // of a tile, at least: a lane's part of a row is one instruction or more, and a
+  // wait that counts too few is only longer
+  constexpr int kStores = 32;
   constexpr int kFree = 40, kEarly = 6;  // MFMAs up to the first barrier, DMAs
                                          // between the two
   // `behind`: stores that follow the DMAs that are waited for
@@ -209,8 +214,8 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
 #pragma unroll
     for (int i = 0; i < 64; ++i) {
       const int mi = i >> 3, f = i & 7;
-      if (first) mfma_first(acc[mi][f], b0[f], a0[mi]);
-      else mfma(acc[mi][f], b0[f], a0[mi]);
+      if (first) mfma_first(acc[mi][f], a0[mi], b0[f]);
+      else mfma(acc[mi][f], a0[mi], b0[f]);
       __builtin_amdgcn_sched_barrier(0);
       if (i < 16 && i % 2 == 0) b1[i / 2] = rdb(buf, 1, i / 2);
       if (i >= 16 && i < 32 && i % 2 == 0)
@@ -238,7 +243,7 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
 #pragma unroll
     for (int i = 0; i < 64; ++i) {
       const int mi = i >> 3, f = i & 7;
-      mfma(acc[mi][f], b1[f], a1[mi]);
+      mfma(acc[mi][f], a1[mi], b1[f]);
       __builtin_amdgcn_sched_barrier(0);
       if (i % 4 == 0 && i < 32) b0[i / 4] = rdb(buf, 0, i / 4);
       if (i % 4 == 0 && i >= 32) a0[i / 4 - 8] = rda(buf, 0, i / 4 - 8);
@@ -261,41 +266,41 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
     // registers that the loop needs)
     int l = lane;
     asm volatile("" : "+v"(l));
-    const int col = t.n * 4 * kCols + wave * kCols + (l >> 4) * 8;
-    u16* to = out +
-              static_cast<int64_t>(t.m * kWideM + (l & 15)) * N + col;
+    const int col = t.n * 4 * kCols + wave * kCols + (l & 15) * kEach;
     auto store = [&](bool inside) {
+      if (!inside && col >= N) return;
+      u16* to = out +
+                static_cast<int64_t>(t.m * kWideM + (l >> 4) * 4) * N + col;
 #pragma unroll
       for (int mi = 0; mi < 8; ++mi) {
 #pragma unroll
-        for (int f = 0; f < kCols / 16; f += 2) {
-          if (inside || col + f * 16 < N) {
-            bf16x8 o;
+        for (int r = 0; r < 4; ++r) {
+          struct alignas(2 * kEach) {
+            u16 h[kEach];
+          } o;
 #pragma unroll
-            for (int p = 0; p < 2; ++p) {
-              const floatx4 g = acc_of(acc[mi][f + p]);
-              floatx4 u = g;
-              if (GATE_UP) u = acc_of(acc[mi][(f + p + 4) % 8]);
-#pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                float v = g[r];
-                if (MODE == 3) {
-                  const float gt = fminf(v, limit);
-                  const float up1 = fminf(fmaxf(u[r], -limit), limit);
-                  v = (gt / (1.f + __expf(-1.702f * gt))) * (up1 + 1.f);
-                } else if (MODE == 1) {
-                  v = silu(v) * u[r];
-                } else if (MODE == 2) {
-                  v = fmaxf(v, 0.f);
-                  v *= v;
-                }
-                o.h[p * 4 + r] = f32_to_bf16(v);
+          for (int c = 0; c < kEach; ++c) {
+            float v = acc_of(acc[mi][c][r]);
+            if (GATE_UP) {
+              const float u = acc_of(acc[mi][(c + 4) % 8][r]);
+              if (MODE == 3) {
+                const float gt = fminf(v, limit);
+                const float up1 = fminf(fmaxf(u, -limit), limit);
+                v = (gt / (1.f + __expf(-1.702f * gt))) * (up1 + 1.f);
+              } else {
+                v = silu(v) * u;
               }
+            } else if (MODE == 2) {
+              v = fmaxf(v, 0.f);
+              v *= v;
             }
-            *reinterpret_cast<bf16x8*>(to + f * 16) = o;
+            o.h[c] = f32_to_bf16(v);
           }
+          *reinterpret_cast<decltype(o)*>(to) = o;
+          // (a step at a time, or all rows' places would be kept)
+          to += static_cast<int64_t>(r < 3 ? 1 : 13) * N;
+          asm volatile("" : "+v"(to));
         }
-        to += static_cast<int64_t>(16) * N;
       }
     };
     behind = (t.n + 1) * 4 * kCols <= N;

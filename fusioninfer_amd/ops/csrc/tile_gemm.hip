@@ -25,8 +25,15 @@
 // Rows lie in LDS as eight chunks of 16 bytes, chunk c of row r at c ^ key(r):
 // the 16 lanes that LDS serves together then touch all its banks (no
 // conflicts counted), and a DMA still reads whole lines of eight rows.
-// bf16: MFMA 16x16x32 with A = W, B = x; the W rows of a fragment pair are
-// dealt so that a lane ends with eight neighbouring outputs of one row of x.
+//
+// MFMA with A = x, B = W, 16x16x32 in bf16. A wave's 128 columns are dealt to the
+// places of its fragments so that lane i of 16 has columns 8 i to 8 i + 7 of a
+// row, 16 bytes beside the next lane's: a CU takes stores 64 bytes of neighbouring
+// lanes at a time, a tile's 128 KB in 0.9 us so, in 3.5 with A = W, where
+// neighbouring lanes have neighbouring rows. (Once all CUs write at the same time
+// memory takes as long.) us, the latter and this: 8000 x 2048, N 5120 142.9 and
+// 139.4; e4m3, 8 bytes a lane, 8100 x 4096, N 6144, 4096, 24576 166, 106, 603 and
+// 161, 101, 585; 4099 x 4096, N 6144 102 and 98.
 //
 // What whole rounds of 256 tiles leave over is cut along K into equal pieces
 // (tile_plan), which a second kernel sums in a fixed order.
@@ -90,26 +97,14 @@ FI_DEV Tile tile_at(const TilePlan& p, int at) {
 }
 
 // What the operands' type decides. A fragment is kRows rows of either operand
-// by half a stage of K; a lane has kChunks chunks of a row of it and kQuads
-// times four results of a product.
-//
-// w_row: W row (of the tile) of fragment f's row 0 in wave column wn; w_at:
-// how much further on row i of the fragment lies. A lane's results are then
-// neighbouring outputs of one row of x: eight of a fragment pair (bf16), 16
-// of a fragment (e4m3).
+// by half a stage of K; a lane has kChunks chunks of a row of it and, of a
+// product, kQuads times four results, neighbouring rows of x in one column.
 template <bool FP8>
 struct Kind {
   using Elem = u16;
   using Frag = short8;
   using Acc = floatx4;
   static constexpr int kRows = 16, kChunks = 1, kQuads = 1;
-  static constexpr int w_row(int f, bool silu_mul) {
-    return silu_mul ? (f >> 2) * 128 + (f >> 1 & 1) * 32 + (f & 1) * 4
-                    : (f >> 1) * 32 + (f & 1) * 4;
-  }
-  FI_DEV static int w_at(int i) { return (i >> 2) * 8 + (i & 3); }
-  // three bits of W's row that tell a fragment's rows of one parity apart
-  FI_DEV static u32 w_key(int r) { return (r >> 1 & 1) | (r >> 3 & 3) << 1; }
   FI_DEV static void put(Frag& f, int, const short8& v) { f = v; }
 };
 template <>
@@ -118,11 +113,6 @@ struct Kind<true> {
   using Frag = intx8;
   using Acc = floatx16;
   static constexpr int kRows = 32, kChunks = 2, kQuads = 4;
-  static constexpr int w_row(int f, bool) { return f * 32; }
-  FI_DEV static int w_at(int i) {
-    return (i >> 2 & 1) * 16 + (i >> 3) * 4 + (i & 3);
-  }
-  FI_DEV static u32 w_key(int r) { return (r >> 1 & 3) | (r >> 4 & 1) << 2; }
   FI_DEV static void put(Frag& f, int chunk, const short8& v) {
     const intx4 q = __builtin_bit_cast(intx4, v);
 #pragma unroll
@@ -133,30 +123,41 @@ struct Kind<true> {
 // what becomes of the products: nothing, + bias, silu(gate) * up, gelu
 enum { PLAIN, BIAS, SILU, GELU };
 
-// eight outputs of a row of x: sums a, b; SILU: of gate values, the up values
-// that go with them in u, v. FP8: times xs, the row's scale, and the scales
-// of W's rows at ws.
-template <int MODE, bool FP8>
-FI_DEV void store8(u16* to, const u16* bias, floatx4 a, floatx4 b,
-                   const floatx4& u, const floatx4& v, float xs,
-                   const floatx4* ws) {
-  bf16x8 o, add;
-  if (MODE == BIAS) add = *reinterpret_cast<const bf16x8*>(bias);
-  if (FP8) {
-    a *= xs * ws[0];
-    b *= xs * ws[1];
-  }
+// C neighbouring outputs of a row of x, from its sums and (SILU) the up values
+// that go with them. FP8: times xs, the row's scale, and ws, those of W's rows.
+template <int MODE, bool FP8, int C>
+FI_DEV void store_row(u16* to, const u16* bias, const float (&sum)[C],
+                      const float (&up)[C], float xs, const float* ws) {
+  struct alignas(2 * C) Outputs {
+    u16 h[C];
+  } o, add;
+  if (MODE == BIAS) add = *reinterpret_cast<const Outputs*>(bias);
 #pragma unroll
-  for (int r = 0; r < 8; ++r) {
-    float y = r < 4 ? a[r] : b[r - 4];
-    if (MODE == SILU)
-      y = silu(y) * (r < 4 ? u[r] : v[r - 4]);
+  for (int c = 0; c < C; ++c) {
+    float y = sum[c];
+    if (FP8) y *= xs * ws[c];
+    if (MODE == SILU) y = silu(y) * up[c];
     if (MODE == GELU) y = gelu(y);
-    if (MODE == BIAS) y += bf16_to_f32(add.h[r]);
-    o.h[r] = f32_to_bf16(y);
+    if (MODE == BIAS) y += bf16_to_f32(add.h[c]);
+    o.h[c] = f32_to_bf16(y);
   }
-  *reinterpret_cast<bf16x8*>(to) = o;
+  *reinterpret_cast<Outputs*>(to) = o;
 }
+
+// Where a lane's results lie. Slot i of fragment f holds column i * kLaneCols +
+// f % kLaneCols of the wave's, so a lane has the kLaneCols neighbouring columns
+// of its kLaneRows rows of a fragment of x.
+template <bool FP8, bool SILU_MUL>
+struct Lanes {
+  static constexpr int kRows = Kind<FP8>::kRows, kFrags = 128 / kRows;
+  static constexpr int kLaneRows = kRows * kRows / kWaveSize;
+  static constexpr int kLaneCols = SILU_MUL ? kFrags / 2 : kFrags;
+  static_assert(!FP8 || !SILU_MUL);
+  // row of a fragment that a lane's result r of it belongs to
+  FI_DEV static int row(int lane, int r) {
+    return (r >> 2) * 8 + lane / kRows * 4 + (r & 3);
+  }
+};
 
 template <int MODE, bool FP8>
 __global__ __launch_bounds__(256, 1)
@@ -219,14 +220,21 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
   // offset, and need not be right where that is negative).
   const u32 ab = static_cast<u32>(x_stride) * kElemB, wb = K * kElemB;
   u32 a_voff[8], b_voff[4];
+  using L = Lanes<FP8, SILU_MUL>;
+  // the W row of the half tile that lies in its slot s
+  auto column_at = [](int s) {
+    constexpr int kWave = L::kRows * L::kLaneCols;
+    return s / kWave * kWave + s % L::kRows * L::kLaneCols +
+           s % kWave / L::kRows;
+  };
 #pragma unroll
   for (int j = 0; j < 8; ++j)
     a_voff[j] = ((wave + 4 * j) * 8 + (lane >> 3)) * ab +
                 (((lane & 7) ^ ((lane >> 4) | ((wave & 1) << 2))) << 4);
 #pragma unroll
   for (int j = 0; j < 4; ++j)
-    b_voff[j] = ((wave + 4 * j) * 8 + (lane >> 3)) * wb +
-                (((lane & 7) ^ T::w_key(wave * 8 + (lane >> 3))) << 4);
+    b_voff[j] = column_at((wave + 4 * j) * 8 + (lane >> 3)) * wb +
+                (((lane & 7) ^ ((lane >> 4) | ((wave & 1) << 2))) << 4);
   u32x4 da, db, dc;             // x rows, first and second half of W's rows
   constexpr int kPast = 1 << 30;
   int ru = 0, rs = 0, rend = 0, rlo = 0, left = 0;
@@ -281,9 +289,8 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
   constexpr int kRows = T::kRows, kChunks = T::kChunks, kFrags = 8 / kChunks;
   const int ir = lane % kRows, q = lane / kRows * kChunks;
   const u32 a_rd = (wm * 128 + ir) * kRowB + ((q ^ (ir >> 1 & 7)) << 4);
-  const u32 b_rd = kHalfB +
-                   (wn * (SILU_MUL ? 64 : 128) + T::w_at(ir)) * kRowB +
-                   ((q ^ T::w_key(T::w_at(ir))) << 4);
+  const u32 b_rd = kHalfB + (wn * (SILU_MUL ? 64 : 128) + ir) * kRowB +
+                   ((q ^ (ir >> 1 & 7)) << 4);
   using Frag = typename T::Frag;
   auto rda = [&](Frag (&to)[kFrags], int buf, int half, int i) {
     const int mi = i / kChunks, c = i % kChunks;
@@ -295,7 +302,7 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
     const int f = i / kChunks, c = i % kChunks;
     T::put(to[f], c, *reinterpret_cast<const short8*>(
         smem + buf * kStageB + (b_rd ^ (half * 64 + c * 16)) +
-        T::w_row(f, SILU_MUL) * kRowB));
+        (SILU_MUL ? (f >> 2) * 128 + (f & 3) * 16 : f * kRows) * kRowB));
   };
   Frag a0[kFrags], b0[kFrags], a1[kFrags], b1[kFrags];
   typename T::Acc acc[kFrags][kFrags];
@@ -306,8 +313,8 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
     constexpr int kEach = 64 / (kFrags * kFrags);
     const int mi = i / kEach / kFrags, f = i / kEach % kFrags;
     if (i % kEach == 0) {
-      if (first) mfma_first(acc[mi][f], b[f], a[mi]);
-      else mfma(acc[mi][f], b[f], a[mi]);
+      if (first) mfma_first(acc[mi][f], a[mi], b[f]);
+      else mfma(acc[mi][f], a[mi], b[f]);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -331,9 +338,9 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
   int buf = 0;
   constexpr int kFree = 40, kEarly = 6;  // MFMAs up to the first barrier, DMAs
                                          // between the two
-  // of a whole tile, at least: 16 bytes are one instruction or more, and a
-  // wait that counts too few is only longer
-  constexpr int kStores = SILU_MUL ? 16 : 32;
+  // of a whole tile, at least (a row's outputs are one instruction or more, and a
+  // wait that counts too few is only longer), as far as the counter goes
+  constexpr int kStores = FP8 ? 63 - kEarly : 32;
   // `behind`: that many follow the DMAs that are waited for
   auto stage = [&](auto first, bool behind) {
 #pragma unroll
@@ -391,57 +398,59 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
     asm volatile("" : "+v"(l));
     const int row0 = t.m * kTile + wm * 128;
     if (t.count == SK) {
-      const int row1 = row0 + l % kRows;
-      const int col1 = t.n * kCols + wn * (kCols / 2) +
-                       l / kRows * (FP8 ? 16 : 8);
-      u16* to = out + row1 * out_stride + col1;
-      const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
-      // eight outputs at a time: 16 columns on per fragment (pairs of them in
-      // bf16, halves of them in e4m3)
-      constexpr int kEights = SILU_MUL ? 4 : 8;
+      constexpr int kLaneCols = L::kLaneCols;
+      const int row1 = row0 + L::row(l, 0);
+      const int col1 = t.n * kCols + wn * (kCols / 2) + l % kRows * kLaneCols;
       // scales, all of them before the first store and waited for on every
       // path: a load behind a store waits for it too, and one that may still
       // be under way at the next stage would make that wait for all DMAs
-      float xs[4] = {};
-      floatx4 ws[16] = {};
+      floatx4 xs[16] = {}, ws = {};
       if (FP8) {
+        if (row0 + 128 <= M) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) xs[i] = x_scales[min(row1 + i * 32, M - 1)];
+          for (int i = 0; i < 16; ++i)
+            __builtin_memcpy(&xs[i], x_scales + row1 + i * 8, 16);
+        } else {
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
-          ws[i] = reinterpret_cast<const floatx4*>(
-              w_scales + min(col1 + i / 4 * 32, cols - 16))[i % 4];
+          for (int i = 0; i < 16; ++i)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(xs[i]));
+            for (int r = 0; r < 4; ++r)
+              xs[i][r] = x_scales[min(row1 + i * 8 + r, M - 1)];
+        }
+        ws = *reinterpret_cast<const floatx4*>(w_scales + min(col1, cols - 4));
 #pragma unroll
-        for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(ws[i]));
+        for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(xs[i]));
+        asm volatile("" : "+v"(ws));
       }
       auto store = [&](bool inside) {
+        if (!inside && col1 >= cols) return;
+        const u16* add = MODE == BIAS ? bias + col1 : nullptr;
+        constexpr int kGroups = L::kLaneRows / 4, kGap = kRows / kGroups;
+        u16* to = out + row1 * out_stride + col1;
+        int row = row1;
 #pragma unroll
-        for (int mi = 0; mi < kFrags; ++mi) {
-          if (inside || row1 + mi * kRows < M) {
+        for (int g = 0; g < kFrags * kGroups; ++g) {
 #pragma unroll
-            for (int i = 0; i < kEights; i += 2) {
-              if (inside || col1 + i * 16 < cols) {
-                const u16* add = MODE == BIAS ? bias + col1 + i * 16 : nullptr;
-                if constexpr (FP8) {
+          for (int r = 0; r < 4; ++r) {
+            const auto& of = acc[g / kGroups];
+            const int at = g % kGroups * 4 + r;
+            if (inside || row < M) {
+              float sum[kLaneCols], up[kLaneCols];
 #pragma unroll
-                  for (int e = 0; e < 2; ++e)
-                    store8<MODE, FP8>(to + i * 16 + e * 8, nullptr,
-                                      quad_of(acc[mi][i / 2], 2 * e),
-                                      quad_of(acc[mi][i / 2], 2 * e + 1), zero,
-                                      zero, xs[mi], &ws[i * 2 + e * 2]);
-                } else {
-                  store8<MODE, FP8>(
-                      to + i * 16, add, acc_of(acc[mi][i]),
-                      acc_of(acc[mi][i + 1]),
-                      SILU_MUL ? acc_of(acc[mi][(i + 4) % 8]) : zero,
-                      SILU_MUL ? acc_of(acc[mi][(i + 5) % 8]) : zero, 0.f, ws);
-                }
+              for (int c = 0; c < kLaneCols; ++c) {
+                sum[c] = acc_of(of[c][at]);
+                up[c] = SILU_MUL ? acc_of(of[c + kFrags - kLaneCols][at]) : 0.f;
               }
+              store_row<MODE, FP8, kLaneCols>(
+                  to, add, sum, up, xs[FP8 ? g : 0][r],
+                  reinterpret_cast<const float*>(&ws));
             }
+            // (a step at a time, or all rows' places would be kept)
+            const int step = r < 3 ? 1 : kGap - 3;
+            to += step * out_stride;
+            row += step;
+            asm volatile("" : "+v"(to), "+v"(row));
           }
-          to += kRows * out_stride;
         }
       };
       behind = t.m * kTile + kTile <= M && t.n * kCols + kCols <= cols;
@@ -450,18 +459,22 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
       else
         store(false);
     } else {
+      // four columns (of a lane's) of a row at a time
       floatx4* p = pieces + static_cast<int64_t>(place) * kPiece +
                    wave * 64 * kWaveSize + l;
 #pragma unroll
       for (int mi = 0; mi < kFrags; ++mi) {
         if (row0 + mi * kRows < M) {
 #pragma unroll
-          for (int f = 0; f < kFrags; ++f)
+          for (int r = 0; r < L::kLaneRows; ++r)
 #pragma unroll
-            for (int g = 0; g < T::kQuads; ++g)
-              p[(f * T::kQuads + g) * kWaveSize] = quad_of(acc[mi][f], g);
+            for (int f = 0; f < kFrags; f += 4)
+              p[(r * kFrags + f) / 4 * kWaveSize] =
+                  floatx4{acc_of(acc[mi][f][r]), acc_of(acc[mi][f + 1][r]),
+                          acc_of(acc[mi][f + 2][r]),
+                          acc_of(acc[mi][f + 3][r])};
         }
-        p += kFrags * T::kQuads * kWaveSize;
+        p += L::kLaneRows * kFrags / 4 * kWaveSize;
       }
     }
   }
@@ -469,8 +482,8 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-// Sums the pieces of the cut tiles: blockIdx.y is the tile, a thread takes
-// eight outputs.
+// Sums the pieces of the cut tiles: blockIdx.y is the tile, a thread takes a
+// lane's columns of one row, in kOps quads.
 template <int MODE, bool FP8>
 __global__ __launch_bounds__(256)
 void tile_gemm_join_kernel(u16* __restrict__ out,
@@ -480,31 +493,24 @@ void tile_gemm_join_kernel(u16* __restrict__ out,
                            const float* __restrict__ w_scales, const int M,
                            const int N, const int64_t out_stride,
                            const TilePlan plan) {
-  using T = Kind<FP8>;
   constexpr bool SILU_MUL = MODE == SILU;
-  constexpr int kCols = SILU_MUL ? kTile / 2 : kTile;
+  using L = Lanes<FP8, SILU_MUL>;
+  constexpr int kCols = SILU_MUL ? kTile / 2 : kTile, kRows = L::kRows;
   const int cols = SILU_MUL ? N / 2 : N;
-  constexpr int kFrags = 8 / T::kChunks, kQuads = kFrags * T::kQuads;
-  // pairs of quads of a wave's row of fragments (SILU: of its gate half)
-  constexpr int kPairs = kQuads / (SILU_MUL ? 4 : 2);
+  constexpr int kOps = L::kFrags / 4, kLaneCols = L::kLaneCols;
   const int i = blockIdx.x * 256 + threadIdx.x;
-  const int lane = i % kWaveSize, pair = i / kWaveSize % kPairs;
-  const int mi = i / kWaveSize / kPairs % kFrags;
-  const int wave = i / kWaveSize / kPairs / kFrags;
+  const int lane = i % kWaveSize, r = i / kWaveSize % L::kLaneRows;
+  const int mi = i / kWaveSize / L::kLaneRows % L::kFrags;
+  const int wave = i / kWaveSize / L::kLaneRows / L::kFrags;
   const Tile tile = tile_at(plan, plan.whole * kChip + blockIdx.y);
-  const int m = tile.m, n = tile.n;
-  const int row = m * kTile + (wave >> 1) * 128 + mi * T::kRows +
-                  lane % T::kRows;
-  const int col = n * kCols + (wave & 1) * (kCols / 2) +
-                  (FP8 ? (pair >> 1) * 32 + lane / T::kRows * 16 +
-                             (pair & 1) * 8
-                       : pair * 32 + lane / T::kRows * 8);
+  const int row = tile.m * kTile + (wave >> 1) * 128 + mi * kRows +
+                  L::row(lane, r);
+  const int col = tile.n * kCols + (wave & 1) * (kCols / 2) +
+                  lane % kRows * kLaneCols;
   if (row >= M || col >= cols) return;
-  constexpr int kOps = SILU_MUL ? 4 : 2;
-  floatx4 s[4];
-  const floatx4* p =
-      pieces + static_cast<int64_t>(blockIdx.y) * kPiece +
-      ((wave * kFrags + mi) * kQuads + pair * 2) * kWaveSize + lane;
+  floatx4 s[kOps];
+  const floatx4* p = pieces + static_cast<int64_t>(blockIdx.y) * kPiece +
+                     i / kWaveSize * kOps * kWaveSize + lane;
   const int64_t next = static_cast<int64_t>(plan.rest) * kPiece;
   for (int c = 0; c < plan.cut; c += 4) {
     floatx4 v[4][kOps];
@@ -512,19 +518,22 @@ void tile_gemm_join_kernel(u16* __restrict__ out,
     for (int k = 0; k < 4; ++k)   // pieces past the last repeat it
 #pragma unroll
       for (int o = 0; o < kOps; ++o)
-        v[k][o] = p[min(c + k, plan.cut - 1) * next +
-                    ((o & 1) + (o >> 1) * (kQuads / 2)) * kWaveSize];
+        v[k][o] = p[min(c + k, plan.cut - 1) * next + o * kWaveSize];
 #pragma unroll
     for (int k = 0; k < 4; ++k)
       if (c + k < plan.cut)
 #pragma unroll
         for (int o = 0; o < kOps; ++o) s[o] = c + k ? s[o] + v[k][o] : v[k][o];
   }
-  store8<MODE, FP8>(out + row * out_stride + col,
-                    MODE == BIAS ? bias + col : nullptr, s[0], s[1],
-                    s[SILU_MUL ? 2 : 0], s[SILU_MUL ? 3 : 1],
-                    FP8 ? x_scales[row] : 0.f,
-                    reinterpret_cast<const floatx4*>(w_scales + col));
+  float sum[kLaneCols], up[kLaneCols];
+#pragma unroll
+  for (int c = 0; c < kLaneCols; ++c) {
+    sum[c] = s[c / 4][c % 4];
+    up[c] = SILU_MUL ? s[kOps - 1][c % 4] : 0.f;
+  }
+  store_row<MODE, FP8, kLaneCols>(out + row * out_stride + col,
+                                  MODE == BIAS ? bias + col : nullptr, sum, up,
+                                  FP8 ? x_scales[row] : 0.f, w_scales + col);
 }
 
 // A stage takes 1.42 us (e4m3 too); a piece costs 0.06 us of the way through
@@ -570,7 +579,7 @@ void launch(u16* out, float* pieces, const typename Kind<FP8>::Elem* x,
                      x_stride, out_stride, p, turn);
   if (p.cut > 1)
     hipLaunchKernelGGL((tile_gemm_join_kernel<MODE, FP8>),
-                       dim3(MODE == SILU ? 16 : 32, p.rest), dim3(256), 0,
+                       dim3(FP8 ? 64 : 32, p.rest), dim3(256), 0,
                        stream, out, pc, bias, x_scales, w_scales, M, N,
                        out_stride, p);
 }
