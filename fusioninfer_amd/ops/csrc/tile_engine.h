@@ -90,12 +90,6 @@ FI_DEV float acc_of(float a) {
 FI_DEV floatx4 acc_of(const floatx4& a) {
   return floatx4{acc_of(a[0]), acc_of(a[1]), acc_of(a[2]), acc_of(a[3])};
 }
-// four of a lane's results of a wave's fragment
-FI_DEV floatx4 quad_of(const floatx4& a, int) { return acc_of(a); }
-FI_DEV floatx4 quad_of(const floatx16& a, int g) {
-  return floatx4{acc_of(a[4 * g]), acc_of(a[4 * g + 1]), acc_of(a[4 * g + 2]),
-                 acc_of(a[4 * g + 3])};
-}
 FI_DEV void settle() {
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);

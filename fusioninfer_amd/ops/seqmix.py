@@ -14,6 +14,7 @@ these ops compiles only these sources on first use.
 
 from __future__ import annotations
 
+import itertools
 from typing import Optional
 
 import numpy as np
@@ -507,9 +508,24 @@ class ContextRows:
             table[i, : c - lo] = a + pos - lo
         place = np.concatenate([np.arange(c - lo - n, c - lo)
                                 for n, c, lo, _ in spans])
-        self.slots = torch.from_numpy(slots).to(device)
-        self.table = torch.from_numpy(table).to(device)
-        self.positions = torch.from_numpy(place.astype(np.int32)).to(device)
+        self.slots, self.table, self.positions = _to_device(
+            (slots, table, place.astype(np.int32)), device)
+
+
+def _to_device(arrays, device):
+    """int32 arrays on a device, in one copy that the host does not wait for.
+    (Copies out of pageable memory wait for all that the GPU still has to do:
+    three of them in a prompt's first latent layer, and the GPU then had nothing
+    while the host launched the other layers. Four prompts of 1.8 thousand
+    tokens, four layers, and eight tokens each: 5245 us a pass, 5120 without.)"""
+    starts = list(itertools.accumulate((-(-a.size // 4) * 4 for a in arrays),
+                                       initial=0))
+    host = torch.empty(starts[-1], dtype=torch.int32,
+                       pin_memory=torch.device(device).type == "cuda")
+    for a, at in zip(arrays, starts):
+        host[at: at + a.size].view(a.shape).copy_(torch.from_numpy(a))
+    dev = host.to(device, non_blocking=True)
+    return [dev[at: at + a.size].view(a.shape) for a, at in zip(arrays, starts)]
 
 
 def context_starts(spans, window: int):

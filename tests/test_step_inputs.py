@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 import torch
 
+from fusioninfer_amd.ops import seqmix
 from test_engine import make_engine
 
 
@@ -69,3 +70,33 @@ def test_decode_inputs_and_padding_rows(runner, n, bs):
     runner._fill_decode_inputs(dict(payload, ids=None), bs)
     assert st["ids"][:bs].tolist() == [6] * n + [0] * pad
     runner._static = {}
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param(
+    "cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("window", [0, 24])
+def test_context_rows_in_one_copy(device, window):
+    """The rows of portions at the start of, within and across blocks, made
+    without a wait for the GPU."""
+    spans = [(5, 5, [3]), (16, 33, [7, 1, 4]), (1, 50, [9, 2, 8, 0]),
+             (40, 40, [5, 6, 10])]
+    if device == "cuda":
+        torch.cuda.init()
+        torch.cuda.set_sync_debug_mode("error")
+    try:
+        rows = seqmix.ContextRows(spans, 16, device, window)
+    finally:
+        if device == "cuda":
+            torch.cuda.set_sync_debug_mode("default")
+    slots, places, first = [], [], 0
+    for (n, c, blocks), lo in zip(spans, seqmix.context_starts(spans, window)):
+        assert rows.table[len(places), : c - lo].tolist() == list(
+            range(first, first + c - lo))
+        assert not rows.table[len(places), c - lo:].any()
+        slots += [blocks[p // 16] * 16 + p % 16 for p in range(lo, c)]
+        places.append(list(range(c - lo - n, c - lo)))
+        first += c - lo
+    assert rows.count == first and rows.slots.tolist() == slots
+    assert rows.positions.tolist() == sum(places, [])
+    assert {t.dtype for t in (rows.slots, rows.table, rows.positions)} == {
+        torch.int32}
