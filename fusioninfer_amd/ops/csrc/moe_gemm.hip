@@ -249,24 +249,26 @@ __global__ __launch_bounds__(256) void moe_gemm_fp8_kernel(
 
 }  // namespace
 
-// Whether blocks of 128 rows go by tiles of 512 columns, one per CU, or by
-// those of 256, two per CU. A round of the wide ones takes 0.85 of the time
-// that the others need for as many products, but a round that is begun takes
-// all of it; the others lose a quarter of a round. How many blocks there are
-// only the GPU knows: every expert is taken to leave half a block empty.
-// Where experts have less than a block and a half on average, gate and up
-// are bound by the weights and the wide tiles, with fewer loads in flight,
-// lose 5 % (128 experts, 2048 x 768, 1024 rows of top 8: 157 us, wide 165).
-// Over 62 products of six shapes of experts (256 to 8765 rows) this choice
-// takes 2.1 % longer than the better of the two, the narrow tiles alone 6.8,
-// the wide ones alone 4.7; against the narrow ones it loses 2 % at most.
+// Whether blocks of 128 rows go by tiles of 512 columns, one per CU (256 of two
+// blocks), or by those of 256, two per CU. A round of the wide ones takes 0.82
+// (gathered rows: 0.88) of the time that the others need for as many products,
+// but a round that is begun takes all of it; the others lose a quarter of a
+// round. How many blocks there are only the GPU knows: every expert is taken to
+// leave half a block empty. Where most experts have one block, gate and up are
+// bound by the weights and the wide tiles, with fewer loads in flight, lose 6 %;
+// where most have two, whose weights a CU then loads once for both, they gain 15
+// (128 experts, 2048 x 768, top 8, us, narrow and wide: 1024 rows 161 and 171,
+// 2048 203 and 216, 2500 230 and 196, 3000 215 and 193; 64 experts, 2048 x 1408,
+// top 6: 1024 rows 153 and 169, 1500 216 and 203). Over 54 products of three
+// shapes of experts (600 to 8100 rows) this choice takes 0.9 % longer than the
+// better of the two, the narrow tiles alone 11.
 bool wide_tiles(int max_mtiles, int experts, int K, int N, int mode) {
   if (K % 64 != 0 || K < 128) return false;
   const int cols = mode == 1 || mode == 3 ? 256 : 512;
-  if (mode != 0 && 2 * max_mtiles < 5 * experts) return false;
+  if (mode != 0 && 10 * max_mtiles < 21 * experts) return false;
   const double blocks = max_mtiles - 0.5 * experts;
   const double rounds = std::ceil(blocks * ceil_div(N, cols) / 256);
-  return 0.85 * rounds < blocks * N / cols / 256 + 0.25;
+  return (mode == 0 ? 0.82 : 0.88) * rounds < blocks * N / cols / 256 + 0.25;
 }
 
 // block_m 16: few rows per expert, bound by the weights; 128: many.

@@ -9,6 +9,15 @@
 // (48 bytes a cycle and CU, of 64 that the first-level cache delivers; here
 // 40).
 //
+// Two neighbouring blocks of an expert take tiles of 256 rows by 256 columns
+// instead, waves two by two: 64 KB a stage, not 80, and every fragment of B once
+// for both. (All that differs is where a wave's requests go and what it reads; a
+// wave's products are the same.) 128 experts, top 8, 2048 x 768, both products,
+// us, blocks apart and in pairs: 8100 rows 645 and 614, 4000 401 and 380; 64
+// experts, 2048 x 1408, top 6, 8192 rows 850 and 806; 8 experts, 4096 x 6144, top
+// 2, 8192 rows 2128 and 2102. (K begun elsewhere by columns or by blocks, so that
+// CUs read other channels: 630 and 635 instead of 614.)
+//
 // A stage is 64 of K: 128 gathered rows of 128 bytes, and 64 of B's packed
 // fragments (1 KB each), 80 KB in all; two of them are kept, all of a CU's
 // LDS. As in the dense kernel of 256 x 256 tiles a stage is used in two halves:
@@ -83,89 +92,144 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
   const int end = min(run0 + per, total);
   if (first >= end) return;
   constexpr int kNext = kChip / 8;
+  // A place in the order is a block's n-th wide tile. Where it and a neighbour
+  // are a pair, the places of both are the pair's square tiles, of half as many
+  // columns; there may be one fewer.
   struct Place {
-    int m, n;
+    int m, n;      // first block, columns
+    int square, none;
   };
-  auto place_of = [&](int at) {
+  const ConstInts experts = const_ints(expert_ids);
+  auto place_of = [&](int at) __attribute__((always_inline)) {
     const int m0 = at / (kRunRows * NT) * kRunRows;
     const int rows = min(kRunRows, nv - m0);
     const int in = at - m0 * NT;
-    const int n = in / rows;
-    return Place{m0 + in - n * rows, n};
+    const int n = in / rows, m = m0 + in - n * rows;
+    const int e = experts[m];
+    int before = 0;              // blocks of the expert in front of this one
+    for (int top = m; top > 0;) {
+      constexpr int kLook = 8;   // ids at a time
+      const int from = max(top - kLook, 0);
+      int id[kLook], same = 0;
+#pragma unroll
+      for (int i = 0; i < kLook; ++i) id[i] = experts[max(top - 1 - i, from)];
+#pragma unroll
+      for (int i = 0; i < kLook; ++i)
+        same += same == i && top - i > from && id[i] == e;
+      before += same;
+      if (same < top - from) break;
+      top = from;
+    }
+    const bool second = before & 1;
+    if (!second && !(m + 1 < nv && experts[min(m + 1, nv - 1)] == e))
+      return Place{m, n, 0, 0};
+    const int column = (second ? NT : 0) + n;
+    return Place{m - second, column, 1, column * (GATE_UP ? 128 : 256) >= N};
   };
 
-  // ---- requests: DMAs 0 to 3 bring eight rows of A each, the others a
-  // fragment of this wave's B
+  // ---- requests. Of a wide tile DMAs 0 to 3 bring eight rows of A each and 4 to
+  // 19 a fragment of this wave's B; of a square one 0 to 7 rows and 8 to 15 the
+  // fragments of half a stage of two waves' B.
   const int NB16 = (GATE_UP ? 2 * N : N) / 16;
   const u32 b_step = static_cast<u32>(NB16) * 1024;   // 32 of K
   constexpr int kOwn = GATE_UP ? 4 : 8;   // fragments apart from up's
   const u32 up = N / 16 * 1024u;
-  u32 a_voff[4];
+  u32 a_voff[8] = {};
   u32x4 da, db;
   int rat = first, left = 0;
-  u32 a_soff = 0, b_soff = 0, b_col[kOwn];
-  auto aim = [&] {
-    a_soff = b_soff = 0;
-    if (rat >= end) {           // past the end the last tile's beginning again
+  u32 a_soff = 0, b_soff[2] = {}, b_col[kOwn];
+  // where DMAs 0 to 3, 4 to 7, 8 to 11 and the others go in a stage, less 1 KB
+  // each for those before
+  u32 to_lds[4];
+  int rsquare = 0;
+  Place next{}, after{}, third{};   // tiles that are requested, not yet done
+  int waiting = 0;
+  auto put = [&](Place& at, const Place& t, int turn) {
+    at.m = waiting == turn ? t.m : at.m;
+    at.n = waiting == turn ? t.n : at.n;
+    at.square = waiting == turn ? t.square : at.square;
+  };
+  // (out of line captures would be in memory, and no value uniform)
+  auto aim = [&]() __attribute__((always_inline)) {
+    Place t{0, 0, 0, 1};
+    for (; rat < end && t.none; rat += kNext) t = place_of(rat);
+    a_soff = 0;
+    if (t.none) {               // past the end the last tile's beginning again
+      b_soff[0] = rsquare ? (wave & 1) * b_step : 0;
+      b_soff[1] = rsquare ? b_soff[0] : b_step;
       left = 1 << 30;
       return;
     }
-    const Place t = place_of(rat);
-    rat += kNext;
-    int ids[32];
-    if (MODE != 0) {
-      const auto from = const_ints(sorted_ids + t.m * kWideM + wave * 32);
+    put(next, t, 0);
+    put(after, t, 1);
+    put(third, t, 2);
+    ++waiting;
+    rsquare = t.square;
+    b_soff[0] = rsquare ? (wave & 1) * b_step : 0;
+    b_soff[1] = rsquare ? b_soff[0] : b_step;
+    to_lds[0] = wave * (rsquare ? 8192 : 4096);
+    to_lds[1] = rsquare ? to_lds[0] : kRowsB + wave * kWaveB - 4096;
+    to_lds[2] = rsquare ? 2 * kRowsB + wave * 8192 - 4096 : to_lds[1];
+    to_lds[3] = rsquare ? to_lds[2] - 8192 : to_lds[1];
 #pragma unroll
-      for (int i = 0; i < 32; ++i) ids[i] = from[i];
-      // in scalar registers, or the choice by lane becomes a vector load
-#pragma unroll
-      for (int i = 0; i < 32; ++i) asm volatile("" : "+s"(ids[i]));
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      int row = wave * 32 + i * 8 + (lane >> 3);
+    for (int h = 0; h < 2; ++h) {
+      // (a wide tile's a second time: around a branch they would be vector loads)
+      const int row0 = wave * (rsquare ? 64 : 32) + (rsquare ? h * 32 : 0);
+      int ids[32];
       if (MODE != 0) {
-        row = ids[i * 8];
+        const auto from =
+            const_ints(sorted_ids + t.m * kWideM + row0);
 #pragma unroll
-        for (int r = 1; r < 8; ++r)
-          row = (lane >> 3) == r ? ids[i * 8 + r] : row;
+        for (int i = 0; i < 32; ++i) ids[i] = from[i];
+        // in scalar registers, or the choice by lane becomes a vector load
+#pragma unroll
+        for (int i = 0; i < 32; ++i) asm volatile("" : "+s"(ids[i]));
       }
-      a_voff[i] = static_cast<u32>(row) * (K * 2) +
-                  (((lane & 7) ^ (lane >> 4 | (i & 1) << 2)) << 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        int row = row0 + i * 8 + (lane >> 3);
+        if (MODE != 0) {
+          row = ids[i * 8];
+#pragma unroll
+          for (int r = 1; r < 8; ++r)
+            row = (lane >> 3) == r ? ids[i * 8 + r] : row;
+        }
+        a_voff[h * 4 + i] = static_cast<u32>(row) * (K * 2) +
+                            (((lane & 7) ^ (lane >> 4 | (i & 1) << 2)) << 4);
+      }
     }
     da = MODE != 0 ? uniform_descriptor(a, a_bytes)
                    : uniform_descriptor(
                          a + static_cast<int64_t>(t.m) * kWideM * K,
-                         kWideM * K * 2);
-    const int e = const_ints(expert_ids)[t.m];
+                         kWideM * K * (rsquare ? 4 : 2));
     db = uniform_descriptor(
-        b + static_cast<int64_t>(e) * (K / 32) * NB16 * 512,
+        b + static_cast<int64_t>(experts[t.m]) * (K / 32) * NB16 * 512,
         K / 32 * b_step);
+    const int group = rsquare ? t.n * 2 + (wave >> 1) : t.n * 4 + wave;
 #pragma unroll
     for (int f = 0; f < kOwn; ++f)
-      b_col[f] = min((t.n * 4 + wave) * kOwn + f, N / 16 - 1) * 1024;
+      b_col[f] = min(group * kOwn + f, N / 16 - 1) * 1024;
     left = SK;
   };
   aim();
+  if (waiting == 0) return;
   u32 rbuf = lds0;
-  auto m0_of = [&](int j) {
-    set_m0(j < 4 ? rbuf + wave * 4096 + j * 1024
-                 : rbuf + kRowsB + wave * kWaveB + (j - 4) * 1024);
-  };
-  auto load_of = [&](int j) {
-    if (j < 4) {
-      load_lds(da, a_voff[j], a_soff);
+  auto m0_of = [&](int j) { set_m0(rbuf + to_lds[min(j / 4, 3)] + j * 1024); };
+  auto load_of = [&](int j) __attribute__((always_inline)) {
+    if (j >= 16 && rsquare) return;
+    if (j < 4 || (j < 8 && rsquare)) {
+      load_lds(da, a_voff[j % 8], a_soff);
     } else {
       const int f = (j - 4) % 8, half = (j - 4) / 8;
       load_lds(db, (lane ^ f) * 16u,
-               b_soff + half * b_step + b_col[f % kOwn] +
-                   (f >= kOwn ? up : 0));
+               b_soff[half] + b_col[f % kOwn] + (f >= kOwn ? up : 0));
     }
   };
-  auto requested = [&] {
+  auto requested = [&]() __attribute__((always_inline)) {
     rbuf = 2 * lds0 + kWideStageB - rbuf;
     a_soff += 128;
-    b_soff += 2 * b_step;
+    b_soff[0] += 2 * b_step;
+    b_soff[1] += 2 * b_step;
     if (--left == 0) aim();
   };
 
@@ -173,15 +237,22 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
   const int i16 = lane & 15, q = lane >> 4;
   const u32 a_rd = i16 * 128 + ((q ^ (i16 >> 1)) << 4);
   constexpr int kEach = GATE_UP ? 4 : 8;   // of a lane's columns in a row
-  const u32 b_rd = kRowsB + wave * kWaveB + i16 * kEach / 16 * 1024 +
+  const u32 b_rd = i16 * kEach / 16 * 1024 +
                    (q * 16 + ((i16 * kEach & 15) | i16 * kEach / 16)) * 16;
+  u32 a_at, b_at;                // of this wave in a stage
+  auto read_at = [&](int square) {
+    a_at = square ? (wave >> 1) * kRowsB : 0;
+    b_at = square ? 2 * kRowsB + (wave & 1) * kWaveB : kRowsB + wave * kWaveB;
+  };
+  read_at(next.square);
   auto rda = [&](u32 buf, int half, int mi) {
     return *reinterpret_cast<const short8*>(
-        smem + buf + (a_rd ^ (half * 64)) + mi * 2048);
+        smem + (buf + a_at) + (a_rd ^ (half * 64)) + mi * 2048);
   };
   auto rdb = [&](u32 buf, int half, int f) {
     return *reinterpret_cast<const short8*>(
-        smem + buf + (b_rd ^ (f * 16)) + half * 8192 + f / kEach * 4096);
+        smem + (buf + b_at) + (b_rd ^ (f * 16)) + half * 8192 +
+        f / kEach * 4096);
   };
   short8 a0[8], b0[8], a1[8], b1[8];
   floatx4 acc[8][8];
@@ -195,7 +266,7 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
     }
     requested();
   }
-  asm volatile("s_waitcnt vmcnt(20)" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
   sync_waves();
 #pragma unroll
   for (int f = 0; f < 8; ++f) {
@@ -209,8 +280,9 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
   constexpr int kStores = 32;
   constexpr int kFree = 40, kEarly = 6;  // MFMAs up to the first barrier, DMAs
                                          // between the two
-  // `behind`: stores that follow the DMAs that are waited for
-  auto stage = [&](auto first, bool behind) {
+  // `behind`: stores that follow the DMAs that are waited for; `last`: of the tile
+  auto stage = [&](auto first, bool behind,
+                   bool last) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 64; ++i) {
       const int mi = i >> 3, f = i & 7;
@@ -240,6 +312,7 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kEarly) : "memory");
     sync_waves();
     buf = kWideStageB - buf;
+    if (last) read_at(after.square);
 #pragma unroll
     for (int i = 0; i < 64; ++i) {
       const int mi = i >> 3, f = i & 7;
@@ -257,20 +330,25 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
   };
 
   bool behind = false;
-  for (int at = first; at < end; at += kNext) {
-    stage(std::true_type{}, behind);
-    for (int s = 1; s < SK; ++s) stage(std::false_type{}, false);
+  while (waiting > 0) {
+    stage(std::true_type{}, behind, false);
+    for (int s = 1; s < SK; ++s) stage(std::false_type{}, false, s == SK - 1);
     settle();
-    const Place t = place_of(at);
+    const Place t = next;
+    next = after;
+    after = third;
+    --waiting;
+    const int group = t.square ? t.n * 2 + (wave & 1) : t.n * 4 + wave;
+    const int block = t.square ? t.m + (wave >> 1) : t.m;
     // (from a fresh copy of the lane, or the addresses would be kept in
     // registers that the loop needs)
     int l = lane;
     asm volatile("" : "+v"(l));
-    const int col = t.n * 4 * kCols + wave * kCols + (l & 15) * kEach;
+    const int col = group * kCols + (l & 15) * kEach;
     auto store = [&](bool inside) {
       if (!inside && col >= N) return;
       u16* to = out +
-                static_cast<int64_t>(t.m * kWideM + (l >> 4) * 4) * N + col;
+                static_cast<int64_t>(block * kWideM + (l >> 4) * 4) * N + col;
 #pragma unroll
       for (int mi = 0; mi < 8; ++mi) {
 #pragma unroll
@@ -303,7 +381,7 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
         }
       }
     };
-    behind = (t.n + 1) * 4 * kCols <= N;
+    behind = (group + 1) * kCols <= N;
     if (behind) store(true);
     else store(false);
   }

@@ -2185,6 +2185,36 @@ def test_moe_gemm_wide_tiles_are_the_narrow_ones():
     assert torch.equal(out, few)
 
 
+@pytest.mark.parametrize("n,gate_up", [
+    (896, True), (1792, False),     # one square tile fewer than places
+    (1024, True), (2048, False)])
+def test_moe_gemm_pairs_of_blocks(n, gate_up):
+    """Experts of one block, whole pairs and pairs and one, and of more blocks
+    than are looked at together, have the bits of blocks taken alone."""
+    counts = [1, 2, 8, 9, 3, 16, 1, 16]
+    g = torch.Generator().manual_seed(n)
+    k, T, experts = 192, 700, len(counts)
+    eid = torch.tensor(sum(([e] * c for e, c in enumerate(counts)), []),
+                       dtype=torch.int32, device=DEV)
+    blocks = len(eid)
+    nv = torch.tensor([blocks], dtype=torch.int32, device=DEV)
+    sid = torch.randint(0, T, (blocks * 128,), generator=g).int().to(DEV)
+    x = torch.randn(T if gate_up else blocks * 128, k, generator=g)
+    w = torch.randn(experts, k, n * (2 if gate_up else 1), generator=g)
+    x, b = x.bfloat16().to(DEV), ops.pack_moe_weights(w.bfloat16().to(DEV))
+    wide, mode = ops._moe_native().moe_gemm_wide, 1 if gate_up else 0
+    assert wide(blocks, experts, k, n, mode)
+    assert not wide(8, experts, k, n, mode)
+    out = torch.zeros(blocks * 128, n, dtype=torch.bfloat16, device=DEV)
+    few = torch.zeros_like(out)
+    ops.moe_gemm(out, x, b, sid, eid, nv, 128, gate_up)
+    for m in range(0, blocks, 8):
+        rows = slice(m * 128, (m + 8) * 128)
+        ops.moe_gemm(few[rows], x if gate_up else x[rows], b, sid[rows],
+                     eid[m:m + 8], torch.full_like(nv, 8), 128, gate_up)
+    assert torch.equal(out, few)
+
+
 @pytest.mark.parametrize("k", [32, 224, 512, 768, 1024, 2080, 2624])
 @pytest.mark.parametrize("n,gate_up,act", [
     (64, True, None), (320, True, "clamped_glu"), (192, False, "relu_sq"),
