@@ -69,9 +69,9 @@ SEQMIX_SOURCES = [
 ]
 
 EXTENSIONS = {
-    "core": ("_C", SOURCES, ["common.h", "pieces.h", "prefill_kernel.h", "prefill_pair.h", "tile_engine.h"]),
+    "core": ("_C", SOURCES, ["common.h", "pieces.h", "prefill_kernel.h", "prefill_pair.h", "prefill_rows.h", "tile_engine.h"]),
     "seqmix": ("_C_seqmix", SEQMIX_SOURCES, ["common.h", "seqmix.h", "seqmix_bind.h",
-                "seqmix_hyper.h", "seqmix_scan.h", "prefill_kernel.h"]),
+                "seqmix_hyper.h", "seqmix_scan.h", "prefill_kernel.h", "prefill_rows.h"]),
     "moe": ("_C_moe", MOE_SOURCES, ["common.h", "seqmix.h", "tile_engine.h"]),
 }
 

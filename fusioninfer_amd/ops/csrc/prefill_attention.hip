@@ -2,6 +2,7 @@
 // the launch itself.
 
 #include "prefill_pair.h"
+#include "prefill_rows.h"
 
 #include <cmath>
 
@@ -181,7 +182,8 @@ void launch_prefill_attn(u16* out, const u16* q, const void* k, const void* v,
   a.nq = pl.nq;
   a.scale = scale;
   const dim3 block(pl.waves * kWaveSize);
-  const dim3 grid(num_q_heads / pl.hpb * pl.nq);
+  const dim3 grid(rows_grid(static_cast<int64_t>(num_q_heads / pl.hpb) *
+                            pl.nq, head_dim));
 #define FI_PF_LAUNCH(DD, PP, F8)                                              \
   do {                                                                        \
     if (pl.split) {                                                           \
@@ -189,14 +191,14 @@ void launch_prefill_attn(u16* out, const u16* q, const void* k, const void* v,
         hipLaunchKernelGGL((prefill_pair_kernel<4>), dim3(pl.slots),          \
                            dim3(4 * kWaveSize), 0, stream, a);                \
       else                                                                    \
-        hipLaunchKernelGGL((prefill_attn_kernel<DD, PP, F8, true>),           \
+        hipLaunchKernelGGL((prefill_attn_kernel<DD, PP, F8>),                 \
                            dim3(pl.slots), block, 0, stream, a);              \
       hipLaunchKernelGGL((prefill_attn_join_kernel<DD, PP>),                  \
                          dim3(pl.slots, pl.waves),                            \
                          dim3(DD / 16 * kWaveSize), 0, stream, a);            \
     } else {                                                                  \
-      hipLaunchKernelGGL((prefill_attn_kernel<DD, PP, F8, false>), grid,      \
-                         block, 0, stream, a);                                \
+      hipLaunchKernelGGL((prefill_rows_kernel<DD, PP, F8>), grid, block, 0,   \
+                         stream, a);                                          \
     }                                                                         \
   } while (0)
   if (fp8 && !paged) abort();  // fp8 KV is a cache format; dense is bf16

@@ -28,14 +28,11 @@
 //  * Rows are stored swizzled in 16-byte chunks so that both read patterns
 //    touch every bank evenly.
 // Bound by the vector ALU beside the matrix cores: a tile costs a wave 1024
-// cycles of MFMA and about as many of exponentials, maxima and packs, which
-// two waves per SIMD overlap in part. LDS reads (each wave reads the whole
-// tile) are at two thirds of their rate then.
+// cycles of MFMA and more of exponentials (512), scaling, sums, maxima, packs and
+// addresses, which two waves per SIMD overlap in part.
 //
-// Measured (32 query heads, 8 K/V heads, D 128; before -> now): 8 x 1024
-// tokens 225 -> 101 us (680 TFLOP/s); 1 x 8192 1405 -> 546 us (1008); 4099
-// tokens behind 16384 cached 2867 -> 1250 us (990, split); 43 behind 16384
-// 792 -> 85 us (split).
+// Here: what the forms share, and the split form. Whole query tiles:
+// prefill_rows.h; 64 query vectors per wave: prefill_pair.h.
 //
 // SPLIT: when whole query tiles would leave the chip idle, the K/V tiles of
 // all query tiles form one line that up to 256 workgroups cut into equal
@@ -198,30 +195,227 @@ struct Parts {
 // V pass through registers with an exact conversion (half the bytes from
 // memory), one tile ahead.
 //
-// SPLIT runs one workgroup of 8 waves per CU, which reads K/V half as often,
-// with three buffers; the other form two workgroups of 4 waves with two, so
-// that one computes while the other fills its first tile (8 x 1024 tokens:
-// 101 us against 116 us with 8 waves; equal from 4096 rows on).
+// The split form runs one workgroup of 8 waves per CU, which reads K/V half as
+// often, with three buffers; the other form two workgroups of 4 waves with two,
+// so that one computes while the other is between two query tiles.
 constexpr int attn_waves(bool split) { return split ? 8 : 4; }
 
+// (in asm, or each operand that comes from a product is made canonical first)
+FI_DEV float largest(float a, float b, float c) {
+  float v = a;
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(v) : "v"(a), "v"(b), "v"(c));
+#endif
+  return v;
+}
+
+// What a wave does with a tile in LDS: 32 query vectors, one per lane and its
+// half-wave partner.
 //
-// EXT (whole query tiles, bf16): positions instead of context lengths, cache
-// blocks of any size, a sink, a gate, a sliding window that keeps the first
-// keys. Tiles that no row of the workgroup sees are left out.
-template <int D, bool PAGED, bool FP8, bool SPLIT, bool EXT = false>
-__global__ __launch_bounds__(attn_waves(SPLIT) * kWaveSize, 2)
+// The order is pinned: fragments are read four products ahead of their use, V's
+// first ones before the softmax, and a 16-deep step's products go between the
+// exponentials of the next one. (Left to the compiler, each product of V waits
+// for its own read just issued, which two waves per SIMD hide in part: 8 x 1024
+// rows 104 us and 94 so, one of 8192 569 and 536, 4099 behind 16384 1250 and 1190.)
+template <int D>
+struct RowSoftmax {
+  static constexpr int KF = D / 16;      // QK^T 16-deep steps over head dim
+  static constexpr int CB = D / 32;      // 32-dim blocks of the output
+  static constexpr int kRowB = D * 2;    // bytes of a K or V row
+  static constexpr int kChunk = D / 8;   // 16-byte chunks of a row
+  static constexpr int kTileB = kKVTile * kRowB;
+  static constexpr int kRowsPerDma = 1024 / kRowB;
+  static constexpr int kAhead = 4;       // fragments
+  static_assert(D == 128 || D == 64, "swizzles are for these row sizes");
+
+  int k_off, v_off;                      // of fragment 0
+  float c;                               // scale * log2(e)
+  float m_row, l_row;                    // l of this half-wave's keys
+  floatx16 o_acc[CB];
+  short8 v_frag[kAhead];
+
+  // swizzled chunk of a row: K rows are read one chunk per lane over 32
+  // rows, V rows four lanes to 32 bytes over 8 rows
+  FI_DEV static int k_swz(int row) {
+    return D == 128 ? row & 15 : (row >> 1) & 7;
+  }
+  FI_DEV static int v_swz(int row) {
+    return D == 128 ? (row & 3) << 2 : ((row >> 1) & 1) << 2;
+  }
+  FI_DEV RowSoftmax(int lane, float scale) {
+    const int col = lane & 31, hi1 = lane >> 5;
+    k_off = col * kRowB + ((hi1 ^ k_swz(col)) * 16);
+    const int row = 4 * hi1 + ((lane & 15) >> 2);
+    v_off = row * kRowB +
+            (((((lane >> 4) & 1) * 2 + ((lane & 3) >> 1)) ^ v_swz(row)) * 16) +
+            (lane & 1) * 8;
+    c = scale == 0.f ? 1.f : fabsf(scale) * 1.4426950408889634f;
+  }
+  FI_DEV void clear() {
+    m_row = kPNegInf;
+    l_row = 0.f;
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o_acc[cb][r] = 0.f;
+  }
+  FI_DEV static void pin() { __builtin_amdgcn_sched_barrier(0); }
+  // fragment n of K: step n / 2, keys 32 (n & 1) on
+  FI_DEV short8 read_k(const unsigned char* smem, int at, int n) const {
+    return *reinterpret_cast<const short8*>(
+        smem + ((at + k_off) ^ ((n >> 1) * 32)) + (n & 1) * 32 * kRowB);
+  }
+  // of V: step n / CB, dims 32 (n % CB) on
+  FI_DEV short8 read_v(const unsigned char* smem, int at, int n) const {
+    const unsigned char* a =
+        smem + ((at + v_off) ^ (n % CB * 64)) + n / CB * 16 * kRowB;
+    const short4v lo = lds_read_tr4(a), hi = lds_read_tr4(a + 8 * kRowB);
+    return short8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  }
+  // S^T[kv 64 x q 32] of the tile whose K and V begin at k_at and v_at
+  FI_DEV void scores(const unsigned char* smem, int k_at, int v_at,
+                     const short8 (&b_q)[KF], floatx16 (&s_acc)[2]) {
+    short8 k_frag[kAhead];
+#pragma unroll
+    for (int n = 0; n < kAhead; ++n) k_frag[n] = read_k(smem, k_at, n);
+    __builtin_amdgcn_s_setprio(1);
+    pin();
+#pragma unroll
+    for (int n = 0; n < 2 * KF; ++n) {
+      const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f,
+                             0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      s_acc[n & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          k_frag[n % kAhead], b_q[n >> 1], n < 2 ? zero : s_acc[n & 1], 0, 0,
+          0);
+      pin();
+      if (n + kAhead < 2 * KF)
+        k_frag[n % kAhead] = read_k(smem, k_at, n + kAhead);
+      else
+        v_frag[n + kAhead - 2 * KF] =
+            read_v(smem, v_at, n + kAhead - 2 * KF);
+      pin();
+    }
+    __builtin_amdgcn_s_setprio(0);
+  }
+  // the online softmax, and O^T[D x q 32] += V^T[D x 64] P^T[64 x 32]
+  FI_DEV void add(const unsigned char* smem, int v_at,
+                  const floatx16 (&s_acc)[2]) {
+    // (the products' results are not waited for in front of asm)
+    asm volatile("s_nop 15" ::: "memory");
+    pin();
+    float rm = s_acc[0][0];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) rm = largest(rm, s_acc[0][r], s_acc[1][r]);
+    rm = fmaxf(rm, half_swap(rm));
+    if (!__all((rm - m_row) * c <= kDeferThr)) {
+      const float m_new = fmaxf(m_row, rm);
+      const float alpha = __builtin_amdgcn_exp2f((m_row - m_new) * c);
+      m_row = m_new;
+      l_row *= alpha;
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o_acc[cb][r] *= alpha;
+    }
+    const float mc = m_row * c;
+    float rs[4] = {0.f, 0.f, 0.f, 0.f};
+    bf16x8 w[2];                         // this step's weights and the next's
+    auto weights = [&](int kc, int from, int to) {
+#pragma unroll
+      for (int j = from; j < to; ++j) {
+        const float pv = __builtin_amdgcn_exp2f(
+            fmaf(s_acc[kc >> 1][8 * (kc & 1) + j], c, -mc));
+        rs[j & 3] += pv;
+        w[kc & 1].h[j] = f32_to_bf16(pv);
+      }
+    };
+    weights(0, 0, 8);
+    pin();
+#pragma unroll
+    for (int n = 0; n < 4 * CB; ++n) {
+      const int kc = n / CB, cb = n % CB;
+      o_acc[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          v_frag[n % kAhead], __builtin_bit_cast(short8, w[kc & 1]),
+          o_acc[cb], 0, 0, 0);
+      pin();
+      if (n + kAhead < 4 * CB)
+        v_frag[n % kAhead] = read_v(smem, v_at, n + kAhead);
+      if (kc < 3) weights(kc + 1, cb * 8 / CB, (cb + 1) * 8 / CB);
+      pin();
+    }
+    l_row += (rs[0] + rs[1]) + (rs[2] + rs[3]);
+  }
+};
+
+// the other sign's queries, or none for a scale of zero, so that the maximum
+// can be taken over unscaled scores
+FI_DEV float sign_of(float scale) {
+  return scale > 0.f ? 1.f : (scale < 0.f ? -1.f : 0.f);
+}
+template <int KF>
+FI_DEV void turn_queries(short8 (&b_q)[KF], float sgn) {
+  if (sgn == 1.f) return;
+#pragma unroll
+  for (int f = 0; f < KF; ++f) {
+    bf16x8 h = __builtin_bit_cast(bf16x8, b_q[f]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      h.h[j] = f32_to_bf16(bf16_to_f32(h.h[j]) * sgn);
+    b_q[f] = __builtin_bit_cast(short8, h);
+  }
+}
+
+// A wave's 32 rows of results leave through LDS (`mine`, 32 rows that nobody
+// else uses), neighbouring lanes neighbouring dims: from the lanes' own places
+// a store would be 64 pieces of 8 bytes (8 x 1024 rows, 32 heads, 67 MB: 113.0
+// and 110.4 us, 8 of 1376 to 553 rows 144.4 and 134.3). w(cb, r) are dims
+// cb * 32 + crow(r, hi1) on of this lane's row; `rows` of the 32 are there.
+template <int D, class W>
+FI_DEV void put_rows(unsigned char* mine, u16* out, int64_t stride, int rows,
+                     int lane, const W& w) {
+  using R = RowSoftmax<D>;
+  const int col = lane & 31, hi1 = lane >> 5;
+#pragma unroll
+  for (int cb = 0; cb < R::CB; ++cb)
+#pragma unroll
+    for (int r = 0; r < 16; r += 4)
+      *reinterpret_cast<bf16x4*>(
+          mine + col * R::kRowB +
+          (((cb * 4 + r / 4) ^ (col & (R::kChunk - 1))) * 16) + hi1 * 8) =
+          w(cb, r);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  const bool wide = reinterpret_cast<uintptr_t>(out) % 16 == 0;
+  const int ch = lane % R::kChunk;
+  auto store = [&](bool all) {
+#pragma unroll
+    for (int i = 0; i < 32 / R::kRowsPerDma; ++i) {
+      const int r = i * R::kRowsPerDma + lane / R::kChunk;
+      if (!all && r >= rows) continue;
+      const uint4 v = *reinterpret_cast<const uint4*>(
+          mine + r * R::kRowB + ((ch ^ (r & (R::kChunk - 1))) * 16));
+      u16* to = out + r * stride + ch * 8;
+      if (all || wide) {
+        *reinterpret_cast<uint4*>(to) = v;
+      } else {                         // rows off the 16-byte grid
+        reinterpret_cast<uint2*>(to)[0] = make_uint2(v.x, v.y);
+        reinterpret_cast<uint2*>(to)[1] = make_uint2(v.z, v.w);
+      }
+    }
+  };
+  if (wide && rows >= 32) store(true);
+  else store(false);
+}
+
+// The split form.
+template <int D, bool PAGED, bool FP8>
+__global__ __launch_bounds__(attn_waves(true) * kWaveSize, 2)
 void prefill_attn_kernel(const PrefillArgs p) {
-  static_assert(!EXT || (PAGED && !FP8 && !SPLIT));
-  constexpr int kWaves = attn_waves(SPLIT), kBufs = SPLIT ? 3 : 2;
-  constexpr int KF = D / 16;           // QK^T 16-deep steps over head dim
-  constexpr int CB = D / 32;           // 32-dim blocks of the output
-  constexpr int kRowB = D * 2;         // bytes of a K or V row
-  constexpr int kChunk = D / 8;        // 16-byte chunks of a row
-  constexpr int kTileB = kKVTile * kRowB;
-  constexpr int kRowsPerDma = 1024 / kRowB;
+  using R = RowSoftmax<D>;
+  constexpr int kWaves = attn_waves(true), kBufs = 3;
+  constexpr int KF = R::KF, CB = R::CB, kRowB = R::kRowB, kChunk = R::kChunk;
+  constexpr int kTileB = R::kTileB, kRowsPerDma = R::kRowsPerDma;
   constexpr int kWRows = kKVTile / kWaves;   // rows a wave copies
   constexpr int kDma = kWRows / kRowsPerDma;  // DMAs per wave and matrix
-  static_assert(D == 128 || D == 64, "swizzles are for these row sizes");
 
   __shared__ __attribute__((aligned(1024)))
   unsigned char smem[2 * kBufs * kTileB];
@@ -235,81 +429,47 @@ void prefill_attn_kernel(const PrefillArgs p) {
   const int hi1 = lane >> 5;
   const int wph = kWaves / p.hpb;      // waves per query head
 
-  // swizzled chunk of a row: K rows are read one chunk per lane over 32
-  // rows, V rows four lanes to 32 bytes over 8 rows
-  auto k_swz = [](int row) { return D == 128 ? row & 15 : (row >> 1) & 7; };
-  auto v_swz = [](int row) {
-    return D == 128 ? (row & 3) << 2 : ((row >> 1) & 1) << 2;
-  };
-  int k_off[KF], v_off[CB];
-#pragma unroll
-  for (int f = 0; f < KF; ++f)
-    k_off[f] = col * kRowB + (((2 * f + hi1) ^ k_swz(col)) * 16);
-  {
-    const int row = 4 * hi1 + ((lane & 15) >> 2);
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb)
-      v_off[cb] = row * kRowB +
-                  (((cb * 4 + ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1)) ^
-                    v_swz(row)) * 16) + (lane & 1) * 8;
-  }
+  RowSoftmax<D> row(lane, p.scale);
+  const float sgn = sign_of(p.scale);
 
-  // a negative scale turns the queries round, a zero one clears them, so
-  // that the maximum can be taken over unscaled scores
-  const float sgn = p.scale > 0.f ? 1.f : (p.scale < 0.f ? -1.f : 0.f);
-  const float c = p.scale == 0.f
-      ? 1.f : fabsf(p.scale) * 1.4426950408889634f;  // log2(e)
-
-  int64_t pos = 0, pos_end = 1;
-  int slot = 0, hg = 0, qt, from = 0;
-  // SPLIT: (head group, query tile, slot behind the last piece's, 0) of the
+  int hg = 0, qt = 0, from = 0;
+  // (head group, query tile, slot behind the last piece's, 0) of the
   // tile that begins in this part and is cut by its end; -1: none
   int4 cut = make_int4(0, -1, 0, 0);
-  if (SPLIT) {
-    const int u = total_work<PAGED>(p, lane);
-    const int64_t total = static_cast<int64_t>(u) * (p.num_q_heads / p.hpb);
-    slot = split_slot(blockIdx.x, p.slots);
-    const Parts parts(total, p.slots);
-    pos = parts.begin(slot);
-    pos_end = parts.begin(slot + 1);
-    if (pos < pos_end) {
-      hg = static_cast<int>(pos / u);
-      qt = find_tile<PAGED>(p, lane, static_cast<int>(pos - int64_t(hg) * u),
-                            &from);
-    }
-    // the tile at the end: the part itself or a later one finishes it
-    if (pos < pos_end && pos_end < total) {
-      const int h = static_cast<int>(pos_end / u);
-      int within;
-      const int i = find_tile<PAGED>(
-          p, lane, static_cast<int>(pos_end - int64_t(h) * u), &within);
-      if (within > 0 && pos_end - within >= pos) {
-        const int64_t end = pos_end - within + q_tile<PAGED>(p, i).work;
-        cut = make_int4(h, i, slot + 1, 0);
-        while (cut.z < p.slots && parts.begin(cut.z) < end) ++cut.z;
-      }
-    }
-    if (tid == 0) p.cut[slot] = cut;
-  } else {
-    // head groups side by side (neighbouring workgroups go to different
-    // XCDs), the longest query tiles first
-    const int groups = p.num_q_heads / p.hpb;
-    hg = blockIdx.x % groups;
-    qt = p.nq - 1 - blockIdx.x / groups;
+  const int u = total_work<PAGED>(p, lane);
+  const int64_t total = static_cast<int64_t>(u) * (p.num_q_heads / p.hpb);
+  const int slot = split_slot(blockIdx.x, p.slots);
+  const Parts parts(total, p.slots);
+  int64_t pos = parts.begin(slot);
+  const int64_t pos_end = parts.begin(slot + 1);
+  if (pos < pos_end) {
+    hg = static_cast<int>(pos / u);
+    qt = find_tile<PAGED>(p, lane, static_cast<int>(pos - int64_t(hg) * u),
+                          &from);
   }
+  // the tile at the end: the part itself or a later one finishes it
+  if (pos < pos_end && pos_end < total) {
+    const int h = static_cast<int>(pos_end / u);
+    int within;
+    const int i = find_tile<PAGED>(
+        p, lane, static_cast<int>(pos_end - int64_t(h) * u), &within);
+    if (within > 0 && pos_end - within >= pos) {
+      const int64_t end = pos_end - within + q_tile<PAGED>(p, i).work;
+      cut = make_int4(h, i, slot + 1, 0);
+      while (cut.z < p.slots && parts.begin(cut.z) < end) ++cut.z;
+    }
+  }
+  if (tid == 0) p.cut[slot] = cut;
 
   while (pos < pos_end) {
-    const QTile t = uniform_tile(q_tile<PAGED, EXT>(p, qt));
+    const QTile t = uniform_tile(q_tile<PAGED>(p, qt));
     if (t.work == 0) {                 // rows past the sequence's end
-      if (!SPLIT) return;
       if (++qt == p.nq) { qt = 0; ++hg; }
       continue;
     }
     const int ta = from;
-    const int tb = SPLIT
-        ? static_cast<int>(min(static_cast<int64_t>(t.work),
-                               from + (pos_end - pos)))
-        : t.work;
+    const int tb = static_cast<int>(
+        min(static_cast<int64_t>(t.work), from + (pos_end - pos)));
     const int head = hg * p.hpb + wave / wph;
     const int kv_head = hg * p.hpb / (p.num_q_heads / p.num_kv_heads);
     const int ctx_start = t.k_len - t.seq_len;
@@ -353,6 +513,17 @@ void prefill_attn_kernel(const PrefillArgs p) {
         ks = p.k_stride;
         vs = p.v_stride;
       }
+      if (PAGED && limit >= first + kWRows - 1) {  // no row past the end
+        const int r0 = first + lane / kChunk;
+        const u32 ko = r0 * kRowB + ((lane % kChunk) ^ R::k_swz(r0)) * 16;
+        const u32 vo = r0 * kRowB + ((lane % kChunk) ^ R::v_swz(r0)) * 16;
+#pragma unroll
+        for (int i = 0; i < kDma; ++i) {
+          dma_to_lds16(kdst + i * 1024, kb, ko ^ (i * (1024 + 64)));
+          dma_to_lds16(vdst + i * 1024, vb, vo ^ (i * 1024));
+        }
+        return;
+      }
 #pragma unroll
       for (int i = 0; i < kDma; ++i) {
         const int r = i * kRowsPerDma + lane / kChunk;  // row of the wave
@@ -360,52 +531,13 @@ void prefill_attn_kernel(const PrefillArgs p) {
         const int src = min(first + r, limit);
         const u32 ko = static_cast<u32>(
             src * static_cast<int>(ks) * 2 +
-            (((lane % kChunk) ^ k_swz(tr)) * 16));
+            (((lane % kChunk) ^ R::k_swz(tr)) * 16));
         const u32 vo = static_cast<u32>(
             src * static_cast<int>(vs) * 2 +
-            (((lane % kChunk) ^ v_swz(tr)) * 16));
+            (((lane % kChunk) ^ R::v_swz(tr)) * 16));
         dma_to_lds16(kdst + i * 1024, kb, ko);
         dma_to_lds16(vdst + i * 1024, vb, vo);
       }
-    };
-    // EXT, blocks of other sizes than 16: this lane's rows of a tile
-    const bool by_row = EXT && p.block_size != 16;
-    int64_t row_at[EXT ? kDma : 1];
-    auto rows_of = [&](int tile) {
-      const int* bt = p.block_tables + static_cast<int64_t>(t.seq) *
-                                           p.max_blocks;
-#pragma unroll
-      for (int i = 0; i < kDma; ++i) {
-        const int key = min(tile * kKVTile + wave * kWRows +
-                                i * kRowsPerDma + lane / kChunk,
-                            t.k_len - 1);
-        row_at[i] = (static_cast<int64_t>(bt[key / p.block_size]) *
-                         p.num_kv_heads + kv_head) * p.block_size +
-                    key % p.block_size;
-      }
-    };
-    auto stage_rows = [&](int buf) {
-      const u32 kdst = lds0 + buf * kTileB + wave * kWRows * kRowB;
-      const u32 vdst = kdst + kBufs * kTileB;
-#pragma unroll
-      for (int i = 0; i < kDma; ++i) {
-        const int tr = wave * kWRows + i * kRowsPerDma + lane / kChunk;
-        const int64_t at = row_at[i] * kRowB;
-        dma_to_lds16_at(kdst + i * 1024,
-                        static_cast<const unsigned char*>(p.k) + at +
-                            ((lane % kChunk) ^ k_swz(tr)) * 16);
-        dma_to_lds16_at(vdst + i * 1024,
-                        static_cast<const unsigned char*>(p.v) + at +
-                            ((lane % kChunk) ^ v_swz(tr)) * 16);
-      }
-    };
-    // tiles between the kept first keys and the window of the first row
-    const int skip_lo = EXT ? ceil_div(p.keep_first, kKVTile) : 0;
-    const int skip_hi = EXT && p.window > 0
-        ? max(ctx_start + t.row0 - p.window + 1, 0) / kKVTile : 0;
-    auto next_tile = [&](int tile) {
-      const int n = tile + 1;
-      return EXT && n >= skip_lo && n < skip_hi ? skip_hi : n;
     };
     // fp8: a thread owns 16 dims of one row of K and of V
     constexpr int kParts = D / 16;
@@ -448,34 +580,21 @@ void prefill_attn_kernel(const PrefillArgs p) {
 #pragma unroll
       for (int i = 0; i < kSteps; ++i) {
         const int r = f_row0 + i * kStep;
-        put(smem + buf * kTileB, k_raw[i], r, k_swz(r));
-        put(smem + (kBufs + buf) * kTileB, v_raw[i], r, v_swz(r));
+        put(smem + buf * kTileB, k_raw[i], r, R::k_swz(r));
+        put(smem + (kBufs + buf) * kTileB, v_raw[i], r, R::v_swz(r));
       }
     };
 
     // the previous query tile's LDS reads are over in every wave
-    if (SPLIT) __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_s_barrier();
     int blk = 0;
-    const int first_tile =
-        EXT && skip_lo == 0 && skip_hi > 0 ? skip_hi : ta;
     if (FP8) {
       load_fp8(ta);
       write_fp8(0);
       if (ta + 1 < tb) load_fp8(ta + 1);
-    } else if (EXT) {
-      const int n = next_tile(first_tile);
-      if (by_row) {
-        rows_of(first_tile);
-        stage_rows(0);
-        rows_of(n);
-      } else {
-        stage_dma(first_tile, block_of(first_tile), 0);
-        blk = block_of(n);
-      }
     } else {
       stage_dma(ta, PAGED ? block_of(ta) : 0, 0);
-      if (kBufs == 3 && ta + 1 < tb)
-        stage_dma(ta + 1, PAGED ? block_of(ta + 1) : 0, 1);
+      if (ta + 1 < tb) stage_dma(ta + 1, PAGED ? block_of(ta + 1) : 0, 1);
       if (PAGED) blk = block_of(ta + kBufs - 1);
     }
 
@@ -487,38 +606,25 @@ void prefill_attn_kernel(const PrefillArgs p) {
       const u16* qrow = p.q + (t.seq_start + qr) * p.q_stride +
                         static_cast<int64_t>(head) * D;
 #pragma unroll
-      for (int f = 0; f < KF; ++f) {
+      for (int f = 0; f < KF; ++f)
         b_q[f] = *reinterpret_cast<const short8*>(qrow + f * 16 + hi1 * 8);
-        if (sgn != 1.f) {
-          bf16x8 h = __builtin_bit_cast(bf16x8, b_q[f]);
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            h.h[j] = f32_to_bf16(bf16_to_f32(h.h[j]) * sgn);
-          b_q[f] = __builtin_bit_cast(short8, h);
-        }
-      }
+      turn_queries(b_q, sgn);
       // arrived here, not at their first use: that is inside the loop,
       // where the wait would take in the DMAs of every tile
 #pragma unroll
       for (int f = 0; f < KF; ++f) asm volatile("" : "+v"(b_q[f]));
     }
 
-    float m_row = kPNegInf, l_row = 0.f;   // l of this half-wave's keys
-    floatx16 o_acc[CB];
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) o_acc[cb][r] = 0.f;
-
+    row.clear();
     const int my_q_max = ctx_start + min(row0 + 32, t.seq_len) - 1;
     const int q_pos = ctx_start + row0 + col;
     int buf = 0;
-    for (int tile = first_tile; tile < tb; tile = next_tile(tile)) {
+    for (int tile = ta; tile < tb; ++tile) {
       const int kv0 = tile * kKVTile;
       // this tile has landed (this wave's part; the barrier covers the
       // others'), and nobody reads the buffer that is filled next
       if (!FP8) {
-        if (kBufs == 3 && tile + 1 < tb)
+        if (tile + 1 < tb)
           asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kDma) : "memory");
         else
           asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -529,51 +635,15 @@ void prefill_attn_kernel(const PrefillArgs p) {
       if (FP8) {
         if (tile + 1 < tb) write_fp8(buf1);
         if (tile + 2 < tb) load_fp8(tile + 2);
-      } else if (EXT) {
-        const int n = next_tile(tile);
-        if (n < tb) {
-          if (by_row) {
-            stage_rows(buf1);
-            rows_of(next_tile(n));
-          } else {
-            stage_dma(n, blk, buf1);
-            blk = block_of(next_tile(n));
-          }
-        }
       } else if (tile + kBufs - 1 < tb) {
-        stage_dma(tile + kBufs - 1, blk,
-                  kBufs == 2 ? buf1 : (buf1 == kBufs - 1 ? 0 : buf1 + 1));
+        stage_dma(tile + kBufs - 1, blk, buf1 == kBufs - 1 ? 0 : buf1 + 1);
         if (PAGED) blk = block_of(tile + kBufs);
       }
 
-      // outside the window of every row of the wave
-      const bool behind = EXT && p.window > 0 && kv0 >= p.keep_first &&
-                          kv0 + kKVTile <= ctx_start + row0 - p.window + 1;
-      if (active && kv0 <= my_q_max && !behind) {
-        const unsigned char* kbase = smem + buf * kTileB;
-        const unsigned char* vbase = smem + (kBufs + buf) * kTileB;
-        // ---- S^T[kv 64 x q 32] ----
+      if (active && kv0 <= my_q_max) {
         floatx16 s_acc[2];
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int f = 0; f < KF; ++f)
-#pragma unroll
-          for (int b = 0; b < 2; ++b) {
-            const short8 a_k = *reinterpret_cast<const short8*>(
-                kbase + k_off[f] + b * 32 * kRowB);
-            if (f == 0) {
-              const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f,
-                                     0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-              s_acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                  a_k, b_q[f], zero, 0, 0, 0);
-            } else {
-              s_acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                  a_k, b_q[f], s_acc[b], 0, 0, 0);
-            }
-          }
-        __builtin_amdgcn_s_setprio(0);
-
-        // ---- online softmax; only tiles at the diagonal or the end mask
+        row.scores(smem, buf * kTileB, (kBufs + buf) * kTileB, b_q, s_acc);
+        // only tiles at the diagonal or the end mask
         if (kv0 + kKVTile - 1 > ctx_start + row0) {
 #pragma unroll
           for (int b = 0; b < 2; ++b)
@@ -582,114 +652,33 @@ void prefill_attn_kernel(const PrefillArgs p) {
               if (kv0 + 32 * b + crow(r, hi1) > q_pos)
                 s_acc[b][r] = -INFINITY;
         }
-        if (EXT && p.window > 0 && kv0 + kKVTile > p.keep_first &&
-            my_q_max - kv0 >= p.window) {
-#pragma unroll
-          for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              const int key = kv0 + 32 * b + crow(r, hi1);
-              if (q_pos - key >= p.window && key >= p.keep_first)
-                s_acc[b][r] = -INFINITY;
-            }
-        }
-        float rm = fmaxf(s_acc[0][0], s_acc[1][0]);
-#pragma unroll
-        for (int r = 1; r < 16; ++r)
-          rm = fmaxf(rm, fmaxf(s_acc[0][r], s_acc[1][r]));
-        rm = fmaxf(rm, half_swap(rm));
-        if (!__all((rm - m_row) * c <= kDeferThr)) {
-          const float m_new = fmaxf(m_row, rm);
-          const float alpha = __builtin_amdgcn_exp2f((m_row - m_new) * c);
-          m_row = m_new;
-          l_row *= alpha;
-#pragma unroll
-          for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) o_acc[cb][r] *= alpha;
-        }
-        const float mc = m_row * c;
-        float rs[4] = {0.f, 0.f, 0.f, 0.f};
-        short8 b_p[4];
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            bf16x8 w;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-              const float pv = __builtin_amdgcn_exp2f(
-                  fmaf(s_acc[b][8 * h + j], c, -mc));
-              rs[j & 3] += pv;
-              w.h[j] = f32_to_bf16(pv);
-            }
-            b_p[2 * b + h] = __builtin_bit_cast(short8, w);
-          }
-        l_row += (rs[0] + rs[1]) + (rs[2] + rs[3]);
-
-        // ---- O^T[D x q 32] += V^T[D x 64] P^T[64 x 32] ----
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int kc = 0; kc < 4; ++kc)
-#pragma unroll
-          for (int cb = 0; cb < CB; ++cb) {
-            const unsigned char* a = vbase + v_off[cb] + kc * 16 * kRowB;
-            const short4v lo = lds_read_tr4(a);
-            const short4v hi = lds_read_tr4(a + 8 * kRowB);
-            const short8 a_v = {lo[0], lo[1], lo[2], lo[3],
-                                hi[0], hi[1], hi[2], hi[3]};
-            o_acc[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                a_v, b_p[kc], o_acc[cb], 0, 0, 0);
-          }
-        __builtin_amdgcn_s_setprio(0);
+        row.add(smem, (kBufs + buf) * kTileB, s_acc);
       }
       buf = buf1;
     }
 
     // ---- epilogue ----
-    l_row += half_swap(l_row);
-    const bool whole = !SPLIT || (ta == 0 && tb == t.work);
-    if (whole) {
-      if (active && row0 + col < t.seq_len) {
-        float inv = l_row > 0.f ? 1.f / l_row : 0.f;
-        const u16* gp = nullptr;
-        if (EXT) {
-          const int64_t row = t.seq_start + row0 + col;
-          if (p.sink != nullptr) {
-            // in the domain of whichever is larger
-            const float sk = p.sink[head] * 1.4426950408889634f;
-            const float mc = m_row * c, top = fmaxf(mc, sk);
-            const float a = __builtin_amdgcn_exp2f(mc - top);
-            inv = a / (l_row * a + __builtin_amdgcn_exp2f(sk - top));
-          }
-          if (p.gate != nullptr) {
-            gp = p.gate + row * p.g_stride;
-            if (p.gate_elem) {
-              gp += static_cast<int64_t>(head) * D;
-            } else {
-              inv *= 1.f / (1.f + expf(-bf16_to_f32(gp[head])));
-              gp = nullptr;
-            }
-          }
-        }
-        u16* orow = p.out + (static_cast<int64_t>(t.seq_start + row0 + col) *
-                                 p.num_q_heads + head) * D;
+    row.l_row += half_swap(row.l_row);
+    if (ta == 0 && tb == t.work) {
+      // turned over in the buffers that nobody reads or fills any more
+      constexpr int kHalves = kTileB / (32 * kRowB);   // waves per buffer
+      const int free_buf = (buf + wave / kHalves % (kBufs - 1)) % kBufs;
+      unsigned char* mine =
+          smem + (wave / kHalves / (kBufs - 1) * kBufs + free_buf) * kTileB +
+          wave % kHalves * 32 * kRowB;
+      const float inv = row.l_row > 0.f ? 1.f / row.l_row : 0.f;
+      if (active)
+        put_rows<D>(mine,
+                    p.out + (static_cast<int64_t>(t.seq_start + row0) *
+                                 p.num_q_heads + head) * D,
+                    static_cast<int64_t>(p.num_q_heads) * D,
+                    t.seq_len - row0, lane, [&](int cb, int r) {
+                      bf16x4 w;
 #pragma unroll
-        for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-          for (int r = 0; r < 16; r += 4) {
-            bf16x4 w;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              float v = o_acc[cb][r + j] * inv;
-              if (EXT && gp != nullptr)
-                v *= 1.f / (1.f + expf(-bf16_to_f32(
-                                      gp[cb * 32 + crow(r, hi1) + j])));
-              w.h[j] = f32_to_bf16(v);
-            }
-            *reinterpret_cast<bf16x4*>(orow + cb * 32 + crow(r, hi1)) = w;
-          }
-      }
+                      for (int j = 0; j < 4; ++j)
+                        w.h[j] = f32_to_bf16(row.o_acc[cb][r + j] * inv);
+                      return w;
+                    });
     } else {
       const int piece = slot * 2 + (ta > 0 ? 0 : 1);
       float* o = p.piece_o + (static_cast<int64_t>(piece) * kWaves + wave) *
@@ -697,12 +686,11 @@ void prefill_attn_kernel(const PrefillArgs p) {
 #pragma unroll
       for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) o[(cb * 16 + r) * 64] = o_acc[cb][r];
+        for (int r = 0; r < 16; ++r) o[(cb * 16 + r) * 64] = row.o_acc[cb][r];
       float2* ml = reinterpret_cast<float2*>(p.piece_ml) +
                    (static_cast<int64_t>(piece) * kWaves + wave) * 64 + lane;
-      *ml = make_float2(m_row, l_row);
+      *ml = make_float2(row.m_row, row.l_row);
     }
-    if (!SPLIT) return;
     pos += tb - ta;
     from = 0;
     if (++qt == p.nq) { qt = 0; ++hg; }

@@ -29,7 +29,7 @@
 
 #include <type_traits>
 
-#include "prefill_kernel.h"
+#include "prefill_rows.h"
 #include "seqmix.h"
 
 namespace fi {
@@ -892,12 +892,13 @@ bool launch_equal_sizes(u16* out, const u16* q, const u16* k_cache,
   a.block_size = block_size;
   a.window = window;
   a.keep_first = keep_first;
-  const dim3 grid(H / a.hpb * a.nq), block(attn_waves(false) * kWaveSize);
+  const dim3 grid(rows_grid(static_cast<int64_t>(H / a.hpb) * a.nq, DK));
+  const dim3 block(kRowsWaves * kWaveSize);
   if (DK == 128)
-    hipLaunchKernelGGL((prefill_attn_kernel<128, true, false, false, true>),
+    hipLaunchKernelGGL((prefill_rows_kernel<128, true, false, true>),
                        grid, block, 0, s, a);
   else
-    hipLaunchKernelGGL((prefill_attn_kernel<64, true, false, false, true>),
+    hipLaunchKernelGGL((prefill_rows_kernel<64, true, false, true>),
                        grid, block, 0, s, a);
   return true;
 }

@@ -6,6 +6,7 @@ ops/reference.py on random inputs.
 """
 
 import math
+import random
 
 import pytest
 import torch
@@ -619,6 +620,85 @@ def test_prefill_attention_long_parts(hq, hk, scale_by):
             err = (out[at:at + n, h].double() - want).abs()
             assert (err <= 2.4e-2).all(), (i, h, err.max())
         at += n
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("hq,hk,head_dim,seqs,longest", [
+    (32, 8, 128, 9, 700),     # a few query tiles each, of very uneven work
+    (8, 2, 64, 60, 150),      # lists that end with none
+    (24, 8, 128, 150, 70),    # three heads a group: one per workgroup
+    (32, 8, 128, 1040, 9),    # more query tiles than are put in order
+    (64, 64, 64, 420, 3),     # more than a list holds: more workgroups
+])
+def test_prefill_attention_lists_of_query_tiles(hq, hk, head_dim, seqs,
+                                                longest, fp8):
+    """Workgroups that take several query tiles one after the other, against
+    launches so small that each takes one: the same bits for every row, rows of
+    other requests and behind a context's end never read."""
+    rng = random.Random(seqs)
+    g = torch.Generator().manual_seed(seqs)
+    new = [rng.randint(1, longest) for _ in range(seqs)]
+    past = [rng.choice([0, 0, 5, 40]) for _ in range(seqs)]
+    ctx = [a + b for a, b in zip(new, past)]
+    need = [-(-c // 16) for c in ctx]
+    perm = (torch.randperm(sum(need), generator=g) + 1).int()
+    bt = torch.zeros(seqs, max(need), dtype=torch.int32)
+    for i, row in enumerate(perm.split(need)):
+        bt[i, :need[i]] = row
+    q = torch.randn(sum(new), hq, head_dim, generator=g).bfloat16().to(DEV)
+    kc, vc = (torch.randn(sum(need) + 1, hk, 16, head_dim,
+                          generator=g).bfloat16().to(DEV) for _ in range(2))
+    if fp8:
+        kc, vc = _fp8_cache(kc), _fp8_cache(vc)
+    else:
+        for i, c in enumerate(ctx):
+            if c % 16:
+                for t in (kc, vc):
+                    t[int(bt[i, need[i] - 1]), :, c % 16:] = float("nan")
+    bt = bt.to(DEV)
+
+    def run(i, j):
+        first = sum(new[:i])
+        rows = q[first:first + sum(new[i:j])]
+        cu = torch.tensor([0] + list(torch.tensor(new[i:j]).cumsum(0)),
+                          dtype=torch.int32, device=DEV)
+        lens = torch.tensor(ctx[i:j], dtype=torch.int32, device=DEV)
+        table = ops.build_prefill_tiles(new[i:j], device=DEV, rows=256)
+        plan = ops._C.prefill_plan(table[0].shape[0], 256, hq, hk, len(rows),
+                                   max(need) * 16, head_dim, True, fp8)
+        if plan[0]:                      # parts round elsewhere
+            return None
+        return ops.prefill_attention_paged(rows, kc, vc, bt[i:j], cu, lens,
+                                           head_dim ** -0.5, *table, 256)
+
+    out = run(0, seqs)
+    assert out is not None and torch.isfinite(out).all()
+    # 256 rows of a group of one head are two query tiles or more, and 512
+    # query tiles over all heads go one to a workgroup
+    per = 256 * hq // 128
+    step = max(1, 512 // per) if longest <= 256 else 1
+    picks = range(0, seqs, step) if seqs <= 150 else \
+        rng.sample(range(seqs - step), 40)
+    tested = 0
+    for i in picks:
+        want = run(i, min(i + step, seqs))
+        if want is not None:
+            at = sum(new[:i])
+            assert torch.equal(out[at:at + len(want)], want), i
+            tested += 1
+    assert tested > 0
+    i = max(range(seqs), key=lambda n: new[n])
+    at = sum(new[:i])
+    b = bt[i, :need[i]].long()
+    k, v = (t[b].float().permute(1, 0, 2, 3).reshape(hk, -1, head_dim)
+            [:, :ctx[i]].repeat_interleave(hq // hk, 0).cpu() for t in (kc, vc))
+    s = q[at:at + new[i]].float().cpu().transpose(0, 1) @ k.transpose(1, 2)
+    hide = torch.arange(ctx[i]) > torch.arange(past[i], ctx[i])[:, None]
+    want = torch.softmax((s * head_dim ** -0.5).masked_fill(hide, -math.inf),
+                         -1) @ v
+    # P and the output are rounded to bf16 (2^-9 each), |v| stays below 5
+    assert_close_bf16(out[at:at + new[i]].cpu(),
+                      want.transpose(0, 1).bfloat16(), atol=2e-2, rtol=2e-2)
 
 
 @pytest.mark.parametrize("hq,hk", [(2, 2), (3, 1)])
