@@ -212,11 +212,11 @@ FI_DEV float largest(float a, float b, float c) {
 // What a wave does with a tile in LDS: 32 query vectors, one per lane and its
 // half-wave partner.
 //
-// The order is pinned: fragments are read four products ahead of their use, V's
-// first ones before the softmax, and a 16-deep step's products go between the
-// exponentials of the next one. (Left to the compiler, each product of V waits
-// for its own read just issued, which two waves per SIMD hide in part: 8 x 1024
-// rows 104 us and 94 so, one of 8192 569 and 536, 4099 behind 16384 1250 and 1190.)
+// The order is pinned: fragments are read four products ahead of their use (two
+// for heads of 64), V's first ones before the softmax, and a 16-deep step's
+// products go between the exponentials and sums of the next one. (Left to the
+// compiler, each product of V waits for its own read just issued, which two waves
+// per SIMD hide in part: 8 x 1024 rows 104 us and 94 so, one of 8192 569 and 536.)
 template <int D>
 struct RowSoftmax {
   static constexpr int KF = D / 16;      // QK^T 16-deep steps over head dim
@@ -225,7 +225,10 @@ struct RowSoftmax {
   static constexpr int kChunk = D / 8;   // 16-byte chunks of a row
   static constexpr int kTileB = kKVTile * kRowB;
   static constexpr int kRowsPerDma = 1024 / kRowB;
-  static constexpr int kAhead = 4;       // fragments
+  static constexpr int kAhead = D == 64 ? 2 : 4;   // fragments
+  // places that each tile or query tile needs again are made again, not kept:
+  // three or four workgroups share a CU's registers
+  static constexpr bool kFew = D == 64;
   static_assert(D == 128 || D == 64, "swizzles are for these row sizes");
 
   int k_off, v_off;                      // of fragment 0
@@ -249,7 +252,9 @@ struct RowSoftmax {
     v_off = row * kRowB +
             (((((lane >> 4) & 1) * 2 + ((lane & 3) >> 1)) ^ v_swz(row)) * 16) +
             (lane & 1) * 8;
-    c = scale == 0.f ? 1.f : fabsf(scale) * 1.4426950408889634f;
+    // (uniform: in a scalar register)
+    c = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(
+        scale == 0.f ? 1.f : fabsf(scale) * 1.4426950408889634f)));
   }
   FI_DEV void clear() {
     m_row = kPNegInf;
@@ -328,6 +333,9 @@ struct RowSoftmax {
         rs[j & 3] += pv;
         w[kc & 1].h[j] = f32_to_bf16(pv);
       }
+      // (here, or all weights would be kept for sums at the tile's end)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(rs[i]));
     };
     weights(0, 0, 8);
     pin();
@@ -365,41 +373,46 @@ FI_DEV void turn_queries(short8 (&b_q)[KF], float sgn) {
   }
 }
 
-// A wave's 32 rows of results leave through LDS (`mine`, 32 rows that nobody
+// A wave's 32 rows of results leave through LDS (32 rows from `at` on that nobody
 // else uses), neighbouring lanes neighbouring dims: from the lanes' own places
 // a store would be 64 pieces of 8 bytes (8 x 1024 rows, 32 heads, 67 MB: 113.0
 // and 110.4 us, 8 of 1376 to 553 rows 144.4 and 134.3). w(cb, r) are dims
 // cb * 32 + crow(r, hi1) on of this lane's row; `rows` of the 32 are there.
 template <int D, class W>
-FI_DEV void put_rows(unsigned char* mine, u16* out, int64_t stride, int rows,
-                     int lane, const W& w) {
+FI_DEV void put_rows(unsigned char* smem, int at, u16* out, int64_t stride,
+                     int rows, int lane, const W& w) {
   using R = RowSoftmax<D>;
+  if (R::kFew) asm volatile("" : "+v"(lane));
   const int col = lane & 31, hi1 = lane >> 5;
+  // 16-byte chunk c of row r sits at c ^ r
+  const int put = at + col * R::kRowB + (col & (R::kChunk - 1)) * 16 + hi1 * 8;
 #pragma unroll
   for (int cb = 0; cb < R::CB; ++cb)
 #pragma unroll
     for (int r = 0; r < 16; r += 4)
-      *reinterpret_cast<bf16x4*>(
-          mine + col * R::kRowB +
-          (((cb * 4 + r / 4) ^ (col & (R::kChunk - 1))) * 16) + hi1 * 8) =
+      *reinterpret_cast<bf16x4*>(smem + (put ^ ((cb * 4 + r / 4) * 16))) =
           w(cb, r);
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   const bool wide = reinterpret_cast<uintptr_t>(out) % 16 == 0;
-  const int ch = lane % R::kChunk;
+  const int r0 = lane / R::kChunk, ch = lane % R::kChunk;
+  const int get = at + r0 * R::kRowB + (ch ^ r0) * 16;
+  u16* to = out + r0 * stride + ch * 8;
   auto store = [&](bool all) {
 #pragma unroll
     for (int i = 0; i < 32 / R::kRowsPerDma; ++i) {
-      const int r = i * R::kRowsPerDma + lane / R::kChunk;
-      if (!all && r >= rows) continue;
-      const uint4 v = *reinterpret_cast<const uint4*>(
-          mine + r * R::kRowB + ((ch ^ (r & (R::kChunk - 1))) * 16));
-      u16* to = out + r * stride + ch * 8;
-      if (all || wide) {
-        *reinterpret_cast<uint4*>(to) = v;
-      } else {                         // rows off the 16-byte grid
-        reinterpret_cast<uint2*>(to)[0] = make_uint2(v.x, v.y);
-        reinterpret_cast<uint2*>(to)[1] = make_uint2(v.z, v.w);
+      const int r = i * R::kRowsPerDma;
+      if (all || r + r0 < rows) {
+        const uint4 v = *reinterpret_cast<const uint4*>(
+            smem + (get ^ (r & (R::kChunk - 1)) * 16) + r * R::kRowB);
+        if (all || wide) {
+          *reinterpret_cast<uint4*>(to) = v;
+        } else {                       // rows off the 16-byte grid
+          reinterpret_cast<uint2*>(to)[0] = make_uint2(v.x, v.y);
+          reinterpret_cast<uint2*>(to)[1] = make_uint2(v.z, v.w);
+        }
       }
+      to += R::kRowsPerDma * stride;
+      if (R::kFew) asm volatile("" : "+v"(to));
     }
   };
   if (wide && rows >= 32) store(true);
@@ -663,12 +676,12 @@ void prefill_attn_kernel(const PrefillArgs p) {
       // turned over in the buffers that nobody reads or fills any more
       constexpr int kHalves = kTileB / (32 * kRowB);   // waves per buffer
       const int free_buf = (buf + wave / kHalves % (kBufs - 1)) % kBufs;
-      unsigned char* mine =
-          smem + (wave / kHalves / (kBufs - 1) * kBufs + free_buf) * kTileB +
+      const int mine =
+          (wave / kHalves / (kBufs - 1) * kBufs + free_buf) * kTileB +
           wave % kHalves * 32 * kRowB;
       const float inv = row.l_row > 0.f ? 1.f / row.l_row : 0.f;
       if (active)
-        put_rows<D>(mine,
+        put_rows<D>(smem, mine,
                     p.out + (static_cast<int64_t>(t.seq_start + row0) *
                                  p.num_q_heads + head) * D,
                     static_cast<int64_t>(p.num_q_heads) * D,

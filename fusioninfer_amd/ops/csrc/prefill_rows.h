@@ -23,6 +23,11 @@
 // heads of 64 66 and 64. A prompt of 1024 alone 30 and 28. Matrix cores are busy 40
 // to 52 % of the time, vector instructions issue for 50, LDS reads for 25.
 //
+// No form keeps registers in scratch memory: a value read back from there waits
+// for the stores and for the next tile's keys in front of it (us with and without:
+// 8 of 1376 to 553 rows, e4m3, 135 and 132; heads of 64, 64 x 128 rows, 33 and 27;
+// the mixers' 4 x 1800 rows, 16 heads of 128 on 16, 85 and 82).
+//
 // EXT (bf16): positions instead of context lengths, cache blocks of any size, a
 // sink, a gate, a sliding window that keeps the first keys. Tiles that no row
 // of the workgroup sees are left out.
@@ -209,10 +214,12 @@ void prefill_rows_kernel(const PrefillArgs p) {
     if (EXT && by_row) {
       const int* bt = p.block_tables + static_cast<int64_t>(ahead.t.seq) *
                                            p.max_blocks;
+      int r0 = lane / kChunk;
+      if (R::kFew) asm volatile("" : "+v"(r0));
 #pragma unroll
       for (int i = 0; i < kDma; ++i) {
         const int key = min(atile * kKVTile + wave * kWRows +
-                                i * kRowsPerDma + lane / kChunk,
+                                i * kRowsPerDma + r0,
                             ahead.t.k_len - 1);
         row_at[i] = (static_cast<int64_t>(bt[key / p.block_size]) *
                          p.num_kv_heads + kv_head_of(ahead)) * p.block_size +
@@ -233,17 +240,20 @@ void prefill_rows_kernel(const PrefillArgs p) {
   auto stage = [&](int buf) {
     const u32 kdst = lds0 + buf * kTileB + wave * kWRows * kRowB;
     const u32 vdst = kdst + kBufs * kTileB;
+    // of a row, where rows are not side by side
+    u32 k_in = k_from, v_in = v_from;
+    int r0 = lane / kChunk;
+    if (R::kFew) asm volatile("" : "+v"(k_in), "+v"(v_in), "+v"(r0));
     if (EXT && by_row) {
 #pragma unroll
       for (int i = 0; i < kDma; ++i) {
-        const int tr = wave * kWRows + i * kRowsPerDma + lane / kChunk;
         const int64_t at = row_at[i] * kRowB;
         dma_to_lds16_at(kdst + i * 1024,
                         static_cast<const unsigned char*>(p.k) + at +
-                            ((lane % kChunk) ^ R::k_swz(tr)) * 16);
+                            ((k_in ^ (i * 64)) & (kRowB - 1)));
         dma_to_lds16_at(vdst + i * 1024,
                         static_cast<const unsigned char*>(p.v) + at +
-                            ((lane % kChunk) ^ R::v_swz(tr)) * 16);
+                            (v_in & (kRowB - 1)));
       }
       return;
     }
@@ -261,15 +271,15 @@ void prefill_rows_kernel(const PrefillArgs p) {
               min(atile * 4 + wave, (ahead.t.k_len - 1) >> 4) * 16;
       ks = vs = D;
     } else {
-      const int r0 = min(atile * kKVTile, ahead.t.k_len - 1);
+      const int row = min(atile * kKVTile, ahead.t.k_len - 1);
       kb = static_cast<const u16*>(p.k) +
-           (ahead.t.seq_start + r0) * p.k_stride +
+           (ahead.t.seq_start + row) * p.k_stride +
            int64_t(kv_head_of(ahead)) * D;
       vb = static_cast<const u16*>(p.v) +
-           (ahead.t.seq_start + r0) * p.v_stride +
+           (ahead.t.seq_start + row) * p.v_stride +
            int64_t(kv_head_of(ahead)) * D;
       first = wave * kWRows;
-      limit = ahead.t.k_len - 1 - r0;
+      limit = ahead.t.k_len - 1 - row;
       ks = p.k_stride;
       vs = p.v_stride;
     }
@@ -283,17 +293,12 @@ void prefill_rows_kernel(const PrefillArgs p) {
     }
 #pragma unroll
     for (int i = 0; i < kDma; ++i) {
-      const int r = i * kRowsPerDma + lane / kChunk;  // row of the wave
-      const int tr = wave * kWRows + r;                    // row of the tile
-      const int src = min(first + r, limit);
+      const int src = min(first + i * kRowsPerDma + r0, limit);
       dma_to_lds16(kdst + i * 1024, kb,
-                   static_cast<u32>(
-                       src * static_cast<int>(ks) * 2 +
-                       (((lane % kChunk) ^ R::k_swz(tr)) * 16)));
+                   src * static_cast<int>(ks) * 2 +
+                       ((k_in ^ (i * 64)) & (kRowB - 1)));
       dma_to_lds16(vdst + i * 1024, vb,
-                   static_cast<u32>(
-                       src * static_cast<int>(vs) * 2 +
-                       (((lane % kChunk) ^ R::v_swz(tr)) * 16)));
+                   src * static_cast<int>(vs) * 2 + (v_in & (kRowB - 1)));
     }
   };
   // fp8: a thread owns 16 dims of one row of K and of V
@@ -404,7 +409,8 @@ void prefill_rows_kernel(const PrefillArgs p) {
     const bool active = row0 < it.t.seq_len;
     const int ctx_start = it.t.k_len - it.t.seq_len;
     const int my_q_max = ctx_start + min(row0 + 32, it.t.seq_len) - 1;
-    const int q_pos = ctx_start + row0 + col;
+    // of this lane's query vector, less what its keys lie further on than crow's
+    const int q_at = ctx_start + row0 + col - 4 * hi1;
     floatx16 s_acc[2];
     bool seen = false;
     int tile = it.first;
@@ -417,7 +423,7 @@ void prefill_rows_kernel(const PrefillArgs p) {
         for (int b = 0; b < 2; ++b)
 #pragma unroll
           for (int r = 0; r < 16; ++r)
-            if (kv0 + 32 * b + crow(r, hi1) > q_pos)
+            if (kv0 + 32 * b + crow(r, 0) > q_at)
               s_acc[b][r] = -INFINITY;
       }
       if (EXT && p.window > 0 && kv0 + kKVTile > p.keep_first &&
@@ -426,8 +432,8 @@ void prefill_rows_kernel(const PrefillArgs p) {
         for (int b = 0; b < 2; ++b)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            const int key = kv0 + 32 * b + crow(r, hi1);
-            if (q_pos - key >= p.window && key >= p.keep_first)
+            const int key = kv0 + 32 * b + crow(r, 0);
+            if (q_at - key >= p.window && key + 4 * hi1 >= p.keep_first)
               s_acc[b][r] = -INFINITY;
           }
       }
@@ -486,6 +492,10 @@ void prefill_rows_kernel(const PrefillArgs p) {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (active) {
+      // (made again, not kept)
+      const int lane = __builtin_amdgcn_mbcnt_hi(
+          ~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+      const int col = lane & 31, hi1 = lane >> 5;
       row.l_row += half_swap(row.l_row);
       float inv = row.l_row > 0.f ? 1.f / row.l_row : 0.f;
       const u16* gp = nullptr;
@@ -512,8 +522,8 @@ void prefill_rows_kernel(const PrefillArgs p) {
       u16* out = p.out + (static_cast<int64_t>(now.t.seq_start + row0) *
                               p.num_q_heads + head) * D;
       put_rows<D>(
-          smem + (wave / 2 * kBufs + buf) * kTileB + wave % 2 * 32 * kRowB,
-          out, static_cast<int64_t>(p.num_q_heads) * D, rows, lane,
+          smem, (wave / 2 * kBufs + buf) * kTileB + wave % 2 * 32 * kRowB, out,
+          static_cast<int64_t>(p.num_q_heads) * D, rows, lane,
           [&](int cb, int r) {
             bf16x4 w;
 #pragma unroll
