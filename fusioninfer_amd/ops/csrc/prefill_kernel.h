@@ -338,6 +338,10 @@ struct RowSoftmax {
       for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(rs[i]));
     };
     weights(0, 0, 8);
+    // (a wave with products in front of one without; us without and with, 32
+    // heads of 128 on 8, e4m3: 4099 rows behind 16384 1281 and 1265, 8 of 1376 to
+    // 553 131 and 126; heads of 64, one of 8192: 312 and 330)
+    if (!kFew) __builtin_amdgcn_s_setprio(1);
     pin();
 #pragma unroll
     for (int n = 0; n < 4 * CB; ++n) {
@@ -351,6 +355,7 @@ struct RowSoftmax {
       if (kc < 3) weights(kc + 1, cb * 8 / CB, (cb + 1) * 8 / CB);
       pin();
     }
+    if (!kFew) __builtin_amdgcn_s_setprio(0);
     l_row += (rs[0] + rs[1]) + (rs[2] + rs[3]);
   }
 };
