@@ -109,9 +109,9 @@ __host__ __device__ __forceinline__ constexpr int ceil_div(int a, int b) {
 
 // How a launch of the prefill attention kernel is laid out: query heads and
 // rows of a workgroup, workgroup row blocks per tile-table entry and in all,
-// and whether K/V ranges are cut into equal parts.
+// whether K/V ranges are cut into equal parts, and the longest context's bound.
 struct PrefillPlan {
-  int waves, hpb, rows, sub, nq, slots;
+  int waves, hpb, rows, sub, nq, slots, longest;
   bool split, pair;
 };
 

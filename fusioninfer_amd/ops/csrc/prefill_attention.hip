@@ -115,6 +115,7 @@ PrefillPlan plan_prefill_attn(int ntiles, int tile_rows, int num_q_heads,
     pl.sub = ceil_div(tile_rows, pl.rows);
     pl.nq = ntiles * pl.sub;
     pl.slots = 0;
+    pl.longest = max_k_len;
     return pl;
   };
   PrefillPlan pl = layout(true);
@@ -151,7 +152,7 @@ void launch_prefill_attn(u16* out, const u16* q, const void* k, const void* v,
                          float scale, bool fp8, const PrefillPlan& pl,
                          float* pieces, hipStream_t stream) {
   const bool paged = block_tables != nullptr;
-  PrefillArgs a;
+  PrefillArgs a = {};
   a.out = out;
   a.q = q;
   a.k = k;
@@ -182,8 +183,6 @@ void launch_prefill_attn(u16* out, const u16* q, const void* k, const void* v,
   a.nq = pl.nq;
   a.scale = scale;
   const dim3 block(pl.waves * kWaveSize);
-  const dim3 grid(rows_grid(static_cast<int64_t>(num_q_heads / pl.hpb) *
-                            pl.nq, head_dim));
 #define FI_PF_LAUNCH(DD, PP, F8)                                              \
   do {                                                                        \
     if (pl.split) {                                                           \
@@ -197,8 +196,7 @@ void launch_prefill_attn(u16* out, const u16* q, const void* k, const void* v,
                          dim3(pl.slots, pl.waves),                            \
                          dim3(DD / 16 * kWaveSize), 0, stream, a);            \
     } else {                                                                  \
-      hipLaunchKernelGGL((prefill_rows_kernel<DD, PP, F8>), grid, block, 0,   \
-                         stream, a);                                          \
+      launch_rows<DD, PP, F8, false>(a, pl.longest, stream);                  \
     }                                                                         \
   } while (0)
   if (fp8 && !paged) abort();  // fp8 KV is a cache format; dense is bf16

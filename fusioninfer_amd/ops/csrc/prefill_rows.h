@@ -1,32 +1,38 @@
-// Prefill attention by whole query tiles: two workgroups of four waves on a
-// CU, each with a list of query tiles that it goes through without a pause.
+// Prefill attention by whole query tiles: workgroups of four waves, two of them
+// on a CU (three or four for heads of 64), each with one query tile, or with a
+// list of them that it goes through without a pause (LISTS).
 //
 // One workgroup per query tile, as many as there are tiles, spends 7 to 10 us
 // of each on other things than products: its start, the tile table and what
 // that leads to one after the other, the first keys' and the queries' way, the
 // results' way out; a prompt of a thousand tokens has 8 key tiles of 2 us for
-// a query tile on average. Here at most 512 workgroups run, and the next query
-// tile's first keys are requested while the last ones of this tile are worked
-// on, its queries while those are weighed.
+// a query tile on average. By lists only as many workgroups run as fit on the
+// chip (rows_grid; more where a list would be longer than kRowsList), and the
+// next query tile's first keys are requested while the last ones of this tile
+// are worked on, its queries while those are weighed.
 //
 // Who takes which tile is settled in advance: query tiles in order of their
 // work (key tiles), the longest first, dealt to the workgroups of an XCD to and
 // fro. Every workgroup counts the tiles of each work into LDS and finds its own
 // from that (the order of equal ones is their order in the table), so that no
-// counter outlives the launch. A query tile's products and their order are the
+// counter outlives the launch. Of more than kRowsSort query tiles the order is
+// the table's from its end. A query tile's products and their order are the
 // same whoever takes it.
 //
-// One workgroup per query tile and this, us on one card, 32 query heads, 8 K/V
-// heads of 128 (TFLOP/s of the visible pairs): 8 x 1024 rows 116 and 97 (711), 8 of
-// 1376 to 553 rows 144 and 117 (732), 4 x 2048 188 and 173, 64 x 128 51 and 38, one
-// of 8192 588 and 566 (971); e4m3 8 x 1024 129 and 114; 16 query heads 70 and 52;
-// heads of 64 66 and 64. A prompt of 1024 alone 30 and 28. Matrix cores are busy 40
-// to 52 % of the time, vector instructions issue for 50, LDS reads for 25.
+// One workgroup per query tile as it was, without rows stored whole and fragments
+// read ahead, and this, us on one card, 32 query heads, 8 K/V heads of 128
+// (TFLOP/s of the visible pairs): 8 x 1024 rows 115 and 94 (730), 8 of 1376 to 553
+// rows 141 and 114 (750), 4 x 2048 183 and 163, 64 x 128 50 and 37, 200 x 100 145
+// and 105, one of 8192 574 and 536 (1026); e4m3 8 x 1024 129 and 105; 16 query heads
+// 71 and 52. A prompt of 1024 alone 30 and 27. Heads of 64: 8 x 1024 66 and 59, 16
+// on 16 46 and 35, one of 8192 334 and 312. Of the mixers, 4 x 1800 rows, 16 heads
+// of 128 on 16: 96 and 75, of 64 64 and 50; 8 x 1024, 32 on 8, behind a window of
+// 512 99 and 92. Matrix cores are busy 40 to 52 % of the time, vector
+// instructions issue for 50, LDS reads for 25.
 //
 // No form keeps registers in scratch memory: a value read back from there waits
 // for the stores and for the next tile's keys in front of it (us with and without:
-// 8 of 1376 to 553 rows, e4m3, 135 and 132; heads of 64, 64 x 128 rows, 33 and 27;
-// the mixers' 4 x 1800 rows, 16 heads of 128 on 16, 85 and 82).
+// 8 of 1376 to 553 rows, e4m3, 136 and 131; heads of 64, 64 x 128 rows, 33 and 23).
 //
 // EXT (bf16): positions instead of context lengths, cache blocks of any size, a
 // sink, a gate, a sliding window that keeps the first keys. Tiles that no row
@@ -41,24 +47,53 @@ namespace fi {
 
 constexpr int kRowsWaves = attn_waves(false);
 // workgroups of a CU, by their registers, and in all
-constexpr int rows_each(int head_dim) { return head_dim == 64 ? 3 : 2; }
-constexpr int rows_groups(int head_dim) { return 256 * rows_each(head_dim); }
+constexpr int rows_each(int head_dim, bool lists) {
+  return head_dim == 64 ? (lists ? 3 : 4) : 2;
+}
+constexpr int rows_groups(int head_dim) {
+  return 256 * rows_each(head_dim, true);
+}
 constexpr int kRowsList = kWaveSize;   // query tiles of one, at most
 constexpr int kRowsSort = 8192;        // query tiles that are put in order
 
-// workgroups of a launch with `items` query tiles of all head groups
-inline int rows_grid(int64_t items, int head_dim) {
+// Whether a launch goes by lists. A list's start takes 4 to 6 us more (every
+// query tile's lengths, their order), and at its end some CUs have nothing left
+// while others still go through theirs, up to a tenth of the work of two or
+// three rounds; what it saves is a start and an end per further query tile.
+//  * One round: there is nothing to save.
+//  * A window: tiles are short and alike, and CUs that take them as they come
+//    end together (us, lists and one each: 2 x 4000, 32 heads of 128 on 8, 123 and
+//    111, 16 on 4 66 and 61; 8 x 1024 95 and 95).
+//  * Heads of 64, where a tile takes half as long and more of them run at once:
+//    for up to three rounds of contexts that are neither short nor long (8 x 1024,
+//    16 heads on 16, 35 and 42, 32 on 8 59 and 60, 64 on 8 114 and 101; 24 x 256 25
+//    and 23; one of 8192 340 and 308; 4 x 1800, mixers, 50 and 61).
+//  * Otherwise always (8 x 1024 94 and 102, 400 x 40 98 and 164, one of 8192 530
+//    and 535), but for short contexts of one query tile per entry of the tile
+//    table, where there are no empty ones to skip (mixers, 16 heads on 16: 60 x 64
+//    22 and 20, 40 x 128 27 and 23, 16 x 512 41 and 47).
+// sub: query tiles per entry; longest: no context is longer.
+inline bool rows_by_lists(int64_t items, int head_dim, int sub, int window,
+                          int64_t longest) {
   const int groups = rows_groups(head_dim);
-  if (items <= groups) return static_cast<int>(items);
-  constexpr int64_t kRound = 8 * kRowsList;
-  return static_cast<int>(
-      std::max<int64_t>(groups, (items + kRound - 1) / kRound * 8));
+  if (items <= groups || window > 0) return false;
+  if (head_dim == 64)
+    return items <= 3 * groups && longest >= 512 && longest <= 4096;
+  return sub > 1 || longest >= 512;
 }
 
-template <int D, bool PAGED, bool FP8, bool EXT = false>
-__global__ __launch_bounds__(kRowsWaves * kWaveSize, rows_each(D))
+// workgroups of a launch by lists with `items` query tiles of all head groups
+inline int rows_grid(int64_t items, int head_dim) {
+  constexpr int64_t kRound = 8 * kRowsList;
+  return static_cast<int>(std::max<int64_t>(
+      rows_groups(head_dim), (items + kRound - 1) / kRound * 8));
+}
+
+template <int D, bool PAGED, bool FP8, bool EXT, bool LISTS>
+__global__ __launch_bounds__(kRowsWaves * kWaveSize, rows_each(D, LISTS))
 void prefill_rows_kernel(const PrefillArgs p) {
   static_assert(!EXT || (PAGED && !FP8));
+  constexpr bool kWindow = EXT && !LISTS;   // launches with one
   using R = RowSoftmax<D>;
   constexpr int kWaves = kRowsWaves, kBufs = 2;
   constexpr int KF = R::KF, kRowB = R::kRowB, kChunk = R::kChunk;
@@ -84,123 +119,129 @@ void prefill_rows_kernel(const PrefillArgs p) {
   // ---- this workgroup's query tiles: its r-th is place place_of(r) in the
   // order, head groups side by side (neighbouring workgroups go to different
   // XCDs), the longest first
-  const bool one = p.nq * groups <= rows_groups(D);   // query tile each
-  const int per = gridDim.x / 8;       // workgroups of an XCD
   auto place_of = [&](int r) {
-    const int b = blockIdx.x, j = b / 8;
-    return one ? b : 8 * (r * per + (r & 1 ? per - 1 - j : j)) + (b & 7);
+    const int b = blockIdx.x, j = b / 8, per = gridDim.x / 8;
+    return LISTS ? 8 * (r * per + (r & 1 ? per - 1 - j : j)) + (b & 7) : b;
   };
-  const int my_place = place_of(lane);
-  int my_qt = -1;
-  if (one) {
-    if (lane == 0) my_qt = p.nq - 1 - my_place / groups;
-  } else if (p.nq > kRowsSort) {
-    if (my_place < p.nq * groups) my_qt = p.nq - 1 - my_place / groups;
+  QTile mine = {};                     // lane r: of the r-th
+  unsigned long long to_do = 1;
+  if (!LISTS) {
+    mine = uniform_tile(q_tile<PAGED, EXT>(p, p.nq - 1 - place_of(0) / groups));
+    if (mine.work == 0) return;
   } else {
-    // bucket b of works at (b % 32) * 64 + b / 32, so that lane b / 32 reads
-    // its 32 without conflicts; the last bucket has all longer ones too
-    constexpr int kBuckets = 2048;
-    int* count = reinterpret_cast<int*>(smem);
-    u16* works = reinterpret_cast<u16*>(smem + kBuckets * 4);
-    int* found = reinterpret_cast<int*>(smem + kBuckets * 4 + kRowsSort * 2);
-    static_assert(kBuckets * 4 + kRowsSort * 2 + kRowsList * 4 <=
-                  2 * kBufs * kTileB);
-    constexpr int kThreads = kWaves * kWaveSize;
-    for (int i = tid; i < kBuckets; i += kThreads) count[i] = 0;
-    __syncthreads();
-    for (int i = tid; i < p.nq; i += kThreads) {
-      const int b = min(q_tile<PAGED, EXT>(p, i).work, kBuckets - 1);
-      works[i] = b;
-      if (b > 0) atomicAdd(&count[b % 32 * 64 + b / 32], 1);
-    }
-    __syncthreads();
-    // lane l: buckets 2047 - 32 l down to 2016 - 32 l
-    const int line = 63 - lane;
-    int own = 0;
-    for (int k = 0; k < 32; ++k) own += count[k * 64 + line];
-    int incl = own;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int o = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += o;
-    }
-    const int all = __shfl(incl, 63, 64);
-    if (tid < kRowsList) found[tid] = -1;
-    __syncthreads();
-    for (int r = wave; r < kRowsList; r += kWaves) {
-      int rank = place_of(r) / groups;
-      if (rank >= all) break;          // places ascend
-      const int l = __builtin_ctzll(__ballot(incl > rank));
-      rank -= __shfl(incl, l, 64) - __shfl(own, l, 64);
-      // the bucket: lane k has the k-th from the line's top
-      int in = lane < 32 ? count[(31 - lane) * 64 + 63 - l] : 0;
-      const int here = in;
-#pragma unroll
-      for (int off = 1; off < 32; off <<= 1) {
-        const int o = __shfl_up(in, off, 64);
-        if (lane >= off) in += o;
+    int my_qt = -1;
+    if (p.nq > kRowsSort) {
+      const int place = place_of(lane);
+      if (place < p.nq * groups) my_qt = p.nq - 1 - place / groups;
+    } else {
+      // bucket b of works at (b % 32) * 64 + b / 32, so that lane b / 32 reads
+      // its 32 without conflicts; the last bucket has all longer ones too
+      constexpr int kBuckets = 2048;
+      int* count = reinterpret_cast<int*>(smem);
+      u16* works = reinterpret_cast<u16*>(smem + kBuckets * 4);
+      int* found = reinterpret_cast<int*>(smem + kBuckets * 4 + kRowsSort * 2);
+      static_assert(kBuckets * 4 + kRowsSort * 2 + kRowsList * 4 <=
+                    2 * kBufs * kTileB);
+      constexpr int kThreads = kWaves * kWaveSize;
+      for (int i = tid; i < kBuckets; i += kThreads) count[i] = 0;
+      __syncthreads();
+      for (int i = tid; i < p.nq; i += kThreads) {
+        const int b = min(q_tile<PAGED, EXT>(p, i).work, kBuckets - 1);
+        works[i] = b;
+        if (b > 0) atomicAdd(&count[b % 32 * 64 + b / 32], 1);
       }
-      const int k =
-          __builtin_ctzll(__ballot(lane < 32 && in > rank));
-      rank -= __shfl(in, k, 64) - __shfl(here, k, 64);
-      const int work = (63 - l) * 32 + 31 - k;
-      // its rank-th query tile
-      for (int i0 = 0; i0 < p.nq; i0 += kWaveSize) {
-        const int i = i0 + lane;
-        const unsigned long long same =
-            __ballot(i < p.nq && works[min(i, p.nq - 1)] == work);
-        const int n = __builtin_popcountll(same);
-        if (rank < n) {
-          const int before = __builtin_popcountll(
-              same & ((1ull << lane) - 1));
-          if ((same >> lane & 1) && before == rank) found[r] = i;
-          break;
+      __syncthreads();
+      // lane l: buckets 2047 - 32 l down to 2016 - 32 l
+      const int line = 63 - lane;
+      int own = 0;
+      for (int k = 0; k < 32; ++k) own += count[k * 64 + line];
+      int incl = own;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int o = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += o;
+      }
+      const int all = __shfl(incl, 63, 64);
+      if (tid < kRowsList) found[tid] = -1;
+      __syncthreads();
+      for (int r = wave; r < kRowsList; r += kWaves) {
+        int rank = place_of(r) / groups;
+        if (rank >= all) break;          // places ascend
+        const int l = __builtin_ctzll(__ballot(incl > rank));
+        rank -= __shfl(incl, l, 64) - __shfl(own, l, 64);
+        // the bucket: lane k has the k-th from the line's top
+        int in = lane < 32 ? count[(31 - lane) * 64 + 63 - l] : 0;
+        const int here = in;
+#pragma unroll
+        for (int off = 1; off < 32; off <<= 1) {
+          const int o = __shfl_up(in, off, 64);
+          if (lane >= off) in += o;
         }
-        rank -= n;
+        const int k =
+            __builtin_ctzll(__ballot(lane < 32 && in > rank));
+        rank -= __shfl(in, k, 64) - __shfl(here, k, 64);
+        const int work = (63 - l) * 32 + 31 - k;
+        // its rank-th query tile
+        for (int i0 = 0; i0 < p.nq; i0 += kWaveSize) {
+          const int i = i0 + lane;
+          const unsigned long long same =
+              __ballot(i < p.nq && works[min(i, p.nq - 1)] == work);
+          const int n = __builtin_popcountll(same);
+          if (rank < n) {
+            const int before = __builtin_popcountll(
+                same & ((1ull << lane) - 1));
+            if ((same >> lane & 1) && before == rank) found[r] = i;
+            break;
+          }
+          rank -= n;
+        }
       }
+      __syncthreads();
+      my_qt = found[lane];
     }
-    __syncthreads();
-    my_qt = found[lane];
+    if (my_qt >= 0) mine = q_tile<PAGED, EXT>(p, my_qt);
+    to_do = __ballot(my_qt >= 0 && mine.work > 0);
+    if (to_do == 0) return;
+    __syncthreads();                   // the lists' LDS is free
   }
-  QTile mine = {};
-  if (my_qt >= 0) mine = q_tile<PAGED, EXT>(p, my_qt);
-  unsigned long long to_do = __ballot(my_qt >= 0 && mine.work > 0);
-  if (to_do == 0) return;
-  if (!one) __syncthreads();           // the lists' LDS is free
 
-  // the r-th of them, uniform
+  // the first of `of`, uniform
   struct Item {
     QTile t;
     int hg, first, skip_lo, skip_hi;   // first and skipped key tiles
   };
-  auto item_of = [&](int r) {
+  auto item_of = [&](unsigned long long of) {
+    const int r = LISTS ? __builtin_ctzll(of) : 0;
     Item it;
-    it.t.seq = __builtin_amdgcn_readlane(mine.seq, r);
-    it.t.row0 = __builtin_amdgcn_readlane(mine.row0, r);
-    it.t.seq_start = __builtin_amdgcn_readlane(mine.seq_start, r);
-    it.t.seq_len = __builtin_amdgcn_readlane(mine.seq_len, r);
-    it.t.k_len = __builtin_amdgcn_readlane(mine.k_len, r);
-    it.t.work = __builtin_amdgcn_readlane(mine.work, r);
+    it.t = mine;
+    if (LISTS) {
+      it.t.seq = __builtin_amdgcn_readlane(mine.seq, r);
+      it.t.row0 = __builtin_amdgcn_readlane(mine.row0, r);
+      it.t.seq_start = __builtin_amdgcn_readlane(mine.seq_start, r);
+      it.t.seq_len = __builtin_amdgcn_readlane(mine.seq_len, r);
+      it.t.k_len = __builtin_amdgcn_readlane(mine.k_len, r);
+      it.t.work = __builtin_amdgcn_readlane(mine.work, r);
+    }
     it.hg = place_of(r) % groups;
     // tiles between the kept first keys and the window of the first row
-    it.skip_lo = EXT ? ceil_div(p.keep_first, kKVTile) : 0;
-    it.skip_hi = EXT && p.window > 0
+    it.skip_lo = kWindow ? ceil_div(p.keep_first, kKVTile) : 0;
+    it.skip_hi = kWindow && p.window > 0
         ? max(it.t.k_len - it.t.seq_len + it.t.row0 - p.window + 1, 0) /
               kKVTile
         : 0;
-    it.first = EXT && it.skip_lo == 0 ? it.skip_hi : 0;
+    it.first = kWindow && it.skip_lo == 0 ? it.skip_hi : 0;
     return it;
   };
   auto after = [&](const Item& it, int tile) {
     const int n = tile + 1;
-    return EXT && n >= it.skip_lo && n < it.skip_hi ? it.skip_hi : n;
+    return kWindow && n >= it.skip_lo && n < it.skip_hi ? it.skip_hi : n;
   };
 
   // ---- staging: the next key tile to request, of this query tile or a later
   // one. Wave w copies rows 16w..16w+15 of it, one cache block. Rows past
   // the end repeat the last one (finite values; their scores are masked).
-  unsigned long long to_request = to_do & (to_do - 1);
-  Item ahead = item_of(__builtin_ctzll(to_do));
+  unsigned long long to_request = LISTS ? to_do & (to_do - 1) : 0;
+  Item ahead = item_of(to_do);
   int atile = ahead.first;
   bool more = true;                    // there is such a tile
   int blk = 0;
@@ -349,11 +390,11 @@ void prefill_rows_kernel(const PrefillArgs p) {
   auto step_ahead = [&] {
     atile = after(ahead, atile);
     if (atile < ahead.t.work) return;
-    if (to_request == 0) {
+    if (!LISTS || to_request == 0) {
       more = false;
       return;
     }
-    ahead = item_of(__builtin_ctzll(to_request));
+    ahead = item_of(to_request);
     to_request &= to_request - 1;
     atile = ahead.first;
   };
@@ -390,7 +431,7 @@ void prefill_rows_kernel(const PrefillArgs p) {
     for (int f = 0; f < KF; ++f)
       b_q[f] = *reinterpret_cast<const short8*>(qrow + f * 16 + hi1 * 8);
   };
-  Item it = item_of(__builtin_ctzll(to_do));
+  Item it = item_of(to_do);
   load_q(it);
 
   RowSoftmax<D> row(lane, p.scale);
@@ -426,7 +467,7 @@ void prefill_rows_kernel(const PrefillArgs p) {
             if (kv0 + 32 * b + crow(r, 0) > q_at)
               s_acc[b][r] = -INFINITY;
       }
-      if (EXT && p.window > 0 && kv0 + kKVTile > p.keep_first &&
+      if (kWindow && p.window > 0 && kv0 + kKVTile > p.keep_first &&
           my_q_max - kv0 >= p.window) {
 #pragma unroll
         for (int b = 0; b < 2; ++b)
@@ -467,24 +508,25 @@ void prefill_rows_kernel(const PrefillArgs p) {
       const int kv0 = tile * kKVTile;
       // (or outside the window of every row of the wave)
       seen = active && kv0 <= my_q_max &&
-             !(EXT && p.window > 0 && kv0 >= p.keep_first &&
+             !(kWindow && p.window > 0 && kv0 >= p.keep_first &&
                kv0 + kKVTile <= ctx_start + row0 - p.window + 1);
       if (seen)
         row.scores(smem, buf * kTileB, (kBufs + buf) * kTileB, b_q, s_acc);
       const int n = after(it, tile);
-      if (n >= it.t.work) break;
+      if (LISTS && n >= it.t.work) break;
       weigh();
+      if (!LISTS && n >= it.t.work) break;
       tile = n;
       buf ^= 1;
     }
     // the next query tile's queries, while the last keys are weighed
     to_do &= to_do - 1;
     const Item now = it;
-    if (to_do != 0) {
-      it = item_of(__builtin_ctzll(to_do));
+    if (LISTS && to_do != 0) {
+      it = item_of(to_do);
       load_q(it);
     }
-    weigh();
+    if (LISTS) weigh();
 
     // ---- epilogue: every wave is done with the tile, whose place the
     // results are turned over in
@@ -538,9 +580,22 @@ void prefill_rows_kernel(const PrefillArgs p) {
           });
       behind = rows >= 32 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
     }
-    if (to_do == 0) return;
+    if (!LISTS || to_do == 0) return;
     buf ^= 1;
   }
+}
+
+// `longest`: no key lies further on in its context
+template <int D, bool PAGED, bool FP8, bool EXT>
+void launch_rows(const PrefillArgs& a, int64_t longest, hipStream_t stream) {
+  const int64_t items = static_cast<int64_t>(a.num_q_heads / a.hpb) * a.nq;
+  const dim3 block(kRowsWaves * kWaveSize);
+  if (rows_by_lists(items, D, a.sub, a.window, longest))
+    hipLaunchKernelGGL((prefill_rows_kernel<D, PAGED, FP8, EXT, true>),
+                       dim3(rows_grid(items, D)), block, 0, stream, a);
+  else
+    hipLaunchKernelGGL((prefill_rows_kernel<D, PAGED, FP8, EXT, false>),
+                       dim3(static_cast<unsigned>(items)), block, 0, stream, a);
 }
 
 }  // namespace fi

@@ -892,14 +892,11 @@ bool launch_equal_sizes(u16* out, const u16* q, const u16* k_cache,
   a.block_size = block_size;
   a.window = window;
   a.keep_first = keep_first;
-  const dim3 grid(rows_grid(static_cast<int64_t>(H / a.hpb) * a.nq, DK));
-  const dim3 block(kRowsWaves * kWaveSize);
+  const int64_t longest = static_cast<int64_t>(bt_stride) * block_size;
   if (DK == 128)
-    hipLaunchKernelGGL((prefill_rows_kernel<128, true, false, true>),
-                       grid, block, 0, s, a);
+    launch_rows<128, true, false, true>(a, longest, s);
   else
-    hipLaunchKernelGGL((prefill_rows_kernel<64, true, false, true>),
-                       grid, block, 0, s, a);
+    launch_rows<64, true, false, true>(a, longest, s);
   return true;
 }
 

@@ -625,10 +625,12 @@ def test_prefill_attention_long_parts(hq, hk, scale_by):
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("hq,hk,head_dim,seqs,longest", [
     (32, 8, 128, 9, 700),     # a few query tiles each, of very uneven work
-    (8, 2, 64, 60, 150),      # lists that end with none
+    (8, 2, 128, 60, 150),     # lists that end with none
+    (64, 64, 128, 420, 3),    # more than a list holds: more workgroups
+    (8, 2, 64, 60, 150),      # heads of 64: one each, whatever their number
     (24, 8, 128, 150, 70),    # three heads a group: one per workgroup
     (32, 8, 128, 1040, 9),    # more query tiles than are put in order
-    (64, 64, 64, 420, 3),     # more than a list holds: more workgroups
+    (64, 64, 64, 420, 3),
 ])
 def test_prefill_attention_lists_of_query_tiles(hq, hk, head_dim, seqs,
                                                 longest, fp8):
@@ -699,6 +701,125 @@ def test_prefill_attention_lists_of_query_tiles(hq, hk, head_dim, seqs,
     # P and the output are rounded to bf16 (2^-9 each), |v| stays below 5
     assert_close_bf16(out[at:at + new[i]].cpu(),
                       want.transpose(0, 1).bfloat16(), atol=2e-2, rtol=2e-2)
+
+
+LIST_LENS = [700, 1, 130, 513, 64, 900, 300]   # new rows of the requests
+
+
+@pytest.mark.parametrize("hq,hk,head_dim", [
+    (32, 8, 128),     # a group's heads side by side in a workgroup
+    (40, 8, 128),     # one head a workgroup
+    (32, 8, 64), (32, 32, 64)])
+def test_prefill_attention_dense_lists_of_query_tiles(hq, hk, head_dim):
+    """Dense rows, more query tiles than workgroups: the bits of each request
+    alone; rows of the next request are never read for this one's."""
+    g = torch.Generator().manual_seed(hq + head_dim)
+    lens = LIST_LENS
+    q, k, v = (torch.randn(sum(lens), h, head_dim, generator=g).bfloat16()
+               .to(DEV) for h in (hq, hk, hk))
+    at = [0, *torch.tensor(lens).cumsum(0).tolist()]
+
+    def run(i, j):
+        cu = torch.tensor([n - at[i] for n in at[i:j + 1]], dtype=torch.int32,
+                          device=DEV)
+        rows = slice(at[i], at[j])
+        return ops.prefill_attention(q[rows], k[rows], v[rows], cu)
+
+    out = run(0, len(lens))
+    for i in range(len(lens)):
+        assert torch.equal(out[at[i]:at[i + 1]], run(i, i + 1)), i
+
+
+@pytest.mark.parametrize("hq,hk,fp8", [(32, 8, False), (32, 8, True),
+                                       (32, 32, False), (32, 32, True)])
+def test_prefill_attention_lists_of_query_tiles_heads_of_64(hq, hk, fp8):
+    """Heads of 64 go by lists between one round of workgroups and three, of
+    contexts of 512 to 4096 (here 960 query tiles; contexts of 944 and fewer):
+    the bits of each request alone. And rows off the 16-byte grid."""
+    g = torch.Generator().manual_seed(hk)
+    new, past = LIST_LENS, [40, 0, 0, 5, 0, 40, 0]
+    ctx = [a + b for a, b in zip(new, past)]
+    need = [-(-c // 16) for c in ctx]
+    bt = torch.zeros(len(new), max(need), dtype=torch.int32)
+    for i, row in enumerate((torch.randperm(sum(need), generator=g) + 1)
+                            .int().split(need)):
+        bt[i, :need[i]] = row
+    q = torch.randn(sum(new), hq, 64, generator=g).bfloat16().to(DEV)
+    kc, vc = (torch.randn(sum(need) + 1, hk, 16, 64, generator=g).bfloat16()
+              .to(DEV) for _ in range(2))
+    if fp8:
+        kc, vc = _fp8_cache(kc), _fp8_cache(vc)
+    bt = bt.to(DEV)
+    at = [0, *torch.tensor(new).cumsum(0).tolist()]
+
+    def run(i, j, out=None):
+        cu = torch.tensor([n - at[i] for n in at[i:j + 1]], dtype=torch.int32,
+                          device=DEV)
+        lens = torch.tensor(ctx[i:j], dtype=torch.int32, device=DEV)
+        return ops.prefill_attention_paged(q[at[i]:at[j]], kc, vc, bt[i:j], cu,
+                                           lens, out=out)
+
+    out = run(0, len(new))
+    for i in range(len(new)):
+        assert torch.equal(out[at[i]:at[i + 1]], run(i, i + 1)), i
+    off = torch.full((out.numel() + 8,), 7.0, dtype=out.dtype, device=DEV)
+    run(0, len(new), off[4:-4].view(out.shape))
+    assert torch.equal(off[4:-4].view(out.shape), out)
+    assert (off[:4] == 7).all() and (off[-4:] == 7).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("heads,groups,block,window,keep,gate", [
+    (32, 8, 16, 0, 0, None), (32, 8, 1, 0, 0, "entry"),
+    (32, 32, 8, 0, 0, "head"),     # one head a workgroup
+    (32, 8, 16, 200, 70, "entry"),  # a window: one query tile a workgroup
+    (40, 8, 1, 33, 0, "head")])
+def test_sink_attention_many_row_tiles(D, heads, groups, block, window, keep,
+                                       gate):
+    """More query tiles than workgroups (832 and more), the next one's keys of
+    another portion: the bits of each portion alone, also off the 16-byte grid."""
+    from fusioninfer_amd.ops import seqmix
+
+    g = torch.Generator().manual_seed(D + heads + window)
+    new, past = LIST_LENS, [40, 0, 277, 5, 0, 64, 0]
+    ctx = [a + b for a, b in zip(new, past)]
+    need = [-(-c // block) for c in ctx]
+    order = torch.randperm(sum(need) + 2, generator=g)
+    table = torch.zeros(len(new), max(need), dtype=torch.int32)
+    for i, row in enumerate(order[:sum(need)].int().split(need)):
+        table[i, :need[i]] = row
+    T = sum(new)
+    q = torch.randn(T, heads, D, generator=g).bfloat16().to(DEV)
+    k, v = (torch.randn(len(order), groups, block, D, generator=g).bfloat16()
+            .to(DEV) for _ in range(2))
+    sink = (torch.randn(heads, generator=g) * 3).to(DEV)
+    og = {"head": torch.randn(T, heads, generator=g),
+          "entry": torch.randn(T, heads * D, generator=g)}.get(gate)
+    og = None if og is None else og.bfloat16().to(DEV)
+    at = [0, *torch.tensor(new).cumsum(0).tolist()]
+
+    def run(i, j, out=None):
+        rows = slice(at[i], at[j])
+        return seqmix.sink_paged_attention(
+            q[rows], k, v, table[i:j].to(DEV),
+            torch.cat([torch.full((n,), m) for m, n in enumerate(new[i:j])])
+            .int().to(DEV),
+            torch.cat([torch.arange(p, p + n) for n, p in
+                       zip(new[i:j], past[i:j])]).int().to(DEV), D ** -0.5,
+            sink=sink, out_gate=None if og is None else og[rows],
+            seq_cu=torch.tensor([n - at[i] for n in at[i:j + 1]],
+                                dtype=torch.int32, device=DEV),
+            tiles=seqmix.build_attention_tiles(new[i:j], device=DEV),
+            window=window, keep_first=keep, out=out)
+
+    out = run(0, len(new))
+    assert torch.isfinite(out).all()
+    for i in range(len(new)):
+        assert torch.equal(out[at[i]:at[i + 1]], run(i, i + 1)), i
+    off = torch.full((out.numel() + 8,), 7.0, dtype=out.dtype, device=DEV)
+    run(0, len(new), off[4:-4].view(out.shape))
+    assert torch.equal(off[4:-4].view(out.shape), out)
+    assert (off[:4] == 7).all() and (off[-4:] == 7).all()
 
 
 @pytest.mark.parametrize("hq,hk", [(2, 2), (3, 1)])
