@@ -100,6 +100,17 @@ FI_DEV float block_reduce_sum(float wave_val, float* scratch) {
   return total;
 }
 
+// 8 or 16 bytes to global memory. Where a pointer has been through asm the
+// compiler no longer sees that it is one to there; its store is then a flat one,
+// which LDS waits wait for too and which a counted wait must not rely on the
+// order of.
+template <class T>
+FI_DEV void store_global(u16* to, const T& value) {
+  typedef __attribute__((ext_vector_type(sizeof(T) / 4))) u32 Words;
+  *(__attribute__((address_space(1))) Words*)to =
+      __builtin_bit_cast(Words, value);
+}
+
 // more than the memory-side cache holds: what is read once better goes past it
 inline bool beyond_caches(int64_t bytes) { return bytes > int64_t{256} << 20; }
 

@@ -374,7 +374,7 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
             }
             o.h[c] = f32_to_bf16(v);
           }
-          *reinterpret_cast<decltype(o)*>(to) = o;
+          store_global(to, o);
           // (a step at a time, or all rows' places would be kept)
           to += static_cast<int64_t>(r < 3 ? 1 : 13) * N;
           asm volatile("" : "+v"(to));

@@ -410,10 +410,10 @@ FI_DEV void put_rows(unsigned char* smem, int at, u16* out, int64_t stride,
         const uint4 v = *reinterpret_cast<const uint4*>(
             smem + (get ^ (r & (R::kChunk - 1)) * 16) + r * R::kRowB);
         if (all || wide) {
-          *reinterpret_cast<uint4*>(to) = v;
+          store_global(to, v);
         } else {                       // rows off the 16-byte grid
-          reinterpret_cast<uint2*>(to)[0] = make_uint2(v.x, v.y);
-          reinterpret_cast<uint2*>(to)[1] = make_uint2(v.z, v.w);
+          store_global(to, make_uint2(v.x, v.y));
+          store_global(to + 4, make_uint2(v.z, v.w));
         }
       }
       to += R::kRowsPerDma * stride;

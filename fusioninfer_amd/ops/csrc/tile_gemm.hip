@@ -141,7 +141,7 @@ FI_DEV void store_row(u16* to, const u16* bias, const float (&sum)[C],
     if (MODE == BIAS) y += bf16_to_f32(add.h[c]);
     o.h[c] = f32_to_bf16(y);
   }
-  *reinterpret_cast<Outputs*>(to) = o;
+  store_global(to, o);
 }
 
 // Where a lane's results lie. Slot i of fragment f holds column i * kLaneCols +
