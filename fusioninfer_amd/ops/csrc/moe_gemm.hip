@@ -30,7 +30,8 @@ namespace fi {
 void launch_moe_tile(u16*, const u16*, const u16*, const int*, const int*,
                      const int*, int, int, int, int, int, float, hipStream_t);
 void launch_moe_wide(u16*, const u16*, const u16*, const int*, const int*,
-                     const int*, int, int, int, int, float, hipStream_t);
+                     const int*, int, int, int, int, int, int, float,
+                     hipStream_t);
 void launch_moe_stream(u16*, const u16*, const u16*, const int*, const int*,
                        const int*, int, int, int, int, int, float,
                        hipStream_t);
@@ -289,8 +290,8 @@ void launch_moe_gemm(u16* out, const u16* a, const u16* b,
   else if (wide_tiles(max_mtiles, experts, K, N, mode) &&
            reinterpret_cast<uintptr_t>(b) % 16 == 0 &&
            reinterpret_cast<uintptr_t>(out) % 16 == 0)
-    launch_moe_wide(out, a, b, sorted_ids, expert_ids, n_valid, rows, K, N,
-                    mode, limit, stream);
+    launch_moe_wide(out, a, b, sorted_ids, expert_ids, n_valid, max_mtiles,
+                    experts, rows, K, N, mode, limit, stream);
   else
     launch_moe_tile(out, a, b, sorted_ids, expert_ids, n_valid, max_mtiles,
                     rows, K, N, mode, limit, stream);

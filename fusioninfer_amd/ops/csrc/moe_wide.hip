@@ -10,21 +10,24 @@
 // 40).
 //
 // Two neighbouring blocks of an expert take tiles of 256 rows by 256 columns
-// instead, waves two by two: 64 KB a stage, not 80, and every fragment of B once
-// for both. (All that differs is where a wave's requests go and what it reads; a
-// wave's products are the same.) 128 experts, top 8, 2048 x 768, both products,
-// us, blocks apart and in pairs: 8100 rows 645 and 614, 4000 401 and 380; 64
-// experts, 2048 x 1408, top 6, 8192 rows 850 and 806; 8 experts, 4096 x 6144, top
-// 2, 8192 rows 2128 and 2102. (K begun elsewhere by columns or by blocks, so that
-// CUs read other channels: 630 and 635 instead of 614.)
+// instead (PAIRS), waves two by two: 64 KB a stage, not 80, and every fragment of B
+// once for both. (All that differs is where a wave's requests go and what it reads;
+// a wave's products are the same.) us, blocks apart and in pairs: down, 128 experts,
+// top 8, 2048 x 768, 8100 rows 242 and 227, 4000 146 and 139; 64 experts, 2048 x
+// 1408, top 6, 8192 rows 281 and 278; 8 experts, 4096 x 6144, top 2, 8192 rows 767
+// and 743. Rows that are gathered gain where experts have few blocks
+// (launch_moe_wide).
 //
 // A stage is 64 of K: 128 gathered rows of 128 bytes, and 64 of B's packed
 // fragments (1 KB each), 80 KB in all; two of them are kept, all of a CU's
 // LDS. As in the dense kernel of 256 x 256 tiles a stage is used in two halves:
 // the second half's fragments are read while the first is multiplied, then
 // the stage's place is free and the stage after the next is requested into
-// it. Every MFMA is followed by at most one other instruction, in an order
-// that is pinned. The DMAs run on over the borders of tiles; the rows' ids
+// it. Every MFMA is followed by at most one other step, in an order that is
+// pinned; with PAIRS eight of the requests ask for the tile's shape first. (A body
+// per shape does not fit the registers; requests that ask nothing, with the four
+// that a square tile has no use for out of range: gate|up the same, down 225 and
+// 239 us at 8100 rows.) The DMAs run on over the borders of tiles; the rows' ids
 // come through the scalar cache, since a vector load would wait for all DMAs
 // in front of it.
 //
@@ -44,12 +47,11 @@
 // 416; 4000 rows 152 and 146.
 //
 // A stage takes 1.4 to 1.7 us; a tile's end 5 to 7, most of it until its results
-// have left (the stages after the first wait for them). Measured, us (TFLOP/s
-// of the real rows), 128 x 256 tiles and these: 8765 rows, 128 experts, top 8,
-// 2048 x 768: gate|up 467 (945) and 445 (992), down 308 (717) and 266 (831);
-// 8192 rows, 64 experts, top 6, 2048 x 1408: 544 (1040) and 549, down 324 and
-// 284 (997); 8192 rows, 8 experts, top 2, 4096 x 6144 gate|up 1385 (1190) and
-// 1324 (1245).
+// have left (the stages after the first wait for them). Tiles of 128 x 256, two to
+// a CU, and these, us (TFLOP/s of the real rows, now): 8765 rows, 128 experts, top
+// 8, 2048 x 768: gate|up 467 and 466 (946), down 308 and 254 (869); 8192 rows, 64
+// experts, top 6, 2048 x 1408: 544 and 555 (1022), down 324 and 278 (1020); 8192
+// rows, 8 experts, top 2, 4096 x 6144: gate|up 1385 and 1335 (1235).
 
 #include <hip/hip_runtime.h>
 
@@ -66,7 +68,51 @@ constexpr int kRowsB = kWideM * 128, kWaveB = 16 * 1024;  // A's, a wave's B
 constexpr int kWideStageB = kRowsB + 4 * kWaveB;
 constexpr int kRunRows = 8;                               // row blocks of a run
 
-template <int MODE>
+// Which blocks are the second of a pair: lane l of `lo` and `hi` has those of
+// blocks 64 l to 64 l + 63, of the first 4096; others go alone.
+struct Pairs {
+  u32 lo = 0, hi = 0;
+  FI_DEV bool second(int m) const {
+    const u32 l = __builtin_amdgcn_readlane(lo, m / 64 & 63);
+    const u32 h = __builtin_amdgcn_readlane(hi, m / 64 & 63);
+    return m < 64 * kWaveSize && ((m & 32 ? h : l) >> (m & 31) & 1);
+  }
+};
+
+// From one pass over the ids. (Looked up for every place, back to the beginning
+// of its expert's blocks, it costs more the more of them there are: 8 experts,
+// 2048 x 1408, 32768 rows with half of them on one, down 381 and 337 us so.)
+FI_DEV Pairs pairs_of(const int* __restrict__ expert_ids, int nv, int lane) {
+  Pairs p;
+  const int words = min((nv + 63) / 64, kWaveSize);
+  int last = 0, last_id = -1;    // beginning, id of the word before
+  constexpr int kAtOnce = 16;
+  for (int w0 = 0; w0 < words; w0 += kAtOnce) {
+    int id[kAtOnce];
+#pragma unroll
+    for (int i = 0; i < kAtOnce; ++i)
+      id[i] = expert_ids[min((w0 + i) * 64 + lane, nv - 1)];
+#pragma unroll
+    for (int i = 0; i < kAtOnce; ++i) {
+      if (w0 + i >= words) break;
+      const int base = (w0 + i) * 64, m = base + lane;
+      const int up = __shfl_up(id[i], 1, kWaveSize);
+      const int before = lane == 0 ? last_id : up;
+      const unsigned long long begins =
+          __ballot(m < nv && (m == 0 || id[i] != before));
+      const unsigned long long up_to = begins & (~0ull >> (63 - lane));
+      const int of = m - (up_to ? base + 63 - __builtin_clzll(up_to) : last);
+      const unsigned long long seconds = __ballot(m < nv && (of & 1));
+      if (begins) last = base + 63 - __builtin_clzll(begins);
+      last_id = __builtin_amdgcn_readlane(id[i], kWaveSize - 1);
+      p.lo = lane == w0 + i ? static_cast<u32>(seconds) : p.lo;
+      p.hi = lane == w0 + i ? static_cast<u32>(seconds >> 32) : p.hi;
+    }
+  }
+  return p;
+}
+
+template <int MODE, bool PAIRS>
 __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
     u16* __restrict__ out,              // [PM, N]
     const u16* __restrict__ a,          // gathered x [T, K]; MODE 0 [PM, K]
@@ -100,28 +146,15 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
     int square, none;
   };
   const ConstInts experts = const_ints(expert_ids);
+  Pairs pairs;
+  if (PAIRS) pairs = pairs_of(expert_ids, nv, lane);
   auto place_of = [&](int at) __attribute__((always_inline)) {
     const int m0 = at / (kRunRows * NT) * kRunRows;
     const int rows = min(kRunRows, nv - m0);
     const int in = at - m0 * NT;
     const int n = in / rows, m = m0 + in - n * rows;
-    const int e = experts[m];
-    int before = 0;              // blocks of the expert in front of this one
-    for (int top = m; top > 0;) {
-      constexpr int kLook = 8;   // ids at a time
-      const int from = max(top - kLook, 0);
-      int id[kLook], same = 0;
-#pragma unroll
-      for (int i = 0; i < kLook; ++i) id[i] = experts[max(top - 1 - i, from)];
-#pragma unroll
-      for (int i = 0; i < kLook; ++i)
-        same += same == i && top - i > from && id[i] == e;
-      before += same;
-      if (same < top - from) break;
-      top = from;
-    }
-    const bool second = before & 1;
-    if (!second && !(m + 1 < nv && experts[min(m + 1, nv - 1)] == e))
+    const bool second = PAIRS && pairs.second(m);
+    if (!PAIRS || !(second || (m + 1 < nv && pairs.second(m + 1))))
       return Place{m, n, 0, 0};
     const int column = (second ? NT : 0) + n;
     return Place{m - second, column, 1, column * (GATE_UP ? 128 : 256) >= N};
@@ -172,7 +205,7 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
     to_lds[2] = rsquare ? 2 * kRowsB + wave * 8192 - 4096 : to_lds[1];
     to_lds[3] = rsquare ? to_lds[2] - 8192 : to_lds[1];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < (PAIRS ? 2 : 1); ++h) {
       // (a wide tile's a second time: around a branch they would be vector loads)
       const int row0 = wave * (rsquare ? 64 : 32) + (rsquare ? h * 32 : 0);
       int ids[32];
@@ -215,9 +248,9 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
   if (waiting == 0) return;
   u32 rbuf = lds0;
   auto m0_of = [&](int j) { set_m0(rbuf + to_lds[min(j / 4, 3)] + j * 1024); };
-  auto load_of = [&](int j) __attribute__((always_inline)) {
-    if (j >= 16 && rsquare) return;
-    if (j < 4 || (j < 8 && rsquare)) {
+  auto load_of = [&](int j, auto square) __attribute__((always_inline)) {
+    if (j >= 16 && square) return;
+    if (j < 4 || (j < 8 && square)) {
       load_lds(da, a_voff[j % 8], a_soff);
     } else {
       const int f = (j - 4) % 8, half = (j - 4) / 8;
@@ -262,7 +295,7 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
     for (int j = 0; j < 20; ++j) {
       m0_of(j);
       asm volatile("s_nop 4");
-      load_of(j);
+      load_of(j, rsquare);
     }
     requested();
   }
@@ -280,9 +313,10 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
   constexpr int kStores = 32;
   constexpr int kFree = 40, kEarly = 6;  // MFMAs up to the first barrier, DMAs
                                          // between the two
-  // `behind`: stores that follow the DMAs that are waited for; `last`: of the tile
-  auto stage = [&](auto first, bool behind,
-                   bool last) __attribute__((always_inline)) {
+  // `square`: of the tile that is requested. `behind`: stores that follow the DMAs
+  // that are waited for; `last`: of the tile
+  auto stage_for = [&](auto first, auto square, bool behind,
+                       bool last) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 64; ++i) {
       const int mi = i >> 3, f = i & 7;
@@ -300,7 +334,7 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
       const int j = i - kFree - 1;
       if (j >= 0 && j < 2 * kEarly) {
         if (j % 2 == 0) m0_of(j / 2);
-        else load_of(j / 2);
+        else load_of(j / 2, square);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -322,11 +356,16 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
       if (i % 4 == 0 && i >= 32) a0[i / 4 - 8] = rda(buf, 0, i / 4 - 8);
       if (i / 4 < 20 - kEarly) {
         if (i % 4 == 1) m0_of(kEarly + i / 4);
-        if (i % 4 == 2) load_of(kEarly + i / 4);
+        if (i % 4 == 2) load_of(kEarly + i / 4, square);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
     requested();
+  };
+  // (asked once a stage: a question per DMA would part its products)
+  auto stage = [&](auto first, bool behind,
+                   bool last) __attribute__((always_inline)) {
+    stage_for(first, rsquare, behind, last);
   };
 
   bool behind = false;
@@ -391,19 +430,37 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
 
 }  // namespace
 
+// Gathered rows go in pairs unless experts have about 16 blocks or more (every one
+// is taken to leave half a block empty): the ids of a pair's rows, and the questions
+// of its shape, cost a tile 2 to 4 us, which pays while few blocks share the
+// weights. us, both products, gate|up apart and in pairs: 128 experts, 2048 x 768, 2
+// blocks each 331 and 315, 2.3 each 396 and 388, 4.4 each 632 and 621, 8.5 each 1165
+// and 1140; 64 of 2048 x 1408, 6.5 each, 848 and 824, 12.5 each 1531 and 1513; 8 of
+// 4096 x 6144, 16 each, 2083 and 2090, 33 each, one of them 129, 3941 and 3960. (With
+// a lower clock, as after long steps: 4.4 each 650 and 651, 6.5 each 871 and 863.)
+// Where few experts have all rows the host does not see it: 8100 rows for 16 of 128
+// 545 and 554.
 void launch_moe_wide(u16* out, const u16* a, const u16* b,
                      const int* sorted_ids, const int* expert_ids,
-                     const int* n_valid, int rows, int K, int N, int mode,
-                     float limit, hipStream_t stream) {
+                     const int* n_valid, int max_mtiles, int experts,
+                     int rows, int K, int N, int mode, float limit,
+                     hipStream_t stream) {
   const int nt = ceil_div(N, mode == 1 || mode == 3 ? 256 : 512);
-#define FI_WIDE(M)                                                           \
-  hipLaunchKernelGGL((moe_wide_kernel<M>), dim3(kChip), dim3(256), 0,        \
+#define FI_WIDE(M, P)                                                        \
+  hipLaunchKernelGGL((moe_wide_kernel<M, P>), dim3(kChip), dim3(256), 0,     \
                      stream, out, a, b, sorted_ids, expert_ids, n_valid, K,  \
                      N, nt, static_cast<u32>(rows) * (K * 2), limit)
-  if (mode == 1) FI_WIDE(1);
-  else if (mode == 2) FI_WIDE(2);
-  else if (mode == 3) FI_WIDE(3);
-  else FI_WIDE(0);
+  if (mode == 0) {
+    FI_WIDE(0, true);
+  } else if (max_mtiles <= 16 * experts) {
+    if (mode == 1) FI_WIDE(1, true);
+    else if (mode == 2) FI_WIDE(2, true);
+    else FI_WIDE(3, true);
+  } else {
+    if (mode == 1) FI_WIDE(1, false);
+    else if (mode == 2) FI_WIDE(2, false);
+    else FI_WIDE(3, false);
+  }
 #undef FI_WIDE
 }
 

@@ -2416,6 +2416,43 @@ def test_moe_gemm_pairs_of_blocks(n, gate_up):
     assert torch.equal(out, few)
 
 
+@pytest.mark.parametrize("gate_up", [True, False])
+@pytest.mark.parametrize("counts", [
+    [1, 2, 8, 9, 3, 16, 1, 16] + [1] * 8 + [2] * 4,
+    [1] * 60 + [43, 1, 70, 3, 64],   # pairs over the ends of 64 blocks
+    [1, 62, 3, 70, 130],   # many blocks an expert: gathered rows go alone
+])
+def test_moe_gemm_pairs_of_many_blocks(counts, gate_up):
+    """Few and many blocks an expert, more than a word of the pairs' bits holds: the
+    bits of blocks taken alone."""
+    g = torch.Generator().manual_seed(len(counts))
+    k, T, experts = 128, 700, len(counts)
+    eid = torch.tensor(sum(([e] * c for e, c in enumerate(counts)), []),
+                       dtype=torch.int32, device=DEV)
+    blocks = len(eid)
+    wide, mode = ops._moe_native().moe_gemm_wide, 1 if gate_up else 0
+    n = next(n for n in range(640, 4096, 128)
+             if wide(blocks, experts, k, n, mode))
+    few_blocks = next(m for m in range(8, 64, 8)
+                      if not wide(m, experts, k, n, mode))
+    nv = torch.tensor([blocks], dtype=torch.int32, device=DEV)
+    sid = torch.randint(0, T, (blocks * 128,), generator=g).int().to(DEV)
+    x = torch.randn(T if gate_up else blocks * 128, k, generator=g)
+    w = torch.randn(experts, k, n * (2 if gate_up else 1), generator=g)
+    x, b = x.bfloat16().to(DEV), ops.pack_moe_weights(w.bfloat16().to(DEV))
+    out = torch.zeros(blocks * 128, n, dtype=torch.bfloat16, device=DEV)
+    few = torch.zeros_like(out)
+    ops.moe_gemm(out, x, b, sid, eid, nv, 128, gate_up)
+    for m in range(0, blocks, few_blocks):
+        rows = slice(m * 128, min(m + few_blocks, blocks) * 128)
+        ids = torch.zeros(few_blocks, dtype=torch.int32, device=DEV)
+        ids[:len(eid[m:m + few_blocks])] = eid[m:m + few_blocks]
+        ops.moe_gemm(few[rows], x if gate_up else x[rows], b, sid[rows], ids,
+                     torch.full_like(nv, len(eid[m:m + few_blocks])), 128,
+                     gate_up)
+    assert torch.equal(out, few)
+
+
 @pytest.mark.parametrize("k", [32, 224, 512, 768, 1024, 2080, 2624])
 @pytest.mark.parametrize("n,gate_up,act", [
     (64, True, None), (320, True, "clamped_glu"), (192, False, "relu_sq"),
