@@ -484,8 +484,19 @@ void tile_gemm_kernel(u16* __restrict__ out, floatx4* __restrict__ pieces,
 
 // Sums the pieces of the cut tiles: blockIdx.y is the tile, a thread takes a
 // lane's columns of one row, in kOps quads.
+//
+// Which parts of a piece a workgroup reads, and so which XCD, decides how fast the
+// next launch writes its pieces: with 32 workgroups of 256 threads a tile the
+// products in front of a join take 2 to 4 us longer than with 16 of 512 (joined gate
+// and up, M x K x N, us: 257 x 1024 x 4096 26.4 and 23.4, 511 x 1408 x 2048 30.4 and
+// 27.2, 257 x 2048 x 2816 29.2 and 25.5; plain 26.6 and 23.4, 30.7 and 27.8, 29.2 and
+// 25.7). e4m3: 64 of 256, 257 x 2048 x 4096 23.8 and 26.6, 511 x 4096 x 2560 31.7 and
+// 34.7.
+template <bool FP8>
+constexpr int kJoinThreads = FP8 ? 256 : 512;
+
 template <int MODE, bool FP8>
-__global__ __launch_bounds__(256)
+__global__ __launch_bounds__(kJoinThreads<FP8>)
 void tile_gemm_join_kernel(u16* __restrict__ out,
                            const floatx4* __restrict__ pieces,
                            const u16* __restrict__ bias,
@@ -498,7 +509,7 @@ void tile_gemm_join_kernel(u16* __restrict__ out,
   constexpr int kCols = SILU_MUL ? kTile / 2 : kTile, kRows = L::kRows;
   const int cols = SILU_MUL ? N / 2 : N;
   constexpr int kOps = L::kFrags / 4, kLaneCols = L::kLaneCols;
-  const int i = blockIdx.x * 256 + threadIdx.x;
+  const int i = blockIdx.x * kJoinThreads<FP8> + threadIdx.x;
   const int lane = i % kWaveSize, r = i / kWaveSize % L::kLaneRows;
   const int mi = i / kWaveSize / L::kLaneRows % L::kFrags;
   const int wave = i / kWaveSize / L::kLaneRows / L::kFrags;
@@ -579,7 +590,7 @@ void launch(u16* out, float* pieces, const typename Kind<FP8>::Elem* x,
                      x_stride, out_stride, p, turn);
   if (p.cut > 1)
     hipLaunchKernelGGL((tile_gemm_join_kernel<MODE, FP8>),
-                       dim3(FP8 ? 64 : 32, p.rest), dim3(256), 0,
+                       dim3(FP8 ? 64 : 16, p.rest), dim3(kJoinThreads<FP8>), 0,
                        stream, out, pc, bias, x_scales, w_scales, M, N,
                        out_stride, p);
 }
