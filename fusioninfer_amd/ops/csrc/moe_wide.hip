@@ -248,7 +248,7 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
   if (waiting == 0) return;
   u32 rbuf = lds0;
   auto m0_of = [&](int j) { set_m0(rbuf + to_lds[min(j / 4, 3)] + j * 1024); };
-  auto load_of = [&](int j, auto square) __attribute__((always_inline)) {
+  auto load_of = [&](int j, int square) __attribute__((always_inline)) {
     if (j >= 16 && square) return;
     if (j < 4 || (j < 8 && square)) {
       load_lds(da, a_voff[j % 8], a_soff);
@@ -313,10 +313,10 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
   constexpr int kStores = 32;
   constexpr int kFree = 40, kEarly = 6;  // MFMAs up to the first barrier, DMAs
                                          // between the two
-  // `square`: of the tile that is requested. `behind`: stores that follow the DMAs
-  // that are waited for; `last`: of the tile
-  auto stage_for = [&](auto first, auto square, bool behind,
-                       bool last) __attribute__((always_inline)) {
+  // `behind`: stores that follow the DMAs that are waited for; `last`: of the tile
+  auto stage = [&](auto first, bool behind,
+                   bool last) __attribute__((always_inline)) {
+    const int square = rsquare;  // of the tile that is requested
 #pragma unroll
     for (int i = 0; i < 64; ++i) {
       const int mi = i >> 3, f = i & 7;
@@ -361,11 +361,6 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
       __builtin_amdgcn_sched_barrier(0);
     }
     requested();
-  };
-  // (asked once a stage: a question per DMA would part its products)
-  auto stage = [&](auto first, bool behind,
-                   bool last) __attribute__((always_inline)) {
-    stage_for(first, rsquare, behind, last);
   };
 
   bool behind = false;

@@ -98,13 +98,13 @@ FI_DEV Tile tile_at(const TilePlan& p, int at) {
 
 // What the operands' type decides. A fragment is kRows rows of either operand
 // by half a stage of K; a lane has kChunks chunks of a row of it and, of a
-// product, kQuads times four results, neighbouring rows of x in one column.
+// product, results in one column, four neighbouring rows of x at a time.
 template <bool FP8>
 struct Kind {
   using Elem = u16;
   using Frag = short8;
   using Acc = floatx4;
-  static constexpr int kRows = 16, kChunks = 1, kQuads = 1;
+  static constexpr int kRows = 16, kChunks = 1;
   FI_DEV static void put(Frag& f, int, const short8& v) { f = v; }
 };
 template <>
@@ -112,7 +112,7 @@ struct Kind<true> {
   using Elem = unsigned char;
   using Frag = intx8;
   using Acc = floatx16;
-  static constexpr int kRows = 32, kChunks = 2, kQuads = 4;
+  static constexpr int kRows = 32, kChunks = 2;
   FI_DEV static void put(Frag& f, int chunk, const short8& v) {
     const intx4 q = __builtin_bit_cast(intx4, v);
 #pragma unroll
