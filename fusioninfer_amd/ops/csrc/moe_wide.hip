@@ -432,7 +432,10 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
 // blocks each 331 and 315, 2.3 each 396 and 388, 4.4 each 632 and 621, 8.5 each 1165
 // and 1140; 64 of 2048 x 1408, 6.5 each, 848 and 824, 12.5 each 1531 and 1513; 8 of
 // 4096 x 6144, 16 each, 2083 and 2090, 33 each, one of them 129, 3941 and 3960. (With
-// a lower clock, as after long steps: 4.4 each 650 and 651, 6.5 each 871 and 863.)
+// a lower clock, as after long steps: 4.4 each 650 and 651, 6.5 each 871 and 863. In
+// whole steps of four layers, one after the other, pairs are ahead, 4.4 each 5113
+// and 5068, 8.5 9378 and 9252; behind a pause of 0.1 s they lose 1 to 1.5 %, 6320 and
+// 6421, 11532 and 11644.)
 // Where few experts have all rows the host does not see it: 8100 rows for 16 of 128
 // 545 and 554.
 void launch_moe_wide(u16* out, const u16* a, const u16* b,

@@ -89,17 +89,22 @@ void prefill_attn_join_kernel(const PrefillArgs p) {
 // times as fast); the split form takes `fill` of them and about 35 us more
 // for its schedule, the pieces and the second launch, which is what 26 tiles
 // take. Where the new rows are most of the context, tiles differ in length
-// and longest-first already evens them out. Measured, whole / split in us:
-// 16 rows behind 2000: 47 / 33; 1024 behind 1024: 53 / 61; 1024 behind 8192:
-// 217 / 178; 4099 behind 16384: 1448 / 1250; 4096 behind 16384 (exactly two
-// rounds): 1190 / 1224; 2048 from the start: 57 / 100.
+// and longest-first already evens them out. Measured, whole / split in us, 32
+// query heads, 8 K/V heads of 128: 16 rows behind 2000 42 / 33; 512 behind 2048
+// 52 / 50; 1024 behind 1024 44 / 59; 1024 behind 8192 184 / 170; 4099 behind 16384
+// 1443 / 1201; 4096 behind 16384 (exactly two rounds) 1125 / 1127; 2048 from the
+// start 52 / 88. Of 22 portions of 16 to 4099 rows behind 1024 to 16384 the choice
+// is the faster one or within 4 %; with an e4m3 cache, whose whole tiles take a
+// tenth longer, within 14, with heads of 64 within 17. Of several contexts it
+// takes all for the longest, and can miss: 16 heads, four of 300 rows behind 1200
+// to 4000 87 / 61, whole; 32 heads, 700, 33 and 1200 behind 6000 212 / 234, split.
 //
 // The split form with 64 query vectors per wave (`pair`) takes 0.92 of the
 // time per tile, but 15 us more for its longer pipeline and the tiles that go
 // step by step: it is ahead from parts of 128 tiles on (8 query heads, 4 K/V
-// heads, 1024 rows behind 8192, parts of 17: 79 us, 94 with pairs; 32 and 8,
-// 700 + 33 + 1200 behind 6000, parts of 120: 240 and 250; 1000 behind 30000,
-// parts of 242: 519 and 489). `pairs`: whether that kernel takes the operands,
+// heads, 1024 rows behind 8192, parts of 17: 82 us, 96 with pairs; 32 and 8,
+// 700 + 33 + 1200 behind 6000, parts of 120: 239 and 255; 1000 behind 30000,
+// parts of 242: 509 and 484; 4099 behind 16384 1285 and 1188). `pairs`: whether that kernel takes the operands,
 // bf16 rows of 128 in a paged cache.
 PrefillPlan plan_prefill_attn(int ntiles, int tile_rows, int num_q_heads,
                               int num_kv_heads, int new_rows, int max_k_len,

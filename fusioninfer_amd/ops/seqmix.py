@@ -517,7 +517,9 @@ def _to_device(arrays, device):
     (Copies out of pageable memory wait for all that the GPU still has to do:
     three of them in a prompt's first latent layer, and the GPU then had nothing
     while the host launched the other layers. Four prompts of 1.8 thousand
-    tokens, four layers, and eight tokens each: 5245 us a pass, 5120 without.)"""
+    tokens, four layers, and eight tokens each: 5245 us a pass, 5120 without; less
+    where pinned memory of such a size is not at hand yet, the first pass over new
+    inputs with the other changes of that time 6509 and 6446.)"""
     starts = list(itertools.accumulate((-(-a.size // 4) * 4 for a in arrays),
                                        initial=0))
     host = torch.empty(starts[-1], dtype=torch.int32,
