@@ -436,8 +436,12 @@ __global__ __launch_bounds__(256, 1) void moe_wide_kernel(
 // whole steps of four layers, one after the other, pairs are ahead, 4.4 each 5113
 // and 5068, 8.5 9378 and 9252; behind a pause of 0.1 s they lose 1 to 1.5 %, 6320 and
 // 6421, 11532 and 11644.)
-// Where few experts have all rows the host does not see it: 8100 rows for 16 of 128
-// 545 and 554.
+// Where few experts have all rows the host does not see it, and pairs lose: 8100 rows
+// for 16 of 128 545 and 554; gate|up alone, 8 of 128 with 24 blocks each, 136 and 146
+// (130 by tiles of 128 x 256), 16 with 32 each 306 and 316. Uneven rows as such do
+// not: 128 experts of 58 to 2 blocks 364 and 369, of 17 to 3 389 and 384, 64 of 72 to
+// 2 672 and 666. (Asking in the kernel how many experts there are, and taking blocks
+// alone then, gives nothing back: 316 and 322, 64 experts 440 and 466.)
 void launch_moe_wide(u16* out, const u16* a, const u16* b,
                      const int* sorted_ids, const int* expert_ids,
                      const int* n_valid, int max_mtiles, int experts,
